@@ -3,6 +3,7 @@
   libdynamiq_eden.so   HIP kernels + C ABI (hipcc, gfx950)
   eden_utils*.so       pybind11 / libtorch binding with the reference module's
                        function names (g++), linked against libdynamiq_eden.so
+  _host*.so            the package's own host path (g++), likewise
   tests/cxx/liblaunchers_probe.so
                        test helper: a C++ caller of include/dynamiq_eden_launchers.hpp
                        (amdclang++, host code only), linked against libdynamiq_eden.so
@@ -30,6 +31,7 @@ HIP_SOURCES = [
     "dq_scaling_tile16.hip",
     "dq_grouping.hip", "dq_bitrate.hip", "dq_sort.hip",
     "dq_scaling_mixed.hip",
+    "dq_single_pass.hip",
     "dq_rht_scaling.hip", "dq_rht_compress_philox.hip", "dq_rht_compress_bf16.hip", "dq_rht_compress_f32.hip", "dq_rht_decompress.hip",
     "dq_superchunk.hip",
     "dq_hadamard.hip",
@@ -102,32 +104,41 @@ def build_kernels(verbose=True, jobs=6, only_changed=False):
     return LIB_PATH
 
 
-def extension_path():
+# module name -> source
+EXTENSIONS = {"eden_utils": "eden_utils_module.cpp", "_host": "dq_host_module.cpp"}
+
+
+def extension_path(name="eden_utils"):
     suffix = sysconfig.get_config_var("EXT_SUFFIX") or ".so"
-    return os.path.join(PKG_DIR, "eden_utils" + suffix)
+    return os.path.join(PKG_DIR, name + suffix)
 
 
-def build_extension(verbose=True):
+def _build_extension(name, verbose):
     import torch
     from torch.utils import cpp_extension as ce
 
-    out = extension_path()
+    out = extension_path(name)
     torch_lib = os.path.join(os.path.dirname(torch.__file__), "lib")
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared",
-           "-DTORCH_EXTENSION_NAME=eden_utils", "-DTORCH_API_INCLUDE_EXTENSION_H",
+           "-DTORCH_EXTENSION_NAME=" + name, "-DTORCH_API_INCLUDE_EXTENSION_H",
            # c10's HIP stream / caching-allocator headers pull in the HIP runtime API (declarations only)
            "-D__HIP_PLATFORM_AMD__=1", "-I" + os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "include"),
            "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch._C._GLIBCXX_USE_CXX11_ABI)]
     cmd += ["-I" + p for p in ce.include_paths()]
     cmd += ["-I" + sysconfig.get_paths()["include"], "-I" + os.path.join(PKG_DIR, "..", "include")]
-    cmd += [os.path.join(CSRC, "eden_utils_module.cpp"), "-o", out]
+    cmd += [os.path.join(CSRC, EXTENSIONS[name]), "-o", out]
     cmd += ["-L" + PKG_DIR, "-l:" + LIB_NAME, "-Wl,-rpath,$ORIGIN",
             "-L" + torch_lib, "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip", "-ltorch_python",
             "-Wl,-rpath," + torch_lib]
-    dt = _run(cmd, "g++ eden_utils_module.cpp")
+    dt = _run(cmd, "g++ " + EXTENSIONS[name])
     if verbose:
         print("  g++   %-28s %.1fs" % (os.path.basename(out), dt))
     return out
+
+
+def build_extension(verbose=True, names=tuple(EXTENSIONS)):
+    with ThreadPoolExecutor(max_workers=len(names)) as ex:
+        return list(ex.map(lambda name: _build_extension(name, verbose), names))[0]
 
 
 PROBE_SRC = os.path.join(PKG_DIR, "..", "tests", "cxx", "launchers_probe.cpp")
@@ -167,5 +178,7 @@ if __name__ == "__main__":
         build_kernels(only_changed="--changed" in sys.argv)
     if only in ("all", "ext"):
         build_extension()
+    if only in EXTENSIONS:
+        build_extension(names=(only,))
     if only in ("all", "probe"):
         build_launchers_probe()

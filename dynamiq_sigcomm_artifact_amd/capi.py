@@ -6,6 +6,7 @@ device index and a stream handle straight to ``libdynamiq_eden.so`` and raises
 library must be present; there is no fallback path.
 """
 import ctypes
+import importlib
 import threading
 import os
 
@@ -26,7 +27,7 @@ EXPORTS = [
     "dq_group_plan_stats_dev_u", "dq_group_plan_sorted", "dq_bitrate_hist_ints", "dq_norm_histogram", "dq_bitrate_search",
     "dq_scaling_compress_rows", "dq_scaling_dec_comp_rows", "dq_scaling_decompress_rows",
     "dq_mixed_required_bytes", "dq_mixed_compress", "dq_mixed_decompress", "dq_superchunk_stats",
-    "dq_dynamic_bitrate_bucket", "dq_streams_overlap", "dq_stream_order_after", "dq_tile_io_floor",
+    "dq_dynamic_bitrate_bucket", "dq_bucket_roundtrip", "dq_ranks_max", "dq_ranks_allreduce", "dq_streams_overlap", "dq_stream_order_after", "dq_tile_io_floor",
     "dq_superchunk_mean_center", "dq_superchunk_add_mean_copy",
     "dq_hadamard", "dq_rht_blocked", "dq_rand_diag", "dq_rand_diag_bits", "dq_rht_scaling_compress", "dq_rht_scaling_compress_mfma16", "dq_scaling_decompress_irht", "dq_pack_signs",
     "dq_bins_to_bits", "dq_bits_to_bins", "dq_quantization",
@@ -123,6 +124,8 @@ def lib():
         L.dq_superchunk_stats.argtypes = [vp, vp, vp, i64, i32, i32, i32, vp]
         L.dq_dynamic_bitrate_bucket.restype = i32
         L.dq_dynamic_bitrate_bucket.argtypes = [c.POINTER(Bucket), i32, i32, vp]
+        L.dq_ranks_max.restype = i32
+        L.dq_ranks_max.argtypes = [i32]
         L.dq_tile_io_floor.restype = i32
         L.dq_tile_io_floor.argtypes = [i32, vp, i32, vp, i32, vp, i32, i64, i32, vp]
         L.dq_stream_order_after.restype = i32
@@ -177,6 +180,21 @@ def lib():
         L.dq_quantization.argtypes = [vp, i64, i32, f32, f32, u64, vp]
         _lib = L
     return _lib
+
+
+_host = None
+
+
+def host():
+    """the native host path (csrc/dq_host_module.cpp)"""
+    global _host
+    if _host is None:
+        lib()
+        try:
+            _host = importlib.import_module(__package__ + "._host")
+        except ImportError as exc:
+            raise RuntimeError("the _host extension is not built (%s): run `python -m dynamiq_sigcomm_artifact_amd.build`" % exc) from exc
+    return _host
 
 
 def dtype_code(t):
@@ -430,6 +448,11 @@ def mixed_decompress(src, dst, order, counts, nsc, strategy, stats=None, n_limit
     _call(lib().dq_mixed_decompress, _p(src), _p(dst), _p(order), _p(counts), ring_chunk,
                                      ring_world, _ptr(stats), nsc * 256 if n_limit is None else n_limit, nsc,
                                      dtype_code(dst), _dev(dst), strategy, _stream(stream))
+
+
+def ranks_max(pooled=False):
+    """simulated ranks that one launch of the all-reduce without a packed stream takes"""
+    return int(lib().dq_ranks_max(1 if pooled else 0))
 
 
 def bucket_descriptor(src, n, stats, mean, order, work, packed, strategy=2, out=None, u=0.0, reduced_stats=None,

@@ -558,6 +558,103 @@ int dq_dynamic_bitrate_bucket(const dq_bucket_t *b, int stages, int device, dq_s
     return finish(e);
 }
 
+int dq_bucket_roundtrip(const dq_roundtrip_t *buckets, int count, int dtype, int strategy, int center_world, double u,
+                        const double *u_dev, uint64_t seed, uint64_t *step_dev, uint64_t step_more, uint32_t *hist,
+                        int64_t hist_ints, int device, dq_stream_t stream)
+{
+    if (!buckets) return fail(DQ_ERR_NULL);
+    if (!(count > 0)) return fail(DQ_ERR_N, "count");
+    if (strategy != 2 && strategy != 3) return fail(DQ_ERR_STRATEGY);
+    if (dtype != DQ_BF16 && dtype != DQ_F32) return fail(DQ_ERR_DTYPE);
+    if (!(center_world > 0)) return fail(DQ_ERR_WORLD_SIZE);
+    if (!u_dev && u != u) return fail(DQ_ERR_SIZE, "u must be a number");
+    if (hist && hist_ints < dq::bitrate_hist_ints()) return fail(DQ_ERR_SIZE, "hist buffer is too small");
+    int64_t tiles = 0;
+    for (int k = 0; k < count; k++) {
+        const dq_roundtrip_t &b = buckets[k];
+        if (!(b.n > 0) || (b.n + 255) / 256 > (int64_t)0x7fffffff) return fail(DQ_ERR_N);
+        if (!b.src || !b.out || !b.stats || !b.counts) return fail(DQ_ERR_NULL);
+        if (reinterpret_cast<uintptr_t>(b.stats) & 3) return fail(DQ_ERR_SIZE, "stats must be 4-byte aligned");
+    }
+    int rc;
+    if ((rc = select_device(device))) return rc;
+    const dq::MeeParams mp[3] = {mee_params(8), mee_params(4), mee_params(2)};
+    for (int k = 0; k < count;) {
+        // as many buckets as the descriptors of a launch and its grid hold
+        int take = 0;
+        tiles = 0;
+        while (k + take < count && take < dq::kMaxBuckets && (take == 0 || tiles + (buckets[k + take].n >> 10) < (int64_t)0x7fffff00))
+            tiles += (buckets[k + take++].n >> 10) + 1;
+        const hipError_t e = dq::launch_roundtrip(buckets + k, take, center_world, (float)u, u_dev, seed, step_dev, step_more, hist, dtype,
+                                                  strategy == 3, mp, static_cast<hipStream_t>(stream));
+        if (e != hipSuccess) return finish(e);
+        step_more = 0; // the first launch has advanced the counter
+        k += take;
+    }
+    return ok();
+}
+
+int dq_ranks_max(int pooled) { return pooled ? dq::kMaxPoolRanks : dq::kMaxRanks; }
+
+int dq_ranks_allreduce(const dq_ranks_t *r, int stages, int device, dq_stream_t stream)
+{
+    if (!r) return fail(DQ_ERR_NULL);
+    if (stages <= 0 || stages > 7) return fail(DQ_ERR_SIZE, "stages must be a combination of DQ_RANKS_*");
+    if (!(r->n > 0)) return fail(DQ_ERR_N);
+    const int64_t nsc = (r->n + 255) / 256;
+    int rc = check_mixed(nsc, 0, r->world, r->dtype, r->strategy, false);
+    if (rc) return fail(rc);
+    if (r->world > dq_ranks_max(r->pool != nullptr)) return fail(DQ_ERR_WORLD_SIZE, "more ranks than one launch takes (dq_ranks_max)");
+    const bool s_stats = stages & DQ_RANKS_STATS, s_plan = stages & DQ_RANKS_PLAN, s_ring = stages & DQ_RANKS_RING;
+    if (!r->total || ((s_stats || s_ring) && (!r->src || !r->mean)) || ((s_plan || s_ring) && (!r->order || !r->work)) ||
+        (s_ring && (!r->out || (r->pool && !r->first))))
+        return fail(DQ_ERR_NULL);
+    if (reinterpret_cast<uintptr_t>(r->total) & 3) return fail(DQ_ERR_SIZE, "total must be 4-byte aligned");
+    for (int k = 0; k < r->world; k++) {
+        if ((s_stats || s_ring) && !r->src[k]) return fail(DQ_ERR_NULL);
+        if (s_ring && !r->out[k]) return fail(DQ_ERR_NULL);
+    }
+    if (s_plan && r->sorted_plan) {
+        if (r->top_count < 0 || r->bottom_count < 0 || r->top_count + r->bottom_count > nsc)
+            return fail(DQ_ERR_SIZE, "top_count and bottom_count must be non-negative and sum to at most nsc");
+        if (r->work_ints < dq_group_plan_sorted_work_ints(nsc)) return fail(DQ_ERR_SIZE, "work buffer is too small");
+    } else if (s_plan) {
+        if (r->work_ints < dq::group_plan_work_ints(nsc)) return fail(DQ_ERR_SIZE, "work buffer is too small");
+        if (r->hist && r->hist_ints < dq::bitrate_hist_ints()) return fail(DQ_ERR_SIZE, "hist buffer is too small");
+        if (!r->u_dev && r->u != r->u) return fail(DQ_ERR_SIZE, "u must be a number");
+    }
+    if ((rc = select_device(device))) return rc;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    hipError_t e = hipSuccess;
+    if (s_stats) e = dq::launch_ranks_stats(r->src, r->world, r->n, r->total, r->mean, r->dtype, s);
+    if (e == hipSuccess && s_plan) {
+        // (with u in device memory the histogram is filled by a few more workgroups of the plan launch)
+        if (!r->sorted_plan && r->hist && !r->u_dev) e = dq::launch_norm_histogram(r->total, nsc, r->hist, s);
+        if (e != hipSuccess) return finish(e);
+        if (!r->sorted_plan)
+            e = dq::launch_group_plan_stats(r->total, (float)r->u, r->u_dev, nsc, nullptr, r->order, r->work, r->u_dev ? r->hist : nullptr, s);
+        else if (nsc > kSortedPlanOneLaunch)
+            e = dq::launch_group_plan_sorted_large(r->total, nsc, r->top_count, r->bottom_count, nullptr, r->order, r->work, r->work_ints, s);
+        else
+            e = dq::launch_group_plan_sorted(r->total, nsc, r->top_count, r->bottom_count, nullptr, r->order, r->work, s);
+    }
+    if (e == hipSuccess && s_ring) {
+        const dq::MeeParams mp[3] = {mee_params(8), mee_params(4), mee_params(2)};
+        dq::RingDesc d;
+        memset(&d, 0, sizeof(d));
+        d.src = r->src; d.out = r->out; d.world = r->world; d.n = r->n; d.total = r->total; d.mean = r->mean;
+        d.order = r->order; d.counts = r->work; d.seed = r->seed; d.pooled = r->pool != nullptr;
+        for (int g = 0; d.pooled && g < 3; g++) {
+            for (int k = 0; k < r->world; k++) {
+                d.pool[g][k] = r->pool[g * r->world + k];
+                for (int step = 0; step < r->world; step++) d.first[g][k][step] = r->first[(g * r->world + k) * r->world + step];
+            }
+        }
+        e = dq::launch_ring(d, r->dtype, r->strategy == 3, mp, s);
+    }
+    return finish(e);
+}
+
 int dq_scaling_compress_philox(const void *src, uint8_t *dst, int64_t n, int nbits, int chunk_size, int dtype, int device,
                                int strategy, uint64_t seed, uint64_t step, dq_stream_t stream)
 {

@@ -1050,7 +1050,7 @@ static int host_qbits_of_norm(uint32_t norm_bits, float u) // qbits_of_norm of d
 
 // the smallest pattern in [0, kMaxPattern] whose width is >= target, kMaxPattern + 1 if none (the width is a
 // monotone step function of the pattern: width_thresholds() on the device relies on the same)
-static int host_width_threshold(float u, int target)
+int host_width_threshold(float u, int target)
 {
     int lo = 0, hi = kMaxPattern + 1; // the answer lies in [lo, hi]
     while (lo < hi) {

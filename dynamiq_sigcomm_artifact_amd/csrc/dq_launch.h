@@ -89,6 +89,34 @@ hipError_t launch_mixed_decompress(const uint8_t *src, void *dst, const int32_t 
                                    int ring_chunk, int ring_world, const void *stats, int64_t limit, int64_t nsc,
                                    int dtype, bool mee, const MeeParams *mp, hipStream_t stream);
 
+// the all-reduce of buckets whose ranks share this GPU's memory, without a packed stream (dq_single_pass.hip)
+constexpr int kMaxBuckets = 32;   // per launch of the one-rank kernel (their descriptors are kernel arguments)
+constexpr int kMaxRanks = 16;     // simulated ranks, likewise
+constexpr int kMaxPoolRanks = 8;  // simulated ranks with random pools: three tables of ranks x steps travel with the launch
+typedef dq_roundtrip_t RoundtripDesc;
+// *step_dev + step_more is added to every bucket's step, and *step_dev left there, when step_dev is set
+hipError_t launch_roundtrip(const RoundtripDesc *desc, int count, int world, float u, const double *u_dev, uint64_t seed,
+                            uint64_t *step_dev, uint64_t step_more, uint32_t *hist, int dtype, bool mee, const MeeParams *mp,
+                            hipStream_t stream);
+// total: bf16 pairs [nsc], mean: float [world][nsc]
+hipError_t launch_ranks_stats(const void *const *src, int world, int64_t n, void *total, float *mean, int dtype,
+                              hipStream_t stream);
+struct RingDesc {
+    const void *const *src;
+    void *const *out;
+    int world;
+    int64_t n;
+    const void *total;
+    const float *mean;
+    const int32_t *order, *counts;
+    uint64_t seed;                               // rank r draws from seed + r, step s of the ring from step s
+    bool pooled;                                 // or the random values come from pools:
+    const void *pool[3][kMaxPoolRanks];          // by width (8, 4, 2 bits) and rank
+    int32_t first[3][kMaxPoolRanks][kMaxPoolRanks]; // first row of 16 values, by width, rank and step
+};
+hipError_t launch_ring(const RingDesc &d, int dtype, bool mee, const MeeParams *mp, hipStream_t stream);
+int host_width_threshold(float u, int target);
+
 // superchunk mean-centring (dq_superchunk.hip)
 // residual == nullptr: statistics only; mean_out (nullable) receives the binary32 means
 hipError_t launch_mean_center(const void *src, void *residual, void *stats, float *mean_out, int64_t n,

@@ -1,0 +1,554 @@
+// The compressed all-reduce of a bucket without a packed stream in memory.
+//
+// Where all ranks of a ring live in one GPU's memory -- a ring of one rank, or W simulated ones -- the records that a
+// ring step writes are read back by the next step's launch and by nobody else.  A superchunk's way through the ring
+// touches no other superchunk: compress on the first rank, decode + add + recompress on each of the others, decode on
+// all.  So a wave takes a tile of four superchunks and runs that whole chain in registers (dq_widths.cuh: the levels
+// of a chunk instead of its bits), reading every rank's elements once and writing every rank's result once.
+//
+//   roundtrip_kernel   one rank: statistics, width, centring, compress, decompress, mean add -- one pass over the
+//                      bucket, and up to kMaxBuckets buckets per launch
+//   tally_kernel       behind it: the widths' counts per bucket and the norm histogram of the search for u
+//   ranks_stats_kernel W ranks: every rank's means, and the reduced statistics
+//   ring_kernel        W ranks, after a plan of the reduced statistics: the ring
+//
+// Measured, start -> now (bit-identical results): 8 ranks x 124,439,808 bf16 elements 2,884 -> 1,186 us per all-reduce (one
+// launch per rank and ring step, packed streams and their exchange copies, against three launches whose traffic is the
+// vectors alone), 8 x 1,000,003 elements 1,493 -> 31 us (257 launches against 3), a step of nine 25 MB buckets on one rank
+// 250 -> 102 us (four launches per bucket on two streams against two launches per step, and the search for u).
+//
+// Numerics: csrc/cuda_hadamard.cu:1257-1369 (centring, mean add), csrc/cuda_hierarchical_mee.cu:203-696 (codec),
+// testbed_evaluation/new_comm_hooks/ring_rdma.py:590-631 (order of the ring), comm_hooks.py:64-70 (widths).
+#include <stddef.h>
+#include <string.h>
+
+#include <type_traits>
+
+#include "dq_widths.cuh"
+#include "dq_bitwidth.cuh"
+#include "dq_launch.h"
+
+namespace dq {
+
+namespace {
+
+// the tile's values leave as whole superchunks: through LDS (slots swizzled), then contiguous 16-byte streaming stores.
+// sc: the superchunk of this lane's row; stage holds 64 * kSlots 16-byte slots of this wave.
+template <int DT> __device__ __forceinline__ void stage_tile(const Raw16<DT> &out, uint4 *stage, int lane)
+{
+    constexpr int S = Raw16<DT>::kSlots;
+#pragma unroll
+    for (int k = 0; k < S; k++) stage[swz(S * lane + k)] = out.slot(k);
+    wave_lds_sync();
+}
+
+template <int DT>
+__device__ __forceinline__ void store_tile(void *dst, const Raw16<DT> &out, const uint4 *stage, int64_t sc, int rows_here, int64_t n,
+                                           bool vec, int lane)
+{
+    constexpr int S = Raw16<DT>::kSlots;
+    constexpr int ESZ = DT == DQ_F32 ? 4 : 2;
+    constexpr int EP = 16 / ESZ;
+    char *bytes = static_cast<char *>(dst);
+    if (vec) {
+#pragma unroll
+        for (int k = 0; k < S; k++) {
+            const int s = 64 * k + lane;
+            const int row = s / (16 * S);
+            const int64_t e = (int64_t)__shfl((int)sc, row * 16, 64) * 256 + (s % (16 * S)) * EP;
+            if (row < rows_here) {
+                const uint4 val = stage[swz(s)];
+                if (e + EP <= n) {
+                    stream_store(reinterpret_cast<uint4 *>(bytes + e * ESZ), val);
+                } else {
+                    const uint32_t part[4] = {val.x, val.y, val.z, val.w};
+#pragma unroll
+                    for (int i = 0; i < EP; i++) {
+                        if (e + i < n) {
+                            if (DT == DQ_F32)
+                                reinterpret_cast<uint32_t *>(bytes)[e + i] = part[i];
+                            else
+                                reinterpret_cast<uint16_t *>(bytes)[e + i] = (uint16_t)(part[i >> 1] >> (16 * (i & 1)));
+                        }
+                    }
+                }
+            }
+        }
+    } else if ((lane >> 4) < rows_here) {
+        const int64_t e = sc * 256 + (lane & 15) * 16;
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            if (e + i < n) {
+                if (DT == DQ_F32)
+                    reinterpret_cast<uint32_t *>(bytes)[e + i] = out.w[i];
+                else
+                    reinterpret_cast<uint16_t *>(bytes)[e + i] = (uint16_t)(out.w[i >> 1] >> (16 * (i & 1)));
+            }
+        }
+    }
+}
+
+// T(T(level * step) + mean)
+template <int DT> __device__ __forceinline__ void decode_with_mean(Raw16<DT> &out, float (&lev)[16], float step, float mean)
+{
+#pragma unroll
+    for (int i = 0; i < 16; i++) lev[i] = lev[i] * step;
+    out.set(lev);
+#pragma unroll
+    for (int i = 0; i < 16; i++) lev[i] = out.get(i) + mean;
+    out.set(lev);
+}
+
+// ---- one rank -------------------------------------------------------------------------------------------
+
+struct RoundtripBucket {
+    const void *src;
+    void *out;
+    uint32_t *stats;
+    int32_t *counts;
+    int64_t n;
+    uint64_t step;
+    int vec; // src and out 16-byte aligned
+};
+
+struct WidthRule {
+    float u;
+    const double *u_dev; // when set: u is *u_dev
+    int thr[2];          // with u a number: the patterns of width 4 and 8 found on the host, else -1
+};
+
+struct RoundtripArgs {
+    uint32_t first_tile[kMaxBuckets]; // ascending; 2^32 - 1 behind the last bucket
+    RoundtripBucket bucket[kMaxBuckets];
+    WidthRule rule;
+    WorldDiv wd;
+    uint64_t seed;
+    const uint64_t *step_dev; // null, or added to every bucket's step
+    uint64_t step_more;       // (with step_dev) and this, which tally_kernel leaves in *step_dev
+    WidthSet widths;
+};
+
+__device__ __forceinline__ int class_of_norm(uint32_t pattern, float u, const int (&thr)[2])
+{
+    if (thr[0] >= 0 && __builtin_amdgcn_ballot_w64(pattern > (uint32_t)kMaxPattern) == 0)
+        return (int)pattern >= thr[1] ? 0 : ((int)pattern >= thr[0] ? 1 : 2);
+    const int64_t q = qbits_of_norm(pattern, u);
+    return q == 8 ? 0 : (q == 4 ? 1 : 2);
+}
+
+template <int DT, bool MEE> __global__ __launch_bounds__(64) void roundtrip_kernel(RoundtripArgs a)
+{
+    constexpr int kStage = 64 * Raw16<DT>::kSlots * 16;
+    __shared__ __attribute__((aligned(16))) uint8_t lds[StatsTile<DT>::BYTES > kStage ? StatsTile<DT>::BYTES : kStage];
+    __shared__ float levels[MEE ? kLevelCount : 1];
+    const int lane = threadIdx.x, row = lane >> 4, j = lane & 15;
+
+    uint64_t step = a.step_dev ? *a.step_dev + a.step_more : 0;
+    const float u = a.rule.u_dev ? (float)*a.rule.u_dev : a.rule.u;
+    int at = 0;
+#pragma unroll
+    for (int k = 1; k < kMaxBuckets; k++) at += blockIdx.x >= a.first_tile[k] ? 1 : 0;
+    const RoundtripBucket &b = a.bucket[at];
+    const int64_t n = b.n, nsc = (n + 255) >> 8;
+    const int64_t sc0 = (int64_t)(blockIdx.x - a.first_tile[at]) * kRowsPerWave;
+    if (sc0 >= nsc) return;
+    const int rows_here = (int)min((int64_t)kRowsPerWave, nsc - sc0);
+    const bool active = row < rows_here;
+    const int64_t sc = sc0 + min(row, rows_here - 1);
+    const int64_t e0 = sc * 256 + j * 16;
+
+    Raw16<DT> v;
+    v.zero();
+    if (active) load_chunk<DT>(v, b.src, e0, n, b.vec != 0);
+    if (MEE) levels_to_lds(a.widths, levels, lane);
+    // the rounding stream's arithmetic while the elements are on their way
+    Raw16<DQ_PHILOX> r;
+    r.generate(RandKey{a.seed, b.step + step}, sc * 16 + j);
+    r.pin();
+
+    float sum, sq;
+    tile_sums<DT>(v, a.wd, lds, lane, sum, sq);
+    const float mean = __shfl(superchunk_mean(sum, min((int64_t)256, n - sc * 256)), lane & 48, 64);
+    const uint32_t norm = (uint32_t)__shfl((int)f32_to_bf16_bits(sq), lane & 48, 64);
+    const uint32_t mean_bits = f32_to_bf16_bits(mean);
+    if (active && j == 0) b.stats[sc] = mean_bits | (norm << 16);
+    if (sc0 == 0 && lane < 4) b.counts[lane] = 0; // (tally_kernel adds to them)
+
+    const WidthRegs<MEE> w = width_regs<MEE>(a.widths, class_of_norm(norm, u, a.rule.thr), levels);
+    center_loaded<DT>(v, a.wd, active ? mean : 0.0f, e0, n);
+    float lev[16];
+    const float scale = quantize_chunk<MEE>(v, r, w, lev);
+    decode_with_mean<DT>(v, lev, scale, bf16_bits_to_f32(mean_bits));
+    wave_lds_sync(); // the statistics' tile has been read
+    stage_tile<DT>(v, reinterpret_cast<uint4 *>(lds), lane);
+    store_tile<DT>(b.out, v, reinterpret_cast<const uint4 *>(lds), sc, rows_here, n, b.vec != 0, lane);
+}
+
+struct TallyBucket {
+    const uint16_t *stats;
+    int32_t *counts;
+    int64_t nsc;
+};
+
+struct TallyArgs {
+    uint32_t first_block[kMaxBuckets];
+    TallyBucket bucket[kMaxBuckets];
+    WidthRule rule;
+    uint32_t *hist;
+    uint64_t *step_dev;
+    uint64_t step_more;
+};
+
+constexpr int kTallyThreads = kHistThreads; // a workgroup takes kHistBatch superchunks of one bucket
+
+template <bool HIST> __global__ __launch_bounds__(kTallyThreads) void tally_kernel(TallyArgs a)
+{
+    __shared__ uint32_t local[HIST ? kHistWords : 1];
+    __shared__ int thr[2];
+    __shared__ uint32_t total[2];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int at = 0;
+#pragma unroll
+    for (int k = 1; k < kMaxBuckets; k++) at += blockIdx.x >= a.first_block[k] ? 1 : 0;
+    const TallyBucket b = a.bucket[at];
+    const int64_t begin = (int64_t)(blockIdx.x - a.first_block[at]) * kHistBatch;
+    const int64_t end = min(begin + (int64_t)kHistBatch, b.nsc);
+    constexpr int kPer = kHistBatch / kTallyThreads;
+    uint32_t norm[kPer];
+#pragma unroll
+    for (int k = 0; k < kPer; k++) {
+        const int64_t i = begin + k * kTallyThreads + threadIdx.x;
+        norm[k] = i < end ? (uint32_t)b.stats[2 * i + 1] : 0u;
+    }
+    const float u = a.rule.u_dev ? (float)*a.rule.u_dev : a.rule.u;
+    if (a.rule.thr[0] >= 0) {
+        if (threadIdx.x < 2) thr[threadIdx.x] = a.rule.thr[threadIdx.x];
+    } else {
+        width_thresholds(u, thr, wave, lane);
+    }
+    if (threadIdx.x < 2) total[threadIdx.x] = 0u;
+    if (HIST) {
+        for (int w = threadIdx.x; w < kHistWords; w += kTallyThreads) local[w] = 0u;
+    }
+    __syncthreads();
+    const int t2[2] = {thr[0], thr[1]};
+    uint32_t n8 = 0, n4 = 0;
+#pragma unroll
+    for (int k = 0; k < kPer; k++) {
+        const int64_t i = begin + k * kTallyThreads + threadIdx.x;
+        const bool in = i < end;
+        const int c = class_of_norm(norm[k], u, t2);
+        n8 += (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(in && c == 0));
+        n4 += (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(in && c == 1));
+        if (HIST && in) {
+            const int bin = bin_of(norm[k]);
+            atomicAdd(&local[bin >> 1], 1u << (16 * (bin & 1)));
+        }
+    }
+    if (lane == 0 && n8) atomicAdd(&total[0], n8);
+    if (lane == 0 && n4) atomicAdd(&total[1], n4);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const int c8 = (int)total[0], c4 = (int)total[1], c2 = (int)(end - begin) - c8 - c4;
+        if (c8) atomicAdd(&b.counts[0], c8);
+        if (c4) atomicAdd(&b.counts[1], c4);
+        if (c2) atomicAdd(&b.counts[2], c2);
+        if (blockIdx.x == 0 && a.step_dev && a.step_more) *a.step_dev += a.step_more;
+    }
+    if (HIST) {
+        for (int w = threadIdx.x; w < kHistWords; w += kTallyThreads) {
+            const uint32_t pair = local[w];
+            if (pair & 0xffffu) atomicAdd(&a.hist[2 * w], pair & 0xffffu);
+            if (pair >> 16) atomicAdd(&a.hist[2 * w + 1], pair >> 16);
+        }
+    }
+}
+
+// ---- W ranks --------------------------------------------------------------------------------------------
+
+struct RankPointers {
+    const void *src[kMaxRanks];
+};
+
+constexpr int kStatsWaves = 8; // ranks in flight per workgroup of ranks_stats_kernel
+
+// A workgroup takes a tile of four superchunks, a wave of it the tile of one rank (of every kStatsWaves-th one in a larger
+// world): means and norms per rank, and the statistics all-reduce as the reference's chain of bf16 additions in rank order.
+template <int DT>
+__global__ __launch_bounds__(64 * kStatsWaves) void ranks_stats_kernel(RankPointers ranks, int world, int64_t n, int vec,
+                                                                      uint32_t *__restrict__ total, float *__restrict__ mean_out,
+                                                                      WorldDiv wd)
+{
+    extern __shared__ __attribute__((aligned(16))) uint8_t tiles[];
+    __shared__ uint32_t pairs[kMaxRanks][kRowsPerWave];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
+    const int row = lane >> 4, j = lane & 15;
+    const int64_t nsc = (n + 255) >> 8;
+    const int64_t sc0 = (int64_t)blockIdx.x * kRowsPerWave;
+    const int rows_here = (int)min((int64_t)kRowsPerWave, nsc - sc0);
+    const int64_t sc = sc0 + min(row, rows_here - 1);
+    uint8_t *lds = tiles + wave * StatsTile<DT>::BYTES;
+    for (int rank = wave; rank < world; rank += waves) {
+        Raw16<DT> v;
+        v.zero();
+        if (row < rows_here) load_chunk<DT>(v, ranks.src[rank], sc * 256 + j * 16, n, vec != 0);
+        float sum, sq;
+        tile_sums<DT>(v, wd, lds, lane, sum, sq);
+        wave_lds_sync();
+        if (j == 0) {
+            const float mean = superchunk_mean(sum, min((int64_t)256, n - sc * 256));
+            pairs[rank][row] = f32_to_bf16_bits(mean) | (f32_to_bf16_bits(sq) << 16);
+            if (row < rows_here) mean_out[rank * nsc + sc] = mean;
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < rows_here) {
+        uint32_t acc = pairs[0][threadIdx.x];
+        for (int rank = 1; rank < world; rank++) {
+            const uint32_t p = pairs[rank][threadIdx.x];
+            const float lo = bf16_bits_to_f32(acc & 0xffffu) + bf16_bits_to_f32(p & 0xffffu);
+            const float hi = bf16_bits_to_f32(acc >> 16) + bf16_bits_to_f32(p >> 16);
+            acc = f32_to_bf16_bits(lo) | (f32_to_bf16_bits(hi) << 16);
+        }
+        total[sc0 + threadIdx.x] = acc;
+    }
+}
+
+// rounding randomness out of the compressors' pools: which rank uses which rows of which pool in which step
+struct NoPools {};
+struct Pools {
+    const void *pool[3][kMaxPoolRanks];                          // one per width (8, 4, 2 bits) and rank
+    int32_t first[3][kMaxPoolRanks][kMaxPoolRanks];              // first row of 16 values: [width][rank][step]
+};
+
+template <bool POOL> struct RingArgs {
+    const void *src[kMaxRanks];
+    void *out[kMaxRanks];
+    const float *mean;      // [world][nsc]
+    const uint16_t *total;  // reduced statistics
+    const int32_t *order;   // the plan: row lists and group sizes
+    const int32_t *counts;
+    int64_t n;
+    int nsc, world, vec;
+    RandKey key;
+    WorldDiv wd;
+    WidthSet widths;
+    typename std::conditional<POOL, Pools, NoPools>::type pools;
+};
+
+// Workgroup (x, y): tile x of ring chunk y -- rank y compresses it first, rank y + 1 decodes, adds and recompresses, and
+// so on around the ring; the last one's records are what every rank decodes.  The runs of the chunk follow one another as in
+// dq_scaling_mixed.hip (8-bit, 4-bit, 2-bit), so a wave has one width and one first rank.
+template <int DT, int RDT, bool MEE> __global__ __launch_bounds__(64) void ring_kernel(RingArgs<RDT != DQ_PHILOX> a)
+{
+    __shared__ __attribute__((aligned(16))) uint4 stage[64 * Raw16<DT>::kSlots];
+    __shared__ float levels[MEE ? kLevelCount : 1];
+    const int lane = threadIdx.x, row = lane >> 4, j = lane & 15;
+    const int chunk = blockIdx.y, world = a.world;
+    // the run this tile lies in: group sizes clamped so that a corrupt count cannot lead outside the lists
+    int cls = 3, tile = blockIdx.x, cnt = 0;
+    int64_t row0 = 0;
+    {
+        int used = 0;
+        const int counts[3] = {a.counts[0], a.counts[1], a.counts[2]};
+#pragma unroll
+        for (int g = 0; g < 3; g++) {
+            const int m = min(max(counts[g], 0), a.nsc - used);
+            const int per = (m + world - 1) / world;
+            const int begin = (int)min((int64_t)per * chunk, (int64_t)m);
+            const int here = min(per, m - begin);
+            const int tiles = (here + kRowsPerWave - 1) / kRowsPerWave;
+            if (cls == 3) {
+                if (tile < tiles) {
+                    cls = g; cnt = here; row0 = (int64_t)g * a.nsc + begin;
+                } else {
+                    tile -= tiles;
+                }
+            }
+            used += m;
+        }
+    }
+    if (cls == 3) return;
+    const int k0 = tile * kRowsPerWave;
+    const int rows_here = min(kRowsPerWave, cnt - k0);
+    const bool active = row < rows_here;
+    const int64_t sc = a.order[row0 + k0 + min(row, rows_here - 1)];
+    const int64_t e0 = sc * 256 + j * 16;
+    if (MEE) levels_to_lds(a.widths, levels, lane);
+    const WidthRegs<MEE> w = width_regs<MEE>(a.widths, cls, levels);
+    const uint32_t total_mean = a.total[2 * sc];
+
+    // the next rank's elements (and random values) are on their way while this rank's are quantised
+    Raw16<DT> next;
+    Raw16<RDT> next_r;
+    float next_mean = 0.0f;
+    next.zero();
+    next_r.zero();
+    const auto fetch = [&](int step) {
+        int rank = chunk + step;
+        if (rank >= world) rank -= world;
+        if (active) {
+            load_chunk<DT>(next, a.src[rank], e0, a.n, a.vec & 1);
+            next_mean = a.mean[(int64_t)rank * a.nsc + sc];
+            if constexpr (RDT != DQ_PHILOX)
+                next_r.load(a.pools.pool[cls][rank], ((int64_t)a.pools.first[cls][rank][step] + k0 * 16 + lane) * 16, (a.vec & 4) != 0);
+        }
+    };
+    fetch(0);
+    Raw16<DT> v;
+    float lev[16], scale = 0.0f;
+#pragma unroll 1
+    for (int step = 0; step < world; step++) {
+        v = next;
+        Raw16<RDT> r = next_r;
+        const float mean = next_mean;
+        if (step + 1 < world) fetch(step + 1);
+        if constexpr (RDT == DQ_PHILOX) {
+            int rank = chunk + step;
+            if (rank >= world) rank -= world;
+            r.generate(RandKey{a.key.seed + (uint64_t)rank, (uint64_t)step}, sc * 16 + j);
+        }
+        center_loaded<DT>(v, a.wd, mean, e0, a.n);
+        if (step > 0) {
+#pragma unroll
+            for (int i = 0; i < 16; i++) lev[i] = __builtin_fmaf(lev[i], scale, v.get(i));
+            v.set(lev); // the sum in the element type
+        }
+        scale = quantize_chunk<MEE>(v, r, w, lev);
+    }
+    decode_with_mean<DT>(v, lev, scale, bf16_bits_to_f32(total_mean));
+    stage_tile<DT>(v, stage, lane);
+    for (int rank = 0; rank < world; rank++) store_tile<DT>(a.out[rank], v, stage, sc, rows_here, a.n, (a.vec & 2) != 0, lane);
+}
+
+WidthRule make_rule(float u, const double *u_dev)
+{
+    WidthRule r{u, u_dev, {-1, -1}};
+    if (!u_dev && u == u) {
+        r.thr[0] = host_width_threshold(u, 4);
+        r.thr[1] = host_width_threshold(u, 8);
+    }
+    return r;
+}
+
+} // namespace
+
+// count <= kMaxBuckets
+hipError_t launch_roundtrip(const RoundtripDesc *desc, int count, int world, float u, const double *u_dev, uint64_t seed,
+                            uint64_t *step_dev, uint64_t step_more, uint32_t *hist, int dtype, bool mee, const MeeParams *mp,
+                            hipStream_t stream)
+{
+    RoundtripArgs a;
+    TallyArgs t;
+    memset(&t, 0, sizeof(t));
+    memset(&a, 0, offsetof(RoundtripArgs, rule));
+    uint32_t tiles = 0, blocks = 0;
+    for (int k = 0; k < kMaxBuckets; k++) {
+        if (k >= count) {
+            a.first_tile[k] = t.first_block[k] = 0xffffffffu;
+            continue;
+        }
+        const RoundtripDesc &d = desc[k];
+        const int64_t nsc = (d.n + 255) / 256;
+        a.first_tile[k] = tiles;
+        t.first_block[k] = blocks;
+        a.bucket[k] = RoundtripBucket{d.src, d.out, static_cast<uint32_t *>(d.stats), d.counts, d.n, d.step,
+                                      aligned16(d.src) && aligned16(d.out) ? 1 : 0};
+        t.bucket[k] = TallyBucket{static_cast<const uint16_t *>(d.stats), d.counts, nsc};
+        tiles += (uint32_t)((nsc + kRowsPerWave - 1) / kRowsPerWave);
+        blocks += (uint32_t)((nsc + kHistBatch - 1) / kHistBatch);
+    }
+    a.rule = t.rule = make_rule(u, u_dev);
+    a.wd = make_world_div(world, dtype == DQ_F32 ? 4 : 2);
+    a.seed = seed;
+    a.step_dev = step_dev;
+    a.step_more = step_more;
+    a.widths = make_width_set(mp, mee);
+    t.hist = hist;
+    t.step_dev = step_dev;
+    t.step_more = step_more;
+    if (dtype == DQ_BF16) {
+        if (mee) hipLaunchKernelGGL((roundtrip_kernel<DQ_BF16, true>), dim3(tiles), dim3(64), 0, stream, a);
+        else hipLaunchKernelGGL((roundtrip_kernel<DQ_BF16, false>), dim3(tiles), dim3(64), 0, stream, a);
+    } else {
+        if (mee) hipLaunchKernelGGL((roundtrip_kernel<DQ_F32, true>), dim3(tiles), dim3(64), 0, stream, a);
+        else hipLaunchKernelGGL((roundtrip_kernel<DQ_F32, false>), dim3(tiles), dim3(64), 0, stream, a);
+    }
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    if (hist) hipLaunchKernelGGL(tally_kernel<true>, dim3(blocks), dim3(kTallyThreads), 0, stream, t);
+    else hipLaunchKernelGGL(tally_kernel<false>, dim3(blocks), dim3(kTallyThreads), 0, stream, t);
+    return hipGetLastError();
+}
+
+hipError_t launch_ranks_stats(const void *const *src, int world, int64_t n, void *total, float *mean, int dtype, hipStream_t stream)
+{
+    RankPointers p;
+    int vec = 1;
+    for (int r = 0; r < kMaxRanks; r++) {
+        p.src[r] = r < world ? src[r] : nullptr;
+        if (r < world && !aligned16(src[r])) vec = 0;
+    }
+    const int64_t nsc = (n + 255) / 256;
+    const dim3 grid((unsigned)((nsc + kRowsPerWave - 1) / kRowsPerWave));
+    const int waves = world < kStatsWaves ? world : kStatsWaves;
+    const WorldDiv wd = make_world_div(world, dtype == DQ_F32 ? 4 : 2);
+    uint32_t *tot = static_cast<uint32_t *>(total);
+    if (dtype == DQ_BF16)
+        hipLaunchKernelGGL(ranks_stats_kernel<DQ_BF16>, grid, dim3(64 * waves), waves * StatsTile<DQ_BF16>::BYTES, stream, p, world, n, vec,
+                           tot, mean, wd);
+    else
+        hipLaunchKernelGGL(ranks_stats_kernel<DQ_F32>, grid, dim3(64 * waves), waves * StatsTile<DQ_F32>::BYTES, stream, p, world, n, vec,
+                           tot, mean, wd);
+    return hipGetLastError();
+}
+
+template <int DT, int RDT>
+static hipError_t run_ring(const RingDesc &d, bool mee, const MeeParams *mp, hipStream_t stream)
+{
+    constexpr bool POOL = RDT != DQ_PHILOX;
+    RingArgs<POOL> a;
+    memset(&a, 0, sizeof(a));
+    bool in = true, out = true, pool = true;
+    for (int r = 0; r < d.world; r++) {
+        a.src[r] = d.src[r];
+        a.out[r] = d.out[r];
+        in = in && aligned16(d.src[r]);
+        out = out && aligned16(d.out[r]);
+        if constexpr (POOL) {
+            for (int g = 0; g < 3; g++) {
+                a.pools.pool[g][r] = d.pool[g][r];
+                pool = pool && aligned16(d.pool[g][r]);
+                for (int s = 0; s < d.world; s++) a.pools.first[g][r][s] = d.first[g][r][s];
+            }
+        }
+    }
+    a.mean = d.mean;
+    a.total = static_cast<const uint16_t *>(d.total);
+    a.order = d.order;
+    a.counts = d.counts;
+    a.n = d.n;
+    a.nsc = (int)((d.n + 255) / 256);
+    a.world = d.world;
+    a.vec = (in ? 1 : 0) | (out ? 2 : 0) | (pool ? 4 : 0);
+    a.key = RandKey{d.seed, 0};
+    a.wd = make_world_div(d.world, DT == DQ_F32 ? 4 : 2);
+    a.widths = make_width_set(mp, mee);
+    // every run rounds its superchunks per ring chunk up to whole tiles
+    const dim3 grid((unsigned)(a.nsc / (kRowsPerWave * d.world) + 4), (unsigned)d.world);
+    if (mee) hipLaunchKernelGGL((ring_kernel<DT, RDT, true>), grid, dim3(64), 0, stream, a);
+    else hipLaunchKernelGGL((ring_kernel<DT, RDT, false>), grid, dim3(64), 0, stream, a);
+    return hipGetLastError();
+}
+
+hipError_t launch_ring(const RingDesc &d, int dtype, bool mee, const MeeParams *mp, hipStream_t stream)
+{
+    if (dtype == DQ_BF16) {
+        if (d.pooled) return run_ring<DQ_BF16, DQ_BF16>(d, mee, mp, stream);
+        return run_ring<DQ_BF16, DQ_PHILOX>(d, mee, mp, stream);
+    }
+    if (d.pooled) return run_ring<DQ_F32, DQ_F32>(d, mee, mp, stream);
+    return run_ring<DQ_F32, DQ_PHILOX>(d, mee, mp, stream);
+}
+
+} // namespace dq

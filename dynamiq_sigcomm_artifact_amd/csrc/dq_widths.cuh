@@ -1,0 +1,306 @@
+// Quantise and dequantise a chunk of 16 elements in registers, with the bit width as a value instead of a template
+// parameter: what the kernels need that run compress -> decompress (or a whole chain of ring steps) without a packed
+// stream in between.  Without the packing there is nothing in a chunk's arithmetic that depends on the width but a
+// dozen constants, so one body serves the three widths of the dynamic mix, also where they differ inside a wave.
+//
+// The levels are those of chunk_encode_* followed by chunk_decode (dq_hier16_tiles.cuh), operation by operation; a code
+// travels as the float level it decodes to instead of a bit field.
+#pragma once
+
+#include "dq_hier16_tiles.cuh"
+
+namespace dq {
+
+// 8, 4 and 2 bits, in this order everywhere
+struct WidthConst {
+    double inv_top;            // 1 / R (AEE) or 1 / chunk_max_mee (MEE)
+    double inv_c, inv_l2b;     // MEE
+    float r;                   // R = 2^(bits - 1) - 1
+    float bias, two_delta;     // of the code estimate: R + 1 + kDelta, 2 kDelta (estimate_codes)
+    float c, cmm, l2b;         // MEE
+};
+
+constexpr int kLevels[3] = {0, 256, 272}; // where each width's level table starts
+constexpr int kLevelCount = 276;
+
+struct WidthSet {
+    WidthConst w[3];
+    uint16_t levels[280]; // MEE: binary16 level tables of the three widths end to end
+};
+
+// one width's constants in registers; table: its levels as floats in LDS (MEE)
+template <bool MEE> struct WidthRegs {
+    double inv_top, inv_c, inv_l2b;
+    float r, bias, two_delta, c, cmm, l2b;
+    const float *table;
+};
+
+template <bool MEE> __device__ __forceinline__ WidthRegs<MEE> width_regs(const WidthSet &s, int cls, const float *levels)
+{
+    WidthRegs<MEE> x;
+    const auto pick = [cls](auto a, auto b, auto c) { return cls == 0 ? a : (cls == 1 ? b : c); };
+    x.inv_top = pick(s.w[0].inv_top, s.w[1].inv_top, s.w[2].inv_top);
+    x.r = pick(s.w[0].r, s.w[1].r, s.w[2].r);
+    x.bias = pick(s.w[0].bias, s.w[1].bias, s.w[2].bias);
+    x.two_delta = pick(s.w[0].two_delta, s.w[1].two_delta, s.w[2].two_delta);
+    if (MEE) {
+        x.inv_c = pick(s.w[0].inv_c, s.w[1].inv_c, s.w[2].inv_c);
+        x.inv_l2b = pick(s.w[0].inv_l2b, s.w[1].inv_l2b, s.w[2].inv_l2b);
+        x.c = pick(s.w[0].c, s.w[1].c, s.w[2].c);
+        x.cmm = pick(s.w[0].cmm, s.w[1].cmm, s.w[2].cmm);
+        x.l2b = pick(s.w[0].l2b, s.w[1].l2b, s.w[2].l2b);
+        x.table = levels + pick(kLevels[0], kLevels[1], kLevels[2]);
+    } else {
+        x.inv_c = x.inv_l2b = 0.0;
+        x.c = x.cmm = x.l2b = 0.0f;
+        x.table = nullptr;
+    }
+    return x;
+}
+
+// the three level tables into LDS (kLevelCount floats): the kernel-argument loads of every lane leave together
+__device__ __forceinline__ void levels_to_lds(const WidthSet &s, float *levels, int lane)
+{
+    const uint32_t *pairs = reinterpret_cast<const uint32_t *>(s.levels);
+    uint32_t p[3];
+#pragma unroll
+    for (int k = 0; k < 3; k++) p[k] = lane + 64 * k < kLevelCount / 2 ? pairs[lane + 64 * k] : 0u;
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        const int at = lane + 64 * k;
+        if (at < kLevelCount / 2) {
+            levels[2 * at] = f16_bits_to_f32(p[k] & 0xffffu);
+            levels[2 * at + 1] = f16_bits_to_f32(p[k] >> 16);
+        }
+    }
+}
+
+// the quantiser with every guard of the reference (chunk_encode_guarded): lev[i] = level of element i, returns the
+// chunk's step (chunk_decode's sc)
+template <bool MEE, class RV, class RR>
+__device__ __forceinline__ float quantize_guarded(const RV &v, const RR &rnd, const WidthRegs<MEE> &w, float (&lev)[16])
+{
+    float a = __builtin_fabsf(v.get(0));
+#pragma unroll
+    for (int i = 1; i < 16; i++) a = __builtin_fmaxf(a, __builtin_fabsf(v.get(i)));
+    const float s = pos_scale(MEE ? a / pos_scale(w.cmm) + 1e-7f : a / w.r + 1e-7f);
+    const float g = pos_scale(row16_max(s));
+    const uint32_t unit_bits = f32_to_bf16_bits(pos_scale(g / 255.0f));
+    const float unit = pos_scale(bf16_bits_to_f32(unit_bits));
+    float ratio = pos_scale(s) / pos_scale(g) * 255.0f;
+    if (!__builtin_isfinite(ratio)) ratio = ratio > 0.0f ? 255.0f : 1.0f;
+    const int qi = min(max(sat_u16(__builtin_ceilf(ratio)), 1), 255);
+    const float d = pos_scale(pos_scale((float)qi * unit));
+    const int top = (int)w.r;
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+        float x = v.get(i) / d;
+        if (MEE) x = mee_inverse_guarded(x, w.c, w.l2b);
+        const int code = clamp_code(sr_guarded(x, rnd.get(i)), top);
+        lev[i] = MEE ? w.table[code] : (float)(code - top);
+    }
+    return nonneg_scale((float)qi * nonneg_scale(bf16_bits_to_f32(unit_bits)));
+}
+
+// chunk_encode_fast + estimate_codes: elements finite and <= 2^100, random values in [0, 1]
+template <bool MEE, class RV, class RR>
+__device__ __forceinline__ float quantize_fast(const RV &v, const RR &rnd, uint32_t amax_bits, const WidthRegs<MEE> &w, float (&lev)[16])
+{
+    const float s = div_by(__uint_as_float(amax_bits), w.inv_top) + 1e-7f; // (2 bits: R = 1, the product with 1)
+    const float g = row16_max_pos(s);
+    const float unit = bf16_bits_to_f32(f32_to_bf16_bits(div_by(g, 1.0 / 255.0)));
+    const float ratio = div_by(s, recip_f64(g)) * 255.0f;
+    const int qi = min(max((int)__builtin_ceilf(ratio), 1), 255);
+    const float d = (float)qi * unit;
+    const float rd = __builtin_amdgcn_rcpf(d);
+    const float rc = MEE ? (float)w.inv_c : 0.0f, rl2b = MEE ? (float)w.inv_l2b : 0.0f;
+    const float two_r = w.r + w.r;
+    bool doubt[16];
+    uint64_t lanes_in_doubt[16], any = 0;
+    float code[16];
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+        const float vi = v.get(i);
+        const float off = below(rnd, i, w.bias);
+        float t;
+        if (MEE)
+            t = __builtin_fmaf(__builtin_amdgcn_logf(__builtin_fmaf(__builtin_fabsf(vi * rd), rc, 1.0f)), __builtin_copysignf(rl2b, vi), off);
+        else
+            t = __builtin_fmaf(vi, rd, off);
+        const float fr = __builtin_amdgcn_fractf(t);
+        doubt[i] = fr < w.two_delta;
+        lanes_in_doubt[i] = __builtin_amdgcn_ballot_w64(doubt[i]);
+        any |= lanes_in_doubt[i];
+        // floor(t); -1 < t < 2 R + 2, so the two bounds are the clamp of the code
+        code[i] = __builtin_amdgcn_fmed3f(t - fr, 0.0f, two_r);
+    }
+    if (any != 0) {
+        const double yd = recip_f64(d);
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            if (lanes_in_doubt[i] != 0) {
+                const float sv = (float)exact_code_fast<MEE>(v.get(i), rnd.get(i), d, yd, w);
+                if (doubt[i]) code[i] = __builtin_amdgcn_fmed3f(sv, -w.r, w.r) + w.r;
+            }
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 16; i++) lev[i] = MEE ? w.table[(int)code[i]] : code[i] - w.r;
+    return nonneg_scale((float)qi * nonneg_scale(unit));
+}
+
+// levels and step of the lane's chunk; every lane of the wave must call
+template <bool MEE, class RV, class RR>
+__device__ __forceinline__ float quantize_chunk(const RV &v, const RR &rnd, const WidthRegs<MEE> &w, float (&lev)[16])
+{
+    const uint32_t amax = v.absmax_bits();
+    const bool lane_fast = amax <= kFastMaxBits && rnd.unit_interval();
+    if (__builtin_amdgcn_ballot_w64(!lane_fast) == 0) return quantize_fast<MEE>(v, rnd, amax, w, lev);
+    return quantize_guarded<MEE>(v, rnd, w, lev);
+}
+
+// mp: the MEE parameters of 8, 4 and 2 bits
+inline WidthSet make_width_set(const MeeParams *mp, bool mee)
+{
+    static const int bits[3] = {8, 4, 2};
+    WidthSet s;
+    __builtin_memset(&s, 0, sizeof(s));
+    for (int k = 0; k < 3; k++) {
+        WidthConst &w = s.w[k];
+        const int top = (1 << (bits[k] - 1)) - 1;
+        // EstimateGuard: kDelta of estimate_codes
+        const float delta = mee ? (bits[k] >= 6 ? 0x1p-12f : 0x1p-14f) : (float)(1 << (bits[k] - 1)) * 0x1p-20f;
+        w.r = (float)top;
+        w.bias = (float)(top + 1) + delta;
+        w.two_delta = 2.0f * delta;
+        w.c = mp[k].c; w.cmm = mp[k].cmm; w.l2b = mp[k].l2b;
+        w.inv_top = mee ? 1.0 / (double)mp[k].cmm : 1.0 / (double)top;
+        w.inv_c = 1.0 / (double)mp[k].c;
+        w.inv_l2b = 1.0 / (double)mp[k].l2b;
+        for (int j = 0; mee && j < (1 << bits[k]); j++) s.levels[kLevels[k] + j] = mp[k].table[j];
+    }
+    return s;
+}
+
+// ---- a lane's chunk at the ragged end of a vector ------------------------------------------------------
+
+template <int DT> __device__ __forceinline__ void load_chunk_guarded(Raw16<DT> &v, const void *src, int64_t e0, int64_t n)
+{
+    v.zero();
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+        if (e0 + i < n) {
+            if (DT == DQ_F32)
+                v.w[i] = static_cast<const uint32_t *>(src)[e0 + i];
+            else
+                v.w[i >> 1] |= (uint32_t) static_cast<const uint16_t *>(src)[e0 + i] << (16 * (i & 1));
+        }
+    }
+}
+
+// elements [e0, e0 + 16) of src, zero at and beyond n
+template <int DT> __device__ __forceinline__ void load_chunk(Raw16<DT> &v, const void *src, int64_t e0, int64_t n, bool vec)
+{
+    if (e0 + 16 <= n)
+        v.load(src, e0, vec);
+    else
+        load_chunk_guarded<DT>(v, src, e0, n);
+}
+
+// v becomes T(v / world - mean), zero at and beyond element n of the vector (center_chunk without its own loads)
+template <int DT>
+__device__ __forceinline__ void center_loaded(Raw16<DT> &v, const WorldDiv &wd, float mean, int64_t e0, int64_t n)
+{
+    float t[16];
+    if (DT != DQ_F32 && wd.fuse16) {
+#pragma unroll
+        for (int i = 0; i < 16; i++) t[i] = __builtin_fmaf(v.get(i), wd.inv, -mean);
+    } else if (wd.pow2) {
+#pragma unroll
+        for (int i = 0; i < 16; i++) t[i] = v.get(i) * wd.inv - mean;
+    } else {
+#pragma unroll
+        for (int i = 0; i < 16; i++) t[i] = v.get(i);
+        wd.divide16(t);
+#pragma unroll
+        for (int i = 0; i < 16; i++) t[i] -= mean;
+    }
+    if (e0 + 16 > n) {
+#pragma unroll
+        for (int i = 0; i < 16; i++) t[i] = e0 + i < n ? t[i] : 0.0f;
+    }
+    v.set(t);
+}
+
+// ---- statistics of a tile of four superchunks -----------------------------------------------------------
+
+template <int CTRL> __device__ __forceinline__ float dpp_row_shift(float v)
+{
+    // lanes without a source inside the row receive 0; they only feed partial sums that are never read again
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+
+template <int DT> struct StatsTile {
+    static constexpr int ESZ = DT == DQ_F32 ? 4 : 2;
+    static constexpr int RS = 256 * ESZ + 16 * ESZ; // padded row stride: the four rows use disjoint banks
+    static constexpr int BYTES = 4 * RS;
+};
+
+// Sum and sum of squares of v / world over each superchunk of the wave's tile in the reference's reduction order
+// (csrc/cuda_hadamard.cu:1286-1292: strides 128 ... 1), from the lane's chunk: the elements go through LDS once so that
+// lane (row r, column j) holds elements j + 16 k of superchunk r -- strides 128 .. 16 are then additions in the lane,
+// strides 8 .. 1 row shifts.  lds: StatsTile<DT>::BYTES, 16-byte aligned, owned by this wave.  sum and sq are complete in
+// the lanes j == 0.
+template <int DT>
+__device__ __forceinline__ void tile_sums(const Raw16<DT> &v, const WorldDiv &wd, uint8_t *lds, int lane, float &sum, float &sq)
+{
+    typedef StatsTile<DT> ST;
+    const int row = lane >> 4, j = lane & 15;
+#pragma unroll
+    for (int k = 0; k < Raw16<DT>::kSlots; k++)
+        *reinterpret_cast<uint4 *>(lds + row * ST::RS + j * 16 * ST::ESZ + 16 * k) = v.slot(k);
+    wave_lds_sync();
+    const uint8_t *mine = lds + row * ST::RS + j * ST::ESZ;
+    float t[16];
+#pragma unroll
+    for (int k = 0; k < 16; k++) {
+        if (DT == DQ_F32)
+            t[k] = *reinterpret_cast<const float *>(mine + 16 * k * ST::ESZ);
+        else
+            t[k] = bf16_bits_to_f32(*reinterpret_cast<const uint16_t *>(mine + 16 * k * ST::ESZ));
+    }
+    if (wd.pow2) {
+        if (wd.inv != 1.0f) {
+#pragma unroll
+            for (int k = 0; k < 16; k++) t[k] = t[k] * wd.inv;
+        }
+    } else {
+        wd.divide16(t);
+    }
+    float a[8], b[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        a[k] = t[k] + t[k + 8];
+        b[k] = t[k] * t[k] + t[k + 8] * t[k + 8];
+    }
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        a[k] += a[k + 4];
+        b[k] += b[k + 4];
+    }
+    sum = (a[0] + a[2]) + (a[1] + a[3]);
+    sq = (b[0] + b[2]) + (b[1] + b[3]);
+    sum += dpp_row_shift<0x108>(sum);
+    sq += dpp_row_shift<0x108>(sq);
+    sum += dpp_row_shift<0x104>(sum);
+    sq += dpp_row_shift<0x104>(sq);
+    sum += dpp_row_shift<0x102>(sum);
+    sq += dpp_row_shift<0x102>(sq);
+    sum += dpp_row_shift<0x101>(sum);
+    sq += dpp_row_shift<0x101>(sq);
+}
+
+// the mean the reference divides out: sum / 256 exactly, or by the count of a ragged last superchunk
+__device__ __forceinline__ float superchunk_mean(float sum, int64_t valid) { return valid >= 256 ? sum * 0.00390625f : sum / (float)valid; }
+
+} // namespace dq

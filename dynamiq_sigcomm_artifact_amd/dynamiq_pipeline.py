@@ -20,6 +20,7 @@ from . import load_eden_utils
 from .ring_sim import ring_allreduce, ring_allreduce_rows
 
 SUPERCHUNK = 256
+_U64 = 0xFFFFFFFFFFFFFFFF
 
 
 def dynamic_bitrate_allreduce(rank_vecs, u, compressors, out=None):
@@ -201,15 +202,15 @@ def fixed_proportion_allreduce_grouped(rank_vecs, thresholds, compressors, out=N
 
 def dynamic_bitrate_allreduce_single_pass(rank_vecs, u, strategy=2, seed=0, out=None, work=None, stream=None,
                                           norm_histogram=None):
-    """The same all-reduce with every stage kept on the device: no residual buffers (the centring is folded
-    into the codec's loads), no group tensors, no per-width launches and no read-back of the group sizes --
-    a fixed sequence of launches per bucket (statistics, plan, and one codec launch per ring step for all
-    three bit widths), which can be captured once and replayed as a graph.
+    """The same all-reduce with every stage kept on the device and without packed streams: the records of a ring step
+    between ranks that share this GPU's memory are read by the next step only, so a superchunk goes through the whole
+    ring in registers (csrc/dq_single_pass.hip).  Three launches per bucket (statistics of all ranks, plan, ring) -- two
+    with one rank, where nothing depends on another superchunk -- whatever the number of ranks; nothing is read back, and
+    the launches can be captured once and replayed as a graph.
 
-    Per rank: superchunk_stats -> (stats sum) -> group_plan_stats -> ring over mixed_compress /
-    mixed_decompress.  The bit widths follow the device rule of group_plan_stats; the rounding randomness is
-    the in-kernel stream keyed by (seed + rank, ring step, index of the chunk in the vector), so results are
-    reproducible but not those of dynamic_bitrate_allreduce, whose random values come from the pool.
+    The bit widths follow the device rule of group_plan_stats; the rounding randomness is the in-kernel stream keyed by
+    (seed + rank, ring step, index of the chunk in the vector), so results are reproducible but not those of
+    dynamic_bitrate_allreduce, whose random values come from the pool.
 
     u: the offset of the width rule, a number or a float64 device tensor (e.g. result[0:1] of the offset search: then
     nothing of the step is read back).
@@ -220,11 +221,45 @@ def dynamic_bitrate_allreduce_single_pass(rank_vecs, u, strategy=2, seed=0, out=
     from . import capi
     W = len(rank_vecs)
     n = rank_vecs[0].numel()
-    nsc = (n + SUPERCHUNK - 1) // SUPERCHUNK
     dev, dt = rank_vecs[0].device, rank_vecs[0].dtype
     if work is None:
         work = {}
+    if W > capi.ranks_max():
+        return _single_pass_in_steps(rank_vecs, u, strategy, seed, out, work, stream, norm_histogram)
+    nsc = (n + SUPERCHUNK - 1) // SUPERCHUNK
     key = ("single_pass", nsc, dt, W)
+    if work.get("key") != key:
+        work.clear()
+        work["key"] = key
+        work["total"] = torch.empty((nsc, 2), dtype=torch.bfloat16, device=dev)
+        work["plan"] = torch.zeros(capi.group_plan_work_ints(nsc) if W > 1 else 4, dtype=torch.int32, device=dev)
+        work["counts"] = work["plan"][:4]
+        if W > 1:
+            work["mean"] = torch.empty(W * nsc, dtype=torch.float32, device=dev)
+            work["order"] = torch.empty(3 * nsc, dtype=torch.int32, device=dev)
+    outs = out if out is not None else [torch.empty(n, dtype=dt, device=dev) for _ in range(W)]
+    hist = None
+    if norm_histogram is not None:
+        hist = norm_histogram.hist
+        norm_histogram.count += nsc
+    total = work["total"]
+    if W == 1:
+        capi.host().roundtrip(rank_vecs[0], outs[0], n, total, work["counts"], u, hist, seed & _U64, strategy, stream)
+    else:
+        capi.host().ranks_dynamic(rank_vecs, outs, n, total, work["mean"], work["order"], work["plan"], u, hist, seed & _U64,
+                                  strategy, stream)
+    return outs, total, work["counts"]
+
+
+def _single_pass_in_steps(rank_vecs, u, strategy, seed, out, work, stream, norm_histogram):
+    """the same with one launch per rank and ring step and the packed streams in memory: for more simulated ranks than the
+    arguments of one launch hold"""
+    from . import capi
+    W = len(rank_vecs)
+    n = rank_vecs[0].numel()
+    nsc = (n + SUPERCHUNK - 1) // SUPERCHUNK
+    dev, dt = rank_vecs[0].device, rank_vecs[0].dtype
+    key = ("single_pass in steps", nsc, dt, W)
     if work.get("key") != key:
         work.clear()
         work["key"] = key
@@ -235,7 +270,7 @@ def dynamic_bitrate_allreduce_single_pass(rank_vecs, u, strategy=2, seed=0, out=
         work["order"] = torch.empty(3 * nsc, dtype=torch.int32, device=dev)
         work["plan"] = torch.zeros(capi.group_plan_work_ints(nsc), dtype=torch.int32, device=dev)
         work["send"] = [torch.zeros(cap, dtype=torch.uint8, device=dev) for _ in range(W)]
-        work["recv"] = [torch.zeros(cap, dtype=torch.uint8, device=dev) for _ in range(W if W > 1 else 0)]
+        work["recv"] = [torch.zeros(cap, dtype=torch.uint8, device=dev) for _ in range(W)]
     stats, mean, order, plan = work["stats"], work["mean"], work["order"], work["plan"]
     send, recv = work["send"], work["recv"]
     # one stream for the kernels and for the torch ops between them (the statistics sum, the exchange copies):
@@ -244,14 +279,11 @@ def dynamic_bitrate_allreduce_single_pass(rank_vecs, u, strategy=2, seed=0, out=
     stream = torch_stream.cuda_stream
     for r in range(W):
         capi.superchunk_stats(rank_vecs[r], stats[r], mean[r], n, W, stream=stream)
-    if W == 1:
-        total = stats[0]
-    else:
-        total = work["total"]
-        with torch.cuda.stream(torch_stream):
-            total.copy_(stats[0])
-            for r in range(1, W):
-                total.add_(stats[r])
+    total = work["total"]
+    with torch.cuda.stream(torch_stream):
+        total.copy_(stats[0])
+        for r in range(1, W):
+            total.add_(stats[r])
     # with u on the device the histogram is filled by a few more workgroups of the plan launch, otherwise by a launch of its own
     capi.group_plan_stats(total, u if isinstance(u, torch.Tensor) else float(u), None, order, plan, stream=stream,
                           hist=None if norm_histogram is None else norm_histogram.hist)
@@ -266,11 +298,6 @@ def dynamic_bitrate_allreduce_single_pass(rank_vecs, u, strategy=2, seed=0, out=
     def decode(r, packed, chunk):
         capi.mixed_decompress(packed, outs[r], order, plan, nsc, strategy, stats=total, n_limit=n, ring_chunk=chunk,
                               ring_world=W, stream=stream)
-
-    if W == 1:
-        encode(0, 0, 0)
-        decode(0, send[0], 0)
-        return outs, total, plan[:4]
 
     def exchange(src_bufs, dst_bufs):
         with torch.cuda.stream(torch_stream):
@@ -322,27 +349,24 @@ def pick_streams(device, want, tries=16):
 
 class SinglePassBuckets(object):
     """The single-pass dynamic-bitrate path for a stream of buckets on one rank (a ring of one: statistics, widths,
-    partition, encode, decode, mean add -- what dynamic_bitrate_allreduce_single_pass does for W = 1), shaped for
-    25 MB buckets, where the four kernels of a bucket take about as long as four host calls and every launch waits
-    for the one before:
+    encode, decode, mean add -- what dynamic_bitrate_allreduce_single_pass does for W = 1).  A superchunk's result depends
+    on no other superchunk, so one launch makes one pass over the bucket, and over as many buckets as are at hand:
 
-      * one host call per bucket (capi.dynamic_bitrate_bucket) instead of four (``run``);
-      * eager buckets of the first of the ``streams`` slots run on the caller's own stream (``inline_first``): handing a
-        bucket to another stream costs an event record, a wait and a dearer first launch behind it -- measured 17 us of
-        host time against 13 us for the four kernels themselves;
-      * ``streams`` buckets are in flight at a time, each on a stream of its own with scratch of its own (statistics,
-        means, plan, packed stream): the latency-bound statistics and plan launches of one bucket overlap the codec
-        launches of its neighbour.  The streams are chosen so that they do run side by side (``pick_streams``);
-      * with ``graphs=True``, ``run_all`` records a whole step's buckets once -- one graph per stream -- and replays
-        them: one graph launch per stream and step instead of one host call per bucket.  DDP hands the hook the same
-        bucket views on every step, so the list of (source, output) pairs is the natural key; a replay reads whatever
-        the sources hold then.  (A graph per bucket was measured and is slower than the eager call: launching a graph
-        costs the host more than one call that enqueues four kernels.)
+      * ``run(x, out)`` enqueues one bucket: two launches, the pass and the tally of its widths (and norms);
+      * ``run_all`` enqueues a whole step's buckets, two launches for every 32 of them.  DDP hands the hook the same
+        bucket views on every step: the list is laid out once and recognised afterwards.
 
-    The offset u of the width rule is read from device memory when the plan runs (``set_u`` or a float64 tensor of the
+    Everything runs on the caller's current stream: a launch that fills the GPU gains nothing from a second stream beside
+    it, and handing a bucket to another stream costs the host more than enqueueing it.  ``streams`` says how many slots
+    run() deals the buckets out to (the index it returns, and counts() takes); the streams of that many slots
+    (``pipe.streams``, found on first use to run side by side with the caller's, see pick_streams) are at the caller's
+    disposal.  ``graphs`` and ``inline_first`` are accepted and change nothing: there is no longer a host cost per bucket
+    that a recorded graph would save.
+
+    The offset u of the width rule is read from device memory when a launch runs (``set_u`` or a float64 tensor of the
     caller's, e.g. the result of the offset search), and the rounding stream of the encoder is (seed, bucket ordinal *
-    2^32 + the step counter in device memory, one copy per stream): ``begin_step`` advances the counters once per
-    training step, so a replayed launch draws fresh random values on every step.
+    2^32 + the step counter in device memory): ``begin_step`` once per training step makes the next launch advance the
+    counter, so a replayed launch draws fresh random values on every step.
 
     run(x, out) enqueues a bucket and returns at once; join() makes the caller's current stream wait for everything
     enqueued so far.  The caller must not overwrite x or read out before join()."""
@@ -352,185 +376,106 @@ class SinglePassBuckets(object):
         self.capi = capi
         self.device = torch.device(device)
         self.strategy, self.seed, self.graphs, self.inline_first = strategy, int(seed), graphs, bool(inline_first)
-        self.streams, self.side_by_side = pick_streams(self.device, max(1, int(streams)))
-        self.scratch = [dict() for _ in self.streams]
-        self.pending = [False] * len(self.streams)
-        # one step counter per stream, advanced on that stream: no hand-over between streams at a step boundary
-        self.step_devs = [torch.zeros(1, dtype=torch.int64, device=self.device) for _ in self.streams]
+        self.slots = max(1, int(streams))
+        self.step_dev = torch.zeros(1, dtype=torch.int64, device=self.device)
         self.u_dev = u if isinstance(u, torch.Tensor) else torch.full((1,), 60.0 if u is None else float(u), dtype=torch.float64,
                                                                      device=self.device)
         self.hist = norm_histogram
-        ready = torch.cuda.Event()
-        ready.record(torch.cuda.current_stream(self.device))
-        for st in self.streams:
-            st.wait_event(ready)         # the counters and u are initialised on the caller's stream
-        self.cache = {}          # (x.data_ptr(), out.data_ptr(), n, dtype) -> _entry(); ("step", keys) -> [graphs, uses]
-        self._enqueue = capi.lib().dq_dynamic_bitrate_bucket
-        self._order = capi.lib().dq_stream_order_after
+        self._host = capi.host()
+        self._buckets = self._host.Buckets(strategy, self.seed & _U64, self.step_dev, self.u_dev,
+                                           None if norm_histogram is None else norm_histogram.hist)
+        self._room = (0, 0)
+        self._stats = self._counts = None
+        self._last = None        # the list run_all saw last: (batch, superchunks)
+        self.cache = {}          # addresses and sizes of a list of buckets -> (batch, superchunks, slots)
         self.ordinals = {}       # (x.data_ptr(), n) -> ordinal of the bucket in the random stream
+        self._rows = {}          # slot -> row of the counts of its last bucket
         self.superchunks = 0
+
+    def _pick(self):
+        if "_streams" not in self.__dict__:
+            self._streams, self._side_by_side = pick_streams(self.device, self.slots)
+
+    @property
+    def streams(self):
+        self._pick()
+        return self._streams
+
+    @property
+    def side_by_side(self):
+        self._pick()
+        return self._side_by_side
 
     # ---- once per training step ----------------------------------------------------------------------------
     def set_u(self, u):
         """the offset of the width rule for the buckets enqueued from now on (a number; a tensor was given at construction)"""
-        cur = torch.cuda.current_stream(self.device)
-        for k, st in enumerate(self.streams):
-            if self.pending[k]:
-                cur.wait_stream(st)
+        self.join()
         self.u_dev.fill_(float(u))
-        self._fence = torch.cuda.Event()
-        self._fence.record(cur)
-        for st in self.streams:
-            st.wait_event(self._fence)
 
     def begin_step(self):
-        """advance the step counter of the rounding stream: one small kernel per stream and training step, enqueued on
-        that stream, so it is ordered with the stream's buckets and nothing waits for another stream"""
-        for k, (st, counter) in enumerate(zip(self.streams, self.step_devs)):
-            if k == 0 and self.inline_first:
-                # slot 0 runs on the caller's stream when eager and on its worker stream when recorded: its counter is
-                # advanced on the caller's stream, after whatever the worker stream still has of the previous step (a
-                # recorded step orders the worker streams after the caller's before it starts)
-                if self.pending[0]:
-                    cur = torch.cuda.current_stream(self.device)
-                    cur.wait_stream(st)
-                    self.pending[0] = False
-                counter.add_(1)
-            else:
-                with torch.cuda.stream(st):
-                    counter.add_(1)
+        """advance the step counter of the rounding stream: the next launch does it on its way"""
+        self._buckets.begin_step()
 
     # ---- per bucket ---------------------------------------------------------------------------------------------
-    def _scratch(self, k, nsc):
-        sc = self.scratch[k]
-        if sc.get("nsc", 0) < nsc:
-            capi, dev = self.capi, self.device
-            sc["nsc"] = nsc
-            sc["stats"] = torch.empty((nsc, 2), dtype=torch.bfloat16, device=dev)
-            sc["mean"] = torch.empty(nsc, dtype=torch.float32, device=dev)
-            sc["order"] = torch.empty(3 * nsc, dtype=torch.int32, device=dev)
-            sc["work"] = torch.zeros(capi.group_plan_work_ints(nsc), dtype=torch.int32, device=dev)
-            sc["packed"] = torch.zeros(capi.mixed_required_bytes(nsc, 1), dtype=torch.uint8, device=dev)
-            for name in ("stats", "mean", "order", "work", "packed"):
-                sc[name].record_stream(self.streams[k])     # allocated on the caller's stream, used on this one
-            # scratch of another size invalidates what was recorded against the old buffers
-            for key in [key for key, entry in self.cache.items() if key[0] == "step" or entry[3] == k]:
-                del self.cache[key]
-        return sc
-
-    def _entry(self, x, out, n, key):
-        """descriptor of a bucket seen for the first time (or again after its stream's scratch grew)"""
-        import ctypes
-        capi = self.capi
-        nsc = (n + 255) // 256
-        # a source keeps its ordinal, and with it its stream and its recorded launches, from step to step
-        ordinal = self.ordinals.setdefault((key[0], n), len(self.ordinals))
-        k = ordinal % len(self.streams)
-        sc = self._scratch(k, nsc)
-        desc, dev = capi.bucket_descriptor(x, n, sc["stats"][:nsc], sc["mean"], sc["order"], sc["work"], sc["packed"],
-                                           strategy=self.strategy, out=out, u=self.u_dev,
-                                           hist=None if self.hist is None else self.hist.hist, seed=self.seed,
-                                           step=ordinal << 32, step_dev=self.step_devs[k])
-        # (descriptor, its reference for the call, device, stream index, superchunks, the stream's handle)
-        entry = (desc, ctypes.byref(desc), dev, k, nsc, ctypes.c_void_p(self.streams[k].cuda_stream))
-        self.cache[key] = entry
+    def _batch(self, pairs, key, one):
+        """lays out a list of buckets seen for the first time (or again after the scratch grew).  The counts of a bucket of
+        run() have the row of its slot, those of a list the rows behind."""
+        sizes = [(x.numel() + SUPERCHUNK - 1) // SUPERCHUNK for x, _ in pairs]
+        total = sum(sizes)
+        rows = self.slots + (0 if one else len(pairs))
+        if total > self._room[0] or rows > self._room[1]:
+            self.join()
+            self._room = (max(total, self._room[0]), max(rows, self._room[1]))
+            self._stats = torch.empty((self._room[0], 2), dtype=torch.bfloat16, device=self.device)
+            counts = torch.zeros((self._room[1], 4), dtype=torch.int32, device=self.device)
+            if self._counts is not None:
+                counts[:self._counts.shape[0]].copy_(self._counts)
+            self._counts = counts
+            self._buckets.scratch(self._stats, self._counts)
+            self.cache.clear()       # what was laid out over the old buffers
+            self._last = None
+        # a source keeps its ordinal, and with it its random stream and its slot, from step to step
+        ordinals = [self.ordinals.setdefault((x.data_ptr(), x.numel()), len(self.ordinals)) for x, _ in pairs]
+        slots = [o % self.slots for o in ordinals]
+        rows = slots if one else range(self.slots, self.slots + len(pairs))
+        batch = self._host.Batch(self._buckets, pairs, [(o << 32) & _U64 for o in ordinals], list(rows))
+        entry = self.cache[key] = (batch, total, dict(zip(slots, rows)))
         return entry
 
+    def _enqueue(self, entry):
+        batch, superchunks, rows = entry
+        batch.launch(self._buckets)
+        self._rows.update(rows)
+        if self.hist is not None:
+            self.hist.count += superchunks
+        self.superchunks += superchunks
+
     def run(self, x, out):
-        """enqueue one bucket: out = decode(encode(x)) with the widths of its reduced norms; returns the index of the
-        stream it went to.  The hot path of an eager caller: two library calls (order the worker stream after the
-        caller's, enqueue the bucket's four kernels) and one dictionary look-up."""
-        n = x.numel()
-        key = (x.data_ptr(), out.data_ptr(), n, x.dtype)
+        """enqueue one bucket: out = decode(encode(x)) with the widths of its reduced norms; returns its slot"""
+        key = (x.data_ptr(), out.data_ptr(), x.numel(), x.dtype)
         entry = self.cache.get(key)
         if entry is None:
-            entry = self._entry(x, out, n, key)
-        _, ref, dev, k, nsc, handle = entry
-        cur = torch.cuda.current_stream(self.device).cuda_stream
-        if k == 0 and self.inline_first:
-            # the first bucket of every round of `streams` goes to the caller's own stream: nothing to order, and ordering a
-            # worker stream after the caller's costs the host more than enqueueing the bucket's four kernels does
-            if self.pending[0]:                 # (a recorded step ran on the worker stream of this slot)
-                if self._order(cur, self.streams[0].cuda_stream, dev):
-                    raise RuntimeError(self.capi.lib().dq_last_error().decode())
-                self.pending[0] = False
-            if self._enqueue(ref, 15, dev, cur):
-                raise RuntimeError(self.capi.lib().dq_last_error().decode())
-        else:
-            if self._order(handle, cur, dev) or self._enqueue(ref, 15, dev, handle):
-                raise RuntimeError(self.capi.lib().dq_last_error().decode())
-            self.pending[k] = True
-        if self.hist is not None:
-            self.hist.count += nsc
-        self.superchunks += nsc
-        return k
+            entry = self._batch([(x, out)], key, True)
+        self._enqueue(entry)
+        return next(iter(entry[2]))
 
     def run_all(self, pairs):
-        """enqueue a whole step's buckets, [(x, out), ...].  A list that has been seen before (the same tensors in the
-        same order: DDP's buckets) is replayed from one recorded graph per stream -- one graph launch per stream and
-        step instead of one host call per bucket; the first time it runs bucket by bucket, the second time it records."""
-        key = tuple((x.data_ptr(), o.data_ptr(), x.numel(), x.dtype) for x, o in pairs)
-        entry = self.cache.get(("step", key))
-        cur = torch.cuda.current_stream(self.device)
-        if entry is None or not self.graphs:
-            for x, o in pairs:
-                self.run(x, o)
-            if entry is None:
-                self.cache[("step", key)] = [None, 1]
-            return
-        graphs, uses = entry
-        if graphs is None:
-            # per stream: the buckets that go to it, in order, recorded as one graph
-            share = [[] for _ in self.streams]
-            for (x, o), bkey in zip(pairs, key):
-                item = self.cache.get(bkey)
-                if item is None:                # (cannot happen after a first eager pass with unchanged scratch)
-                    self.run(x, o)
-                    item = self.cache[bkey]
-                share[item[3]].append(item)
-            self.join()
-            graphs = []
-            for k, st in enumerate(self.streams):
-                if not share[k]:
-                    graphs.append(None)
-                    continue
-                g = torch.cuda.CUDAGraph()
-                with torch.cuda.stream(st):
-                    with torch.cuda.graph(g, stream=st):
-                        for item in share[k]:
-                            if self._enqueue(item[1], 15, item[2], item[5]):
-                                raise RuntimeError(self.capi.lib().dq_last_error().decode())
-                graphs.append(g)
-            entry[0] = graphs
-        # one event for all streams, recorded before the first replay: an event recorded on the caller's stream between
-        # two replays could complete only after the first of them (see pick_streams)
-        fence = torch.cuda.Event()
-        fence.record(cur)
-        for k, st in enumerate(self.streams):
-            if graphs[k] is not None:
-                st.wait_event(fence)
-        for k, st in enumerate(self.streams):
-            if graphs[k] is None:
-                continue
-            with torch.cuda.stream(st):
-                graphs[k].replay()
-            self.pending[k] = True
-        entry[1] = uses + 1
-        total = sum((x.numel() + 255) // 256 for x, _ in pairs)
-        if self.hist is not None:
-            self.hist.count += total
-        self.superchunks += total
+        """enqueue a whole step's buckets, [(x, out), ...]"""
+        last = self._last
+        if last is None or not last[0].matches(pairs):
+            if not pairs:
+                return
+            key = tuple((x.data_ptr(), o.data_ptr(), x.numel(), x.dtype) for x, o in pairs)
+            last = self.cache.get(key)
+            if last is None:
+                last = self._batch(pairs, key, False)
+            self._last = last
+        self._enqueue(last)
 
     def counts(self, k):
-        """device int32 tensor [n8, n4, n2, other] of the last bucket that ran on stream k"""
-        return self.scratch[k]["work"][:4]
+        """device int32 tensor [n8, n4, n2, other] of the last bucket of slot k"""
+        return self._counts[self._rows[k]]
 
     def join(self):
         """the caller's current stream waits for everything enqueued so far"""
-        cur = torch.cuda.current_stream(self.device).cuda_stream
-        index = self.device.index if self.device.index is not None else torch.cuda.current_device()
-        for k, st in enumerate(self.streams):
-            if self.pending[k]:
-                if self._order(cur, st.cuda_stream, index):
-                    raise RuntimeError(self.capi.lib().dq_last_error().decode())
-                self.pending[k] = False
+        self._buckets.join()

@@ -375,6 +375,74 @@ typedef struct dq_bucket {
 
 int dq_dynamic_bitrate_bucket(const dq_bucket_t *bucket, int stages, int device, dq_stream_t stream);
 
+/* ---- ranks that share one GPU's memory: no packed stream -------------------
+ *
+ * In a ring of one rank, or of several ranks simulated in one GPU's memory, the
+ * records of a ring step are read by the next step and by nobody else.  These
+ * calls run the whole way of a superchunk through the ring in registers; their
+ * results are bit for bit those of the calls above chained.
+ *
+ * dq_bucket_roundtrip: dq_dynamic_bitrate_bucket with all four stages and
+ * ring_world 1 for `count` buckets, two launches for every 32 of them.  Bucket
+ * k draws its rounding randomness from (seed, buckets[k].step); with step_dev
+ * (may be NULL) *step_dev + step_more is added to that, and the call leaves
+ * *step_dev + step_more in *step_dev -- a caller that passes step_more = 1 with
+ * the first buckets of a training step advances the counter without a launch of
+ * its own.  hist (may be NULL, else dq_bitrate_hist_ints() entries): the norm
+ * patterns are added to it. */
+typedef struct dq_roundtrip {
+    const void *src;  /* n elements of dtype (DQ_BF16 or DQ_F32) */
+    void *out;        /* n elements of dtype, written */
+    void *stats;      /* bf16 [nsc, 2], 4-byte aligned, written: mean, sum of squares */
+    int32_t *counts;  /* int32 [4], written: superchunks of 8, 4, 2 bits, 0 */
+    int64_t n;
+    uint64_t step;
+} dq_roundtrip_t;
+
+int dq_bucket_roundtrip(const dq_roundtrip_t *buckets, int count, int dtype, int strategy, int center_world, double u,
+                        const double *u_dev, uint64_t seed, uint64_t *step_dev, uint64_t step_more, uint32_t *hist,
+                        int64_t hist_ints, int device, dq_stream_t stream);
+
+/* dq_ranks_allreduce: one bucket of an all-reduce over `world` simulated ranks
+ * (world <= dq_ranks_max(pooled)), any run of the stages:
+ *   DQ_RANKS_STATS  src -> mean, total: what dq_superchunk_stats (center_world =
+ *                   world) gives per rank, the statistics summed in rank order
+ *                   in bf16 (the reference's all-reduce of them)
+ *   DQ_RANKS_PLAN   total -> order, work: dq_group_plan_stats with u or *u_dev
+ *                   (+ hist), or, with sorted_plan, dq_group_plan_sorted with
+ *                   top_count and bottom_count
+ *   DQ_RANKS_RING   the compressed ring (ring_rdma.py:590-631) over the three
+ *                   groups, its result with the mean of `total` in every out[r].
+ * Rounding randomness: the in-kernel stream, rank r in ring step s drawing from
+ * (seed + r, s, chunk index); or with pool != NULL rank r's random values of
+ * step s for the group of width index g (0: 8 bits, 1: 4, 2: 2) are the rows
+ * first[(g * world + r) * world + s] onwards of pool[g * world + r], 16 values
+ * of dtype per row, one row per chunk of the rank's list of superchunks. */
+enum { DQ_RANKS_STATS = 1, DQ_RANKS_PLAN = 2, DQ_RANKS_RING = 4 };
+
+typedef struct dq_ranks {
+    const void *const *src;     /* world pointers to n elements of dtype (DQ_BF16 or DQ_F32) */
+    void *const *out;           /* likewise, written by RING */
+    int64_t n;
+    int32_t world, dtype, strategy, sorted_plan;
+    void *total;                /* bf16 [nsc, 2], 4-byte aligned */
+    float *mean;                /* float [world, nsc] */
+    int32_t *order;             /* int32 [3 nsc] */
+    int32_t *work;              /* int32 [work_ints]: dq_group_plan_work_ints / dq_group_plan_sorted_work_ints (nsc) */
+    int64_t work_ints;
+    double u;
+    const double *u_dev;        /* may be NULL */
+    uint32_t *hist;             /* may be NULL */
+    int64_t hist_ints;
+    int64_t top_count, bottom_count;
+    uint64_t seed;
+    const void *const *pool;    /* may be NULL */
+    const int32_t *first;
+} dq_ranks_t;
+
+int dq_ranks_max(int pooled);
+int dq_ranks_allreduce(const dq_ranks_t *ranks, int stages, int device, dq_stream_t stream);
+
 /* No counterpart in the reference (its hooks run every bucket on one stream).
  * A caller that keeps several buckets in flight, each on a stream of its own,
  * gains from it only when the streams run side by side: the runtime maps the

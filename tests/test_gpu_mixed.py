@@ -654,3 +654,33 @@ def test_single_pass_buckets_alternating_between_recorded_and_eager_steps(capi, 
             x = x_then[step - 1][k]
             want = _four_calls(capi, x, x.numel(), us[step - 1], 2, seed, (k << 32) + step)[5]
             assert torch.equal(bits_t(o_then[step - 1][k]), bits_t(want)), (step, mode, k)
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("W,n", [(1, 256), (1, 255), (1, 256 * 9 - 3), (2, 256 * 8), (3, 256 * 37 + 1), (8, 1), (8, 256 * 70 - 255), (16, 256 * 201)])
+def test_ranks_in_registers_equal_the_ring_in_steps(capi, W, n, dt):
+    """the all-reduce without packed streams at the edges of its tiles, runs and ring chunks, on unaligned vectors too and with
+    every guard of the quantiser firing, against one launch per rank and ring step: same bits, same counts, same statistics"""
+    from dynamiq_sigcomm_artifact_amd.bitrate import NormHistogram
+    from dynamiq_sigcomm_artifact_amd.dynamiq_pipeline import _single_pass_in_steps, dynamic_bitrate_allreduce_single_pass
+    nsc = (n + 255) // 256
+    for strategy, shift, u in ((2, 0, 6.0), (3, 1, 6.5)):
+        g = torch.Generator().manual_seed(n + W + strategy)
+        scales = torch.exp(torch.randn(nsc, 1, generator=g) * 6.0) * 1e-3
+        vecs = []
+        for r in range(W):
+            v = torch.zeros(n + shift, dtype=dt, device=DEV)
+            v[shift:].copy_(((torch.randn(nsc, 256, generator=g) * scales).reshape(-1)[:n] + 1e-4).to(dt))
+            if r == W - 1 and n > 3000:
+                v[shift + 5], v[shift + 700], v[shift + 1500:shift + 1756] = float("nan"), float("inf"), 0.0
+            vecs.append(v[shift:])
+        a, b = NormHistogram(DEV), NormHistogram(DEV)
+        outs, total, counts = dynamic_bitrate_allreduce_single_pass(vecs, u, strategy=strategy, seed=11, norm_histogram=a)
+        ref, total2, counts2 = _single_pass_in_steps(vecs, u, strategy, 11, None, {}, None, b)
+        assert counts.tolist() == counts2.tolist()
+        assert torch.equal(bits_t(total), bits_t(total2)) and torch.equal(a.hist, b.hist) and a.count == b.count
+        for r in range(W):
+            assert torch.equal(bits_t(outs[r]), bits_t(ref[r])), (strategy, r)
+        u_dev = torch.full((1,), u, dtype=torch.float64, device=DEV)
+        again, _, _ = dynamic_bitrate_allreduce_single_pass(vecs, u_dev, strategy=strategy, seed=11)
+        assert all(torch.equal(bits_t(x), bits_t(y)) for x, y in zip(again, ref))
