@@ -1,9 +1,12 @@
-"""ctypes binding of the C ABI (``include/dynamiq_eden.h``) for torch tensors.
+"""Binding of the C ABI (``include/dynamiq_eden.h``) for torch tensors.
 
 Thin and explicit on purpose: each wrapper passes ``data_ptr()``, sizes, the
 device index and a stream handle straight to ``libdynamiq_eden.so`` and raises
 ``RuntimeError`` with the library's message when the status is non-zero.  The
-library must be present; there is no fallback path.
+codec calls that sit in a training loop go through the native ``_host`` module
+(a call through ctypes costs 8 us of host time, more than the kernel of a 25 MB
+bucket); set-up, plan and measurement calls go through ctypes.  Both libraries
+must be present; there is no fallback path.
 """
 import ctypes
 import importlib
@@ -309,18 +312,15 @@ def mee_lookup_table(nbits):
 
 
 def scaling_compress(src, dst, rand_pool, n, nbits, chunk_size, strategy, stream=None):
-    _call(lib().dq_scaling_compress, _p(src), _p(dst), _p(rand_pool), n, nbits, chunk_size,
-                                     _pair_code(src, rand_pool), _dev(src), strategy, _stream(stream))
+    (_host or host()).scaling_compress(src, dst, rand_pool, n, nbits, chunk_size, strategy, stream)
 
 
 def scaling_decompress(src, dst, n, nbits, chunk_size, strategy, add=False, stream=None):
-    _call(lib().dq_scaling_decompress, _p(src), _p(dst), n, nbits, chunk_size, dtype_code(dst), _dev(dst),
-                                       strategy, _stream(stream), 1 if add else 0)
+    (_host or host()).scaling_decompress(src, dst, n, nbits, chunk_size, strategy, add, stream)
 
 
 def scaling_dec_comp(recv, inp, send, rand_pool, n, nbits, chunk_size, strategy, stream=None):
-    _call(lib().dq_scaling_dec_comp, _p(recv), _p(inp), _p(send), _p(rand_pool), n, nbits,
-                                     chunk_size, _pair_code(inp, rand_pool), _dev(inp), strategy, _stream(stream))
+    (_host or host()).scaling_dec_comp(recv, inp, send, rand_pool, n, nbits, chunk_size, strategy, stream)
 
 
 def group_plan_work_ints(nsc):
@@ -606,14 +606,7 @@ def rht_scaling_compress(src, sign, dst, block, scale, nbits, strategy, rand_poo
     """rht_blocked (forward) + scaling_compress of the rotated fp32 vector in one launch; src is not modified.
     sign: None, float32 +-1 values, or the int32 bit vector of pack_signs.
     rand_pool: float32 or bfloat16 [n], or None for the in-kernel rounding stream keyed by (seed, step, chunk)"""
-    if src.dtype != torch.float32:
-        raise RuntimeError("rht_scaling_compress: src must be float32")
-    code = 0
-    if rand_pool is not None:
-        code = dtype_code(rand_pool)
-    _call(lib().dq_rht_scaling_compress, _p(src), _ptr(sign), _packed(sign), _p(dst), _ptr(rand_pool), code, src.numel(),
-                                         block, float(scale), nbits, _dev(src), strategy, int(seed), int(step),
-                                         _stream(stream))
+    (_host or host()).rht_scaling_compress(src, sign, dst, block, scale, nbits, strategy, rand_pool, seed, step, stream)
 
 
 def rht_scaling_compress_mfma16(src, sign, dst, block, scale, seed=0, step=0, stream=None):
@@ -628,10 +621,7 @@ def rht_scaling_compress_mfma16(src, sign, dst, block, scale, seed=0, step=0, st
 
 def scaling_decompress_irht(src, sign, dst, block, scale, nbits, strategy, stream=None):
     """scaling_decompress into float32 + rht_blocked (inverse) in one launch"""
-    if dst.dtype != torch.float32:
-        raise RuntimeError("scaling_decompress_irht: dst must be float32")
-    _call(lib().dq_scaling_decompress_irht, _p(src), _ptr(sign), _packed(sign), _p(dst), dst.numel(), block, float(scale),
-                                            nbits, _dev(dst), strategy, _stream(stream))
+    (_host or host()).scaling_decompress_irht(src, sign, dst, block, scale, nbits, strategy, stream)
 
 
 def rand_diag(out, seed, stream=None):

@@ -11,7 +11,7 @@ without gathering it first.
 """
 import torch
 
-from . import load_eden_utils
+from . import capi, load_eden_utils
 
 _U32 = 0xFFFFFFFF
 _SUPERGROUP = 16                      # chunks per superchunk
@@ -37,15 +37,7 @@ class _DynamicRangeGPUKern(object):
     given_pool_dtype = None           # dtype a pool passed in params["rand_pool_tensor"] is kept in (None: its own)
 
     def __init__(self, nbits, chunk_size, params, device="cuda", generator=None):
-        eu = self.eden_utils = load_eden_utils()
-        # the reference module takes 2/4/8-bit codes and fp16/bf16 buffers; other widths and fp32 buffers go through
-        # the *_ex entry points, on request only
-        suffix = "_ex" if params.get("extended", False) or nbits not in (2, 4, 8) else ""
-        self._compress = getattr(eu, "scaling_compress" + suffix)
-        self._decompress = getattr(eu, "scaling_decompress" + suffix)
-        self._decompress_add = getattr(eu, "scaling_decompress_add" + suffix)
-        self._dec_comp = getattr(eu, "scaling_dec_comp" + suffix)
-
+        self.eden_utils = load_eden_utils()
         self.nbits, self.chunk_size, self.params, self.device = nbits, chunk_size, params, device
         self.supergroup = _SUPERGROUP
         self.range = (1 << (nbits - 1)) - 1
@@ -55,14 +47,15 @@ class _DynamicRangeGPUKern(object):
         # pool rows: three times the chunks of the longest vector, shared out over the ranks (:384-386)
         self.cur_max_size = max([(d + chunk_size) // chunk_size for d in params["d"].values()] + [0])
         self.three_times_cur_max_size = 3 * self.cur_max_size // self.nclients
-        self.rand_seed = (nbits * 998244353) & _U32
-
+        # the calls of the ring schedules, the LCG and the pools are the native object's: a call is 3 us of GPU time.
+        # The reference module takes 2/4/8-bit codes and fp16/bf16 buffers; other widths and fp32 buffers on request only.
+        self._codec = capi.host().Codec(nbits, chunk_size, self.strategy, bool(params.get("extended", False)) or nbits not in (2, 4, 8),
+                                        (nbits * 998244353) & _U32, None, {})
         self.philox_seed = params.get("philox_seed")
-        self.randomized_vec_pool, self.randomized_vec_pools = None, {}
         if self.philox_seed is not None:
             # one stream per rank, one step per call
             self.philox_seed = (int(self.philox_seed) + self.client_rank * 0x9E3779B97F4A7C15) & 0xFFFFFFFFFFFFFFFF
-            self.philox_step = nbits << 32
+            self._codec.philox, self._codec.philox_seed, self._codec.philox_step = True, self.philox_seed, nbits << 32
             return
         rows = self.three_times_cur_max_size
         given = params.get("rand_pool_tensor")          # the reference's "correlated" mode loads its pool from disk
@@ -76,6 +69,36 @@ class _DynamicRangeGPUKern(object):
                 pool = pool.to(dtype=self.given_pool_dtype)
         self.randomized_vec_pool = pool
         self.randomized_vec_pools[pool.dtype] = pool
+
+    # ---- state the reference's callers may read (and that the native object works with) ----------------------
+    @property
+    def rand_seed(self):
+        return self._codec.rand_seed
+
+    @rand_seed.setter
+    def rand_seed(self, seed):
+        self._codec.rand_seed = seed & _U32
+
+    @property
+    def philox_step(self):
+        return self._codec.philox_step
+
+    @philox_step.setter
+    def philox_step(self, step):
+        self._codec.philox_step = step
+
+    @property
+    def randomized_vec_pool(self):
+        return self._codec.base
+
+    @randomized_vec_pool.setter
+    def randomized_vec_pool(self, pool):
+        self._codec.base = pool
+
+    @property
+    def randomized_vec_pools(self):
+        """dtype -> the pool in that dtype (converted when a call first needs it)"""
+        return self._codec.pools
 
     # ---- sizes --------------------------------------------------------------------------------------------
     def padded_n(self, n):
@@ -107,47 +130,22 @@ class _DynamicRangeGPUKern(object):
         first = self.gen_next_rand() % choices
         return pool[first:first + rows, :]
 
-    def _next_step(self):
-        self.philox_step += 1
-        return self.philox_step
-
     @staticmethod
     def _stream():
         return torch.cuda.current_stream().cuda_stream
 
     # ---- the calls of the ring schedules (:422-466) ------------------------------------------------------
     def compression(self, input_chunk, send_chunk, interm_chunk=None):
-        n = input_chunk.numel()
-        if n == 0:
-            return
-        tail = (n, self.nbits, self.chunk_size)
-        if self.philox_seed is None:
-            self._compress(input_chunk, send_chunk, self.rand_pool(n, input_chunk.dtype), *tail, self._stream(), self.strategy)
-        else:
-            self.eden_utils.scaling_compress_philox(input_chunk, send_chunk, *tail, self.philox_seed, self._next_step(),
-                                                    self._stream(), self.strategy)
+        self._codec.compress(input_chunk, send_chunk)
 
     def decompression(self, recv_chunk, input_chunk, interm_chunk=None):
-        n = input_chunk.numel()
-        if n:
-            self._decompress(recv_chunk, input_chunk, n, self.nbits, self.chunk_size, self._stream(), self.strategy)
+        self._codec.decompress(recv_chunk, input_chunk, False)
 
     def decompression_add(self, recv_chunk, input_chunk, interm_chunk=None):
-        n = input_chunk.numel()
-        if n:
-            self._decompress_add(recv_chunk, input_chunk, n, self.nbits, self.chunk_size, self._stream(), self.strategy)
+        self._codec.decompress(recv_chunk, input_chunk, True)
 
     def dec_compression(self, recv_chunk, input_chunk, send_chunk, interm_chunk=None, interm_chunk2=None):
-        n = input_chunk.numel()
-        if n == 0:
-            return
-        tail = (n, self.nbits, self.chunk_size)
-        if self.philox_seed is None:
-            self._dec_comp(recv_chunk, input_chunk, send_chunk, self.rand_pool(n, input_chunk.dtype), *tail, self._stream(),
-                           self.strategy)
-        else:
-            self.eden_utils.scaling_dec_comp_philox(recv_chunk, input_chunk, send_chunk, *tail, self.philox_seed,
-                                                    self._next_step(), self._stream(), self.strategy)
+        self._codec.dec_comp(recv_chunk, input_chunk, send_chunk)
 
     # ---- the same steps over a list of superchunk indices: index_select + the call above + index_copy_
     #      (comm_hooks.py:1001-1011) without the gathered copy; no counterpart in the reference ----

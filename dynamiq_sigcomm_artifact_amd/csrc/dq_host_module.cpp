@@ -10,8 +10,12 @@
 #include <ATen/core/Tensor.h>
 #include <c10/hip/HIPStream.h>
 #include <pybind11/pybind11.h>
+#include <torch/csrc/DynamicTypes.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <string.h>
+
+#include <algorithm>
 #include <stdexcept>
 #include <string>
 #include <vector>
@@ -313,10 +317,410 @@ void ranks_dynamic(py::sequence vecs, py::sequence outs, int64_t n, py::handle t
     k.enqueue(DQ_RANKS_STATS | DQ_RANKS_PLAN | DQ_RANKS_RING, a.device, stream_of(stream));
 }
 
+// ---- compressor objects ------------------------------------------------------------------------------------
+
+void need(bool ok, const char *text)
+{
+    if (!ok) refuse(text);
+}
+
+// The calls of a compressor object (compressors.py): element counts, the rows of the random pool and their LCG, the
+// checks and texts of the module's scaling_* functions, torch's current stream, the launch.
+struct Codec {
+    int nbits, chunk, strategy;
+    bool extended; // float32 buffers and 3/5/6/7-bit codes
+    uint32_t rand_seed;
+    bool philox = false;
+    uint64_t philox_seed = 0, philox_step = 0;
+    py::object base;  // the pool as drawn or loaded, [rows, chunk]
+    py::dict pools;   // dtype -> the pool in that dtype
+
+    Codec(int nbits_, int chunk_, int strategy_, bool extended_, uint32_t seed, py::object base_, py::dict pools_)
+        : nbits(nbits_), chunk(chunk_), strategy(strategy_), extended(extended_), rand_seed(seed), base(base_), pools(pools_)
+    {
+    }
+    uint32_t next_rand()
+    {
+        rand_seed = rand_seed * 671431u + 1000000007u; // utils_aggregation.py:391-393
+        return rand_seed;
+    }
+    const at::Tensor &pool(at::ScalarType dtype)
+    {
+        PyObject *key = reinterpret_cast<PyObject *>(torch::getTHPDtype(dtype));
+        PyObject *have = PyDict_GetItem(pools.ptr(), key);
+        if (!have) {
+            if (!THPVariable_Check(base.ptr())) refuse("this compressor has no random pool");
+            const py::object made = base.attr("to")(py::reinterpret_borrow<py::object>(key));
+            PyDict_SetItem(pools.ptr(), key, made.ptr());
+            have = made.ptr(); // the dictionary holds it
+        }
+        return THPVariable_Unpack(have);
+    }
+    // first of n / chunk consecutive rows, where the LCG points (utils_aggregation.py:409-420)
+    int64_t first_row(const at::Tensor &p, int64_t n)
+    {
+        const int64_t choices = p.size(0) - n / chunk - 1;
+        need(choices > 0, "randomized_vec_pool is too small for scaling quantization");
+        return (int64_t)next_rand() % choices;
+    }
+    const void *random_rows(const at::Tensor &like, int64_t n)
+    {
+        const at::Tensor &p = pool(like.scalar_type());
+        need(p.is_cuda(), "rand_pool must be a CUDA tensor");
+        need(p.is_contiguous(), "rand_pool must be contiguous");
+        need(p.device() == like.device(), "tensor arguments live on different devices");
+        return static_cast<const char *>(p.data_ptr()) + first_row(p, n) * chunk * (int64_t)like.element_size();
+    }
+    void check_common(int64_t n) const
+    {
+        need(n > 0, "n must be positive");
+        if (!extended) need(nbits == 2 || nbits == 4 || nbits == 8, "nbits must be one of {2, 4, 8}");
+        const int rc = dq_scaling_check_common(n, nbits, chunk, strategy, 0);
+        if (rc) refuse(dq_last_error());
+    }
+    bool data_dtype(const at::Tensor &t) const
+    {
+        const at::ScalarType d = t.scalar_type();
+        return d == at::kBFloat16 || d == at::kHalf || (d == at::kFloat && (extended || philox));
+    }
+    static const at::Tensor &cuda(py::handle h, const char *text)
+    {
+        if (!THPVariable_Check(h.ptr())) refuse(std::string("a tensor argument is required, got ") + Py_TYPE(h.ptr())->tp_name);
+        const at::Tensor &t = THPVariable_Unpack(h.ptr());
+        need(t.is_cuda(), text);
+        return t;
+    }
+    int64_t bytes(int64_t n) const { return dq_scaling_required_bytes(n, nbits, chunk, strategy); }
+
+    void compress(py::handle input, py::handle send)
+    {
+        const at::Tensor &src = cuda(input, "input must be a CUDA tensor");
+        const int64_t n = src.numel();
+        if (n == 0) return;
+        const at::Tensor &dst = cuda(send, "output must be a CUDA tensor");
+        need(data_dtype(src), "input must be torch.float16 or torch.bfloat16");
+        const void *rnd = philox ? nullptr : random_rows(src, n);
+        need(dst.scalar_type() == at::kByte, "output must be torch.uint8");
+        need(src.is_contiguous(), "input must be contiguous");
+        need(dst.is_contiguous(), "output must be contiguous");
+        need(dst.device() == src.device(), "tensor arguments live on different devices");
+        check_common(n);
+        need(dst.numel() >= bytes(n), "output buffer is too small");
+        const void *x = src.data_ptr();
+        uint8_t *y = dst.data_ptr<uint8_t>();
+        const int code = dtype_code(src), device = src.device().index();
+        const dq_stream_t s = c10::hip::getCurrentHIPStream().stream();
+        const uint64_t step = philox ? ++philox_step : 0;
+        int rc;
+        {
+            py::gil_scoped_release nogil;
+            rc = philox ? dq_scaling_compress_philox(x, y, n, nbits, chunk, code, device, strategy, philox_seed, step, s)
+                        : dq_scaling_compress(x, y, rnd, n, nbits, chunk, code, device, strategy, s);
+        }
+        check(rc);
+    }
+    void decompress(py::handle recv, py::handle output, bool add)
+    {
+        const at::Tensor &dst = cuda(output, "output must be a CUDA tensor");
+        const int64_t n = dst.numel();
+        if (n == 0) return;
+        const at::Tensor &src = cuda(recv, "input must be a CUDA tensor");
+        need(src.scalar_type() == at::kByte, "input must be torch.uint8");
+        need(data_dtype(dst), "output must be torch.float16 or torch.bfloat16");
+        need(src.is_contiguous(), "input must be contiguous");
+        need(dst.is_contiguous(), "output must be contiguous");
+        need(dst.device() == src.device(), "tensor arguments live on different devices");
+        check_common(n);
+        need(src.numel() >= bytes(n), "input buffer is too small");
+        const uint8_t *x = src.data_ptr<uint8_t>();
+        void *y = dst.data_ptr();
+        const int code = dtype_code(dst), device = dst.device().index();
+        const dq_stream_t s = c10::hip::getCurrentHIPStream().stream();
+        int rc;
+        {
+            py::gil_scoped_release nogil;
+            rc = dq_scaling_decompress(x, y, n, nbits, chunk, code, device, strategy, s, add ? 1 : 0);
+        }
+        check(rc);
+    }
+    void dec_comp(py::handle recv_, py::handle input, py::handle send_)
+    {
+        const at::Tensor &inp = cuda(input, "inp must be a CUDA tensor");
+        const int64_t n = inp.numel();
+        if (n == 0) return;
+        const at::Tensor &recv = cuda(recv_, "recv must be a CUDA tensor"), &send = cuda(send_, "send must be a CUDA tensor");
+        need(recv.scalar_type() == at::kByte, "recv must be torch.uint8");
+        need(data_dtype(inp), "inp must be torch.float16 or torch.bfloat16");
+        const void *rnd = philox ? nullptr : random_rows(inp, n);
+        need(send.scalar_type() == at::kByte, "send must be torch.uint8");
+        need(recv.is_contiguous(), "recv must be contiguous");
+        need(inp.is_contiguous(), "inp must be contiguous");
+        need(send.is_contiguous(), "send must be contiguous");
+        need(recv.device() == inp.device() && send.device() == inp.device(), "tensor arguments live on different devices");
+        check_common(n);
+        need(recv.numel() >= bytes(n), "recv buffer is too small");
+        need(send.numel() >= bytes(n), "send buffer is too small");
+        const uint8_t *r = recv.data_ptr<uint8_t>();
+        void *x = inp.data_ptr();
+        uint8_t *y = send.data_ptr<uint8_t>();
+        const int code = dtype_code(inp), device = inp.device().index();
+        const dq_stream_t s = c10::hip::getCurrentHIPStream().stream();
+        const uint64_t step = philox ? ++philox_step : 0;
+        int rc;
+        {
+            py::gil_scoped_release nogil;
+            rc = philox ? dq_scaling_dec_comp_philox(r, x, y, n, nbits, chunk, code, device, strategy, philox_seed, step, s)
+                        : dq_scaling_dec_comp(r, x, y, rnd, n, nbits, chunk, code, device, strategy, s);
+        }
+        check(rc);
+    }
+};
+
+// ---- ranks with random pools --------------------------------------------------------------------------------
+
+// One bucket of the fixed-proportion (sorted_plan) or dynamic all-reduce with compressor objects: codecs holds one list per
+// width (8, 4, 2 bits), group sizes counts.  Walks every codec's LCG as the ring's calls on its non-empty chunks would, in
+// the order of the widths and, per rank, of the steps: rank r works on chunk (r - step) mod world in that step.
+void ranks_pooled(py::sequence vecs, py::sequence outs, int64_t n, py::handle total, py::handle mean, py::handle order,
+                  py::handle work, py::sequence codecs, py::sequence counts, int stages, int strategy)
+{
+    Args a;
+    Ranks k(a, vecs, outs, n, total, mean, order, work, strategy);
+    const int world = k.r.world;
+    const at::ScalarType dtype = THPVariable_Unpack(py::object(vecs[0]).ptr()).scalar_type();
+    std::vector<const void *> pool(3 * world, nullptr);
+    std::vector<int32_t> first(3 * world * world, 0);
+    int64_t size[3];
+    for (int g = 0; g < 3; g++) size[g] = py::cast<int64_t>(counts[g]);
+    for (int g = 0; g < 3; g++) {
+        if (size[g] == 0) continue;
+        const py::sequence of_width = codecs[g];
+        const int64_t per = (size[g] + world - 1) / world;
+        for (int r = 0; r < world; r++) {
+            Codec &c = py::cast<Codec &>(of_width[r]);
+            const at::Tensor &p = c.pool(dtype);
+            need(p.is_cuda() && p.is_contiguous() && p.device().index() == a.device, "rand_pool must be a contiguous tensor on the vectors' device");
+            pool[g * world + r] = p.data_ptr();
+            for (int step = 0; step < world; step++) {
+                const int chunk = (r - step + world) % world;
+                const int64_t rows = std::max<int64_t>(0, std::min(per, size[g] - per * chunk));
+                if (rows == 0) continue;
+                const int64_t at = c.first_row(p, rows * 256);
+                need(at <= 0x7fffffff, "randomized_vec_pool has too many rows");
+                first[(g * world + r) * world + step] = (int32_t)at;
+            }
+        }
+    }
+    k.r.pool = pool.data();
+    k.r.first = first.data();
+    k.r.sorted_plan = 1;
+    k.r.top_count = size[0];
+    k.r.bottom_count = size[2];
+    k.enqueue(stages, a.device, c10::hip::getCurrentHIPStream().stream());
+}
+
+// ---- codec calls on tensors (capi.py) ------------------------------------------------------------------------
+// positional arguments only, no argument-conversion layer: capi.py's functions give them in order
+
+template <class F> PyObject *guarded(Py_ssize_t have, Py_ssize_t want, F body)
+{
+    try {
+        if (have != want) refuse("wrong number of arguments");
+        body();
+    } catch (py::error_already_set &e) {
+        e.restore();
+        return nullptr;
+    } catch (const std::exception &e) {
+        PyErr_SetString(PyExc_RuntimeError, e.what());
+        return nullptr;
+    }
+    Py_RETURN_NONE;
+}
+
+int64_t integer(PyObject *o)
+{
+    const long long v = PyLong_AsLongLong(o);
+    if (v == -1 && PyErr_Occurred()) throw py::error_already_set();
+    return v;
+}
+
+int small_integer(PyObject *o) { return (int)integer(o); }
+
+uint64_t word(PyObject *o)
+{
+    const unsigned long long v = PyLong_AsUnsignedLongLongMask(o);
+    if (v == (unsigned long long)-1 && PyErr_Occurred()) throw py::error_already_set();
+    return v;
+}
+
+float real(PyObject *o)
+{
+    const double v = PyFloat_AsDouble(o);
+    if (v == -1.0 && PyErr_Occurred()) throw py::error_already_set();
+    return (float)v;
+}
+
+// fp32 elements may come with a bf16 pool
+int pair_code(const at::Tensor &elem, const at::Tensor &pool)
+{
+    const int code = dtype_code(elem);
+    if (pool.scalar_type() == elem.scalar_type()) return code;
+    if (code == DQ_F32 && pool.scalar_type() == at::kBFloat16) return code | DQ_RAND_BF16;
+    refuse("rand_pool dtype must match input dtype");
+}
+
+// src, dst, rand_pool, n, nbits, chunk_size, strategy, stream
+PyObject *scaling_compress(PyObject *, PyObject *const *v, Py_ssize_t have)
+{
+    return guarded(have, 8, [&] {
+        Args a;
+        const at::Tensor &src = a.tensor(v[0]), &dst = a.tensor(v[1]), &pool = a.tensor(v[2]);
+        const int code = pair_code(src, pool), nbits = small_integer(v[4]), chunk = small_integer(v[5]), strategy = small_integer(v[6]);
+        const int64_t n = integer(v[3]);
+        const dq_stream_t s = stream_of(v[7]);
+        const void *x = src.data_ptr(), *r = pool.data_ptr();
+        uint8_t *y = static_cast<uint8_t *>(dst.data_ptr());
+        int rc;
+        {
+            py::gil_scoped_release nogil;
+            rc = dq_scaling_compress(x, y, r, n, nbits, chunk, code, a.device, strategy, s);
+        }
+        check(rc);
+    });
+}
+
+// src, dst, n, nbits, chunk_size, strategy, add, stream
+PyObject *scaling_decompress(PyObject *, PyObject *const *v, Py_ssize_t have)
+{
+    return guarded(have, 8, [&] {
+        Args a;
+        const at::Tensor &src = a.tensor(v[0]), &dst = a.tensor(v[1]);
+        const int code = dtype_code(dst), nbits = small_integer(v[3]), chunk = small_integer(v[4]), strategy = small_integer(v[5]);
+        const int64_t n = integer(v[2]);
+        const int add = PyObject_IsTrue(v[6]);
+        const dq_stream_t s = stream_of(v[7]);
+        const uint8_t *x = static_cast<const uint8_t *>(src.data_ptr());
+        void *y = dst.data_ptr();
+        int rc;
+        {
+            py::gil_scoped_release nogil;
+            rc = dq_scaling_decompress(x, y, n, nbits, chunk, code, a.device, strategy, s, add);
+        }
+        check(rc);
+    });
+}
+
+// recv, inp, send, rand_pool, n, nbits, chunk_size, strategy, stream
+PyObject *scaling_dec_comp(PyObject *, PyObject *const *v, Py_ssize_t have)
+{
+    return guarded(have, 9, [&] {
+        Args a;
+        const at::Tensor &recv = a.tensor(v[0]), &inp = a.tensor(v[1]), &send = a.tensor(v[2]), &pool = a.tensor(v[3]);
+        const int code = pair_code(inp, pool), nbits = small_integer(v[5]), chunk = small_integer(v[6]), strategy = small_integer(v[7]);
+        const int64_t n = integer(v[4]);
+        const dq_stream_t s = stream_of(v[8]);
+        const uint8_t *x = static_cast<const uint8_t *>(recv.data_ptr());
+        uint8_t *y = static_cast<uint8_t *>(send.data_ptr());
+        void *i = inp.data_ptr();
+        const void *r = pool.data_ptr();
+        int rc;
+        {
+            py::gil_scoped_release nogil;
+            rc = dq_scaling_dec_comp(x, i, y, r, n, nbits, chunk, code, a.device, strategy, s);
+        }
+        check(rc);
+    });
+}
+
+const void *sign_of(Args &a, PyObject *sign, int *packed)
+{
+    *packed = 0;
+    if (sign == Py_None) return nullptr;
+    const at::Tensor &t = a.tensor(sign);
+    *packed = t.scalar_type() == at::kInt ? 1 : 0;
+    return t.data_ptr();
+}
+
+// src, sign, dst, block, scale, nbits, strategy, rand_pool, seed, step, stream
+PyObject *rht_scaling_compress(PyObject *, PyObject *const *v, Py_ssize_t have)
+{
+    return guarded(have, 11, [&] {
+        Args a;
+        const at::Tensor &src = a.tensor(v[0]);
+        need(src.scalar_type() == at::kFloat, "rht_scaling_compress: src must be float32");
+        int packed, rcode = 0;
+        const void *sign = sign_of(a, v[1], &packed);
+        uint8_t *y = static_cast<uint8_t *>(a.tensor(v[2]).data_ptr());
+        const void *pool = nullptr;
+        if (v[7] != Py_None) {
+            const at::Tensor &p = a.tensor(v[7]);
+            rcode = dtype_code(p);
+            pool = p.data_ptr();
+        }
+        const int64_t block = integer(v[3]), n = src.numel();
+        const float scale = real(v[4]), *x = static_cast<const float *>(src.data_ptr());
+        const int nbits = small_integer(v[5]), strategy = small_integer(v[6]);
+        const uint64_t seed = word(v[8]), step = word(v[9]);
+        const dq_stream_t s = stream_of(v[10]);
+        int rc;
+        {
+            py::gil_scoped_release nogil;
+            rc = dq_rht_scaling_compress(x, sign, packed, y, pool, rcode, n, block, scale, nbits, a.device, strategy, seed, step, s);
+        }
+        check(rc);
+    });
+}
+
+// src, sign, dst, block, scale, nbits, strategy, stream
+PyObject *scaling_decompress_irht(PyObject *, PyObject *const *v, Py_ssize_t have)
+{
+    return guarded(have, 8, [&] {
+        Args a;
+        const uint8_t *x = static_cast<const uint8_t *>(a.tensor(v[0]).data_ptr());
+        int packed;
+        const void *sign = sign_of(a, v[1], &packed);
+        const at::Tensor &dst = a.tensor(v[2]);
+        need(dst.scalar_type() == at::kFloat, "scaling_decompress_irht: dst must be float32");
+        const int64_t block = integer(v[3]), n = dst.numel();
+        float *y = static_cast<float *>(dst.data_ptr());
+        const float scale = real(v[4]);
+        const int nbits = small_integer(v[5]), strategy = small_integer(v[6]);
+        const dq_stream_t s = stream_of(v[7]);
+        int rc;
+        {
+            py::gil_scoped_release nogil;
+            rc = dq_scaling_decompress_irht(x, sign, packed, y, n, block, scale, nbits, a.device, strategy, s);
+        }
+        check(rc);
+    });
+}
+
+PyMethodDef kFunctions[] = {
+    {"scaling_compress", reinterpret_cast<PyCFunction>(scaling_compress), METH_FASTCALL, nullptr},
+    {"scaling_decompress", reinterpret_cast<PyCFunction>(scaling_decompress), METH_FASTCALL, nullptr},
+    {"scaling_dec_comp", reinterpret_cast<PyCFunction>(scaling_dec_comp), METH_FASTCALL, nullptr},
+    {"rht_scaling_compress", reinterpret_cast<PyCFunction>(rht_scaling_compress), METH_FASTCALL, nullptr},
+    {"scaling_decompress_irht", reinterpret_cast<PyCFunction>(scaling_decompress_irht), METH_FASTCALL, nullptr},
+    {nullptr, nullptr, 0, nullptr},
+};
+
 } // namespace
 
 PYBIND11_MODULE(_host, m)
 {
+    PyModule_AddFunctions(m.ptr(), kFunctions);
+    py::class_<Codec>(m, "Codec")
+        .def(py::init<int, int, int, bool, uint32_t, py::object, py::dict>())
+        .def_readwrite("rand_seed", &Codec::rand_seed)
+        .def_readwrite("philox", &Codec::philox)
+        .def_readwrite("philox_seed", &Codec::philox_seed)
+        .def_readwrite("philox_step", &Codec::philox_step)
+        .def_readwrite("base", &Codec::base)
+        .def_readwrite("pools", &Codec::pools)
+        .def("compress", &Codec::compress)
+        .def("decompress", &Codec::decompress)
+        .def("dec_comp", &Codec::dec_comp);
+    m.def("ranks_pooled", &ranks_pooled);
     m.doc() = "native host path of dynamiq_sigcomm_artifact_amd";
     py::class_<Buckets>(m, "Buckets")
         .def(py::init<int, uint64_t, py::object, py::object, py::object>())
