@@ -15,7 +15,8 @@ size == 1).
 import torch
 
 from . import bitrate
-from .compressors import superchunk_add_mean_copy, superchunk_mean_center
+from .compressors import (Aee_Dynamic_Range_GPU_kern, Mee_Dynamic_Range_GPU_kern, superchunk_add_mean_copy,
+                          superchunk_mean_center)
 from . import load_eden_utils
 from .ring_sim import ring_allreduce, ring_allreduce_rows
 
@@ -64,15 +65,37 @@ def dynamic_bitrate_allreduce(rank_vecs, u, compressors, out=None):
     return outs, total, qbits
 
 
+_RANKS_STATS, _RANKS_PLAN, _RANKS_RING = 1, 2, 4
+
+
+def _pooled_codecs(rank_vecs, compressors):
+    """the native objects of the compressors, one list per width (8, 4, 2 bits), when the whole all-reduce can run without
+    packed streams (csrc/dq_single_pass.hip): the package's own pooled compressors of one strategy, bf16 vectors and no
+    more ranks than the arguments of one launch hold.  Else None: the ring then runs call by call."""
+    from . import capi
+    W = len(rank_vecs)
+    if W > capi.ranks_max(True) or rank_vecs[0].dtype != torch.bfloat16:
+        return None
+    every = [c for q in (8, 4, 2) for c in compressors.get(q, ())]
+    if not all(type(c) in (Aee_Dynamic_Range_GPU_kern, Mee_Dynamic_Range_GPU_kern) and c.philox_seed is None and c.chunk_size == 16 and
+               c.strategy == every[0].strategy for c in every):
+        return None
+    if any(len(compressors.get(q, ())) < W or compressors[q][0].nbits != q for q in (8, 4, 2)):
+        return None
+    return [[c._codec for c in compressors[q]] for q in (8, 4, 2)]
+
+
 def dynamic_bitrate_allreduce_grouped(rank_vecs, u, compressors, out=None, work=None, device_qbits=False):
     """Same inputs, same results (bit for bit) as dynamic_bitrate_allreduce, with the gather, the scatter
     and the final mean add folded into the codec kernels: one device-side partition of the superchunk
     indices by width (a single 16-byte read-back for the three group sizes, in place of three
     torch.nonzero), no group tensors, no index_select / index_copy_ / superchunk_add_mean_copy passes.
+    With the package's pooled compressors the ring itself is one launch for all ranks, steps and widths.
 
     device_qbits=True also computes the bit widths inside the partition call (the rule of
     bitrate.dynamic_bitrate_qbits with the library's fixed-polynomial log2 in place of torch.log2; the two
     agree except where a log2 value lies within a few binary32 ulps of a bf16 rounding boundary)."""
+    from . import capi
     eu = load_eden_utils()
     W = len(rank_vecs)
     n = rank_vecs[0].numel()
@@ -80,30 +103,43 @@ def dynamic_bitrate_allreduce_grouped(rank_vecs, u, compressors, out=None, work=
     dev, dt = rank_vecs[0].device, rank_vecs[0].dtype
     if work is None:
         work = {}
-    key = (nsc, dt, W)
+    codecs = _pooled_codecs(rank_vecs, compressors)
+    key = (nsc, dt, W, codecs is None)
     if work.get("key") != key:
         work["key"] = key
-        work["residuals"] = [torch.empty(nsc * SUPERCHUNK, dtype=dt, device=dev) for _ in range(W)]
-        work["stats"] = [torch.empty((nsc, 2), dtype=torch.bfloat16, device=dev) for _ in range(W)]
+        work["residuals"] = [] if codecs else [torch.empty(nsc * SUPERCHUNK, dtype=dt, device=dev) for _ in range(W)]
+        work["stats"] = [] if codecs else [torch.empty((nsc, 2), dtype=torch.bfloat16, device=dev) for _ in range(W)]
         work["order"] = torch.empty(3 * nsc, dtype=torch.int32, device=dev)
+        work["mean"] = torch.empty(W * nsc, dtype=torch.float32, device=dev) if codecs else None
     residuals, stats, order = work["residuals"], work["stats"], work["order"]
     stream = torch.cuda.current_stream().cuda_stream
-    for r in range(W):
-        superchunk_mean_center(rank_vecs[r], residuals[r], stats[r], n, W, SUPERCHUNK)
-    total = stats[0] if W == 1 else stats[0].clone()
-    for r in range(1, W):
-        total.add_(stats[r])
+    outs = out if out is not None else [torch.empty(n, dtype=dt, device=dev) for _ in range(W)]
+    if codecs:
+        # all ranks' statistics and their sum in one launch; nothing is centred yet
+        total = torch.empty((nsc, 2), dtype=torch.bfloat16, device=dev)
+        capi.host().ranks_pooled(rank_vecs, outs, n, total, work["mean"], order, order, codecs, (0, 0, 0), _RANKS_STATS,
+                                 compressors[8][0].strategy)
+    else:
+        for r in range(W):
+            superchunk_mean_center(rank_vecs[r], residuals[r], stats[r], n, W, SUPERCHUNK)
+        total = stats[0] if W == 1 else stats[0].clone()
+        for r in range(1, W):
+            total.add_(stats[r])
     if device_qbits:
         qbits = work.get("qbits")
         if qbits is None or qbits.numel() != nsc:
             qbits = work["qbits"] = torch.empty(nsc, dtype=torch.int64, device=dev)
-        counts = eu.group_plan_stats(total, float(u), order, qbits, stream).tolist()
+        sizes = eu.group_plan_stats(total, float(u), order, qbits, stream)
     else:
         qbits = bitrate.dynamic_bitrate_qbits(total[:, 1], u)
-        counts = eu.group_plan(qbits, order, stream).tolist()
+        sizes = eu.group_plan(qbits, order, stream)
+    counts = sizes.tolist()
     assert counts[3] == 0, "bit widths outside {2, 4, 8}"
 
-    outs = out if out is not None else [torch.empty(n, dtype=dt, device=dev) for _ in range(W)]
+    if codecs:
+        capi.host().ranks_pooled(rank_vecs, outs, n, total, work["mean"], order, sizes, codecs, counts[:3], _RANKS_RING,
+                                 compressors[8][0].strategy)
+        return outs, total, qbits
     for g, (q, cnt) in enumerate(zip((8, 4, 2), counts[:3])):
         if cnt == 0:
             continue
@@ -163,13 +199,29 @@ def fixed_proportion_allreduce(rank_vecs, thresholds, compressors, out=None, fix
 
 def fixed_proportion_allreduce_grouped(rank_vecs, thresholds, compressors, out=None, fixed_4bit_only=False):
     """The same all-reduce, bit for bit, with the sort, the slices, the gathers, the scatters and the final mean add
-    replaced by one launch of the device plan (group_plan_sorted) and the row-list codec calls; the group sizes follow
-    from the fractions on the host, so nothing is read back."""
+    replaced by one launch of the device plan (group_plan_sorted) and, with the package's pooled compressors, one launch of
+    the whole ring (else the row-list codec calls); the group sizes follow from the fractions on the host, so nothing is
+    read back."""
+    from . import capi
     eu = load_eden_utils()
     W = len(rank_vecs)
     n = rank_vecs[0].numel()
     nsc = (n + SUPERCHUNK - 1) // SUPERCHUNK
     dev, dt = rank_vecs[0].device, rank_vecs[0].dtype
+    counts = bitrate.fixed_proportion_counts(nsc, thresholds)
+    codecs = _pooled_codecs(rank_vecs, compressors)
+    if codecs and not (fixed_4bit_only and counts[1] != nsc):
+        # three launches for all ranks, steps and widths: statistics, sorted plan, ring
+        outs = out if out is not None else [torch.empty(n, dtype=dt, device=dev) for _ in range(W)]
+        total = torch.empty((nsc, 2), dtype=torch.bfloat16, device=dev)
+        # one block of scratch: row lists (they are returned), plan, means
+        plan_ints = capi.group_plan_sorted_work_ints(nsc)
+        ints = torch.empty(3 * nsc + W * nsc + plan_ints, dtype=torch.int32, device=dev)
+        order = ints[:3 * nsc]
+        capi.host().ranks_pooled(rank_vecs, outs, n, total, ints[3 * nsc:3 * nsc + W * nsc].view(torch.float32), order,
+                                 ints[3 * nsc + W * nsc:], codecs, counts, _RANKS_STATS | _RANKS_PLAN | _RANKS_RING,
+                                 compressors[8][0].strategy)
+        return outs, total, order, counts
     residuals = [torch.empty(nsc * SUPERCHUNK, dtype=dt, device=dev) for _ in range(W)]
     stats = [torch.empty((nsc, 2), dtype=torch.bfloat16, device=dev) for _ in range(W)]
     for r in range(W):
@@ -177,7 +229,6 @@ def fixed_proportion_allreduce_grouped(rank_vecs, thresholds, compressors, out=N
     total = stats[0] if W == 1 else stats[0].clone()
     for r in range(1, W):
         total.add_(stats[r])
-    counts = bitrate.fixed_proportion_counts(nsc, thresholds)
     order = torch.empty(3 * nsc, dtype=torch.int32, device=dev)
     eu.group_plan_sorted(total, counts[0], counts[2], order, None, torch.cuda.current_stream().cuda_stream)
     outs = out if out is not None else [torch.empty(n, dtype=dt, device=dev) for _ in range(W)]

@@ -230,3 +230,32 @@ def test_sorted_plan_of_a_long_bucket(capi, oracle, nsc, method):
     q = qb.cpu().numpy()
     assert (q[want[:n8]] == 8).all() and (q[want[n8:n8 + n4]] == 4).all() and (q[want[n8 + n4:]] == 2).all()
     assert np.array_equal(order.cpu().numpy()[:n8], want[:n8])
+
+
+@pytest.mark.parametrize("W,n", [(1, 255), (8, 256 * 9), (8, 256 * 203 - 1), (9, 256 * 40 + 3)])
+def test_pooled_ring_in_registers_equals_op_sequence(capi, W, n):
+    """one launch for the whole ring against the op sequence at the edges of its tiles and ring chunks (a rank without a
+    chunk does not advance its LCG), on unaligned vectors, and with one rank more than a launch takes; two buckets in a row
+    walk the pools on"""
+    from dynamiq_sigcomm_artifact_amd.compressors import Aee_Dynamic_Range_GPU_kern, Mee_Dynamic_Range_GPU_kern
+    from dynamiq_sigcomm_artifact_amd.dynamiq_pipeline import fixed_proportion_allreduce, fixed_proportion_allreduce_grouped
+    nsc = (n + 255) // 256
+    for K, shift, thr in ((Aee_Dynamic_Range_GPU_kern, 0, {8: 0.35, 4: 0.45, 2: 0.2}), (Mee_Dynamic_Range_GPU_kern, 1, {8: 0.05, 4: 0.95, 2: 0.0})):
+        g = torch.Generator().manual_seed(n + W)
+        vecs = []
+        for _ in range(W):
+            v = torch.zeros(n + shift, dtype=torch.bfloat16, device=DEV)
+            v[shift:].copy_((torch.randn(nsc, 256, generator=g) * torch.exp(torch.randn(nsc, 1, generator=g))).reshape(-1)[:n])
+            vecs.append(v[shift:])
+
+        def comps():
+            gen = torch.Generator(device=DEV).manual_seed(5)
+            return {q: [K(q, 16, {"d": {0: (n + 256) * W}, "world_size": W, "rank": r}, generator=gen)
+                        for r in range(W)] for q in (8, 4, 2)}
+        a, b = comps(), comps()
+        for _ in range(2):
+            ref, total, _ = fixed_proportion_allreduce(vecs, thr, a)
+            out, total2, _, _ = fixed_proportion_allreduce_grouped(vecs, thr, b)
+            assert torch.equal(total.view(torch.int16), total2.view(torch.int16))
+            assert all(torch.equal(x.view(torch.int16), y.view(torch.int16)) for x, y in zip(ref, out))
+        assert all(x.rand_seed == y.rand_seed for q in (8, 4, 2) for x, y in zip(a[q], b[q]))
