@@ -905,6 +905,106 @@ int dq_eden_dequantize(const uint32_t *packed, int64_t n, const float *centroids
     return finish(dq::launch_eden_dequantize(packed, n, centroids, nbits, out, static_cast<hipStream_t>(stream)));
 }
 
+int64_t dq_eden_slice_bytes(int64_t n) { return n >= 32 && (n & (n - 1)) == 0 ? dq::eden_slice_bytes(n) : 0; }
+
+static int check_eden_slice(int64_t count, int64_t n, int dtype, int rotations, int nbits, int64_t scratch_bytes, const void *scratch)
+{
+    if (n < 32 || (n & (n - 1)) != 0) return fail(DQ_ERR_POW2, "the padded size of a slice (at least 32)");
+    if (!(count > 0) || count > n) return fail(DQ_ERR_SIZE, "count must lie in [1, n]");
+    if (!dtype_ok(dtype)) return fail(DQ_ERR_DTYPE);
+    if (nbits < 1 || nbits > 8) return fail(DQ_ERR_NBITS, "nbits must be in [1, 8]");
+    if (rotations < 0) return fail(DQ_ERR_SIZE, "rotations must not be negative");
+    if (!scratch) return fail(DQ_ERR_NULL);
+    if (scratch_bytes < dq::eden_slice_bytes(n) || (reinterpret_cast<uintptr_t>(scratch) & 255))
+        return fail(DQ_ERR_SIZE, "scratch must be 256-byte aligned and hold dq_eden_slice_bytes");
+    return DQ_OK;
+}
+
+int dq_eden_compress(const void *src, int dtype, int64_t count, int64_t n, int rotations, int64_t seed, const float *boundaries,
+                     const float *centroids, int nbits, uint32_t *packed, float *result, void *scratch, int64_t scratch_bytes,
+                     int device, dq_stream_t stream)
+{
+    int rc = check_eden_slice(count, n, dtype, rotations, nbits, scratch_bytes, scratch);
+    if (rc) return rc;
+    if (!src || !boundaries || !centroids || !packed || !result) return fail(DQ_ERR_NULL);
+    if ((rc = select_device(device))) return rc;
+    return finish(dq::launch_eden_compress(src, dtype, count, n, rotations, seed, boundaries, centroids, nbits, packed, result, scratch,
+                                           static_cast<hipStream_t>(stream)));
+}
+
+int dq_eden_decompress(const uint32_t *packed, int64_t n, int rotations, int64_t seed, const float *centroids, int nbits,
+                       const float *scale, void *out, int dtype, int64_t count, void *scratch, int64_t scratch_bytes, int device,
+                       dq_stream_t stream)
+{
+    int rc = check_eden_slice(count, n, dtype, rotations, nbits, scratch_bytes, scratch);
+    if (rc) return rc;
+    if (!packed || !centroids || !scale || !out) return fail(DQ_ERR_NULL);
+    if ((rc = select_device(device))) return rc;
+    return finish(dq::launch_eden_decompress(packed, n, rotations, seed, centroids, nbits, scale, out, dtype, count, scratch,
+                                             static_cast<hipStream_t>(stream)));
+}
+
+static int thc_ends(const dq_thc_grid_t *g, dq::TransformEnds &ends)
+{
+    if (!g) return fail(DQ_ERR_NULL);
+    if (g->norm) {
+        ends.grid.kind = dq::ThcGrid::NORM;
+        ends.grid.norm = g->norm;
+        ends.grid.t = g->t;
+        ends.grid.inv_sqrt = g->inv_sqrt;
+        ends.grid.inv_levels = g->inv_levels;
+        ends.grid.inv_clients = g->inv_clients;
+    } else {
+        ends.grid.kind = dq::ThcGrid::HOST;
+        ends.grid.lo = g->lo;
+        ends.grid.spacing = g->spacing;
+        ends.grid.step = g->step;
+    }
+    return DQ_OK;
+}
+
+int dq_thc_compress(const void *src, int dtype, int64_t count, float *work, const uint32_t *sign_bits, const float *uniform,
+                    void *levels_bf16, int64_t n, float scale, const dq_thc_grid_t *grid, int levels, int device, dq_stream_t stream)
+{
+    if (n < 1024 || (n & (n - 1)) != 0) return fail(DQ_ERR_POW2, "the dimension (at least 1024)");
+    if (!(count > 0) || count > n) return fail(DQ_ERR_SIZE, "count must lie in [1, n]");
+    if (levels < 2 || levels > 256) return fail(DQ_ERR_SIZE, "levels must be in [2, 256]");
+    if (!dtype_ok(dtype)) return fail(DQ_ERR_DTYPE);
+    if (!src || !work || !sign_bits || !uniform || !levels_bf16) return fail(DQ_ERR_NULL);
+    if ((reinterpret_cast<uintptr_t>(work) | reinterpret_cast<uintptr_t>(uniform) | reinterpret_cast<uintptr_t>(levels_bf16)) & 15)
+        return fail(DQ_ERR_SIZE, "work, uniform and the levels must be 16-byte aligned");
+    dq::TransformEnds ends;
+    int rc = thc_ends(grid, ends);
+    if (rc) return rc;
+    ends.in_src = src;
+    ends.in_dtype = dtype;
+    ends.in_count = count;
+    ends.out_levels = static_cast<uint16_t *>(levels_bf16);
+    ends.uniform = uniform;
+    ends.out_top = (float)(levels - 1);
+    if ((rc = select_device(device))) return rc;
+    return finish(dq::launch_rht_ends(work, sign_bits, true, n, n, scale, 0, ends, static_cast<hipStream_t>(stream)));
+}
+
+int dq_thc_decompress(const void *levels_bf16, const uint32_t *sign_bits, float *out, int64_t count, int64_t n, float scale,
+                      const dq_thc_grid_t *grid, int device, dq_stream_t stream)
+{
+    if (n < 1024 || (n & (n - 1)) != 0) return fail(DQ_ERR_POW2, "the dimension (at least 1024)");
+    if (!(count > 0) || count > n) return fail(DQ_ERR_SIZE, "count must lie in [1, n]");
+    if (!levels_bf16 || !sign_bits || !out) return fail(DQ_ERR_NULL);
+    if ((reinterpret_cast<uintptr_t>(levels_bf16) | reinterpret_cast<uintptr_t>(out)) & 15)
+        return fail(DQ_ERR_SIZE, "the levels and out must be 16-byte aligned");
+    dq::TransformEnds ends;
+    int rc = thc_ends(grid, ends);
+    if (rc) return rc;
+    ends.in_levels = static_cast<const uint16_t *>(levels_bf16);
+    ends.out_dst = out;
+    ends.out_dtype = DQ_F32;
+    ends.out_count = count;
+    if ((rc = select_device(device))) return rc;
+    return finish(dq::launch_rht_ends(out, sign_bits, true, n, n, scale, 1, ends, static_cast<hipStream_t>(stream)));
+}
+
 int dq_thc_quantize(const float *rotated, const float *uniform, void *levels_bf16, int64_t n, const float *lo,
                     const float *delta, int levels, int device, dq_stream_t stream)
 {

@@ -444,4 +444,159 @@ hipError_t launch_thc_dequantize(const void *levels, float *out, int64_t n, cons
     return hipGetLastError();
 }
 
+// ---- a slice of EDEN's compress / decompress in one call -------------------------------------------------
+//
+// The reference (and the element-wise sequence this replaced) copies the slice to float32, copies it again or pads it, and
+// writes the diagonal to memory before every rotation.  Here the first pass of the first rotation reads the caller's vector
+// in its own type with the padding's zeros, the diagonal is drawn in the pass that applies it, and the last pass of the last
+// inverse rotation multiplies by the scale and stores the caller's type.  2^20 fp32 elements at 4 bits, both directions:
+// eight launches and three copies,
+// 94 us, against seven launches, 40 us.
+
+namespace {
+
+// Longer vectors read the diagonal from memory, one bit per element, written by a launch of its own (about 4 us): drawing it
+// costs 25 instruction slots per element, 2.7 us at 2^22 elements.
+constexpr int64_t kEdenDrawnSigns = (int64_t)1 << 22;
+
+// slices of less than 1024 elements (the ends of short vectors): the rotations of dq_hadamard.hip on a padded copy
+__global__ __launch_bounds__(256) void eden_pad_kernel(const void *__restrict__ src, int dtype, int64_t count, int64_t n,
+                                                       float *__restrict__ out)
+{
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    float v = 0.0f;
+    if (i < count)
+        v = dtype == DQ_F32 ? ElemIO<DQ_F32>::load(src, i) : (dtype == DQ_BF16 ? ElemIO<DQ_BF16>::load(src, i) : ElemIO<DQ_F16>::load(src, i));
+    out[i] = v;
+}
+
+// out = T(scale * vec), elements below count
+__global__ __launch_bounds__(256) void eden_finish_kernel(const float *__restrict__ vec, const float *__restrict__ scale,
+                                                          void *__restrict__ out, int dtype, int64_t count)
+{
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= count) return;
+    const float v = *scale * vec[i];
+    if (dtype == DQ_F32)
+        ElemIO<DQ_F32>::store(out, i, v);
+    else if (dtype == DQ_BF16)
+        ElemIO<DQ_BF16>::store(out, i, v);
+    else
+        ElemIO<DQ_F16>::store(out, i, v);
+}
+
+struct SliceScratch {
+    float *vec;
+    double *work;
+    void *signs; // bits, or floats where n is not a multiple of 256
+};
+
+int64_t round_up(int64_t v) { return (v + 255) & ~(int64_t)255; }
+
+SliceScratch slice_scratch(void *p, int64_t n)
+{
+    char *c = static_cast<char *>(p);
+    SliceScratch s;
+    s.vec = reinterpret_cast<float *>(c);
+    s.work = reinterpret_cast<double *>(c + round_up(4 * n));
+    s.signs = c + round_up(4 * n) + round_up(8 * eden_work_doubles(n));
+    return s;
+}
+
+float inv_sqrt_of(int64_t n) { return 1.0f / (float)sqrt((double)n); } // as torch divides by a host scalar on the device
+
+// the diagonal of one rotation into memory; *packed: as bits
+hipError_t write_signs(const SliceScratch &s, int64_t n, int64_t seed, bool *packed, hipStream_t stream)
+{
+    *packed = n % 256 == 0;
+    return *packed ? launch_rand_diag_bits(static_cast<uint32_t *>(s.signs), n, seed, stream)
+                   : launch_rand_diag(static_cast<float *>(s.signs), n, seed, stream);
+}
+
+// one rotation of a slice of at least 1024 elements
+hipError_t rotate(const SliceScratch &s, int64_t n, int64_t seed, int inverse, TransformEnds ends, hipStream_t stream)
+{
+    const void *sign = nullptr;
+    bool packed = false;
+    if (n <= kEdenDrawnSigns) {
+        ends.gen = sign_seed(n, seed);
+    } else {
+        const hipError_t e = write_signs(s, n, seed, &packed, stream);
+        if (e != hipSuccess) return e;
+        sign = s.signs;
+    }
+    return launch_rht_ends(s.vec, sign, packed, n, n, inv_sqrt_of(n), inverse, ends, stream);
+}
+
+} // namespace
+
+int64_t eden_slice_bytes(int64_t n)
+{
+    return round_up(4 * n) + round_up(8 * eden_work_doubles(n)) + round_up(n % 256 == 0 ? n / 8 : 4 * n);
+}
+
+hipError_t launch_eden_compress(const void *src, int dtype, int64_t count, int64_t n, int rotations, int64_t seed,
+                                const float *boundaries, const float *centroids, int nbits, uint32_t *packed, float *result,
+                                void *scratch, hipStream_t stream)
+{
+    const SliceScratch s = slice_scratch(scratch, n);
+    hipError_t e = hipSuccess;
+    if (n < 1024 || rotations == 0) {
+        hipLaunchKernelGGL(eden_pad_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, src, dtype, count, n, s.vec);
+        e = hipGetLastError();
+    }
+    for (int i = 0; e == hipSuccess && i < rotations; i++) {
+        if (n < 1024) {
+            bool bits;
+            e = write_signs(s, n, seed + i, &bits, stream);
+            if (e == hipSuccess) e = launch_rht_blocked(s.vec, s.signs, bits, n, n, inv_sqrt_of(n), 0, stream);
+        } else {
+            TransformEnds ends;
+            if (i == 0) {
+                ends.in_src = src;
+                ends.in_dtype = dtype;
+                ends.in_count = count;
+            }
+            e = rotate(s, n, seed + i, 0, ends, stream);
+        }
+    }
+    if (e != hipSuccess) return e;
+    return launch_eden_quantize(s.vec, n, boundaries, centroids, nbits, packed, result, s.work, stream);
+}
+
+hipError_t launch_eden_decompress(const uint32_t *packed, int64_t n, int rotations, int64_t seed, const float *centroids, int nbits,
+                                  const float *scale, void *out, int dtype, int64_t count, void *scratch, hipStream_t stream)
+{
+    const SliceScratch s = slice_scratch(scratch, n);
+    hipError_t e = hipSuccess;
+    if (n < 1024 || rotations == 0) {
+        e = launch_eden_dequantize(packed, n, centroids, nbits, s.vec, stream);
+        for (int i = 0; e == hipSuccess && i < rotations; i++) {
+            bool bits;
+            e = write_signs(s, n, seed + rotations - 1 - i, &bits, stream);
+            if (e == hipSuccess) e = launch_rht_blocked(s.vec, s.signs, bits, n, n, inv_sqrt_of(n), 1, stream);
+        }
+        if (e != hipSuccess) return e;
+        hipLaunchKernelGGL(eden_finish_kernel, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, stream, s.vec, scale, out, dtype, count);
+        return hipGetLastError();
+    }
+    for (int i = 0; e == hipSuccess && i < rotations; i++) {
+        TransformEnds ends;
+        if (i == 0) {
+            ends.in_planes = packed;
+            ends.in_centroids = centroids;
+            ends.in_nbits = nbits;
+        }
+        if (i == rotations - 1) {
+            ends.post_scale = scale;
+            ends.out_dst = out;
+            ends.out_dtype = dtype;
+            ends.out_count = count;
+        }
+        e = rotate(s, n, seed + rotations - 1 - i, 1, ends, stream);
+    }
+    return e;
+}
+
 } // namespace dq

@@ -246,14 +246,18 @@ static hipError_t fwht_blocks(float *x, const void *sign, bool sign_packed, int6
     a.post_scale = nullptr;
     a.out_levels = nullptr; a.uniform = thc.uniform; a.out_lo = thc.out_lo; a.out_delta = thc.out_delta;
     a.out_top = thc.out_top;
-    const int sign_fwd = (sign && !inverse) ? 1 : 0, sign_inv = (sign && inverse) ? 2 : 0;
+    const bool diagonal = sign || thc.gen.bits != 0;
+    const int sign_fwd = (diagonal && !inverse) ? 1 : 0, sign_inv = (diagonal && inverse) ? 2 : 0;
     // Passes of at least 1024 elements run as the chunk-first kernels of dq_rht_scaling_impl.cuh; a quantiser at an end needs
     // the 16-byte paths there
-    const bool plain = !thc.in_levels && !thc.in_planes && !thc.out_levels && !thc.post_scale;
+    const bool plain = thc.plain();
     const bool ends_ok = plain || (vec16 && (n & 31) == 0 && (reinterpret_cast<uintptr_t>(thc.in_levels) & 15) == 0);
     TransformEnds first = thc, last = thc, none;
-    first.out_levels = nullptr; first.post_scale = nullptr;
-    last.in_levels = nullptr; last.in_planes = nullptr;
+    first.out_levels = nullptr; first.post_scale = nullptr; first.out_dst = nullptr;
+    last.in_levels = nullptr; last.in_planes = nullptr; last.in_src = nullptr;
+    // the diagonal belongs to the first pass of a forward transform and to the last of an inverse one
+    if (inverse) first.gen = SignSeed();
+    else last.gen = SignSeed();
 
     if (kb <= kMaxTileBits) {
         // single pass; small blocks share a tile
@@ -275,7 +279,9 @@ static hipError_t fwht_blocks(float *x, const void *sign, bool sign_packed, int6
     }
 
     // long transform: contiguous pass over the low bits, strided passes above
-    int kt = kPrefTileBits;
+    // (at least four bits are left for the strided pass: fewer would send it to fwht_tile_kernel, which knows neither the
+    // drawn diagonal nor a source or destination of its own)
+    const int kt = kb - kPrefTileBits < 4 ? kb - 4 : kPrefTileBits;
     a.kt = kt; a.b0 = 0; a.b1 = kt; a.cbits = kt; a.sbits = kt;
     a.apply_scale = 0; a.sign_mode = sign_fwd; a.vec = vec16;
     a.in_levels = thc.in_levels;
@@ -303,12 +309,25 @@ static hipError_t fwht_blocks(float *x, const void *sign, bool sign_packed, int6
         if (r >= 4 && ends_ok && (n & (((int64_t)1 << (s + r)) - 1)) == 0)
             e = launch_rht_strided(x, sign, sign_packed ? 1 : 0, n, r, s, scale, a.apply_scale, a.sign_mode, a.vec,
                                    last_pass ? last : none, stream);
+        else if (last_pass && (thc.out_dst || thc.gen.bits != 0 || thc.grid.kind != ThcGrid::POINTERS))
+            e = hipErrorInvalidValue; // (not reached: see above and launch_rht_ends)
         else
             e = launch_tile(a, n >> a.kt, stream);
         if (e != hipSuccess) return e;
         s += r;
     }
     return hipSuccess;
+}
+
+hipError_t launch_rht_ends(float *x, const void *sign, bool sign_packed, int64_t n, int64_t block, float scale, int inverse,
+                           const TransformEnds &ends, hipStream_t stream)
+{
+    // only the passes of dq_rht_scaling_impl.cuh know these ends, and they need the 16-byte paths
+    const uintptr_t every = reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(ends.in_levels) |
+                            reinterpret_cast<uintptr_t>(ends.out_levels) | reinterpret_cast<uintptr_t>(ends.uniform) |
+                            (sign_packed ? 0 : reinterpret_cast<uintptr_t>(sign));
+    if (block < 1024 || n % block != 0 || (every & 15) != 0) return hipErrorInvalidValue;
+    return fwht_blocks(x, sign, sign_packed, n, ilog2(block), scale, 1, inverse, stream, ends);
 }
 
 hipError_t launch_hadamard(float *vec, int64_t n, hipStream_t stream)
@@ -420,6 +439,14 @@ static uint64_t rand_diag_seed(int64_t seed)
     const uint64_t M = 0xffffffffull;
     uint64_t ss = ((uint64_t)seed * 1664525ull + 1013904223ull) & M;
     return (ss * 8121ull + 28411ull) & M;
+}
+
+SignSeed sign_seed(int64_t size, int64_t seed)
+{
+    SignSeed s;
+    s.bits = ilog2(size) - 3;
+    s.ss = (uint32_t)rand_diag_seed(seed);
+    return s;
 }
 
 hipError_t launch_rand_diag(float *out, int64_t size, int64_t seed, hipStream_t stream)

@@ -7,7 +7,7 @@
 // behind document (capi.py, dynamiq_pipeline.py).
 #include <Python.h>
 
-#include <ATen/core/Tensor.h>
+#include <ATen/ATen.h>
 #include <c10/hip/HIPStream.h>
 #include <pybind11/pybind11.h>
 #include <torch/csrc/DynamicTypes.h>
@@ -519,6 +519,139 @@ void ranks_pooled(py::sequence vecs, py::sequence outs, int64_t n, py::handle to
     k.enqueue(stages, a.device, c10::hip::getCurrentHIPStream().stream());
 }
 
+// ---- EDEN and THC (eden.py, thc.py) --------------------------------------------------------------------------
+
+at::Tensor empty_on(int device, int64_t n, at::ScalarType dtype)
+{
+    return at::empty({n}, at::TensorOptions().dtype(dtype).device(at::kCUDA, (c10::DeviceIndex)device));
+}
+
+// Eden.compress: slices as (start, elements, padded size, rotations); returns one (packed, scale) per slice.  The slices run
+// one after the other on the current stream and share one scratch block.
+py::list eden_compress(py::handle vec, py::handle boundaries, py::handle centroids, int nbits, int64_t seed, py::sequence slices)
+{
+    Args a;
+    const at::Tensor &v = a.tensor(vec);
+    const int64_t levels = (int64_t)1 << nbits;
+    const float *b = a.typed(boundaries, at::kFloat, levels - 1, "boundaries").data_ptr<float>();
+    const float *c = a.typed(centroids, at::kFloat, levels, "centroids").data_ptr<float>();
+    const int code = dtype_code(v), elem = (int)v.element_size();
+    struct Slice {
+        int64_t start, count, n;
+        int rotations;
+    };
+    std::vector<Slice> all;
+    int64_t room = 0;
+    for (size_t k = 0; k < py::len(slices); k++) {
+        const py::sequence s = slices[k];
+        const Slice x{py::cast<int64_t>(s[0]), py::cast<int64_t>(s[1]), py::cast<int64_t>(s[2]), py::cast<int>(s[3])};
+        if (x.start < 0 || x.count <= 0 || x.start + x.count > v.numel()) refuse("a slice lies outside the vector");
+        room = std::max(room, dq_eden_slice_bytes(x.n));
+        all.push_back(x);
+    }
+    const dq_stream_t s = c10::hip::getCurrentHIPStream().stream();
+    at::Tensor scratch = empty_on(a.device, room, at::kByte);
+    py::list out;
+    for (const Slice &x : all) {
+        at::Tensor packed = empty_on(a.device, x.n / 32 * nbits, at::kInt), result = empty_on(a.device, 4, at::kFloat);
+        check(dq_eden_compress(static_cast<const char *>(v.data_ptr()) + x.start * elem, code, x.count, x.n, x.rotations, seed, b, c, nbits,
+                               reinterpret_cast<uint32_t *>(packed.data_ptr<int32_t>()), result.data_ptr<float>(), scratch.data_ptr(), room,
+                               a.device, s));
+        out.append(py::make_tuple(py::reinterpret_steal<py::object>(THPVariable_Wrap(packed)),
+                                  py::reinterpret_steal<py::object>(THPVariable_Wrap(result.select(0, 2)))));
+    }
+    return out;
+}
+
+// Eden.decompress: slices as (packed, nbits, centroids, scale, elements, rotations, seed), stored one after the other to out
+void eden_decompress(py::handle out, py::sequence slices)
+{
+    Args a;
+    const at::Tensor &y = a.tensor(out);
+    const int code = dtype_code(y), elem = (int)y.element_size();
+    struct Slice {
+        const uint32_t *packed;
+        const float *centroids, *scale;
+        int64_t n, count, seed;
+        int nbits, rotations;
+    };
+    std::vector<Slice> all;
+    int64_t room = 0, total = 0;
+    for (size_t k = 0; k < py::len(slices); k++) {
+        const py::sequence s = slices[k];
+        Slice x;
+        const at::Tensor &p = a.typed(py::object(s[0]), at::kInt, 1, "packed_bins");
+        x.nbits = py::cast<int>(s[1]);
+        if (x.nbits < 1 || x.nbits > 8) refuse("nbits must be in [1, 8]");
+        x.packed = reinterpret_cast<const uint32_t *>(p.data_ptr<int32_t>());
+        x.n = p.numel() / x.nbits * 32;
+        x.centroids = a.typed(py::object(s[2]), at::kFloat, (int64_t)1 << x.nbits, "centroids").data_ptr<float>();
+        x.scale = a.typed(py::object(s[3]), at::kFloat, 1, "scale").data_ptr<float>();
+        x.count = py::cast<int64_t>(s[4]);
+        x.rotations = py::cast<int>(s[5]);
+        x.seed = py::cast<int64_t>(s[6]);
+        total += x.count;
+        room = std::max(room, dq_eden_slice_bytes(x.n));
+        all.push_back(x);
+    }
+    if (total > y.numel()) refuse("out is too small");
+    const dq_stream_t s = c10::hip::getCurrentHIPStream().stream();
+    at::Tensor scratch = empty_on(a.device, room, at::kByte);
+    char *at = static_cast<char *>(y.data_ptr());
+    for (const Slice &x : all) {
+        check(dq_eden_decompress(x.packed, x.n, x.rotations, x.seed, x.centroids, x.nbits, x.scale, at, code, x.count, scratch.data_ptr(), room,
+                                 a.device, s));
+        at += x.count * elem;
+    }
+}
+
+// norm: a float32 device scalar, with (t, inv_sqrt, inv_levels, inv_clients); or None, with (lo, spacing, step) numbers
+dq_thc_grid_t thc_grid(Args &a, py::handle norm, const py::tuple &numbers)
+{
+    dq_thc_grid_t g;
+    memset(&g, 0, sizeof(g));
+    if (norm.is_none()) {
+        g.lo = py::cast<float>(numbers[0]);
+        g.spacing = py::cast<float>(numbers[1]);
+        g.step = py::cast<float>(numbers[2]);
+    } else {
+        g.norm = a.typed(norm, at::kFloat, 1, "max_norm").data_ptr<float>();
+        g.t = py::cast<float>(numbers[0]);
+        g.inv_sqrt = py::cast<float>(numbers[1]);
+        g.inv_levels = py::cast<float>(numbers[2]);
+        g.inv_clients = py::cast<float>(numbers[3]);
+    }
+    return g;
+}
+
+py::object thc_compress(py::handle src, int64_t count, py::handle work, py::handle bits, py::handle uniform, double scale,
+                        py::handle norm, py::tuple numbers, int levels)
+{
+    Args a;
+    const at::Tensor &x = a.tensor(src), &w = a.tensor(work);
+    const int64_t n = w.numel();
+    if (x.numel() < count || w.scalar_type() != at::kFloat) refuse("thc_compress: a buffer is too small or of the wrong dtype");
+    const uint32_t *sign = reinterpret_cast<const uint32_t *>(a.typed(bits, at::kInt, n / 32, "sign").data_ptr<int32_t>());
+    const float *u = a.typed(uniform, at::kFloat, n, "uniform").data_ptr<float>();
+    const dq_thc_grid_t g = thc_grid(a, norm, numbers);
+    at::Tensor out = empty_on(a.device, n, at::kBFloat16);
+    check(dq_thc_compress(x.data_ptr(), dtype_code(x), count, w.data_ptr<float>(), sign, u, out.data_ptr(), n, (float)scale, &g, levels,
+                          a.device, c10::hip::getCurrentHIPStream().stream()));
+    return py::reinterpret_steal<py::object>(THPVariable_Wrap(out));
+}
+
+void thc_decompress(py::handle levels, py::handle bits, py::handle out, int64_t count, double scale, py::handle norm, py::tuple numbers)
+{
+    Args a;
+    const at::Tensor &y = a.tensor(out);
+    const int64_t n = y.numel();
+    if (y.scalar_type() != at::kFloat) refuse("thc_decompress: out must be float32");
+    const void *l = a.typed(levels, at::kBFloat16, n, "levels").data_ptr();
+    const uint32_t *sign = reinterpret_cast<const uint32_t *>(a.typed(bits, at::kInt, n / 32, "sign").data_ptr<int32_t>());
+    const dq_thc_grid_t g = thc_grid(a, norm, numbers);
+    check(dq_thc_decompress(l, sign, y.data_ptr<float>(), count, n, (float)scale, &g, a.device, c10::hip::getCurrentHIPStream().stream()));
+}
+
 // ---- codec calls on tensors (capi.py) ------------------------------------------------------------------------
 // positional arguments only, no argument-conversion layer: capi.py's functions give them in order
 
@@ -721,6 +854,10 @@ PYBIND11_MODULE(_host, m)
         .def("decompress", &Codec::decompress)
         .def("dec_comp", &Codec::dec_comp);
     m.def("ranks_pooled", &ranks_pooled);
+    m.def("eden_compress", &eden_compress);
+    m.def("eden_decompress", &eden_decompress);
+    m.def("thc_compress", &thc_compress);
+    m.def("thc_decompress", &thc_decompress);
     m.doc() = "native host path of dynamiq_sigcomm_artifact_amd";
     py::class_<Buckets>(m, "Buckets")
         .def(py::init<int, uint64_t, py::object, py::object, py::object>())

@@ -125,6 +125,7 @@ hipError_t launch_add_mean_copy(const void *residual, void *dst, const void *sta
                                 int dtype, hipStream_t stream);
 
 // Walsh-Hadamard (dq_hadamard.hip)
+struct TransformEnds;
 hipError_t launch_hadamard(float *vec, int64_t n, hipStream_t stream);
 // sign: float +-1 values, or (sign_packed) the bit vector of launch_pack_signs; may be null
 hipError_t launch_rht_blocked(float *vec, const void *sign, bool sign_packed, int64_t n, int64_t block, float scale,
@@ -134,6 +135,10 @@ hipError_t launch_rht_blocked(float *vec, const void *sign, bool sign_packed, in
 hipError_t launch_eden_dequantize_irht(const uint32_t *packed, const float *centroids, int nbits, const void *sign,
                                        bool sign_packed, float *out, int64_t n, int64_t block, float scale,
                                        const float *post_scale, hipStream_t stream);
+// rht_blocked with quantisers, a source or a destination of another type at its ends; x (fp32 [n], 16-byte aligned) is
+// where the passes meet and where the result goes unless ends.out_* say otherwise; n a multiple of 1024, block >= 1024
+hipError_t launch_rht_ends(float *x, const void *sign, bool sign_packed, int64_t n, int64_t block, float scale, int inverse,
+                           const TransformEnds &ends, hipStream_t stream);
 hipError_t launch_rand_diag(float *out, int64_t size, int64_t seed, hipStream_t stream);
 // the same diagonal as packed bits (set where the value is -1); size a multiple of 256
 hipError_t launch_rand_diag_bits(uint32_t *bits, int64_t size, int64_t seed, hipStream_t stream);
@@ -155,9 +160,43 @@ hipError_t launch_rht_compress_mfma16(const float *src, const void *sign, int si
                                       float scale, const MeeParams &mp, uint64_t seed, uint64_t step, hipStream_t stream);
 hipError_t launch_irht_decompress(const uint8_t *src, const void *sign, int sign_bits, float *dst, int64_t n, int64_t block,
                                   float scale, int nbits, bool mee, const MeeParams &mp, hipStream_t stream);
+// THC's grid (thc_hooks.py:143-147) where it is not a pair of device scalars: numbers from the host, or worked out from the
+// norm on the device with the operations of torch's float32 scalars in their order -- top = (t * norm) * inv_sqrt, lowest
+// level -top, spacing ((top + top) * inv_levels) + 1e-23, step of an aggregate spacing * inv_clients, the inv_* being
+// float32 reciprocals of host numbers
+struct ThcGrid {
+    enum { POINTERS, HOST, NORM };
+    int kind = POINTERS;
+    float lo = 0.0f, spacing = 0.0f, step = 0.0f;
+    const float *norm = nullptr;
+    float t = 0.0f, inv_sqrt = 0.0f, inv_levels = 0.0f, inv_clients = 0.0f;
+};
+// the diagonal of rand_diag(size, seed), drawn where it is applied; size = 8 * 2^bits >= 1024
+struct SignSeed {
+    int bits = 0; // 0: none
+    uint32_t ss = 0;
+};
+SignSeed sign_seed(int64_t size, int64_t seed);
+
 // Quantisers folded into the two ends of a transform (all null: the plain transform).  `in_*` replace the load of the
 // first pass, `out_*` / `post_scale` act on the store of the last one.
 struct TransformEnds {
+    // the first pass loads in_count elements of in_dtype from in_src, zeros behind them, instead of x
+    const void *in_src = nullptr;
+    int in_dtype = 0;
+    int64_t in_count = 0;
+    // the last pass stores its first out_count elements as out_dtype to out_dst, and nothing to x
+    void *out_dst = nullptr;
+    int out_dtype = 0;
+    int64_t out_count = 0;
+    // THC with the grid worked out in the kernels instead of in_step / in_lo / out_lo / out_delta
+    ThcGrid grid;
+    // the diagonal drawn in the kernels instead of a sign vector
+    SignSeed gen;
+    bool plain_in() const { return !in_src && !in_levels && !in_planes; }
+    bool plain_out() const { return !out_dst && !out_levels && !post_scale; }
+    bool plain() const { return plain_in() && plain_out() && gen.bits == 0; }
+
     // THC: the pass loads float(level) * *in_step + *in_lo instead of x
     const uint16_t *in_levels = nullptr;
     const float *in_step = nullptr, *in_lo = nullptr;
@@ -202,6 +241,14 @@ hipError_t launch_eden_quantize_static(const float *vec, int64_t n, const float 
                                        hipStream_t stream);
 hipError_t launch_eden_dequantize(const uint32_t *packed, int64_t n, const float *centroids, int nbits,
                                   float *out, hipStream_t stream);
+// one slice of EDEN's compress / decompress (srrcomp.py:293-361): count elements of dtype, padded with zeros to n = 2^k >= 32,
+// `rotations` randomized transforms with the diagonals of seed, seed + 1, ...; scratch: eden_slice_bytes(n), 256-byte aligned
+int64_t eden_slice_bytes(int64_t n);
+hipError_t launch_eden_compress(const void *src, int dtype, int64_t count, int64_t n, int rotations, int64_t seed,
+                                const float *boundaries, const float *centroids, int nbits, uint32_t *packed, float *result,
+                                void *scratch, hipStream_t stream);
+hipError_t launch_eden_decompress(const uint32_t *packed, int64_t n, int rotations, int64_t seed, const float *centroids, int nbits,
+                                  const float *scale, void *out, int dtype, int64_t count, void *scratch, hipStream_t stream);
 hipError_t launch_thc_quantize(const float *rotated, const float *uniform, void *out, int64_t n,
                                const float *lo, const float *delta, int levels, hipStream_t stream);
 hipError_t launch_thc_dequantize(const void *levels, float *out, int64_t n, const float *step,

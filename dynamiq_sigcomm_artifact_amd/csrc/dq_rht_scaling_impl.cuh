@@ -56,12 +56,38 @@ struct RhtTileArgs {
     int kb;            // log2 transform block, <= kt
     float scale;
     int vec;           // 16-byte accesses to the fp32 vector and the sign vector allowed
+    SignSeed gen;      // the diagonal drawn here instead (sign is then null); served by flip4 and flip16 only
 };
+
+// Element g of the diagonal of rand_diag (srrcomp.py:61-106; rand_diag_word of dq_hadamard.hip in 32-bit arithmetic: only
+// the low word of every product is used, and the one carry that is, of the addition, is added back by hand).  Four
+// multiplications at a quarter of the rate, about 25 instruction slots per element: cheaper than a launch that writes
+// the bits while the vector is short (the rule is in launch_eden_compress).
+__device__ __forceinline__ uint32_t rand_diag_negative(const SignSeed &s, uint32_t k, uint32_t j)
+{
+    uint32_t r = j + s.ss;
+    r = 1103515245u * r + 12345u + s.ss;
+    r = 1140671485u * r + 12820163u + s.ss;
+    const uint32_t q = r + 0x9e3779b9u;
+    const uint32_t carry = q < r ? 0x10000u : 0u;
+    r = (q ^ ((q >> 16) | carry)) * 0x85ebca6bu;
+    r = (r ^ (r >> 13)) * 0xc2b2ae35u;
+    r ^= r >> 16;
+    return ~(r << (28 - 4 * k)) & 0x80000000u; // +1 where the nibble is >= 8
+}
 
 // the sign flip of elements g .. g + 3 (g a multiple of 4) / of element g.  A packed sign flips the sign bit,
 // which is what the multiplication by -1.0f does to every number
 __device__ __forceinline__ void flip4(float4 &v, const RhtTileArgs &a, int64_t g)
 {
+    if (a.gen.bits != 0) {
+        const uint32_t k = (uint32_t)(g >> a.gen.bits), j = (uint32_t)g & ((1u << a.gen.bits) - 1u); // the four share a segment
+        v.x = __uint_as_float(__float_as_uint(v.x) ^ rand_diag_negative(a.gen, k, j));
+        v.y = __uint_as_float(__float_as_uint(v.y) ^ rand_diag_negative(a.gen, k, j + 1));
+        v.z = __uint_as_float(__float_as_uint(v.z) ^ rand_diag_negative(a.gen, k, j + 2));
+        v.w = __uint_as_float(__float_as_uint(v.w) ^ rand_diag_negative(a.gen, k, j + 3));
+        return;
+    }
     if (!a.sign) return;
     if (a.sign_bits) {
         const uint32_t w = static_cast<const uint32_t *>(a.sign)[g >> 5] >> (g & 31);
@@ -290,12 +316,95 @@ __global__ void irht_decompress_kernel(const uint8_t *__restrict__ src, float *_
 // the sign flip of a chunk that is already in registers (g a multiple of 16; 16-byte accesses to a float sign vector)
 __device__ __forceinline__ void flip16(float (&v)[16], const RhtTileArgs &a, int64_t g)
 {
-    if (!a.sign) return;
+    if (!a.sign && a.gen.bits == 0) return;
 #pragma unroll
     for (int k = 0; k < 4; k++) {
         float4 q = make_float4(v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3]);
         flip4(q, a, g + 4 * k);
         v[4 * k] = q.x; v[4 * k + 1] = q.y; v[4 * k + 2] = q.z; v[4 * k + 3] = q.w;
+    }
+}
+
+// lowest level and spacing of THC's grid
+__device__ __forceinline__ void grid_of(const ThcGrid &d, const float *lo_p, const float *spacing_p, float &lo, float &spacing)
+{
+    if (d.kind == ThcGrid::NORM) {
+        const float a = d.t * *d.norm, top = a * d.inv_sqrt;
+        const float b = (top + top) * d.inv_levels;
+        lo = -top;
+        spacing = b + 1e-23f;
+    } else if (d.kind == ThcGrid::HOST) {
+        lo = d.lo;
+        spacing = d.spacing;
+    } else {
+        lo = *lo_p;
+        spacing = *spacing_p;
+    }
+}
+
+// sixteen elements of a source of another type or length than the transform
+__device__ __forceinline__ void load_source(float (&v)[16], const TransformEnds &e, int64_t g)
+{
+    const bool whole = g + 16 <= e.in_count && (reinterpret_cast<uintptr_t>(e.in_src) & 15) == 0;
+    if (e.in_dtype == DQ_F32) {
+        const float *p = static_cast<const float *>(e.in_src) + g;
+        if (whole) {
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const float4 q = reinterpret_cast<const float4 *>(p)[k];
+                v[4 * k] = q.x; v[4 * k + 1] = q.y; v[4 * k + 2] = q.z; v[4 * k + 3] = q.w;
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < 16; i++) v[i] = g + i < e.in_count ? p[i] : 0.0f;
+        }
+        return;
+    }
+    const uint16_t *p = static_cast<const uint16_t *>(e.in_src) + g;
+    uint32_t w[8];
+    if (whole) {
+        const uint4 a = reinterpret_cast<const uint4 *>(p)[0], b = reinterpret_cast<const uint4 *>(p)[1];
+        w[0] = a.x; w[1] = a.y; w[2] = a.z; w[3] = a.w; w[4] = b.x; w[5] = b.y; w[6] = b.z; w[7] = b.w;
+    } else {
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            w[k] = g + 2 * k < e.in_count ? p[2 * k] : 0u;
+            if (g + 2 * k + 1 < e.in_count) w[k] |= (uint32_t)p[2 * k + 1] << 16;
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        v[2 * k] = e.in_dtype == DQ_BF16 ? bf16_bits_to_f32(w[k] & 0xffffu) : f16_bits_to_f32(w[k] & 0xffffu);
+        v[2 * k + 1] = e.in_dtype == DQ_BF16 ? bf16_bits_to_f32(w[k] >> 16) : f16_bits_to_f32(w[k] >> 16);
+    }
+}
+
+// four elements of a destination of another type or length (out_dst aligned to four elements, or element by element)
+__device__ __forceinline__ void store_destination(const TransformEnds &e, float4 v, int64_t g)
+{
+    if (g >= e.out_count) return;
+    const float f[4] = {v.x, v.y, v.z, v.w};
+    if (e.out_dtype == DQ_F32) {
+        float *p = static_cast<float *>(e.out_dst) + g;
+        if (g + 4 <= e.out_count && (reinterpret_cast<uintptr_t>(e.out_dst) & 15) == 0) {
+            *reinterpret_cast<float4 *>(p) = v;
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                if (g + i < e.out_count) p[i] = f[i];
+        }
+        return;
+    }
+    uint16_t *p = static_cast<uint16_t *>(e.out_dst) + g;
+    uint32_t h[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) h[i] = e.out_dtype == DQ_BF16 ? f32_to_bf16_bits(f[i]) : f32_to_f16_bits(f[i]);
+    if (g + 4 <= e.out_count && (reinterpret_cast<uintptr_t>(e.out_dst) & 7) == 0) {
+        *reinterpret_cast<uint2 *>(p) = make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            if (g + i < e.out_count) p[i] = (uint16_t)h[i];
     }
 }
 
@@ -307,8 +416,9 @@ template <bool ENDS>
 __device__ __forceinline__ void fetch_chunk(float (&v)[16], const float *__restrict__ x, const RhtTileArgs &in,
                                             const TransformEnds &e, const float *cen, int64_t g)
 {
-    if (!ENDS || (!e.in_levels && !e.in_planes)) {
+    if (!ENDS || (!e.in_levels && !e.in_planes && !e.in_src)) {
         load_chunk(v, x, in, g);
+        if (ENDS && in.gen.bits != 0) flip16(v, in, g);
         return;
     }
     if (g >= in.n) {
@@ -316,11 +426,16 @@ __device__ __forceinline__ void fetch_chunk(float (&v)[16], const float *__restr
         for (int i = 0; i < 16; i++) v[i] = 0.0f;
         return;
     }
-    if (e.in_levels) {
+    if (e.in_src) {
+        load_source(v, e, g);
+    } else if (e.in_levels) {
         const uint4 *p = reinterpret_cast<const uint4 *>(e.in_levels + g);
         const uint4 l0 = p[0], l1 = p[1];
         const uint32_t w[8] = {l0.x, l0.y, l0.z, l0.w, l1.x, l1.y, l1.z, l1.w};
-        const float step = *e.in_step, lo = *e.in_lo;
+        float step, lo;
+        grid_of(e.grid, e.in_lo, e.in_step, lo, step);
+        if (e.grid.kind == ThcGrid::NORM) step = step * e.grid.inv_clients;
+        if (e.grid.kind == ThcGrid::HOST) step = e.grid.step;
 #pragma unroll
         for (int k = 0; k < 8; k++) {
             const float p0 = bf16_bits_to_f32(w[k] & 0xffffu) * step, p1 = bf16_bits_to_f32(w[k] >> 16) * step;
@@ -362,11 +477,14 @@ __device__ __forceinline__ void store4(float *__restrict__ x, float4 v, const Rh
     }
     if (ENDS && e.out_levels) {
         const float4 u = *reinterpret_cast<const float4 *>(e.uniform + g);
-        const float lo = *e.out_lo, delta = *e.out_delta;
+        float lo, delta;
+        grid_of(e.grid, e.out_lo, e.out_delta, lo, delta);
         uint2 o;
         o.x = f32x2_to_bf16x2(thc_level(v.x, u.x, lo, delta, e.out_top), thc_level(v.y, u.y, lo, delta, e.out_top));
         o.y = f32x2_to_bf16x2(thc_level(v.z, u.z, lo, delta, e.out_top), thc_level(v.w, u.w, lo, delta, e.out_top));
         *reinterpret_cast<uint2 *>(e.out_levels + g) = o;
+    } else if (ENDS && e.out_dst) {
+        store_destination(e, v, g);
     } else {
         *reinterpret_cast<float4 *>(x + g) = v;
     }
@@ -387,7 +505,10 @@ __global__ void rht_tile_kernel(float *__restrict__ x, RhtTileArgs a, int sign_m
     const int tile = 1 << a.kt;
     const int64_t origin = (int64_t)blockIdx.x << a.kt;
     RhtTileArgs in = a;
-    if (sign_mode != 1) in.sign = nullptr;
+    if (sign_mode != 1) {
+        in.sign = nullptr;
+        in.gen.bits = 0;
+    }
     const float *cen = lds + padded_tile_floats(a.kt); // EDEN's centroids sit behind the tile
     if (ENDS && e.in_planes) {
         for (int k = tid; k < (1 << e.in_nbits); k += nthreads) lds[padded_tile_floats(a.kt) + k] = e.in_centroids[k];
@@ -925,10 +1046,11 @@ hipError_t launch_rht_tile(float *x, const void *sign, int sign_bits, int64_t n,
                            int sign_mode, int vec, const TransformEnds &ends, hipStream_t stream)
 {
     if (kt < 10 || kt > 15 || kb > kt || kb < 0) return hipErrorInvalidValue;
-    const bool plain = !ends.in_levels && !ends.in_planes && !ends.out_levels && !ends.post_scale;
+    const bool plain = ends.plain();
     if (!plain && (!vec || (n & 31) != 0)) return hipErrorInvalidValue;
     RhtTileArgs a;
-    a.sign = sign; a.sign_bits = sign_bits; a.n = n; a.kt = kt; a.kb = kb; a.scale = scale; a.vec = vec;
+    a.sign = sign; a.sign_bits = sign_bits; a.n = n; a.kt = kt; a.kb = kb; a.scale = scale; a.vec = vec; a.gen = ends.gen;
+    const bool diagonal = sign || ends.gen.bits != 0;
     const int tile = 1 << kt;
     if (plain && kt == kSplitBits && kb == kSplitBits && (n & (tile - 1)) == 0) {
         // whole blocks of 2^15: half the LDS, two workgroups per CU
@@ -949,7 +1071,7 @@ hipError_t launch_rht_tile(float *x, const void *sign, int sign_bits, int64_t n,
     } else {
         hipError_t e = allow_lds(rht_tile_kernel<true>, lds);
         if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(rht_tile_kernel<true>, grid, dim3(threads), lds, stream, x, a, sign ? sign_mode : 0, apply_scale, ends);
+        hipLaunchKernelGGL(rht_tile_kernel<true>, grid, dim3(threads), lds, stream, x, a, diagonal ? sign_mode : 0, apply_scale, ends);
     }
     return hipGetLastError();
 }
@@ -959,10 +1081,10 @@ hipError_t launch_rht_strided(float *x, const void *sign, int sign_bits, int64_t
                               int apply_scale, int sign_mode, int vec, const TransformEnds &ends, hipStream_t stream)
 {
     if (rbits < 4 || rbits > 10 || sbits < 5 || (n & (((int64_t)1 << (sbits + rbits)) - 1)) != 0) return hipErrorInvalidValue;
-    const bool plain = !ends.out_levels && !ends.post_scale;
+    const bool plain = ends.plain_out() && ends.gen.bits == 0;
     if (!plain && !vec) return hipErrorInvalidValue;
     RhtTileArgs a;
-    a.sign = sign; a.sign_bits = sign_bits; a.n = n; a.kt = rbits + 5; a.kb = 0; a.scale = scale; a.vec = vec;
+    a.sign = sign; a.sign_bits = sign_bits; a.n = n; a.kt = rbits + 5; a.kb = 0; a.scale = scale; a.vec = vec; a.gen = ends.gen;
     const int tile = 1 << (rbits + 5);
     const unsigned threads = (unsigned)std::min(1024, tile / 16);
     const size_t lds = (size_t)padded_tile_floats(rbits + 5) * sizeof(float);
@@ -975,7 +1097,7 @@ hipError_t launch_rht_strided(float *x, const void *sign, int sign_bits, int64_t
     } else {
         hipError_t e = allow_lds(rht_strided_kernel<true>, lds);
         if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(rht_strided_kernel<true>, grid, dim3(threads), lds, stream, x, a, rbits, sbits, sign ? sign_mode : 0,
+        hipLaunchKernelGGL(rht_strided_kernel<true>, grid, dim3(threads), lds, stream, x, a, rbits, sbits, sign || ends.gen.bits != 0 ? sign_mode : 0,
                            apply_scale, ends);
     }
     return hipGetLastError();

@@ -2,10 +2,10 @@
 (cuda_kernels/src/srrcomp/srrcomp.py:13-447): the same slicing rule, the same
 ``compress`` / ``decompress`` signatures and the same per-slice dictionaries, with
 
-  * randDiag + Hadamard + 1/sqrt(n) in one launch per rotation (``rht_blocked``),
-  * ``_quantize`` + ``EdenBinsToBits`` in one call (``eden_quantize``: norm, bucketize,
-    bit planes, dot product and scale on the device, no host synchronisation),
-  * ``EdenBitsToBins`` + the centroid lookup in one call (``eden_dequantize``).
+  * one native call for all slices of a vector in either direction (``dq_eden_compress``, ``dq_eden_decompress``): the
+    rotations read the caller's vector and type directly, pad, and draw the diagonal themselves,
+  * norm, bucketize, bit planes, dot product and scale on the device, no host synchronisation,
+  * the bit planes decoded in the load of the inverse rotation, scale and type conversion in its store.
 
 Tables.  The reference carries its Lloyd-Max tables as literals.  Here the centroids
 are computed: the stationary point of the Lloyd-Max conditions for N(0, 1) with
@@ -21,6 +21,7 @@ import torch
 from . import capi
 
 _TABLES = {}
+_STORED = {torch.float32, torch.bfloat16, torch.float16}        # what the kernels read and store themselves
 
 
 def _conditional_means(c):
@@ -120,7 +121,9 @@ class Eden(SRRCompUtils):
     # ---- srrcomp.py:251-291 ----
     def compress(self, vec, nbits, seed):
         vec_type = vec.dtype
-        vec = vec.to(self.device, torch.float32).clone()        # the kernels only take buffers of self.device
+        if vec_type not in _STORED:
+            vec = vec.to(torch.float32)
+        vec = vec.to(self.device).contiguous()                  # the kernels only take buffers of self.device
 
         def low_po2(n):
             return 2 ** int(np.log2(n)) if n else 0
@@ -128,60 +131,19 @@ class Eden(SRRCompUtils):
         def high_po2(n):
             return 2 ** (int(np.ceil(np.log2(n)))) if n else 0
 
-        res = []
+        slices = []                                             # (start, elements, padded size, rotations)
         dim = remaining = vec.numel()
         curr_index = 0
         while (high_po2(remaining) - remaining) / dim > self.max_padding_overhead:
             low = low_po2(remaining)
-            num_hadamard = 1 + (low < 2 ** 10)
-            res.append(self._compress_slice(vec[curr_index: curr_index + low], vec_type, nbits, num_hadamard, seed))
+            slices.append((curr_index, low, max(low, 32), 1 + (low < 2 ** 10)))
             curr_index += low
             remaining -= low
-        num_hadamard = 1 + (dim - curr_index < 2 ** 10)
-        res.append(self._compress_slice(vec[curr_index:], vec_type, nbits, num_hadamard, seed))
-        return res
-
-    @staticmethod
-    def _inv_sqrt(n):
-        # the divisor of `Hadamard(vec) / np.sqrt(n)` as torch applies a host scalar on the device: a product
-        # with the float32 reciprocal
-        return float(np.float32(1.0) / np.float32(math.sqrt(n)))
-
-    # the diagonal of randDiag (srrcomp.py:61-106): one bit per element where the size allows it (multiples of 256),
-    # the float vector otherwise -- the transform takes either
-    def _diag_buffer(self, n):
-        if n % 256 == 0:
-            return torch.empty(n // 32, dtype=torch.int32, device=self.device)
-        return torch.empty(n, dtype=torch.float32, device=self.device)
-
-    @staticmethod
-    def _rand_diag(diag, n, seed):
-        if diag.dtype == torch.int32:
-            capi.rand_diag_bits(diag, n, seed)
-        else:
-            capi.rand_diag(diag, seed)
-
-    # ---- srrcomp.py:293-326 ----
-    def _compress_slice(self, vec, vec_type, nbits, num_hadamard, seed):
-        orig_dim = n = vec.numel()
-        if not n & (n - 1) == 0 or n < 32:
-            padded_dim = max(int(2 ** (np.ceil(np.log2(n)))), 32)
-            padded = torch.zeros(padded_dim, device=self.device)
-            padded[:n] = vec
-            n, vec = padded_dim, padded
-        else:
-            vec = vec.contiguous().clone()
-        diag = self._diag_buffer(n)
-        for i in range(num_hadamard):
-            self._rand_diag(diag, n, seed + i)
-            capi.rht_blocked(vec, diag, n, self._inv_sqrt(n), False)
+        slices.append((curr_index, remaining, max(high_po2(remaining), 32), 1 + (remaining < 2 ** 10)))
         centroids, boundaries = self._tables(nbits)
-        packed = torch.empty(n // 32 * nbits, dtype=torch.int32, device=self.device)
-        result = torch.empty(4, dtype=torch.float32, device=self.device)
-        work = torch.empty(capi.eden_work_doubles(n), dtype=torch.float64, device=self.device)
-        capi.eden_quantize(vec, boundaries, centroids, nbits, packed, result, work)
-        return {"packed_bins": packed, "vec_type": vec_type, "nbits": nbits, "scale": result[2], "orig_dim": orig_dim,
-                "num_hadamard": num_hadamard, "seed": seed}
+        parts = capi.host().eden_compress(vec, boundaries, centroids, nbits, seed, slices)
+        return [{"packed_bins": packed, "vec_type": vec_type, "nbits": nbits, "scale": scale, "orig_dim": count,
+                 "num_hadamard": rotations, "seed": seed} for (packed, scale), (_, count, _, rotations) in zip(parts, slices)]
 
     # ---- srrcomp.py:356-361 ----
     def _quantize(self, vec, nbits):
@@ -200,30 +162,18 @@ class Eden(SRRCompUtils):
 
     # ---- srrcomp.py:328-354 ----
     def decompress(self, data):
-        return torch.cat([self._decompress_slice(d["packed_bins"], d["vec_type"], d["nbits"], d["scale"], d["orig_dim"],
-                                                 d["num_hadamard"], d["seed"]) for d in data])
-
-    def _decompress_slice(self, packed_bins, vec_type, nbits, scale, orig_dim, num_hadamard, seed):
-        n = packed_bins.numel() // nbits * 32
-        centroids, _ = self._tables(nbits)
-        vec = torch.empty(n, dtype=torch.float32, device=self.device)
-        if num_hadamard == 0:
-            capi.eden_dequantize(packed_bins.to(self.device, torch.int32), n, centroids, nbits, vec)
-            return (scale * vec)[:orig_dim].to(vec_type)
-        # the dequantiser rides on the first pass of the first rotation, the product with the scale on the last pass of
-        # the last one: same bits as eden_dequantize, the rotations and `scale * vec`
-        scale32 = scale.reshape(1).to(device=self.device, dtype=torch.float32) if isinstance(scale, torch.Tensor) else \
-            torch.tensor([scale], dtype=torch.float32, device=self.device)
-        diag = self._diag_buffer(n)
-        for i in range(num_hadamard):
-            self._rand_diag(diag, n, seed + num_hadamard - 1 - i)
-            last = scale32 if i == num_hadamard - 1 else None
-            if i == 0:
-                capi.eden_dequantize_irht(packed_bins.to(self.device, torch.int32), n, centroids, nbits, diag, vec, n, self._inv_sqrt(n),
-                                          post_scale=last)
-            elif last is None:
-                capi.rht_blocked(vec, diag, n, self._inv_sqrt(n), True)
-            else:
-                capi.rht_blocked(vec, diag, n, self._inv_sqrt(n), True)
-                vec = scale32 * vec
-        return vec[:orig_dim].to(vec_type)
+        stored = {d["vec_type"] for d in data}
+        dtype = next(iter(stored)) if len(stored) == 1 and stored <= _STORED else torch.float32
+        slices = []
+        for d in data:
+            scale = d["scale"]
+            scale = scale.reshape(1).to(device=self.device, dtype=torch.float32) if isinstance(scale, torch.Tensor) else \
+                torch.tensor([scale], dtype=torch.float32, device=self.device)
+            slices.append((d["packed_bins"].to(self.device, torch.int32).contiguous(), d["nbits"], self._tables(d["nbits"])[0], scale,
+                           d["orig_dim"], d["num_hadamard"], d["seed"]))
+        out = torch.empty(sum(d["orig_dim"] for d in data), dtype=dtype, device=self.device)
+        capi.host().eden_decompress(out, slices)
+        if stored <= {dtype}:
+            return out
+        # slices of several types (or of one the kernels do not store): each in its own, put together as torch does
+        return torch.cat([part.to(d["vec_type"]) for part, d in zip(out.split([d["orig_dim"] for d in data]), data)])

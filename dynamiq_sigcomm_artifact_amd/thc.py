@@ -23,6 +23,7 @@ import torch
 
 from . import capi
 
+_READ = {torch.float32, torch.bfloat16, torch.float16}         # what the transform's first pass reads itself
 _TABLE_FILE = "{table_size}_tablesize_{max_val}_maxval_16_qlevels_{overflow_frequency}_ofreq_data.txt"
 _TABLE_DEFAULTS = {"table_size": 10001, "max_val": 42, "overflow_frequency": 1024}
 
@@ -131,18 +132,38 @@ class OldINCACudaHadamardCompressor:
             return v.to(device=device, dtype=torch.float32).reshape(1)
         return torch.tensor([v], dtype=torch.float32, device=device)
 
+    def _native_grid(self, max_norm, dim):
+        """the grid for the native calls: (device norm or None, numbers), worked out in the kernels from a float32 norm on
+        the device (the same operations), on the host from a number; None where torch has to (norms of other types)"""
+        reciprocal = lambda v: float(np.float32(1.0) / np.float32(v))      # what torch's division by a host scalar uses
+        if isinstance(max_norm, torch.Tensor):
+            if max_norm.dtype != torch.float32 or not max_norm.is_cuda or max_norm.numel() != 1:
+                return None
+            return max_norm, (self.data["T"], reciprocal(math.sqrt(dim)), reciprocal(self.quantization_levels - 1), reciprocal(self.nclients))
+        low, spacing = self._grid(max_norm, dim)
+        return None, (low, spacing, spacing / self.nclients)
+
     def compress(self, tensor, name, max_norm, uniform=None):
         dim, used = self.ds[name], self.original_size[name]
         self.max_norm_dict[name] = max_norm
         work = self._buffer(name, "work")
+        if uniform is None:
+            uniform = self._buffer(name, "uniform").uniform_(0.0, 1.0, generator=self.sender_prng)
+        rot = self.hadamards[name]
+        grid = self._native_grid(max_norm, dim) if dim >= 1024 and uniform.data_ptr() % 16 == 0 else None
+        if grid is not None:
+            # the transform's first pass reads the caller's tensor, in its own type where the kernels know it
+            if tensor.dim() != 1 or tensor.numel() != used or not tensor.is_cuda or not tensor.is_contiguous() or \
+                    tensor.dtype not in _READ:
+                work[:used].copy_(tensor.float())
+                tensor = work
+            return capi.host().thc_compress(tensor, used, work, rot.diagonal_bits, uniform, rot.inv_sqrt, grid[0], grid[1],
+                                            self.quantization_levels)
         work[:used].copy_(tensor.float())
         if dim > used:
             work[used:].zero_()
         low, spacing = self._grid(max_norm, dim)
-        if uniform is None:
-            uniform = self._buffer(name, "uniform").uniform_(0.0, 1.0, generator=self.sender_prng)
         levels = torch.empty(dim, dtype=torch.bfloat16, device=self.device)
-        rot = self.hadamards[name]
         capi.thc_rht_quantize(work, rot.diagonal_bits, uniform, levels, dim, rot.inv_sqrt, self._scalar(low, self.device),
                               self._scalar(spacing, self.device), self.quantization_levels)
         return levels
@@ -151,9 +172,13 @@ class OldINCACudaHadamardCompressor:
         if max_norm is None:
             max_norm = self.max_norm_dict[name]
         dim, used = self.ds[name], self.original_size[name]
-        low, spacing = self._grid(max_norm, dim)
         out = self._buffer(name, "work")
         rot = self.hadamards[name]
+        grid = self._native_grid(max_norm, dim) if dim >= 1024 and tensor.data_ptr() % 16 == 0 else None
+        if grid is not None:
+            capi.host().thc_decompress(tensor, rot.diagonal_bits, out, used, rot.inv_sqrt, grid[0], grid[1])
+            return out[:used]
+        low, spacing = self._grid(max_norm, dim)
         capi.thc_dequantize_irht(tensor, rot.diagonal_bits, out, dim, rot.inv_sqrt,
                                  self._scalar(spacing / self.nclients, self.device), self._scalar(low, self.device))
         return out[:used]

@@ -551,6 +551,45 @@ int dq_eden_dequantize_irht(const uint32_t *packed, int64_t n, const float *cent
                             float scale, const float *post_scale, int device,
                             dq_stream_t stream);
 
+/* srrcomp.py:293-326 / :328-354, one slice in one call: `count` elements of
+ * dtype (any of the three), padded with zeros to n = 2^k >= 32, go through
+ * `rotations` randomized transforms (the diagonals of seed, seed + 1, ... as
+ * dq_rand_diag makes them, the scale 1 / sqrt(n)) and dq_eden_quantize; and the
+ * way back, scaled by *scale and stored as `count` elements of dtype.  The same
+ * bits as the single calls; the slice is not copied or converted in memory and
+ * the diagonal of a short slice never written.  scratch: dq_eden_slice_bytes(n)
+ * bytes, 256-byte aligned, contents undefined before and after. */
+int64_t dq_eden_slice_bytes(int64_t n);
+int dq_eden_compress(const void *src, int dtype, int64_t count, int64_t n, int rotations, int64_t seed,
+                     const float *boundaries, const float *centroids, int nbits, uint32_t *packed, float *result,
+                     void *scratch, int64_t scratch_bytes, int device, dq_stream_t stream);
+int dq_eden_decompress(const uint32_t *packed, int64_t n, int rotations, int64_t seed, const float *centroids, int nbits,
+                       const float *scale, void *out, int dtype, int64_t count, void *scratch, int64_t scratch_bytes,
+                       int device, dq_stream_t stream);
+
+/* THC's grid of levels (thc_hooks.py:143-147): numbers of the host (norm NULL:
+ * lo, spacing, step of an aggregate), or worked out in the kernels from a
+ * float32 norm in device memory: top = (t * *norm) * inv_sqrt, lo = -top,
+ * spacing = ((top + top) * inv_levels) + 1e-23, step = spacing * inv_clients --
+ * torch's operations on a float32 scalar, divisions by host numbers being
+ * products with their float32 reciprocals. */
+typedef struct dq_thc_grid {
+    const float *norm;
+    float t, inv_sqrt, inv_levels, inv_clients;
+    float lo, spacing, step;
+} dq_thc_grid_t;
+
+/* thc_hooks.py:149-166 / :168-181 in one call for one vector of n = 2^k >= 1024
+ * elements (one transform block): dq_thc_rht_quantize reading `count` elements
+ * of dtype straight from src, zeros behind them; dq_thc_dequantize_irht storing
+ * the first `count` elements only (out: n floats, the others hold intermediate
+ * values).  sign_bits: dq_pack_signs.  16-byte aligned buffers (not src). */
+int dq_thc_compress(const void *src, int dtype, int64_t count, float *work, const uint32_t *sign_bits, const float *uniform,
+                    void *levels_bf16, int64_t n, float scale, const dq_thc_grid_t *grid, int levels, int device,
+                    dq_stream_t stream);
+int dq_thc_decompress(const void *levels_bf16, const uint32_t *sign_bits, float *out, int64_t count, int64_t n, float scale,
+                      const dq_thc_grid_t *grid, int device, dq_stream_t stream);
+
 /* thc_hooks.py:176-178: out = float(levels) * *step + *lo (two roundings). */
 int dq_thc_dequantize(const void *levels_bf16, float *out, int64_t n, const float *step,
                       const float *lo, int device, dq_stream_t stream);

@@ -351,3 +351,77 @@ def test_srrcomp_utils_surface(capi, oracle):
     # against torch's own ops away from the boundaries: at most a handful of bins differ by the rounding of the quotient
     ref = torch.bucketize(v * (n ** 0.5) / torch.norm(v, 2), bnd)
     assert int((ref != q_bins).sum()) <= 2
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n", [1, 33, 1000, 1024, 1500, 4097, 32768 - 7, 65536, 100003, (1 << 22) + (1 << 20), (1 << 23) - 5])
+def test_slices_in_one_call_equal_the_single_calls(capi, n, dt):
+    """compress and decompress of a vector whose slices are tiny, ragged, of one pass and of two, with drawn and with written
+    diagonals, aligned and not, against the calls they stand for: padding, rand_diag, rht_blocked, eden_quantize; and back"""
+    import math
+    from dynamiq_sigcomm_artifact_amd.eden import Eden
+    dev = "cuda:0"
+    eden = Eden(device=dev)
+    g = torch.Generator(device=dev).manual_seed(n)
+    nbits, seed = 3 + n % 3, 17
+    vec = (torch.randn(n + 1, generator=g, device=dev) * 1e-2).to(dt)[n & 1:][:n]
+    print("case", n, dt, flush=True)
+    data = eden.compress(vec, nbits, seed)
+    assert sum(d["orig_dim"] for d in data) == n
+    centroids, boundaries = eden._tables(nbits)
+    at, want = 0, []
+    for d in data:
+        size = d["packed_bins"].numel() // nbits * 32
+        inv = float(np.float32(1.0) / np.float32(math.sqrt(size)))
+        x = torch.zeros(size, device=dev)
+        x[:d["orig_dim"]] = vec[at:at + d["orig_dim"]].float()
+        at += d["orig_dim"]
+        diags = []
+        for i in range(d["num_hadamard"]):
+            diags.append(torch.empty(size, device=dev))
+            capi.rand_diag(diags[-1], seed + i)
+            capi.rht_blocked(x, diags[-1], size, inv, False)
+        packed = torch.empty(size // 32 * nbits, dtype=torch.int32, device=dev)
+        result = torch.empty(4, device=dev)
+        capi.eden_quantize(x, boundaries, centroids, nbits, packed, result, torch.empty(capi.eden_work_doubles(size), dtype=torch.float64, device=dev))
+        assert torch.equal(packed, d["packed_bins"]) and torch.equal(result[2].view(torch.int32), d["scale"].view(torch.int32))
+        y = torch.empty(size, device=dev)
+        capi.eden_dequantize(packed, size, centroids, nbits, y)
+        for diag in reversed(diags):
+            capi.rht_blocked(y, diag, size, inv, True)
+        want.append((result[2] * y)[:d["orig_dim"]].to(dt))
+    got = eden.decompress(data)
+    assert got.dtype == dt and torch.equal(got, torch.cat(want))
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n,dim", [(1024, 1024), (40000, 65536), (1 << 20, 1 << 20), (1000, 1024), ((1 << 21) + 5, 1 << 22)])
+def test_thc_grid_and_source_in_the_passes(capi, n, dim, dt):
+    """THC's compress and decompress with the grid from a norm on the device, from a number, and as torch works it out
+    (a norm of another type takes the single calls); sources of another type, length and alignment than the transform"""
+    from dynamiq_sigcomm_artifact_amd.thc import OldINCACudaHadamardCompressor
+    dev = "cuda:0"
+    c = OldINCACudaHadamardCompressor({"d": {(0, 1): dim}, "size": {(0, 1): n}, "T": 2.7, "device": dev, "nclients": 6, "rank": 0})
+    g = torch.Generator(device=dev).manual_seed(dim)
+    x = torch.randn(n + 1, generator=g, device=dev).to(dt)[n & 1:][:n]
+    norm = x.float().norm()
+    u = torch.rand(dim, generator=g, device=dev)
+    name = (0, 1)
+    levels = c.compress(x, name, norm, uniform=u)
+    work = torch.zeros(dim, device=dev)
+    work[:n] = x.float()
+    low, spacing = c._grid(norm, dim)
+    want = torch.empty(dim, dtype=torch.bfloat16, device=dev)
+    rot = c.hadamards[name]
+    capi.thc_rht_quantize(work, rot.diagonal_bits, u, want, dim, rot.inv_sqrt, low.reshape(1), spacing.reshape(1), 64)
+    assert torch.equal(levels, want)
+    total = (levels.float() * 6).to(torch.bfloat16)
+    got = c.decompress(total, name).clone()
+    back = torch.empty(dim, device=dev)
+    capi.thc_dequantize_irht(total, rot.diagonal_bits, back, dim, rot.inv_sqrt, (spacing / 6).reshape(1), low.reshape(1))
+    assert got.numel() == n and torch.equal(got, back[:n])
+    host = c.compress(x, name, float(norm), uniform=u)                         # the grid from a number: rounded once
+    assert (host.float() - want.float()).abs().max() <= 1 and (host != want).float().mean() < 1e-3
+    assert (c.decompress(total, name) - got).norm() < 1e-5 * got.norm()
+    double = c.compress(x, name, norm.double(), uniform=u)
+    assert (double != host).float().mean() < 1e-3
