@@ -25,6 +25,23 @@ __device__ __forceinline__ int64_t qbits_of_norm(uint32_t norm_bits, float u)
     return (int64_t)1 << z;
 }
 
+// The same width as a class (0: 8 bits, 1: 4, 2: 2) for all lanes of a wave, most of the time without the rule's seventy
+// instructions: the score s = scale log2(F) + u decides (below 4: 2 bits, below 8: 4, else 8) unless it lies near 4 or 8.
+// The rule rounds to bf16 four times in front of its comparison with 4 or 8 (F is bf16 already): log2 F to 2^-9 of at most
+// 67 for the F taken here, times the scale 0.133 -> 0.018; the product, at most 8.9, to 2^-9 of it -> 0.018; the sum near
+// 8 -> 0.016; and the second log2, of a number near 8, rounds to 3 from 2^-8 below -> a factor 2^(1/256) of s, 0.022.
+// Together 0.074; the hardware's log2 and the products here add less than 1e-4.  A band of 0.125 is kept.
+__device__ __forceinline__ int width_class_of_norm(uint32_t norm_bits, float u)
+{
+    const float f = bf16_bits_to_f32(norm_bits);
+    const float s = __builtin_fmaf(__builtin_amdgcn_logf(f), (float)(4.0 / (512.0 / 17.0)), u);
+    const float off = __builtin_fminf(__builtin_fabsf(s - 4.0f), __builtin_fabsf(s - 8.0f));
+    // (NaN fails both comparisons)
+    if (__builtin_amdgcn_ballot_w64(!(f >= 0x1p-60f && f <= 0x1p60f && off >= 0.125f)) == 0) return s < 4.0f ? 2 : (s < 8.0f ? 1 : 0);
+    const int64_t q = qbits_of_norm(norm_bits, u);
+    return q == 8 ? 0 : (q == 4 ? 1 : 2);
+}
+
 constexpr int kMaxPattern = 0x7f80; // +infinity: the patterns 0 .. 0x7f80 are the non-negative norms in ascending order
 
 // The width is a monotone step function of the bf16 norm pattern (every operation of the rule is monotone, and

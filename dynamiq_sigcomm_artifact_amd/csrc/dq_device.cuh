@@ -259,6 +259,16 @@ struct MeeParams {
 
 // ---- counter-based random stream ----------------------------------------------------
 
+// a ^ b ^ c in one instruction (the compiler makes two of it)
+__host__ __device__ __forceinline__ uint32_t xor3(uint32_t a, uint32_t b, uint32_t c)
+{
+#ifdef __HIP_DEVICE_COMPILE__
+    return __builtin_amdgcn_bitop3_b32(a, b, c, 0x96);
+#else
+    return a ^ b ^ c;
+#endif
+}
+
 // Philox4x32-10 (Salmon et al., SC'11): counter c, key (k0, k1)
 __host__ __device__ __forceinline__ void philox4x32_10(uint32_t (&c)[4], uint32_t k0, uint32_t k1)
 {
@@ -266,9 +276,9 @@ __host__ __device__ __forceinline__ void philox4x32_10(uint32_t (&c)[4], uint32_
     for (int r = 0; r < 10; r++) {
         const uint64_t p0 = (uint64_t)0xD2511F53u * c[0];
         const uint64_t p1 = (uint64_t)0xCD9E8D57u * c[2];
-        const uint32_t n0 = (uint32_t)(p1 >> 32) ^ c[1] ^ k0;
+        const uint32_t n0 = xor3((uint32_t)(p1 >> 32), c[1], k0);
         const uint32_t n1 = (uint32_t)p1;
-        const uint32_t n2 = (uint32_t)(p0 >> 32) ^ c[3] ^ k1;
+        const uint32_t n2 = xor3((uint32_t)(p0 >> 32), c[3], k1);
         const uint32_t n3 = (uint32_t)p0;
         c[0] = n0; c[1] = n1; c[2] = n2; c[3] = n3;
         k0 += 0x9E3779B9u;

@@ -62,9 +62,10 @@ __device__ __forceinline__ void store_tile(void *dst, const Raw16<DT> &out, cons
                     stream_store(reinterpret_cast<uint4 *>(bytes + e * ESZ), val);
                 } else {
                     const uint32_t part[4] = {val.x, val.y, val.z, val.w};
+                    const int left = left_here(n, e, EP);
 #pragma unroll
                     for (int i = 0; i < EP; i++) {
-                        if (e + i < n) {
+                        if (i < left) {
                             if (DT == DQ_F32)
                                 reinterpret_cast<uint32_t *>(bytes)[e + i] = part[i];
                             else
@@ -76,9 +77,10 @@ __device__ __forceinline__ void store_tile(void *dst, const Raw16<DT> &out, cons
         }
     } else if ((lane >> 4) < rows_here) {
         const int64_t e = sc * 256 + (lane & 15) * 16;
+        const int left = left_here(n, e, 16);
 #pragma unroll
         for (int i = 0; i < 16; i++) {
-            if (e + i < n) {
+            if (i < left) {
                 if (DT == DQ_F32)
                     reinterpret_cast<uint32_t *>(bytes)[e + i] = out.w[i];
                 else
@@ -118,8 +120,9 @@ struct WidthRule {
 };
 
 struct RoundtripArgs {
-    uint32_t first_tile[kMaxBuckets]; // ascending; 2^32 - 1 behind the last bucket
+    uint32_t first_tile[kMaxBuckets]; // ascending
     RoundtripBucket bucket[kMaxBuckets];
+    int buckets;
     WidthRule rule;
     WorldDiv wd;
     uint64_t seed;
@@ -132,8 +135,22 @@ __device__ __forceinline__ int class_of_norm(uint32_t pattern, float u, const in
 {
     if (thr[0] >= 0 && __builtin_amdgcn_ballot_w64(pattern > (uint32_t)kMaxPattern) == 0)
         return (int)pattern >= thr[1] ? 0 : ((int)pattern >= thr[0] ? 1 : 2);
-    const int64_t q = qbits_of_norm(pattern, u);
-    return q == 8 ? 0 : (q == 4 ? 1 : 2);
+    return width_class_of_norm(pattern, u);
+}
+
+// the last entry of an ascending list that is <= x, by halving (scalar: as a sum of comparisons over the whole list it
+// becomes sixty vector instructions)
+__device__ __forceinline__ int last_at_most(const uint32_t *list, int count, uint32_t x)
+{
+    int lo = 0, hi = count - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (list[mid] <= x)
+            lo = mid;
+        else
+            hi = mid - 1;
+    }
+    return lo;
 }
 
 template <int DT, bool MEE> __global__ __launch_bounds__(64) void roundtrip_kernel(RoundtripArgs a)
@@ -145,21 +162,19 @@ template <int DT, bool MEE> __global__ __launch_bounds__(64) void roundtrip_kern
 
     uint64_t step = a.step_dev ? *a.step_dev + a.step_more : 0;
     const float u = a.rule.u_dev ? (float)*a.rule.u_dev : a.rule.u;
-    int at = 0;
-#pragma unroll
-    for (int k = 1; k < kMaxBuckets; k++) at += blockIdx.x >= a.first_tile[k] ? 1 : 0;
+    const int at = last_at_most(a.first_tile, a.buckets, blockIdx.x);
     const RoundtripBucket &b = a.bucket[at];
     const int64_t n = b.n, nsc = (n + 255) >> 8;
     const int64_t sc0 = (int64_t)(blockIdx.x - a.first_tile[at]) * kRowsPerWave;
     if (sc0 >= nsc) return;
     const int rows_here = (int)min((int64_t)kRowsPerWave, nsc - sc0);
-    const bool active = row < rows_here;
+    const bool active = row < rows_here, ragged = (sc0 + kRowsPerWave) * 256 > n;
     const int64_t sc = sc0 + min(row, rows_here - 1);
     const int64_t e0 = sc * 256 + j * 16;
 
     Raw16<DT> v;
     v.zero();
-    if (active) load_chunk<DT>(v, b.src, e0, n, b.vec != 0);
+    if (active) load_chunk<DT>(v, b.src, e0, n, b.vec != 0, ragged);
     if (MEE) levels_to_lds(a.widths, levels, lane);
     // the rounding stream's arithmetic while the elements are on their way
     Raw16<DQ_PHILOX> r;
@@ -168,14 +183,14 @@ template <int DT, bool MEE> __global__ __launch_bounds__(64) void roundtrip_kern
 
     float sum, sq;
     tile_sums<DT>(v, a.wd, lds, lane, sum, sq);
-    const float mean = __shfl(superchunk_mean(sum, min((int64_t)256, n - sc * 256)), lane & 48, 64);
+    const float mean = __shfl(superchunk_mean(sum, sc * 256, n, ragged), lane & 48, 64);
     const uint32_t norm = (uint32_t)__shfl((int)f32_to_bf16_bits(sq), lane & 48, 64);
     const uint32_t mean_bits = f32_to_bf16_bits(mean);
     if (active && j == 0) b.stats[sc] = mean_bits | (norm << 16);
     if (sc0 == 0 && lane < 4) b.counts[lane] = 0; // (tally_kernel adds to them)
 
     const WidthRegs<MEE> w = width_regs<MEE>(a.widths, class_of_norm(norm, u, a.rule.thr), levels);
-    center_loaded<DT>(v, a.wd, active ? mean : 0.0f, e0, n);
+    center_loaded<DT>(v, a.wd, active ? mean : 0.0f, e0, n, ragged);
     float lev[16];
     const float scale = quantize_chunk<MEE>(v, r, w, lev);
     decode_with_mean<DT>(v, lev, scale, bf16_bits_to_f32(mean_bits));
@@ -193,6 +208,7 @@ struct TallyBucket {
 struct TallyArgs {
     uint32_t first_block[kMaxBuckets];
     TallyBucket bucket[kMaxBuckets];
+    int buckets;
     WidthRule rule;
     uint32_t *hist;
     uint64_t *step_dev;
@@ -207,9 +223,7 @@ template <bool HIST> __global__ __launch_bounds__(kTallyThreads) void tally_kern
     __shared__ int thr[2];
     __shared__ uint32_t total[2];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    int at = 0;
-#pragma unroll
-    for (int k = 1; k < kMaxBuckets; k++) at += blockIdx.x >= a.first_block[k] ? 1 : 0;
+    const int at = last_at_most(a.first_block, a.buckets, blockIdx.x);
     const TallyBucket b = a.bucket[at];
     const int64_t begin = (int64_t)(blockIdx.x - a.first_block[at]) * kHistBatch;
     const int64_t end = min(begin + (int64_t)kHistBatch, b.nsc);
@@ -287,16 +301,17 @@ __global__ __launch_bounds__(64 * kStatsWaves) void ranks_stats_kernel(RankPoint
     const int64_t sc0 = (int64_t)blockIdx.x * kRowsPerWave;
     const int rows_here = (int)min((int64_t)kRowsPerWave, nsc - sc0);
     const int64_t sc = sc0 + min(row, rows_here - 1);
+    const bool ragged = (sc0 + kRowsPerWave) * 256 > n;
     uint8_t *lds = tiles + wave * StatsTile<DT>::BYTES;
     for (int rank = wave; rank < world; rank += waves) {
         Raw16<DT> v;
         v.zero();
-        if (row < rows_here) load_chunk<DT>(v, ranks.src[rank], sc * 256 + j * 16, n, vec != 0);
+        if (row < rows_here) load_chunk<DT>(v, ranks.src[rank], sc * 256 + j * 16, n, vec != 0, ragged);
         float sum, sq;
         tile_sums<DT>(v, wd, lds, lane, sum, sq);
         wave_lds_sync();
         if (j == 0) {
-            const float mean = superchunk_mean(sum, min((int64_t)256, n - sc * 256));
+            const float mean = superchunk_mean(sum, sc * 256, n, ragged);
             pairs[rank][row] = f32_to_bf16_bits(mean) | (f32_to_bf16_bits(sq) << 16);
             if (row < rows_here) mean_out[rank * nsc + sc] = mean;
         }
@@ -374,6 +389,7 @@ template <int DT, int RDT, bool MEE> __global__ __launch_bounds__(64) void ring_
     const bool active = row < rows_here;
     const int64_t sc = a.order[row0 + k0 + min(row, rows_here - 1)];
     const int64_t e0 = sc * 256 + j * 16;
+    const bool ragged = __builtin_amdgcn_ballot_w64(e0 + 16 > a.n) != 0;
     if (MEE) levels_to_lds(a.widths, levels, lane);
     const WidthRegs<MEE> w = width_regs<MEE>(a.widths, cls, levels);
     const uint32_t total_mean = a.total[2 * sc];
@@ -388,7 +404,7 @@ template <int DT, int RDT, bool MEE> __global__ __launch_bounds__(64) void ring_
         int rank = chunk + step;
         if (rank >= world) rank -= world;
         if (active) {
-            load_chunk<DT>(next, a.src[rank], e0, a.n, a.vec & 1);
+            load_chunk<DT>(next, a.src[rank], e0, a.n, a.vec & 1, ragged);
             next_mean = a.mean[(int64_t)rank * a.nsc + sc];
             if constexpr (RDT != DQ_PHILOX)
                 next_r.load(a.pools.pool[cls][rank], ((int64_t)a.pools.first[cls][rank][step] + k0 * 16 + lane) * 16, (a.vec & 4) != 0);
@@ -408,7 +424,7 @@ template <int DT, int RDT, bool MEE> __global__ __launch_bounds__(64) void ring_
             if (rank >= world) rank -= world;
             r.generate(RandKey{a.key.seed + (uint64_t)rank, (uint64_t)step}, sc * 16 + j);
         }
-        center_loaded<DT>(v, a.wd, mean, e0, a.n);
+        center_loaded<DT>(v, a.wd, mean, e0, a.n, ragged);
         if (step > 0) {
 #pragma unroll
             for (int i = 0; i < 16; i++) lev[i] = __builtin_fmaf(lev[i], scale, v.get(i));
@@ -444,10 +460,7 @@ hipError_t launch_roundtrip(const RoundtripDesc *desc, int count, int world, flo
     memset(&a, 0, offsetof(RoundtripArgs, rule));
     uint32_t tiles = 0, blocks = 0;
     for (int k = 0; k < kMaxBuckets; k++) {
-        if (k >= count) {
-            a.first_tile[k] = t.first_block[k] = 0xffffffffu;
-            continue;
-        }
+        if (k >= count) break;
         const RoundtripDesc &d = desc[k];
         const int64_t nsc = (d.n + 255) / 256;
         a.first_tile[k] = tiles;
@@ -458,6 +471,7 @@ hipError_t launch_roundtrip(const RoundtripDesc *desc, int count, int world, flo
         tiles += (uint32_t)((nsc + kRowsPerWave - 1) / kRowsPerWave);
         blocks += (uint32_t)((nsc + kHistBatch - 1) / kHistBatch);
     }
+    a.buckets = t.buckets = count;
     a.rule = t.rule = make_rule(u, u_dev);
     a.wd = make_world_div(world, dtype == DQ_F32 ? 4 : 2);
     a.seed = seed;

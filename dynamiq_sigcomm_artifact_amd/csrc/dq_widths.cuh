@@ -16,7 +16,7 @@ struct WidthConst {
     double inv_top;            // 1 / R (AEE) or 1 / chunk_max_mee (MEE)
     double inv_c, inv_l2b;     // MEE
     float r;                   // R = 2^(bits - 1) - 1
-    float bias, two_delta;     // of the code estimate: R + 1 + kDelta, 2 kDelta (estimate_codes)
+    float bias, two_delta;     // of the level estimate: 1 + kDelta, 2 kDelta
     float c, cmm, l2b;         // MEE
 };
 
@@ -28,7 +28,7 @@ struct WidthSet {
     uint16_t levels[280]; // MEE: binary16 level tables of the three widths end to end
 };
 
-// one width's constants in registers; table: its levels as floats in LDS (MEE)
+// one width's constants in registers; table: its level zero among the floats in LDS (MEE)
 template <bool MEE> struct WidthRegs {
     double inv_top, inv_c, inv_l2b;
     float r, bias, two_delta, c, cmm, l2b;
@@ -49,7 +49,7 @@ template <bool MEE> __device__ __forceinline__ WidthRegs<MEE> width_regs(const W
         x.c = pick(s.w[0].c, s.w[1].c, s.w[2].c);
         x.cmm = pick(s.w[0].cmm, s.w[1].cmm, s.w[2].cmm);
         x.l2b = pick(s.w[0].l2b, s.w[1].l2b, s.w[2].l2b);
-        x.table = levels + pick(kLevels[0], kLevels[1], kLevels[2]);
+        x.table = levels + pick(kLevels[0] + 127, kLevels[1] + 7, kLevels[2] + 1);
     } else {
         x.inv_c = x.inv_l2b = 0.0;
         x.c = x.cmm = x.l2b = 0.0f;
@@ -96,13 +96,15 @@ __device__ __forceinline__ float quantize_guarded(const RV &v, const RR &rnd, co
     for (int i = 0; i < 16; i++) {
         float x = v.get(i) / d;
         if (MEE) x = mee_inverse_guarded(x, w.c, w.l2b);
-        const int code = clamp_code(sr_guarded(x, rnd.get(i)), top);
-        lev[i] = MEE ? w.table[code] : (float)(code - top);
+        const int level = clamp_code(sr_guarded(x, rnd.get(i)), top) - top;
+        lev[i] = MEE ? w.table[level] : (float)level;
     }
     return nonneg_scale((float)qi * nonneg_scale(bf16_bits_to_f32(unit_bits)));
 }
 
-// chunk_encode_fast + estimate_codes: elements finite and <= 2^100, random values in [0, 1]
+// chunk_encode_fast + estimate_codes: elements finite and <= 2^100, random values in [0, 1].  The estimate is that of
+// L - r + 1 instead of L - r + R + 1 -- its floor is the signed level -- against the same guard: the constant 1 + kDelta
+// minus r is as exact (1 and 20 bits of fraction), and the fused multiply-add rounds a number of less magnitude.
 template <bool MEE, class RV, class RR>
 __device__ __forceinline__ float quantize_fast(const RV &v, const RR &rnd, uint32_t amax_bits, const WidthRegs<MEE> &w, float (&lev)[16])
 {
@@ -114,10 +116,8 @@ __device__ __forceinline__ float quantize_fast(const RV &v, const RR &rnd, uint3
     const float d = (float)qi * unit;
     const float rd = __builtin_amdgcn_rcpf(d);
     const float rc = MEE ? (float)w.inv_c : 0.0f, rl2b = MEE ? (float)w.inv_l2b : 0.0f;
-    const float two_r = w.r + w.r;
     bool doubt[16];
     uint64_t lanes_in_doubt[16], any = 0;
-    float code[16];
 #pragma unroll
     for (int i = 0; i < 16; i++) {
         const float vi = v.get(i);
@@ -131,8 +131,7 @@ __device__ __forceinline__ float quantize_fast(const RV &v, const RR &rnd, uint3
         doubt[i] = fr < w.two_delta;
         lanes_in_doubt[i] = __builtin_amdgcn_ballot_w64(doubt[i]);
         any |= lanes_in_doubt[i];
-        // floor(t); -1 < t < 2 R + 2, so the two bounds are the clamp of the code
-        code[i] = __builtin_amdgcn_fmed3f(t - fr, 0.0f, two_r);
+        lev[i] = __builtin_amdgcn_fmed3f(t - fr, -w.r, w.r); // t - fr = floor(t), exact
     }
     if (any != 0) {
         const double yd = recip_f64(d);
@@ -140,12 +139,14 @@ __device__ __forceinline__ float quantize_fast(const RV &v, const RR &rnd, uint3
         for (int i = 0; i < 16; i++) {
             if (lanes_in_doubt[i] != 0) {
                 const float sv = (float)exact_code_fast<MEE>(v.get(i), rnd.get(i), d, yd, w);
-                if (doubt[i]) code[i] = __builtin_amdgcn_fmed3f(sv, -w.r, w.r) + w.r;
+                if (doubt[i]) lev[i] = __builtin_amdgcn_fmed3f(sv, -w.r, w.r);
             }
         }
     }
+    if (MEE) {
 #pragma unroll
-    for (int i = 0; i < 16; i++) lev[i] = MEE ? w.table[(int)code[i]] : code[i] - w.r;
+        for (int i = 0; i < 16; i++) lev[i] = w.table[(int)lev[i]];
+    }
     return nonneg_scale((float)qi * nonneg_scale(unit));
 }
 
@@ -171,7 +172,7 @@ inline WidthSet make_width_set(const MeeParams *mp, bool mee)
         // EstimateGuard: kDelta of estimate_codes
         const float delta = mee ? (bits[k] >= 6 ? 0x1p-12f : 0x1p-14f) : (float)(1 << (bits[k] - 1)) * 0x1p-20f;
         w.r = (float)top;
-        w.bias = (float)(top + 1) + delta;
+        w.bias = 1.0f + delta;
         w.two_delta = 2.0f * delta;
         w.c = mp[k].c; w.cmm = mp[k].cmm; w.l2b = mp[k].l2b;
         w.inv_top = mee ? 1.0 / (double)mp[k].cmm : 1.0 / (double)top;
@@ -184,24 +185,41 @@ inline WidthSet make_width_set(const MeeParams *mp, bool mee)
 
 // ---- a lane's chunk at the ragged end of a vector ------------------------------------------------------
 
+// Elements of a vector of n at and behind e (at most `most`, at least 0), where only the ragged end of the vector or an
+// unaligned buffer looks at it: written as comparisons of e + i with n -- sixteen of 64 bits per chunk -- the compiler moves
+// them out of that branch, in front of every tile (about 60 of the 270 vector instructions of a wave of ranks_stats_kernel).
+__device__ __forceinline__ int left_here(int64_t n, int64_t e, int most)
+{
+    asm volatile("" : "+s"(n));
+    return (int)max((int64_t)0, min((int64_t)most, n - e));
+}
+
+// Every element is loaded, those beyond the end from the last one's address, and then masked: sixteen loads in flight
+// together.  (Each behind its own comparison they went one by one, and the one ragged wave of a launch outlasted the others:
+// 4 of 26 us on 8 x 1,000,003 elements.)
 template <int DT> __device__ __forceinline__ void load_chunk_guarded(Raw16<DT> &v, const void *src, int64_t e0, int64_t n)
 {
+    typedef typename ElemIO<DT>::storage elem;
+    const int left = left_here(n, e0, 16), last = max(left - 1, 0);
+    const elem *p = static_cast<const elem *>(src) + min(e0, n - 1);
+    elem x[16];
+#pragma unroll
+    for (int i = 0; i < 16; i++) x[i] = p[min(i, last)];
     v.zero();
 #pragma unroll
     for (int i = 0; i < 16; i++) {
-        if (e0 + i < n) {
-            if (DT == DQ_F32)
-                v.w[i] = static_cast<const uint32_t *>(src)[e0 + i];
-            else
-                v.w[i >> 1] |= (uint32_t) static_cast<const uint16_t *>(src)[e0 + i] << (16 * (i & 1));
-        }
+        if (DT == DQ_F32)
+            v.w[i] = i < left ? __builtin_bit_cast(uint32_t, (float)x[i]) : 0u;
+        else
+            v.w[i >> 1] |= (i < left ? (uint32_t)x[i] : 0u) << (16 * (i & 1));
     }
 }
 
-// elements [e0, e0 + 16) of src, zero at and beyond n
-template <int DT> __device__ __forceinline__ void load_chunk(Raw16<DT> &v, const void *src, int64_t e0, int64_t n, bool vec)
+// elements [e0, e0 + 16) of src, zero at and beyond n; ragged: the wave's tile reaches beyond n (uniform)
+template <int DT>
+__device__ __forceinline__ void load_chunk(Raw16<DT> &v, const void *src, int64_t e0, int64_t n, bool vec, bool ragged)
 {
-    if (e0 + 16 <= n)
+    if (!ragged)
         v.load(src, e0, vec);
     else
         load_chunk_guarded<DT>(v, src, e0, n);
@@ -209,7 +227,7 @@ template <int DT> __device__ __forceinline__ void load_chunk(Raw16<DT> &v, const
 
 // v becomes T(v / world - mean), zero at and beyond element n of the vector (center_chunk without its own loads)
 template <int DT>
-__device__ __forceinline__ void center_loaded(Raw16<DT> &v, const WorldDiv &wd, float mean, int64_t e0, int64_t n)
+__device__ __forceinline__ void center_loaded(Raw16<DT> &v, const WorldDiv &wd, float mean, int64_t e0, int64_t n, bool ragged)
 {
     float t[16];
     if (DT != DQ_F32 && wd.fuse16) {
@@ -225,9 +243,10 @@ __device__ __forceinline__ void center_loaded(Raw16<DT> &v, const WorldDiv &wd, 
 #pragma unroll
         for (int i = 0; i < 16; i++) t[i] -= mean;
     }
-    if (e0 + 16 > n) {
+    if (ragged) {
+        const int left = left_here(n, e0, 16);
 #pragma unroll
-        for (int i = 0; i < 16; i++) t[i] = e0 + i < n ? t[i] : 0.0f;
+        for (int i = 0; i < 16; i++) t[i] = i < left ? t[i] : 0.0f;
     }
     v.set(t);
 }
@@ -301,6 +320,11 @@ __device__ __forceinline__ void tile_sums(const Raw16<DT> &v, const WorldDiv &wd
 }
 
 // the mean the reference divides out: sum / 256 exactly, or by the count of a ragged last superchunk
-__device__ __forceinline__ float superchunk_mean(float sum, int64_t valid) { return valid >= 256 ? sum * 0.00390625f : sum / (float)valid; }
+__device__ __forceinline__ float superchunk_mean(float sum, int64_t first, int64_t n, bool ragged)
+{
+    if (!ragged) return sum * 0.00390625f;
+    const int valid = left_here(n, first, 256);
+    return valid >= 256 ? sum * 0.00390625f : sum / (float)valid;
+}
 
 } // namespace dq

@@ -684,3 +684,23 @@ def test_ranks_in_registers_equal_the_ring_in_steps(capi, W, n, dt):
         u_dev = torch.full((1,), u, dtype=torch.float64, device=DEV)
         again, _, _ = dynamic_bitrate_allreduce_single_pass(vecs, u_dev, strategy=strategy, seed=11)
         assert all(torch.equal(bits_t(x), bits_t(y)) for x, y in zip(again, ref))
+
+
+@pytest.mark.parametrize("u", [-4.0, 0.0, 3.984375, 6.0, 8.0, 15.5])
+def test_widths_of_every_norm_in_the_one_rank_pass(capi, u):
+    """the width that the one-rank pass picks by its quick score equals the width rule's for every bf16 norm from 2^-63 to 2^62 --
+    each fills one wave (four superchunks), so that no other norm sends the wave to the rule itself"""
+    from dynamiq_sigcomm_artifact_amd.dynamiq_pipeline import SinglePassBuckets
+    norms = torch.arange(64 << 7, (189 << 7) + 1, dtype=torch.int16, device=DEV).view(torch.bfloat16).float()
+    norms = torch.cat([norms.repeat_interleave(4), torch.tensor([0.0, float("inf")], device=DEV).repeat_interleave(4)])
+    signs = torch.tensor([1.0, -1.0], device=DEV).repeat(128)
+    x = (norms[:, None] / 16 * signs).reshape(-1).contiguous()      # 256 elements of +-norm / 16: mean zero
+    out = torch.zeros_like(x)
+    pipe = SinglePassBuckets(DEV, strategy=2, seed=5, streams=1, u=u)
+    pipe.begin_step()
+    pipe.run(x, out)
+    pipe.join()
+    torch.cuda.synchronize()
+    work, _, want = _four_calls(capi, x, x.numel(), u, 2, 5, 1)[3:]
+    assert torch.equal(bits_t(out), bits_t(want))
+    assert pipe.counts(0)[:3].tolist() == work[:3].tolist()
