@@ -127,11 +127,12 @@ __device__ __forceinline__ float quantize_fast(const RV &v, const RR &rnd, uint3
             t = __builtin_fmaf(__builtin_amdgcn_logf(__builtin_fmaf(__builtin_fabsf(vi * rd), rc, 1.0f)), __builtin_copysignf(rl2b, vi), off);
         else
             t = __builtin_fmaf(vi, rd, off);
-        const float fr = __builtin_amdgcn_fractf(t);
-        doubt[i] = fr < w.two_delta;
+        // (floor and not t minus its fraction: in -2^-25 < t < 0 the fraction rounds to 1 - 2^-24 and the difference is not -1)
+        const float fl = __builtin_floorf(t);
+        doubt[i] = t - fl < w.two_delta;
         lanes_in_doubt[i] = __builtin_amdgcn_ballot_w64(doubt[i]);
         any |= lanes_in_doubt[i];
-        lev[i] = __builtin_amdgcn_fmed3f(t - fr, -w.r, w.r); // t - fr = floor(t), exact
+        lev[i] = __builtin_amdgcn_fmed3f(fl, -w.r, w.r);
     }
     if (any != 0) {
         const double yd = recip_f64(d);

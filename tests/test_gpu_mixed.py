@@ -704,3 +704,27 @@ def test_widths_of_every_norm_in_the_one_rank_pass(capi, u):
     work, _, want = _four_calls(capi, x, x.numel(), u, 2, 5, 1)[3:]
     assert torch.equal(bits_t(out), bits_t(want))
     assert pipe.counts(0)[:3].tolist() == work[:3].tolist()
+
+
+@pytest.mark.parametrize("bits,u", [(8, 60.0), (2, -60.0)])
+def test_estimates_just_below_zero_round_down(capi, bits, u):
+    """elements whose rounding estimate falls a few 2^-25 around zero, where the fraction of a negative number rounds up to one:
+    the one-rank pass against the four calls"""
+    from dynamiq_sigcomm_artifact_amd.dynamiq_pipeline import SinglePassBuckets
+    nsc, top = 4096, float(2 ** (bits - 1) - 1)
+    rnd = torch.empty(nsc * 256, dtype=torch.float32, device=DEV)
+    capi.philox_uniform(rnd, 5, 1)
+    step = 255 * torch.tensor((1.0 + 1e-7) / 255).to(torch.bfloat16).double().item()      # of a chunk with maximum `top`
+    jitter = 1 + (torch.arange(nsc * 256, device=DEV) // 2 % 13 - 6).double() * 2.0 ** -24
+    x = (step * (rnd.double() - 1 - 2.0 ** (bits - 21)) * jitter).float().view(-1, 16)
+    x[:, 0] = top
+    x[:, 1::2] = -x[:, 0::2]                                        # pairs: mean zero
+    x = x.reshape(-1).contiguous()
+    out = torch.zeros_like(x)
+    pipe = SinglePassBuckets(DEV, strategy=2, seed=5, streams=1, u=u)
+    pipe.begin_step()
+    pipe.run(x, out)
+    pipe.join()
+    torch.cuda.synchronize()
+    assert pipe.counts(0).tolist() == [nsc if bits == w else 0 for w in (8, 4, 2)] + [0]
+    assert torch.equal(out, _four_calls(capi, x, x.numel(), u, 2, 5, 1)[5])
