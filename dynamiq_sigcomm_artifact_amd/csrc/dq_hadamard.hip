@@ -225,6 +225,22 @@ constexpr int kMaxTileBits = 15; // 2^15 floats = 128 KiB (+ padding) of the 160
 constexpr int kPrefTileBits = 13; // 32 KiB tiles keep several workgroups per CU in flight
 constexpr int kStridedCols = 5;   // 32 consecutive floats (128 B) per row of a strided tile
 
+// How a transform of 2^kb > 2^15 elements is divided: index bits of the contiguous pass, the rest go to strided passes.
+// Both passes are bound by memory (or, short, by how many workgroups there are to hide its latency), so the tiles should be
+// small enough for several workgroups per CU and there should be two passes:
+//   up to 2^18  128 rows per strided tile (16 KB): the vector has only 32 to 128 tiles of that size
+//   to 2^22     256 rows (32 KB), and the contiguous tiles grow with the vector
+//   to 2^25     1024 rows, the most that fit the LDS: anything less makes three passes of it from 2^24 on
+//   beyond      three passes in any case, 32 KB contiguous tiles
+// In place, against 2^13 everywhere: 2^18 9.1 -> 8.2 us, 2^19 10.0 -> 9.4, 2^22 27.3 -> 20.5, 2^24 65.3 -> 54.9,
+// 2^25 127 -> 112; 2^20, 2^21 and 2^23 keep theirs to within 2%.
+static int contiguous_bits(int kb)
+{
+    if (kb <= 18) return kb - 7 < 10 ? 10 : kb - 7;
+    if (kb <= 22) return kb - 8;
+    return kb <= 25 ? kb - 10 : kPrefTileBits;
+}
+
 // transform index bits [0, kb) of every aligned block of 2^kb elements of x[0..n); `thc`: quantisers at the ends
 typedef TransformEnds ThcEnds;
 
@@ -281,7 +297,7 @@ static hipError_t fwht_blocks(float *x, const void *sign, bool sign_packed, int6
     // long transform: contiguous pass over the low bits, strided passes above
     // (at least four bits are left for the strided pass: fewer would send it to fwht_tile_kernel, which knows neither the
     // drawn diagonal nor a source or destination of its own)
-    const int kt = kb - kPrefTileBits < 4 ? kb - 4 : kPrefTileBits;
+    const int kt = contiguous_bits(kb);
     a.kt = kt; a.b0 = 0; a.b1 = kt; a.cbits = kt; a.sbits = kt;
     a.apply_scale = 0; a.sign_mode = sign_fwd; a.vec = vec16;
     a.in_levels = thc.in_levels;

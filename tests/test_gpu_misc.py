@@ -87,6 +87,14 @@ def test_hadamard_whole_vector(capi, oracle, k):
     _eq("fwht 2^%d" % k, x_d.cpu().numpy(), oracle.fwht(x.numpy()))
 
 
+def test_hadamard_of_the_longest_two_passes(capi, oracle):
+    g = torch.Generator().manual_seed(25)
+    x = torch.randn(1 << 25, generator=g)
+    x_d = x.to(DEV)
+    capi.hadamard(x_d)
+    _eq("fwht 2^25", x_d.cpu().numpy(), oracle.fwht(x.numpy()))
+
+
 def test_hadamard_identities(capi):
     """H(e_i) = i-th Walsh row (+-1), H(1) = n e_0, H(H(x)) = n x on small integers"""
     n = 1 << 14
