@@ -36,7 +36,7 @@ HIP_SOURCES = [
     "dq_superchunk.hip",
     "dq_hadamard.hip",
     "dq_packing.hip",
-    "dq_eden.hip",
+    "dq_eden.hip", "dq_eden_short.hip",
     "dq_streams.hip",
     "dq_io_floor.hip",
 ]

@@ -907,41 +907,44 @@ int dq_eden_dequantize(const uint32_t *packed, int64_t n, const float *centroids
 
 int64_t dq_eden_slice_bytes(int64_t n) { return n >= 32 && (n & (n - 1)) == 0 ? dq::eden_slice_bytes(n) : 0; }
 
-static int check_eden_slice(int64_t count, int64_t n, int dtype, int rotations, int nbits, int64_t scratch_bytes, const void *scratch)
+static int check_eden_slices(const dq_eden_slice_t *s, int count, int dtype, bool compress, const void *scratch, int64_t scratch_bytes)
 {
-    if (n < 32 || (n & (n - 1)) != 0) return fail(DQ_ERR_POW2, "the padded size of a slice (at least 32)");
-    if (!(count > 0) || count > n) return fail(DQ_ERR_SIZE, "count must lie in [1, n]");
+    if (!s || !scratch) return fail(DQ_ERR_NULL);
+    if (count < 1) return fail(DQ_ERR_SIZE, "no slices");
     if (!dtype_ok(dtype)) return fail(DQ_ERR_DTYPE);
-    if (nbits < 1 || nbits > 8) return fail(DQ_ERR_NBITS, "nbits must be in [1, 8]");
-    if (rotations < 0) return fail(DQ_ERR_SIZE, "rotations must not be negative");
-    if (!scratch) return fail(DQ_ERR_NULL);
-    if (scratch_bytes < dq::eden_slice_bytes(n) || (reinterpret_cast<uintptr_t>(scratch) & 255))
-        return fail(DQ_ERR_SIZE, "scratch must be 256-byte aligned and hold dq_eden_slice_bytes");
+    int64_t bytes = 0;
+    for (int k = 0; k < count; k++) {
+        if (s[k].n < 32 || (s[k].n & (s[k].n - 1)) != 0) return fail(DQ_ERR_POW2, "the padded size of a slice (at least 32)");
+        if (!(s[k].count > 0) || s[k].count > s[k].n) return fail(DQ_ERR_SIZE, "count must lie in [1, n]");
+        if (s[k].nbits < 1 || s[k].nbits > 8) return fail(DQ_ERR_NBITS, "nbits must be in [1, 8]");
+        if (s[k].rotations < 0) return fail(DQ_ERR_SIZE, "rotations must not be negative");
+        if (!s[k].vec || !s[k].packed || !s[k].result || !s[k].centroids || (compress && !s[k].boundaries)) return fail(DQ_ERR_NULL);
+        if (compress && (s[k].nbits != s[0].nbits || s[k].boundaries != s[0].boundaries || s[k].centroids != s[0].centroids))
+            return fail(DQ_ERR_SIZE, "the slices of a compress call share nbits and tables");
+        bytes += dq::eden_slice_bytes(s[k].n);
+    }
+    if (scratch_bytes < bytes || (reinterpret_cast<uintptr_t>(scratch) & 255))
+        return fail(DQ_ERR_SIZE, "scratch must be 256-byte aligned and hold dq_eden_slice_bytes of every slice");
     return DQ_OK;
 }
 
-int dq_eden_compress(const void *src, int dtype, int64_t count, int64_t n, int rotations, int64_t seed, const float *boundaries,
-                     const float *centroids, int nbits, uint32_t *packed, float *result, void *scratch, int64_t scratch_bytes,
-                     int device, dq_stream_t stream)
-{
-    int rc = check_eden_slice(count, n, dtype, rotations, nbits, scratch_bytes, scratch);
-    if (rc) return rc;
-    if (!src || !boundaries || !centroids || !packed || !result) return fail(DQ_ERR_NULL);
-    if ((rc = select_device(device))) return rc;
-    return finish(dq::launch_eden_compress(src, dtype, count, n, rotations, seed, boundaries, centroids, nbits, packed, result, scratch,
-                                           static_cast<hipStream_t>(stream)));
-}
-
-int dq_eden_decompress(const uint32_t *packed, int64_t n, int rotations, int64_t seed, const float *centroids, int nbits,
-                       const float *scale, void *out, int dtype, int64_t count, void *scratch, int64_t scratch_bytes, int device,
+static int eden_slices(const dq_eden_slice_t *slices, int count, int dtype, bool decompress, void *scratch, int64_t scratch_bytes, int device,
                        dq_stream_t stream)
 {
-    int rc = check_eden_slice(count, n, dtype, rotations, nbits, scratch_bytes, scratch);
+    int rc = check_eden_slices(slices, count, dtype, !decompress, scratch, scratch_bytes);
     if (rc) return rc;
-    if (!packed || !centroids || !scale || !out) return fail(DQ_ERR_NULL);
     if ((rc = select_device(device))) return rc;
-    return finish(dq::launch_eden_decompress(packed, n, rotations, seed, centroids, nbits, scale, out, dtype, count, scratch,
-                                             static_cast<hipStream_t>(stream)));
+    return finish(dq::launch_eden_slices(slices, count, dtype, decompress, scratch, static_cast<hipStream_t>(stream)));
+}
+
+int dq_eden_compress(const dq_eden_slice_t *slices, int count, int dtype, void *scratch, int64_t scratch_bytes, int device, dq_stream_t stream)
+{
+    return eden_slices(slices, count, dtype, false, scratch, scratch_bytes, device, stream);
+}
+
+int dq_eden_decompress(const dq_eden_slice_t *slices, int count, int dtype, void *scratch, int64_t scratch_bytes, int device, dq_stream_t stream)
+{
+    return eden_slices(slices, count, dtype, true, scratch, scratch_bytes, device, stream);
 }
 
 static int thc_ends(const dq_thc_grid_t *g, dq::TransformEnds &ends)

@@ -3,62 +3,67 @@
 // (testbed_evaluation/new_comm_hooks/thc_hooks.py:149-181), which the reference runs as chains of
 // torch element-wise ops and reductions around eden_utils.Hadamard.
 //
-// EDEN quantise, four launches (three for vectors of up to 2^22 elements, where every workgroup of `bins` folds the
-// partial sums of `sumsq` itself instead of waiting for a launch of one workgroup to do it), no host synchronisation:
+// EDEN quantise, three launches, no host synchronisation:
 //   sumsq   tile b = elements [4096 b, 4096 b + 4096): thread t adds v^2 of elements t + 256 k (k ascending)
 //           in double, the 256 sums are halved (stride 128 .. 1) -> work[b]
-//   norm    one workgroup folds work[] the same way -> sumsq (double); norm = sqrtf((float)sumsq)
-//   bins    x = (v * (float)sqrt(n)) / norm; bin = number of boundaries b with !(b >= x) (torch.bucketize, right=False: NaN -> last bin);
+//   bins    every workgroup folds work[] the same way -> sumsq (double); norm = sqrtf((float)sumsq);
+//           x = (v * (float)sqrt(n)) / norm; bin = number of boundaries b with !(b >= x) (torch.bucketize, right=False: NaN -> last bin);
 //           bit plane p of 32 consecutive bins -> packed[p * n/32 + w]; the products centroid[bin] * v are
-//           summed in double, thread t adding elements 16 t + k of the tile (k ascending), then halved -> work[b]
-//   scale   dot = fold(work[]); scale = (norm * norm) / (float)dot
+//           summed in double, thread t adding elements 16 t + k of the tile (k ascending), then halved -> work[tiles + b]
+//   scale   dot = fold(work[tiles ..]); scale = (norm * norm) / (float)dot
+// Beyond 2^22 elements the fold of sumsq is a launch of its own (eden_norm_kernel): in every workgroup it would read more
+// than the workgroup's own elements; the products then go to work[b].
+// (scale inside bins, by the workgroup that finishes last: its release of the other XCDs' sums costs more than the launch --
+// bins 5.7 -> 10.8 us at 2^20 elements, against 1.8 us for scale.)
 // The sums are in double with a fixed association, so the result does not depend on the launch geometry
 // and the CPU restatement reproduces it bit for bit.
 #include <mutex>
+#include <vector>
 
+#include "dq_eden.cuh"
 #include "dq_launch.h"
-#include "dq_tile16.cuh"
 
 namespace dq {
 
 namespace {
 
-constexpr int kEdenThreads = 256;
-constexpr int kEdenPerThread = 16;
-constexpr int kEdenTile = kEdenThreads * kEdenPerThread; // 4096 elements
+// several slices in one launch: slice k owns the workgroups from first[k] on, one per tile
+struct QuantizeSet {
+    QuantizeSlice s[kMaxEdenSlices];
+    unsigned first[kMaxEdenSlices];
+    int count;
+};
 
-// sum[l] += sum[l + stride], stride 128 .. 1; returns the total in every thread
-__device__ __forceinline__ double fold256(double v, double *lds)
+__device__ __forceinline__ int slice_of_block(const unsigned *first, int count)
 {
-    const int t = threadIdx.x;
-    lds[t] = v;
-    __syncthreads();
-#pragma unroll
-    for (int stride = 128; stride > 0; stride >>= 1) {
-        if (t < stride) lds[t] += lds[t + stride];
-        __syncthreads();
-    }
-    const double total = lds[0];
-    __syncthreads();
-    return total;
+    int k = 0;
+    for (int i = 1; i < count; i++)
+        if (blockIdx.x >= first[i]) k = i;
+    return k;
 }
 
-__global__ __launch_bounds__(kEdenThreads) void eden_sumsq_kernel(const float *__restrict__ vec, int64_t n,
-                                                                 double *__restrict__ work)
+// A whole tile's loads leave together; behind a comparison each they wait for one another (6.9 -> 3.2 us at 2^20 elements).
+__global__ __launch_bounds__(kEdenThreads) void eden_sumsq_kernel(QuantizeSet set)
 {
     __shared__ double lds[kEdenThreads];
-    const int64_t base = (int64_t)blockIdx.x * kEdenTile;
+    const int which = slice_of_block(set.first, set.count);
+    const QuantizeSlice &s = set.s[which];
+    const int64_t tile = blockIdx.x - set.first[which], base = tile * kEdenTile;
+    const float *vec = s.vec + base + threadIdx.x;
+    const int left = (int)min((int64_t)kEdenTile, s.n - base);
+    float v[kEdenPerThread];
+    if (left == kEdenTile) {
+#pragma unroll
+        for (int k = 0; k < kEdenPerThread; k++) v[k] = vec[kEdenThreads * k];
+    } else {
+#pragma unroll
+        for (int k = 0; k < kEdenPerThread; k++) v[k] = (int)threadIdx.x + kEdenThreads * k < left ? vec[kEdenThreads * k] : 0.0f;
+    }
     double acc = 0.0;
 #pragma unroll
-    for (int k = 0; k < kEdenPerThread; k++) {
-        const int64_t i = base + threadIdx.x + (int64_t)kEdenThreads * k;
-        if (i < n) {
-            const double v = (double)vec[i];
-            acc += v * v;
-        }
-    }
-    const double total = fold256(acc, lds);
-    if (threadIdx.x == 0) work[blockIdx.x] = total;
+    for (int k = 0; k < kEdenPerThread; k++) acc = __builtin_fma((double)v[k], (double)v[k], acc); // (the square is exact)
+    const double total = fold256(acc, lds, threadIdx.x);
+    if (threadIdx.x == 0) s.work[tile] = total;
 }
 
 // folds work[0 .. count): thread t adds entries t + 256 k (k ascending), then the halving tree
@@ -66,7 +71,7 @@ __device__ __forceinline__ double fold_array(const double *work, int64_t count, 
 {
     double acc = 0.0;
     for (int64_t i = threadIdx.x; i < count; i += kEdenThreads) acc += work[i];
-    return fold256(acc, lds);
+    return fold256(acc, lds, threadIdx.x);
 }
 
 // result[0] = (float)sumsq, result[3] = norm
@@ -83,53 +88,27 @@ __global__ __launch_bounds__(kEdenThreads) void eden_norm_kernel(const double *_
 }
 
 // Every thread owns sixteen consecutive elements (four 16-byte loads), so that it builds its half word of every
-// bit plane in registers.  The boundaries sit in LDS in breadth-first order of the search tree (node 1 = the
-// middle boundary, children of node i at 2 i and 2 i + 1): the lanes of a wave read one level of the tree at a
-// time, consecutive words, where the sorted layout puts a whole level into a few banks.
-// FOLD: the norm is not in result[3] yet; the workgroup folds the `tiles` partial sums in `sums` the way eden_norm_kernel
-// does (the same association: the same bits), and workgroup 0 leaves result[0] and result[3] as that kernel would.  `work`
-// (the products) is then a region of its own: other workgroups are still reading `sums`.
+// bit plane in registers.
+// FOLD: the norm is not in result[3] yet; the workgroup folds the partial sums in work[0 .. tiles) the way eden_norm_kernel
+// does (the same association: the same bits), workgroup 0 leaves result[0] and result[3] as that kernel would, and the
+// products go to a region of their own (other workgroups are still reading the sums).
 template <int NBITS, bool FOLD>
-__global__ __launch_bounds__(kEdenThreads) void eden_bins_kernel(const float *__restrict__ vec, int64_t n,
-                                                                const float *__restrict__ boundaries,
-                                                                const float *__restrict__ centroids,
-                                                                float *__restrict__ result, float sqrt_n,
-                                                                uint32_t *__restrict__ packed, double *__restrict__ work,
-                                                                const double *__restrict__ sums, int64_t tiles)
+__global__ __launch_bounds__(kEdenThreads) void eden_bins_kernel(QuantizeSet set, const float *__restrict__ boundaries,
+                                                                const float *__restrict__ centroids)
 {
     constexpr int L = 1 << NBITS;
     __shared__ double lds[kEdenThreads];
     __shared__ float tree[L], cen[L];
-    for (int k = threadIdx.x; k < L; k += kEdenThreads) {
-        cen[k] = centroids[k];
-        if (k < L - 1) {
-            // sorted position k = (2 r + 1) 2^(NBITS - 1 - level) - 1 is node 2^level + r
-            const int tz = __builtin_ctz(k + 1);
-            tree[(1 << (NBITS - 1 - tz)) + ((k + 1) >> (tz + 1))] = boundaries[k];
-        }
-    }
-    __syncthreads();
-    float norm;
-    if constexpr (FOLD) {
-        const float s = (float)fold_array(sums, tiles, lds);
-        norm = __builtin_sqrtf(s);
-        if (blockIdx.x == 0 && threadIdx.x == 0) {
-            result[0] = s;
-            result[3] = norm;
-        }
-    } else {
-        norm = result[3];
-    }
-    const uint32_t nb = __float_as_uint(norm);
-    const bool ordinary = nb >= 0x0d800000u && nb <= 0x71800000u; // uniform over the grid
-    const double yn = ordinary ? recip_f64(norm) : 0.0;
-    const int64_t words = n >> 5;
-    const int64_t first = (int64_t)blockIdx.x * kEdenTile + (int64_t)threadIdx.x * kEdenPerThread;
+    const int which = FOLD ? slice_of_block(set.first, set.count) : 0;
+    const QuantizeSlice &s = set.s[which];
+    const int64_t tile = blockIdx.x - (FOLD ? set.first[which] : 0u);
+    const int64_t tiles = eden_tiles(s.n);
     // n is a multiple of 32: the sixteen elements are all inside the vector or all outside
-    const bool in = first < n;
-    float v[kEdenPerThread], x[kEdenPerThread];
-    int node[kEdenPerThread];
+    const int64_t first = tile * kEdenTile + (int64_t)threadIdx.x * kEdenPerThread;
+    const bool in = first < s.n;
+    float v[kEdenPerThread];
     if (in) {
+        const float *vec = s.vec;
         if ((reinterpret_cast<uintptr_t>(vec) & 15) == 0) { // uniform over the grid
 #pragma unroll
             for (int q = 0; q < kEdenPerThread / 4; q++) {
@@ -144,63 +123,38 @@ __global__ __launch_bounds__(kEdenThreads) void eden_bins_kernel(const float *__
 #pragma unroll
         for (int k = 0; k < kEdenPerThread; k++) v[k] = 0.0f;
     }
-    if (ordinary) {
-#pragma unroll
-        for (int k = 0; k < kEdenPerThread; k++) x[k] = div_exact(v[k] * sqrt_n, norm, yn);
-    } else {
-#pragma unroll
-        for (int k = 0; k < kEdenPerThread; k++) x[k] = (v[k] * sqrt_n) / norm;
-    }
-    // the sixteen searches advance level by level: sixteen independent LDS reads per level; node[] holds the
-    // node's byte offset into the table
-#pragma unroll
-    for (int k = 0; k < kEdenPerThread; k++) node[k] = 4;
-#pragma unroll
-    for (int level = 0; level < NBITS; level++) {
-#pragma unroll
-        for (int k = 0; k < kEdenPerThread; k++) {
-            const float b = *reinterpret_cast<const float *>(reinterpret_cast<const char *>(tree) + node[k]);
-            node[k] = 2 * node[k] + (!(b >= x[k]) ? 4 : 0); // torch's lower bound: a NaN goes right at every level
+    eden_tables<NBITS>(boundaries, centroids, tree, cen, threadIdx.x, kEdenThreads);
+    __syncthreads();
+    float norm;
+    if constexpr (FOLD) {
+        const float sum = (float)fold_array(s.work, tiles, lds);
+        norm = __builtin_sqrtf(sum);
+        if (tile == 0 && threadIdx.x == 0) {
+            s.result[0] = sum;
+            s.result[3] = norm;
         }
+    } else {
+        norm = s.result[3];
     }
-    // the product of two floats is exact in double, so the fused multiply-add rounds like multiply, then add;
-    // threads past the end hold zeros and drop their sum below
-    double acc = 0.0;
-    uint32_t four[kEdenPerThread / 4];
-#pragma unroll
-    for (int q = 0; q < kEdenPerThread / 4; q++) four[q] = 0;
-#pragma unroll
-    for (int k = 0; k < kEdenPerThread; k++) {
-        const uint32_t off = (uint32_t)(node[k] - 4 * L); // 4 * bin
-        const float c = *reinterpret_cast<const float *>(reinterpret_cast<const char *>(cen) + off);
-        acc = __builtin_fma((double)c, (double)v[k], acc);
-        four[k >> 2] |= (k & 3) ? off << (8 * (k & 3) - 2) : off >> 2;
-    }
-    if (!in) acc = 0.0;
-    if (in) {
-        const uint64_t lo8 = transpose8x8((uint64_t)four[0] | ((uint64_t)four[1] << 32));
-        const uint64_t hi8 = transpose8x8((uint64_t)four[2] | ((uint64_t)four[3] << 32));
-        // plane p, word (first >> 5), half (first >> 4) & 1
-        uint16_t *half = reinterpret_cast<uint16_t *>(packed) + (first >> 4);
-#pragma unroll
-        for (int p = 0; p < NBITS; p++)
-            half[(int64_t)p * words * 2] = (uint16_t)(((lo8 >> (8 * p)) & 0xffu) | (((hi8 >> (8 * p)) & 0xffu) << 8));
-    }
-    const double total = fold256(acc, lds);
-    if (threadIdx.x == 0) work[blockIdx.x] = total;
+    // plane p, word (first >> 5), half (first >> 4) & 1; threads past the end hold zeros and drop their sum
+    uint16_t *half = in ? reinterpret_cast<uint16_t *>(s.packed) + (first >> 4) : nullptr;
+    const double acc = eden_bins16<NBITS>(v, norm, s.sqrt_n, tree, cen, half, s.n >> 5);
+    const double total = fold256(in ? acc : 0.0, lds, threadIdx.x);
+    if (threadIdx.x == 0) s.work[(FOLD ? tiles : 0) + tile] = total;
 }
 
-// result[1] = (float)dot, result[2] = scale
-__global__ __launch_bounds__(kEdenThreads) void eden_scale_kernel(const double *__restrict__ work, int64_t count,
-                                                                 float *__restrict__ result)
+// one workgroup per slice: result[1] = (float)dot, result[2] = scale
+__global__ __launch_bounds__(kEdenThreads) void eden_scale_kernel(QuantizeSet set, bool fold)
 {
     __shared__ double lds[kEdenThreads];
-    const double dot = fold_array(work, count, lds);
+    const QuantizeSlice &s = set.s[blockIdx.x];
+    const int64_t tiles = eden_tiles(s.n);
+    const double dot = fold_array(s.work + (fold ? tiles : 0), tiles, lds);
     if (threadIdx.x == 0) {
         const float d = (float)dot;
-        const float norm = result[3];
-        result[1] = d;
-        result[2] = (norm * norm) / d;
+        const float norm = s.result[3];
+        s.result[1] = d;
+        s.result[2] = (norm * norm) / d;
     }
 }
 
@@ -292,12 +246,7 @@ __global__ __launch_bounds__(256) void thc_dequantize_kernel(const uint16_t *__r
     }
 }
 
-inline int64_t eden_tiles(int64_t n) { return (n + kEdenTile - 1) / kEdenTile; }
-
 } // namespace
-
-// vectors of up to kEdenFoldTiles tiles take three launches and keep the two kinds of partial sums apart
-constexpr int64_t kEdenFoldTiles = 1024;
 
 int64_t eden_work_doubles(int64_t n)
 {
@@ -305,24 +254,29 @@ int64_t eden_work_doubles(int64_t n)
     return tiles <= kEdenFoldTiles ? 2 * tiles : tiles;
 }
 
-hipError_t launch_eden_quantize(const float *vec, int64_t n, const float *boundaries, const float *centroids, int nbits,
-                                uint32_t *packed, float *result, double *work, hipStream_t stream)
+// slices of at most kEdenFoldTiles tiles, or one of any length; bits of an NBITS-wide code for all of them
+hipError_t launch_eden_quantize_slices(const QuantizeSlice *slices, int count, const float *boundaries, const float *centroids,
+                                       int nbits, hipStream_t stream)
 {
-    const int64_t tiles = eden_tiles(n);
-    const float sqrt_n = (float)sqrt((double)n);
-    dim3 grid((unsigned)tiles), block(kEdenThreads);
-    const bool fold = tiles <= kEdenFoldTiles;
-    double *products = fold ? work + tiles : work;
-    hipLaunchKernelGGL(eden_sumsq_kernel, grid, block, 0, stream, vec, n, work);
-    if (!fold) hipLaunchKernelGGL(eden_norm_kernel, dim3(1), block, 0, stream, work, tiles, result);
-#define DQ_EDEN_BINS(B)                                                                                                   \
-    do {                                                                                                                  \
-        if (fold)                                                                                                         \
-            hipLaunchKernelGGL((eden_bins_kernel<B, true>), grid, block, 0, stream, vec, n, boundaries, centroids, result, \
-                               sqrt_n, packed, products, work, tiles);                                                    \
-        else                                                                                                              \
-            hipLaunchKernelGGL((eden_bins_kernel<B, false>), grid, block, 0, stream, vec, n, boundaries, centroids, result, \
-                               sqrt_n, packed, products, work, tiles);                                                    \
+    QuantizeSet set;
+    set.count = count;
+    int64_t blocks = 0;
+    for (int k = 0; k < count; k++) {
+        set.s[k] = slices[k];
+        set.s[k].sqrt_n = (float)sqrt((double)slices[k].n);
+        set.first[k] = (unsigned)blocks;
+        blocks += eden_tiles(slices[k].n);
+    }
+    const bool fold = count > 1 || blocks <= kEdenFoldTiles;
+    dim3 grid((unsigned)blocks), block(kEdenThreads);
+    hipLaunchKernelGGL(eden_sumsq_kernel, grid, block, 0, stream, set);
+    if (!fold) hipLaunchKernelGGL(eden_norm_kernel, dim3(1), block, 0, stream, slices[0].work, blocks, slices[0].result);
+#define DQ_EDEN_BINS(B)                                                                                       \
+    do {                                                                                                      \
+        if (fold)                                                                                             \
+            hipLaunchKernelGGL((eden_bins_kernel<B, true>), grid, block, 0, stream, set, boundaries, centroids); \
+        else                                                                                                  \
+            hipLaunchKernelGGL((eden_bins_kernel<B, false>), grid, block, 0, stream, set, boundaries, centroids); \
     } while (0)
     switch (nbits) {
     case 1: DQ_EDEN_BINS(1); break;
@@ -335,8 +289,15 @@ hipError_t launch_eden_quantize(const float *vec, int64_t n, const float *bounda
     default: DQ_EDEN_BINS(8); break;
     }
 #undef DQ_EDEN_BINS
-    hipLaunchKernelGGL(eden_scale_kernel, dim3(1), block, 0, stream, products, tiles, result);
+    hipLaunchKernelGGL(eden_scale_kernel, dim3((unsigned)count), block, 0, stream, set, fold);
     return hipGetLastError();
+}
+
+hipError_t launch_eden_quantize(const float *vec, int64_t n, const float *boundaries, const float *centroids, int nbits,
+                                uint32_t *packed, float *result, double *work, hipStream_t stream)
+{
+    const QuantizeSlice s{vec, n, packed, result, work, 0.0f};
+    return launch_eden_quantize_slices(&s, 1, boundaries, centroids, nbits, stream);
 }
 
 } // namespace dq
@@ -444,14 +405,22 @@ hipError_t launch_thc_dequantize(const void *levels, float *out, int64_t n, cons
     return hipGetLastError();
 }
 
-// ---- a slice of EDEN's compress / decompress in one call -------------------------------------------------
+// ---- the slices of EDEN's compress / decompress in one call ----------------------------------------------
 //
-// The reference (and the element-wise sequence this replaced) copies the slice to float32, copies it again or pads it, and
+// The reference (and the element-wise sequence this replaced) copies a slice to float32, copies it again or pads it, and
 // writes the diagonal to memory before every rotation.  Here the first pass of the first rotation reads the caller's vector
 // in its own type with the padding's zeros, the diagonal is drawn in the pass that applies it, and the last pass of the last
-// inverse rotation multiplies by the scale and stores the caller's type.  2^20 fp32 elements at 4 bits, both directions:
-// eight launches and three copies,
-// 94 us, against seven launches, 40 us.
+// inverse rotation multiplies by the scale and stores the caller's type.
+//
+// A launch costs about 3.4 us whatever it does, and a vector has up to five slices, each half as long as the one before or
+// less: the time of a vector of less than a few million elements was its launches.  So the slices travel together:
+//   up to 2^13 elements   one workgroup per slice does all of it, all slices in one launch (dq_eden_short.hip); 2^14 as well
+//                         where no longer slice travels with the next kind's launches anyway
+//   up to 2^22            one launch per pass for all slices: tiles, strided pass, sumsq, bins, scale; tiles, strided pass
+//   beyond                one after the other: their launches fill the GPU, and their diagonal is read from memory
+// Slices that are not plain powers of one rotation (only a caller's own dictionary asks for that) go one by one as well.
+// Both directions at 4 bits, fp32: 2^20 elements (one slice) 94 -> 38 -> 36 us, 20,000 (two) 165 -> 22, 115,387 (four) 364 -> 135 -> 54, 419,364
+// (three) 266 -> 115 -> 37, 6,000,000 (two) 186 -> 80: at first, (with one native call per slice,) together.
 
 namespace {
 
@@ -459,7 +428,7 @@ namespace {
 // costs 25 instruction slots per element, 2.7 us at 2^22 elements.
 constexpr int64_t kEdenDrawnSigns = (int64_t)1 << 22;
 
-// slices of less than 1024 elements (the ends of short vectors): the rotations of dq_hadamard.hip on a padded copy
+// no rotation at all: the slice padded and converted / scaled and converted
 __global__ __launch_bounds__(256) void eden_pad_kernel(const void *__restrict__ src, int dtype, int64_t count, int64_t n,
                                                        float *__restrict__ out)
 {
@@ -489,112 +458,155 @@ __global__ __launch_bounds__(256) void eden_finish_kernel(const float *__restric
 struct SliceScratch {
     float *vec;
     double *work;
-    void *signs; // bits, or floats where n is not a multiple of 256
+    uint32_t *signs;
 };
 
 int64_t round_up(int64_t v) { return (v + 255) & ~(int64_t)255; }
 
-SliceScratch slice_scratch(void *p, int64_t n)
+// (short slices need none; their share is taken all the same, it is small)
+SliceScratch slice_scratch(char *c, int64_t n)
 {
-    char *c = static_cast<char *>(p);
     SliceScratch s;
     s.vec = reinterpret_cast<float *>(c);
     s.work = reinterpret_cast<double *>(c + round_up(4 * n));
-    s.signs = c + round_up(4 * n) + round_up(8 * eden_work_doubles(n));
+    s.signs = reinterpret_cast<uint32_t *>(c + round_up(4 * n) + round_up(8 * eden_work_doubles(n)));
     return s;
 }
 
 float inv_sqrt_of(int64_t n) { return 1.0f / (float)sqrt((double)n); } // as torch divides by a host scalar on the device
 
-// the diagonal of one rotation into memory; *packed: as bits
-hipError_t write_signs(const SliceScratch &s, int64_t n, int64_t seed, bool *packed, hipStream_t stream)
-{
-    *packed = n % 256 == 0;
-    return *packed ? launch_rand_diag_bits(static_cast<uint32_t *>(s.signs), n, seed, stream)
-                   : launch_rand_diag(static_cast<float *>(s.signs), n, seed, stream);
-}
-
 // one rotation of a slice of at least 1024 elements
 hipError_t rotate(const SliceScratch &s, int64_t n, int64_t seed, int inverse, TransformEnds ends, hipStream_t stream)
 {
     const void *sign = nullptr;
-    bool packed = false;
     if (n <= kEdenDrawnSigns) {
         ends.gen = sign_seed(n, seed);
     } else {
-        const hipError_t e = write_signs(s, n, seed, &packed, stream);
+        const hipError_t e = launch_rand_diag_bits(s.signs, n, seed, stream);
         if (e != hipSuccess) return e;
         sign = s.signs;
     }
-    return launch_rht_ends(s.vec, sign, packed, n, n, inv_sqrt_of(n), inverse, ends, stream);
+    return launch_rht_ends(s.vec, sign, sign != nullptr, n, n, inv_sqrt_of(n), inverse, ends, stream);
+}
+
+TransformEnds compress_ends(const dq_eden_slice_t &s, int dtype)
+{
+    TransformEnds ends;
+    ends.in_src = s.vec;
+    ends.in_dtype = dtype;
+    ends.in_count = s.count;
+    return ends;
+}
+
+// the first (planes) and last (destination) ends of an inverse
+TransformEnds decompress_ends(const dq_eden_slice_t &s, int dtype, bool planes, bool destination)
+{
+    TransformEnds ends;
+    if (planes) {
+        ends.in_planes = s.packed;
+        ends.in_centroids = s.centroids;
+        ends.in_nbits = s.nbits;
+    }
+    if (destination) {
+        ends.post_scale = s.result;
+        ends.out_dst = s.vec;
+        ends.out_dtype = dtype;
+        ends.out_count = s.count;
+    }
+    return ends;
+}
+
+// a slice by itself, n > kEdenShort / 2
+hipError_t compress_one(const dq_eden_slice_t &x, int dtype, const SliceScratch &s, hipStream_t stream)
+{
+    hipError_t e = hipSuccess;
+    if (x.rotations == 0) {
+        hipLaunchKernelGGL(eden_pad_kernel, dim3((unsigned)((x.n + 255) / 256)), dim3(256), 0, stream, x.vec, dtype, x.count, x.n, s.vec);
+        e = hipGetLastError();
+    }
+    for (int i = 0; e == hipSuccess && i < x.rotations; i++)
+        e = rotate(s, x.n, x.seed + i, 0, i == 0 ? compress_ends(x, dtype) : TransformEnds(), stream);
+    return e == hipSuccess ? launch_eden_quantize(s.vec, x.n, x.boundaries, x.centroids, x.nbits, x.packed, x.result, s.work, stream) : e;
+}
+
+hipError_t decompress_one(const dq_eden_slice_t &x, int dtype, const SliceScratch &s, hipStream_t stream)
+{
+    hipError_t e = hipSuccess;
+    if (x.rotations == 0) {
+        e = launch_eden_dequantize(x.packed, x.n, x.centroids, x.nbits, s.vec, stream);
+        if (e != hipSuccess) return e;
+        hipLaunchKernelGGL(eden_finish_kernel, dim3((unsigned)((x.count + 255) / 256)), dim3(256), 0, stream, s.vec, x.result, x.vec, dtype, x.count);
+        return hipGetLastError();
+    }
+    for (int i = 0; e == hipSuccess && i < x.rotations; i++)
+        e = rotate(s, x.n, x.seed + x.rotations - 1 - i, 1, decompress_ends(x, dtype, i == 0, i == x.rotations - 1), stream);
+    return e;
+}
+
+bool travels_together(const dq_eden_slice_t &x) { return x.n <= kEdenDrawnSigns && x.rotations == 1; }
+
+// the slices of one kind, kMaxEdenSlices at a time
+template <class Mine, class Launch>
+hipError_t in_groups(const dq_eden_slice_t *slices, char *const *scratch, int count, Mine mine, Launch launch)
+{
+    dq_eden_slice_t group[kMaxEdenSlices];
+    SliceScratch room[kMaxEdenSlices];
+    int have = 0;
+    for (int k = 0; k <= count; k++) {
+        if (k < count && mine(slices[k])) {
+            group[have] = slices[k];
+            room[have++] = slice_scratch(scratch[k], slices[k].n);
+        }
+        if (have == kMaxEdenSlices || (k == count && have > 0)) {
+            const hipError_t e = launch(group, room, have);
+            if (e != hipSuccess) return e;
+            have = 0;
+        }
+    }
+    return hipSuccess;
 }
 
 } // namespace
 
-int64_t eden_slice_bytes(int64_t n)
-{
-    return round_up(4 * n) + round_up(8 * eden_work_doubles(n)) + round_up(n % 256 == 0 ? n / 8 : 4 * n);
-}
+int64_t eden_slice_bytes(int64_t n) { return round_up(4 * n) + round_up(8 * eden_work_doubles(n)) + round_up(n / 8); }
 
-hipError_t launch_eden_compress(const void *src, int dtype, int64_t count, int64_t n, int rotations, int64_t seed,
-                                const float *boundaries, const float *centroids, int nbits, uint32_t *packed, float *result,
-                                void *scratch, hipStream_t stream)
+// compress: slices share nbits, boundaries and centroids
+hipError_t launch_eden_slices(const dq_eden_slice_t *slices, int count, int dtype, bool decompress, void *scratch, hipStream_t stream)
 {
-    const SliceScratch s = slice_scratch(scratch, n);
-    hipError_t e = hipSuccess;
-    if (n < 1024 || rotations == 0) {
-        hipLaunchKernelGGL(eden_pad_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, src, dtype, count, n, s.vec);
-        e = hipGetLastError();
+    std::vector<char *> at(count);
+    char *c = static_cast<char *>(scratch);
+    for (int k = 0; k < count; k++) {
+        at[k] = c;
+        c += eden_slice_bytes(slices[k].n);
     }
-    for (int i = 0; e == hipSuccess && i < rotations; i++) {
-        if (n < 1024) {
-            bool bits;
-            e = write_signs(s, n, seed + i, &bits, stream);
-            if (e == hipSuccess) e = launch_rht_blocked(s.vec, s.signs, bits, n, n, inv_sqrt_of(n), 0, stream);
-        } else {
-            TransformEnds ends;
-            if (i == 0) {
-                ends.in_src = src;
-                ends.in_dtype = dtype;
-                ends.in_count = count;
-            }
-            e = rotate(s, n, seed + i, 0, ends, stream);
+    bool longer = false;
+    for (int k = 0; k < count; k++) longer = longer || (slices[k].n > kEdenShort && travels_together(slices[k]));
+    const auto is_short = [longer](const dq_eden_slice_t &x) { return x.n <= (longer ? kEdenShort / 2 : kEdenShort); };
+    hipError_t e = in_groups(slices, at.data(), count, [&](const dq_eden_slice_t &x) { return !is_short(x) && travels_together(x); },
+                             [&](const dq_eden_slice_t *group, const SliceScratch *room, int have) {
+        TransformSlice t[kMaxEdenSlices];
+        QuantizeSlice q[kMaxEdenSlices];
+        for (int k = 0; k < have; k++) {
+            t[k].x = room[k].vec;
+            t[k].n = group[k].n;
+            t[k].scale = inv_sqrt_of(group[k].n);
+            t[k].ends = decompress ? decompress_ends(group[k], dtype, true, true) : compress_ends(group[k], dtype);
+            t[k].ends.gen = sign_seed(group[k].n, group[k].seed);
+            q[k] = QuantizeSlice{room[k].vec, group[k].n, group[k].packed, group[k].result, room[k].work, 0.0f};
         }
-    }
-    if (e != hipSuccess) return e;
-    return launch_eden_quantize(s.vec, n, boundaries, centroids, nbits, packed, result, s.work, stream);
-}
-
-hipError_t launch_eden_decompress(const uint32_t *packed, int64_t n, int rotations, int64_t seed, const float *centroids, int nbits,
-                                  const float *scale, void *out, int dtype, int64_t count, void *scratch, hipStream_t stream)
-{
-    const SliceScratch s = slice_scratch(scratch, n);
-    hipError_t e = hipSuccess;
-    if (n < 1024 || rotations == 0) {
-        e = launch_eden_dequantize(packed, n, centroids, nbits, s.vec, stream);
-        for (int i = 0; e == hipSuccess && i < rotations; i++) {
-            bool bits;
-            e = write_signs(s, n, seed + rotations - 1 - i, &bits, stream);
-            if (e == hipSuccess) e = launch_rht_blocked(s.vec, s.signs, bits, n, n, inv_sqrt_of(n), 1, stream);
-        }
-        if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(eden_finish_kernel, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, stream, s.vec, scale, out, dtype, count);
-        return hipGetLastError();
-    }
-    for (int i = 0; e == hipSuccess && i < rotations; i++) {
-        TransformEnds ends;
-        if (i == 0) {
-            ends.in_planes = packed;
-            ends.in_centroids = centroids;
-            ends.in_nbits = nbits;
-        }
-        if (i == rotations - 1) {
-            ends.post_scale = scale;
-            ends.out_dst = out;
-            ends.out_dtype = dtype;
-            ends.out_count = count;
-        }
-        e = rotate(s, n, seed + rotations - 1 - i, 1, ends, stream);
+        const hipError_t r = launch_rht_slices(t, have, decompress ? 1 : 0, stream);
+        if (r != hipSuccess || decompress) return r;
+        return launch_eden_quantize_slices(q, have, group[0].boundaries, group[0].centroids, group[0].nbits, stream);
+    });
+    if (e == hipSuccess)
+        e = in_groups(slices, at.data(), count, is_short,
+                      [&](const dq_eden_slice_t *group, const SliceScratch *, int have) {
+            return decompress ? launch_eden_short_decompress(group, have, dtype, stream) : launch_eden_short_compress(group, have, dtype, stream);
+        });
+    for (int k = 0; e == hipSuccess && k < count; k++) {
+        if (is_short(slices[k]) || travels_together(slices[k])) continue;
+        const SliceScratch s = slice_scratch(at[k], slices[k].n);
+        e = decompress ? decompress_one(slices[k], dtype, s, stream) : compress_one(slices[k], dtype, s, stream);
     }
     return e;
 }

@@ -1,0 +1,205 @@
+// EDEN's compress and decompress (srrcomp.py:293-361) of slices of at most 2^14 elements: one workgroup does the whole slice
+// -- the load in the caller's type with the padding, every rotation, the sums, the bins and their planes, the scale -- and
+// one launch all short slices of a vector.
+//
+// Such a slice is all latency: as launches of its own it took eight to ten of about 3.4 us each, every one of them a few
+// workgroups.  A thread holds a chunk of sixteen consecutive elements, as in the tile passes of dq_rht_scaling_impl.cuh, and
+// the chunk is what the quantiser wants of it too; LDS is only for the stages beyond the chunk and for the sums, whose
+// association is that of dq_eden.hip.  The bits are those of the kernels there.
+#define DQ_RHT_PART 0
+#include "dq_eden.cuh"
+#include "dq_rht_scaling_impl.cuh"
+
+namespace dq {
+
+namespace {
+
+constexpr int kShortThreads = kEdenShort / 16;
+
+struct ShortSet {
+    dq_eden_slice_t s[kMaxEdenSlices];
+    float inv[kMaxEdenSlices], sqrt_n[kMaxEdenSlices]; // 1 / sqrt(n) and sqrt(n) as torch takes them
+    int dtype;
+};
+
+// the diagonal of one rotation (sign_seed of dq_hadamard.hip in 32-bit arithmetic: only low words are used)
+__device__ __forceinline__ RhtTileArgs diagonal(int kb, int64_t seed)
+{
+    RhtTileArgs a;
+    a.sign = nullptr;
+    a.sign_bits = 0;
+    a.gen.bits = kb - 3;
+    a.gen.ss = ((uint32_t)seed * 1664525u + 1013904223u) * 8121u + 28411u;
+    return a;
+}
+
+// all stages of the slice of 2^kb elements whose chunk tid is v, times scale
+__device__ __forceinline__ void transform_chunk(float (&v)[16], int kb, float scale, float *lds, int tid, int nthreads)
+{
+    const bool mine = tid < (1 << kb) / 16;
+    float *own = lds + chunk_word(tid);
+    chunk_stages(v, kb);
+    if (mine) {
+#pragma unroll
+        for (int i = 0; i < 16; i++) own[i] = v[i];
+    }
+    fwht_lds_stages_after4(lds, kb, kb, tid, nthreads);
+    if (mine) {
+#pragma unroll
+        for (int i = 0; i < 16; i++) v[i] = own[i] * scale;
+    }
+}
+
+// the fold of the one, two or four tiles' sums, each in the first of its tile's slots
+__device__ __forceinline__ double fold_tiles(const double *sums, int n)
+{
+    if (n <= kEdenTile) return sums[0];
+    if (n <= 2 * kEdenTile) return sums[0] + sums[kEdenThreads];
+    return (sums[0] + sums[2 * kEdenThreads]) + (sums[kEdenThreads] + sums[3 * kEdenThreads]);
+}
+
+template <int NBITS> __global__ __launch_bounds__(kShortThreads) void eden_short_compress_kernel(ShortSet set)
+{
+    constexpr int L = 1 << NBITS;
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    __shared__ double sums[kShortThreads];
+    __shared__ float tree[L], cen[L];
+    const int tid = threadIdx.x, nthreads = blockDim.x;
+    const dq_eden_slice_t &s = set.s[blockIdx.x];
+    const int n = (int)s.n, kb = 31 - __builtin_clz((unsigned)n);
+    const bool mine = tid < n / 16;
+    float v[16];
+    TransformEnds e;
+    e.in_src = s.vec;
+    e.in_dtype = set.dtype;
+    e.in_count = s.count;
+#pragma unroll
+    for (int i = 0; i < 16; i++) v[i] = 0.0f;
+    if (mine) load_source(v, e, tid * 16);
+    eden_tables<NBITS>(s.boundaries, s.centroids, tree, cen, tid, nthreads);
+    for (int i = 0; i < s.rotations; i++) {
+        if (mine) flip16(v, diagonal(kb, s.seed + i), tid * 16);
+        transform_chunk(v, kb, set.inv[blockIdx.x], lds, tid, nthreads);
+    }
+    if (mine) {
+#pragma unroll
+        for (int i = 0; i < 16; i++) lds[chunk_word(tid) + i] = v[i];
+    }
+    __syncthreads();
+    // tile g = threads 256 g .. 256 g + 255 (nthreads is a multiple of 256)
+    const int t = tid & (kEdenThreads - 1), g = tid / kEdenThreads;
+    double acc = 0.0;
+#pragma unroll
+    for (int k = 0; k < kEdenPerThread; k++) {
+        const int i = g * kEdenTile + t + kEdenThreads * k;
+        if (i < n) {
+            const double x = (double)lds[pad_idx(i)];
+            acc += x * x;
+        }
+    }
+    fold256(acc, sums + g * kEdenThreads, t);
+    const float sum = (float)fold_tiles(sums, n);
+    const float norm = __builtin_sqrtf(sum);
+    __syncthreads();
+    uint16_t *half = mine ? reinterpret_cast<uint16_t *>(s.packed) + tid : nullptr;
+    const double dots = eden_bins16<NBITS>(v, norm, set.sqrt_n[blockIdx.x], tree, cen, half, n >> 5);
+    fold256(mine ? dots : 0.0, sums + g * kEdenThreads, t);
+    if (tid == 0) {
+        const float d = (float)fold_tiles(sums, n);
+        s.result[0] = sum;
+        s.result[1] = d;
+        s.result[2] = (norm * norm) / d;
+        s.result[3] = norm;
+    }
+}
+
+__global__ __launch_bounds__(kShortThreads) void eden_short_decompress_kernel(ShortSet set)
+{
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    __shared__ float cen[256];
+    const int tid = threadIdx.x, nthreads = blockDim.x;
+    const dq_eden_slice_t &s = set.s[blockIdx.x];
+    const int n = (int)s.n, kb = 31 - __builtin_clz((unsigned)n);
+    const bool mine = tid < n / 16;
+    for (int k = tid; k < (1 << s.nbits); k += nthreads) cen[k] = s.centroids[k];
+    __syncthreads();
+    float v[16];
+    TransformEnds e;
+    e.in_planes = s.packed;
+    e.in_nbits = s.nbits;
+    e.out_dst = s.vec;
+    e.out_dtype = set.dtype;
+    e.out_count = s.count;
+#pragma unroll
+    for (int i = 0; i < 16; i++) v[i] = 0.0f;
+    if (mine) load_planes(v, e, cen, tid * 16, n >> 5);
+    for (int i = s.rotations - 1; i >= 0; i--) {
+        transform_chunk(v, kb, set.inv[blockIdx.x], lds, tid, nthreads);
+        if (mine) flip16(v, diagonal(kb, s.seed + i), tid * 16);
+    }
+    if (!mine) return;
+    const float scale = *s.result;
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+        store_destination(e, make_float4(v[4 * k] * scale, v[4 * k + 1] * scale, v[4 * k + 2] * scale, v[4 * k + 3] * scale), tid * 16 + 4 * k);
+}
+
+// threads: a multiple of 256 that gives every chunk of the longest slice one
+hipError_t short_set(const dq_eden_slice_t *slices, int count, int dtype, ShortSet &set, unsigned *threads, size_t *lds)
+{
+    int64_t most = 32;
+    if (count < 1 || count > kMaxEdenSlices) return hipErrorInvalidValue;
+    for (int k = 0; k < count; k++) {
+        if (slices[k].n > kEdenShort) return hipErrorInvalidValue;
+        most = std::max(most, slices[k].n);
+        set.s[k] = slices[k];
+        set.sqrt_n[k] = (float)sqrt((double)slices[k].n);
+        set.inv[k] = 1.0f / set.sqrt_n[k];
+    }
+    set.dtype = dtype;
+    *threads = (unsigned)((most / 16 + kEdenThreads - 1) / kEdenThreads * kEdenThreads);
+    *lds = (size_t)padded_tile_floats(ilog2(most)) * sizeof(float);
+    return hipSuccess;
+}
+
+} // namespace
+
+hipError_t launch_eden_short_compress(const dq_eden_slice_t *slices, int count, int dtype, hipStream_t stream)
+{
+    ShortSet set;
+    unsigned threads;
+    size_t lds;
+    hipError_t e = short_set(slices, count, dtype, set, &threads, &lds);
+    if (e != hipSuccess) return e;
+    const auto go = [&](auto kernel) {
+        e = allow_lds(kernel, lds);
+        if (e == hipSuccess) hipLaunchKernelGGL(kernel, dim3((unsigned)count), dim3(threads), lds, stream, set);
+    };
+    switch (slices[0].nbits) {
+    case 1: go(eden_short_compress_kernel<1>); break;
+    case 2: go(eden_short_compress_kernel<2>); break;
+    case 3: go(eden_short_compress_kernel<3>); break;
+    case 4: go(eden_short_compress_kernel<4>); break;
+    case 5: go(eden_short_compress_kernel<5>); break;
+    case 6: go(eden_short_compress_kernel<6>); break;
+    case 7: go(eden_short_compress_kernel<7>); break;
+    default: go(eden_short_compress_kernel<8>); break;
+    }
+    if (e != hipSuccess) return e;
+    return hipGetLastError();
+}
+
+hipError_t launch_eden_short_decompress(const dq_eden_slice_t *slices, int count, int dtype, hipStream_t stream)
+{
+    ShortSet set;
+    unsigned threads;
+    size_t lds;
+    hipError_t e = short_set(slices, count, dtype, set, &threads, &lds);
+    if (e != hipSuccess) return e;
+    e = allow_lds(eden_short_decompress_kernel, lds);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(eden_short_decompress_kernel, dim3((unsigned)count), dim3(threads), lds, stream, set);
+    return hipGetLastError();
+}
+
+} // namespace dq

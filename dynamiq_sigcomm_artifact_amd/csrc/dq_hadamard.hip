@@ -23,6 +23,8 @@
 // 16-byte alignment.  Either kind can take a quantiser at the ends of the transform
 // (THC's levels, EDEN's bit planes and scale).  The LDS index is
 // padded by one float per 32 (dq_fwht.cuh).
+#include <algorithm>
+
 #include "dq_fwht.cuh"
 #include "dq_launch.h"
 
@@ -344,6 +346,35 @@ hipError_t launch_rht_ends(float *x, const void *sign, bool sign_packed, int64_t
                             (sign_packed ? 0 : reinterpret_cast<uintptr_t>(sign));
     if (block < 1024 || n % block != 0 || (every & 15) != 0) return hipErrorInvalidValue;
     return fwht_blocks(x, sign, sign_packed, n, ilog2(block), scale, 1, inverse, stream, ends);
+}
+
+// The longest vector's contiguous pass sets the tile; a shorter one leaves at least four bits to its strided pass.
+hipError_t launch_rht_slices(const TransformSlice *slices, int count, int inverse, hipStream_t stream)
+{
+    TilePass tiles[kMaxEdenSlices], strided[kMaxEdenSlices];
+    if (count < 1 || count > kMaxEdenSlices) return hipErrorInvalidValue;
+    int most = 10;
+    for (int k = 0; k < count; k++) most = std::max(most, contiguous_bits(ilog2(slices[k].n)));
+    for (int k = 0; k < count; k++) {
+        const TransformSlice &s = slices[k];
+        const int kb = ilog2(s.n), kt = std::min(most, kb - 4);
+        if (kb < 14 || kb > 22) return hipErrorInvalidValue;
+        TilePass &t = tiles[k], &r = strided[k];
+        t.x = s.x; t.n = s.n; t.scale = s.scale;
+        t.kt = t.kb = kt;
+        t.rbits = kb - kt; t.sbits = kt;
+        t.first = 0;
+        r = t;
+        t.sign_mode = inverse ? 0 : 1; t.apply_scale = 0;
+        r.sign_mode = inverse ? 2 : 0; r.apply_scale = 1;
+        // the ends of the vector go with the pass that works on them, and so does the diagonal
+        t.ends = r.ends = s.ends;
+        t.ends.out_dst = nullptr; t.ends.out_levels = nullptr; t.ends.post_scale = nullptr;
+        r.ends.in_src = nullptr; r.ends.in_levels = nullptr; r.ends.in_planes = nullptr;
+        (inverse ? t : r).ends.gen = SignSeed();
+    }
+    const hipError_t e = launch_rht_tile_passes(tiles, count, stream);
+    return e == hipSuccess ? launch_rht_strided_passes(strided, count, stream) : e;
 }
 
 hipError_t launch_hadamard(float *vec, int64_t n, hipStream_t stream)

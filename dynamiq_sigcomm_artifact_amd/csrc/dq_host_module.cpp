@@ -526,8 +526,7 @@ at::Tensor empty_on(int device, int64_t n, at::ScalarType dtype)
     return at::empty({n}, at::TensorOptions().dtype(dtype).device(at::kCUDA, (c10::DeviceIndex)device));
 }
 
-// Eden.compress: slices as (start, elements, padded size, rotations); returns one (packed, scale) per slice.  The slices run
-// one after the other on the current stream and share one scratch block.
+// Eden.compress: slices as (start, elements, padded size, rotations); returns one (packed, scale) per slice
 py::list eden_compress(py::handle vec, py::handle boundaries, py::handle centroids, int nbits, int64_t seed, py::sequence slices)
 {
     Args a;
@@ -535,31 +534,37 @@ py::list eden_compress(py::handle vec, py::handle boundaries, py::handle centroi
     const int64_t levels = (int64_t)1 << nbits;
     const float *b = a.typed(boundaries, at::kFloat, levels - 1, "boundaries").data_ptr<float>();
     const float *c = a.typed(centroids, at::kFloat, levels, "centroids").data_ptr<float>();
-    const int code = dtype_code(v), elem = (int)v.element_size();
-    struct Slice {
-        int64_t start, count, n;
-        int rotations;
-    };
-    std::vector<Slice> all;
+    const int elem = (int)v.element_size();
+    std::vector<dq_eden_slice_t> all;
+    std::vector<at::Tensor> planes;
+    const int64_t many = (int64_t)py::len(slices);
+    const at::Tensor results = empty_on(a.device, 4 * many, at::kFloat);
     int64_t room = 0;
-    for (size_t k = 0; k < py::len(slices); k++) {
+    for (int64_t k = 0; k < many; k++) {
         const py::sequence s = slices[k];
-        const Slice x{py::cast<int64_t>(s[0]), py::cast<int64_t>(s[1]), py::cast<int64_t>(s[2]), py::cast<int>(s[3])};
-        if (x.start < 0 || x.count <= 0 || x.start + x.count > v.numel()) refuse("a slice lies outside the vector");
-        room = std::max(room, dq_eden_slice_bytes(x.n));
+        const int64_t start = py::cast<int64_t>(s[0]);
+        dq_eden_slice_t x;
+        x.count = py::cast<int64_t>(s[1]);
+        x.n = py::cast<int64_t>(s[2]);
+        x.rotations = py::cast<int>(s[3]);
+        if (start < 0 || x.count <= 0 || start + x.count > v.numel()) refuse("a slice lies outside the vector");
+        x.vec = static_cast<char *>(v.data_ptr()) + start * elem;
+        x.seed = seed;
+        x.nbits = nbits;
+        x.boundaries = b;
+        x.centroids = c;
+        planes.push_back(empty_on(a.device, x.n / 32 * nbits, at::kInt));
+        x.packed = reinterpret_cast<uint32_t *>(planes.back().data_ptr<int32_t>());
+        x.result = results.data_ptr<float>() + 4 * k;
+        room += dq_eden_slice_bytes(x.n);
         all.push_back(x);
     }
-    const dq_stream_t s = c10::hip::getCurrentHIPStream().stream();
     at::Tensor scratch = empty_on(a.device, room, at::kByte);
+    check(dq_eden_compress(all.data(), (int)all.size(), dtype_code(v), scratch.data_ptr(), room, a.device, c10::hip::getCurrentHIPStream().stream()));
     py::list out;
-    for (const Slice &x : all) {
-        at::Tensor packed = empty_on(a.device, x.n / 32 * nbits, at::kInt), result = empty_on(a.device, 4, at::kFloat);
-        check(dq_eden_compress(static_cast<const char *>(v.data_ptr()) + x.start * elem, code, x.count, x.n, x.rotations, seed, b, c, nbits,
-                               reinterpret_cast<uint32_t *>(packed.data_ptr<int32_t>()), result.data_ptr<float>(), scratch.data_ptr(), room,
-                               a.device, s));
-        out.append(py::make_tuple(py::reinterpret_steal<py::object>(THPVariable_Wrap(packed)),
-                                  py::reinterpret_steal<py::object>(THPVariable_Wrap(result.select(0, 2)))));
-    }
+    for (size_t k = 0; k < all.size(); k++)
+        out.append(py::make_tuple(py::reinterpret_steal<py::object>(THPVariable_Wrap(planes[k])),
+                                  py::reinterpret_steal<py::object>(THPVariable_Wrap(results.select(0, 4 * (int64_t)k + 2)))));
     return out;
 }
 
@@ -568,41 +573,31 @@ void eden_decompress(py::handle out, py::sequence slices)
 {
     Args a;
     const at::Tensor &y = a.tensor(out);
-    const int code = dtype_code(y), elem = (int)y.element_size();
-    struct Slice {
-        const uint32_t *packed;
-        const float *centroids, *scale;
-        int64_t n, count, seed;
-        int nbits, rotations;
-    };
-    std::vector<Slice> all;
+    const int64_t elem = y.element_size();
+    std::vector<dq_eden_slice_t> all;
     int64_t room = 0, total = 0;
     for (size_t k = 0; k < py::len(slices); k++) {
         const py::sequence s = slices[k];
-        Slice x;
+        dq_eden_slice_t x;
         const at::Tensor &p = a.typed(py::object(s[0]), at::kInt, 1, "packed_bins");
         x.nbits = py::cast<int>(s[1]);
         if (x.nbits < 1 || x.nbits > 8) refuse("nbits must be in [1, 8]");
-        x.packed = reinterpret_cast<const uint32_t *>(p.data_ptr<int32_t>());
+        x.packed = reinterpret_cast<uint32_t *>(p.data_ptr<int32_t>());
         x.n = p.numel() / x.nbits * 32;
         x.centroids = a.typed(py::object(s[2]), at::kFloat, (int64_t)1 << x.nbits, "centroids").data_ptr<float>();
-        x.scale = a.typed(py::object(s[3]), at::kFloat, 1, "scale").data_ptr<float>();
+        x.boundaries = nullptr;
+        x.result = a.typed(py::object(s[3]), at::kFloat, 1, "scale").data_ptr<float>();
         x.count = py::cast<int64_t>(s[4]);
         x.rotations = py::cast<int>(s[5]);
         x.seed = py::cast<int64_t>(s[6]);
+        x.vec = static_cast<char *>(y.data_ptr()) + total * elem;
         total += x.count;
-        room = std::max(room, dq_eden_slice_bytes(x.n));
+        room += dq_eden_slice_bytes(x.n);
         all.push_back(x);
     }
     if (total > y.numel()) refuse("out is too small");
-    const dq_stream_t s = c10::hip::getCurrentHIPStream().stream();
     at::Tensor scratch = empty_on(a.device, room, at::kByte);
-    char *at = static_cast<char *>(y.data_ptr());
-    for (const Slice &x : all) {
-        check(dq_eden_decompress(x.packed, x.n, x.rotations, x.seed, x.centroids, x.nbits, x.scale, at, code, x.count, scratch.data_ptr(), room,
-                                 a.device, s));
-        at += x.count * elem;
-    }
+    check(dq_eden_decompress(all.data(), (int)all.size(), dtype_code(y), scratch.data_ptr(), room, a.device, c10::hip::getCurrentHIPStream().stream()));
 }
 
 // norm: a float32 device scalar, with (t, inv_sqrt, inv_levels, inv_clients); or None, with (lo, spacing, step) numbers

@@ -216,7 +216,39 @@ hipError_t launch_rht_tile(float *x, const void *sign, int sign_bits, int64_t n,
 hipError_t launch_rht_strided(float *x, const void *sign, int sign_bits, int64_t n, int rbits, int sbits, float scale,
                               int apply_scale, int sign_mode, int vec, const TransformEnds &ends, hipStream_t stream);
 
+// whole-vector transforms of 2^14 to 2^22 elements, at most kMaxEdenSlices of them, in one launch per pass; scale and the
+// diagonal of ends.gen as in launch_rht_ends
+constexpr int kMaxEdenSlices = 8;
+struct TransformSlice {
+    float *x;
+    int64_t n;
+    float scale;
+    TransformEnds ends;
+};
+hipError_t launch_rht_slices(const TransformSlice *slices, int count, int inverse, hipStream_t stream);
+// the two launches behind it: pass k owns the workgroups from `first` on
+struct TilePass {
+    float *x;
+    int64_t n;
+    float scale;
+    int kt, kb;          // tile pass: tile bits, stages [0, kb)
+    int rbits, sbits;    // strided pass: stages [sbits, sbits + rbits)
+    int sign_mode, apply_scale;
+    unsigned first;
+    TransformEnds ends;
+};
+hipError_t launch_rht_tile_passes(const TilePass *passes, int count, hipStream_t stream);
+hipError_t launch_rht_strided_passes(const TilePass *passes, int count, hipStream_t stream);
+
 // EDEN Lloyd-Max quantiser + packer, THC uniform quantiser (dq_eden.hip)
+struct QuantizeSlice {
+    const float *vec;
+    int64_t n;
+    uint32_t *packed;
+    float *result;
+    double *work;
+    float sqrt_n;
+};
 int64_t eden_work_doubles(int64_t n);
 hipError_t launch_eden_quantize(const float *vec, int64_t n, const float *boundaries, const float *centroids,
                                 int nbits, uint32_t *packed, float *result, double *work,
@@ -241,14 +273,14 @@ hipError_t launch_eden_quantize_static(const float *vec, int64_t n, const float 
                                        hipStream_t stream);
 hipError_t launch_eden_dequantize(const uint32_t *packed, int64_t n, const float *centroids, int nbits,
                                   float *out, hipStream_t stream);
-// one slice of EDEN's compress / decompress (srrcomp.py:293-361): count elements of dtype, padded with zeros to n = 2^k >= 32,
-// `rotations` randomized transforms with the diagonals of seed, seed + 1, ...; scratch: eden_slice_bytes(n), 256-byte aligned
+// the slices of EDEN's compress / decompress (srrcomp.py:293-361); scratch: eden_slice_bytes of every slice, one after the
+// other, 256-byte aligned.  compress: all slices of the same nbits, boundaries and centroids
 int64_t eden_slice_bytes(int64_t n);
-hipError_t launch_eden_compress(const void *src, int dtype, int64_t count, int64_t n, int rotations, int64_t seed,
-                                const float *boundaries, const float *centroids, int nbits, uint32_t *packed, float *result,
-                                void *scratch, hipStream_t stream);
-hipError_t launch_eden_decompress(const uint32_t *packed, int64_t n, int rotations, int64_t seed, const float *centroids, int nbits,
-                                  const float *scale, void *out, int dtype, int64_t count, void *scratch, hipStream_t stream);
+hipError_t launch_eden_slices(const dq_eden_slice_t *slices, int count, int dtype, bool decompress, void *scratch, hipStream_t stream);
+// slices of at most kEdenShort elements, at most kMaxEdenSlices of them, one workgroup each (dq_eden_short.hip)
+constexpr int kEdenShort = 1 << 14;
+hipError_t launch_eden_short_compress(const dq_eden_slice_t *slices, int count, int dtype, hipStream_t stream);
+hipError_t launch_eden_short_decompress(const dq_eden_slice_t *slices, int count, int dtype, hipStream_t stream);
 hipError_t launch_thc_quantize(const float *rotated, const float *uniform, void *out, int64_t n,
                                const float *lo, const float *delta, int levels, hipStream_t stream);
 hipError_t launch_thc_dequantize(const void *levels, float *out, int64_t n, const float *step,

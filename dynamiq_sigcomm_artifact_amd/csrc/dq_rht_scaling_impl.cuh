@@ -408,6 +408,25 @@ __device__ __forceinline__ void store_destination(const TransformEnds &e, float4
     }
 }
 
+// the centroids of sixteen consecutive bins, from the thread's half word of every plane (two 8 x 8 bit transposes)
+__device__ __forceinline__ void load_planes(float (&v)[16], const TransformEnds &e, const float *cen, int64_t g, int64_t words)
+{
+    const uint16_t *half = reinterpret_cast<const uint16_t *>(e.in_planes) + (g >> 4);
+    uint64_t lo8 = 0, hi8 = 0;
+    for (int p = 0; p < e.in_nbits; p++) {
+        const uint32_t h = half[(int64_t)p * words * 2];
+        lo8 |= (uint64_t)(h & 0xffu) << (8 * p);
+        hi8 |= (uint64_t)(h >> 8) << (8 * p);
+    }
+    lo8 = transpose8x8(lo8);
+    hi8 = transpose8x8(hi8);
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        v[k] = cen[(lo8 >> (8 * k)) & 0xffu];
+        v[8 + k] = cen[(hi8 >> (8 * k)) & 0xffu];
+    }
+}
+
 // The chunk at g (a multiple of 16; n is a multiple of 32, so the chunk is inside the vector or outside) as the first
 // pass sees it: the floats of x, or THC's levels times step plus lo (thc_hooks.py:176-178: two roundings), or the
 // centroids of EDEN's bins, read from the bit planes (srrcomp.py:343-354); then the sign flip of a forward transform.
@@ -443,22 +462,7 @@ __device__ __forceinline__ void fetch_chunk(float (&v)[16], const float *__restr
             v[2 * k + 1] = p1 + lo;
         }
     } else {
-        // sixteen consecutive bins from the thread's half word of every plane (two 8 x 8 bit transposes)
-        const uint16_t *half = reinterpret_cast<const uint16_t *>(e.in_planes) + (g >> 4);
-        const int64_t words = in.n >> 5;
-        uint64_t lo8 = 0, hi8 = 0;
-        for (int p = 0; p < e.in_nbits; p++) {
-            const uint32_t h = half[(int64_t)p * words * 2];
-            lo8 |= (uint64_t)(h & 0xffu) << (8 * p);
-            hi8 |= (uint64_t)(h >> 8) << (8 * p);
-        }
-        lo8 = transpose8x8(lo8);
-        hi8 = transpose8x8(hi8);
-#pragma unroll
-        for (int k = 0; k < 8; k++) {
-            v[k] = cen[(lo8 >> (8 * k)) & 0xffu];
-            v[8 + k] = cen[(hi8 >> (8 * k)) & 0xffu];
-        }
+        load_planes(v, e, cen, g, in.n >> 5);
     }
     flip16(v, in, g);
 }
@@ -498,12 +502,12 @@ __device__ __forceinline__ void store4(float *__restrict__ x, float4 v, const Rh
 // sign_mode: 0 no flip, 1 flip on load, 2 flip on store
 // ENDS: a quantiser may sit at either end (TransformEnds; 16-byte accesses only: a.vec is set)
 template <bool ENDS>
-__global__ void rht_tile_kernel(float *__restrict__ x, RhtTileArgs a, int sign_mode, int apply_scale, TransformEnds e)
+__device__ __forceinline__ void tile_pass(float *__restrict__ x, const RhtTileArgs &a, int sign_mode, int apply_scale,
+                                          const TransformEnds &e, unsigned block, float *lds)
 {
-    extern __shared__ __attribute__((aligned(16))) float lds[];
     const int tid = threadIdx.x, nthreads = blockDim.x;
     const int tile = 1 << a.kt;
-    const int64_t origin = (int64_t)blockIdx.x << a.kt;
+    const int64_t origin = (int64_t)block << a.kt;
     RhtTileArgs in = a;
     if (sign_mode != 1) {
         in.sign = nullptr;
@@ -556,21 +560,27 @@ __global__ void rht_tile_kernel(float *__restrict__ x, RhtTileArgs a, int sign_m
     }
 }
 
+template <bool ENDS>
+__global__ void rht_tile_kernel(float *__restrict__ x, RhtTileArgs a, int sign_mode, int apply_scale, TransformEnds e)
+{
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    tile_pass<ENDS>(x, a, sign_mode, apply_scale, e, blockIdx.x, lds);
+}
+
 // A later pass of a transform longer than one tile: index bits [sbits, sbits + rbits) of the vector.  A tile is
 // 2^rbits rows of 32 consecutive floats (128 bytes), row stride 2^sbits elements; in LDS it is row-major, so row bit b
 // is tile bit b + 5.  A thread owns column tid % 32 of sixteen consecutive rows: it loads them (every load instruction of
 // a wave covers two whole 128-byte row segments), does the four lowest row stages on its registers and leaves the other
 // rbits - 4 (at most 6) to one or two LDS passes.  sign_mode: 0, or 2 = flip on store (the last pass of an inverse).
 template <bool ENDS>
-__global__ void rht_strided_kernel(float *__restrict__ x, RhtTileArgs a, int rbits, int sbits, int sign_mode, int apply_scale,
-                                   TransformEnds e)
+__device__ __forceinline__ void strided_pass(float *__restrict__ x, const RhtTileArgs &a, int rbits, int sbits, int sign_mode,
+                                             int apply_scale, const TransformEnds &e, unsigned block, float *lds)
 {
-    extern __shared__ __attribute__((aligned(16))) float lds[];
     const int tid = threadIdx.x, nthreads = blockDim.x;
     const int tile = 1 << (rbits + 5);
     // (shift and mask: written as a quotient and remainder by the power of two, the compiler expands a 64-bit
     // division in front of the kernel's first loads)
-    const int64_t hi = (int64_t)(blockIdx.x >> (sbits - 5)), mid = (int64_t)(blockIdx.x & ((1u << (sbits - 5)) - 1u));
+    const int64_t hi = (int64_t)(block >> (sbits - 5)), mid = (int64_t)(block & ((1u << (sbits - 5)) - 1u));
     const int64_t origin = (hi << (sbits + rbits)) + (mid << 5);
     const int col = tid & 31;
     const int groups = tile >> 9; // groups of sixteen rows
@@ -627,6 +637,53 @@ __global__ void rht_strided_kernel(float *__restrict__ x, RhtTileArgs a, int rbi
         }
     }
 }
+
+template <bool ENDS>
+__global__ void rht_strided_kernel(float *__restrict__ x, RhtTileArgs a, int rbits, int sbits, int sign_mode, int apply_scale,
+                                   TransformEnds e)
+{
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    strided_pass<ENDS>(x, a, rbits, sbits, sign_mode, apply_scale, e, blockIdx.x, lds);
+}
+
+#if DQ_RHT_PART & DQ_RHT_TRANSFORM
+// ---- several vectors per launch (launch_rht_slices) -------------------------------------------------------------
+
+struct PassSet {
+    TilePass p[kMaxEdenSlices];
+    int count;
+};
+
+__device__ __forceinline__ const TilePass &pass_of_block(const PassSet &set)
+{
+    int k = 0;
+    for (int i = 1; i < set.count; i++)
+        if (blockIdx.x >= set.p[i].first) k = i;
+    return set.p[k];
+}
+
+__device__ __forceinline__ RhtTileArgs pass_args(const TilePass &p)
+{
+    RhtTileArgs a;
+    a.sign = nullptr; a.sign_bits = 0; a.n = p.n; a.kt = p.kt; a.kb = p.kb; a.scale = p.scale; a.vec = 1; a.gen = p.ends.gen;
+    return a;
+}
+
+// (the largest pass gives every workgroup its threads and LDS: smaller tiles leave some of both idle)
+__global__ void rht_tile_passes_kernel(PassSet set)
+{
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    const TilePass &p = pass_of_block(set);
+    tile_pass<true>(p.x, pass_args(p), p.sign_mode, p.apply_scale, p.ends, blockIdx.x - p.first, lds);
+}
+
+__global__ void rht_strided_passes_kernel(PassSet set)
+{
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    const TilePass &p = pass_of_block(set);
+    strided_pass<true>(p.x, pass_args(p), p.rbits, p.sbits, p.sign_mode, p.apply_scale, p.ends, blockIdx.x - p.first, lds);
+}
+#endif
 
 // ---- blocks of 2^15: the tile in two halves -----------------------------------------------------------
 //
@@ -1100,6 +1157,51 @@ hipError_t launch_rht_strided(float *x, const void *sign, int sign_bits, int64_t
         hipLaunchKernelGGL(rht_strided_kernel<true>, grid, dim3(threads), lds, stream, x, a, rbits, sbits, sign || ends.gen.bits != 0 ? sign_mode : 0,
                            apply_scale, ends);
     }
+    return hipGetLastError();
+}
+
+// every x 16-byte aligned, n a multiple of 2^kt and 10 <= kt <= 14
+hipError_t launch_rht_tile_passes(const TilePass *passes, int count, hipStream_t stream)
+{
+    PassSet set;
+    set.count = count;
+    unsigned blocks = 0;
+    int most = 10;
+    for (int k = 0; k < count; k++) {
+        if (passes[k].kt < 10 || passes[k].kt > 14 || passes[k].kb > passes[k].kt || (passes[k].n & ((1 << passes[k].kt) - 1)) != 0 || !aligned16(passes[k].x))
+            return hipErrorInvalidValue;
+        set.p[k] = passes[k];
+        set.p[k].first = blocks;
+        blocks += (unsigned)(passes[k].n >> passes[k].kt);
+        most = std::max(most, passes[k].kt);
+    }
+    const size_t lds = ((size_t)padded_tile_floats(most) + 256) * sizeof(float);
+    const hipError_t e = allow_lds(rht_tile_passes_kernel, lds);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(rht_tile_passes_kernel, dim3(blocks), dim3(1u << (most - 4)), lds, stream, set);
+    return hipGetLastError();
+}
+
+// every x 16-byte aligned, n a multiple of 2^(sbits + rbits), 4 <= rbits <= 8
+hipError_t launch_rht_strided_passes(const TilePass *passes, int count, hipStream_t stream)
+{
+    PassSet set;
+    set.count = count;
+    unsigned blocks = 0;
+    int most = 4;
+    for (int k = 0; k < count; k++) {
+        if (passes[k].rbits < 4 || passes[k].rbits > 8 || passes[k].sbits < 5 || (passes[k].n & (((int64_t)1 << (passes[k].sbits + passes[k].rbits)) - 1)) != 0 ||
+            !aligned16(passes[k].x))
+            return hipErrorInvalidValue;
+        set.p[k] = passes[k];
+        set.p[k].first = blocks;
+        blocks += (unsigned)(passes[k].n >> (passes[k].rbits + 5));
+        most = std::max(most, passes[k].rbits);
+    }
+    const size_t lds = (size_t)padded_tile_floats(most + 5) * sizeof(float);
+    const hipError_t e = allow_lds(rht_strided_passes_kernel, lds);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(rht_strided_passes_kernel, dim3(blocks), dim3(1u << (most + 1)), lds, stream, set);
     return hipGetLastError();
 }
 

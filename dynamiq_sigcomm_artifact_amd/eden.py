@@ -126,10 +126,10 @@ class Eden(SRRCompUtils):
         vec = vec.to(self.device).contiguous()                  # the kernels only take buffers of self.device
 
         def low_po2(n):
-            return 2 ** int(np.log2(n)) if n else 0
+            return 1 << n.bit_length() - 1 if n else 0
 
         def high_po2(n):
-            return 2 ** (int(np.ceil(np.log2(n)))) if n else 0
+            return 1 << (n - 1).bit_length() if n else 0
 
         slices = []                                             # (start, elements, padded size, rotations)
         dim = remaining = vec.numel()
@@ -167,7 +167,7 @@ class Eden(SRRCompUtils):
         slices = []
         for d in data:
             scale = d["scale"]
-            scale = scale.reshape(1).to(device=self.device, dtype=torch.float32) if isinstance(scale, torch.Tensor) else \
+            scale = scale.to(self.device, torch.float32) if isinstance(scale, torch.Tensor) else \
                 torch.tensor([scale], dtype=torch.float32, device=self.device)
             slices.append((d["packed_bins"].to(self.device, torch.int32).contiguous(), d["nbits"], self._tables(d["nbits"])[0], scale,
                            d["orig_dim"], d["num_hadamard"], d["seed"]))

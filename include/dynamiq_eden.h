@@ -551,20 +551,28 @@ int dq_eden_dequantize_irht(const uint32_t *packed, int64_t n, const float *cent
                             float scale, const float *post_scale, int device,
                             dq_stream_t stream);
 
-/* srrcomp.py:293-326 / :328-354, one slice in one call: `count` elements of
- * dtype (any of the three), padded with zeros to n = 2^k >= 32, go through
- * `rotations` randomized transforms (the diagonals of seed, seed + 1, ... as
- * dq_rand_diag makes them, the scale 1 / sqrt(n)) and dq_eden_quantize; and the
- * way back, scaled by *scale and stored as `count` elements of dtype.  The same
- * bits as the single calls; the slice is not copied or converted in memory and
- * the diagonal of a short slice never written.  scratch: dq_eden_slice_bytes(n)
+/* srrcomp.py:293-326 / :328-354, the slices of a vector in one call: `count`
+ * elements of dtype (any of the three), padded with zeros to n = 2^k >= 32, go
+ * through `rotations` randomized transforms (the diagonals of seed, seed + 1,
+ * ... as dq_rand_diag makes them, the scale 1 / sqrt(n)) and dq_eden_quantize;
+ * and the way back, scaled by *result and stored as `count` elements of dtype.
+ * The same bits as the single calls; a slice is not copied or converted in
+ * memory, the diagonal of a short one never written, and slices of up to 2^22
+ * elements share their launches.  scratch: the sum of dq_eden_slice_bytes(n)
  * bytes, 256-byte aligned, contents undefined before and after. */
+typedef struct dq_eden_slice {
+    void *vec;               /* compress: read; decompress: written */
+    int64_t count, n, seed;
+    int rotations, nbits;
+    uint32_t *packed;        /* compress: written (n / 32 * nbits words); decompress: read */
+    float *result;           /* compress: float[4] as dq_eden_quantize leaves it; decompress: the scale, read */
+    const float *boundaries; /* compress only */
+    const float *centroids;  /* compress: as boundaries and nbits, the same for all slices of a call */
+} dq_eden_slice_t;
 int64_t dq_eden_slice_bytes(int64_t n);
-int dq_eden_compress(const void *src, int dtype, int64_t count, int64_t n, int rotations, int64_t seed,
-                     const float *boundaries, const float *centroids, int nbits, uint32_t *packed, float *result,
-                     void *scratch, int64_t scratch_bytes, int device, dq_stream_t stream);
-int dq_eden_decompress(const uint32_t *packed, int64_t n, int rotations, int64_t seed, const float *centroids, int nbits,
-                       const float *scale, void *out, int dtype, int64_t count, void *scratch, int64_t scratch_bytes,
+int dq_eden_compress(const dq_eden_slice_t *slices, int count, int dtype, void *scratch, int64_t scratch_bytes,
+                     int device, dq_stream_t stream);
+int dq_eden_decompress(const dq_eden_slice_t *slices, int count, int dtype, void *scratch, int64_t scratch_bytes,
                        int device, dq_stream_t stream);
 
 /* THC's grid of levels (thc_hooks.py:143-147): numbers of the host (norm NULL:

@@ -394,6 +394,49 @@ def test_slices_in_one_call_equal_the_single_calls(capi, n, dt):
     assert got.dtype == dt and torch.equal(got, torch.cat(want))
 
 
+@pytest.mark.parametrize("dt", [torch.float32, torch.float16])
+@pytest.mark.parametrize("nbits", [1, 8])
+@pytest.mark.parametrize("sizes", [[(32, 1), (32, 3), (512, 2), (1024, 0), (4096, 1), (8192, 2), (8192, 1), (256, 1), (2048, 1), (64, 2)],
+                                   [(16384, 1)] * 9 + [(1 << 15, 1), (1 << 17, 1), (16384, 2), (16384, 0), (1 << 16, 3)],
+                                   [(16384, 1), (16384, 2), (8192, 1), (16384, 0), (1 << 15, 2)],
+                                   [(1 << 22, 1), (1 << 14, 1), (1 << 13, 1), (1 << 23, 1), (1 << 18, 2)]])
+def test_many_slices_share_launches(capi, sizes, nbits, dt):
+    """slices of every kind in one call -- more than a launch takes, one workgroup each, passes shared, by themselves, with no, one
+    and several rotations, ragged -- against the calls they stand for"""
+    import math
+    from dynamiq_sigcomm_artifact_amd.eden import Eden
+    eden, host, seed = Eden(device=DEV), capi.host(), -3
+    centroids, boundaries = eden._tables(nbits)
+    slices, start = [], 0
+    for k, (size, rotations) in enumerate(sizes):
+        count = size - (k % 3) * (size // 40 + 1)
+        slices.append((start, count, size, rotations))
+        start += count
+    g = torch.Generator(device=DEV).manual_seed(nbits)
+    vec = (torch.randn(start, generator=g, device=DEV) * 1e-2).to(dt)
+    got = host.eden_compress(vec, boundaries, centroids, nbits, seed, slices)
+    want = []
+    for (packed, scale), (at, count, size, rotations) in zip(got, slices):
+        inv = float(np.float32(1.0) / np.float32(math.sqrt(size)))
+        x = torch.zeros(size, device=DEV)
+        x[:count] = vec[at:at + count].float()
+        diags = [torch.empty(size, device=DEV) for _ in range(rotations)]
+        for i, diag in enumerate(diags):
+            capi.rand_diag(diag, seed + i)
+            capi.rht_blocked(x, diag, size, inv, False)
+        ref, result = torch.empty_like(packed), torch.empty(4, device=DEV)
+        capi.eden_quantize(x, boundaries, centroids, nbits, ref, result, torch.empty(capi.eden_work_doubles(size), dtype=torch.float64, device=DEV))
+        assert torch.equal(packed, ref) and torch.equal(scale.view(torch.int32), result[2].view(torch.int32)), (count, size, rotations)
+        y = torch.empty(size, device=DEV)
+        capi.eden_dequantize(ref, size, centroids, nbits, y)
+        for diag in reversed(diags):
+            capi.rht_blocked(y, diag, size, inv, True)
+        want.append((result[2] * y)[:count].to(dt))
+    out = torch.empty(start, dtype=dt, device=DEV)
+    host.eden_decompress(out, [(p, nbits, centroids, s, count, rotations, seed) for (p, s), (_, count, _, rotations) in zip(got, slices)])
+    assert torch.equal(out, torch.cat(want))
+
+
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("n,dim", [(1024, 1024), (40000, 65536), (1 << 20, 1 << 20), (1000, 1024), ((1 << 21) + 5, 1 << 22)])
 def test_thc_grid_and_source_in_the_passes(capi, n, dim, dt):
