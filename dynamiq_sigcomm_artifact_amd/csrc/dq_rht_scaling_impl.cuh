@@ -937,12 +937,21 @@ template <class K> hipError_t allow_lds(K kernel, size_t bytes)
     return hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
 }
 
+// Blocks of 2^10 .. 2^14 as whole tiles, one chunk per thread, or in two halves, two chunks per thread.  Up to 2^23 elements
+// all chunks fit the GPU at once (256 CUs x 2048 threads x 16 elements): then the halves only leave threads idle, and a block
+// takes twice as long through its workgroup.  Beyond, the halves keep more loads in flight per thread and their tiles leave
+// room for more workgroups.  Compress + decompress at 4 bits, in halves -> whole: 2^20 elements in blocks of 2^12 12.4 -> 10.1
+// us, 2^14 17.1 -> 14.9, 2^22 15.9 -> 14.5, 2^23 23.7 -> 21.6, 2^24 39.7 -> 37.1; 2^25 68.6 against 68.7 and, in blocks of
+// 2^10, 64.6 against 69.5.
+constexpr int64_t kWholeTiles = (int64_t)1 << 23;
+
 template <int RDT, int NBITS, bool MEE>
 hipError_t run_compress(const float *src, const void *sign, int sign_bits, uint8_t *dst, const void *rnd, int64_t n, int64_t block,
                         float scale, const MeeParams &mp, RandKey key, hipStream_t stream)
 {
     const Geometry g = geometry(src, sign, sign_bits, n, block, scale);
-    if (g.a.kb == 10 && (n & 2047) == 0) {
+    const bool halves = n > kWholeTiles || g.a.kb == kSplitBits;
+    if (halves && g.a.kb == 10 && (n & 2047) == 0) {
         // blocks of 2^10, two per wave
         auto kernel = rht_compress_split_kernel<RDT, NBITS, MEE, 10, false>;
         const size_t lds = split_lds_bytes<NBITS, 10>();
@@ -950,7 +959,7 @@ hipError_t run_compress(const float *src, const void *sign, int sign_bits, uint8
                            make_arg<NBITS, MEE>(mp));
         return hipGetLastError();
     }
-    if (g.a.kb >= kSplitBits - 4 && g.a.kb <= kSplitBits && (n & ((1 << g.a.kb) - 1)) == 0) {
+    if (halves && g.a.kb >= kSplitBits - 4 && g.a.kb <= kSplitBits && (n & ((1 << g.a.kb) - 1)) == 0) {
         // blocks of 2^11 .. 2^15: two halves per workgroup
         auto launch = [&](auto kernel, size_t lds, int half_bits) -> hipError_t {
             hipError_t es = allow_lds(kernel, lds);
@@ -988,7 +997,8 @@ hipError_t run_decompress(const uint8_t *src, const void *sign, int sign_bits, f
                           const MeeParams &mp, hipStream_t stream)
 {
     const Geometry g = geometry(dst, sign, sign_bits, n, block, scale);
-    if (g.a.kb >= 10 && g.a.kb <= kSplitBits && (n & ((g.a.kb == 10 ? 2048 : (1 << g.a.kb)) - 1)) == 0) {
+    const bool halves = n > kWholeTiles || g.a.kb == kSplitBits;
+    if (halves && g.a.kb >= 10 && g.a.kb <= kSplitBits && (n & ((g.a.kb == 10 ? 2048 : (1 << g.a.kb)) - 1)) == 0) {
         // blocks of 2^11 .. 2^15 in two halves per workgroup, blocks of 2^10 two per wave
         auto launch = [&](auto kernel, int half_bits) -> hipError_t {
             const size_t tile = (size_t)padded_tile_floats(half_bits) * sizeof(float);

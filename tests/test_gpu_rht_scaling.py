@@ -101,6 +101,39 @@ def test_blocks_taken_in_two_halves_every_width(capi, nbits, strategy, block):
     assert torch.equal(back.view(torch.int32), dec.view(torch.int32))
 
 
+@pytest.mark.parametrize("block", [1 << 10, 1 << 11, 1 << 12, 1 << 13, 1 << 14])
+@pytest.mark.parametrize("blocks_more", [0, 1, 2])
+def test_whole_tiles_to_halves(capi, block, blocks_more):
+    """around 2^23 elements, where blocks of 2^10 .. 2^14 go from whole tiles to halves, against the two calls"""
+    n = (1 << 23) + blocks_more * block
+    g = torch.Generator(device=DEV).manual_seed(block + blocks_more)
+    x = torch.randn(n, generator=g, device=DEV) * 1e-3
+    sign = torch.empty(n // 32, dtype=torch.int32, device=DEV)
+    capi.rand_diag_bits(sign, n, 7)
+    scale = 1.0 / block ** 0.5
+    for nbits, strategy, pool in ((2, 2, None), (4, 3, torch.float32), (5, 2, torch.bfloat16), (8, 3, None)):
+        rnd = torch.empty(n, dtype=pool or torch.float32, device=DEV)
+        if pool is None:
+            capi.philox_uniform(rnd, 3, 4)
+        else:
+            rnd.copy_(torch.rand(n, generator=g, device=DEV))
+        want = torch.zeros(capi.required_bytes(n, nbits, 16, strategy), dtype=torch.uint8, device=DEV)
+        got = torch.zeros_like(want)
+        rot = x.clone()
+        capi.rht_blocked(rot, sign, block, scale, False)
+        capi.scaling_compress(rot, want, rnd, n, nbits, 16, strategy)
+        if pool is None:
+            capi.rht_scaling_compress(x, sign, got, block, scale, nbits, strategy, seed=3, step=4)
+        else:
+            capi.rht_scaling_compress(x, sign, got, block, scale, nbits, strategy, rand_pool=rnd)
+        assert torch.equal(got, want), (nbits, strategy)
+        back, ref = torch.empty_like(x), torch.empty_like(x)
+        capi.scaling_decompress_irht(got, sign, back, block, scale, nbits, strategy)
+        capi.scaling_decompress(want, ref, n, nbits, 16, strategy)
+        capi.rht_blocked(ref, sign, block, scale, True)
+        assert torch.equal(back, ref), (nbits, strategy)
+
+
 @pytest.mark.parametrize("n,block", [(256, 256), (256, 16), (512, 512), (768, 256), (1280, 256), (2048, 1024)])
 def test_small_vectors_no_sign_unaligned(capi, n, block):
     g, x, _ = _case(n, n + block)
