@@ -480,7 +480,7 @@ struct Codec {
 
 // One bucket of the fixed-proportion (sorted_plan) or dynamic all-reduce with compressor objects: codecs holds one list per
 // width (8, 4, 2 bits), group sizes counts.  Walks every codec's LCG as the ring's calls on its non-empty chunks would, in
-// the order of the widths and, per rank, of the steps: rank r works on chunk (r - step) mod world in that step.
+// the order of the widths, the steps and the ranks: rank r works on chunk (r - step) mod world in that step.
 void ranks_pooled(py::sequence vecs, py::sequence outs, int64_t n, py::handle total, py::handle mean, py::handle order,
                   py::handle work, py::sequence codecs, py::sequence counts, int stages, int strategy)
 {
@@ -496,12 +496,13 @@ void ranks_pooled(py::sequence vecs, py::sequence outs, int64_t n, py::handle to
         if (size[g] == 0) continue;
         const py::sequence of_width = codecs[g];
         const int64_t per = (size[g] + world - 1) / world;
-        for (int r = 0; r < world; r++) {
-            Codec &c = py::cast<Codec &>(of_width[r]);
-            const at::Tensor &p = c.pool(dtype);
-            need(p.is_cuda() && p.is_contiguous() && p.device().index() == a.device, "rand_pool must be a contiguous tensor on the vectors' device");
-            pool[g * world + r] = p.data_ptr();
-            for (int step = 0; step < world; step++) {
+        // step by step, as the ring's calls go: ranks may share a compressor
+        for (int step = 0; step < world; step++) {
+            for (int r = 0; r < world; r++) {
+                Codec &c = py::cast<Codec &>(of_width[r]);
+                const at::Tensor &p = c.pool(dtype);
+                need(p.is_cuda() && p.is_contiguous() && p.device().index() == a.device, "rand_pool must be a contiguous tensor on the vectors' device");
+                pool[g * world + r] = p.data_ptr();
                 const int chunk = (r - step + world) % world;
                 const int64_t rows = std::max<int64_t>(0, std::min(per, size[g] - per * chunk));
                 if (rows == 0) continue;

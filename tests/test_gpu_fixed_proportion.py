@@ -259,3 +259,24 @@ def test_pooled_ring_in_registers_equals_op_sequence(capi, W, n):
             assert torch.equal(total.view(torch.int16), total2.view(torch.int16))
             assert all(torch.equal(x.view(torch.int16), y.view(torch.int16)) for x, y in zip(ref, out))
         assert all(x.rand_seed == y.rand_seed for q in (8, 4, 2) for x, y in zip(a[q], b[q]))
+
+
+def test_ranks_that_share_a_compressor(capi):
+    """one compressor object for all ranks: its pool is walked in the order of the ring's calls, step by step; a compressor of
+    another width in a list takes the call-by-call ring"""
+    from dynamiq_sigcomm_artifact_amd.compressors import Aee_Dynamic_Range_GPU_kern as K
+    from dynamiq_sigcomm_artifact_amd.dynamiq_pipeline import _pooled_codecs, fixed_proportion_allreduce, fixed_proportion_allreduce_grouped
+    W, n, thr = 3, 256 * 50, {8: 0.35, 4: 0.45, 2: 0.2}
+    vecs = [torch.randn(n, generator=torch.Generator().manual_seed(r)).to(torch.bfloat16).to(DEV) for r in range(W)]
+
+    def comps():
+        gen = torch.Generator(device=DEV).manual_seed(5)
+        return {q: [K(q, 16, {"d": {0: n * W}, "world_size": W, "rank": 0}, generator=gen)] * W for q in (8, 4, 2)}
+    a, b = comps(), comps()
+    ref, _, _ = fixed_proportion_allreduce(vecs, thr, a)
+    out, _, _, _ = fixed_proportion_allreduce_grouped(vecs, thr, b)
+    assert _pooled_codecs(vecs, b) is not None
+    assert all(torch.equal(x.view(torch.int16), y.view(torch.int16)) for x, y in zip(ref, out))
+    assert all(a[q][0].rand_seed == b[q][0].rand_seed for q in (8, 4, 2))
+    b[8] = [b[8][0], b[8][0], b[4][0]]
+    assert _pooled_codecs(vecs, b) is None
