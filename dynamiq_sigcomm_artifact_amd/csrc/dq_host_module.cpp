@@ -110,9 +110,16 @@ uint32_t *hist_of(Args &a, py::handle h, int64_t *entries)
 
 // The state of a SinglePassBuckets object.  Its buckets share scratch and run on the caller's stream; a caller that comes
 // back on another stream is ordered behind the one before.
+//
+// A launch takes the steps begun since the last one along and advances the counter in device memory itself.  That holds for
+// eager launches only: a recorded launch is replayed without this object taking part.  So a step begun while recording is a
+// node of the graph, steps begun before the recording that no launch has taken along yet go into `base`, a constant of every
+// later launch, and once a graph exists a step is begun on the device at once, where the next replay finds it.
 struct Buckets {
     int strategy, device;
     uint64_t seed, pending = 0; // training steps begun since the last launch
+    uint64_t base = 0;          // steps that the counter in device memory never gets
+    bool recorded = false;      // a graph with launches of this object may exist
     py::object step_dev, u_dev, hist, stats, counts;
     uint64_t *step_ptr = nullptr;
     const double *u_ptr = nullptr;
@@ -121,8 +128,11 @@ struct Buckets {
     char *stats_ptr = nullptr;
     int64_t stats_room = 0, counts_room = 0;
     int32_t *counts_ptr = nullptr;
-    hipStream_t last = nullptr;
+    hipStream_t last = nullptr; // of the last eager launch
     bool used = false;
+    std::vector<hipStream_t> kept_for; // streams beside the one that the tensors were made on
+    hipStream_t last_recorded = nullptr; // of the last launch of the recording with this id
+    unsigned long long recording = 0;
 
     Buckets(int strategy_, uint64_t seed_, py::object step, py::object u, py::object h) : strategy(strategy_), seed(seed_)
     {
@@ -145,17 +155,67 @@ struct Buckets {
         counts_room = c.numel() / 4;
         stats = stats_;
         counts = counts_;
+        kept_for.clear();
     }
-    void follow(hipStream_t s)
+    // is s recording a graph, and which?
+    static bool capturing(hipStream_t s, unsigned long long *id)
     {
-        if (used && s != last) check(dq_stream_order_after(s, last, device));
+        hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+        if (hipStreamGetCaptureInfo(s, &status, id) != hipSuccess) {
+            (void)hipGetLastError(); // (of the null stream while another one records)
+            return false;
+        }
+        return status == hipStreamCaptureStatusActive;
+    }
+    // the memory may not go to another tensor before s, torch's current stream, is done with it
+    void keep_for(hipStream_t s)
+    {
+        if (std::find(kept_for.begin(), kept_for.end(), s) != kept_for.end()) return;
+        const py::object stream = py::module_::import("torch.cuda").attr("current_stream")(device);
+        for (const py::object *o : {&step_dev, &u_dev, &hist, &stats, &counts})
+            if (*o && !o->is_none()) o->attr("record_stream")(stream);
+        kept_for.push_back(s);
+    }
+    // orders s behind what was enqueued so far; true while s is recording.  (A recording cannot wait for eager work: whoever
+    // records has waited for it, as torch.cuda.graph does.)
+    bool follow(hipStream_t s)
+    {
+        unsigned long long id = 0;
+        if (capturing(s, &id)) {
+            if (recording == id && s != last_recorded) check(dq_stream_order_after(s, last_recorded, device));
+            recording = id;
+            last_recorded = s;
+            recorded = true;
+            base += pending;
+            pending = 0;
+            return true;
+        }
+        if (used && s != last) {
+            check(dq_stream_order_after(s, last, device));
+            keep_for(s);
+        }
         last = s;
         used = true;
+        return false;
     }
     void join()
     {
         const hipStream_t s = c10::hip::getCurrentHIPStream(device).stream();
-        if (used && s != last) follow(s);
+        unsigned long long id = 0;
+        const bool now = capturing(s, &id);
+        if (now ? recording == id && s != last_recorded : used && s != last) follow(s);
+    }
+    void begin_step()
+    {
+        const hipStream_t s = c10::hip::getCurrentHIPStream(device).stream();
+        unsigned long long id = 0;
+        if (!recorded && !capturing(s, &id)) {
+            pending++;
+            return;
+        }
+        follow(s);
+        at::Tensor counter = THPVariable_Unpack(step_dev.ptr());
+        counter.add_(1);
     }
 };
 
@@ -215,14 +275,21 @@ struct Batch {
         const hipStream_t s = c10::hip::getCurrentHIPStream(b.device).stream();
         b.follow(s);
         const uint64_t more = b.pending;
+        const dq_roundtrip_t *buckets = desc.data();
+        std::vector<dq_roundtrip_t> moved;
+        if (b.base) {
+            moved = desc;
+            for (dq_roundtrip_t &d : moved) d.step += b.base;
+            buckets = moved.data();
+        }
         int rc;
         {
             py::gil_scoped_release nogil;
-            rc = dq_bucket_roundtrip(desc.data(), (int)desc.size(), dtype, b.strategy, 1, 0.0, b.u_ptr, b.seed, b.step_ptr, more, b.hist_ptr,
+            rc = dq_bucket_roundtrip(buckets, (int)desc.size(), dtype, b.strategy, 1, 0.0, b.u_ptr, b.seed, b.step_ptr, more, b.hist_ptr,
                                      b.hist_ints, b.device, s);
         }
         check(rc);
-        b.pending = 0;
+        b.pending -= more;
     }
 };
 
@@ -859,7 +926,7 @@ PYBIND11_MODULE(_host, m)
         .def(py::init<int, uint64_t, py::object, py::object, py::object>())
         .def("scratch", &Buckets::scratch)
         .def("join", &Buckets::join)
-        .def("begin_step", [](Buckets &b) { b.pending++; });
+        .def("begin_step", &Buckets::begin_step);
     py::class_<Batch>(m, "Batch")
         .def(py::init([](Buckets &b, py::sequence pairs, py::sequence steps, py::sequence rows) {
             std::vector<uint64_t> s;

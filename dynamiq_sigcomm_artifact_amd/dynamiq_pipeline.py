@@ -505,7 +505,7 @@ class SinglePassBuckets(object):
         """enqueue one bucket: out = decode(encode(x)) with the widths of its reduced norms; returns its slot"""
         key = (x.data_ptr(), out.data_ptr(), x.numel(), x.dtype)
         entry = self.cache.get(key)
-        if entry is None:
+        if entry is None or not entry[0].matches([(x, out)]):
             entry = self._batch([(x, out)], key, True)
         self._enqueue(entry)
         return next(iter(entry[2]))
@@ -518,7 +518,7 @@ class SinglePassBuckets(object):
                 return
             key = tuple((x.data_ptr(), o.data_ptr(), x.numel(), x.dtype) for x, o in pairs)
             last = self.cache.get(key)
-            if last is None:
+            if last is None or not last[0].matches(list(map(tuple, pairs))):
                 last = self._batch(pairs, key, False)
             self._last = last
         self._enqueue(last)

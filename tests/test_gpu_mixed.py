@@ -728,3 +728,78 @@ def test_estimates_just_below_zero_round_down(capi, bits, u):
     torch.cuda.synchronize()
     assert pipe.counts(0).tolist() == [nsc if bits == w else 0 for w in (8, 4, 2)] + [0]
     assert torch.equal(out, _four_calls(capi, x, x.numel(), u, 2, 5, 1)[5])
+
+
+@pytest.mark.parametrize("inside", [False, True])
+def test_recorded_step_draws_fresh_values(capi, inside):
+    """a step recorded after eager ones on another stream, with begin_step() inside the recording or before every replay, against
+    the four calls with the counter where it stands; eager steps between the replays go on from there"""
+    from dynamiq_sigcomm_artifact_amd.dynamiq_pipeline import SinglePassBuckets
+    u, seed = 6.0, 7
+    xs = [_llama_like(n, n, torch.bfloat16) for n in (256 * 40 - 9, 256 * 21)]
+    outs = [torch.zeros_like(x) for x in xs]
+    pairs = list(zip(xs, outs))
+    pipe = SinglePassBuckets(DEV, strategy=2, seed=seed, u=u)
+
+    def expect(step):
+        torch.cuda.synchronize()
+        for k, (x, o) in enumerate(pairs):
+            assert torch.equal(bits_t(o), bits_t(_four_calls(capi, x, x.numel(), u, 2, seed, (k << 32) + step)[5])), (step, k)
+            o.zero_()
+
+    step = 0
+    for _ in range(2):
+        pipe.begin_step()
+        step += 1
+        pipe.run_all(pairs)
+        pipe.join()
+        expect(step)
+    if not inside:
+        pipe.begin_step()
+        step += 1
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        if inside:
+            pipe.begin_step()
+        pipe.run_all(pairs)
+        pipe.join()
+    for k in range(4):
+        if inside:
+            step += 1
+        elif k > 0:
+            pipe.begin_step()
+            step += 1
+        graph.replay()
+        expect(step)
+        if k == 1:
+            pipe.begin_step()
+            step += 1
+            pipe.run_all(pairs)
+            pipe.join()
+            expect(step)
+
+
+def test_bucket_seen_before_is_checked_again(capi):
+    """an output at a known address that has become too short is refused, not written beyond its end; scratch in use on two streams
+    grows without disturbing either"""
+    from dynamiq_sigcomm_artifact_amd.dynamiq_pipeline import SinglePassBuckets
+    x = _llama_like(256 * 64, 5, torch.bfloat16)
+    out = torch.zeros_like(x)
+    pipe = SinglePassBuckets(DEV, strategy=2, seed=3, u=6.0)
+    pipe.begin_step()
+    pipe.run(x, out)
+    pipe.run_all([(x, out)])
+    with pytest.raises(RuntimeError, match="output"):
+        pipe.run(x, out[:-256])
+    with pytest.raises(RuntimeError, match="output"):
+        pipe.run_all([(x, out[:-256])])
+    big = _llama_like(256 * 300 + 1, 6, torch.bfloat16)
+    result = torch.zeros_like(big)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        pipe.run(x, out)
+    pipe.run(big, result)
+    torch.cuda.synchronize()
+    for k, (v, o) in enumerate(((x, out), (big, result))):
+        assert torch.equal(bits_t(o), bits_t(_four_calls(capi, v, v.numel(), 6.0, 2, 3, (k << 32) + 1)[5]))
