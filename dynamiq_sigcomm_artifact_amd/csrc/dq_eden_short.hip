@@ -23,9 +23,9 @@ struct ShortSet {
 };
 
 // the diagonal of one rotation (sign_seed of dq_hadamard.hip in 32-bit arithmetic: only low words are used)
-__device__ __forceinline__ RhtTileArgs diagonal(int kb, int64_t seed)
+__device__ __forceinline__ RhtPassArgs diagonal(int kb, int64_t seed)
 {
-    RhtTileArgs a;
+    RhtPassArgs a;
     a.sign = nullptr;
     a.sign_bits = 0;
     a.gen.bits = kb - 3;

@@ -30,6 +30,7 @@
 #pragma once
 
 #include <algorithm>
+#include <type_traits>
 
 #include "dq_fwht.cuh"
 #include "dq_hier16_tiles.cuh"
@@ -56,8 +57,14 @@ struct RhtTileArgs {
     int kb;            // log2 transform block, <= kt
     float scale;
     int vec;           // 16-byte accesses to the fp32 vector and the sign vector allowed
-    SignSeed gen;      // the diagonal drawn here instead (sign is then null); served by flip4 and flip16 only
 };
+
+// The diagonal drawn where it is applied (sign is then null); flip4 and flip16 serve it.  A type of its own: the kernels
+// fused with the codec run on 64 registers, and a test for a seed that they never have costs them time (2^30 elements there and back 2134 -> 2118 us without it).
+struct RhtPassArgs : RhtTileArgs {
+    SignSeed gen;
+};
+template <bool ENDS> using PassArgs = typename std::conditional<ENDS, RhtPassArgs, RhtTileArgs>::type;
 
 // Element g of the diagonal of rand_diag (srrcomp.py:61-106; rand_diag_word of dq_hadamard.hip in 32-bit arithmetic: only
 // the low word of every product is used, and the one carry that is, of the addition, is added back by hand).  Four
@@ -80,14 +87,6 @@ __device__ __forceinline__ uint32_t rand_diag_negative(const SignSeed &s, uint32
 // which is what the multiplication by -1.0f does to every number
 __device__ __forceinline__ void flip4(float4 &v, const RhtTileArgs &a, int64_t g)
 {
-    if (a.gen.bits != 0) {
-        const uint32_t k = (uint32_t)(g >> a.gen.bits), j = (uint32_t)g & ((1u << a.gen.bits) - 1u); // the four share a segment
-        v.x = __uint_as_float(__float_as_uint(v.x) ^ rand_diag_negative(a.gen, k, j));
-        v.y = __uint_as_float(__float_as_uint(v.y) ^ rand_diag_negative(a.gen, k, j + 1));
-        v.z = __uint_as_float(__float_as_uint(v.z) ^ rand_diag_negative(a.gen, k, j + 2));
-        v.w = __uint_as_float(__float_as_uint(v.w) ^ rand_diag_negative(a.gen, k, j + 3));
-        return;
-    }
     if (!a.sign) return;
     if (a.sign_bits) {
         const uint32_t w = static_cast<const uint32_t *>(a.sign)[g >> 5] >> (g & 31);
@@ -99,6 +98,19 @@ __device__ __forceinline__ void flip4(float4 &v, const RhtTileArgs &a, int64_t g
         const float4 s = *reinterpret_cast<const float4 *>(static_cast<const float *>(a.sign) + g);
         v.x *= s.x; v.y *= s.y; v.z *= s.z; v.w *= s.w;
     }
+}
+
+__device__ __forceinline__ void flip4(float4 &v, const RhtPassArgs &a, int64_t g)
+{
+    if (a.gen.bits != 0) {
+        const uint32_t k = (uint32_t)(g >> a.gen.bits), j = (uint32_t)g & ((1u << a.gen.bits) - 1u); // the four share a segment
+        v.x = __uint_as_float(__float_as_uint(v.x) ^ rand_diag_negative(a.gen, k, j));
+        v.y = __uint_as_float(__float_as_uint(v.y) ^ rand_diag_negative(a.gen, k, j + 1));
+        v.z = __uint_as_float(__float_as_uint(v.z) ^ rand_diag_negative(a.gen, k, j + 2));
+        v.w = __uint_as_float(__float_as_uint(v.w) ^ rand_diag_negative(a.gen, k, j + 3));
+        return;
+    }
+    flip4(v, static_cast<const RhtTileArgs &>(a), g);
 }
 
 __device__ __forceinline__ float flip1(float v, const RhtTileArgs &a, int64_t g)
@@ -314,9 +326,12 @@ __global__ void irht_decompress_kernel(const uint8_t *__restrict__ src, float *_
 // ---- quantisers folded into the ends of the plain transform (TransformEnds) ------------------------------------
 
 // the sign flip of a chunk that is already in registers (g a multiple of 16; 16-byte accesses to a float sign vector)
-__device__ __forceinline__ void flip16(float (&v)[16], const RhtTileArgs &a, int64_t g)
+__device__ __forceinline__ bool has_diagonal(const RhtTileArgs &a) { return a.sign != nullptr; }
+__device__ __forceinline__ bool has_diagonal(const RhtPassArgs &a) { return a.sign || a.gen.bits != 0; }
+
+template <class A> __device__ __forceinline__ void flip16(float (&v)[16], const A &a, int64_t g)
 {
-    if (!a.sign && a.gen.bits == 0) return;
+    if (!has_diagonal(a)) return;
 #pragma unroll
     for (int k = 0; k < 4; k++) {
         float4 q = make_float4(v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3]);
@@ -432,12 +447,14 @@ __device__ __forceinline__ void load_planes(float (&v)[16], const TransformEnds 
 // centroids of EDEN's bins, read from the bit planes (srrcomp.py:343-354); then the sign flip of a forward transform.
 // cen: the centroid table in LDS.
 template <bool ENDS>
-__device__ __forceinline__ void fetch_chunk(float (&v)[16], const float *__restrict__ x, const RhtTileArgs &in,
+__device__ __forceinline__ void fetch_chunk(float (&v)[16], const float *__restrict__ x, const PassArgs<ENDS> &in,
                                             const TransformEnds &e, const float *cen, int64_t g)
 {
     if (!ENDS || (!e.in_levels && !e.in_planes && !e.in_src)) {
         load_chunk(v, x, in, g);
-        if (ENDS && in.gen.bits != 0) flip16(v, in, g);
+        if constexpr (ENDS) {
+            if (in.gen.bits != 0) flip16(v, in, g);
+        }
         return;
     }
     if (g >= in.n) {
@@ -470,7 +487,7 @@ __device__ __forceinline__ void fetch_chunk(float (&v)[16], const float *__restr
 // four consecutive elements of the last pass on their way out: scale, sign flip of an inverse transform, EDEN's scale,
 // then the float store or THC's quantiser (thc_hooks.py:161-166) and a bf16 store
 template <bool ENDS>
-__device__ __forceinline__ void store4(float *__restrict__ x, float4 v, const RhtTileArgs &a, const TransformEnds &e, int sign_mode,
+__device__ __forceinline__ void store4(float *__restrict__ x, float4 v, const PassArgs<ENDS> &a, const TransformEnds &e, int sign_mode,
                                        int apply_scale, int64_t g)
 {
     if (apply_scale) { v.x *= a.scale; v.y *= a.scale; v.z *= a.scale; v.w *= a.scale; }
@@ -502,16 +519,16 @@ __device__ __forceinline__ void store4(float *__restrict__ x, float4 v, const Rh
 // sign_mode: 0 no flip, 1 flip on load, 2 flip on store
 // ENDS: a quantiser may sit at either end (TransformEnds; 16-byte accesses only: a.vec is set)
 template <bool ENDS>
-__device__ __forceinline__ void tile_pass(float *__restrict__ x, const RhtTileArgs &a, int sign_mode, int apply_scale,
+__device__ __forceinline__ void tile_pass(float *__restrict__ x, const PassArgs<ENDS> &a, int sign_mode, int apply_scale,
                                           const TransformEnds &e, unsigned block, float *lds)
 {
     const int tid = threadIdx.x, nthreads = blockDim.x;
     const int tile = 1 << a.kt;
     const int64_t origin = (int64_t)block << a.kt;
-    RhtTileArgs in = a;
+    PassArgs<ENDS> in = a;
     if (sign_mode != 1) {
         in.sign = nullptr;
-        in.gen.bits = 0;
+        if constexpr (ENDS) in.gen.bits = 0;
     }
     const float *cen = lds + padded_tile_floats(a.kt); // EDEN's centroids sit behind the tile
     if (ENDS && e.in_planes) {
@@ -561,7 +578,7 @@ __device__ __forceinline__ void tile_pass(float *__restrict__ x, const RhtTileAr
 }
 
 template <bool ENDS>
-__global__ void rht_tile_kernel(float *__restrict__ x, RhtTileArgs a, int sign_mode, int apply_scale, TransformEnds e)
+__global__ void rht_tile_kernel(float *__restrict__ x, PassArgs<ENDS> a, int sign_mode, int apply_scale, TransformEnds e)
 {
     extern __shared__ __attribute__((aligned(16))) float lds[];
     tile_pass<ENDS>(x, a, sign_mode, apply_scale, e, blockIdx.x, lds);
@@ -573,7 +590,7 @@ __global__ void rht_tile_kernel(float *__restrict__ x, RhtTileArgs a, int sign_m
 // a wave covers two whole 128-byte row segments), does the four lowest row stages on its registers and leaves the other
 // rbits - 4 (at most 6) to one or two LDS passes.  sign_mode: 0, or 2 = flip on store (the last pass of an inverse).
 template <bool ENDS>
-__device__ __forceinline__ void strided_pass(float *__restrict__ x, const RhtTileArgs &a, int rbits, int sbits, int sign_mode,
+__device__ __forceinline__ void strided_pass(float *__restrict__ x, const PassArgs<ENDS> &a, int rbits, int sbits, int sign_mode,
                                              int apply_scale, const TransformEnds &e, unsigned block, float *lds)
 {
     const int tid = threadIdx.x, nthreads = blockDim.x;
@@ -639,7 +656,7 @@ __device__ __forceinline__ void strided_pass(float *__restrict__ x, const RhtTil
 }
 
 template <bool ENDS>
-__global__ void rht_strided_kernel(float *__restrict__ x, RhtTileArgs a, int rbits, int sbits, int sign_mode, int apply_scale,
+__global__ void rht_strided_kernel(float *__restrict__ x, PassArgs<ENDS> a, int rbits, int sbits, int sign_mode, int apply_scale,
                                    TransformEnds e)
 {
     extern __shared__ __attribute__((aligned(16))) float lds[];
@@ -662,9 +679,9 @@ __device__ __forceinline__ const TilePass &pass_of_block(const PassSet &set)
     return set.p[k];
 }
 
-__device__ __forceinline__ RhtTileArgs pass_args(const TilePass &p)
+__device__ __forceinline__ RhtPassArgs pass_args(const TilePass &p)
 {
-    RhtTileArgs a;
+    RhtPassArgs a;
     a.sign = nullptr; a.sign_bits = 0; a.n = p.n; a.kt = p.kt; a.kb = p.kb; a.scale = p.scale; a.vec = 1; a.gen = p.ends.gen;
     return a;
 }
@@ -1115,16 +1132,17 @@ hipError_t launch_rht_tile(float *x, const void *sign, int sign_bits, int64_t n,
     if (kt < 10 || kt > 15 || kb > kt || kb < 0) return hipErrorInvalidValue;
     const bool plain = ends.plain();
     if (!plain && (!vec || (n & 31) != 0)) return hipErrorInvalidValue;
-    RhtTileArgs a;
+    RhtPassArgs a;
     a.sign = sign; a.sign_bits = sign_bits; a.n = n; a.kt = kt; a.kb = kb; a.scale = scale; a.vec = vec; a.gen = ends.gen;
     const bool diagonal = sign || ends.gen.bits != 0;
+    const RhtTileArgs &plain_args = a;
     const int tile = 1 << kt;
     if (plain && kt == kSplitBits && kb == kSplitBits && (n & (tile - 1)) == 0) {
         // whole blocks of 2^15: half the LDS, two workgroups per CU
         const size_t half_lds = (size_t)padded_tile_floats(kHalfBits) * sizeof(float);
         hipError_t es = allow_lds(rht_tile_split_kernel, half_lds);
         if (es != hipSuccess) return es;
-        hipLaunchKernelGGL(rht_tile_split_kernel, dim3((unsigned)(n >> kSplitBits)), dim3(kSplitThreads), half_lds, stream, x, a,
+        hipLaunchKernelGGL(rht_tile_split_kernel, dim3((unsigned)(n >> kSplitBits)), dim3(kSplitThreads), half_lds, stream, x, plain_args,
                            sign ? sign_mode : 0, apply_scale);
         return hipGetLastError();
     }
@@ -1134,7 +1152,7 @@ hipError_t launch_rht_tile(float *x, const void *sign, int sign_bits, int64_t n,
     if (plain) {
         hipError_t e = allow_lds(rht_tile_kernel<false>, lds);
         if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(rht_tile_kernel<false>, grid, dim3(threads), lds, stream, x, a, sign ? sign_mode : 0, apply_scale, ends);
+        hipLaunchKernelGGL(rht_tile_kernel<false>, grid, dim3(threads), lds, stream, x, plain_args, sign ? sign_mode : 0, apply_scale, ends);
     } else {
         hipError_t e = allow_lds(rht_tile_kernel<true>, lds);
         if (e != hipSuccess) return e;
@@ -1150,8 +1168,9 @@ hipError_t launch_rht_strided(float *x, const void *sign, int sign_bits, int64_t
     if (rbits < 4 || rbits > 10 || sbits < 5 || (n & (((int64_t)1 << (sbits + rbits)) - 1)) != 0) return hipErrorInvalidValue;
     const bool plain = ends.plain_out() && ends.gen.bits == 0;
     if (!plain && !vec) return hipErrorInvalidValue;
-    RhtTileArgs a;
+    RhtPassArgs a;
     a.sign = sign; a.sign_bits = sign_bits; a.n = n; a.kt = rbits + 5; a.kb = 0; a.scale = scale; a.vec = vec; a.gen = ends.gen;
+    const RhtTileArgs &plain_args = a;
     const int tile = 1 << (rbits + 5);
     const unsigned threads = (unsigned)std::min(1024, tile / 16);
     const size_t lds = (size_t)padded_tile_floats(rbits + 5) * sizeof(float);
@@ -1159,7 +1178,7 @@ hipError_t launch_rht_strided(float *x, const void *sign, int sign_bits, int64_t
     if (plain) {
         hipError_t e = allow_lds(rht_strided_kernel<false>, lds);
         if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(rht_strided_kernel<false>, grid, dim3(threads), lds, stream, x, a, rbits, sbits, sign ? sign_mode : 0,
+        hipLaunchKernelGGL(rht_strided_kernel<false>, grid, dim3(threads), lds, stream, x, plain_args, rbits, sbits, sign ? sign_mode : 0,
                            apply_scale, ends);
     } else {
         hipError_t e = allow_lds(rht_strided_kernel<true>, lds);
