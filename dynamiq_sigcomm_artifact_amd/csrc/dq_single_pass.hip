@@ -286,35 +286,45 @@ struct RankPointers {
 };
 
 constexpr int kStatsWaves = 8; // ranks in flight per workgroup of ranks_stats_kernel
+// From so many tiles (of all ranks) on a wave takes two of a rank and has both on their way before it adds up the first: 454 ->
+// 409 us for 8 x 121,524 tiles.  Below, the second tile is better in a wave of its own.
+constexpr int64_t kStatsTwoTiles = 32768;
 
-// A workgroup takes a tile of four superchunks, a wave of it the tile of one rank (of every kStatsWaves-th one in a larger
+// A workgroup takes TILES tiles of four superchunks, a wave of it the tiles of one rank (of every kStatsWaves-th one in a larger
 // world): means and norms per rank, and the statistics all-reduce as the reference's chain of bf16 additions in rank order.
-template <int DT>
+template <int DT, int TILES>
 __global__ __launch_bounds__(64 * kStatsWaves) void ranks_stats_kernel(RankPointers ranks, int world, int64_t n, int vec,
                                                                       uint32_t *__restrict__ total, float *__restrict__ mean_out,
                                                                       WorldDiv wd)
 {
     extern __shared__ __attribute__((aligned(16))) uint8_t tiles[];
-    __shared__ uint32_t pairs[kMaxRanks][kRowsPerWave];
+    __shared__ uint32_t pairs[kMaxRanks][TILES * kRowsPerWave];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
     const int row = lane >> 4, j = lane & 15;
     const int64_t nsc = (n + 255) >> 8;
-    const int64_t sc0 = (int64_t)blockIdx.x * kRowsPerWave;
-    const int rows_here = (int)min((int64_t)kRowsPerWave, nsc - sc0);
-    const int64_t sc = sc0 + min(row, rows_here - 1);
-    const bool ragged = (sc0 + kRowsPerWave) * 256 > n;
+    const int64_t sc0 = (int64_t)blockIdx.x * (TILES * kRowsPerWave);
+    const int rows_here = (int)min((int64_t)(TILES * kRowsPerWave), nsc - sc0);
+    const bool ragged = (sc0 + TILES * kRowsPerWave) * 256 > n;
     uint8_t *lds = tiles + wave * StatsTile<DT>::BYTES;
     for (int rank = wave; rank < world; rank += waves) {
-        Raw16<DT> v;
-        v.zero();
-        if (row < rows_here) load_chunk<DT>(v, ranks.src[rank], sc * 256 + j * 16, n, vec != 0, ragged);
-        float sum, sq;
-        tile_sums<DT>(v, wd, lds, lane, sum, sq);
-        wave_lds_sync();
-        if (j == 0) {
-            const float mean = superchunk_mean(sum, sc * 256, n, ragged);
-            pairs[rank][row] = f32_to_bf16_bits(mean) | (f32_to_bf16_bits(sq) << 16);
-            if (row < rows_here) mean_out[rank * nsc + sc] = mean;
+        Raw16<DT> v[TILES];
+#pragma unroll
+        for (int t = 0; t < TILES; t++) {
+            const int r = t * kRowsPerWave + row;
+            v[t].zero();
+            if (r < rows_here) load_chunk<DT>(v[t], ranks.src[rank], (sc0 + r) * 256 + j * 16, n, vec != 0, ragged);
+        }
+#pragma unroll
+        for (int t = 0; t < TILES; t++) {
+            const int r = t * kRowsPerWave + row;
+            float sum, sq;
+            tile_sums<DT>(v[t], wd, lds, lane, sum, sq);
+            wave_lds_sync();
+            if (j == 0 && r < rows_here) {
+                const float mean = superchunk_mean(sum, (sc0 + r) * 256, n, ragged);
+                pairs[rank][r] = f32_to_bf16_bits(mean) | (f32_to_bf16_bits(sq) << 16);
+                mean_out[rank * nsc + sc0 + r] = mean;
+            }
         }
     }
     __syncthreads();
@@ -520,16 +530,22 @@ hipError_t launch_ranks_stats(const void *const *src, int world, int64_t n, void
         if (r < world && !aligned16(src[r])) vec = 0;
     }
     const int64_t nsc = (n + 255) / 256;
-    const dim3 grid((unsigned)((nsc + kRowsPerWave - 1) / kRowsPerWave));
+    const int64_t one = (nsc + kRowsPerWave - 1) / kRowsPerWave;
+    const bool two = one * world >= kStatsTwoTiles;
+    const dim3 grid((unsigned)(two ? (one + 1) / 2 : one));
     const int waves = world < kStatsWaves ? world : kStatsWaves;
     const WorldDiv wd = make_world_div(world, dtype == DQ_F32 ? 4 : 2);
     uint32_t *tot = static_cast<uint32_t *>(total);
-    if (dtype == DQ_BF16)
-        hipLaunchKernelGGL(ranks_stats_kernel<DQ_BF16>, grid, dim3(64 * waves), waves * StatsTile<DQ_BF16>::BYTES, stream, p, world, n, vec,
-                           tot, mean, wd);
-    else
-        hipLaunchKernelGGL(ranks_stats_kernel<DQ_F32>, grid, dim3(64 * waves), waves * StatsTile<DQ_F32>::BYTES, stream, p, world, n, vec,
-                           tot, mean, wd);
+    const dim3 block(64 * waves);
+    if (dtype == DQ_BF16) {
+        const size_t lds = waves * StatsTile<DQ_BF16>::BYTES;
+        if (two) hipLaunchKernelGGL((ranks_stats_kernel<DQ_BF16, 2>), grid, block, lds, stream, p, world, n, vec, tot, mean, wd);
+        else hipLaunchKernelGGL((ranks_stats_kernel<DQ_BF16, 1>), grid, block, lds, stream, p, world, n, vec, tot, mean, wd);
+    } else {
+        const size_t lds = waves * StatsTile<DQ_F32>::BYTES;
+        if (two) hipLaunchKernelGGL((ranks_stats_kernel<DQ_F32, 2>), grid, block, lds, stream, p, world, n, vec, tot, mean, wd);
+        else hipLaunchKernelGGL((ranks_stats_kernel<DQ_F32, 1>), grid, block, lds, stream, p, world, n, vec, tot, mean, wd);
+    }
     return hipGetLastError();
 }
 

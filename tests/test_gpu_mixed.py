@@ -803,3 +803,11 @@ def test_bucket_seen_before_is_checked_again(capi):
     torch.cuda.synchronize()
     for k, (v, o) in enumerate(((x, out), (big, result))):
         assert torch.equal(bits_t(o), bits_t(_four_calls(capi, v, v.numel(), 6.0, 2, 3, (k << 32) + 1)[5]))
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("W,n", [(8, 1024 * 4096), (8, 1024 * 4097 - 300), (8, 1024 * 4095), (9, 1024 * 3642 + 257)])
+def test_statistics_of_two_tiles_per_wave(capi, W, n, dt):
+    """around 2^15 tiles of all ranks, where a wave of the statistics takes two of them: an odd number of tiles, a ragged last one,
+    more ranks than a workgroup has waves"""
+    test_ranks_in_registers_equal_the_ring_in_steps(capi, W, n, dt)
