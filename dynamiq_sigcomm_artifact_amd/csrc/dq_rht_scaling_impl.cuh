@@ -60,7 +60,8 @@ struct RhtTileArgs {
 };
 
 // The diagonal drawn where it is applied (sign is then null); flip4 and flip16 serve it.  A type of its own: the kernels
-// fused with the codec run on 64 registers, and a test for a seed that they never have costs them time (2^30 elements there and back 2134 -> 2118 us without it).
+// fused with the codec run on 64 registers, and a test for a seed that they never have costs them time (2^30 elements there
+// and back 2134 -> 2118 us without it).
 struct RhtPassArgs : RhtTileArgs {
     SignSeed gen;
 };

@@ -12,10 +12,10 @@
 //   ranks_stats_kernel W ranks: every rank's means, and the reduced statistics
 //   ring_kernel        W ranks, after a plan of the reduced statistics: the ring
 //
-// Measured, start -> now (bit-identical results): 8 ranks x 124,439,808 bf16 elements 2,884 -> 1,186 us per all-reduce (one
+// Measured, start -> now (bit-identical results): 8 ranks x 124,439,808 bf16 elements 2,896 -> 1,143 us per all-reduce (one
 // launch per rank and ring step, packed streams and their exchange copies, against three launches whose traffic is the
-// vectors alone), 8 x 1,000,003 elements 1,493 -> 31 us (257 launches against 3), a step of nine 25 MB buckets on one rank
-// 250 -> 102 us (four launches per bucket on two streams against two launches per step, and the search for u).
+// vectors alone), 8 x 1,000,003 elements 1,488 -> 32 us (257 launches against 3), a step of nine 25 MB buckets on one rank
+// 252 -> 60 us (four launches per bucket on two streams against two launches per step, and the search for u).
 //
 // Numerics: csrc/cuda_hadamard.cu:1257-1369 (centring, mean add), csrc/cuda_hierarchical_mee.cu:203-696 (codec),
 // testbed_evaluation/new_comm_hooks/ring_rdma.py:590-631 (order of the ring), comm_hooks.py:64-70 (widths).
