@@ -34,7 +34,8 @@ __global__ __launch_bounds__(kHistThreads) void norm_histogram_kernel(const uint
 // turned into suffix counts in registers and lands in LDS, and a round of probes asks for up to eight values of u at once,
 // one pair of waves each: the seven midpoints of the next three steps of the bisection, or the next eight corrections, which
 // all follow from the first probe's deficit.  The walk through them is the reference's, probe by probe.
-// Kernel time of a converged correction (one probe): 39.7 -> 10.7 us.  With the events around it and 200,000 norms: one probe
+// Kernel time of a converged correction (one probe): 39.7 -> 10.4 us, 9.0 with the first round's thresholds found while the
+// histogram is on its way.  With the events around it and 200,000 norms: one probe
 // 48 -> 17 us, a bisection of ten probes 60 -> 24 us.
 constexpr int kBins = 32768;                     // >= kNanBin + 1
 constexpr int kSlabs = kBins / (4 * kSearchThreads);
@@ -69,6 +70,7 @@ __global__ __launch_bounds__(kSearchThreads) void bitrate_search_kernel(uint32_t
     __shared__ uint32_t at_least[2][kProbes]; // norms of width >= 4, >= 8
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
 
+    if (prev_u_dev) prev_u = *prev_u_dev; // (the first load: waited for alone; read by every thread long before thread 0 writes out[])
     uint4 v[kSlabs]; // bins 4 (t + 1024 k) ..
     // (read, then left zeroed for the next accumulation)
     if ((reinterpret_cast<uintptr_t>(hist) & 15) == 0) {
@@ -85,7 +87,34 @@ __global__ __launch_bounds__(kSearchThreads) void bitrate_search_kernel(uint32_t
             h[0] = h[1] = h[2] = h[3] = 0u;
         }
     }
-    if (prev_u_dev) prev_u = *prev_u_dev; // read by every thread long before thread 0 writes out[]
+    // the thresholds of a value of u, for the wave's share of them; they need nothing of the histogram, so those of the first
+    // round are found while it is on its way
+    const double u_min = -10.0, u_max = 60.0, tol = 0.1;
+    const int pair = wave >> 1;
+    const auto find = [&](double mine) {
+        const float u = (float)mine;
+        const int64_t width = (wave & 1) ? 8 : 4;
+        int p = kMaxPattern + 1;
+        const int a = first_width_probe(u, -1, 512, lane, width);
+        if (a < 64) {
+            const int lo = -1 + 512 * a;
+            const int lo2 = lo + 8 * first_width_probe(u, lo, 8, lane, width);
+            p = lo2 + 1 + first_width_probe(u, lo2, 1, lane, width);
+        }
+        return p;
+    };
+    // the midpoint of this pair's node below [l, h]
+    const auto node_mid = [&](double l, double h) {
+        double mid = (l + h) * 0.5;
+        for (int bit = pair >= 4 ? 1 : (pair >= 2 ? 0 : -1); bit >= 0; bit--) { // from the root down
+            if ((pair >> bit) & 1) h = mid;
+            else l = mid;
+            mid = (l + h) * 0.5;
+        }
+        return mid;
+    };
+    const double start = __builtin_fmax(u_min, __builtin_fmin(u_max, prev_u));
+    const int p_first = find(mode == 0 ? (pair == 0 ? u_max : node_mid(u_min, u_max)) : start);
     uint32_t incl[kSlabs];
 #pragma unroll
     for (int k = 0; k < kSlabs; k++) {
@@ -123,17 +152,8 @@ __global__ __launch_bounds__(kSearchThreads) void bitrate_search_kernel(uint32_t
 
     // every thread evaluates the same doubles, so the control flow below is uniform without a broadcast
     int probes = 0;
-    // one round: candidate[k] for k < count (waves 2 k and 2 k + 1 find its thresholds)
-    const auto round = [&](double mine) { // mine: the u of this wave's pair
-        const float u = (float)mine;
-        const int64_t width = (wave & 1) ? 8 : 4;
-        int p = kMaxPattern + 1;
-        const int a = first_width_probe(u, -1, 512, lane, width);
-        if (a < 64) {
-            const int lo = -1 + 512 * a;
-            const int lo2 = lo + 8 * first_width_probe(u, lo, 8, lane, width);
-            p = lo2 + 1 + first_width_probe(u, lo2, 1, lane, width);
-        }
+    // one round: waves 2 k and 2 k + 1 hold the thresholds of candidate k
+    const auto publish = [&](int p) {
         __syncthreads(); // the previous round has been read
         if (lane == 0) at_least[wave & 1][wave >> 1] = p <= kMaxPattern ? suffix[p] : 0u;
         __syncthreads();
@@ -146,8 +166,6 @@ __global__ __launch_bounds__(kSearchThreads) void bitrate_search_kernel(uint32_t
         r.delta = target - r.avg;
         return r;
     };
-    const double u_min = -10.0, u_max = 60.0, tol = 0.1;
-    const int pair = wave >> 1;
     double res_u, res_avg, res_delta;
     if (mode == 0) {
         // comm_hooks.py:94-114.  A round holds the nodes 1 .. 7 of the tree of the next three midpoints (node h: below it
@@ -155,14 +173,7 @@ __global__ __launch_bounds__(kSearchThreads) void bitrate_search_kernel(uint32_t
         double low = u_min, high = u_max, best_u = high, best_avg = 0.0, best_delta = 0.0;
         bool done = false, first = true;
         for (int it = 0; it < 32 && !done;) {
-            double l = low, h = high;
-            double mid = (l + h) * 0.5;
-            for (int bit = pair >= 4 ? 1 : (pair >= 2 ? 0 : -1); bit >= 0; bit--) { // this pair's node from the root down
-                if ((pair >> bit) & 1) h = mid;
-                else l = mid;
-                mid = (l + h) * 0.5;
-            }
-            round(pair == 0 ? high : mid);
+            publish(first ? p_first : find(pair == 0 ? high : node_mid(low, high)));
             if (first) {
                 const Probe r = result(0);
                 best_avg = r.avg;
@@ -191,8 +202,7 @@ __global__ __launch_bounds__(kSearchThreads) void bitrate_search_kernel(uint32_t
         res_u = best_u; res_avg = best_avg; res_delta = best_delta;
     } else {
         // comm_hooks.py:117-139
-        const double start = __builtin_fmax(u_min, __builtin_fmin(u_max, prev_u));
-        round(start);
+        publish(p_first);
         Probe r = result(0);
         res_u = start; res_avg = r.avg; res_delta = r.delta;
         if (!(__builtin_fabs(r.delta) <= tol)) {
@@ -202,7 +212,7 @@ __global__ __launch_bounds__(kSearchThreads) void bitrate_search_kernel(uint32_t
             for (int it = 0; it < 32 && !done; it += kProbes) {
                 double mine = step;
                 for (int k = 0; k < pair; k++) mine *= 0.5;
-                round(__builtin_fmax(u_min, __builtin_fmin(u_max, start + mine)));
+                publish(find(__builtin_fmax(u_min, __builtin_fmin(u_max, start + mine))));
                 for (int k = 0; k < kProbes && !done; k++) {
                     const double cand = __builtin_fmax(u_min, __builtin_fmin(u_max, start + step));
                     r = result(k);

@@ -15,7 +15,7 @@
 // Measured, start -> now (bit-identical results): 8 ranks x 124,439,808 bf16 elements 2,896 -> 1,143 us per all-reduce (one
 // launch per rank and ring step, packed streams and their exchange copies, against three launches whose traffic is the
 // vectors alone), 8 x 1,000,003 elements 1,488 -> 32 us (257 launches against 3), a step of nine 25 MB buckets on one rank
-// 252 -> 60 us (four launches per bucket on two streams against two launches per step, and the search for u).
+// 252 -> 59 us (four launches per bucket on two streams against two launches per step, and the search for u).
 //
 // Numerics: csrc/cuda_hadamard.cu:1257-1369 (centring, mean add), csrc/cuda_hierarchical_mee.cu:203-696 (codec),
 // testbed_evaluation/new_comm_hooks/ring_rdma.py:590-631 (order of the ring), comm_hooks.py:64-70 (widths).
@@ -216,12 +216,13 @@ struct TallyArgs {
 };
 
 // A workgroup takes kTallyBatch superchunks of one bucket.  A wave's norms are alike and meet in a few counters of the LDS, so the
-// counting is better spread over more workgroups: 209,716 norms with 8192 each 7.9 us, 4096 6.6, 2048 and 1024 6.4.
+// counting is better spread over more workgroups: 209,716 norms with 8192 each 7.9 us, 4096 6.6, 2048 and 1024 6.4 (5.9 since
+// the thresholds are searched beside the counting).
 constexpr int kTallyThreads = 1024, kTallyBatch = 2048;
 
 template <bool HIST> __global__ __launch_bounds__(kTallyThreads) void tally_kernel(TallyArgs a)
 {
-    __shared__ uint32_t local[HIST ? kHistWords : 1];
+    __shared__ __attribute__((aligned(16))) uint32_t local[HIST ? kHistWords : 4];
     __shared__ int thr[2];
     __shared__ uint32_t total[2];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -237,14 +238,26 @@ template <bool HIST> __global__ __launch_bounds__(kTallyThreads) void tally_kern
 #pragma unroll
     for (int k = 0; k < kPer; k++) norm[k] = mine[2 * min(k * kTallyThreads + (int)threadIdx.x, have - 1)];
     const float u = a.rule.u_dev ? (float)*a.rule.u_dev : a.rule.u;
+    if (threadIdx.x < 2) total[threadIdx.x] = 0u;
+    if (HIST) {
+        uint4 *l4 = reinterpret_cast<uint4 *>(local);
+        for (int w = threadIdx.x; w < kHistWords / 4; w += kTallyThreads) l4[w] = make_uint4(0u, 0u, 0u, 0u);
+        __syncthreads();
+    }
+    // two waves search the thresholds while the others count
     if (a.rule.thr[0] >= 0) {
         if (threadIdx.x < 2) thr[threadIdx.x] = a.rule.thr[threadIdx.x];
     } else {
         width_thresholds(u, thr, wave, lane);
     }
-    if (threadIdx.x < 2) total[threadIdx.x] = 0u;
     if (HIST) {
-        for (int w = threadIdx.x; w < kHistWords; w += kTallyThreads) local[w] = 0u;
+#pragma unroll
+        for (int k = 0; k < kPer; k++) {
+            if (k * kTallyThreads + (int)threadIdx.x < have) {
+                const int bin = bin_of(norm[k]);
+                atomicAdd(&local[bin >> 1], 1u << (16 * (bin & 1)));
+            }
+        }
     }
     __syncthreads();
     const int t2[2] = {thr[0], thr[1]};
@@ -255,10 +268,6 @@ template <bool HIST> __global__ __launch_bounds__(kTallyThreads) void tally_kern
         const int c = class_of_norm(norm[k], u, t2);
         n8 += (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(in && c == 0));
         n4 += (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(in && c == 1));
-        if (HIST && in) {
-            const int bin = bin_of(norm[k]);
-            atomicAdd(&local[bin >> 1], 1u << (16 * (bin & 1)));
-        }
     }
     if (lane == 0 && n8) atomicAdd(&total[0], n8);
     if (lane == 0 && n4) atomicAdd(&total[1], n4);
@@ -271,6 +280,7 @@ template <bool HIST> __global__ __launch_bounds__(kTallyThreads) void tally_kern
         if (blockIdx.x == 0 && a.step_dev && a.step_more) *a.step_dev += a.step_more;
     }
     if (HIST) {
+        // (a word per thread: the counters in use lie side by side)
         for (int w = threadIdx.x; w < kHistWords; w += kTallyThreads) {
             const uint32_t pair = local[w];
             if (pair & 0xffffu) atomicAdd(&a.hist[2 * w], pair & 0xffffu);
