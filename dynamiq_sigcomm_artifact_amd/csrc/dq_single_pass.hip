@@ -415,46 +415,31 @@ template <int DT, int RDT, bool MEE> __global__ __launch_bounds__(64) void ring_
     const WidthRegs<MEE> w = width_regs<MEE>(a.widths, cls, levels);
     const uint32_t total_mean = a.total[2 * sc];
 
-    // The elements (and random values) of the next kAhead ranks are on their way while this rank's are quantised.  Two ranks
-    // ahead instead of one: 735 -> 725 us at 8 x 124,439,808; with random values to load as well the registers are worth more
-    // (two ranks of 6,553,523 elements 16.4 -> 17.6 us).
-    constexpr int kAhead = RDT == DQ_PHILOX ? 2 : 1;
-    Raw16<DT> ahead[kAhead];
-    Raw16<RDT> ahead_r[kAhead];
-    float ahead_mean[kAhead];
-#pragma unroll
-    for (int k = 0; k < kAhead; k++) {
-        ahead[k].zero();
-        ahead_r[k].zero();
-        ahead_mean[k] = 0.0f;
-    }
-    const auto fetch = [&](int step, int slot) {
+    // the next rank's elements (and random values) are on their way while this rank's are quantised
+    Raw16<DT> next;
+    Raw16<RDT> next_r;
+    float next_mean = 0.0f;
+    next.zero();
+    next_r.zero();
+    const auto fetch = [&](int step) {
         int rank = chunk + step;
         if (rank >= world) rank -= world;
         if (active) {
-            load_chunk<DT>(ahead[slot], a.src[rank], e0, a.n, a.vec & 1, ragged);
-            ahead_mean[slot] = a.mean[(int64_t)rank * a.nsc + sc];
+            load_chunk<DT>(next, a.src[rank], e0, a.n, a.vec & 1, ragged);
+            next_mean = a.mean[(int64_t)rank * a.nsc + sc];
             if constexpr (RDT != DQ_PHILOX)
-                ahead_r[slot].load(a.pools.pool[cls][rank], ((int64_t)a.pools.first[cls][rank][step] + k0 * 16 + lane) * 16, (a.vec & 4) != 0);
+                next_r.load(a.pools.pool[cls][rank], ((int64_t)a.pools.first[cls][rank][step] + k0 * 16 + lane) * 16, (a.vec & 4) != 0);
         }
     };
-#pragma unroll
-    for (int k = 0; k < kAhead; k++)
-        if (k < world) fetch(k, k);
+    fetch(0);
     Raw16<DT> v;
     float lev[16], scale = 0.0f;
 #pragma unroll 1
     for (int step = 0; step < world; step++) {
-        v = ahead[0];
-        Raw16<RDT> r = ahead_r[0];
-        const float mean = ahead_mean[0];
-#pragma unroll
-        for (int k = 0; k + 1 < kAhead; k++) {
-            ahead[k] = ahead[k + 1];
-            ahead_r[k] = ahead_r[k + 1];
-            ahead_mean[k] = ahead_mean[k + 1];
-        }
-        if (step + kAhead < world) fetch(step + kAhead, kAhead - 1);
+        v = next;
+        Raw16<RDT> r = next_r;
+        const float mean = next_mean;
+        if (step + 1 < world) fetch(step + 1);
         if constexpr (RDT == DQ_PHILOX) {
             int rank = chunk + step;
             if (rank >= world) rank -= world;
