@@ -12,7 +12,7 @@
 //   ranks_stats_kernel W ranks: every rank's means, and the reduced statistics
 //   ring_kernel        W ranks, after a plan of the reduced statistics: the ring
 //
-// Measured, start -> now (bit-identical results): 8 ranks x 124,439,808 bf16 elements 2,896 -> 1,143 us per all-reduce (one
+// Measured, start -> now (bit-identical results): 8 ranks x 124,439,808 bf16 elements 2,896 -> 1,149 us per all-reduce (one
 // launch per rank and ring step, packed streams and their exchange copies, against three launches whose traffic is the
 // vectors alone), 8 x 1,000,003 elements 1,488 -> 32 us (257 launches against 3), a step of nine 25 MB buckets on one rank
 // 252 -> 59 us (four launches per bucket on two streams against two launches per step, and the search for u).
@@ -297,8 +297,9 @@ struct RankPointers {
 
 constexpr int kStatsWaves = 8; // ranks in flight per workgroup of ranks_stats_kernel
 // From so many tiles (of all ranks) on a wave takes two of a rank and has both on their way before it adds up the first: 454 ->
-// 409 us for 8 x 121,524 tiles.  Below, the second tile is better in a wave of its own: 8.2 -> 8.8 us for 2 x 6,400.
-constexpr int64_t kStatsTwoTiles = 32768;
+// 409 us for 8 x 121,524 tiles.  Below, the second tile is better in a wave of its own: 8.2 -> 8.8 us for 2 x 6,400 (the whole
+// all-reduce of 4 x 15,625: 72.2 -> 73.6 us; of 8 x 15,625 135.5 -> 134.3, about where the two meet).
+constexpr int64_t kStatsTwoTiles = (int64_t)1 << 17;
 
 // A workgroup takes TILES tiles of four superchunks, a wave of it the tiles of one rank (of every kStatsWaves-th one in a larger
 // world): means and norms per rank, and the statistics all-reduce as the reference's chain of bf16 additions in rank order.
