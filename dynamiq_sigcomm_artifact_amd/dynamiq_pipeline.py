@@ -416,8 +416,9 @@ class SinglePassBuckets(object):
 
     The offset u of the width rule is read from device memory when a launch runs (``set_u`` or a float64 tensor of the
     caller's, e.g. the result of the offset search), and the rounding stream of the encoder is (seed, bucket ordinal *
-    2^32 + the step counter in device memory): ``begin_step`` once per training step makes the next launch advance the
-    counter, so a replayed launch draws fresh random values on every step.
+    2^32 + the step counter in device memory): ``begin_step`` once per training step advances the counter, with the next
+    launch or, once launches of the object have been recorded into a graph, at once -- a replay draws fresh random values
+    if begin_step was recorded with it or is called before it.
 
     run(x, out) enqueues a bucket and returns at once; join() makes the caller's current stream wait for everything
     enqueued so far.  The caller must not overwrite x or read out before join()."""
