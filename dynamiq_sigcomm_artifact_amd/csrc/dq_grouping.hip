@@ -670,8 +670,10 @@ __global__ __launch_bounds__(kThreads) void plan_place_stats_kernel(WidthsFromSt
 // -- a counting sort.  As in plan_one_kernel no workgroup waits for another: the workgroup of tile b (256
 // superchunks) counts the keys of the whole bucket itself, in an LDS histogram (128 KB, 144 KB with its padding),
 // in two steps: first the superchunks before its tile (the counter of key_i is then the part of E(i) that lies in
-// earlier tiles), then the rest; an in-place exclusive scan of the histogram gives G.  The part of E inside the tile
-// comes from comparing the tile's keys with each other.  nsc <= 65535, so no counter overflows.
+// earlier tiles), then the rest; an in-place exclusive scan of the histogram gives G.  In between the tile's own four
+// waves take turns: a wave reads its counters and adds its keys, and inside a wave the lanes with the same key find one
+// another by a ballot per bit of the key.  (Comparing all 256 keys of the tile with each other, as first written: 12.4 us
+// instead of 11.0 for 25,600 superchunks.)  nsc <= 65535, so no counter overflows.
 //
 // Sort key (ascending key = descending norm, as torch.sort orders floats): NaN (either sign) first, then +inf ...
 // +0 = -0 ... -inf.
@@ -788,53 +790,51 @@ template <bool WIDE>
 __device__ __forceinline__ void sorted_plan_body(const uint32_t *__restrict__ pairs, int nsc, int top, int bottom,
                                                  int64_t *__restrict__ qbits_out, int32_t *__restrict__ order,
                                                  const uint32_t (&cached)[kSortBatch], uint32_t own_pattern, uint32_t *hist,
-                                                 uint16_t *tile_key, int (*part_rank)[kSortTile], uint32_t *wave_sum)
+                                                 uint32_t *wave_sum)
 {
-    const int t = threadIdx.x;
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int nbefore = (int)blockIdx.x * kSortTile;
-    const int e = t & (kSortTile - 1), part = t / kSortTile; // element of the tile, quarter of its predecessors
-    const int own = nbefore + e;
+    const int own = nbefore + t; // of the first kSortTile threads
     const int valid = min(kSortTile, nsc - nbefore);
-    const uint32_t key = e < valid ? sort_key<WIDE>(own_pattern) : 0u;
-    if (part == 0) tile_key[e] = (uint16_t)key;
-    __syncthreads(); // the zeroed histogram and the tile's keys are in place
+    const bool mine = t < valid;
+    const uint32_t key = sort_key<WIDE>(own_pattern);
 
-    // superchunks of the tile with the same key and a smaller index: quarter `part` of the candidates (the quarters
-    // behind the element's own hold none)
-    {
-        int r = 0;
-        const int j0 = part * (kSortTile / 4);
-        if (j0 <= e) {
-            const uint4 *k4 = reinterpret_cast<const uint4 *>(tile_key + j0);
+    // lanes of the wave that hold the same key
+    uint64_t same = 0;
+    if (wave < kSortTile / 64) {
+        same = __builtin_amdgcn_ballot_w64(mine);
 #pragma unroll
-            for (int q = 0; q < kSortTile / 4 / 8; q++) {
-                const uint4 v = k4[q]; // the same address in every lane: a broadcast
-                const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-                for (int h = 0; h < 8; h++) {
-                    const int j = j0 + 8 * q + h;
-                    const uint32_t kj = (w[h >> 1] >> (16 * (h & 1))) & 0xffffu;
-                    r += (kj == key && j < e) ? 1 : 0;
-                }
-            }
+        for (int bit = 0; bit < (WIDE ? 16 : 15); bit++) {
+            const bool set = (key >> bit) & 1u;
+            const uint64_t with = __builtin_amdgcn_ballot_w64(set);
+            same &= set ? with : ~with;
         }
-        part_rank[part][e] = r;
     }
+    const uint64_t lower = same & (((uint64_t)1 << lane) - 1u);
     count_keys<WIDE>(pairs, 0, nbefore, hist, cached);
     __syncthreads();
     int same_before = 0;
-    if (part == 0 && e < valid) {
-        same_before = counter_of<WIDE>(hist, key);
 #pragma unroll
-        for (int q = 0; q < kSortThreads / kSortTile; q++) same_before += part_rank[q][e];
+    for (int w = 0; w < kSortTile / 64; w++) {
+        if (wave == w && mine) {
+            same_before = counter_of<WIDE>(hist, key) + (int)__popcll(lower);
+            __builtin_amdgcn_wave_barrier(); // every lane has read before any adds
+            if (lower == 0) {
+                const uint32_t many = (uint32_t)__popcll(same);
+                if (WIDE)
+                    atomicAdd(&hist[hist_slot(key >> 1)], many << (16 * (key & 1)));
+                else
+                    atomicAdd(&hist[hist_slot(key)], many);
+            }
+        }
+        __syncthreads();
     }
-    __syncthreads();
-    count_keys<WIDE>(pairs, nbefore, nsc, hist, cached);
+    count_keys<WIDE>(pairs, nbefore + valid, nsc, hist, cached);
     __syncthreads();
     scan_counters<WIDE>(hist, wave_sum);
     __syncthreads();
 
-    if (part == 0 && e < valid) {
+    if (mine) {
         const int pos = counter_of<WIDE>(hist, key) + same_before;
         const int mid_end = nsc - bottom;
         int region, at;
@@ -851,8 +851,6 @@ __global__ __launch_bounds__(kSortThreads) void sorted_plan_kernel(const uint32_
                                                                   int32_t *__restrict__ order, int32_t *__restrict__ work)
 {
     __shared__ __align__(16) uint32_t hist[kSortLdsWords];
-    __shared__ __align__(16) uint16_t tile_key[kSortTile];
-    __shared__ int part_rank[kSortThreads / kSortTile][kSortTile];
     __shared__ uint32_t wave_sum[kSortThreads / 64];
     __shared__ int any_negative;
     const int t = threadIdx.x;
@@ -864,8 +862,8 @@ __global__ __launch_bounds__(kSortThreads) void sorted_plan_kernel(const uint32_
         const int i = j * kSortThreads + t;
         cached[j] = i < nsc ? pairs[i] : 0u;
     }
-    const int own = (int)blockIdx.x * kSortTile + (t & (kSortTile - 1));
-    const uint32_t own_pattern = own < nsc ? pairs[own] >> 16 : 0u;
+    const int own = (int)blockIdx.x * kSortTile + t;
+    const uint32_t own_pattern = t < kSortTile && own < nsc ? pairs[own] >> 16 : 0u;
     {
         uint4 *h4 = reinterpret_cast<uint4 *>(hist);
         for (int w = t; w < kSortLdsWords / 4; w += kSortThreads) h4[w] = make_uint4(0u, 0u, 0u, 0u);
@@ -882,9 +880,9 @@ __global__ __launch_bounds__(kSortThreads) void sorted_plan_kernel(const uint32_
     if (__builtin_amdgcn_ballot_w64(negative) != 0 && (t & 63) == 0) any_negative = 1;
     __syncthreads();
     if (any_negative)
-        sorted_plan_body<true>(pairs, nsc, top, bottom, qbits_out, order, cached, own_pattern, hist, tile_key, part_rank, wave_sum);
+        sorted_plan_body<true>(pairs, nsc, top, bottom, qbits_out, order, cached, own_pattern, hist, wave_sum);
     else
-        sorted_plan_body<false>(pairs, nsc, top, bottom, qbits_out, order, cached, own_pattern, hist, tile_key, part_rank, wave_sum);
+        sorted_plan_body<false>(pairs, nsc, top, bottom, qbits_out, order, cached, own_pattern, hist, wave_sum);
     if (blockIdx.x == 0 && t == 0) {
         work[0] = top;
         work[1] = nsc - top - bottom;
