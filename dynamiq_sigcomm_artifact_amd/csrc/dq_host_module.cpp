@@ -120,41 +120,47 @@ struct Buckets {
     uint64_t seed, pending = 0; // training steps begun since the last launch
     uint64_t base = 0;          // steps that the counter in device memory never gets
     bool recorded = false;      // a graph with launches of this object may exist
-    py::object step_dev, u_dev, hist, stats, counts;
+    py::object step_dev, u_dev, hist, counts, stats, spare;
     uint64_t *step_ptr = nullptr;
     const double *u_ptr = nullptr;
     uint32_t *hist_ptr = nullptr;
     int64_t hist_ints = 0;
+    int32_t *counts_ptr = nullptr, *spare_ptr = nullptr; // rows of four: of the slots, and of buckets beside them
     char *stats_ptr = nullptr;
-    int64_t stats_room = 0, counts_room = 0;
-    int32_t *counts_ptr = nullptr;
+    int64_t counts_rows = 0, stats_room = 0, spare_rows = 0;
     hipStream_t last = nullptr; // of the last eager launch
     bool used = false;
     std::vector<hipStream_t> kept_for; // streams beside the one that the tensors were made on
     hipStream_t last_recorded = nullptr; // of the last launch of the recording with this id
     unsigned long long recording = 0;
 
-    Buckets(int strategy_, uint64_t seed_, py::object step, py::object u, py::object h) : strategy(strategy_), seed(seed_)
+    Buckets(int strategy_, uint64_t seed_, py::object step, py::object u, py::object h, py::object counts_)
+        : strategy(strategy_), seed(seed_)
     {
         Args a;
         step_ptr = reinterpret_cast<uint64_t *>(a.typed(step, at::kLong, 1, "step counter").data_ptr());
         u_ptr = a.typed(u, at::kDouble, 1, "u").data_ptr<double>();
         hist_ptr = hist_of(a, h, &hist_ints);
+        const at::Tensor &c = a.typed(counts_, at::kInt, 4, "counts");
+        counts_ptr = c.data_ptr<int32_t>();
+        counts_rows = c.numel() / 4;
         device = a.device;
         step_dev = step;
         u_dev = u;
         hist = h;
+        counts = counts_;
     }
-    void scratch(py::object stats_, py::object counts_)
+    // scratch that grows.  A recorded launch has the addresses of its day: whoever replaces the tensors keeps the old ones.
+    void scratch(py::object stats_, py::object spare_)
     {
         Args a;
-        const at::Tensor &s = a.typed(stats_, at::kBFloat16, 0, "stats"), &c = a.typed(counts_, at::kInt, 0, "counts");
+        const at::Tensor &s = a.typed(stats_, at::kBFloat16, 0, "stats"), &c = a.typed(spare_, at::kInt, 0, "spare counts");
         stats_ptr = static_cast<char *>(s.data_ptr());
-        counts_ptr = c.data_ptr<int32_t>();
+        spare_ptr = c.data_ptr<int32_t>();
         stats_room = s.numel() / 2;
-        counts_room = c.numel() / 4;
+        spare_rows = c.numel() / 4;
         stats = stats_;
-        counts = counts_;
+        spare = spare_;
         kept_for.clear();
     }
     // is s recording a graph, and which?
@@ -172,7 +178,7 @@ struct Buckets {
     {
         if (std::find(kept_for.begin(), kept_for.end(), s) != kept_for.end()) return;
         const py::object stream = py::module_::import("torch.cuda").attr("current_stream")(device);
-        for (const py::object *o : {&step_dev, &u_dev, &hist, &stats, &counts})
+        for (const py::object *o : {&step_dev, &u_dev, &hist, &counts, &stats, &spare})
             if (*o && !o->is_none()) o->attr("record_stream")(stream);
         kept_for.push_back(s);
     }
@@ -224,7 +230,7 @@ struct Batch {
     std::vector<dq_roundtrip_t> desc;
     int dtype = DQ_BF16;
 
-    // rows: where each bucket's counts go
+    // rows: where each bucket's counts go, those of the slots first, then the spare ones
     Batch(Buckets &b, py::sequence pairs, const std::vector<uint64_t> &steps, const std::vector<int64_t> &rows)
     {
         const size_t count = py::len(pairs);
@@ -245,8 +251,9 @@ struct Batch {
             d.out = out.data_ptr();
             d.n = x.numel();
             d.stats = b.stats_ptr + 4 * at;
-            if (rows[k] < 0 || rows[k] >= b.counts_room) refuse("buckets and scratch do not match");
-            d.counts = b.counts_ptr + 4 * rows[k];
+            const int64_t spare = rows[k] - b.counts_rows;
+            if (rows[k] < 0 || spare >= b.spare_rows) refuse("buckets and scratch do not match");
+            d.counts = spare < 0 ? b.counts_ptr + 4 * rows[k] : b.spare_ptr + 4 * spare;
             d.step = steps[k];
             at += (d.n + 255) / 256;
             desc.push_back(d);
@@ -923,7 +930,8 @@ PYBIND11_MODULE(_host, m)
     m.def("thc_decompress", &thc_decompress);
     m.doc() = "native host path of dynamiq_sigcomm_artifact_amd";
     py::class_<Buckets>(m, "Buckets")
-        .def(py::init<int, uint64_t, py::object, py::object, py::object>())
+        .def(py::init<int, uint64_t, py::object, py::object, py::object, py::object>())
+        .def_readonly("recorded", &Buckets::recorded)
         .def("scratch", &Buckets::scratch)
         .def("join", &Buckets::join)
         .def("begin_step", &Buckets::begin_step);

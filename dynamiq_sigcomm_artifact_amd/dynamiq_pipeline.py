@@ -434,14 +434,15 @@ class SinglePassBuckets(object):
                                                                      device=self.device)
         self.hist = norm_histogram
         self._host = capi.host()
+        self._counts = torch.zeros((self.slots, 4), dtype=torch.int32, device=self.device)
         self._buckets = self._host.Buckets(strategy, self.seed & _U64, self.step_dev, self.u_dev,
-                                           None if norm_histogram is None else norm_histogram.hist)
-        self._room = (0, 0)
-        self._stats = self._counts = None
+                                           None if norm_histogram is None else norm_histogram.hist, self._counts)
+        self._room = (0, 0)      # superchunks and buckets that the scratch holds
+        self._scratch = None     # statistics; counts of the buckets that are not the last of their slot
+        self._replaced = []      # scratch that a recorded graph may still write to
         self._last = None        # the list run_all saw last: (batch, superchunks)
         self.cache = {}          # addresses and sizes of a list of buckets -> (batch, superchunks, slots)
         self.ordinals = {}       # (x.data_ptr(), n) -> ordinal of the bucket in the random stream
-        self._rows = {}          # slot -> row of the counts of its last bucket
         self.superchunks = 0
 
     def _pick(self):
@@ -469,35 +470,41 @@ class SinglePassBuckets(object):
         self._buckets.begin_step()
 
     # ---- per bucket ---------------------------------------------------------------------------------------------
-    def _batch(self, pairs, key, one):
-        """lays out a list of buckets seen for the first time (or again after the scratch grew).  The counts of a bucket of
-        run() have the row of its slot, those of a list the rows behind."""
-        sizes = [(x.numel() + SUPERCHUNK - 1) // SUPERCHUNK for x, _ in pairs]
-        total = sum(sizes)
-        rows = self.slots + (0 if one else len(pairs))
-        if total > self._room[0] or rows > self._room[1]:
-            self.join()
-            self._room = (max(total, self._room[0]), max(rows, self._room[1]))
-            self._stats = torch.empty((self._room[0], 2), dtype=torch.bfloat16, device=self.device)
-            counts = torch.zeros((self._room[1], 4), dtype=torch.int32, device=self.device)
-            if self._counts is not None:
-                counts[:self._counts.shape[0]].copy_(self._counts)
-            self._counts = counts
-            self._buckets.scratch(self._stats, self._counts)
-            self.cache.clear()       # what was laid out over the old buffers
-            self._last = None
+    def _grow(self, superchunks, buckets):
+        """scratch for so many superchunks and buckets.  A recorded graph goes on writing to the scratch of its day: from the
+        first recording on, replaced scratch is kept as long as the object, and grows to at least twice, so that all of the
+        replaced together stay below the present."""
+        self.join()
+        factor = 1
+        if self._buckets.recorded and self._scratch is not None:
+            factor = 2
+            self._replaced.append(self._scratch)
+        self._room = (max(superchunks, factor * self._room[0]), max(buckets, factor * self._room[1]))
+        self._scratch = (torch.empty((self._room[0], 2), dtype=torch.bfloat16, device=self.device),
+                         torch.empty((self._room[1], 4), dtype=torch.int32, device=self.device))
+        self._buckets.scratch(*self._scratch)
+        self.cache.clear()       # what was laid out over the old buffers
+        self._last = None
+
+    def _batch(self, pairs, key):
+        """lays out a list of buckets seen for the first time (or again after the scratch grew)"""
+        total = sum((x.numel() + SUPERCHUNK - 1) // SUPERCHUNK for x, _ in pairs)
         # a source keeps its ordinal, and with it its random stream and its slot, from step to step
         ordinals = [self.ordinals.setdefault((x.data_ptr(), x.numel()), len(self.ordinals)) for x, _ in pairs]
         slots = [o % self.slots for o in ordinals]
-        rows = slots if one else range(self.slots, self.slots + len(pairs))
-        batch = self._host.Batch(self._buckets, pairs, [(o << 32) & _U64 for o in ordinals], list(rows))
-        entry = self.cache[key] = (batch, total, dict(zip(slots, rows)))
+        # the counts of a slot are those of its last bucket
+        last = {slot: k for k, slot in enumerate(slots)}
+        rows = [slot if last[slot] == k else self.slots + k for k, slot in enumerate(slots)]
+        spare = max(rows) + 1 - self.slots
+        if total > self._room[0] or spare > self._room[1]:
+            self._grow(total, max(0, spare))
+        batch = self._host.Batch(self._buckets, pairs, [(o << 32) & _U64 for o in ordinals], rows)
+        entry = self.cache[key] = (batch, total, slots[0])
         return entry
 
     def _enqueue(self, entry):
-        batch, superchunks, rows = entry
+        batch, superchunks, _ = entry
         batch.launch(self._buckets)
-        self._rows.update(rows)
         if self.hist is not None:
             self.hist.count += superchunks
         self.superchunks += superchunks
@@ -507,9 +514,9 @@ class SinglePassBuckets(object):
         key = (x.data_ptr(), out.data_ptr(), x.numel(), x.dtype)
         entry = self.cache.get(key)
         if entry is None or not entry[0].matches([(x, out)]):
-            entry = self._batch([(x, out)], key, True)
+            entry = self._batch([(x, out)], key)
         self._enqueue(entry)
-        return next(iter(entry[2]))
+        return entry[2]
 
     def run_all(self, pairs):
         """enqueue a whole step's buckets, [(x, out), ...]"""
@@ -520,13 +527,13 @@ class SinglePassBuckets(object):
             key = tuple((x.data_ptr(), o.data_ptr(), x.numel(), x.dtype) for x, o in pairs)
             last = self.cache.get(key)
             if last is None or not last[0].matches(list(map(tuple, pairs))):
-                last = self._batch(pairs, key, False)
+                last = self._batch(pairs, key)
             self._last = last
         self._enqueue(last)
 
     def counts(self, k):
         """device int32 tensor [n8, n4, n2, other] of the last bucket of slot k"""
-        return self._counts[self._rows[k]]
+        return self._counts[k]
 
     def join(self):
         """the caller's current stream waits for everything enqueued so far"""

@@ -779,6 +779,42 @@ def test_recorded_step_draws_fresh_values(capi, inside):
             expect(step)
 
 
+@pytest.mark.parametrize("streams", [1, 2])
+def test_recorded_step_outlives_its_scratch(capi, streams):
+    """a step recorded before a larger bucket and a longer list have replaced the object's scratch: its replays write outputs and
+    counts of their own, and nothing into memory that the allocator has handed out since"""
+    from dynamiq_sigcomm_artifact_amd.dynamiq_pipeline import SinglePassBuckets
+    u, seed = 6.0, 13
+    pairs = [(x, torch.zeros_like(x)) for x in (_llama_like(n, n) for n in (256 * 50 - 7, 256 * 30, 256 * 41))]
+    pipe = SinglePassBuckets(DEV, strategy=2, seed=seed, streams=streams, u=u)
+    pipe.begin_step()
+    pipe.run_all(pairs)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        pipe.begin_step()
+        pipe.run_all(pairs)
+    room = pipe._room
+    more = [(x, torch.zeros_like(x)) for x in (_llama_like(n, n) for n in (256 * 4000, 256 * 3, 256 * 5, 256, 256 * 2))]
+    pipe.begin_step()
+    pipe.run_all(more)                                     # (step 2: the recording itself has run nothing)
+    assert pipe._room[0] > room[0] and pipe._room[1] > room[1]
+    torch.cuda.synchronize()
+    # whatever the allocator has to give of these sizes
+    canaries = [torch.full((room[0] * 2,), 7.0, dtype=torch.bfloat16, device=DEV) for _ in range(64)]
+    canaries += [torch.full((max(1, room[1]) * 4,), 7, dtype=torch.int32, device=DEV) for _ in range(64)]
+    for step in (3, 4, 5):
+        graph.replay()
+        torch.cuda.synchronize()
+        for k, (x, o) in enumerate(pairs):
+            want = _four_calls(capi, x, x.numel(), u, 2, seed, (k << 32) + step)
+            assert torch.equal(bits_t(o), bits_t(want[5])), (step, k)
+            if k + streams >= len(pairs):                  # the last bucket of its slot
+                assert pipe.counts(k % streams).tolist() == want[3][:4].tolist(), (step, k)
+            o.zero_()
+        assert all(bool((c == 7).all()) for c in canaries)
+
+
 def test_bucket_seen_before_is_checked_again(capi):
     """an output at a known address that has become too short is refused, not written beyond its end; scratch in use on two streams
     grows without disturbing either"""
