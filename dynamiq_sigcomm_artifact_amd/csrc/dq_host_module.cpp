@@ -128,7 +128,7 @@ struct Buckets {
     int32_t *counts_ptr = nullptr, *spare_ptr = nullptr; // rows of four: of the slots, and of buckets beside them
     char *stats_ptr = nullptr;
     int64_t counts_rows = 0, stats_room = 0, spare_rows = 0;
-    hipStream_t last = nullptr; // of the last eager launch
+    hipStream_t last = nullptr; // of the last eager launch, at first of the tensors' making
     bool used = false;
     std::vector<hipStream_t> kept_for; // streams beside the one that the tensors were made on
     hipStream_t last_recorded = nullptr; // of the last launch of the recording with this id
@@ -149,6 +149,7 @@ struct Buckets {
         u_dev = u;
         hist = h;
         counts = counts_;
+        follow(c10::hip::getCurrentHIPStream(device).stream()); // on which the caller has filled them
     }
     // scratch that grows.  A recorded launch has the addresses of its day: whoever replaces the tensors keeps the old ones.
     void scratch(py::object stats_, py::object spare_)

@@ -815,6 +815,53 @@ def test_recorded_step_outlives_its_scratch(capi, streams):
         assert all(bool((c == 7).all()) for c in canaries)
 
 
+@pytest.mark.parametrize("recorded", [False, True])
+def test_first_use_on_another_stream(capi, recorded):
+    """an object made on one stream, behind work that keeps it busy, and used on another without a word from the caller: its step
+    counter and u are there when the first launch reads them, likewise after set_u; eager, and made and used in one recording"""
+    from dynamiq_sigcomm_artifact_amd.dynamiq_pipeline import SinglePassBuckets
+    x = _llama_like(256 * 33, 3)
+    out, second = torch.zeros_like(x), torch.zeros_like(x)
+    maker, user, third = torch.cuda.Stream(), torch.cuda.Stream(), torch.cuda.Stream()
+    busy = torch.zeros(1 << 26, device=DEV)
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+
+    def whole():
+        if recorded:
+            for s in (user, third):
+                s.wait_stream(maker)
+        for _ in range(8):
+            busy.add_(1.0)
+        pipe = SinglePassBuckets(DEV, strategy=2, seed=2, u=6.0)
+        with torch.cuda.stream(user):
+            pipe.begin_step()
+            pipe.run(x, out)
+            pipe.join()
+            pipe.set_u(8.5)
+        with torch.cuda.stream(third):
+            pipe.run(x, second)
+        pipe.join()
+        return pipe
+
+    with torch.cuda.stream(maker):
+        if recorded:
+            with torch.cuda.graph(graph, stream=maker):
+                pipe = whole()
+        else:
+            pipe = whole()
+    for _ in range(3 if recorded else 1):
+        if recorded:
+            out.zero_()
+            second.zero_()
+            torch.cuda.synchronize()
+            graph.replay()
+        torch.cuda.synchronize()
+        for o, u in ((out, 6.0), (second, 8.5)):
+            assert torch.equal(bits_t(o), bits_t(_four_calls(capi, x, x.numel(), u, 2, 2, 1)[5])), u
+    del pipe
+
+
 def test_bucket_seen_before_is_checked_again(capi):
     """an output at a known address that has become too short is refused, not written beyond its end; scratch in use on two streams
     grows without disturbing either"""
