@@ -205,6 +205,7 @@ struct Buckets {
         used = true;
         return false;
     }
+    // the next launch is ordered behind s too: a replay on s right after this call is in order with the launches around it
     void join()
     {
         const hipStream_t s = c10::hip::getCurrentHIPStream(device).stream();

@@ -421,7 +421,14 @@ class SinglePassBuckets(object):
     if begin_step was recorded with it or is called before it.
 
     run(x, out) enqueues a bucket and returns at once; join() makes the caller's current stream wait for everything
-    enqueued so far.  The caller must not overwrite x or read out before join()."""
+    the object has enqueued so far.  The caller must not overwrite x or read out before join().
+
+    A graph that the caller records is replayed without the object knowing: it uses the object's memory (and is not replayed
+    any more once the object is gone), and ``superchunks`` and the histogram's ``count`` count its buckets once, at the
+    recording.  Replays and the object's own launches share the step counter and the statistics, so they have to follow one
+    another.  ``join()`` (or ``begin_step()``) on the stream of the replay just before it does that: the replay waits for
+    what the object has enqueued, and what the object enqueues afterwards, on whichever stream, waits for the replay.
+    Without it, and between replays on different streams, the order is the caller's to see to."""
 
     def __init__(self, device, strategy=2, seed=0, streams=2, graphs=True, u=None, norm_histogram=None, inline_first=True):
         from . import capi
@@ -536,5 +543,6 @@ class SinglePassBuckets(object):
         return self._counts[k]
 
     def join(self):
-        """the caller's current stream waits for everything enqueued so far"""
+        """the caller's current stream waits for everything that the object has enqueued so far, and the object's next launch
+        for what is on that stream by then (a graph replayed there, for instance)"""
         self._buckets.join()

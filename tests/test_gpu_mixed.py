@@ -862,6 +862,43 @@ def test_first_use_on_another_stream(capi, recorded):
     del pipe
 
 
+@pytest.mark.parametrize("inside", [False, True])
+def test_replays_in_order_with_eager_steps_on_another_stream(capi, inside):
+    """join() (begin_step() where it is not part of the recording) on the stream of a replay puts the replay into the object's order:
+    eager steps on another stream before and after it, no other wait between them"""
+    from dynamiq_sigcomm_artifact_amd.dynamiq_pipeline import SinglePassBuckets
+    u, seed = 6.0, 17
+    xs = [_llama_like(n, n) for n in (256 * 3000, 256 * 41 - 3)]
+    pairs = [(x, torch.zeros_like(x)) for x in xs]
+    other = [(x, torch.zeros_like(x)) for x in xs]
+    pipe = SinglePassBuckets(DEV, strategy=2, seed=seed, u=u)
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    busy = torch.zeros(1 << 24, device=DEV)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=a):
+        if inside:
+            pipe.begin_step()
+        pipe.run_all(pairs)
+    seen, step = [], 0
+    for _ in range(6):
+        with torch.cuda.stream(a):
+            busy.add_(1.0)                       # the replay starts late
+            pipe.join() if inside else pipe.begin_step()
+            graph.replay()
+            step += 1
+            seen.append((step, [o.clone() for _, o in pairs]))
+        with torch.cuda.stream(b):
+            pipe.begin_step()
+            step += 1
+            pipe.run_all(other)
+            seen.append((step, [o.clone() for _, o in other]))
+    torch.cuda.synchronize()
+    for step, outs in seen:
+        for k, (x, o) in enumerate(zip(xs, outs)):
+            assert torch.equal(bits_t(o), bits_t(_four_calls(capi, x, x.numel(), u, 2, seed, (k << 32) + step)[5])), (step, k)
+
+
 def test_bucket_seen_before_is_checked_again(capi):
     """an output at a known address that has become too short is refused, not written beyond its end; scratch in use on two streams
     grows without disturbing either"""
