@@ -109,7 +109,8 @@ uint32_t *hist_of(Args &a, py::handle h, int64_t *entries)
 // ---- buckets of one rank ----------------------------------------------------------------------------------
 
 // The state of a SinglePassBuckets object.  Its buckets share scratch and run on the caller's stream; a caller that comes
-// back on another stream is ordered behind the one before.
+// back on another stream is ordered behind the one before.  The object lets one thread in at a time: launch() gives up the
+// interpreter's lock between choosing the order and the steps and the launches that these belong to.
 //
 // A launch takes the steps begun since the last one along and advances the counter in device memory itself.  That holds for
 // eager launches only: a recorded launch is replayed without this object taking part.  So a step begun while recording is a

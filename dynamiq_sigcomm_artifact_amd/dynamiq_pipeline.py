@@ -12,6 +12,8 @@ over the simulated ranks here; with one rank the ring degenerates to
 compress -> decompress of the rank's own chunk (ring_rdma.py:606-621 with
 size == 1).
 """
+import threading
+
 import torch
 
 from . import bitrate
@@ -428,7 +430,10 @@ class SinglePassBuckets(object):
     recording.  Replays and the object's own launches share the step counter and the statistics, so they have to follow one
     another.  ``join()`` (or ``begin_step()``) on the stream of the replay just before it does that: the replay waits for
     what the object has enqueued, and what the object enqueues afterwards, on whichever stream, waits for the replay.
-    Without it, and between replays on different streams, the order is the caller's to see to."""
+    Without it, and between replays on different streams, the order is the caller's to see to.
+
+    Threads may share an object: its calls take turns (the steps that a launch takes along, the order of the launches and the
+    scratch belong together)."""
 
     def __init__(self, device, strategy=2, seed=0, streams=2, graphs=True, u=None, norm_histogram=None, inline_first=True):
         from . import capi
@@ -441,6 +446,7 @@ class SinglePassBuckets(object):
                                                                      device=self.device)
         self.hist = norm_histogram
         self._host = capi.host()
+        self._turn = threading.RLock()
         self._counts = torch.zeros((self.slots, 4), dtype=torch.int32, device=self.device)
         self._buckets = self._host.Buckets(strategy, self.seed & _U64, self.step_dev, self.u_dev,
                                            None if norm_histogram is None else norm_histogram.hist, self._counts)
@@ -469,12 +475,14 @@ class SinglePassBuckets(object):
     # ---- once per training step ----------------------------------------------------------------------------
     def set_u(self, u):
         """the offset of the width rule for the buckets enqueued from now on (a number; a tensor was given at construction)"""
-        self.join()
-        self.u_dev.fill_(float(u))
+        with self._turn:
+            self.join()
+            self.u_dev.fill_(float(u))
 
     def begin_step(self):
         """advance the step counter of the rounding stream: the next launch does it on its way"""
-        self._buckets.begin_step()
+        with self._turn:
+            self._buckets.begin_step()
 
     # ---- per bucket ---------------------------------------------------------------------------------------------
     def _grow(self, superchunks, buckets):
@@ -519,24 +527,26 @@ class SinglePassBuckets(object):
     def run(self, x, out):
         """enqueue one bucket: out = decode(encode(x)) with the widths of its reduced norms; returns its slot"""
         key = (x.data_ptr(), out.data_ptr(), x.numel(), x.dtype)
-        entry = self.cache.get(key)
-        if entry is None or not entry[0].matches([(x, out)]):
-            entry = self._batch([(x, out)], key)
-        self._enqueue(entry)
+        with self._turn:
+            entry = self.cache.get(key)
+            if entry is None or not entry[0].matches([(x, out)]):
+                entry = self._batch([(x, out)], key)
+            self._enqueue(entry)
         return entry[2]
 
     def run_all(self, pairs):
         """enqueue a whole step's buckets, [(x, out), ...]"""
-        last = self._last
-        if last is None or not last[0].matches(pairs):
-            if not pairs:
-                return
-            key = tuple((x.data_ptr(), o.data_ptr(), x.numel(), x.dtype) for x, o in pairs)
-            last = self.cache.get(key)
-            if last is None or not last[0].matches(list(map(tuple, pairs))):
-                last = self._batch(pairs, key)
-            self._last = last
-        self._enqueue(last)
+        with self._turn:
+            last = self._last
+            if last is None or not last[0].matches(pairs):
+                if not pairs:
+                    return
+                key = tuple((x.data_ptr(), o.data_ptr(), x.numel(), x.dtype) for x, o in pairs)
+                last = self.cache.get(key)
+                if last is None or not last[0].matches(list(map(tuple, pairs))):
+                    last = self._batch(pairs, key)
+                self._last = last
+            self._enqueue(last)
 
     def counts(self, k):
         """device int32 tensor [n8, n4, n2, other] of the last bucket of slot k"""
@@ -545,4 +555,5 @@ class SinglePassBuckets(object):
     def join(self):
         """the caller's current stream waits for everything that the object has enqueued so far, and the object's next launch
         for what is on that stream by then (a graph replayed there, for instance)"""
-        self._buckets.join()
+        with self._turn:
+            self._buckets.join()

@@ -899,6 +899,46 @@ def test_replays_in_order_with_eager_steps_on_another_stream(capi, inside):
             assert torch.equal(bits_t(o), bits_t(_four_calls(capi, x, x.numel(), u, 2, seed, (k << 32) + step)[5])), (step, k)
 
 
+def test_threads_share_an_object(capi):
+    """threads that enqueue buckets of one step, each on a stream of its own, with scratch that grows on the way: the step counter
+    advances once a step, and every bucket draws that step's values"""
+    import threading
+    from dynamiq_sigcomm_artifact_amd.dynamiq_pipeline import SinglePassBuckets
+    u, seed, steps, count = 6.0, 23, 6, 4
+    pipe = SinglePassBuckets(DEV, strategy=2, seed=seed, u=u)
+    xs = [[_llama_like(256 * (40 + 500 * t + 7 * k), 10 * t + k) for k in range(3)] for t in range(count)]
+    outs = [[[torch.zeros_like(x) for x in mine] for mine in xs] for _ in range(steps)]
+    for mine in xs:
+        for x in mine:
+            pipe.ordinals[(x.data_ptr(), x.numel())] = len(pipe.ordinals)     # whichever thread comes first
+    torch.cuda.synchronize()
+    failed = []
+
+    def work(t, step):
+        try:
+            with torch.cuda.stream(torch.cuda.Stream()):
+                for x, o in zip(xs[t], outs[step][t]):
+                    pipe.run(x, o)
+                pipe.run_all(list(zip(xs[t], outs[step][t])))
+        except Exception as exc:      # noqa: BLE001 (shown by the assertion below)
+            failed.append(exc)
+
+    for step in range(steps):
+        pipe.begin_step()
+        threads = [threading.Thread(target=work, args=(t, step)) for t in range(count)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join(60)
+    torch.cuda.synchronize()
+    assert not failed and int(pipe.step_dev) == steps
+    for step in range(steps):
+        for t in range(count):
+            for k, (x, o) in enumerate(zip(xs[t], outs[step][t])):
+                want = _four_calls(capi, x, x.numel(), u, 2, seed, ((3 * t + k) << 32) + step + 1)[5]
+                assert torch.equal(bits_t(o), bits_t(want)), (step, t, k)
+
+
 def test_bucket_seen_before_is_checked_again(capi):
     """an output at a known address that has become too short is refused, not written beyond its end; scratch in use on two streams
     grows without disturbing either"""

@@ -1,6 +1,8 @@
 """Host side of dynamiq_pipeline.SinglePassBuckets on the CPU, over a native module that notes what it is given: who keeps
 which memory, in which order launches are enqueued."""
 import gc
+import threading
+import time
 import weakref
 
 import pytest
@@ -96,3 +98,52 @@ def test_counts_of_a_slot_stay_where_they_are(host):
     pipe.run_all(_pairs(*([256 * 300] * 9)))
     assert [pipe.counts(k).data_ptr() for k in range(2)] == before
     assert pipe.run(*pairs[1]) == 1 and host.launches[-1][0].rows == [1]
+
+
+def test_threads_take_turns(host):
+    """a launch gives up the interpreter's lock in the middle: no other call of the object may come in between, and no scratch be
+    replaced under a launch that was laid out over it"""
+    pipe = SinglePassBuckets("cpu")
+    inside, met = [], []
+
+    def alone(body):
+        def call(*args):
+            inside.append(1)
+            if len(inside) > 1:
+                met.append(1)
+            time.sleep(0.002)
+            try:
+                return body(*args)
+            finally:
+                inside.pop()
+        return call
+
+    launch = host.Batch.launch
+
+    def over_its_scratch(batch, buckets):
+        stats = buckets.stats
+        time.sleep(0.002)
+        assert buckets.stats is stats
+        launch(batch, buckets)
+
+    host.Batch.launch = alone(over_its_scratch)
+    pipe._buckets.begin_step = alone(pipe._buckets.begin_step)
+    lists = [_pairs(256 * (8 + 300 * k), 256) for k in range(4)]
+    failed = []
+
+    def work(k):
+        try:
+            for _ in range(5):
+                pipe.begin_step()
+                pipe.run_all(lists[k])
+                pipe.run(*lists[k][0])
+                pipe.set_u(6.0)
+        except Exception as exc:      # noqa: BLE001 (shown by the assertion below)
+            failed.append(exc)
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(len(lists))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(60)
+    assert not failed and not met and len(host.launches) == 40
