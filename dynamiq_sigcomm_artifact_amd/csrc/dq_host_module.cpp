@@ -228,10 +228,14 @@ struct Buckets {
     }
 };
 
-// buckets that are enqueued together: addresses, not tensors (whoever calls launch() keeps those alive)
+// buckets that are enqueued with one call: addresses, not tensors (whoever calls launch() keeps those alive).  A run of
+// buckets of one element type shares launches; the runs follow one another in the list's order.
 struct Batch {
+    struct Run {
+        int dtype, count;
+    };
     std::vector<dq_roundtrip_t> desc;
-    int dtype = DQ_BF16;
+    std::vector<Run> runs;
 
     // rows: where each bucket's counts go, those of the slots first, then the spare ones
     Batch(Buckets &b, py::sequence pairs, const std::vector<uint64_t> &steps, const std::vector<int64_t> &rows)
@@ -246,9 +250,8 @@ struct Batch {
             a.device = b.device;
             const at::Tensor &x = a.tensor(p[0]), &out = a.tensor(p[1]);
             const int code = dtype_code(x);
-            if (k == 0) dtype = code;
-            if (code != dtype || out.scalar_type() != x.scalar_type() || out.numel() < x.numel())
-                refuse("the buckets of a list and their outputs must have one dtype, and every output its bucket's size");
+            if (out.scalar_type() != x.scalar_type() || out.numel() < x.numel())
+                refuse("an output must have its bucket's dtype and size");
             dq_roundtrip_t d;
             d.src = x.data_ptr();
             d.out = out.data_ptr();
@@ -260,6 +263,10 @@ struct Batch {
             d.step = steps[k];
             at += (d.n + 255) / 256;
             desc.push_back(d);
+            if (runs.empty() || runs.back().dtype != code)
+                runs.push_back(Run{code, 1});
+            else
+                runs.back().count++;
         }
         if (at > b.stats_room) refuse("buckets and scratch do not match");
     }
@@ -268,14 +275,17 @@ struct Batch {
     {
         PyObject *list = pairs.ptr();
         if (!PyList_CheckExact(list) || PyList_GET_SIZE(list) != (Py_ssize_t)desc.size()) return false;
-        for (size_t k = 0; k < desc.size(); k++) {
+        size_t run = 0;
+        int left = runs[0].count;
+        for (size_t k = 0; k < desc.size(); k++, left--) {
+            if (left == 0) left = runs[++run].count;
             PyObject *p = PyList_GET_ITEM(list, k);
             if (!PyTuple_CheckExact(p) || PyTuple_GET_SIZE(p) != 2) return false;
             PyObject *xo = PyTuple_GET_ITEM(p, 0), *oo = PyTuple_GET_ITEM(p, 1);
             if (!THPVariable_Check(xo) || !THPVariable_Check(oo)) return false;
             const at::Tensor &x = THPVariable_Unpack(xo), &out = THPVariable_Unpack(oo);
             if (x.data_ptr() != desc[k].src || out.data_ptr() != desc[k].out || x.numel() != desc[k].n || out.numel() < x.numel() ||
-                !x.is_contiguous() || !out.is_contiguous() || out.scalar_type() != x.scalar_type() || dtype_code(x) != dtype)
+                !x.is_contiguous() || !out.is_contiguous() || out.scalar_type() != x.scalar_type() || dtype_code(x) != runs[run].dtype)
                 return false;
         }
         return true;
@@ -284,7 +294,6 @@ struct Batch {
     {
         const hipStream_t s = c10::hip::getCurrentHIPStream(b.device).stream();
         b.follow(s);
-        const uint64_t more = b.pending;
         const dq_roundtrip_t *buckets = desc.data();
         std::vector<dq_roundtrip_t> moved;
         if (b.base) {
@@ -292,14 +301,18 @@ struct Batch {
             for (dq_roundtrip_t &d : moved) d.step += b.base;
             buckets = moved.data();
         }
-        int rc;
-        {
-            py::gil_scoped_release nogil;
-            rc = dq_bucket_roundtrip(buckets, (int)desc.size(), dtype, b.strategy, 1, 0.0, b.u_ptr, b.seed, b.step_ptr, more, b.hist_ptr,
-                                     b.hist_ints, b.device, s);
+        for (const Run &r : runs) {
+            const uint64_t more = b.pending; // (of the first run: it advances the counter)
+            int rc;
+            {
+                py::gil_scoped_release nogil;
+                rc = dq_bucket_roundtrip(buckets, r.count, r.dtype, b.strategy, 1, 0.0, b.u_ptr, b.seed, b.step_ptr, more, b.hist_ptr,
+                                         b.hist_ints, b.device, s);
+            }
+            check(rc);
+            b.pending -= more;
+            buckets += r.count;
         }
-        check(rc);
-        b.pending -= more;
     }
 };
 

@@ -939,6 +939,33 @@ def test_threads_share_an_object(capi):
                 assert torch.equal(bits_t(o), bits_t(want)), (step, t, k)
 
 
+@pytest.mark.parametrize("kinds", ["bf", "fbb", "bfbfb", "b" * 33 + "f" * 34 + "b"])
+def test_list_of_buckets_of_two_types(capi, kinds):
+    """bf16 and fp32 buckets in one list, one step counter for all of them: against the four calls bucket by bucket; the list is
+    recognised on later steps, and is not taken for one of another order of types"""
+    from dynamiq_sigcomm_artifact_amd.bitrate import NormHistogram
+    from dynamiq_sigcomm_artifact_amd.dynamiq_pipeline import SinglePassBuckets
+    types = {"b": torch.bfloat16, "f": torch.float32}
+    u, seed = 6.0, 19
+    xs = [_llama_like(256 * (3 + k % 5) - k % 3, 70 + k, types[t]) for k, t in enumerate(kinds)]
+    pairs = [(x, torch.zeros_like(x)) for x in xs]
+    hist = NormHistogram(DEV)
+    pipe = SinglePassBuckets(DEV, strategy=2, seed=seed, u=u, norm_histogram=hist)
+    for step in range(1, 4):
+        pipe.begin_step()
+        pipe.run_all(pairs)
+        torch.cuda.synchronize()
+        for k, (x, o) in enumerate(pairs):
+            want = _four_calls(capi, x, x.numel(), u, 2, seed, (k << 32) + step)
+            assert torch.equal(bits_t(o), bits_t(want[5])), (step, k)
+            o.zero_()
+        assert pipe.counts((len(pairs) - 1) % 2).tolist() == want[3][:4].tolist()
+    assert int(pipe.step_dev) == 3 and len(pipe.cache) == 1
+    nsc = sum((x.numel() + 255) // 256 for x in xs)
+    assert hist.count == 3 * nsc and int(hist.hist.sum()) == 3 * nsc
+    assert not pipe._last[0].matches(pairs[::-1])
+
+
 def test_bucket_seen_before_is_checked_again(capi):
     """an output at a known address that has become too short is refused, not written beyond its end; scratch in use on two streams
     grows without disturbing either"""
