@@ -229,11 +229,31 @@ struct Buckets {
 };
 
 // buckets that are enqueued with one call: addresses, not tensors (whoever calls launch() keeps those alive).  A run of
-// buckets of one element type shares launches; the runs follow one another in the list's order.
+// buckets of one element type that leave one another's memory alone shares launches; the runs follow one another in the
+// list's order, so a bucket may read what an earlier one of the list has written.
 struct Batch {
     struct Run {
         int dtype, count;
     };
+    struct Span {
+        uintptr_t begin, end;
+        bool meets(const Span &o) const { return begin < o.end && o.begin < end; }
+    };
+    // does bucket b write what a reads or writes, or read what a writes?
+    static bool clash(const Span &a_src, const Span &a_out, const Span &b_src, const Span &b_out)
+    {
+        return b_out.meets(a_src) || b_out.meets(a_out) || b_src.meets(a_out);
+    }
+    // do any two of the spans meet, those of one bucket aside?  (Sorted: each against the one that reaches furthest so far.)
+    static bool any_meet(std::vector<std::pair<Span, size_t>> spans)
+    {
+        std::sort(spans.begin(), spans.end(), [](const auto &a, const auto &b) { return a.first.begin < b.first.begin; });
+        for (size_t k = 1, far = 0; k < spans.size(); k++) {
+            if (spans[k].first.meets(spans[far].first) && spans[k].second != spans[far].second) return true;
+            if (spans[k].first.end > spans[far].first.end) far = k;
+        }
+        return false;
+    }
     std::vector<dq_roundtrip_t> desc;
     std::vector<Run> runs;
 
@@ -243,6 +263,8 @@ struct Batch {
         const size_t count = py::len(pairs);
         if (count == 0 || steps.size() != count || rows.size() != count) refuse("buckets and scratch do not match");
         int64_t at = 0;
+        std::vector<int> codes;
+        std::vector<std::pair<Span, size_t>> spans; // of source and output, one after the other
         for (size_t k = 0; k < count; k++) {
             const py::tuple p = py::cast<py::tuple>(pairs[k]);
             if (p.size() != 2) refuse("a bucket is a pair (x, out)");
@@ -263,10 +285,21 @@ struct Batch {
             d.step = steps[k];
             at += (d.n + 255) / 256;
             desc.push_back(d);
-            if (runs.empty() || runs.back().dtype != code)
-                runs.push_back(Run{code, 1});
-            else
+            codes.push_back(code);
+            for (const void *p : {d.src, static_cast<const void *>(d.out)}) {
+                const uintptr_t begin = reinterpret_cast<uintptr_t>(p);
+                spans.emplace_back(Span{begin, begin + (uintptr_t)d.n * x.element_size()}, k);
+            }
+        }
+        const bool meet = any_meet(spans);
+        for (size_t k = 0; k < count; k++) {
+            bool joins = !runs.empty() && runs.back().dtype == codes[k];
+            for (size_t i = joins && meet ? k - runs.back().count : k; joins && i < k; i++)
+                joins = !clash(spans[2 * i].first, spans[2 * i + 1].first, spans[2 * k].first, spans[2 * k + 1].first);
+            if (joins)
                 runs.back().count++;
+            else
+                runs.push_back(Run{codes[k], 1});
         }
         if (at > b.stats_room) refuse("buckets and scratch do not match");
     }
@@ -960,7 +993,12 @@ PYBIND11_MODULE(_host, m)
             return new Batch(b, pairs, s, at);
         }))
         .def("matches", &Batch::matches)
-        .def("launch", &Batch::launch);
+        .def("launch", &Batch::launch)
+        .def_property_readonly("runs", [](const Batch &b) {
+            py::list counts;
+            for (const Batch::Run &r : b.runs) counts.append(r.count);
+            return counts;
+        });
     m.def("roundtrip", &roundtrip);
     m.def("ranks_dynamic", &ranks_dynamic);
 }

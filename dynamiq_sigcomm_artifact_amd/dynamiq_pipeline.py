@@ -406,9 +406,10 @@ class SinglePassBuckets(object):
     on no other superchunk, so one launch makes one pass over the bucket, and over as many buckets as are at hand:
 
       * ``run(x, out)`` enqueues one bucket: two launches, the pass and the tally of its widths (and norms);
-      * ``run_all`` enqueues a whole step's buckets, two launches for every 32 of them (32 of a run of one element type, where
-        types change along the list).  DDP hands the hook the same bucket views on every step: the list is laid out once and
-        recognised afterwards.
+      * ``run_all`` enqueues a whole step's buckets, two launches for every 32 of them.  The results are those of run() on one
+        bucket after the other: where the element type changes along the list, or a bucket's memory is one that an earlier
+        one writes (or its output one that an earlier one reads), it starts launches of its own.  DDP hands the hook the same
+        bucket views on every step: the list is laid out once and recognised afterwards.
 
     Everything runs on the caller's current stream: a launch that fills the GPU gains nothing from a second stream beside
     it, and handing a bucket to another stream costs the host more than enqueueing it.  ``streams`` says how many slots

@@ -966,6 +966,40 @@ def test_list_of_buckets_of_two_types(capi, kinds):
     assert not pipe._last[0].matches(pairs[::-1])
 
 
+@pytest.mark.parametrize("shape", ["chain", "rewrite", "reuse", "overlap", "in place", "shared source", "views"])
+def test_list_of_buckets_that_share_memory(capi, shape):
+    """buckets of one list that read or write what another of the list writes give the results of one bucket after the other, and
+    those that share nothing (or a source) stay in one run of launches"""
+    from dynamiq_sigcomm_artifact_amd.dynamiq_pipeline import SinglePassBuckets
+    n, u, seed = 256 * 1024, 6.0, 29
+    base = _llama_like(6 * n, 31)
+    t = [base[k * n:(k + 1) * n] for k in range(6)]
+    pairs = {"chain": [(t[0], t[1]), (t[1], t[2]), (t[2], t[3])],
+             "rewrite": [(t[0], t[3]), (t[1], t[3]), (t[2], t[4])],
+             "reuse": [(t[0], t[2]), (t[1], t[0]), (t[0], t[4])],
+             "overlap": [(t[0], base[2 * n - 256:3 * n - 256]), (t[1], t[4]), (base[2 * n + 77:3 * n + 77], t[5])],
+             "in place": [(t[0], t[0]), (t[1], t[1]), (t[2], t[2])],
+             "shared source": [(t[0], t[2]), (t[0], t[3]), (t[1], t[4])],
+             "views": [(base[:n - 3], base[2 * n:3 * n - 3]), (base[n - 3:n], base[3 * n:3 * n + 3]), (t[1], t[4])]}[shape]
+    begin = base.clone()
+    want = begin.clone()
+
+    def of(copy, view):
+        at = (view.data_ptr() - base.data_ptr()) // base.element_size()
+        return copy[at:at + view.numel()]
+
+    pipe = SinglePassBuckets(DEV, strategy=2, seed=seed, u=u)
+    order = [pipe.ordinals.setdefault((x.data_ptr(), x.numel()), len(pipe.ordinals)) for x, _ in pairs]
+    for step in range(1, 4):
+        for (x, o), ordinal in zip(pairs, order):
+            of(want, o).copy_(_four_calls(capi, of(want, x).clone(), x.numel(), u, 2, seed, (ordinal << 32) + step)[5])
+        pipe.begin_step()
+        pipe.run_all(pairs)
+        torch.cuda.synchronize()
+        assert torch.equal(bits_t(base), bits_t(want)), step
+        assert pipe._last[0].runs == {"chain": [1, 1, 1], "rewrite": [1, 2], "reuse": [1, 1, 1], "overlap": [1, 2]}.get(shape, [3])
+
+
 def test_bucket_seen_before_is_checked_again(capi):
     """an output at a known address that has become too short is refused, not written beyond its end; scratch in use on two streams
     grows without disturbing either"""
