@@ -72,10 +72,10 @@ int dtype_code(const at::Tensor &t)
     }
 }
 
-// None: torch's current stream; a raw handle; a torch stream
-dq_stream_t stream_of(py::handle s)
+// None: torch's current stream, of that device if one is named; a raw handle; a torch stream
+dq_stream_t stream_of(py::handle s, int device = -1)
 {
-    if (s.is_none()) return c10::hip::getCurrentHIPStream().stream();
+    if (s.is_none()) return c10::hip::getCurrentHIPStream((c10::DeviceIndex)device).stream();
     if (PyLong_Check(s.ptr())) return reinterpret_cast<dq_stream_t>(PyLong_AsUnsignedLongLong(s.ptr()));
     return reinterpret_cast<dq_stream_t>(static_cast<uintptr_t>(py::cast<uint64_t>(s.attr("cuda_stream"))));
 }
@@ -367,7 +367,7 @@ void roundtrip(py::handle x, py::handle out, int64_t n, py::handle stats, py::ha
     const Offset o(a, u);
     int64_t hist_ints;
     uint32_t *h = hist_of(a, hist, &hist_ints);
-    const dq_stream_t s = stream_of(stream);
+    const dq_stream_t s = stream_of(stream, a.device);
     const int code = dtype_code(src);
     int rc;
     {
@@ -437,7 +437,7 @@ void ranks_dynamic(py::sequence vecs, py::sequence outs, int64_t n, py::handle t
     k.r.u_dev = o.dev;
     k.r.hist = hist_of(a, hist, &k.r.hist_ints);
     k.r.seed = seed;
-    k.enqueue(DQ_RANKS_STATS | DQ_RANKS_PLAN | DQ_RANKS_RING, a.device, stream_of(stream));
+    k.enqueue(DQ_RANKS_STATS | DQ_RANKS_PLAN | DQ_RANKS_RING, a.device, stream_of(stream, a.device));
 }
 
 // ---- compressor objects ------------------------------------------------------------------------------------

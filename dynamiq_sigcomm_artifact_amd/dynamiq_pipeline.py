@@ -267,6 +267,7 @@ def dynamic_bitrate_allreduce_single_pass(rank_vecs, u, strategy=2, seed=0, out=
 
     u: the offset of the width rule, a number or a float64 device tensor (e.g. result[0:1] of the offset search: then
     nothing of the step is read back).
+    stream: a torch stream or a raw handle; None: the current stream of the vectors' device.
     norm_histogram: a bitrate.NormHistogram that collects the reduced norms of the step's buckets for the search of
     the next step's u (comm_hooks.py:962, 904-931).
 

@@ -686,6 +686,30 @@ def test_ranks_in_registers_equal_the_ring_in_steps(capi, W, n, dt):
         assert all(torch.equal(bits_t(x), bits_t(y)) for x, y in zip(again, ref))
 
 
+@pytest.mark.parametrize("W", [1, 3])
+@pytest.mark.parametrize("elsewhere", [False, pytest.param(True, marks=pytest.mark.skipif(
+    not torch.cuda.is_available() or torch.cuda.device_count() < 2, reason="needs a second GPU"))])
+def test_all_reduce_runs_on_the_current_stream_of_the_vectors(capi, W, elsewhere):
+    """without a stream of the caller's the launches go to the current stream of the vectors' device, behind what is on it, also
+    where another device is the current one"""
+    from dynamiq_sigcomm_artifact_amd.dynamiq_pipeline import dynamic_bitrate_allreduce_single_pass
+    device = torch.device("cuda", 1 if elsewhere else 0)
+    vecs = [_llama_like(256 * 50 - 3, r).to(device) for r in range(W)]
+    want, _, _ = dynamic_bitrate_allreduce_single_pass([v * 2 for v in vecs], 6.0, seed=3, stream=torch.cuda.default_stream(device))
+    busy = torch.zeros(1 << 25, device=device)
+    side = torch.cuda.Stream(device=device)
+    torch.cuda.synchronize(device)
+    with torch.cuda.stream(side):                  # (makes the vectors' device current)
+        for _ in range(8):
+            busy.add_(1.0)
+        for v in vecs:
+            v.mul_(2)
+        with torch.cuda.device(0):
+            outs, _, _ = dynamic_bitrate_allreduce_single_pass(vecs, 6.0, seed=3)
+    torch.cuda.synchronize(device)
+    assert all(torch.equal(bits_t(x), bits_t(y)) for x, y in zip(outs, want))
+
+
 @pytest.mark.parametrize("u", [-4.0, 0.0, 3.984375, 6.0, 8.0, 15.5])
 def test_widths_of_every_norm_in_the_one_rank_pass(capi, u):
     """the width that the one-rank pass picks by its quick score equals the width rule's for every bf16 norm from 2^-63 to 2^62 --
