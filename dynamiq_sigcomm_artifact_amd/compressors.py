@@ -32,6 +32,9 @@ def record_geometry(nbits, chunk_size, supergroup=_SUPERGROUP):
     return chunk_size * supergroup, supergroup * (chunk_size * nbits // 8 + 1) + 2
 
 
+_ROW_CHOICE = ("rand_pool", "gen_next_rand")
+
+
 class _DynamicRangeGPUKern(object):
     strategy = 2
     given_pool_dtype = None           # dtype a pool passed in params["rand_pool_tensor"] is kept in (None: its own)
@@ -49,8 +52,10 @@ class _DynamicRangeGPUKern(object):
         self.three_times_cur_max_size = 3 * self.cur_max_size // self.nclients
         # the calls of the ring schedules, the LCG and the pools are the native object's: a call is 3 us of GPU time.
         # The reference module takes 2/4/8-bit codes and fp16/bf16 buffers; other widths and fp32 buffers on request only.
-        self._codec = capi.host().Codec(nbits, chunk_size, self.strategy, bool(params.get("extended", False)) or nbits not in (2, 4, 8),
-                                        (nbits * 998244353) & _U32, None, {})
+        self._extended = bool(params.get("extended", False)) or nbits not in (2, 4, 8)
+        self._codec = capi.host().Codec(nbits, chunk_size, self.strategy, self._extended, (nbits * 998244353) & _U32, None, {})
+        # a class that picks its rows itself is asked for them call by call
+        self._picks_rows = any(getattr(type(self), name) is not getattr(_DynamicRangeGPUKern, name) for name in _ROW_CHOICE)
         self.philox_seed = params.get("philox_seed")
         if self.philox_seed is not None:
             # one stream per rank, one step per call
@@ -69,6 +74,11 @@ class _DynamicRangeGPUKern(object):
                 pool = pool.to(dtype=self.given_pool_dtype)
         self.randomized_vec_pool = pool
         self.randomized_vec_pools[pool.dtype] = pool
+
+    def __setattr__(self, name, value):
+        object.__setattr__(self, name, value)
+        if name in _ROW_CHOICE:                         # an object of its own ways, likewise
+            object.__setattr__(self, "_picks_rows", True)
 
     # ---- state the reference's callers may read (and that the native object works with) ----------------------
     @property
@@ -134,8 +144,17 @@ class _DynamicRangeGPUKern(object):
     def _stream():
         return torch.cuda.current_stream().cuda_stream
 
+    def _with_rows(self, name, source, *buffers):
+        """the module's call on the rows that rand_pool() picks"""
+        n = source.numel()
+        if n:
+            call = getattr(self.eden_utils, name + "_ex" if self._extended else name)
+            call(*buffers, self.rand_pool(n, source.dtype), n, self.nbits, self.chunk_size, self._stream(), self.strategy)
+
     # ---- the calls of the ring schedules (:422-466) ------------------------------------------------------
     def compression(self, input_chunk, send_chunk, interm_chunk=None):
+        if self._picks_rows and self.philox_seed is None:
+            return self._with_rows("scaling_compress", input_chunk, input_chunk, send_chunk)
         self._codec.compress(input_chunk, send_chunk)
 
     def decompression(self, recv_chunk, input_chunk, interm_chunk=None):
@@ -145,6 +164,8 @@ class _DynamicRangeGPUKern(object):
         self._codec.decompress(recv_chunk, input_chunk, True)
 
     def dec_compression(self, recv_chunk, input_chunk, send_chunk, interm_chunk=None, interm_chunk2=None):
+        if self._picks_rows and self.philox_seed is None:
+            return self._with_rows("scaling_dec_comp", input_chunk, recv_chunk, input_chunk, send_chunk)
         self._codec.dec_comp(recv_chunk, input_chunk, send_chunk)
 
     # ---- the same steps over a list of superchunk indices: index_select + the call above + index_copy_

@@ -80,7 +80,7 @@ def _pooled_codecs(rank_vecs, compressors):
         return None
     every = [c for q in (8, 4, 2) for c in compressors.get(q, ())]
     if not all(type(c) in (Aee_Dynamic_Range_GPU_kern, Mee_Dynamic_Range_GPU_kern) and c.philox_seed is None and c.chunk_size == 16 and
-               c.strategy == every[0].strategy for c in every):
+               c.strategy == every[0].strategy and not c._picks_rows for c in every):
         return None
     if any(len(compressors.get(q, ())) < W or any(c.nbits != q for c in compressors[q]) for q in (8, 4, 2)):
         return None

@@ -107,6 +107,72 @@ def test_loaded_random_pool_keeps_the_dtype_the_reference_keeps(eden_utils, orac
         assert (send.cpu().numpy() == want).all()
 
 
+def _own_rows(how, made):
+    """a compressor class, or object, that picks its rows of the pool itself"""
+    from dynamiq_sigcomm_artifact_amd.compressors import Aee_Dynamic_Range_GPU_kern as Base
+
+    class Rows(Base):
+        def rand_pool(self, n, dtype):
+            made.append(self.randomized_vec_pool.to(dtype)[3:3 + n // self.chunk_size])
+            return made[-1]
+
+    class Next(Base):
+        def gen_next_rand(self):
+            made.append(5)
+            return 5
+
+    def one(params, **kw):
+        c = Base(4, 16, params, **kw)
+        c.gen_next_rand = lambda: made.append(5) or 5
+        return c
+
+    return {"rows": lambda params, **kw: Rows(4, 16, params, **kw), "next": lambda params, **kw: Next(4, 16, params, **kw), "object": one}[how]
+
+
+@pytest.mark.parametrize("how", ["rows", "next", "object"])
+def test_own_choice_of_rows_is_asked_for(how):
+    """a subclass (or an object) with a rand_pool or gen_next_rand of its own is called for every encoding call, and the module gets
+    the rows that it picked; an all-reduce with such compressors goes call by call"""
+    from dynamiq_sigcomm_artifact_amd.dynamiq_pipeline import _pooled_codecs
+    made, given = [], []
+    c = _own_rows(how, made)(_params(256 * 40, 1), device="cpu")
+
+    def note(*args):
+        given.append(args)
+
+    c.eden_utils = types.SimpleNamespace(scaling_compress=note, scaling_dec_comp=note)
+    c._stream = lambda: 0
+    x, y = torch.ones(512, dtype=torch.bfloat16), torch.zeros(292, dtype=torch.uint8)
+    c.compression(x, y)
+    c.dec_compression(y, x, y)
+    c.compression(x[:0], y)
+    first = 3 if how == "rows" else 5
+    want = c.randomized_vec_pool.to(torch.bfloat16)[first:first + 32]
+    assert len(given) == 2 and len(made) == 2
+    assert all(torch.equal(rows, want) for rows in (given[0][2], given[1][3]))
+    assert [g[-5:] for g in given] == [(512, 4, 16, 0, 2)] * 2
+    vec = types.SimpleNamespace(dtype=torch.bfloat16)
+    assert _pooled_codecs([vec], {q: [c] for q in (8, 4, 2)}) is None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("how", ["rows", "next", "object"])
+def test_own_choice_of_rows_on_the_gpu(capi, how):
+    made = []
+    c = _own_rows(how, made)(_params(256 * 40, 1), device=DEV)
+    x = (torch.randn(256 * 6, device=DEV) * 1e-3).to(torch.bfloat16)
+    send, want = c.create_tensor(x, torch.uint8), c.create_tensor(x, torch.uint8)
+    c.compression(x, send)
+    first = 3 if how == "rows" else 5
+    pool = c.randomized_vec_pool.to(torch.bfloat16)[first:first + 96].reshape(-1).contiguous()
+    capi.scaling_compress(x, want, pool, x.numel(), 4, 16, 2)
+    assert torch.equal(send, want) and len(made) == 1
+    again = torch.zeros_like(send)
+    c.dec_compression(send, x, again)
+    capi.scaling_dec_comp(want, x, send, pool, x.numel(), 4, 16, 2)
+    assert torch.equal(again, send) and len(made) == 2
+
+
 def _oracle_ring(oracle, vecs_bits, pools, nbits, strategy, W):
     """the same schedule on the CPU with oracle calls (ring_rdma.py:590-631)"""
     n = vecs_bits[0].size
