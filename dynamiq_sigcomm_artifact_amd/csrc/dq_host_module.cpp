@@ -479,20 +479,26 @@ struct Codec {
         }
         return THPVariable_Unpack(have);
     }
-    // first of n / chunk consecutive rows, where the LCG points (utils_aggregation.py:409-420)
-    int64_t first_row(const at::Tensor &p, int64_t n)
+    // first of n / chunk consecutive rows, where the LCG points (utils_aggregation.py:409-420).  The pool is an attribute that
+    // a caller may replace: what the kernels read is checked on every call.
+    int64_t first_row(const at::Tensor &p, int64_t n, at::ScalarType dtype)
     {
+        need(p.scalar_type() == dtype, "rand_pool dtype must match input dtype");
+        need(p.dim() >= 2, "rand_pool must have rows");
+        need(n % chunk || n / chunk * row_width(p) >= n, "rand_pool is too small"); // (a ragged n is refused further on)
         const int64_t choices = p.size(0) - n / chunk - 1;
         need(choices > 0, "randomized_vec_pool is too small for scaling quantization");
         return (int64_t)next_rand() % choices;
     }
+    static int64_t row_width(const at::Tensor &p) { return p.size(0) ? p.numel() / p.size(0) : 0; }
     const void *random_rows(const at::Tensor &like, int64_t n)
     {
         const at::Tensor &p = pool(like.scalar_type());
         need(p.is_cuda(), "rand_pool must be a CUDA tensor");
         need(p.is_contiguous(), "rand_pool must be contiguous");
         need(p.device() == like.device(), "tensor arguments live on different devices");
-        return static_cast<const char *>(p.data_ptr()) + first_row(p, n) * chunk * (int64_t)like.element_size();
+        const int64_t first = first_row(p, n, like.scalar_type());
+        return static_cast<const char *>(p.data_ptr()) + first * row_width(p) * (int64_t)p.element_size();
     }
     void check_common(int64_t n) const
     {
@@ -629,7 +635,8 @@ void ranks_pooled(py::sequence vecs, py::sequence outs, int64_t n, py::handle to
                 const int chunk = (r - step + world) % world;
                 const int64_t rows = std::max<int64_t>(0, std::min(per, size[g] - per * chunk));
                 if (rows == 0) continue;
-                const int64_t at = c.first_row(p, rows * 256);
+                need(p.dim() == 2 && p.size(1) == 16, "rand_pool must have rows of 16 values");
+                const int64_t at = c.first_row(p, rows * 256, dtype);
                 need(at <= 0x7fffffff, "randomized_vec_pool has too many rows");
                 first[(g * world + r) * world + step] = (int32_t)at;
             }

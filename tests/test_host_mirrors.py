@@ -173,6 +173,37 @@ def test_own_choice_of_rows_on_the_gpu(capi, how):
     assert torch.equal(again, send) and len(made) == 2
 
 
+@pytest.mark.gpu
+def test_replaced_pool_is_checked(capi):
+    """a pool that a caller has put in the place of the object's: refused where a call would read beyond its rows or take them for
+    another type; rows that are wider than a chunk are read from their starts, as slices of such a pool are"""
+    from dynamiq_sigcomm_artifact_amd.compressors import Aee_Dynamic_Range_GPU_kern
+    from dynamiq_sigcomm_artifact_amd.dynamiq_pipeline import fixed_proportion_allreduce_grouped
+    c = Aee_Dynamic_Range_GPU_kern(4, 16, _params(256 * 40, 1), device=DEV)
+    x = (torch.randn(256 * 6, device=DEV) * 1e-3).to(torch.bfloat16)
+    send, want = c.create_tensor(x, torch.uint8), c.create_tensor(x, torch.uint8)
+    good = c.randomized_vec_pool
+    thresholds = {8: 0.2, 4: 0.5, 2: 0.3}
+    shared = {q: [Aee_Dynamic_Range_GPU_kern(q, 16, _params(256 * 40, 1), device=DEV)] for q in (8, 4, 2)}
+    for bad, text in ((good.to(torch.float16), "dtype"), (good[:, :8].contiguous(), "too small|16 values"), (good.reshape(-1), "rows"),
+                      (good.cpu(), "CUDA|contiguous tensor"), (good[:, ::2], "contiguous")):
+        for owner in (c, shared[4][0]):
+            owner.randomized_vec_pools[torch.bfloat16] = bad
+        with pytest.raises(RuntimeError, match=text):
+            c.compression(x, send)
+        with pytest.raises(RuntimeError, match=text):
+            c.dec_compression(send, x, want)
+        with pytest.raises(RuntimeError, match=text):
+            fixed_proportion_allreduce_grouped([x], thresholds, shared)
+    wide = torch.rand((500, 48), device=DEV).to(torch.bfloat16)
+    c.randomized_vec_pools[torch.bfloat16] = wide
+    seed = (c.rand_seed * 671431 + 1000000007) & 0xFFFFFFFF
+    c.compression(x, send)
+    first = seed % (500 - 96 - 1)
+    capi.scaling_compress(x, want, wide[first:first + 96].reshape(-1), x.numel(), 4, 16, 2)
+    assert torch.equal(send, want)
+
+
 def _oracle_ring(oracle, vecs_bits, pools, nbits, strategy, W):
     """the same schedule on the CPU with oracle calls (ring_rdma.py:590-631)"""
     n = vecs_bits[0].size
