@@ -33,6 +33,7 @@ def record_geometry(nbits, chunk_size, supergroup=_SUPERGROUP):
 
 
 _ROW_CHOICE = ("rand_pool", "gen_next_rand")
+_CODEC_STATE = {"nbits": "nbits", "chunk_size": "chunk", "strategy": "strategy"}      # attribute -> the native object's
 
 
 class _DynamicRangeGPUKern(object):
@@ -56,11 +57,11 @@ class _DynamicRangeGPUKern(object):
         self._codec = capi.host().Codec(nbits, chunk_size, self.strategy, self._extended, (nbits * 998244353) & _U32, None, {})
         # a class that picks its rows itself is asked for them call by call
         self._picks_rows = any(getattr(type(self), name) is not getattr(_DynamicRangeGPUKern, name) for name in _ROW_CHOICE)
-        self.philox_seed = params.get("philox_seed")
-        if self.philox_seed is not None:
+        seed = params.get("philox_seed")
+        if seed is not None:
             # one stream per rank, one step per call
-            self.philox_seed = (int(self.philox_seed) + self.client_rank * 0x9E3779B97F4A7C15) & 0xFFFFFFFFFFFFFFFF
-            self._codec.philox, self._codec.philox_seed, self._codec.philox_step = True, self.philox_seed, nbits << 32
+            self.philox_seed = int(seed) + self.client_rank * 0x9E3779B97F4A7C15
+            self.philox_step = nbits << 32
             return
         rows = self.three_times_cur_max_size
         given = params.get("rand_pool_tensor")          # the reference's "correlated" mode loads its pool from disk
@@ -79,6 +80,8 @@ class _DynamicRangeGPUKern(object):
         object.__setattr__(self, name, value)
         if name in _ROW_CHOICE:                         # an object of its own ways, likewise
             object.__setattr__(self, "_picks_rows", True)
+        elif name in _CODEC_STATE and "_codec" in self.__dict__:
+            setattr(self._codec, _CODEC_STATE[name], value)
 
     # ---- state the reference's callers may read (and that the native object works with) ----------------------
     @property
@@ -88,6 +91,17 @@ class _DynamicRangeGPUKern(object):
     @rand_seed.setter
     def rand_seed(self, seed):
         self._codec.rand_seed = seed & _U32
+
+    @property
+    def philox_seed(self):
+        """None: rounding randomness from the pool"""
+        return self._codec.philox_seed if self._codec.philox else None
+
+    @philox_seed.setter
+    def philox_seed(self, seed):
+        self._codec.philox = seed is not None
+        if seed is not None:
+            self._codec.philox_seed = int(seed) & 0xFFFFFFFFFFFFFFFF
 
     @property
     def philox_step(self):
@@ -109,6 +123,10 @@ class _DynamicRangeGPUKern(object):
     def randomized_vec_pools(self):
         """dtype -> the pool in that dtype (converted when a call first needs it)"""
         return self._codec.pools
+
+    @randomized_vec_pools.setter
+    def randomized_vec_pools(self, pools):
+        self._codec.pools = pools
 
     # ---- sizes --------------------------------------------------------------------------------------------
     def padded_n(self, n):

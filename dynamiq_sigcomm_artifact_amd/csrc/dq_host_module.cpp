@@ -483,6 +483,7 @@ struct Codec {
     // a caller may replace: what the kernels read is checked on every call.
     int64_t first_row(const at::Tensor &p, int64_t n, at::ScalarType dtype)
     {
+        need(chunk > 0, "chunk_size must be positive");
         need(p.scalar_type() == dtype, "rand_pool dtype must match input dtype");
         need(p.dim() >= 2, "rand_pool must have rows");
         need(n % chunk || n / chunk * row_width(p) >= n, "rand_pool is too small"); // (a ragged n is refused further on)
@@ -970,6 +971,9 @@ PYBIND11_MODULE(_host, m)
     PyModule_AddFunctions(m.ptr(), kFunctions);
     py::class_<Codec>(m, "Codec")
         .def(py::init<int, int, int, bool, uint32_t, py::object, py::dict>())
+        .def_readwrite("nbits", &Codec::nbits)
+        .def_readwrite("chunk", &Codec::chunk)
+        .def_readwrite("strategy", &Codec::strategy)
         .def_readwrite("rand_seed", &Codec::rand_seed)
         .def_readwrite("philox", &Codec::philox)
         .def_readwrite("philox_seed", &Codec::philox_seed)

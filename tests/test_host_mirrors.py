@@ -204,6 +204,50 @@ def test_replaced_pool_is_checked(capi):
     assert torch.equal(send, want)
 
 
+@pytest.mark.gpu
+def test_attributes_of_a_compressor_apply_to_the_next_call(capi):
+    """width, chunk size, strategy, seed of the rounding stream and the pools, set after construction, are what the next call uses;
+    without a seed the pool is"""
+    from dynamiq_sigcomm_artifact_amd.compressors import Aee_Dynamic_Range_GPU_kern
+    n = 256 * 6
+    c = Aee_Dynamic_Range_GPU_kern(4, 16, _params(256 * 40, 1), device=DEV)
+    x = (torch.randn(n, device=DEV) * 1e-3).to(torch.bfloat16)
+    send = torch.zeros(capi.required_bytes(n, 8, 8, 3), dtype=torch.uint8, device=DEV)
+    want = torch.zeros_like(send)
+    c.nbits, c.strategy, c.philox_seed, c.philox_step = 8, 3, 77, 10
+    c.compression(x, send)
+    capi.scaling_compress_philox(x, want, n, 8, 16, 3, 77, 11)
+    assert torch.equal(send, want) and c.philox_step == 11
+    c.chunk_size, c.philox_seed, c.randomized_vec_pools = 8, None, {}
+    c.randomized_vec_pool = torch.rand((600, 8), device=DEV).to(torch.bfloat16)
+    first = ((c.rand_seed * 671431 + 1000000007) & 0xFFFFFFFF) % (600 - n // 8 - 1)
+    c.compression(x, send)
+    pool = c.randomized_vec_pool[first:first + n // 8].reshape(-1)
+    capi.scaling_compress(x, want, pool, n, 8, 8, 3)
+    assert torch.equal(send, want) and c.philox_seed is None
+    out, back = torch.zeros_like(x), torch.zeros_like(x)
+    c.decompression(send, out)
+    capi.scaling_decompress(want, back, n, 8, 8, 3)
+    assert torch.equal(out, back)
+    c.chunk_size = 0
+    with pytest.raises(RuntimeError, match="positive"):
+        c.compression(x, send)
+
+
+def test_attributes_of_a_compressor_on_the_cpu():
+    from dynamiq_sigcomm_artifact_amd.compressors import Mee_Dynamic_Range_GPU_kern
+    c = Mee_Dynamic_Range_GPU_kern(5, 16, dict(_params(256 * 40, 2), philox_seed=3, rank=1), device="cpu")
+    assert c.philox_seed == 3 + 0x9E3779B97F4A7C15 and c.philox_step == 5 << 32 and c.randomized_vec_pool is None
+    c.philox_seed = None
+    assert c.philox_seed is None and not c._codec.philox
+    c.philox_seed = -1
+    assert c.philox_seed == 2 ** 64 - 1 and c._codec.philox
+    c.strategy, c.nbits, c.chunk_size = 2, 4, 32
+    assert (c._codec.strategy, c._codec.nbits, c._codec.chunk) == (2, 4, 32)
+    c.randomized_vec_pools = pools = {}
+    assert c.randomized_vec_pools is pools
+
+
 def _oracle_ring(oracle, vecs_bits, pools, nbits, strategy, W):
     """the same schedule on the CPU with oracle calls (ring_rdma.py:590-631)"""
     n = vecs_bits[0].size
