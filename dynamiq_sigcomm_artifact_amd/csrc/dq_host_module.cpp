@@ -513,6 +513,7 @@ struct Codec {
         const at::ScalarType d = t.scalar_type();
         return d == at::kBFloat16 || d == at::kHalf || (d == at::kFloat && (extended || philox));
     }
+    static bool empty(py::handle h) { return THPVariable_Check(h.ptr()) && THPVariable_Unpack(h.ptr()).numel() == 0; }
     static const at::Tensor &cuda(py::handle h, const char *text)
     {
         if (!THPVariable_Check(h.ptr())) refuse(std::string("a tensor argument is required, got ") + Py_TYPE(h.ptr())->tp_name);
@@ -524,9 +525,9 @@ struct Codec {
 
     void compress(py::handle input, py::handle send)
     {
+        if (empty(input)) return; // nothing to do, wherever it lives
         const at::Tensor &src = cuda(input, "input must be a CUDA tensor");
         const int64_t n = src.numel();
-        if (n == 0) return;
         const at::Tensor &dst = cuda(send, "output must be a CUDA tensor");
         need(data_dtype(src), "input must be torch.float16 or torch.bfloat16");
         const void *rnd = philox ? nullptr : random_rows(src, n);
@@ -551,9 +552,9 @@ struct Codec {
     }
     void decompress(py::handle recv, py::handle output, bool add)
     {
+        if (empty(output)) return;
         const at::Tensor &dst = cuda(output, "output must be a CUDA tensor");
         const int64_t n = dst.numel();
-        if (n == 0) return;
         const at::Tensor &src = cuda(recv, "input must be a CUDA tensor");
         need(src.scalar_type() == at::kByte, "input must be torch.uint8");
         need(data_dtype(dst), "output must be torch.float16 or torch.bfloat16");
@@ -575,9 +576,9 @@ struct Codec {
     }
     void dec_comp(py::handle recv_, py::handle input, py::handle send_)
     {
+        if (empty(input)) return;
         const at::Tensor &inp = cuda(input, "inp must be a CUDA tensor");
         const int64_t n = inp.numel();
-        if (n == 0) return;
         const at::Tensor &recv = cuda(recv_, "recv must be a CUDA tensor"), &send = cuda(send_, "send must be a CUDA tensor");
         need(recv.scalar_type() == at::kByte, "recv must be torch.uint8");
         need(data_dtype(inp), "inp must be torch.float16 or torch.bfloat16");

@@ -248,6 +248,21 @@ def test_attributes_of_a_compressor_on_the_cpu():
     assert c.randomized_vec_pools is pools
 
 
+def test_empty_vectors_are_nothing_to_do():
+    """an empty chunk of a ring returns before anything is checked or drawn, wherever it lives"""
+    from dynamiq_sigcomm_artifact_amd.compressors import Aee_Dynamic_Range_GPU_kern
+    c = Aee_Dynamic_Range_GPU_kern(4, 16, _params(256 * 40, 1), device="cpu")
+    seed = c.rand_seed
+    none, stream = torch.zeros(0, dtype=torch.bfloat16), torch.zeros(0, dtype=torch.uint8)
+    c.compression(none, stream)
+    c.dec_compression(stream, none, stream)
+    c.decompression(stream, none)
+    c.decompression_add(stream, none)
+    assert c.rand_seed == seed
+    with pytest.raises(RuntimeError, match="CUDA"):
+        c.compression(torch.zeros(256, dtype=torch.bfloat16), stream)
+
+
 def _oracle_ring(oracle, vecs_bits, pools, nbits, strategy, W):
     """the same schedule on the CPU with oracle calls (ring_rdma.py:590-631)"""
     n = vecs_bits[0].size
