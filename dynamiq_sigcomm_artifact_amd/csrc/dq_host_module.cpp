@@ -214,6 +214,18 @@ struct Buckets {
         const bool now = capturing(s, &id);
         if (now ? recording == id && s != last_recorded : used && s != last) follow(s);
     }
+    // would join() have to wait?
+    bool behind() const { return used && c10::hip::getCurrentHIPStream(device).stream() != last; }
+    // the counter in device memory takes the steps that wait for a launch
+    void settle()
+    {
+        if (pending == 0) return;
+        if (!follow(c10::hip::getCurrentHIPStream(device).stream())) { // (a recording has put them into `base`)
+            at::Tensor counter = THPVariable_Unpack(step_dev.ptr());
+            counter.add_((int64_t)pending);
+            pending = 0;
+        }
+    }
     void begin_step()
     {
         const hipStream_t s = c10::hip::getCurrentHIPStream(device).stream();
@@ -995,6 +1007,8 @@ PYBIND11_MODULE(_host, m)
         .def_readonly("recorded", &Buckets::recorded)
         .def("scratch", &Buckets::scratch)
         .def("join", &Buckets::join)
+        .def("behind", &Buckets::behind)
+        .def("settle", &Buckets::settle)
         .def("begin_step", &Buckets::begin_step);
     py::class_<Batch>(m, "Batch")
         .def(py::init([](Buckets &b, py::sequence pairs, py::sequence steps, py::sequence rows) {

@@ -444,14 +444,14 @@ class SinglePassBuckets(object):
         self.device = torch.device(device)
         self.strategy, self.seed, self.graphs, self.inline_first = strategy, int(seed), graphs, bool(inline_first)
         self.slots = max(1, int(streams))
-        self.step_dev = torch.zeros(1, dtype=torch.int64, device=self.device)
+        self._step = torch.zeros(1, dtype=torch.int64, device=self.device)
         self.u_dev = u if isinstance(u, torch.Tensor) else torch.full((1,), 60.0 if u is None else float(u), dtype=torch.float64,
                                                                      device=self.device)
         self.hist = norm_histogram
         self._host = capi.host()
         self._turn = threading.RLock()
         self._counts = torch.zeros((self.slots, 4), dtype=torch.int32, device=self.device)
-        self._buckets = self._host.Buckets(strategy, self.seed & _U64, self.step_dev, self.u_dev,
+        self._buckets = self._host.Buckets(strategy, self.seed & _U64, self._step, self.u_dev,
                                            None if norm_histogram is None else norm_histogram.hist, self._counts)
         self._room = (0, 0)      # superchunks and buckets that the scratch holds
         self._scratch = None     # statistics; counts of the buckets that are not the last of their slot
@@ -474,6 +474,32 @@ class SinglePassBuckets(object):
     def side_by_side(self):
         self._pick()
         return self._side_by_side
+
+    # ---- state ----------------------------------------------------------------------------------------------
+    @property
+    def step_dev(self):
+        """the step counter in device memory, int64 [1], with the steps begun so far"""
+        with self._turn:
+            self._buckets.settle()
+        return self._step
+
+    @property
+    def step_devs(self):
+        """the same per slot: all slots have one counter"""
+        return [self.step_dev] * self.slots
+
+    @property
+    def pending(self):
+        """per slot: is there work that the caller's current stream has not been ordered behind (what join() does)?"""
+        with self._turn:
+            return [self._buckets.behind()] * self.slots
+
+    @property
+    def scratch(self):
+        """per slot, once there has been a bucket: the superchunks that the statistics shared by all slots have room for, and the
+        counts of the slot's last bucket (means, row lists and a packed stream are not made)"""
+        with self._turn:
+            return [{"nsc": self._room[0], "work": self._counts[k]} if self._scratch else {} for k in range(self.slots)]
 
     # ---- once per training step ----------------------------------------------------------------------------
     def set_u(self, u):

@@ -1024,6 +1024,35 @@ def test_list_of_buckets_that_share_memory(capi, shape):
         assert pipe._last[0].runs == {"chain": [1, 1, 1], "rewrite": [1, 2], "reuse": [1, 1, 1], "overlap": [1, 2]}.get(shape, [3])
 
 
+@pytest.mark.parametrize("streams", [1, 3])
+def test_state_of_the_pipeline_object(capi, streams):
+    """step_devs, pending and scratch: the steps begun so far, what join() would wait for, room and counts per slot; a counter that
+    the caller sets is the one that the next bucket draws from"""
+    from dynamiq_sigcomm_artifact_amd.dynamiq_pipeline import SinglePassBuckets
+    x = _llama_like(256 * 20, 4)
+    out = torch.zeros_like(x)
+    pipe = SinglePassBuckets(DEV, strategy=2, seed=5, streams=streams, u=6.0)
+    assert pipe.scratch == [{}] * streams and pipe.pending == [False] * streams
+    pipe.begin_step()
+    pipe.begin_step()
+    assert [int(s) for s in pipe.step_devs] == [2] * streams
+    for s in pipe.step_devs:
+        s.fill_(40)
+    pipe.begin_step()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        k = pipe.run(x, out)
+        assert pipe.pending == [False] * streams
+    assert pipe.pending == [True] * streams
+    pipe.join()
+    assert pipe.pending == [False] * streams
+    torch.cuda.synchronize()
+    want = _four_calls(capi, x, x.numel(), 6.0, 2, 5, 41)
+    assert torch.equal(bits_t(out), bits_t(want[5])) and int(pipe.step_dev) == 41
+    assert pipe.scratch[k]["nsc"] == 20 and pipe.scratch[k]["work"][:4].tolist() == want[3][:4].tolist() == pipe.counts(k).tolist()
+
+
 def test_bucket_seen_before_is_checked_again(capi):
     """an output at a known address that has become too short is refused, not written beyond its end; scratch in use on two streams
     grows without disturbing either"""
