@@ -568,11 +568,12 @@ class SinglePassBuckets(object):
         with self._turn:
             last = self._last
             if last is None or not last[0].matches(pairs):
+                pairs = [(x, o) for x, o in pairs]      # whatever holds them
                 if not pairs:
                     return
                 key = tuple((x.data_ptr(), o.data_ptr(), x.numel(), x.dtype) for x, o in pairs)
                 last = self.cache.get(key)
-                if last is None or not last[0].matches(list(map(tuple, pairs))):
+                if last is None or not last[0].matches(pairs):
                     last = self._batch(pairs, key)
                 self._last = last
             self._enqueue(last)

@@ -1053,6 +1053,26 @@ def test_state_of_the_pipeline_object(capi, streams):
     assert pipe.scratch[k]["nsc"] == 20 and pipe.scratch[k]["work"][:4].tolist() == want[3][:4].tolist() == pipe.counts(k).tolist()
 
 
+@pytest.mark.parametrize("form", [list, tuple, lambda p: [list(q) for q in p], lambda p: dict(p).items(), lambda p: ([x, o] for x, o in p)],
+                         ids=["list", "tuple", "lists", "items", "generator"])
+def test_whatever_holds_the_buckets(capi, form):
+    """a step's buckets as a list of pairs, a tuple, a list of lists, a dictionary's items, a generator; and none at all"""
+    from dynamiq_sigcomm_artifact_amd.dynamiq_pipeline import SinglePassBuckets
+    xs = [_llama_like(256 * 5 - k, 90 + k) for k in range(3)]
+    pairs = [(x, torch.zeros_like(x)) for x in xs]
+    pipe = SinglePassBuckets(DEV, strategy=2, seed=5, u=6.0)
+    pipe.run_all(form([]))
+    for step in range(1, 4):
+        pipe.begin_step()
+        pipe.run_all(form(pairs))
+        pipe.run_all(form([]))
+        torch.cuda.synchronize()
+        for k, (x, o) in enumerate(pairs):
+            assert torch.equal(bits_t(o), bits_t(_four_calls(capi, x, x.numel(), 6.0, 2, 5, (k << 32) + step)[5])), (step, k)
+            o.zero_()
+    assert len(pipe.cache) == 1
+
+
 def test_bucket_seen_before_is_checked_again(capi):
     """an output at a known address that has become too short is refused, not written beyond its end; scratch in use on two streams
     grows without disturbing either"""
