@@ -106,6 +106,16 @@ uint32_t *hist_of(Args &a, py::handle h, int64_t *entries)
     return reinterpret_cast<uint32_t *>(t.data_ptr<int32_t>());
 }
 
+// memory that a tensor's first n elements take
+struct Span {
+    uintptr_t begin, end;
+    Span(const at::Tensor &t, int64_t n) : begin(reinterpret_cast<uintptr_t>(t.data_ptr())), end(begin + (uintptr_t)(n * t.element_size())) {}
+    bool meets(const Span &o) const { return begin < o.end && o.begin < end; }
+    // The kernels of one pass read a superchunk and write it where it was, or elsewhere: an output that lies across a source at
+    // another address would be written while other waves still read there.
+    bool across(const Span &o) const { return begin != o.begin && meets(o); }
+};
+
 // ---- buckets of one rank ----------------------------------------------------------------------------------
 
 // The state of a SinglePassBuckets object.  Its buckets share scratch and run on the caller's stream; a caller that comes
@@ -247,10 +257,6 @@ struct Batch {
     struct Run {
         int dtype, count;
     };
-    struct Span {
-        uintptr_t begin, end;
-        bool meets(const Span &o) const { return begin < o.end && o.begin < end; }
-    };
     // does bucket b write what a reads or writes, or read what a writes?
     static bool clash(const Span &a_src, const Span &a_out, const Span &b_src, const Span &b_out)
     {
@@ -298,10 +304,9 @@ struct Batch {
             at += (d.n + 255) / 256;
             desc.push_back(d);
             codes.push_back(code);
-            for (const void *p : {d.src, static_cast<const void *>(d.out)}) {
-                const uintptr_t begin = reinterpret_cast<uintptr_t>(p);
-                spans.emplace_back(Span{begin, begin + (uintptr_t)d.n * x.element_size()}, k);
-            }
+            spans.emplace_back(Span(x, d.n), k);
+            spans.emplace_back(Span(out, d.n), k);
+            if (spans[2 * k + 1].first.across(spans[2 * k].first)) refuse("an output lies across its bucket at another address");
         }
         const bool meet = any_meet(spans);
         for (size_t k = 0; k < count; k++) {
@@ -361,14 +366,15 @@ struct Batch {
     }
 };
 
-// one bucket of one rank outside a SinglePassBuckets object
-void roundtrip(py::handle x, py::handle out, int64_t n, py::handle stats, py::handle counts, py::handle u, py::handle hist,
+// one bucket of one rank outside a SinglePassBuckets object; false: the output lies across the vector, nothing done
+bool roundtrip(py::handle x, py::handle out, int64_t n, py::handle stats, py::handle counts, py::handle u, py::handle hist,
                uint64_t seed, int strategy, py::handle stream)
 {
     Args a;
     const at::Tensor &src = a.tensor(x);
     const at::Tensor &dst = a.tensor(out);
     if (src.numel() < n || dst.numel() < n || dst.scalar_type() != src.scalar_type()) refuse("the output must have the vector's dtype and size");
+    if (Span(dst, n).across(Span(src, n))) return false;
     dq_roundtrip_t d;
     d.src = src.data_ptr();
     d.out = dst.data_ptr();
@@ -387,6 +393,7 @@ void roundtrip(py::handle x, py::handle out, int64_t n, py::handle stats, py::ha
         rc = dq_bucket_roundtrip(&d, 1, code, strategy, 1, o.value, o.dev, seed, nullptr, 0, h, hist_ints, a.device, s);
     }
     check(rc);
+    return true;
 }
 
 // ---- ranks that share the GPU's memory ---------------------------------------------------------------------
@@ -394,6 +401,7 @@ void roundtrip(py::handle x, py::handle out, int64_t n, py::handle stats, py::ha
 struct Ranks {
     std::vector<const void *> src;
     std::vector<void *> out;
+    bool across = false; // an output lies across a vector at another address
     dq_ranks_t r;
 
     Ranks(Args &a, py::sequence vecs, py::sequence outs, int64_t n, py::handle total, py::handle mean, py::handle order,
@@ -403,6 +411,7 @@ struct Ranks {
         const size_t world = py::len(vecs);
         if (world == 0 || py::len(outs) != world) refuse("one vector and one output per rank");
         at::ScalarType dtype = at::kBFloat16;
+        std::vector<Span> reads, writes;
         for (size_t k = 0; k < world; k++) {
             const py::object x = vecs[k], o = outs[k];
             const at::Tensor &s = a.tensor(x), &d = a.tensor(o);
@@ -414,7 +423,11 @@ struct Ranks {
                 refuse("the ranks' vectors and outputs must have one dtype and size");
             src.push_back(s.data_ptr());
             out.push_back(d.data_ptr());
+            reads.emplace_back(s, n);
+            writes.emplace_back(d, n);
         }
+        for (const Span &w : writes)
+            for (const Span &x : reads) across = across || w.across(x);
         const int64_t nsc = (n + 255) / 256;
         r.src = src.data();
         r.out = out.data();
@@ -439,17 +452,20 @@ struct Ranks {
     }
 };
 
-void ranks_dynamic(py::sequence vecs, py::sequence outs, int64_t n, py::handle total, py::handle mean, py::handle order,
+// false: an output lies across a vector, nothing done
+bool ranks_dynamic(py::sequence vecs, py::sequence outs, int64_t n, py::handle total, py::handle mean, py::handle order,
                    py::handle work, py::handle u, py::handle hist, uint64_t seed, int strategy, py::handle stream)
 {
     Args a;
     Ranks k(a, vecs, outs, n, total, mean, order, work, strategy);
+    if (k.across) return false;
     const Offset o(a, u);
     k.r.u = o.value;
     k.r.u_dev = o.dev;
     k.r.hist = hist_of(a, hist, &k.r.hist_ints);
     k.r.seed = seed;
     k.enqueue(DQ_RANKS_STATS | DQ_RANKS_PLAN | DQ_RANKS_RING, a.device, stream_of(stream, a.device));
+    return true;
 }
 
 // ---- compressor objects ------------------------------------------------------------------------------------
@@ -623,12 +639,14 @@ struct Codec {
 
 // One bucket of the fixed-proportion (sorted_plan) or dynamic all-reduce with compressor objects: codecs holds one list per
 // width (8, 4, 2 bits), group sizes counts.  Walks every codec's LCG as the ring's calls on its non-empty chunks would, in
-// the order of the widths, the steps and the ranks: rank r works on chunk (r - step) mod world in that step.
-void ranks_pooled(py::sequence vecs, py::sequence outs, int64_t n, py::handle total, py::handle mean, py::handle order,
+// the order of the widths, the steps and the ranks: rank r works on chunk (r - step) mod world in that step.  False: an output
+// lies across a vector, nothing done.
+bool ranks_pooled(py::sequence vecs, py::sequence outs, int64_t n, py::handle total, py::handle mean, py::handle order,
                   py::handle work, py::sequence codecs, py::sequence counts, int stages, int strategy)
 {
     Args a;
     Ranks k(a, vecs, outs, n, total, mean, order, work, strategy);
+    if (k.across) return false;
     const int world = k.r.world;
     const at::ScalarType dtype = THPVariable_Unpack(py::object(vecs[0]).ptr()).scalar_type();
     std::vector<const void *> pool(3 * world, nullptr);
@@ -662,6 +680,7 @@ void ranks_pooled(py::sequence vecs, py::sequence outs, int64_t n, py::handle to
     k.r.top_count = size[0];
     k.r.bottom_count = size[2];
     k.enqueue(stages, a.device, c10::hip::getCurrentHIPStream().stream());
+    return true;
 }
 
 // ---- EDEN and THC (eden.py, thc.py) --------------------------------------------------------------------------

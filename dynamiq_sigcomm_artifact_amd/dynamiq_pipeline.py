@@ -70,6 +70,12 @@ def dynamic_bitrate_allreduce(rank_vecs, u, compressors, out=None):
 _RANKS_STATS, _RANKS_PLAN, _RANKS_RING = 1, 2, 4
 
 
+def _across(out, x):
+    """does `out` lie across the vector `x` at another address?  The passes that have no buffer between the two cannot do that."""
+    a, b, size = out.data_ptr(), x.data_ptr(), x.numel() * x.element_size()
+    return a != b and a < b + size and b < a + size
+
+
 def _pooled_codecs(rank_vecs, compressors):
     """the native objects of the compressors, one list per width (8, 4, 2 bits), when the whole all-reduce can run without
     packed streams (csrc/dq_single_pass.hip): the package's own pooled compressors of one strategy, bf16 vectors and no
@@ -106,6 +112,8 @@ def dynamic_bitrate_allreduce_grouped(rank_vecs, u, compressors, out=None, work=
     if work is None:
         work = {}
     codecs = _pooled_codecs(rank_vecs, compressors)
+    if codecs and out is not None and any(_across(o, v) for o in out for v in rank_vecs):
+        codecs = None
     key = (nsc, dt, W, codecs is None)
     if work.get("key") != key:
         work["key"] = key
@@ -220,10 +228,10 @@ def fixed_proportion_allreduce_grouped(rank_vecs, thresholds, compressors, out=N
         plan_ints = capi.group_plan_sorted_work_ints(nsc)
         ints = torch.empty(3 * nsc + W * nsc + plan_ints, dtype=torch.int32, device=dev)
         order = ints[:3 * nsc]
-        capi.host().ranks_pooled(rank_vecs, outs, n, total, ints[3 * nsc:3 * nsc + W * nsc].view(torch.float32), order,
-                                 ints[3 * nsc + W * nsc:], codecs, counts, _RANKS_STATS | _RANKS_PLAN | _RANKS_RING,
-                                 compressors[8][0].strategy)
-        return outs, total, order, counts
+        if capi.host().ranks_pooled(rank_vecs, outs, n, total, ints[3 * nsc:3 * nsc + W * nsc].view(torch.float32), order,
+                                    ints[3 * nsc + W * nsc:], codecs, counts, _RANKS_STATS | _RANKS_PLAN | _RANKS_RING,
+                                    compressors[8][0].strategy):
+            return outs, total, order, counts
     residuals = [torch.empty(nsc * SUPERCHUNK, dtype=dt, device=dev) for _ in range(W)]
     stats = [torch.empty((nsc, 2), dtype=torch.bfloat16, device=dev) for _ in range(W)]
     for r in range(W):
@@ -292,22 +300,23 @@ def dynamic_bitrate_allreduce_single_pass(rank_vecs, u, strategy=2, seed=0, out=
             work["mean"] = torch.empty(W * nsc, dtype=torch.float32, device=dev)
             work["order"] = torch.empty(3 * nsc, dtype=torch.int32, device=dev)
     outs = out if out is not None else [torch.empty(n, dtype=dt, device=dev) for _ in range(W)]
-    hist = None
-    if norm_histogram is not None:
-        hist = norm_histogram.hist
-        norm_histogram.count += nsc
+    hist = None if norm_histogram is None else norm_histogram.hist
     total = work["total"]
     if W == 1:
-        capi.host().roundtrip(rank_vecs[0], outs[0], n, total, work["counts"], u, hist, seed & _U64, strategy, stream)
+        done = capi.host().roundtrip(rank_vecs[0], outs[0], n, total, work["counts"], u, hist, seed & _U64, strategy, stream)
     else:
-        capi.host().ranks_dynamic(rank_vecs, outs, n, total, work["mean"], work["order"], work["plan"], u, hist, seed & _U64,
-                                  strategy, stream)
+        done = capi.host().ranks_dynamic(rank_vecs, outs, n, total, work["mean"], work["order"], work["plan"], u, hist, seed & _U64,
+                                         strategy, stream)
+    if not done:        # an output lies across a vector at another address
+        return _single_pass_in_steps(rank_vecs, u, strategy, seed, out, work, stream, norm_histogram)
+    if norm_histogram is not None:
+        norm_histogram.count += nsc
     return outs, total, work["counts"]
 
 
 def _single_pass_in_steps(rank_vecs, u, strategy, seed, out, work, stream, norm_histogram):
     """the same with one launch per rank and ring step and the packed streams in memory: for more simulated ranks than the
-    arguments of one launch hold"""
+    arguments of one launch hold, and for outputs that lie across the vectors"""
     from . import capi
     W = len(rank_vecs)
     n = rank_vecs[0].numel()
@@ -364,7 +373,7 @@ def _single_pass_in_steps(rank_vecs, u, strategy, seed, out, work, stream, norm_
             encode(r, (r - step + W) % W, step, None if step == 0 else recv[r])
         exchange(send, recv)
     for r in range(W):
-        encode(r, (r + 1) % W, W - 1, recv[r])
+        encode(r, (r + 1) % W, W - 1, recv[r] if W > 1 else None)
         decode(r, send[r], (r + 1) % W)
     bufs = [send, recv]
     for step in range(W - 1):
@@ -530,11 +539,12 @@ class SinglePassBuckets(object):
         self.cache.clear()       # what was laid out over the old buffers
         self._last = None
 
-    def _batch(self, pairs, key):
-        """lays out a list of buckets seen for the first time (or again after the scratch grew)"""
+    def _batch(self, pairs, key, given=None):
+        """lays out a list of buckets seen for the first time (or again after the scratch grew); given: what the caller has,
+        where the sources are copies of it for one launch"""
         total = sum((x.numel() + SUPERCHUNK - 1) // SUPERCHUNK for x, _ in pairs)
         # a source keeps its ordinal, and with it its random stream and its slot, from step to step
-        ordinals = [self.ordinals.setdefault((x.data_ptr(), x.numel()), len(self.ordinals)) for x, _ in pairs]
+        ordinals = [self.ordinals.setdefault((x.data_ptr(), x.numel()), len(self.ordinals)) for x, _ in given or pairs]
         slots = [o % self.slots for o in ordinals]
         # the counts of a slot are those of its last bucket
         last = {slot: k for k, slot in enumerate(slots)}
@@ -543,7 +553,9 @@ class SinglePassBuckets(object):
         if total > self._room[0] or spare > self._room[1]:
             self._grow(total, max(0, spare))
         batch = self._host.Batch(self._buckets, pairs, [(o << 32) & _U64 for o in ordinals], rows)
-        entry = self.cache[key] = (batch, total, slots[0])
+        entry = (batch, total, slots[0])
+        if given is None:
+            self.cache[key] = entry
         return entry
 
     def _enqueue(self, entry):
@@ -559,7 +571,12 @@ class SinglePassBuckets(object):
         with self._turn:
             entry = self.cache.get(key)
             if entry is None or not entry[0].matches([(x, out)]):
-                entry = self._batch([(x, out)], key)
+                if _across(out, x):
+                    self.join()
+                    copy = x.clone()
+                    entry = self._batch([(copy, out)], key, [(x, out)])
+                else:
+                    entry = self._batch([(x, out)], key)
             self._enqueue(entry)
         return entry[2]
 
@@ -570,6 +587,10 @@ class SinglePassBuckets(object):
             if last is None or not last[0].matches(pairs):
                 pairs = [(x, o) for x, o in pairs]      # whatever holds them
                 if not pairs:
+                    return
+                if any(_across(o, x) for x, o in pairs):
+                    for x, o in pairs:
+                        self.run(x, o)
                     return
                 key = tuple((x.data_ptr(), o.data_ptr(), x.numel(), x.dtype) for x, o in pairs)
                 last = self.cache.get(key)

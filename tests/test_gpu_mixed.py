@@ -1073,6 +1073,45 @@ def test_whatever_holds_the_buckets(capi, form):
     assert len(pipe.cache) == 1
 
 
+@pytest.mark.parametrize("shift", [-256, 1, 8 * 256])
+@pytest.mark.parametrize("path", ["buckets", "lists", "all-reduce", "grouped", "fixed"])
+def test_outputs_across_their_sources(capi, path, shift):
+    """an output that lies across its source at another address, as every call took it when there were buffers between the two:
+    the results are those with an output elsewhere"""
+    from dynamiq_sigcomm_artifact_amd import dynamiq_pipeline as P
+    from dynamiq_sigcomm_artifact_amd.compressors import Aee_Dynamic_Range_GPU_kern
+    n, u = 256 * 600 - 5, 6.0
+    for W in (1, 3):
+        codecs = lambda: {q: [Aee_Dynamic_Range_GPU_kern(q, 16, {"d": {0: 256 * 1200}, "world_size": 1}, device=DEV,
+                                                         generator=torch.Generator(device=DEV).manual_seed(q + r)) for r in range(W)]
+                          for q in (8, 4, 2)}
+        calls = {"all-reduce": lambda v, o, c: P.dynamic_bitrate_allreduce_single_pass(v, u, seed=4, out=o)[0],
+                 "grouped": lambda v, o, c: P.dynamic_bitrate_allreduce_grouped(v, u, c, out=o)[0],
+                 "fixed": lambda v, o, c: P.fixed_proportion_allreduce_grouped(v, {8: 0.2, 4: 0.5, 2: 0.3}, c, out=o)[0]}
+        data = [_llama_like(n, 50 + r) for r in range(W)]
+        rooms = [torch.zeros(n + 8 * 256 + 512, dtype=torch.bfloat16, device=DEV) for _ in range(W)]
+        vecs = [room[256:256 + n] for room in rooms]
+        outs = [room[256 + shift:256 + shift + n] for room in rooms]
+        pipe = P.SinglePassBuckets(DEV, strategy=2, seed=5, u=u)
+        for step in range(1, 3):
+            for v, d in zip(vecs, data):
+                v.copy_(d)
+            if path in calls:
+                want = calls[path](data, [torch.zeros_like(d) for d in data], codecs())
+                got = calls[path](vecs, outs, codecs())
+            else:
+                pipe.begin_step()
+                if path == "lists":
+                    pipe.run_all(list(zip(vecs, outs)))
+                else:
+                    for v, o in zip(vecs, outs):
+                        pipe.run(v, o)
+                got = outs
+                want = [_four_calls(capi, d, n, u, 2, 5, (r << 32) + step)[5] for r, d in enumerate(data)]
+            torch.cuda.synchronize()
+            assert all(torch.equal(bits_t(x), bits_t(y)) for x, y in zip(got, want)), (W, step)
+
+
 def test_bucket_seen_before_is_checked_again(capi):
     """an output at a known address that has become too short is refused, not written beyond its end; scratch in use on two streams
     grows without disturbing either"""
