@@ -358,8 +358,8 @@ def llama_buckets(dev, count, n=6553600):
 
 def config4_entries(capi, O, dev, reps):
     """the single-pass dynamic-bitrate path per 25 MB bucket through the package's pipeline object: statistics, widths,
-    partition, encode (centring on load), decode (mean add) -- eager with one host call per bucket, and recorded with one,
-    two and three buckets in flight"""
+    encode, decode and mean add in one pass, then the tally -- one host call per bucket, one per step, and the step's call
+    recorded into a graph here and replayed"""
     from dynamiq_sigcomm_artifact_amd import bitrate
     from dynamiq_sigcomm_artifact_amd.dynamiq_pipeline import SinglePassBuckets
     out = []
@@ -374,19 +374,31 @@ def config4_entries(capi, O, dev, reps):
         norms.append(stats[:, 1].clone())
     u, avg, _ = bitrate.dynamic_bitrate_binary_search_u(norms, 4.375)
     pairs = list(zip(xs, outs))
-    for streams, graphs, whole in ((1, False, False), (2, False, False), (1, True, True), (2, True, True), (3, True, True)):
-        pipe = SinglePassBuckets(dev, strategy=2, seed=3, streams=streams, graphs=graphs, u=u)
+    ways = (("run", "one host call per bucket"), ("run_all", "one host call per step"),
+            ("graph", "a step's call recorded once and replayed, begin_step with it"))
+    for way, label in ways:
+        pipe = SinglePassBuckets(dev, strategy=2, seed=3, u=u)
 
-        def step():
+        def enqueue():
             pipe.begin_step()
-            if whole:
-                pipe.run_all(pairs)
-            else:
+            if way == "run":
                 for x, o in pairs:
                     pipe.run(x, o)
+            else:
+                pipe.run_all(pairs)
             pipe.join()
 
-        for _ in range(3):          # the first use of a bucket runs eagerly, the second records
+        step, steps = enqueue, 3 + 8 * reps
+        if way == "graph":
+            steps += 1
+            enqueue()
+            torch.cuda.synchronize()
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph):
+                enqueue()
+            step = graph.replay
+
+        for _ in range(3):
             step()
         torch.cuda.synchronize()
         # `rounds` training steps back to back between two events, the host free to run ahead of the device as it is in a
@@ -403,26 +415,25 @@ def config4_entries(capi, O, dev, reps):
         per = statistics.median(ts)
         entry = {
             "workload": "config 4: single-pass dynamic-bitrate path (u = %.2f, %.2f code bits) per 25 MB bf16 bucket of a "
-                        "Llama-3-8B shaped set, steps of %d distinct buckets back to back, %s, %d bucket(s) in flight; host calls included"
-                        % (u, avg, nb, "one recorded graph per stream and step" if graphs else "eager, one host call per bucket, the first bucket of every round on the caller's own stream", streams),
+                        "Llama-3-8B shaped set, steps of %d distinct buckets back to back, %s; host calls included"
+                        % (u, avg, nb, label),
             "us_per_bucket": round(per * 1e3, 2), "GBps_bf16_in": round(2.0 * n / (per * 1e-3) / 1e9, 1),
         }
-        if not graphs and streams == 1:
-            # the output of the first bucket against the oracle chain on a sample of its superchunks
-            x = xs[0]
-            res, st = O.superchunk_mean_center(host_bits(x), n, 1, O.BF16)
-            qb = O.dynamic_bitrate_qbits(st[1::2].copy(), u)
-            rows = np.nonzero(qb == 4)[0][:512]
-            ok = None
-            if rows.size:
-                uni = (O.philox_uniform_rows(rows, 3, 3 + 8 * reps).view(np.uint32) >> 16).astype(np.uint16)
-                enc = O.scaling_compress(res.reshape(-1, 256)[rows].reshape(-1).copy(), uni, rows.size * 256, 4, 16, 2, O.BF16)
-                dec = np.zeros(rows.size * 256, np.uint16)
-                O.scaling_decompress(enc, dec, dec.size, 4, 16, 2, O.BF16)
-                want = O.superchunk_add_mean_copy(dec, st.reshape(-1, 2)[rows].reshape(-1).copy(), dec.size, O.BF16)
-                got = host_bits(outs[0].view(-1, 256)[torch.from_numpy(rows).to(dev)]).reshape(-1)
-                ok = bool((got == want).all())
-            entry["bit_exact_vs_oracle"] = ok
+        # the output of the first bucket against the oracle chain on a sample of its superchunks
+        x = xs[0]
+        res, st = O.superchunk_mean_center(host_bits(x), n, 1, O.BF16)
+        qb = O.dynamic_bitrate_qbits(st[1::2].copy(), u)
+        rows = np.nonzero(qb == 4)[0][:512]
+        ok = None
+        if rows.size:
+            uni = (O.philox_uniform_rows(rows, 3, steps).view(np.uint32) >> 16).astype(np.uint16)
+            enc = O.scaling_compress(res.reshape(-1, 256)[rows].reshape(-1).copy(), uni, rows.size * 256, 4, 16, 2, O.BF16)
+            dec = np.zeros(rows.size * 256, np.uint16)
+            O.scaling_decompress(enc, dec, dec.size, 4, 16, 2, O.BF16)
+            want = O.superchunk_add_mean_copy(dec, st.reshape(-1, 2)[rows].reshape(-1).copy(), dec.size, O.BF16)
+            got = host_bits(outs[0].view(-1, 256)[torch.from_numpy(rows).to(dev)]).reshape(-1)
+            ok = bool((got == want).all())
+        entry["bit_exact_vs_oracle"] = ok
         out.append(entry)
         del pipe
     return out

@@ -473,8 +473,7 @@ def config4(dev, limit=None):
 def config4_streams(dev, u, nbuckets=48, rounds=8):
     """Back-to-back buckets with no host work between them.  The launches of `nbuckets` buckets are captured into one
     graph per stream (each stream takes every k-th bucket; every capture is an ordinary single-stream one) and the
-    graphs are replayed side by side: with several streams the small launches of a bucket -- statistics, plan -- overlap
-    the codec launches of its neighbours."""
+    graphs are replayed side by side: with several streams the tally of a bucket overlaps the pass over its neighbour."""
     xs = [b.to(torch.bfloat16).clone() for b in _llama_buckets(dev, limit=nbuckets)]
     keep = []                                   # graphs and streams stay alive until the function returns
     target = 5.0 - bitrate.DYNAMIC_BITRATE_HEADROOM

@@ -534,35 +534,49 @@ def test_bucket_call_equals_the_four_calls(capi, eden_utils, dt, strategy):
     torch.cuda.synchronize()
 
 
-@pytest.mark.parametrize("streams,graphs,whole", [(1, False, False), (2, False, False), (2, True, True), (3, True, True),
-                                                  (2, False, True)])
-def test_single_pass_buckets_object(capi, streams, graphs, whole):
-    """a stream of buckets through the pipeline object -- one host call per bucket, or a whole step recorded once and
-    replayed (one graph per stream), several buckets in flight on streams of their own -- gives, on every training step,
-    the outputs of the four calls with the rounding stream (seed, bucket ordinal * 2^32 + step)"""
+@pytest.mark.parametrize("streams,recorded,whole", [(1, False, False), (2, False, False), (2, True, True), (3, True, False),
+                                                    (2, False, True)])
+def test_single_pass_buckets_object(capi, streams, recorded, whole):
+    """a stream of buckets through the pipeline object -- one host call per bucket or per step, enqueued anew or recorded on the
+    second step and replayed -- gives, on every training step, the outputs of the four calls with the rounding stream (seed,
+    bucket ordinal * 2^32 + step)"""
     from dynamiq_sigcomm_artifact_amd.dynamiq_pipeline import SinglePassBuckets
-    sizes = [256 * 123, 256 * 300, 256 * 300 - 5, 256 * 300, 256 * 77 + 1]      # (a later, larger bucket makes a stream's scratch grow)
+    sizes = [256 * 123, 256 * 300, 256 * 300 - 5, 256 * 300, 256 * 77 + 1]      # (a later, larger bucket makes the scratch grow)
     xs = [_llama_like(n, 40 + k) for k, n in enumerate(sizes)]
     outs = [torch.zeros_like(x) for x in xs]
     seed, u = 9, 6.0
-    pipe = SinglePassBuckets(DEV, strategy=2, seed=seed, streams=streams, graphs=graphs, u=u)
-    for step in range(1, 6):
-        if step == 4:
-            u = 7.5
-            pipe.set_u(u)
+    pipe = SinglePassBuckets(DEV, strategy=2, seed=seed, streams=streams, u=u)
+    graph = None
+
+    def enqueue():
         pipe.begin_step()
-        for x in xs:
-            x.mul_(1.25)                      # the sources change between steps; a replay must read the new values
         if whole:
             pipe.run_all(list(zip(xs, outs)))
         else:
             for x, o in zip(xs, outs):
                 pipe.run(x, o)
         pipe.join()
+
+    for step in range(1, 6):
+        if recorded and step == 2:
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph):
+                enqueue()
+        if step == 4:
+            u = 7.5
+            pipe.set_u(u)
+        for x in xs:
+            x.mul_(1.25)                      # the sources change between steps; a replay must read the new values
+        if graph is None:
+            enqueue()
+        else:
+            pipe.join()
+            graph.replay()
         torch.cuda.synchronize()
         for k, (x, o) in enumerate(zip(xs, outs)):
             want = _four_calls(capi, x, x.numel(), u, 2, seed, (k << 32) + step)[5]
             assert torch.equal(bits_t(o), bits_t(want)), (step, k)
+            o.zero_()
 
 
 def test_streams_of_the_pipeline_object_run_side_by_side(capi):
@@ -616,35 +630,45 @@ def test_stream_order_after_orders_two_streams(capi):
 
 @pytest.mark.parametrize("streams", [1, 2, 3])
 def test_single_pass_buckets_alternating_between_recorded_and_eager_steps(capi, streams):
-    """the first slot of the pipeline object runs on the caller's stream when a bucket is enqueued eagerly and on its worker
-    stream when a recorded step is replayed: steps that alternate between the two (and a change of u in between) still
-    give the outputs of the four calls on every step"""
+    """a step recorded at the start is replayed on a stream of its own, between steps that are enqueued on the caller's as a list or
+    bucket by bucket (and a change of u in between): every step gives the outputs of the four calls"""
     from dynamiq_sigcomm_artifact_amd.dynamiq_pipeline import SinglePassBuckets
     sizes = [256 * 200, 256 * 200, 256 * 120 + 3, 256 * 200, 256 * 64]
     xs = [_llama_like(n, 60 + k) for k, n in enumerate(sizes)]
     outs = [torch.zeros_like(x) for x in xs]
     seed, u = 4, 6.5
-    pipe = SinglePassBuckets(DEV, strategy=2, seed=seed, streams=streams, graphs=True, u=u)
+    pipe = SinglePassBuckets(DEV, strategy=2, seed=seed, streams=streams, u=u)
     pairs = list(zip(xs, outs))
-    modes = ["all", "all", "all", "each", "all", "each", "each", "all", "each", "all"]
+    main, side = torch.cuda.current_stream(), torch.cuda.Stream()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        pipe.begin_step()
+        pipe.run_all(pairs)
+    modes = ["list", "each", "replay", "replay", "list", "replay", "each", "each", "replay", "list"]
     x_then = [[None] * len(xs) for _ in modes]
     o_then = [[None] * len(xs) for _ in modes]
     us = []
-    # no synchronisation between the steps: only the object's own ordering keeps them apart
+    # no synchronisation between the steps
     for step, mode in enumerate(modes, start=1):
         if step == 5:
             u = 7.25
             pipe.set_u(u)
         us.append(u)
-        pipe.begin_step()
         for k, x in enumerate(xs):
             x.mul_(1.125)
             x_then[step - 1][k] = x.clone()
-        if mode == "all":
-            pipe.run_all(pairs)
+        if mode == "replay":
+            side.wait_stream(main)                # the sources
+            with torch.cuda.stream(side):
+                pipe.join()
+                graph.replay()
         else:
-            for x, o in pairs:
-                pipe.run(x, o)
+            pipe.begin_step()
+            if mode == "list":
+                pipe.run_all(pairs)
+            else:
+                for x, o in pairs:
+                    pipe.run(x, o)
         pipe.join()
         for k, o in enumerate(outs):
             o_then[step - 1][k] = o.clone()
