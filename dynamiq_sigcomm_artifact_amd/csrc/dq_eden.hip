@@ -428,7 +428,8 @@ namespace {
 // costs 25 instruction slots per element, 2.7 us at 2^22 elements.
 constexpr int64_t kEdenDrawnSigns = (int64_t)1 << 22;
 
-// no rotation at all: the slice padded and converted / scaled and converted
+// no rotation at all, which a slice of the C call may ask for (Eden's own have one or two): the slice padded and converted /
+// scaled and converted
 __global__ __launch_bounds__(256) void eden_pad_kernel(const void *__restrict__ src, int dtype, int64_t count, int64_t n,
                                                        float *__restrict__ out)
 {

@@ -61,7 +61,7 @@ struct RhtTileArgs {
 
 // The diagonal drawn where it is applied (sign is then null); flip4 and flip16 serve it.  A type of its own: the kernels
 // fused with the codec run on 64 registers, and a test for a seed that they never have costs them time (2^30 elements there
-// and back 2134 -> 2118 us without it).
+// and back 2134 us with it, 2118 without, as before there were drawn diagonals).
 struct RhtPassArgs : RhtTileArgs {
     SignSeed gen;
 };

@@ -389,7 +389,9 @@ int dq_dynamic_bitrate_bucket(const dq_bucket_t *bucket, int stages, int device,
  * *step_dev + step_more in *step_dev -- a caller that passes step_more = 1 with
  * the first buckets of a training step advances the counter without a launch of
  * its own.  hist (may be NULL, else dq_bitrate_hist_ints() entries): the norm
- * patterns are added to it. */
+ * patterns are added to it.  An output is its own source or lies apart from
+ * all of them (a bucket is read while others are written), likewise in
+ * dq_ranks_allreduce, where it may also be another rank's source. */
 typedef struct dq_roundtrip {
     const void *src;  /* n elements of dtype (DQ_BF16 or DQ_F32) */
     void *out;        /* n elements of dtype, written */
@@ -553,8 +555,8 @@ int dq_eden_dequantize_irht(const uint32_t *packed, int64_t n, const float *cent
 
 /* srrcomp.py:293-326 / :328-354, the slices of a vector in one call: `count`
  * elements of dtype (any of the three), padded with zeros to n = 2^k >= 32, go
- * through `rotations` randomized transforms (the diagonals of seed, seed + 1,
- * ... as dq_rand_diag makes them, the scale 1 / sqrt(n)) and dq_eden_quantize;
+ * through `rotations` (0 or more) randomized transforms (the diagonals of seed,
+ * seed + 1, ... as dq_rand_diag makes them, the scale 1 / sqrt(n)) and dq_eden_quantize;
  * and the way back, scaled by *result and stored as `count` elements of dtype.
  * The same bits as the single calls; a slice is not copied or converted in
  * memory, the diagonal of a short one never written, and slices of up to 2^22
