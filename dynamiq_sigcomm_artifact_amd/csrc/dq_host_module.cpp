@@ -72,12 +72,20 @@ int dtype_code(const at::Tensor &t)
     }
 }
 
+// modulo 2^64: seeds, steps and handles, whatever int() takes; `whole`: whole numbers only
+uint64_t word(PyObject *o, bool whole = false)
+{
+    const py::object made = py::reinterpret_steal<py::object>(whole ? PyNumber_Index(o) : PyNumber_Long(o));
+    if (!made) throw py::error_already_set();
+    return PyLong_AsUnsignedLongLongMask(made.ptr());
+}
+
 // None: torch's current stream, of that device if one is named; a raw handle; a torch stream
 dq_stream_t stream_of(py::handle s, int device = -1)
 {
     if (s.is_none()) return c10::hip::getCurrentHIPStream((c10::DeviceIndex)device).stream();
-    if (PyLong_Check(s.ptr())) return reinterpret_cast<dq_stream_t>(PyLong_AsUnsignedLongLong(s.ptr()));
-    return reinterpret_cast<dq_stream_t>(static_cast<uintptr_t>(py::cast<uint64_t>(s.attr("cuda_stream"))));
+    const py::object raw = PyLong_Check(s.ptr()) || !py::hasattr(s, "cuda_stream") ? py::reinterpret_borrow<py::object>(s) : s.attr("cuda_stream");
+    return reinterpret_cast<dq_stream_t>(static_cast<uintptr_t>(word(raw.ptr())));
 }
 
 // u of the width rule: a number, or a float64 device tensor
@@ -691,7 +699,7 @@ at::Tensor empty_on(int device, int64_t n, at::ScalarType dtype)
 }
 
 // Eden.compress: slices as (start, elements, padded size, rotations); returns one (packed, scale) per slice
-py::list eden_compress(py::handle vec, py::handle boundaries, py::handle centroids, int nbits, int64_t seed, py::sequence slices)
+py::list eden_compress(py::handle vec, py::handle boundaries, py::handle centroids, int nbits, py::handle seed, py::sequence slices)
 {
     Args a;
     const at::Tensor &v = a.tensor(vec);
@@ -713,7 +721,7 @@ py::list eden_compress(py::handle vec, py::handle boundaries, py::handle centroi
         x.rotations = py::cast<int>(s[3]);
         if (start < 0 || x.count <= 0 || start + x.count > v.numel()) refuse("a slice lies outside the vector");
         x.vec = static_cast<char *>(v.data_ptr()) + start * elem;
-        x.seed = seed;
+        x.seed = (int64_t)word(seed.ptr(), true);
         x.nbits = nbits;
         x.boundaries = b;
         x.centroids = c;
@@ -753,7 +761,7 @@ void eden_decompress(py::handle out, py::sequence slices)
         x.result = a.typed(py::object(s[3]), at::kFloat, 1, "scale").data_ptr<float>();
         x.count = py::cast<int64_t>(s[4]);
         x.rotations = py::cast<int>(s[5]);
-        x.seed = py::cast<int64_t>(s[6]);
+        x.seed = (int64_t)word(py::object(s[6]).ptr(), true);
         x.vec = static_cast<char *>(y.data_ptr()) + total * elem;
         total += x.count;
         room += dq_eden_slice_bytes(x.n);
@@ -837,13 +845,6 @@ int64_t integer(PyObject *o)
 }
 
 int small_integer(PyObject *o) { return (int)integer(o); }
-
-uint64_t word(PyObject *o)
-{
-    const unsigned long long v = PyLong_AsUnsignedLongLongMask(o);
-    if (v == (unsigned long long)-1 && PyErr_Occurred()) throw py::error_already_set();
-    return v;
-}
 
 float real(PyObject *o)
 {

@@ -394,6 +394,35 @@ def test_slices_in_one_call_equal_the_single_calls(capi, n, dt):
     assert got.dtype == dt and torch.equal(got, torch.cat(want))
 
 
+@pytest.mark.parametrize("seed", [2 ** 63 + 5, -(2 ** 63), 2 ** 70 + 9, 2 ** 64 - 1])
+def test_seeds_of_any_size(capi, seed):
+    """a seed is taken modulo 2^64, as the single calls take it; one that is no whole number is refused"""
+    from dynamiq_sigcomm_artifact_amd.eden import Eden
+    eden = Eden(device=DEV)
+    x = torch.randn(3000, device=DEV)
+    data = eden.compress(x, 4, seed)
+    low = (seed + 2 ** 63) % 2 ** 64 - 2 ** 63
+    want = eden.compress(x, 4, low)
+    assert all(torch.equal(a["packed_bins"], b["packed_bins"]) and a["seed"] == seed for a, b in zip(data, want))
+    assert torch.equal(eden.decompress(data), eden.decompress(want))
+    with pytest.raises(TypeError):
+        eden.compress(x, 4, 1.0)
+
+
+def test_handles_and_seeds_that_int_takes(capi):
+    """streams as handles of numpy's types, seeds and steps as floats: whatever int() makes a whole number of"""
+    import math
+    n, side = 1 << 14, torch.cuda.Stream()
+    x = torch.randn(n, device=DEV)
+    size = capi.required_bytes(n, 4, 16, 2)
+    a, b = torch.zeros(size, dtype=torch.uint8, device=DEV), torch.zeros(size, dtype=torch.uint8, device=DEV)
+    torch.cuda.synchronize()
+    capi.rht_scaling_compress(x, None, a, 1024, 1 / math.sqrt(1024), 4, 2, seed=7, step=2 ** 64 + 3, stream=side)
+    capi.rht_scaling_compress(x, None, b, 1024, 1 / math.sqrt(1024), 4, 2, seed=np.float64(7), step=3.0, stream=np.int64(side.cuda_stream))
+    torch.cuda.synchronize()
+    assert torch.equal(a, b) and int(a.sum()) > 0
+
+
 @pytest.mark.parametrize("dt", [torch.float32, torch.float16])
 @pytest.mark.parametrize("nbits", [1, 8])
 @pytest.mark.parametrize("sizes", [[(32, 1), (32, 3), (512, 2), (1024, 0), (4096, 1), (8192, 2), (8192, 1), (256, 1), (2048, 1), (64, 2)],
