@@ -326,24 +326,24 @@ struct WorldDiv {
         if (ties && subnormal(q)) q = v / world;
         return q;
     }
-    // sixteen quotients at once when world is not a power of two; the divisions sit behind one branch of the wave (written
+    // a chunk's quotients at once when world is not a power of two; the divisions sit behind one branch of the wave (written
     // as a choice per element, both quotients would be computed for every element)
-    __device__ __forceinline__ void divide16(float (&v)[16]) const
+    template <int N> __device__ __forceinline__ void divide(float (&v)[N]) const
     {
-        float q[16];
+        float q[N];
 #pragma unroll
-        for (int k = 0; k < 16; k++) q[k] = (float)((double)v[k] * inv_d);
+        for (int k = 0; k < N; k++) q[k] = (float)((double)v[k] * inv_d);
         if (ties) {
             bool sub = false;
 #pragma unroll
-            for (int k = 0; k < 16; k++) sub |= __builtin_amdgcn_class(q[k], 0x90); // a subnormal number of either sign
+            for (int k = 0; k < N; k++) sub |= __builtin_amdgcn_class(q[k], 0x90); // a subnormal number of either sign
             if (__builtin_amdgcn_ballot_w64(sub) != 0) {
 #pragma unroll
-                for (int k = 0; k < 16; k++) q[k] = subnormal(q[k]) ? v[k] / world : q[k];
+                for (int k = 0; k < N; k++) q[k] = subnormal(q[k]) ? v[k] / world : q[k];
             }
         }
 #pragma unroll
-        for (int k = 0; k < 16; k++) v[k] = q[k];
+        for (int k = 0; k < N; k++) v[k] = q[k];
     }
     // With fuse16 set, (*this)(v) - mean for a v that came from a 16-bit element is fma(v, inv, -mean): the product with
     // 2^-k is then exact in binary32 (eight or eleven significant bits, no exponent below the binary32 range for world

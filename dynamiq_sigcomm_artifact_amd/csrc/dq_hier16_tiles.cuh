@@ -111,7 +111,7 @@ __device__ __forceinline__ void center_chunk(Raw16<DT> &v, const void *src, int6
         } else {
 #pragma unroll
             for (int i = 0; i < 16; i++) t[i] = v.get(i);
-            ctr.wd.divide16(t);
+            ctr.wd.divide(t);
 #pragma unroll
             for (int i = 0; i < 16; i++) t[i] -= mean;
         }

@@ -11,6 +11,7 @@
 //   tally_kernel       behind it: the widths' counts per bucket and the norm histogram of the search for u
 //   ranks_stats_kernel W ranks: every rank's means, and the reduced statistics
 //   ring_kernel        W ranks, after a plan of the reduced statistics: the ring
+//   ring_quad_kernel   the same on short vectors, one superchunk per wave
 //
 // Measured, start -> now (bit-identical results): 8 ranks x 124,439,808 bf16 elements 2,896 -> 1,149 us per all-reduce (one
 // launch per rank and ring step, packed streams and their exchange copies, against three launches whose traffic is the
@@ -91,13 +92,13 @@ __device__ __forceinline__ void store_tile(void *dst, const Raw16<DT> &out, cons
 }
 
 // T(T(level * step) + mean)
-template <int DT> __device__ __forceinline__ void decode_with_mean(Raw16<DT> &out, float (&lev)[16], float step, float mean)
+template <class RV> __device__ __forceinline__ void decode_with_mean(RV &out, float (&lev)[RV::kCount], float step, float mean)
 {
 #pragma unroll
-    for (int i = 0; i < 16; i++) lev[i] = lev[i] * step;
+    for (int i = 0; i < RV::kCount; i++) lev[i] = lev[i] * step;
     out.set(lev);
 #pragma unroll
-    for (int i = 0; i < 16; i++) lev[i] = out.get(i) + mean;
+    for (int i = 0; i < RV::kCount; i++) lev[i] = out.get(i) + mean;
     out.set(lev);
 }
 
@@ -193,7 +194,7 @@ template <int DT, bool MEE> __global__ __launch_bounds__(64) void roundtrip_kern
     center_loaded<DT>(v, a.wd, active ? mean : 0.0f, e0, n, ragged);
     float lev[16];
     const float scale = quantize_chunk<MEE>(v, r, w, lev);
-    decode_with_mean<DT>(v, lev, scale, bf16_bits_to_f32(mean_bits));
+    decode_with_mean(v, lev, scale, bf16_bits_to_f32(mean_bits));
     wave_lds_sync(); // the statistics' tile has been read
     stage_tile<DT>(v, reinterpret_cast<uint4 *>(lds), lane);
     store_tile<DT>(b.out, v, reinterpret_cast<const uint4 *>(lds), sc, rows_here, n, b.vec != 0, lane);
@@ -454,10 +455,133 @@ template <int DT, int RDT, bool MEE> __global__ __launch_bounds__(64) void ring_
         }
         scale = quantize_chunk<MEE>(v, r, w, lev);
     }
-    decode_with_mean<DT>(v, lev, scale, bf16_bits_to_f32(total_mean));
+    decode_with_mean(v, lev, scale, bf16_bits_to_f32(total_mean));
     stage_tile<DT>(v, stage, lane);
     for (int rank = 0; rank < world; rank++) store_tile<DT>(a.out[rank], v, stage, sc, rows_here, a.n, (a.vec & 2) != 0, lane);
 }
+
+// four elements of a lane, side by side with those of its neighbours
+template <int DT> __device__ __forceinline__ void store_quarter(void *dst, const Raw4<DT> &out, int64_t e, int64_t n, bool vec, bool ragged)
+{
+    if (vec && !ragged) {
+        if constexpr (DT == DQ_F32) {
+            stream_store(reinterpret_cast<uint4 *>(static_cast<uint32_t *>(dst) + e), make_uint4(out.w[0], out.w[1], out.w[2], out.w[3]));
+        } else {
+            typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+            const u32x2 t = {out.w[0], out.w[1]};
+            __builtin_nontemporal_store(t, reinterpret_cast<u32x2 *>(static_cast<uint16_t *>(dst) + e));
+        }
+        return;
+    }
+    const int left = left_here(n, e, 4);
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        if (i < left) {
+            if constexpr (DT == DQ_F32)
+                static_cast<uint32_t *>(dst)[e + i] = out.w[i];
+            else
+                static_cast<uint16_t *>(dst)[e + i] = (uint16_t)(out.w[i >> 1] >> (16 * (i & 1)));
+        }
+    }
+}
+
+constexpr int kQuadWaves = 4;
+
+// ring_kernel with a superchunk per wave, four elements per lane: short vectors, where a wave's chain of `world` steps is all
+// there is to wait for (2 us a step with one wave of ring_kernel per SIMD, 0.7 us here).
+template <int DT, int RDT, bool MEE>
+__global__ __launch_bounds__(64 * kQuadWaves) void ring_quad_kernel(RingArgs<RDT != DQ_PHILOX> a)
+{
+    __shared__ float levels[MEE ? kLevelCount : 1];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), world = a.world;
+    if (MEE) {
+        if (wave == 0) levels_to_lds(a.widths, levels, lane);
+        __syncthreads();
+    }
+    // entry `at` of the three lists end to end; sizes clamped as in ring_kernel
+    const int at = (int)blockIdx.x * kQuadWaves + wave;
+    int cls = 3, k = 0, chunk = 0, in_run = 0;
+    {
+        int used = 0;
+        const int counts[3] = {a.counts[0], a.counts[1], a.counts[2]};
+#pragma unroll
+        for (int g = 0; g < 3; g++) {
+            const int m = min(max(counts[g], 0), a.nsc - used);
+            if (cls == 3 && at - used < m) {
+                const int per = (m + world - 1) / world;
+                cls = g;
+                k = at - used;
+                chunk = k / per;
+                in_run = k - chunk * per;
+            }
+            used += m;
+        }
+    }
+    if (cls == 3) return;
+    const int64_t sc = a.order[(int64_t)cls * a.nsc + k];
+    const int64_t e0 = sc * 256 + lane * 4;
+    const bool ragged = sc * 256 + 256 > a.n;
+    const WidthRegs<MEE> w = width_regs<MEE>(a.widths, cls, levels);
+    const uint32_t total_mean = a.total[2 * sc];
+
+    // What a step needs besides its elements, in the lanes of a few registers: lane s has the addresses and the mean of the
+    // rank of step s.  (Loaded step by step through the scalar cache they are half of a step's time.)
+    const int my_step = min(lane, world - 1), my_rank = chunk + my_step < world ? chunk + my_step : chunk + my_step - world;
+    const uint64_t my_src = reinterpret_cast<uint64_t>(a.src[my_rank]);
+    const float my_mean = a.mean[(int64_t)my_rank * a.nsc + sc];
+    uint64_t my_pool = 0;
+    if constexpr (RDT != DQ_PHILOX)
+        my_pool = reinterpret_cast<uint64_t>(a.pools.pool[cls][my_rank]) +
+                  (int64_t)(a.pools.first[cls][my_rank][my_step] + in_run * 16) * (16 * (RDT == DQ_F32 ? 4 : 2));
+    const auto of_step = [](uint64_t mine, int step) {
+        const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)mine, step);
+        const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(mine >> 32), step);
+        return reinterpret_cast<const void *>((uint64_t)lo | ((uint64_t)hi << 32));
+    };
+    Raw4<DT> next;
+    Raw4<RDT> next_r;
+    next_r.zero();
+    const auto fetch = [&](int step) {
+        load_chunk<DT>(next, of_step(my_src, step), e0, a.n, a.vec & 1, ragged);
+        if constexpr (RDT != DQ_PHILOX) next_r.load(of_step(my_pool, step), lane * 4, (a.vec & 4) != 0);
+    };
+    fetch(0);
+    Raw4<DT> v;
+    uint32_t draws[4];
+    float lev[4], scale = 0.0f;
+#pragma unroll 1
+    for (int step = 0; step < world; step++) {
+        v = next;
+        Raw4<RDT> r = next_r;
+        const float mean = __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(my_mean), step));
+        if (step + 1 < world) fetch(step + 1);
+        if constexpr (RDT == DQ_PHILOX) {
+            if ((step & 3) == 0) {
+                const int mine = step + (lane & 3);
+                int rank = chunk + mine; // (draws of steps beyond the last go unused)
+                if (rank >= world) rank -= world;
+                quad_words(RandKey{a.key.seed + (uint64_t)rank, (uint64_t)mine}, sc * 16 + (lane >> 2), lane, draws);
+            }
+            r.w = draws[0];
+            draws[0] = draws[1]; draws[1] = draws[2]; draws[2] = draws[3];
+        }
+        center_loaded<DT>(v, a.wd, mean, e0, a.n, ragged);
+        if (step > 0) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) lev[i] = __builtin_fmaf(lev[i], scale, v.get(i));
+            v.set(lev); // the sum in the element type
+        }
+        scale = quantize_chunk<MEE>(v, r, w, lev);
+    }
+    decode_with_mean(v, lev, scale, bf16_bits_to_f32(total_mean));
+    for (int rank = 0; rank < world; rank++) store_quarter<DT>(a.out[rank], v, e0, a.n, (a.vec & 2) != 0, ragged);
+}
+
+// Up to here a superchunk per wave, beyond it four: the quads issue more per element (160 instructions per superchunk and step
+// against 90), and from two waves of ring_kernel per SIMD on (8,192 superchunks) that is what counts.  Kernel alone, ring_kernel
+// -> ring_quad_kernel, bf16: 8 ranks x 65,536 15.7 -> 8.7 us, x 1,000,003 20.0 -> 16.2, x 2,000,000 26.3 -> 25.6, x 3,000,000
+// 33.5 -> 35.2; with pools 2 x 100,000 8.1 -> 4.2, 4 x 2,000,000 15.8 -> 12.1, 3 x 4,000,000 15.6 -> 16.8.
+constexpr int kQuadSuperchunks = 8192;
 
 WidthRule make_rule(float u, const double *u_dev)
 {
@@ -576,6 +700,12 @@ static hipError_t run_ring(const RingDesc &d, bool mee, const MeeParams *mp, hip
     a.key = RandKey{d.seed, 0};
     a.wd = make_world_div(d.world, DT == DQ_F32 ? 4 : 2);
     a.widths = make_width_set(mp, mee);
+    if (a.nsc <= kQuadSuperchunks) {
+        const dim3 grid((unsigned)((a.nsc + kQuadWaves - 1) / kQuadWaves)), block(64 * kQuadWaves);
+        if (mee) hipLaunchKernelGGL((ring_quad_kernel<DT, RDT, true>), grid, block, 0, stream, a);
+        else hipLaunchKernelGGL((ring_quad_kernel<DT, RDT, false>), grid, block, 0, stream, a);
+        return hipGetLastError();
+    }
     // every run rounds its superchunks per ring chunk up to whole tiles
     const dim3 grid((unsigned)(a.nsc / (kRowsPerWave * d.world) + 4), (unsigned)d.world);
     if (mee) hipLaunchKernelGGL((ring_kernel<DT, RDT, true>), grid, dim3(64), 0, stream, a);

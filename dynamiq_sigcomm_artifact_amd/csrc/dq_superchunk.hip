@@ -79,7 +79,7 @@ __global__ __launch_bounds__(64) void mean_center_tile_kernel(const void *__rest
 #pragma unroll
             for (int k = 0; k < 16; k++) v[k] = v[k] * wd.inv;
         } else {
-            wd.divide16(v);
+            wd.divide(v);
         }
     } else {
 #pragma unroll

@@ -40,6 +40,7 @@ __device__ __forceinline__ uint32_t pk_max_u16(uint32_t a, uint32_t b)
 template <int DT> struct Raw16;
 
 template <> struct Raw16<DQ_BF16> {
+    static constexpr int kCount = 16;
     uint32_t w[8];
     __device__ __forceinline__ void zero()
     {
@@ -102,6 +103,7 @@ template <> struct Raw16<DQ_BF16> {
 };
 
 template <> struct Raw16<DQ_F32> {
+    static constexpr int kCount = 16;
     uint32_t w[16];
     __device__ __forceinline__ void zero()
     {
@@ -213,6 +215,9 @@ template <> struct Raw16<DQ_PHILOX> {
     }
     __device__ __forceinline__ bool unit_interval() const { return true; }
 };
+
+// random operands that are bytes of the in-kernel stream
+template <class RR> struct DrawnBytes { static constexpr bool value = std::is_same<RR, Raw16<DQ_PHILOX>>::value; };
 
 // ---- the MEE level table on its way into LDS -------------------------------------------------------
 //
@@ -459,7 +464,7 @@ template <int NBITS, bool MEE> struct EstimateGuard {
 // bias - r_i; exact for the in-kernel random bytes ((256 bias - odd byte) / 256 needs 16 bits)
 template <class RR> __device__ __forceinline__ float below(const RR &r, int i, float bias)
 {
-    if constexpr (std::is_same<RR, Raw16<DQ_PHILOX>>::value)
+    if constexpr (DrawnBytes<RR>::value)
         return __builtin_fmaf(r.odd_byte(i), -0.00390625f, bias);
     else
         return bias - r.get(i);

@@ -75,16 +75,174 @@ __device__ __forceinline__ void levels_to_lds(const WidthSet &s, float *levels, 
     }
 }
 
+// ---- a quarter of a chunk per lane ----------------------------------------------------------------------
+//
+// With sixteen elements per lane a wave works through four superchunks, and a short vector has fewer such waves than the GPU
+// has SIMDs: what counts then is the length of a wave's instruction stream.  A lane with four elements makes it a third as
+// long and the waves four times as many: a chunk is a quad of lanes, a superchunk a wave.
+template <int DT> struct Raw4;
+
+template <> struct Raw4<DQ_BF16> {
+    static constexpr int kCount = 4;
+    uint32_t w[2];
+    __device__ __forceinline__ void zero() { w[0] = w[1] = 0u; }
+    // vec: p is 16-byte aligned (and e a multiple of 4)
+    __device__ __forceinline__ void load(const void *p, int64_t e, bool vec)
+    {
+        const volatile uint16_t *h = static_cast<const volatile uint16_t *>(p) + e;
+        if (vec) {
+            const uint2 q = *reinterpret_cast<const uint2 *>(static_cast<const uint16_t *>(p) + e);
+            w[0] = q.x; w[1] = q.y;
+        } else {
+#pragma unroll
+            for (int k = 0; k < 2; k++) w[k] = (uint32_t)h[2 * k] | ((uint32_t)h[2 * k + 1] << 16);
+        }
+    }
+    __device__ __forceinline__ float get(int i) const
+    {
+        return (i & 1) ? __uint_as_float(w[i >> 1] & 0xffff0000u) : __uint_as_float(w[i >> 1] << 16);
+    }
+    __device__ __forceinline__ void set(const float (&t)[4])
+    {
+        w[0] = f32x2_to_bf16x2(t[0], t[1]);
+        w[1] = f32x2_to_bf16x2(t[2], t[3]);
+    }
+    // of the lane's four elements, as those of Raw16
+    __device__ __forceinline__ uint32_t absmax_bits() const
+    {
+        const uint32_t m = pk_max_u16(w[0] & 0x7fff7fffu, w[1] & 0x7fff7fffu);
+        return max(m << 16, m & 0xffff0000u);
+    }
+    __device__ __forceinline__ bool unit_interval() const
+    {
+        const uint32_t m = pk_max_u16(w[0], w[1]);
+        return max(m & 0xffffu, m >> 16) <= 0x3f80u;
+    }
+};
+
+template <> struct Raw4<DQ_F32> {
+    static constexpr int kCount = 4;
+    uint32_t w[4];
+    __device__ __forceinline__ void zero() { w[0] = w[1] = w[2] = w[3] = 0u; }
+    __device__ __forceinline__ void load(const void *p, int64_t e, bool vec)
+    {
+        const volatile uint32_t *f = static_cast<const volatile uint32_t *>(p) + e;
+        if (vec) {
+            const uint4 q = *reinterpret_cast<const uint4 *>(static_cast<const uint32_t *>(p) + e);
+            w[0] = q.x; w[1] = q.y; w[2] = q.z; w[3] = q.w;
+        } else {
+#pragma unroll
+            for (int k = 0; k < 4; k++) w[k] = f[k];
+        }
+    }
+    __device__ __forceinline__ float get(int i) const { return __uint_as_float(w[i]); }
+    __device__ __forceinline__ void set(const float (&t)[4])
+    {
+#pragma unroll
+        for (int k = 0; k < 4; k++) w[k] = __float_as_uint(t[k]);
+    }
+    __device__ __forceinline__ uint32_t absmax_bits() const
+    {
+        return max(max(w[0] & 0x7fffffffu, w[1] & 0x7fffffffu), max(w[2] & 0x7fffffffu, w[3] & 0x7fffffffu));
+    }
+    __device__ __forceinline__ bool unit_interval() const { return max(max(w[0], w[1]), max(w[2], w[3])) <= 0x3f800000u; }
+};
+
+// word lane & 3 of the chunk's block of the rounding stream
+template <> struct Raw4<DQ_PHILOX> {
+    static constexpr int kCount = 4;
+    uint32_t w; // with the lowest bit of every byte set
+    __device__ __forceinline__ void zero() { w = 0x01010101u; }
+    __device__ __forceinline__ float odd_byte(int i) const { return (float)((w >> (8 * i)) & 0xffu); }
+    __device__ __forceinline__ float get(int i) const { return odd_byte(i) * 0.00390625f; }
+    __device__ __forceinline__ bool unit_interval() const { return true; }
+};
+template <> struct DrawnBytes<Raw4<DQ_PHILOX>> { static constexpr bool value = true; };
+
+// The words that the four lanes of a quad need for four draws, of which lane q makes the q-th: word q of all four (a 4 x 4
+// transpose in two exchanges), so that a draw costs a lane a quarter of a block.
+__device__ __forceinline__ void quad_words(const RandKey &key, int64_t chunk, int lane, uint32_t (&w)[4])
+{
+    chunk_uniform_words(key, chunk, w);
+#pragma unroll
+    for (int k = 0; k < 4; k++) w[k] |= 0x01010101u;
+    const bool odd = (lane & 1) != 0, high = (lane & 2) != 0;
+#pragma unroll
+    for (int k = 0; k < 4; k += 2) {
+        const uint32_t got = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(odd ? w[k] : w[k + 1]), 0xB1, 0xf, 0xf, true);
+        w[k] = odd ? got : w[k];
+        w[k + 1] = odd ? w[k + 1] : got;
+    }
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+        const uint32_t got = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(high ? w[k] : w[k + 2]), 0x4E, 0xf, 0xf, true);
+        w[k] = high ? got : w[k];
+        w[k + 2] = high ? w[k + 2] : got;
+    }
+}
+
+// maximum over the lanes of a chunk (N elements per lane), and over those of a superchunk of values that are alike within
+// a chunk; the integer forms for patterns of positive finite floats
+template <int N> __device__ __forceinline__ uint32_t chunk_max(uint32_t u)
+{
+    if (N == 4) {
+        u = max(u, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)u, 0xB1, 0xf, 0xf, true)); // quad_perm [1,0,3,2]
+        u = max(u, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)u, 0x4E, 0xf, 0xf, true)); // quad_perm [2,3,0,1]
+    }
+    return u;
+}
+
+template <int N> __device__ __forceinline__ float chunk_max(float v)
+{
+    if (N == 4) {
+        v = __builtin_fmaxf(v, dpp_f32<0xB1>(v));
+        v = __builtin_fmaxf(v, dpp_f32<0x4E>(v));
+    }
+    return v;
+}
+
+// the other row of a pair (lane bit 4) / of the other half (lane bit 5): two rows that change places with themselves leave
+// one of them in either register
+template <class F> __device__ __forceinline__ uint32_t across_rows(uint32_t u, F combine)
+{
+    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+    const u32x2 a = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane16_swap(u, u, false, false));
+    u = combine(a[0], a[1]);
+    const u32x2 b = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(u, u, false, false));
+    return combine(b[0], b[1]);
+}
+
+template <int N> __device__ __forceinline__ float superchunk_max_pos(float v)
+{
+    if (N == 16) return row16_max_pos(v);
+    uint32_t u = __float_as_uint(v);
+    u = max(u, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)u, 0x141, 0xf, 0xf, true)); // row_half_mirror
+    u = max(u, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)u, 0x140, 0xf, 0xf, true)); // row_mirror
+    return __uint_as_float(across_rows(u, [](uint32_t p, uint32_t q) { return max(p, q); }));
+}
+
+template <int N> __device__ __forceinline__ float superchunk_max(float v)
+{
+    if (N == 16) return row16_max(v);
+    v = __builtin_fmaxf(v, dpp_f32<0x141>(v));
+    v = __builtin_fmaxf(v, dpp_f32<0x140>(v));
+    return __uint_as_float(across_rows(__float_as_uint(v), [](uint32_t p, uint32_t q) {
+        return __float_as_uint(__builtin_fmaxf(__uint_as_float(p), __uint_as_float(q)));
+    }));
+}
+
 // the quantiser with every guard of the reference (chunk_encode_guarded): lev[i] = level of element i, returns the
 // chunk's step (chunk_decode's sc)
 template <bool MEE, class RV, class RR>
-__device__ __forceinline__ float quantize_guarded(const RV &v, const RR &rnd, const WidthRegs<MEE> &w, float (&lev)[16])
+__device__ __forceinline__ float quantize_guarded(const RV &v, const RR &rnd, const WidthRegs<MEE> &w, float (&lev)[RV::kCount])
 {
+    constexpr int N = RV::kCount;
     float a = __builtin_fabsf(v.get(0));
 #pragma unroll
-    for (int i = 1; i < 16; i++) a = __builtin_fmaxf(a, __builtin_fabsf(v.get(i)));
+    for (int i = 1; i < N; i++) a = __builtin_fmaxf(a, __builtin_fabsf(v.get(i)));
+    a = chunk_max<N>(a);
     const float s = pos_scale(MEE ? a / pos_scale(w.cmm) + 1e-7f : a / w.r + 1e-7f);
-    const float g = pos_scale(row16_max(s));
+    const float g = pos_scale(superchunk_max<N>(s));
     const uint32_t unit_bits = f32_to_bf16_bits(pos_scale(g / 255.0f));
     const float unit = pos_scale(bf16_bits_to_f32(unit_bits));
     float ratio = pos_scale(s) / pos_scale(g) * 255.0f;
@@ -93,7 +251,7 @@ __device__ __forceinline__ float quantize_guarded(const RV &v, const RR &rnd, co
     const float d = pos_scale(pos_scale((float)qi * unit));
     const int top = (int)w.r;
 #pragma unroll
-    for (int i = 0; i < 16; i++) {
+    for (int i = 0; i < N; i++) {
         float x = v.get(i) / d;
         if (MEE) x = mee_inverse_guarded(x, w.c, w.l2b);
         const int level = clamp_code(sr_guarded(x, rnd.get(i)), top) - top;
@@ -106,20 +264,21 @@ __device__ __forceinline__ float quantize_guarded(const RV &v, const RR &rnd, co
 // L - r + 1 instead of L - r + R + 1 -- its floor is the signed level -- against the same guard: the constant 1 + kDelta
 // minus r is as exact (1 and 20 bits of fraction), and the fused multiply-add rounds a number of less magnitude.
 template <bool MEE, class RV, class RR>
-__device__ __forceinline__ float quantize_fast(const RV &v, const RR &rnd, uint32_t amax_bits, const WidthRegs<MEE> &w, float (&lev)[16])
+__device__ __forceinline__ float quantize_fast(const RV &v, const RR &rnd, uint32_t amax_bits, const WidthRegs<MEE> &w, float (&lev)[RV::kCount])
 {
+    constexpr int N = RV::kCount;
     const float s = div_by(__uint_as_float(amax_bits), w.inv_top) + 1e-7f; // (2 bits: R = 1, the product with 1)
-    const float g = row16_max_pos(s);
+    const float g = superchunk_max_pos<N>(s);
     const float unit = bf16_bits_to_f32(f32_to_bf16_bits(div_by(g, 1.0 / 255.0)));
     const float ratio = div_by(s, recip_f64(g)) * 255.0f;
     const int qi = min(max((int)__builtin_ceilf(ratio), 1), 255);
     const float d = (float)qi * unit;
     const float rd = __builtin_amdgcn_rcpf(d);
     const float rc = MEE ? (float)w.inv_c : 0.0f, rl2b = MEE ? (float)w.inv_l2b : 0.0f;
-    bool doubt[16];
-    uint64_t lanes_in_doubt[16], any = 0;
+    bool doubt[N];
+    uint64_t lanes_in_doubt[N], any = 0;
 #pragma unroll
-    for (int i = 0; i < 16; i++) {
+    for (int i = 0; i < N; i++) {
         const float vi = v.get(i);
         const float off = below(rnd, i, w.bias);
         float t;
@@ -137,7 +296,7 @@ __device__ __forceinline__ float quantize_fast(const RV &v, const RR &rnd, uint3
     if (any != 0) {
         const double yd = recip_f64(d);
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
+        for (int i = 0; i < N; i++) {
             if (lanes_in_doubt[i] != 0) {
                 const float sv = (float)exact_code_fast<MEE>(v.get(i), rnd.get(i), d, yd, w);
                 if (doubt[i]) lev[i] = __builtin_amdgcn_fmed3f(sv, -w.r, w.r);
@@ -146,16 +305,16 @@ __device__ __forceinline__ float quantize_fast(const RV &v, const RR &rnd, uint3
     }
     if (MEE) {
 #pragma unroll
-        for (int i = 0; i < 16; i++) lev[i] = w.table[(int)lev[i]];
+        for (int i = 0; i < N; i++) lev[i] = w.table[(int)lev[i]];
     }
     return nonneg_scale((float)qi * nonneg_scale(unit));
 }
 
-// levels and step of the lane's chunk; every lane of the wave must call
+// levels of the lane's elements and step of their chunk; every lane of the wave must call
 template <bool MEE, class RV, class RR>
-__device__ __forceinline__ float quantize_chunk(const RV &v, const RR &rnd, const WidthRegs<MEE> &w, float (&lev)[16])
+__device__ __forceinline__ float quantize_chunk(const RV &v, const RR &rnd, const WidthRegs<MEE> &w, float (&lev)[RV::kCount])
 {
-    const uint32_t amax = v.absmax_bits();
+    const uint32_t amax = chunk_max<RV::kCount>(v.absmax_bits());
     const bool lane_fast = amax <= kFastMaxBits && rnd.unit_interval();
     if (__builtin_amdgcn_ballot_w64(!lane_fast) == 0) return quantize_fast<MEE>(v, rnd, amax, w, lev);
     return quantize_guarded<MEE>(v, rnd, w, lev);
@@ -198,17 +357,18 @@ __device__ __forceinline__ int left_here(int64_t n, int64_t e, int most)
 // Every element is loaded, those beyond the end from the last one's address, and then masked: sixteen loads in flight
 // together.  (Each behind its own comparison they went one by one, and the one ragged wave of a launch outlasted the others:
 // 4 of 26 us on 8 x 1,000,003 elements.)
-template <int DT> __device__ __forceinline__ void load_chunk_guarded(Raw16<DT> &v, const void *src, int64_t e0, int64_t n)
+template <int DT, class RV> __device__ __forceinline__ void load_chunk_guarded(RV &v, const void *src, int64_t e0, int64_t n)
 {
     typedef typename ElemIO<DT>::storage elem;
-    const int left = left_here(n, e0, 16), last = max(left - 1, 0);
+    constexpr int N = RV::kCount;
+    const int left = left_here(n, e0, N), last = max(left - 1, 0);
     const elem *p = static_cast<const elem *>(src) + min(e0, n - 1);
-    elem x[16];
+    elem x[N];
 #pragma unroll
-    for (int i = 0; i < 16; i++) x[i] = p[min(i, last)];
+    for (int i = 0; i < N; i++) x[i] = p[min(i, last)];
     v.zero();
 #pragma unroll
-    for (int i = 0; i < 16; i++) {
+    for (int i = 0; i < N; i++) {
         if (DT == DQ_F32)
             v.w[i] = i < left ? __builtin_bit_cast(uint32_t, (float)x[i]) : 0u;
         else
@@ -216,9 +376,9 @@ template <int DT> __device__ __forceinline__ void load_chunk_guarded(Raw16<DT> &
     }
 }
 
-// elements [e0, e0 + 16) of src, zero at and beyond n; ragged: the wave's tile reaches beyond n (uniform)
-template <int DT>
-__device__ __forceinline__ void load_chunk(Raw16<DT> &v, const void *src, int64_t e0, int64_t n, bool vec, bool ragged)
+// the lane's elements from e0 on, zero at and beyond n; ragged: the wave's tile reaches beyond n (uniform)
+template <int DT, class RV>
+__device__ __forceinline__ void load_chunk(RV &v, const void *src, int64_t e0, int64_t n, bool vec, bool ragged)
 {
     if (!ragged)
         v.load(src, e0, vec);
@@ -227,27 +387,28 @@ __device__ __forceinline__ void load_chunk(Raw16<DT> &v, const void *src, int64_
 }
 
 // v becomes T(v / world - mean), zero at and beyond element n of the vector (center_chunk without its own loads)
-template <int DT>
-__device__ __forceinline__ void center_loaded(Raw16<DT> &v, const WorldDiv &wd, float mean, int64_t e0, int64_t n, bool ragged)
+template <int DT, class RV>
+__device__ __forceinline__ void center_loaded(RV &v, const WorldDiv &wd, float mean, int64_t e0, int64_t n, bool ragged)
 {
-    float t[16];
+    constexpr int N = RV::kCount;
+    float t[N];
     if (DT != DQ_F32 && wd.fuse16) {
 #pragma unroll
-        for (int i = 0; i < 16; i++) t[i] = __builtin_fmaf(v.get(i), wd.inv, -mean);
+        for (int i = 0; i < N; i++) t[i] = __builtin_fmaf(v.get(i), wd.inv, -mean);
     } else if (wd.pow2) {
 #pragma unroll
-        for (int i = 0; i < 16; i++) t[i] = v.get(i) * wd.inv - mean;
+        for (int i = 0; i < N; i++) t[i] = v.get(i) * wd.inv - mean;
     } else {
 #pragma unroll
-        for (int i = 0; i < 16; i++) t[i] = v.get(i);
-        wd.divide16(t);
+        for (int i = 0; i < N; i++) t[i] = v.get(i);
+        wd.divide(t);
 #pragma unroll
-        for (int i = 0; i < 16; i++) t[i] -= mean;
+        for (int i = 0; i < N; i++) t[i] -= mean;
     }
     if (ragged) {
-        const int left = left_here(n, e0, 16);
+        const int left = left_here(n, e0, N);
 #pragma unroll
-        for (int i = 0; i < 16; i++) t[i] = i < left ? t[i] : 0.0f;
+        for (int i = 0; i < N; i++) t[i] = i < left ? t[i] : 0.0f;
     }
     v.set(t);
 }
@@ -295,7 +456,7 @@ __device__ __forceinline__ void tile_sums(const Raw16<DT> &v, const WorldDiv &wd
             for (int k = 0; k < 16; k++) t[k] = t[k] * wd.inv;
         }
     } else {
-        wd.divide16(t);
+        wd.divide(t);
     }
     float a[8], b[8];
 #pragma unroll

@@ -261,6 +261,12 @@ def test_pooled_ring_in_registers_equals_op_sequence(capi, W, n):
         assert all(x.rand_seed == y.rand_seed for q in (8, 4, 2) for x, y in zip(a[q], b[q]))
 
 
+@pytest.mark.parametrize("W,n", [(2, 256 * 8192), (3, 256 * 8193 - 5)])
+def test_pooled_ring_on_either_side_of_a_superchunk_per_wave(capi, W, n):
+    """the last length that takes a wave per superchunk and the first one that takes four superchunks per wave"""
+    test_pooled_ring_in_registers_equals_op_sequence(capi, W, n)
+
+
 def test_ranks_that_share_a_compressor(capi):
     """one compressor object for all ranks: its pool is walked in the order of the ring's calls, step by step; a compressor of
     another width in a list takes the call-by-call ring"""

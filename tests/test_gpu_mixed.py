@@ -710,6 +710,12 @@ def test_ranks_in_registers_equal_the_ring_in_steps(capi, W, n, dt):
         assert all(torch.equal(bits_t(x), bits_t(y)) for x, y in zip(again, ref))
 
 
+@pytest.mark.parametrize("W,n", [(2, 256 * 8192), (3, 256 * 8192 + 1), (5, 256 * 8195)])
+def test_ranks_on_either_side_of_a_superchunk_per_wave(capi, W, n):
+    """the last length that takes a wave per superchunk and the first ones that take four superchunks per wave"""
+    test_ranks_in_registers_equal_the_ring_in_steps(capi, W, n, torch.bfloat16)
+
+
 @pytest.mark.parametrize("W", [1, 3])
 @pytest.mark.parametrize("elsewhere", [False, pytest.param(True, marks=pytest.mark.skipif(
     not torch.cuda.is_available() or torch.cuda.device_count() < 2, reason="needs a second GPU"))])
