@@ -376,6 +376,29 @@ __device__ __forceinline__ float thc_level(float v, float u, float lo, float del
     return fl + ((u < prob) ? 1.0f : 0.0f);
 }
 
+// thc_level of N elements (in and out) with the division as an estimate: the quotient enters level = floor(x) + (u < frac(x)) only
+// through that comparison, so an estimate within e of it decides unless frac(x) - u comes within e of 0 -- or of +-1, where the
+// estimate and the quotient may lie on either side of an integer.  Such elements (one in 10^4 at 64 levels), and everything that is
+// not a number, take thc_level itself.  v_rcp_f32 is good to 1 ulp and the product to half of one, the quotient itself to half: e <
+// top 2^-22, and the clamp can come last.  35 instead of 75 issue cycles per element.
+template <int N> __device__ __forceinline__ void thc_levels(float (&v)[N], const float (&u)[N], float lo, float delta, float top)
+{
+    const float rd = __builtin_amdgcn_rcpf(delta);
+    const float sure = 0.5f - (top + 1.0f) * 0x1p-21f;
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        const float x = (v[i] - lo) * rd;
+        const float fl = __builtin_floorf(x), w = (x - fl) - u[i];
+        const bool decided = __builtin_fabsf(__builtin_fabsf(w) - 0.5f) <= sure;
+        float level = __builtin_amdgcn_fmed3f(fl + (w > 0.0f ? 1.0f : 0.0f), 0.0f, top);
+        if (__builtin_amdgcn_ballot_w64(!decided) != 0) {
+            asm volatile(""); // (a branch of the wave: the compiler would select otherwise)
+            if (!decided) level = thc_level(v[i], u[i], lo, delta, top);
+        }
+        v[i] = level;
+    }
+}
+
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 // A 16-byte store of output that this kernel does not read again, with the non-temporal hint: the decoders' element

@@ -71,7 +71,7 @@ template <bool ENDS> using PassArgs = typename std::conditional<ENDS, RhtPassArg
 // the low word of every product is used, and the one carry that is, of the addition, is added back by hand).  Four
 // multiplications at a quarter of the rate, about 25 instruction slots per element: cheaper than a launch that writes
 // the bits while the vector is short (the rule is in launch_eden_compress).
-__device__ __forceinline__ uint32_t rand_diag_negative(const SignSeed &s, uint32_t k, uint32_t j)
+__device__ __forceinline__ uint32_t rand_diag_column(const SignSeed &s, uint32_t j)
 {
     uint32_t r = j + s.ss;
     r = 1103515245u * r + 12345u + s.ss;
@@ -80,8 +80,15 @@ __device__ __forceinline__ uint32_t rand_diag_negative(const SignSeed &s, uint32
     const uint32_t carry = q < r ? 0x10000u : 0u;
     r = (q ^ ((q >> 16) | carry)) * 0x85ebca6bu;
     r = (r ^ (r >> 13)) * 0xc2b2ae35u;
-    r ^= r >> 16;
-    return ~(r << (28 - 4 * k)) & 0x80000000u; // +1 where the nibble is >= 8
+    return r ^ (r >> 16);
+}
+
+// the sign bit of element j of segment k: +1 where the nibble is >= 8
+__device__ __forceinline__ uint32_t nibble_negative(uint32_t r, uint32_t k) { return ~(r << (28 - 4 * k)) & 0x80000000u; }
+
+__device__ __forceinline__ uint32_t rand_diag_negative(const SignSeed &s, uint32_t k, uint32_t j)
+{
+    return nibble_negative(rand_diag_column(s, j), k);
 }
 
 // the sign flip of elements g .. g + 3 (g a multiple of 4) / of element g.  A packed sign flips the sign bit,
@@ -330,9 +337,25 @@ __global__ void irht_decompress_kernel(const uint8_t *__restrict__ src, float *_
 __device__ __forceinline__ bool has_diagonal(const RhtTileArgs &a) { return a.sign != nullptr; }
 __device__ __forceinline__ bool has_diagonal(const RhtPassArgs &a) { return a.sign || a.gen.bits != 0; }
 
+// sixteen signs from the low half of a word, the first element's in bit 0
+__device__ __forceinline__ void flip16_bits(float (&v)[16], uint32_t w)
+{
+    // from the last element down, its bit at the top: doubling shifts and issues in half the time of a shift
+    w <<= 16;
+#pragma unroll
+    for (int k = 15; k >= 0; k--) {
+        v[k] = __uint_as_float(__float_as_uint(v[k]) ^ (w & 0x80000000u));
+        w += w;
+    }
+}
+
 template <class A> __device__ __forceinline__ void flip16(float (&v)[16], const A &a, int64_t g)
 {
     if (!has_diagonal(a)) return;
+    if (a.sign && a.sign_bits) {
+        flip16_bits(v, static_cast<const uint32_t *>(a.sign)[g >> 5] >> (g & 31));
+        return;
+    }
 #pragma unroll
     for (int k = 0; k < 4; k++) {
         float4 q = make_float4(v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3]);
@@ -512,6 +535,48 @@ __device__ __forceinline__ void store4(float *__restrict__ x, float4 v, const Pa
     }
 }
 
+// lane bit 4 (16) or 5 (32) changes places with register bit RB: one instruction per two registers
+template <int LANES, int RB> __device__ __forceinline__ void swap_lane_bit(float (&v)[16])
+{
+    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+        if ((i >> RB) & 1) continue;
+        const uint32_t a = __float_as_uint(v[i]), b = __float_as_uint(v[i | (1 << RB)]);
+        const u32x2 r = LANES == 16 ? __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane16_swap(a, b, false, false))
+                                    : __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(a, b, false, false));
+        v[i] = __uint_as_float(r[0]);
+        v[i | (1 << RB)] = __uint_as_float(r[1]);
+    }
+}
+
+// the stage of register bit RB
+template <int RB> __device__ __forceinline__ void stage_of(float (&v)[16])
+{
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+        if ((i >> RB) & 1) continue;
+        const float p = v[i], q = v[i | (1 << RB)];
+        v[i] = p + q;
+        v[i | (1 << RB)] = p - q;
+    }
+}
+
+// lds_pass whose results go to memory: consecutive lanes hold consecutive elements (P >= 6)
+template <int P, int M> __device__ __forceinline__ void lds_pass_out(const float *lds, int kt, int tid, int nthreads, float *__restrict__ out)
+{
+    for (int u = tid; u < 1 << (kt - M); u += nthreads) {
+        const int base = tuple_base<P, M>(u, kt - P - M);
+        const float *q = lds + pad_idx(base);
+        float v[1 << M];
+#pragma unroll
+        for (int j = 0; j < (1 << M); j++) v[j] = q[tuple_step<P>(j)];
+        butterflies<M>(v);
+#pragma unroll
+        for (int j = 0; j < (1 << M); j++) out[base + (j << P)] = v[j];
+    }
+}
+
 // The transform alone (dq_rht_blocked, the first pass of a long dq_hadamard) with the structure of the two kernels
 // above: a lane loads its chunk of 16 consecutive floats, does the stages of strides 1..8 on its registers, the rest
 // runs as LDS passes of up to five stages, and the tile leaves as coalesced 16-byte stores with the scale and (inverse
@@ -578,6 +643,79 @@ __device__ __forceinline__ void tile_pass(float *__restrict__ x, const PassArgs<
     }
 }
 
+// The first pass of a long transform: the tile is one block of 2^10 .. 2^14 elements, a chunk per thread, with nothing to do on
+// the way out.  The last stages store from registers, as whole 256-byte runs: one trip through the LDS and one barrier less
+// than tile_pass.  Blocks of 2^13 and 2^14 do one or two more stages in front of the LDS, by lane bit 5 (and 4) changing places with
+// a register bit: what is left then are two passes of four stages that all threads take part in.  Bound like the strided
+// passes; 2^23 elements from bf16 levels 13.4 -> 11.8 us, from a 25 MB gradient 17.3 -> 15.0.
+template <bool ENDS>
+__device__ __forceinline__ void first_pass(float *__restrict__ x, const PassArgs<ENDS> &a, int sign_mode, const TransformEnds &e, unsigned block,
+                                           float *lds)
+{
+    const int tid = threadIdx.x;
+    const int64_t origin = (int64_t)block << a.kt;
+    PassArgs<ENDS> in = a;
+    if (sign_mode != 1) {
+        in.sign = nullptr;
+        if constexpr (ENDS) in.gen.bits = 0;
+    }
+    const float *cen = lds + padded_tile_floats(a.kt); // EDEN's centroids sit behind the tile
+    if (ENDS && e.in_planes) {
+        for (int k = tid; k < (1 << e.in_nbits); k += blockDim.x) lds[padded_tile_floats(a.kt) + k] = e.in_centroids[k];
+        __syncthreads();
+    }
+    const int nthreads = 1 << (a.kt - 4);
+    if (tid < nthreads) { // (a launch of several passes has the threads of the largest; they come in whole waves)
+        const int lane = tid & 63;
+        float v[16];
+        if (a.kt == 13) {
+            const int c = (tid & ~63) | ((lane & 31) << 1) | (lane >> 5);
+            fetch_chunk<ENDS>(v, x, in, e, cen, origin + c * 16);
+            butterflies<4>(v);
+            swap_lane_bit<32, 0>(v);
+            stage_of<0>(v); // e4
+            float *slot = lds + pad_idx(((c >> 1) << 5) | (lane >> 5));
+#pragma unroll
+            for (int i = 0; i < 16; i++) slot[((i & 1) << 4) | (i & 14)] = v[i];
+        } else if (a.kt == 14) {
+            const int c = (tid & ~63) | ((lane & 15) << 2) | (((lane >> 4) & 1) << 1) | (lane >> 5);
+            fetch_chunk<ENDS>(v, x, in, e, cen, origin + c * 16);
+            butterflies<4>(v);
+            swap_lane_bit<32, 1>(v);
+            stage_of<1>(v); // e4
+            swap_lane_bit<16, 0>(v);
+            stage_of<0>(v); // e5
+            float *slot = lds + pad_idx(((c >> 2) << 6) | ((lane >> 5) << 1) | ((lane >> 4) & 1));
+#pragma unroll
+            for (int i = 0; i < 16; i++) slot[pad_idx(((i & 1) << 5) | (((i >> 1) & 1) << 4) | (i & 12))] = v[i];
+        } else {
+            fetch_chunk<ENDS>(v, x, in, e, cen, origin + tid * 16);
+            butterflies<4>(v);
+            float *slot = lds + chunk_word(tid);
+#pragma unroll
+            for (int i = 0; i < 16; i++) slot[i] = v[i];
+        }
+    }
+    __syncthreads();
+    const int step = blockDim.x;
+    switch (a.kt) {
+    case 10: lds_pass<4, 2>(lds, 10, tid, step); break;
+    case 11: lds_pass<4, 3>(lds, 11, tid, step); break;
+    case 12: lds_pass<4, 4>(lds, 12, tid, step); break;
+    case 13: lds_pass<5, 4>(lds, 13, tid, step); break;
+    default: lds_pass<6, 4>(lds, 14, tid, step); break;
+    }
+    __syncthreads();
+    float *out = x + origin;
+    switch (a.kt) {
+    case 10: lds_pass_out<6, 4>(lds, 10, tid, step, out); break;
+    case 11: lds_pass_out<7, 4>(lds, 11, tid, step, out); break;
+    case 12: lds_pass_out<8, 4>(lds, 12, tid, step, out); break;
+    case 13: lds_pass_out<9, 4>(lds, 13, tid, step, out); break;
+    default: lds_pass_out<10, 4>(lds, 14, tid, step, out); break;
+    }
+}
+
 template <bool ENDS>
 __global__ void rht_tile_kernel(float *__restrict__ x, PassArgs<ENDS> a, int sign_mode, int apply_scale, TransformEnds e)
 {
@@ -585,83 +723,208 @@ __global__ void rht_tile_kernel(float *__restrict__ x, PassArgs<ENDS> a, int sig
     tile_pass<ENDS>(x, a, sign_mode, apply_scale, e, blockIdx.x, lds);
 }
 
-// A later pass of a transform longer than one tile: index bits [sbits, sbits + rbits) of the vector.  A tile is
-// 2^rbits rows of 32 consecutive floats (128 bytes), row stride 2^sbits elements; in LDS it is row-major, so row bit b
-// is tile bit b + 5.  A thread owns column tid % 32 of sixteen consecutive rows: it loads them (every load instruction of
-// a wave covers two whole 128-byte row segments), does the four lowest row stages on its registers and leaves the other
-// rbits - 4 (at most 6) to one or two LDS passes.  sign_mode: 0, or 2 = flip on store (the last pass of an inverse).
-template <bool ENDS>
-__device__ __forceinline__ void strided_pass(float *__restrict__ x, const PassArgs<ENDS> &a, int rbits, int sbits, int sign_mode,
-                                             int apply_scale, const TransformEnds &e, unsigned block, float *lds)
+// A later pass of a transform longer than one tile: index bits [sbits, sbits + A + B) of the vector.  A tile is 2^(A + B)
+// rows of 32 consecutive floats (128 bytes), row stride 2^sbits elements.  A thread owns column tid % 32 of 2^A consecutive
+// rows: it loads them (every load instruction of a wave covers two whole 128-byte row segments), does the A lowest row
+// stages on its registers, hands the rows over through the LDS once, does the other B stages on rows 2^A apart and stores
+// them from its registers, as whole row segments again.  The LDS needs no padding: 32 lanes are the 32 columns of a row.
+// A = 4 (5 for 512 and 1024 rows), so a thread has 16 (32) values and a tile tile / 16 (512 and 1024) threads.
+// Bound by the memory's latency: all workgroups of a pass are on the chip at once, load together and store together.
+// One trip through the LDS instead of three or four: 2^23 elements, 1024 rows back to a 25 MB vector 17.2 -> 13.3 us, to THC's
+// levels 19.0 -> 17.8 (67 MB read); both directions of THC on 25 MB 82.6 -> 70.2, on 16,000,000 elements 146.7 -> 118.7, EDEN on
+// 500,000 36.5 -> 31.7, on 12,000,000 157 -> 136 (with the first pass below).
+// sign_mode: 0, or 2 = flip on store (the last pass of an inverse).
+template <bool ENDS, int A, int B>
+__device__ __forceinline__ void strided_rows(float *__restrict__ x, const PassArgs<ENDS> &a, int sbits, int sign_mode, int apply_scale,
+                                             const TransformEnds &e, unsigned block, float *lds)
 {
-    const int tid = threadIdx.x, nthreads = blockDim.x;
-    const int tile = 1 << (rbits + 5);
+    constexpr int R1 = 1 << A, R2 = 1 << B;
+    const int tid = threadIdx.x;
     // (shift and mask: written as a quotient and remainder by the power of two, the compiler expands a 64-bit
     // division in front of the kernel's first loads)
     const int64_t hi = (int64_t)(block >> (sbits - 5)), mid = (int64_t)(block & ((1u << (sbits - 5)) - 1u));
-    const int64_t origin = (hi << (sbits + rbits)) + (mid << 5);
-    const int col = tid & 31;
-    const int groups = tile >> 9; // groups of sixteen rows
-    if (groups == 2 * (nthreads >> 5)) {
-        // 1024 rows: both groups of a thread are loaded before either is used
-        const int r0 = (tid >> 5) * 16, r1 = r0 + (nthreads >> 5) * 16;
-        float v[16], w[16];
+    const int64_t origin = (hi << (sbits + A + B)) + (mid << 5);
+    const int col = tid & 31, group = tid >> 5;
+    const bool mine = group < R2; // (a launch of several passes has the threads of the largest)
+    float v[R1];
+    if (mine) {
+        const float *from = x + origin + ((int64_t)(group << A) << sbits) + col;
 #pragma unroll
-        for (int j = 0; j < 16; j++) v[j] = x[origin + ((int64_t)(r0 + j) << sbits) + col];
+        for (int j = 0; j < R1; j++) v[j] = from[(int64_t)j << sbits];
+        butterflies<A>(v);
+    }
+    // THC's uniform values are on their way while the stages run, where one workgroup has a CU to itself (1024 rows; with 256 they
+    // gain nothing)
+    constexpr bool kAhead = ENDS && A == 5 && B == 5;
+    float u[R2];
+    if constexpr (kAhead) {
+        if (e.out_levels && mine) {
+            const float *from = e.uniform + origin + ((int64_t)group << sbits) + col;
 #pragma unroll
-        for (int j = 0; j < 16; j++) w[j] = x[origin + ((int64_t)(r1 + j) << sbits) + col];
-        butterflies<4>(v);
-        butterflies<4>(w);
-#pragma unroll
-        for (int j = 0; j < 16; j++) lds[pad_idx((r0 + j) * 32 + col)] = v[j];
-#pragma unroll
-        for (int j = 0; j < 16; j++) lds[pad_idx((r1 + j) * 32 + col)] = w[j];
-    } else {
-        for (int grp = tid >> 5; grp < groups; grp += nthreads >> 5) {
-            float v[16];
-#pragma unroll
-            for (int j = 0; j < 16; j++) v[j] = x[origin + ((int64_t)(grp * 16 + j) << sbits) + col];
-            butterflies<4>(v);
-#pragma unroll
-            for (int j = 0; j < 16; j++) lds[pad_idx((grp * 16 + j) * 32 + col)] = v[j];
+            for (int i = 0; i < R2; i++) u[i] = from[(int64_t)i << (A + sbits)];
         }
     }
-    __syncthreads();
-#define DQ_PASS(P, M)                                  \
-    lds_pass<P, M>(lds, rbits + 5, tid, nthreads);     \
-    __syncthreads();
-    switch (rbits - 4) {
-    case 1: DQ_PASS(9, 1) break;
-    case 2: DQ_PASS(9, 2) break;
-    case 3: DQ_PASS(9, 3) break;
-    case 4: DQ_PASS(9, 4) break;
-    case 5: DQ_PASS(9, 5) break;
-    case 6: DQ_PASS(9, 3) DQ_PASS(12, 3) break;
-    default: break;
-    }
-#undef DQ_PASS
-    if (a.vec) {
-        for (int i = tid * 4; i < tile; i += nthreads * 4) {
-            const int64_t g = origin + ((int64_t)(i >> 5) << sbits) + (i & 31);
-            const int q = pad_idx(i);
-            store4<ENDS>(x, make_float4(lds[q], lds[q + 1], lds[q + 2], lds[q + 3]), a, e, sign_mode, apply_scale, g);
+    float post = 1.0f, lo = 0.0f, delta = 1.0f;
+    if (ENDS && e.post_scale) post = *e.post_scale;
+    if (ENDS && e.out_levels) grid_of(e.grid, e.out_lo, e.out_delta, lo, delta);
+    if constexpr (B > 0) {
+        if (mine) {
+#pragma unroll
+            for (int j = 0; j < R1; j++) lds[((group << A) + j) * 32 + col] = v[j];
         }
-    } else {
-        for (int i = tid; i < tile; i += nthreads) {
-            const int64_t g = origin + ((int64_t)(i >> 5) << sbits) + (i & 31);
-            float v = lds[pad_idx(i)];
-            if (apply_scale) v *= a.scale;
-            x[g] = sign_mode == 2 ? flip1(v, a, g) : v;
+        __syncthreads();
+        if (!mine) return;
+    }
+    const bool flips = sign_mode == 2;
+    bool drawn = false;
+    if constexpr (ENDS) drawn = flips && a.gen.bits != 0;
+    // rows i 2^A + row, i < 2^B, of one column
+    const auto finish = [&](float (&w)[R2], int row) {
+        const int64_t first = origin + ((int64_t)row << sbits) + col;
+        if (apply_scale) {
+#pragma unroll
+            for (int i = 0; i < R2; i++) w[i] *= a.scale;
+        }
+        if (drawn) {
+            if constexpr (ENDS) {
+                const uint32_t column_mask = (1u << a.gen.bits) - 1u;
+                if constexpr (B >= 3) {
+                    if (a.gen.bits + 3 == sbits + A + B) {
+                        // the whole vector: the eight elements of a column of the diagonal are 2^(B - 3) of these rows apart
+#pragma unroll
+                        for (int i = 0; i < R2 / 8; i++) {
+                            const uint32_t r = rand_diag_column(a.gen, (uint32_t)(first + ((int64_t)i << (A + sbits))) & column_mask);
+#pragma unroll
+                            for (int k = 0; k < 8; k++) {
+                                const int at = k * (R2 / 8) + i;
+                                w[at] = __uint_as_float(__float_as_uint(w[at]) ^ nibble_negative(r, k));
+                            }
+                        }
+                        drawn = false;
+                    }
+                }
+                if (drawn) {
+#pragma unroll
+                    for (int i = 0; i < R2; i++) {
+                        const int64_t g = first + ((int64_t)i << (A + sbits));
+                        w[i] = __uint_as_float(__float_as_uint(w[i]) ^ rand_diag_negative(a.gen, (uint32_t)(g >> a.gen.bits), (uint32_t)g & column_mask));
+                    }
+                }
+                drawn = true;
+            }
+        } else if (flips && a.sign && a.sign_bits) {
+            // a row's 32 signs are one word: lane i (and R2 + i) fetches that of row i of the lower (upper) half of the wave, and
+            // the two make the lane mask of a select
+            const int lane = tid & 63;
+            const int low_row = B > 0 ? (row & ~1) + ((lane >> B) & 1) : row;
+            const int64_t at = origin + ((int64_t)(((lane & (R2 - 1)) << A) + low_row) << sbits);
+            const uint32_t word = static_cast<const uint32_t *>(a.sign)[at >> 5];
+#pragma unroll
+            for (int i = 0; i < R2; i++) {
+                const uint32_t low = (uint32_t)__builtin_amdgcn_readlane((int)word, i), high = (uint32_t)__builtin_amdgcn_readlane((int)word, R2 + i);
+                const uint64_t mask = (uint64_t)low | ((uint64_t)high << 32);
+                asm("v_cndmask_b32_e64 %0, %0, -%0, %1" : "+v"(w[i]) : "s"(mask));
+            }
+        } else if (flips && a.sign) {
+#pragma unroll
+            for (int i = 0; i < R2; i++) w[i] *= static_cast<const float *>(a.sign)[first + ((int64_t)i << (A + sbits))];
+        }
+        // on their way out: EDEN's scale, then the float store, THC's quantiser (thc_hooks.py:161-166) or a destination of
+        // another type
+        if (ENDS && e.post_scale) {
+#pragma unroll
+            for (int i = 0; i < R2; i++) w[i] *= post;
+        }
+        if (ENDS && e.out_levels) {
+            if constexpr (!kAhead) {
+#pragma unroll
+                for (int i = 0; i < R2; i++) u[i] = e.uniform[first + ((int64_t)i << (A + sbits))];
+            }
+            thc_levels(w, u, lo, delta, e.out_top);
+#pragma unroll
+            for (int i = 0; i < R2; i++) e.out_levels[first + ((int64_t)i << (A + sbits))] = (uint16_t)f32_to_bf16_bits(w[i]);
+        } else if (ENDS && e.out_dst) {
+            // rows that lie inside the destination for the whole wave need no test
+            const int last_row = __builtin_amdgcn_readfirstlane(B > 0 ? row | 1 : row);
+            const int64_t whole = ((e.out_count - 32 - origin - ((int64_t)last_row << sbits)) >> (A + sbits)) + 1;
+            const int rows = (int)min(whole, (int64_t)R2);
+            const auto store = [&](auto *out, auto convert) {
+#pragma unroll
+                for (int i = 0; i < R2; i++) {
+                    const int64_t g = first + ((int64_t)i << (A + sbits));
+                    if (i < rows)
+                        out[g] = convert(w[i]);
+                    else if (g < e.out_count)
+                        out[g] = convert(w[i]);
+                }
+            };
+            if (e.out_dtype == DQ_F32)
+                store(static_cast<float *>(e.out_dst), [](float f) { return f; });
+            else if (e.out_dtype == DQ_BF16)
+                store(static_cast<uint16_t *>(e.out_dst), [](float f) { return (uint16_t)f32_to_bf16_bits(f); });
+            else
+                store(static_cast<uint16_t *>(e.out_dst), [](float f) { return (uint16_t)f32_to_f16_bits(f); });
+        } else {
+#pragma unroll
+            for (int i = 0; i < R2; i++) x[first + ((int64_t)i << (A + sbits))] = w[i];
+        }
+    };
+    if constexpr (B > 0) {
+#pragma unroll 1
+        for (int row = group; row < R1; row += R2) {
+            float w[R2];
+#pragma unroll
+            for (int i = 0; i < R2; i++) w[i] = lds[((i << A) + row) * 32 + col];
+            butterflies<B>(w);
+            finish(w, row);
+        }
+    } else if (mine) {
+#pragma unroll
+        for (int j = 0; j < R1; j++) {
+            float w[1] = {v[j]};
+            finish(w, j);
         }
     }
 }
 
+// threads of the tile of a strided pass
+__host__ __device__ constexpr int strided_threads(int rbits) { return rbits >= 9 ? 1 << rbits : 1 << (rbits + 1); }
+
 template <bool ENDS>
-__global__ void rht_strided_kernel(float *__restrict__ x, PassArgs<ENDS> a, int rbits, int sbits, int sign_mode, int apply_scale,
-                                   TransformEnds e)
+__device__ __forceinline__ void strided_pass(float *__restrict__ x, const PassArgs<ENDS> &a, int rbits, int sbits, int sign_mode,
+                                             int apply_scale, const TransformEnds &e, unsigned block, float *lds)
+{
+    switch (rbits) {
+    case 4: strided_rows<ENDS, 4, 0>(x, a, sbits, sign_mode, apply_scale, e, block, lds); break;
+    case 5: strided_rows<ENDS, 4, 1>(x, a, sbits, sign_mode, apply_scale, e, block, lds); break;
+    case 6: strided_rows<ENDS, 4, 2>(x, a, sbits, sign_mode, apply_scale, e, block, lds); break;
+    case 7: strided_rows<ENDS, 4, 3>(x, a, sbits, sign_mode, apply_scale, e, block, lds); break;
+    default: strided_rows<ENDS, 4, 4>(x, a, sbits, sign_mode, apply_scale, e, block, lds); break;
+    }
+}
+
+template <bool ENDS>
+__global__ __launch_bounds__(512) void rht_strided_kernel(float *__restrict__ x, PassArgs<ENDS> a, int rbits, int sbits, int sign_mode,
+                                                          int apply_scale, TransformEnds e)
 {
     extern __shared__ __attribute__((aligned(16))) float lds[];
     strided_pass<ENDS>(x, a, rbits, sbits, sign_mode, apply_scale, e, blockIdx.x, lds);
+}
+
+// 512 (B = 4) or 1024 rows (B = 5)
+template <bool ENDS, int B>
+__global__ __launch_bounds__(32 << B) void rht_strided_long_kernel(float *__restrict__ x, PassArgs<ENDS> a, int sbits, int sign_mode,
+                                                                   int apply_scale, TransformEnds e)
+{
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    strided_rows<ENDS, 5, B>(x, a, sbits, sign_mode, apply_scale, e, blockIdx.x, lds);
+}
+
+template <bool ENDS>
+__global__ __launch_bounds__(1024) void rht_first_kernel(float *__restrict__ x, PassArgs<ENDS> a, int sign_mode, TransformEnds e)
+{
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    first_pass<ENDS>(x, a, sign_mode, e, blockIdx.x, lds);
 }
 
 #if DQ_RHT_PART & DQ_RHT_TRANSFORM
@@ -688,14 +951,14 @@ __device__ __forceinline__ RhtPassArgs pass_args(const TilePass &p)
 }
 
 // (the largest pass gives every workgroup its threads and LDS: smaller tiles leave some of both idle)
-__global__ void rht_tile_passes_kernel(PassSet set)
+__global__ __launch_bounds__(1024) void rht_tile_passes_kernel(PassSet set)
 {
     extern __shared__ __attribute__((aligned(16))) float lds[];
     const TilePass &p = pass_of_block(set);
-    tile_pass<true>(p.x, pass_args(p), p.sign_mode, p.apply_scale, p.ends, blockIdx.x - p.first, lds);
+    first_pass<true>(p.x, pass_args(p), p.sign_mode, p.ends, blockIdx.x - p.first, lds);
 }
 
-__global__ void rht_strided_passes_kernel(PassSet set)
+__global__ __launch_bounds__(512) void rht_strided_passes_kernel(PassSet set)
 {
     extern __shared__ __attribute__((aligned(16))) float lds[];
     const TilePass &p = pass_of_block(set);
@@ -1150,6 +1413,16 @@ hipError_t launch_rht_tile(float *x, const void *sign, int sign_bits, int64_t n,
     const unsigned threads = (unsigned)std::min(1024, tile / 16);
     const size_t lds = ((size_t)padded_tile_floats(kt) + (ends.in_planes ? 256 : 0)) * sizeof(float);
     const dim3 grid((unsigned)((n + tile - 1) >> kt));
+    if (sign_mode != 2 && !apply_scale && kb == kt && kt <= 14 && vec && (n & (tile - 1)) == 0 && ends.plain_out()) {
+        const int mode = diagonal ? sign_mode : 0;
+        const auto launch = [&](auto kernel, const auto &args) -> hipError_t {
+            const hipError_t e = allow_lds(kernel, lds);
+            if (e != hipSuccess) return e;
+            hipLaunchKernelGGL(kernel, grid, dim3(threads), lds, stream, x, args, mode, ends);
+            return hipGetLastError();
+        };
+        return plain ? launch(rht_first_kernel<false>, plain_args) : launch(rht_first_kernel<true>, a);
+    }
     if (plain) {
         hipError_t e = allow_lds(rht_tile_kernel<false>, lds);
         if (e != hipSuccess) return e;
@@ -1172,22 +1445,22 @@ hipError_t launch_rht_strided(float *x, const void *sign, int sign_bits, int64_t
     RhtPassArgs a;
     a.sign = sign; a.sign_bits = sign_bits; a.n = n; a.kt = rbits + 5; a.kb = 0; a.scale = scale; a.vec = vec; a.gen = ends.gen;
     const RhtTileArgs &plain_args = a;
-    const int tile = 1 << (rbits + 5);
-    const unsigned threads = (unsigned)std::min(1024, tile / 16);
-    const size_t lds = (size_t)padded_tile_floats(rbits + 5) * sizeof(float);
-    const dim3 grid((unsigned)(n >> (rbits + 5)));
+    const dim3 grid((unsigned)(n >> (rbits + 5))), block((unsigned)strided_threads(rbits));
+    const size_t lds = sizeof(float) << (rbits + 5);
+    const auto launch = [&](auto kernel, const auto &args, auto... bits) -> hipError_t {
+        const hipError_t e = allow_lds(kernel, lds);
+        if (e != hipSuccess) return e;
+        hipLaunchKernelGGL(kernel, grid, block, lds, stream, x, args, bits..., sign || ends.gen.bits != 0 ? sign_mode : 0, apply_scale, ends);
+        return hipGetLastError();
+    };
     if (plain) {
-        hipError_t e = allow_lds(rht_strided_kernel<false>, lds);
-        if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(rht_strided_kernel<false>, grid, dim3(threads), lds, stream, x, plain_args, rbits, sbits, sign ? sign_mode : 0,
-                           apply_scale, ends);
-    } else {
-        hipError_t e = allow_lds(rht_strided_kernel<true>, lds);
-        if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(rht_strided_kernel<true>, grid, dim3(threads), lds, stream, x, a, rbits, sbits, sign || ends.gen.bits != 0 ? sign_mode : 0,
-                           apply_scale, ends);
+        if (rbits == 10) return launch(rht_strided_long_kernel<false, 5>, plain_args, sbits);
+        if (rbits == 9) return launch(rht_strided_long_kernel<false, 4>, plain_args, sbits);
+        return launch(rht_strided_kernel<false>, plain_args, rbits, sbits);
     }
-    return hipGetLastError();
+    if (rbits == 10) return launch(rht_strided_long_kernel<true, 5>, a, sbits);
+    if (rbits == 9) return launch(rht_strided_long_kernel<true, 4>, a, sbits);
+    return launch(rht_strided_kernel<true>, a, rbits, sbits);
 }
 
 // every x 16-byte aligned, n a multiple of 2^kt and 10 <= kt <= 14
@@ -1198,7 +1471,7 @@ hipError_t launch_rht_tile_passes(const TilePass *passes, int count, hipStream_t
     unsigned blocks = 0;
     int most = 10;
     for (int k = 0; k < count; k++) {
-        if (passes[k].kt < 10 || passes[k].kt > 14 || passes[k].kb > passes[k].kt || (passes[k].n & ((1 << passes[k].kt) - 1)) != 0 || !aligned16(passes[k].x))
+        if (passes[k].kt < 10 || passes[k].kt > 14 || passes[k].kb != passes[k].kt || passes[k].sign_mode == 2 || passes[k].apply_scale || !passes[k].ends.plain_out() || (passes[k].n & ((1 << passes[k].kt) - 1)) != 0 || !aligned16(passes[k].x))
             return hipErrorInvalidValue;
         set.p[k] = passes[k];
         set.p[k].first = blocks;
@@ -1228,10 +1501,10 @@ hipError_t launch_rht_strided_passes(const TilePass *passes, int count, hipStrea
         blocks += (unsigned)(passes[k].n >> (passes[k].rbits + 5));
         most = std::max(most, passes[k].rbits);
     }
-    const size_t lds = (size_t)padded_tile_floats(most + 5) * sizeof(float);
+    const size_t lds = sizeof(float) << (most + 5);
     const hipError_t e = allow_lds(rht_strided_passes_kernel, lds);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(rht_strided_passes_kernel, dim3(blocks), dim3(1u << (most + 1)), lds, stream, set);
+    hipLaunchKernelGGL(rht_strided_passes_kernel, dim3(blocks), dim3((unsigned)strided_threads(most)), lds, stream, set);
     return hipGetLastError();
 }
 

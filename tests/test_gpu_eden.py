@@ -214,6 +214,57 @@ def test_binding_functions(eden_utils, capi):
         eden_utils.eden_quantize(x, bnd[:5].contiguous(), cen, nbits)
 
 
+@pytest.mark.parametrize("levels", [2, 64, 256])
+@pytest.mark.parametrize("n", [1 << 16, 1 << 20])
+def test_thc_levels_where_the_comparison_is_a_tie(capi, n, levels):
+    """uniform values equal to the fraction they are compared with, their neighbours, 0 and 1, and rotated values on, next to and
+    beyond the grid's ends: the levels of the folded quantiser are those of the quantiser that divides"""
+    g = torch.Generator().manual_seed(n + levels)
+    x = (torch.randn(n, generator=g) * 1e-2).to(DEV)
+    x[7] = 3.0                                                              # (a spike moves whole columns beyond the ends)
+    scale = float(np.float32(1.0) / np.float32(np.sqrt(n)))
+    rot = x.clone()
+    capi.rht_blocked(rot, None, n, scale, False)
+    hi = 1.5 * float(rot.std())
+    lo = torch.tensor([-hi], dtype=torch.float32, device=DEV)
+    delta = torch.tensor([2 * hi / (levels - 1)], dtype=torch.float32, device=DEV)
+    q = ((rot - lo) / delta).clamp(0, levels - 1)
+    frac = q - q.floor()
+    k = torch.arange(n, device=DEV) % 6
+    uni = torch.where(k == 0, frac, torch.where(k == 1, torch.nextafter(frac, torch.ones_like(frac)), torch.where(
+        k == 2, torch.nextafter(frac, -torch.ones_like(frac)).clamp(min=0), torch.where(k == 3, torch.zeros_like(frac), torch.where(
+            k == 4, torch.full_like(frac, 1 - 2.0 ** -24), 1 - frac)))))
+    for bad in (None, float("nan"), float("inf")):
+        if bad is not None:
+            rot.fill_(bad)
+            x[0] = bad
+        want, got = torch.empty(n, dtype=torch.bfloat16, device=DEV), torch.empty(n, dtype=torch.bfloat16, device=DEV)
+        work = x.clone()
+        if bad is not None:
+            rot = x.clone()
+            capi.rht_blocked(rot, None, n, scale, False)
+        capi.thc_quantize(rot, uni, want, lo, delta, levels)
+        capi.thc_rht_quantize(work, None, uni, got, n, scale, lo, delta, levels)
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16)), bad
+
+
+@pytest.mark.parametrize("bits,shift", [(14, 0), (16, 1), (17, 0), (18, 3), (21, 0), (24, 1), (26, 0), (27, 0), (30, 0)])
+def test_long_transforms_of_a_unit_vector(capi, bits, shift):
+    """H e_k = (-1)^popcount(j & k): every element of the contiguous pass and of strided passes of four to ten row bits, on vectors
+    that start anywhere"""
+    n = 1 << bits
+    k = 0x2D5B3A97 & (n - 1)
+    x = torch.zeros(n + shift, device=DEV)[shift:]
+    x[k] = 0.5
+    capi.rht_blocked(x, None, n, 2.0, False)
+    piece = 1 << min(bits, 26)
+    for at in range(0, n, piece):
+        j = torch.arange(at, at + piece, dtype=torch.int32, device=DEV) & k
+        for s in (16, 8, 4, 2, 1):
+            j ^= j >> s
+        assert torch.equal(x[at:at + piece], 1.0 - 2.0 * (j & 1).float()), at
+
+
 @pytest.mark.parametrize("n,block", [(64, 64), (1024, 1024), (1024, 64), (1 << 15, 1 << 15), (1 << 16, 1 << 16),
                                      (1 << 17, 1 << 17), (1 << 20, 1 << 20), (1 << 22, 1 << 22), (1 << 23, 1 << 23), (1 << 18, 1 << 12), (3 << 14, 1 << 14)])
 def test_thc_quantiser_folded_into_the_transform(capi, n, block):
