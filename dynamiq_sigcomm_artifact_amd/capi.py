@@ -34,7 +34,7 @@ EXPORTS = [
     "dq_superchunk_mean_center", "dq_superchunk_add_mean_copy",
     "dq_hadamard", "dq_rht_blocked", "dq_rand_diag", "dq_rand_diag_bits", "dq_rht_scaling_compress", "dq_rht_scaling_compress_mfma16", "dq_scaling_decompress_irht", "dq_pack_signs",
     "dq_bins_to_bits", "dq_bits_to_bins", "dq_quantization",
-    "dq_eden_work_doubles", "dq_eden_quantize", "dq_eden_quantize_static_max_n", "dq_eden_quantize_static", "dq_eden_dequantize", "dq_eden_dequantize_irht", "dq_eden_slice_bytes", "dq_eden_compress", "dq_eden_decompress", "dq_thc_compress", "dq_thc_decompress", "dq_thc_quantize", "dq_thc_dequantize", "dq_thc_rht_quantize", "dq_thc_dequantize_irht",
+    "dq_eden_work_doubles", "dq_eden_quantize", "dq_eden_quantize_static_max_n", "dq_eden_quantize_static", "dq_eden_dequantize", "dq_eden_dequantize_irht", "dq_eden_slice_bytes", "dq_eden_compress", "dq_eden_decompress", "dq_thc_compress", "dq_thc_compress_drawn", "dq_thc_decompress", "dq_thc_quantize", "dq_thc_dequantize", "dq_thc_rht_quantize", "dq_thc_dequantize_irht",
 ]
 
 STAGE_STATS, STAGE_PLAN, STAGE_COMPRESS, STAGE_DECOMPRESS = 1, 2, 4, 8

@@ -966,14 +966,18 @@ static int thc_ends(const dq_thc_grid_t *g, dq::TransformEnds &ends)
     return DQ_OK;
 }
 
-int dq_thc_compress(const void *src, int dtype, int64_t count, float *work, const uint32_t *sign_bits, const float *uniform,
-                    void *levels_bf16, int64_t n, float scale, const dq_thc_grid_t *grid, int levels, int device, dq_stream_t stream)
+static int thc_compress(const void *src, int dtype, int64_t count, float *work, const uint32_t *sign_bits, const float *uniform,
+                        const dq_uniform_stream_t *drawn, void *levels_bf16, int64_t n, float scale, const dq_thc_grid_t *grid, int levels,
+                        int device, dq_stream_t stream)
 {
     if (n < 1024 || (n & (n - 1)) != 0) return fail(DQ_ERR_POW2, "the dimension (at least 1024)");
     if (!(count > 0) || count > n) return fail(DQ_ERR_SIZE, "count must lie in [1, n]");
     if (levels < 2 || levels > 256) return fail(DQ_ERR_SIZE, "levels must be in [2, 256]");
     if (!dtype_ok(dtype)) return fail(DQ_ERR_DTYPE);
-    if (!src || !work || !sign_bits || !uniform || !levels_bf16) return fail(DQ_ERR_NULL);
+    if (!src || !work || !sign_bits || !(uniform || drawn) || !levels_bf16) return fail(DQ_ERR_NULL);
+    if (drawn && (n < dq::kDrawsFrom || n > dq::kDrawsTo)) return fail(DQ_ERR_SIZE, "drawn uniform values: n must lie in [2^19, 2^25]");
+    if (drawn && (drawn->threads < 1 || (drawn->threads & (drawn->threads - 1)) != 0 || drawn->threads > n || (drawn->offset & 3) != 0))
+        return fail(DQ_ERR_SIZE, "the stream's threads must be a power of two of at most n and its offset a multiple of 4");
     if ((reinterpret_cast<uintptr_t>(work) | reinterpret_cast<uintptr_t>(uniform) | reinterpret_cast<uintptr_t>(levels_bf16)) & 15)
         return fail(DQ_ERR_SIZE, "work, uniform and the levels must be 16-byte aligned");
     dq::TransformEnds ends;
@@ -984,9 +988,28 @@ int dq_thc_compress(const void *src, int dtype, int64_t count, float *work, cons
     ends.in_count = count;
     ends.out_levels = static_cast<uint16_t *>(levels_bf16);
     ends.uniform = uniform;
+    if (drawn) {
+        ends.draw.bits = dq::ilog2(drawn->threads);
+        ends.draw.seed = drawn->seed;
+        ends.draw.counter = drawn->offset / 4;
+    }
     ends.out_top = (float)(levels - 1);
     if ((rc = select_device(device))) return rc;
     return finish(dq::launch_rht_ends(work, sign_bits, true, n, n, scale, 0, ends, static_cast<hipStream_t>(stream)));
+}
+
+int dq_thc_compress(const void *src, int dtype, int64_t count, float *work, const uint32_t *sign_bits, const float *uniform,
+                    void *levels_bf16, int64_t n, float scale, const dq_thc_grid_t *grid, int levels, int device, dq_stream_t stream)
+{
+    return thc_compress(src, dtype, count, work, sign_bits, uniform, nullptr, levels_bf16, n, scale, grid, levels, device, stream);
+}
+
+int dq_thc_compress_drawn(const void *src, int dtype, int64_t count, float *work, const uint32_t *sign_bits,
+                          const dq_uniform_stream_t *drawn, void *levels_bf16, int64_t n, float scale, const dq_thc_grid_t *grid, int levels,
+                          int device, dq_stream_t stream)
+{
+    if (!drawn) return fail(DQ_ERR_NULL);
+    return thc_compress(src, dtype, count, work, sign_bits, nullptr, drawn, levels_bf16, n, scale, grid, levels, device, stream);
 }
 
 int dq_thc_decompress(const void *levels_bf16, const uint32_t *sign_bits, float *out, int64_t count, int64_t n, float scale,

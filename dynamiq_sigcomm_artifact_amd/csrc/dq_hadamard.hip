@@ -345,6 +345,8 @@ hipError_t launch_rht_ends(float *x, const void *sign, bool sign_packed, int64_t
                             reinterpret_cast<uintptr_t>(ends.out_levels) | reinterpret_cast<uintptr_t>(ends.uniform) |
                             (sign_packed ? 0 : reinterpret_cast<uintptr_t>(sign));
     if (block < 1024 || n % block != 0 || (every & 15) != 0) return hipErrorInvalidValue;
+    // (the strided pass of 256 or 1024 rows behind the first pass is the one that draws)
+    if (ends.draw.bits >= 0 && (block < kDrawsFrom || block > kDrawsTo || block != n)) return hipErrorInvalidValue;
     return fwht_blocks(x, sign, sign_packed, n, ilog2(block), scale, 1, inverse, stream, ends);
 }
 

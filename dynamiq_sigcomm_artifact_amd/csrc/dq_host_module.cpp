@@ -11,11 +11,13 @@
 #include <c10/hip/HIPStream.h>
 #include <pybind11/pybind11.h>
 #include <torch/csrc/DynamicTypes.h>
+#include <torch/csrc/Generator.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <string.h>
 
 #include <algorithm>
+#include <mutex>
 #include <stdexcept>
 #include <string>
 #include <vector>
@@ -807,6 +809,44 @@ py::object thc_compress(py::handle src, int64_t count, py::handle work, py::hand
     return py::reinterpret_steal<py::object>(THPVariable_Wrap(out));
 }
 
+// thc_compress with the uniform values that generator.uniform_() would fill a vector with, drawn in the kernel: the generator is
+// moved on as that call moves it.  None where it cannot be: a generator of another device, a stream that records (torch
+// keeps the generator's state on the device then), a GPU whose resident threads are no power of two, a length that the kernel does
+// not draw for.
+py::object thc_compress_drawn(py::handle src, int64_t count, py::handle work, py::handle bits, py::handle generator, double scale,
+                              py::handle norm, py::tuple numbers, int levels)
+{
+    Args a;
+    const at::Tensor &x = a.tensor(src), &w = a.tensor(work);
+    const int64_t n = w.numel();
+    if (x.numel() < count || w.scalar_type() != at::kFloat) refuse("thc_compress: a buffer is too small or of the wrong dtype");
+    const uint32_t *sign = reinterpret_cast<const uint32_t *>(a.typed(bits, at::kInt, n / 32, "sign").data_ptr<int32_t>());
+    const dq_thc_grid_t g = thc_grid(a, norm, numbers);
+    if (!THPGenerator_Check(generator.ptr())) return py::none();
+    at::Generator gen = reinterpret_cast<THPGenerator *>(generator.ptr())->cdata;
+    if (!gen.device().is_cuda() || gen.device().index() != a.device || n < (1 << 19) || n > (1 << 25)) return py::none();
+    const hipStream_t stream = c10::hip::getCurrentHIPStream().stream();
+    unsigned long long id = 0;
+    if (Buckets::capturing(stream, &id)) return py::none();
+    int cus = 0, per_cu = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, a.device) != hipSuccess ||
+        hipDeviceGetAttribute(&per_cu, hipDeviceAttributeMaxThreadsPerMultiProcessor, a.device) != hipSuccess)
+        return py::none();
+    dq_uniform_stream_t drawn;
+    drawn.threads = std::min((int64_t)cus * (per_cu / 256), (n + 255) / 256) * 256;
+    if (drawn.threads <= 0 || (drawn.threads & (drawn.threads - 1)) != 0) return py::none();
+    at::Tensor out = empty_on(a.device, n, at::kBFloat16);
+    {
+        const std::lock_guard<std::mutex> lock(gen.mutex());
+        drawn.seed = gen.current_seed();
+        drawn.offset = gen.get_offset();
+        gen.set_offset(drawn.offset + 4 * ((uint64_t)((n - 1) / (4 * drawn.threads)) + 1));
+    }
+    check(dq_thc_compress_drawn(x.data_ptr(), dtype_code(x), count, w.data_ptr<float>(), sign, &drawn, out.data_ptr(), n, (float)scale, &g, levels,
+                                a.device, stream));
+    return py::reinterpret_steal<py::object>(THPVariable_Wrap(out));
+}
+
 void thc_decompress(py::handle levels, py::handle bits, py::handle out, int64_t count, double scale, py::handle norm, py::tuple numbers)
 {
     Args a;
@@ -1020,6 +1060,7 @@ PYBIND11_MODULE(_host, m)
     m.def("eden_compress", &eden_compress);
     m.def("eden_decompress", &eden_decompress);
     m.def("thc_compress", &thc_compress);
+    m.def("thc_compress_drawn", &thc_compress_drawn);
     m.def("thc_decompress", &thc_decompress);
     m.doc() = "native host path of dynamiq_sigcomm_artifact_amd";
     py::class_<Buckets>(m, "Buckets")

@@ -178,6 +178,13 @@ struct SignSeed {
 };
 SignSeed sign_seed(int64_t size, int64_t seed);
 
+// Uniform values drawn where they are compared (dq_uniform_stream_t); bits: log2 of the stream's threads, negative: none
+constexpr int64_t kDrawsFrom = (int64_t)1 << 19, kDrawsTo = (int64_t)1 << 25; // transforms that may
+struct UniformDraw {
+    int bits = -1;
+    uint64_t seed = 0, counter = 0;
+};
+
 // Quantisers folded into the two ends of a transform (all null: the plain transform).  `in_*` replace the load of the
 // first pass, `out_*` / `post_scale` act on the store of the last one.
 struct TransformEnds {
@@ -204,6 +211,7 @@ struct TransformEnds {
     uint16_t *out_levels = nullptr;
     const float *uniform = nullptr, *out_lo = nullptr, *out_delta = nullptr;
     float out_top = 0.0f;
+    UniformDraw draw; // instead of uniform: transforms of 2^19 .. 2^25 elements
     // EDEN: the pass loads centroids[bin] from the bit planes of the bins; the last pass multiplies by *post_scale
     const uint32_t *in_planes = nullptr;
     const float *in_centroids = nullptr;

@@ -723,6 +723,53 @@ __global__ void rht_tile_kernel(float *__restrict__ x, PassArgs<ENDS> a, int sig
     tile_pass<ENDS>(x, a, sign_mode, apply_scale, e, blockIdx.x, lds);
 }
 
+// Uniform values of a stream as torch's generator hands them to the threads of a kernel: thread k of 2^bits takes the blocks
+// counter, counter + 1, ... of subsequence k, and the four words of a block go to elements 2^bits apart.  u[i] is that of element
+// first + i 2^shift.  The bits of i from P on are the number of the word in its block (where they lie outside i, its bits are those
+// of first): one block serves up to four of the elements.  Drawn here while the elements are on their way, they need neither the
+// launch that writes them nor its 33 MB there and back: THC's compress of a 25 MB bucket 46 -> 27 us.
+template <int B, int P>
+__device__ __forceinline__ void draw_rows(float (&u)[1 << B], const UniformDraw &d, int64_t first, int shift)
+{
+    constexpr int kLow = P >= 0 && P < B ? 1 << P : 0, kHigh = P + 1 >= 0 && P + 1 < B ? 1 << (P + 1) : 0;
+#pragma unroll
+    for (int i = 0; i < (1 << B); i++) {
+        if (i & (kLow | kHigh)) continue;
+        const int64_t g = first + ((int64_t)i << shift);
+        const uint32_t at = (uint32_t)(g >> d.bits);
+        const uint64_t counter = d.counter + (at >> 2);
+        uint32_t w[4] = {(uint32_t)counter, (uint32_t)(counter >> 32), (uint32_t)g & ((1u << d.bits) - 1u), 0u};
+        philox4x32_10(w, (uint32_t)d.seed, (uint32_t)(d.seed >> 32));
+        if (!kLow) {
+            w[0] = (at & 1) ? w[1] : w[0];
+            w[2] = (at & 1) ? w[3] : w[2];
+        }
+        if (!kHigh) {
+            w[0] = (at & 2) ? w[2] : w[0];
+            w[1] = (at & 2) ? w[3] : w[1];
+        }
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            if ((!kLow && (k & 1)) || (!kHigh && (k & 2))) continue;
+            // (0, 1] with 1 replaced by 0
+            const float f = __builtin_fmaf((float)w[k], 0x1p-32f, 0x1p-32f);
+            u[i | (k & 1 ? kLow : 0) | (k & 2 ? kHigh : 0)] = f == 1.0f ? 0.0f : f;
+        }
+    }
+}
+
+template <int B> __device__ __forceinline__ void draw_rows(float (&u)[1 << B], const UniformDraw &d, int64_t first, int shift)
+{
+    switch (d.bits - shift) {
+    case -1: draw_rows<B, -1>(u, d, first, shift); break;
+    case 0: draw_rows<B, 0>(u, d, first, shift); break;
+    case 1: draw_rows<B, 1>(u, d, first, shift); break;
+    case 2: draw_rows<B, 2>(u, d, first, shift); break;
+    case 3: draw_rows<B, 3>(u, d, first, shift); break;
+    default: draw_rows<B, B>(u, d, first, shift); break;
+    }
+}
+
 // A later pass of a transform longer than one tile: index bits [sbits, sbits + A + B) of the vector.  A tile is 2^(A + B)
 // rows of 32 consecutive floats (128 bytes), row stride 2^sbits elements.  A thread owns column tid % 32 of 2^A consecutive
 // rows: it loads them (every load instruction of a wave covers two whole 128-byte row segments), does the A lowest row
@@ -751,19 +798,26 @@ __device__ __forceinline__ void strided_rows(float *__restrict__ x, const PassAr
         const float *from = x + origin + ((int64_t)(group << A) << sbits) + col;
 #pragma unroll
         for (int j = 0; j < R1; j++) v[j] = from[(int64_t)j << sbits];
-        butterflies<A>(v);
     }
-    // THC's uniform values are on their way while the stages run, where one workgroup has a CU to itself (1024 rows; with 256 they
-    // gain nothing)
-    constexpr bool kAhead = ENDS && A == 5 && B == 5;
+    // THC's uniform values are drawn while the elements are on their way; or they are on their way while the stages run, where one
+    // workgroup has a CU to itself (1024 rows; with 256 that gains nothing)
+    constexpr bool kDraws = ENDS && A == B, kAhead = kDraws && A == 5;
     float u[R2];
-    if constexpr (kAhead) {
+    bool have_u = false;
+    if constexpr (kDraws) {
         if (e.out_levels && mine) {
-            const float *from = e.uniform + origin + ((int64_t)group << sbits) + col;
+            const int64_t at = origin + ((int64_t)group << sbits) + col;
+            if (e.draw.bits >= 0) {
+                draw_rows<B>(u, e.draw, at, A + sbits);
+                have_u = true;
+            } else if (kAhead) {
 #pragma unroll
-            for (int i = 0; i < R2; i++) u[i] = from[(int64_t)i << (A + sbits)];
+                for (int i = 0; i < R2; i++) u[i] = e.uniform[at + ((int64_t)i << (A + sbits))];
+                have_u = true;
+            }
         }
     }
+    if (mine) butterflies<A>(v);
     float post = 1.0f, lo = 0.0f, delta = 1.0f;
     if (ENDS && e.post_scale) post = *e.post_scale;
     if (ENDS && e.out_levels) grid_of(e.grid, e.out_lo, e.out_delta, lo, delta);
@@ -836,7 +890,7 @@ __device__ __forceinline__ void strided_rows(float *__restrict__ x, const PassAr
             for (int i = 0; i < R2; i++) w[i] *= post;
         }
         if (ENDS && e.out_levels) {
-            if constexpr (!kAhead) {
+            if (!have_u) {
 #pragma unroll
                 for (int i = 0; i < R2; i++) u[i] = e.uniform[first + ((int64_t)i << (A + sbits))];
             }
@@ -1442,6 +1496,7 @@ hipError_t launch_rht_strided(float *x, const void *sign, int sign_bits, int64_t
     if (rbits < 4 || rbits > 10 || sbits < 5 || (n & (((int64_t)1 << (sbits + rbits)) - 1)) != 0) return hipErrorInvalidValue;
     const bool plain = ends.plain_out() && ends.gen.bits == 0;
     if (!plain && !vec) return hipErrorInvalidValue;
+    if (ends.out_levels && ends.draw.bits >= 0 && rbits != 8 && rbits != 10) return hipErrorInvalidValue;
     RhtPassArgs a;
     a.sign = sign; a.sign_bits = sign_bits; a.n = n; a.kt = rbits + 5; a.kb = 0; a.scale = scale; a.vec = vec; a.gen = ends.gen;
     const RhtTileArgs &plain_args = a;

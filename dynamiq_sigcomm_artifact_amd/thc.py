@@ -24,6 +24,7 @@ import torch
 from . import capi
 
 _READ = {torch.float32, torch.bfloat16, torch.float16}         # what the transform's first pass reads itself
+_DRAWN = (1 << 19, 1 << 25)                                     # dimensions whose uniform values the last pass draws itself
 _TABLE_FILE = "{table_size}_tablesize_{max_val}_maxval_16_qlevels_{overflow_frequency}_ofreq_data.txt"
 _TABLE_DEFAULTS = {"table_size": 10001, "max_val": 42, "overflow_frequency": 1024}
 
@@ -118,6 +119,9 @@ class OldINCACudaHadamardCompressor:
             buf = self._scratch[(name, role)] = torch.empty(dim, dtype=torch.float32, device=self.device)
         return buf
 
+    def _uniform(self, name):
+        return self._buffer(name, "uniform").uniform_(0.0, 1.0, generator=self.sender_prng)
+
     def _grid(self, max_norm, dim):
         """(lowest level, level spacing) as float32 device scalars of shape [1]; the arithmetic and its order are the
         reference's (thc_hooks.py:143-147), done on max_norm's own type"""
@@ -147,18 +151,27 @@ class OldINCACudaHadamardCompressor:
         dim, used = self.ds[name], self.original_size[name]
         self.max_norm_dict[name] = max_norm
         work = self._buffer(name, "work")
-        if uniform is None:
-            uniform = self._buffer(name, "uniform").uniform_(0.0, 1.0, generator=self.sender_prng)
         rot = self.hadamards[name]
-        grid = self._native_grid(max_norm, dim) if dim >= 1024 and uniform.data_ptr() % 16 == 0 else None
+        grid = self._native_grid(max_norm, dim) if dim >= 1024 and (uniform is None or uniform.data_ptr() % 16 == 0) else None
         if grid is not None:
             # the transform's first pass reads the caller's tensor, in its own type where the kernels know it
             if tensor.dim() != 1 or tensor.numel() != used or not tensor.is_cuda or not tensor.is_contiguous() or \
                     tensor.dtype not in _READ:
                 work[:used].copy_(tensor.float())
                 tensor = work
+            levels = None
+            if uniform is None and _DRAWN[0] <= dim <= _DRAWN[1]:
+                # the values that uniform_ would draw, drawn by the pass that compares them
+                levels = capi.host().thc_compress_drawn(tensor, used, work, rot.diagonal_bits, self.sender_prng, rot.inv_sqrt, grid[0],
+                                                        grid[1], self.quantization_levels)
+            if levels is not None:
+                return levels
+            if uniform is None:
+                uniform = self._uniform(name)
             return capi.host().thc_compress(tensor, used, work, rot.diagonal_bits, uniform, rot.inv_sqrt, grid[0], grid[1],
                                             self.quantization_levels)
+        if uniform is None:
+            uniform = self._uniform(name)
         work[:used].copy_(tensor.float())
         if dim > used:
             work[used:].zero_()

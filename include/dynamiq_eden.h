@@ -597,6 +597,23 @@ typedef struct dq_thc_grid {
 int dq_thc_compress(const void *src, int dtype, int64_t count, float *work, const uint32_t *sign_bits, const float *uniform,
                     void *levels_bf16, int64_t n, float scale, const dq_thc_grid_t *grid, int levels, int device,
                     dq_stream_t stream);
+
+/* The uniform values of dq_thc_compress drawn in its last pass instead of read:
+ * Philox4x32-10 with key `seed`, thread k of `threads` (a power of two) taking
+ * the blocks offset / 4, offset / 4 + 1, ... of subsequence k (counter words 2, 3)
+ * and the four words of its b-th block going to elements k + threads * (4 b + j);
+ * a word w is the value (w + 1) 2^-32 in binary32, 1 replaced by 0.  That is what
+ * torch's uniform_ over (0, 1) fills a float32 vector with, `seed` and `offset`
+ * being the generator's and `threads` those of its kernel: at most 256-thread
+ * blocks that fit the GPU at once.  n = 2^19 .. 2^25. */
+typedef struct dq_uniform_stream {
+    uint64_t seed, offset;
+    int64_t threads;
+} dq_uniform_stream_t;
+
+int dq_thc_compress_drawn(const void *src, int dtype, int64_t count, float *work, const uint32_t *sign_bits,
+                          const dq_uniform_stream_t *drawn, void *levels_bf16, int64_t n, float scale,
+                          const dq_thc_grid_t *grid, int levels, int device, dq_stream_t stream);
 int dq_thc_decompress(const void *levels_bf16, const uint32_t *sign_bits, float *out, int64_t count, int64_t n, float scale,
                       const dq_thc_grid_t *grid, int device, dq_stream_t stream);
 

@@ -248,6 +248,50 @@ def test_thc_levels_where_the_comparison_is_a_tie(capi, n, levels):
         assert torch.equal(got.view(torch.int16), want.view(torch.int16)), bad
 
 
+@pytest.mark.parametrize("dim", [1 << k for k in range(18, 27)])
+def test_thc_draws_what_torch_would_draw(dim):
+    """compress without uniform values: the levels are those of values that uniform_ drew from a generator in the same state, call
+    after call, and the generator ends where uniform_ leaves it; lengths on either side of those that the kernel draws for"""
+    from dynamiq_sigcomm_artifact_amd.thc import OldINCACudaHadamardCompressor
+    key, used = (0, 0), dim - 77
+    params = {"d": {key: dim}, "size": {key: used}, "seed": 42, "T": 3.0, "device": DEV, "quantization_levels": 64, "nclients": 4, "rank": 1}
+    a, b = OldINCACudaHadamardCompressor(params), OldINCACudaHadamardCompressor(params)
+    for codec in (a, b):                                        # (a seed and an offset with high words)
+        codec.sender_prng.manual_seed(0x1234567890ABCDEF)
+        codec.sender_prng.set_offset((1 << 34) - 4)
+    x = torch.randn(used, generator=torch.Generator(device=DEV).manual_seed(dim), device=DEV)
+    norm = x.norm()
+    for _ in range(3):
+        got = a.compress(x, key, norm)
+        uni = torch.empty(dim, device=DEV).uniform_(0.0, 1.0, generator=b.sender_prng)
+        want = b.compress(x, key, norm, uniform=uni)
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+        assert a.sender_prng.get_offset() == b.sender_prng.get_offset()
+        assert torch.equal(a.sender_prng.get_state(), b.sender_prng.get_state())
+
+
+def test_thc_recorded_draws_are_torchs():
+    """a graph that holds a compress call draws through the generator's registered state: every replay other values, those of an
+    eager call from the same state"""
+    from dynamiq_sigcomm_artifact_amd.thc import OldINCACudaHadamardCompressor
+    key, dim = (0, 0), 1 << 20
+    params = {"d": {key: dim}, "size": {key: dim}, "seed": 42, "T": 3.0, "device": DEV, "quantization_levels": 64, "nclients": 4, "rank": 0}
+    a, b = OldINCACudaHadamardCompressor(params), OldINCACudaHadamardCompressor(params)
+    x = torch.randn(dim, generator=torch.Generator(device=DEV).manual_seed(1), device=DEV)
+    norm = x.norm()
+    a.compress(x, key, norm)
+    b.compress(x, key, norm)
+    graph = torch.cuda.CUDAGraph()
+    graph.register_generator_state(a.sender_prng)
+    with torch.cuda.graph(graph):
+        got = a.compress(x, key, norm)
+    for _ in range(3):
+        graph.replay()
+        want = b.compress(x, key, norm)
+        torch.cuda.synchronize()
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
 @pytest.mark.parametrize("bits,shift", [(14, 0), (16, 1), (17, 0), (18, 3), (21, 0), (24, 1), (26, 0), (27, 0), (30, 0)])
 def test_long_transforms_of_a_unit_vector(capi, bits, shift):
     """H e_k = (-1)^popcount(j & k): every element of the contiguous pass and of strided passes of four to ten row bits, on vectors
