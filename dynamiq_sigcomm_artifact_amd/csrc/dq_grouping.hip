@@ -667,37 +667,45 @@ __global__ __launch_bounds__(kThreads) void plan_place_stats_kernel(WidthsFromSt
 // `top` entries of sorted are the 8-bit group, the last `bottom` the 2-bit group, the rest the 4-bit group, each **in
 // sorted order**.  The norms are bf16 values, so the sort key has 16 bits and the position of superchunk i is
 //     G(key_i) + E(i),   G = superchunks with a key that sorts earlier,   E = superchunks j < i with the same key
-// -- a counting sort.  As in plan_one_kernel no workgroup waits for another: the workgroup of tile b (256
-// superchunks) counts the keys of the whole bucket itself, in an LDS histogram (128 KB, 144 KB with its padding),
-// in two steps: first the superchunks before its tile (the counter of key_i is then the part of E(i) that lies in
-// earlier tiles), then the rest; an in-place exclusive scan of the histogram gives G.  In between the tile's own four
-// waves take turns: a wave reads its counters and adds its keys, and inside a wave the lanes with the same key find one
-// another by a ballot per bit of the key.  (Comparing all 256 keys of the tile with each other, as first written: 12.4 us
-// instead of 11.0 for 25,600 superchunks.)  nsc <= 65535, so no counter overflows.
+// -- a counting sort.  As in plan_one_kernel no workgroup waits for another: the workgroup of a tile counts the keys of
+// the whole bucket itself, in an LDS histogram, from pairs that it loads once and keeps in registers; an exclusive scan
+// turns the histogram into G, and E is what the tile's keys found counted before the tile plus the equal keys before them
+// inside it (a ballot per bit of the key).  nsc <= 65535, so 16 bits hold every count.
 //
 // Sort key (ascending key = descending norm, as torch.sort orders floats): NaN (either sign) first, then +inf ...
 // +0 = -0 ... -inf.
+//
+// What bounds it is the issue rate of the one CU that handles all keys of the bucket, and the chain of a load, three
+// reductions over the workgroup and a store.  Sums of squares are not negative, so normally ONE pass counts, into words
+// that hold two counts: a superchunk before the tile adds 0x10001, any other 1.  The high half ends as the superchunks
+// with the key before the tile (E's share), the low half as all of them, which the scan replaces by G.  Which of three layouts is decided
+// by the greatest and the least pattern of the bucket:
+//   short   no NaN, no sign bit, and the patterns other than +0 lie within kShortKeys - 64 of one another (63 octaves of
+//           the norm, more than 9 decades of the gradients' size): a counter for every pattern between them.  Clearing
+//           and scanning 32 KB instead of 144 is what this saves.
+//   long    no sign bit except on NaNs: a counter for every pattern
+//   signed  two 16-bit counters per word, so two steps: the superchunks before the tile, whose counts the tile's waves
+//           read in turns, each adding its own, then the rest
+// A superchunk of zeros (+0, of which a bucket may hold many, and atomics on one word take turns) counts in one of 64
+// counters at the end of the keys, its lane's; the reader adds them.  Lanes beyond the bucket's end count as zeros
+// behind all others, which moves nobody, so the loads and the counting have neither a branch nor a mask: taken branches
+// in code that runs once cost more (1.3 us for 25,600 superchunks) than what they skip.
+// Norms of 7 layers with scales e^-9 .. e^-3, us, with every pattern counted in one 144 KB histogram in two steps and in
+// the short layout: 256 superchunks 8.0 -> 4.9, 4,096 8.5 -> 5.1, 25,600 9.8 -> 6.1, 32,768 10.3 -> 6.9, 65,535
+// 20.1 -> 13.1; one in four of them zero, 25,600: 12.7 -> 5.5.  The long layout, 25,600: 9.4 -> 7.4.
 constexpr int kSortThreads = 1024;
-constexpr int kSortTile = 256;
-constexpr int kSortWords = 32768;                          // words of the histogram
+constexpr int kSortWords = 32768;                          // counters of the long layout, words of the signed one
 constexpr int kSortLdsWords = kSortWords + kSortWords / 8; // stored with 4 words of padding after every 32
-constexpr int kSortBatch = 32;                             // loads in flight per thread: 32768 superchunks in one round trip
+constexpr int kShortKeys = 8 * kSortThreads;
+static_assert(kSortThreads / 64 == 16, "a row of 16 lanes holds a value of every wave");
 
-// Word w of the histogram lives at w + 4 (w / 32): in the scan thread t owns the 32 words [32 t, 32 t + 32), and with a
-// lane stride of 36 words instead of 32 the 16-byte accesses of neighbouring lanes fall into different banks (unpadded,
-// all lanes of a wave hit the same four banks).
+// Word w of the long and signed histograms lives at w + 4 (w / 32): in the scan thread t owns the 32 words
+// [32 t, 32 t + 32), and with a lane stride of 36 words instead of 32 the 16-byte accesses of neighbouring lanes fall
+// into different banks (unpadded, all lanes of a wave hit the same four banks).
 __device__ __forceinline__ int hist_slot(uint32_t word) { return (int)(word + ((word >> 5) << 2)); }
 
-// Two layouts.  Sums of squares are not negative, so normally every pattern is one of 0 .. 0x7f80 or a NaN: then a key
-// takes 15 bits, NaN -> 0, +inf -> 1, ..., +0 -> 0x7f81, and every counter has a word of its own (narrow).  A bucket that
-// holds a negative pattern (-0 included) takes the general key, 16 bits, with two 16-bit counters per word (wide); its
-// counting and its scan cost about twice the narrow ones.
-__device__ __forceinline__ uint32_t narrow_key(uint32_t pattern)
-{
-    return pattern <= (uint32_t)kMaxPattern ? (uint32_t)kMaxPattern + 1u - pattern : 0u; // NaN (sign bit clear) -> 0
-}
-
-__device__ __forceinline__ uint32_t wide_key(uint32_t pattern)
+// the key of the signed layout, 16 bits
+__device__ __forceinline__ uint32_t signed_key(uint32_t pattern)
 {
     const uint32_t mag = pattern & 0x7fffu;
     if (mag > (uint32_t)kMaxPattern) return 0u;             // NaN
@@ -705,184 +713,279 @@ __device__ __forceinline__ uint32_t wide_key(uint32_t pattern)
     return 0x7fffu - mag;                                   // +inf -> 0x7f, +0 -> 0x7fff
 }
 
-template <bool WIDE> __device__ __forceinline__ uint32_t sort_key(uint32_t pattern) { return WIDE ? wide_key(pattern) : narrow_key(pattern); }
-
-template <bool WIDE> __device__ __forceinline__ void count_one(uint32_t *hist, uint32_t pattern)
+// the largest of the wave's values, in lane 63
+__device__ __forceinline__ uint32_t wave_max_upward(uint32_t x)
 {
-    const uint32_t k = sort_key<WIDE>(pattern);
-    if (WIDE)
-        atomicAdd(&hist[hist_slot(k >> 1)], 1u << (16 * (k & 1)));
-    else
-        atomicAdd(&hist[hist_slot(k)], 1u);
+    x = max(x, dpp_from<0x111, 0xf>(x)); // row_shr:1, 2, 4, 8
+    x = max(x, dpp_from<0x112, 0xf>(x));
+    x = max(x, dpp_from<0x114, 0xf>(x));
+    x = max(x, dpp_from<0x118, 0xf>(x));
+    x = max(x, dpp_from<0x142, 0xa>(x)); // row_bcast:15 into rows 1 and 3
+    return max(x, dpp_from<0x143, 0xc>(x)); // row_bcast:31 into rows 2 and 3
 }
 
-template <bool WIDE> __device__ __forceinline__ int counter_of(const uint32_t *hist, uint32_t k)
+// the sum over a row of 16 lanes, in every lane
+__device__ __forceinline__ uint32_t row_sum(uint32_t x)
 {
-    return WIDE ? (int)((hist[hist_slot(k >> 1)] >> (16 * (k & 1))) & 0xffffu) : (int)hist[hist_slot(k)];
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0xB1, 0xf, 0xf, true);  // quad_perm [1,0,3,2]
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x4E, 0xf, 0xf, true);  // quad_perm [2,3,0,1]
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x141, 0xf, 0xf, true); // row_half_mirror
+    return x + (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x140, 0xf, 0xf, true); // row_mirror
 }
 
-// adds the keys of the superchunks [begin, end) to the histogram; cached: the (mean, norm) pairs of the first
-// kSortBatch * kSortThreads superchunks, already in registers (pair j of thread t = superchunk j * kSortThreads + t)
-template <bool WIDE>
-__device__ __forceinline__ void count_keys(const uint32_t *__restrict__ pairs, int begin, int end, uint32_t *hist,
-                                           const uint32_t (&cached)[kSortBatch])
+// where superchunk `own` of sorted position pos goes
+__device__ __forceinline__ void place_sorted(int pos, int own, int nsc, int top, int bottom, int64_t *__restrict__ qbits_out,
+                                             int32_t *__restrict__ order)
 {
+    const int mid_end = nsc - bottom;
+    int region, at;
+    if (pos < top) region = 0, at = pos;
+    else if (pos < mid_end) region = 1, at = pos - top;
+    else region = 2, at = pos - mid_end;
+    order[(int64_t)region * nsc + at] = own;
+    if (qbits_out) qbits_out[own] = region == 0 ? 8 : (region == 1 ? 4 : 2);
+}
+
+// lanes of the wave whose value has the NBITS bits of `key`
+template <int NBITS> __device__ __forceinline__ uint64_t lanes_with(uint32_t value, uint32_t key)
+{
+    uint32_t low = ~0u, high = ~0u;
 #pragma unroll
-    for (int j = 0; j < kSortBatch; j++) {
-        const int i = j * kSortThreads + (int)threadIdx.x;
-        if (i >= begin && i < end) count_one<WIDE>(hist, cached[j] >> 16);
+    for (int bit = 0; bit < NBITS; bit++) {
+        const uint64_t with = __builtin_amdgcn_ballot_w64((value >> bit) & 1u);
+        const uint32_t mine = (uint32_t)((int32_t)(key << (31 - bit)) >> 31); // all ones if the bit is set
+        low &= ~((uint32_t)with ^ mine);
+        high &= ~((uint32_t)(with >> 32) ^ mine);
     }
-    for (int i0 = max(begin, kSortBatch * kSortThreads) / (kSortBatch * kSortThreads) * (kSortBatch * kSortThreads); i0 < end;
-         i0 += kSortBatch * kSortThreads) {
-        uint32_t raw[kSortBatch];
-#pragma unroll
-        for (int j = 0; j < kSortBatch; j++) {
-            const int i = i0 + j * kSortThreads + (int)threadIdx.x;
-            if (i >= begin && i < end) raw[j] = pairs[i];
-        }
-#pragma unroll
-        for (int j = 0; j < kSortBatch; j++) {
-            const int i = i0 + j * kSortThreads + (int)threadIdx.x;
-            if (i >= begin && i < end) count_one<WIDE>(hist, raw[j] >> 16);
-        }
+    return ((uint64_t)high << 32) | low;
+}
+
+// the pairs of waves of a tile whose keys are compared, one pair per wave of the workgroup: first a wave with itself
+template <int WAVES> constexpr int kTilePairs = WAVES * (WAVES + 1) / 2;
+
+template <int WAVES> __device__ __forceinline__ void tile_pair(int wave, int &row, int &col)
+{
+    row = col = wave;
+    if (wave >= WAVES) {
+        col = wave - WAVES;
+        for (row = 1; col >= row; row++) col -= row;
     }
 }
 
-// exclusive scan of the counters in place; thread t owns the words [32 t, 32 t + 32)
-template <bool WIDE> __device__ __forceinline__ void scan_counters(uint32_t *hist, uint32_t *wave_sum)
+// The short and the long layout.  key = first - pattern for the patterns from `first` down, 0 above (NaN); +0 has the
+// key `last`, the one behind those of all other patterns present.
+template <bool LONG, int TILE, int BATCH>
+__device__ __forceinline__ void sorted_plan_once(int nsc, int top, int bottom, int64_t *__restrict__ qbits_out,
+                                                 int32_t *__restrict__ order, const uint32_t (&cached)[BATCH],
+                                                 uint32_t row_pair, uint32_t col_pair, uint32_t first, uint32_t last,
+                                                 uint32_t *hist, uint32_t *wave_sum, uint32_t *rank)
 {
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    uint4 *mine = reinterpret_cast<uint4 *>(hist + 36 * t); // hist_slot(32 t)
-    uint4 v[8];
-    uint32_t sum = 0;
+    static_assert((uint32_t)kMaxPattern + 1u + 64u <= (uint32_t)kSortWords, "the counters of +0 fit behind the keys");
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int nbefore = (int)blockIdx.x * TILE;
+    const uint32_t base = (first << 16) | 0xffffu; // (base - pair) >> 16 = first - pattern
+    const auto key_of = [&](uint32_t pair, uint32_t end) -> uint32_t {
+        if constexpr (LONG) return pair >> 16 ? __builtin_elementwise_sub_sat(base, pair) >> 16 : end;
+        return min((base - pair) >> 16, end); // (every pattern is at most `first`, +0 comes out at least `end`)
+    };
+    const auto slot = [](uint32_t key) { return LONG ? hist_slot(key) : (int)key; };
+    // (behind the last superchunk a prefix may be 65,536)
+    const auto with_low = [](uint32_t counter, uint32_t prefix) { return (counter & 0xffff0000u) | (prefix & 0xffffu); };
+    const uint32_t end = last + lane;
 #pragma unroll
-    for (int q = 0; q < 8; q++) {
-        v[q] = mine[q];
-        const uint32_t w[4] = {v[q].x, v[q].y, v[q].z, v[q].w};
-#pragma unroll
-        for (int h = 0; h < 4; h++) sum += WIDE ? (w[h] & 0xffffu) + (w[h] >> 16) : w[h];
+    for (int j = 0; j < BATCH; j++) {
+        const int i0 = j * kSortThreads + wave * 64;
+        const uint32_t one = i0 < nbefore ? 0x10001u : 1u;
+        atomicAdd(&hist[slot(key_of(cached[j], end))], one);
     }
-    const uint32_t incl = wave_scan_inclusive(sum);
-    if (lane == 63) wave_sum[wave] = incl;
+    // superchunks of the tile before this one with the same key
+    constexpr int kWaves = TILE / 64;
+    const uint32_t key = key_of(row_pair, last); // of the first kWaves waves, their superchunk's
+    if (wave < kTilePairs<kWaves>) {
+        int row, col;
+        tile_pair<kWaves>(wave, row, col);
+        uint64_t same = lanes_with<LONG ? 15 : 13>(key_of(col_pair, last), key); // (`col` is full if `row` has superchunks)
+        if (row == col) same &= ((uint64_t)1 << lane) - 1u;
+        atomicAdd(&rank[row * 64 + lane], (uint32_t)__popcll(same));
+    }
     __syncthreads();
-    uint32_t run = incl - sum;
-    for (int k = 0; k < wave; k++) run += wave_sum[k];
+    if constexpr (LONG) {
+        // thread t scans the counters [32 t, 32 t + 32)
+        uint4 *mine = reinterpret_cast<uint4 *>(hist + 36 * t); // hist_slot(32 t)
+        uint4 v[8];
+        uint32_t sum = 0;
 #pragma unroll
-    for (int q = 0; q < 8; q++) {
-        uint32_t w[4] = {v[q].x, v[q].y, v[q].z, v[q].w};
-#pragma unroll
-        for (int h = 0; h < 4; h++) {
-            if (WIDE) {
-                const uint32_t lo = w[h] & 0xffffu, hi = w[h] >> 16;
-                w[h] = (run & 0xffffu) | ((run + lo) << 16); // an exclusive prefix is at most nsc - 1 < 65536
-                run += lo + hi;
-            } else {
-                const uint32_t c = w[h];
-                w[h] = run;
-                run += c;
-            }
+        for (int q = 0; q < 8; q++) {
+            v[q] = mine[q];
+            sum += (v[q].x & 0xffffu) + (v[q].y & 0xffffu) + (v[q].z & 0xffffu) + (v[q].w & 0xffffu);
         }
-        mine[q] = make_uint4(w[0], w[1], w[2], w[3]);
+        const uint32_t incl = wave_scan_inclusive(sum);
+        if (lane == 63) wave_sum[wave] = incl;
+        __syncthreads();
+        uint32_t run = row_sum((lane & 15) < wave ? wave_sum[lane & 15] : 0u) + incl - sum;
+#pragma unroll
+        for (int q = 0; q < 8; q++) {
+            const uint32_t x = run, y = x + (v[q].x & 0xffffu), z = y + (v[q].y & 0xffffu), w = z + (v[q].z & 0xffffu);
+            run = w + (v[q].w & 0xffffu);
+            mine[q] = make_uint4(with_low(v[q].x, x), with_low(v[q].y, y), with_low(v[q].z, z), with_low(v[q].w, w));
+        }
+    } else {
+        // thread t scans the counters [4 t, 4 t + 4) and as many from 4 kSortThreads + 4 t on; no sum exceeds 65,535, so
+        // those of the two parts share a word
+        static_assert(kShortKeys == 8 * kSortThreads, "two parts");
+        uint4 *mine = reinterpret_cast<uint4 *>(hist) + t;
+        uint4 v[2];
+        uint32_t sum = 0;
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            v[h] = mine[h * kSortThreads];
+            sum += ((v[h].x & 0xffffu) + (v[h].y & 0xffffu) + (v[h].z & 0xffffu) + (v[h].w & 0xffffu)) << (16 * h);
+        }
+        const uint32_t incl = wave_scan_inclusive(sum);
+        if (lane == 63) wave_sum[wave] = incl;
+        __syncthreads();
+        const uint32_t each = wave_sum[lane & 15];
+        const uint32_t all = row_sum(each) & 0xffffu; // of the first part
+        const uint32_t before = row_sum((lane & 15) < wave ? each : 0u) + incl - sum;
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const uint32_t x = h == 0 ? before & 0xffffu : all + (before >> 16);
+            const uint32_t y = x + (v[h].x & 0xffffu), z = y + (v[h].y & 0xffffu), w = z + (v[h].z & 0xffffu);
+            mine[h * kSortThreads] = make_uint4(with_low(v[h].x, x), with_low(v[h].y, y), with_low(v[h].z, z), with_low(v[h].w, w));
+        }
+    }
+    __syncthreads();
+    if (wave < kWaves) {
+        // the zeros before the tile: of the 64 counters
+        const uint32_t zeros = (uint32_t)__builtin_amdgcn_readlane((int)wave_scan_inclusive(hist[slot(end)] >> 16), 63);
+        const uint32_t at = hist[slot(key)];
+        if (nbefore + t < nsc)
+            place_sorted((int)((at & 0xffffu) + (key == last ? zeros : at >> 16) + rank[t]), nbefore + t, nsc, top, bottom,
+                         qbits_out, order);
     }
 }
 
-template <bool WIDE>
-__device__ __forceinline__ void sorted_plan_body(const uint32_t *__restrict__ pairs, int nsc, int top, int bottom,
-                                                 int64_t *__restrict__ qbits_out, int32_t *__restrict__ order,
-                                                 const uint32_t (&cached)[kSortBatch], uint32_t own_pattern, uint32_t *hist,
-                                                 uint32_t *wave_sum)
+// the signed layout: adds the keys of the superchunks [begin, end)
+__device__ __forceinline__ void count_signed(const uint32_t *__restrict__ pairs, int begin, int end, uint32_t *hist)
+{
+    constexpr int kBatch = 8;
+    for (int i0 = begin + (int)threadIdx.x; i0 < end; i0 += kBatch * kSortThreads) {
+        uint32_t raw[kBatch];
+#pragma unroll
+        for (int j = 0; j < kBatch; j++) raw[j] = pairs[min(i0 + j * kSortThreads, end - 1)];
+#pragma unroll
+        for (int j = 0; j < kBatch; j++) {
+            const uint32_t k = signed_key(raw[j] >> 16);
+            if (i0 + j * kSortThreads < end) atomicAdd(&hist[hist_slot(k >> 1)], 1u << (16 * (k & 1)));
+        }
+    }
+}
+
+template <int TILE>
+__device__ __forceinline__ void sorted_plan_signed(const uint32_t *__restrict__ pairs, int nsc, int top, int bottom,
+                                                   int64_t *__restrict__ qbits_out, int32_t *__restrict__ order, uint32_t *hist,
+                                                   uint32_t *wave_sum)
 {
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    const int nbefore = (int)blockIdx.x * kSortTile;
-    const int own = nbefore + t; // of the first kSortTile threads
-    const int valid = min(kSortTile, nsc - nbefore);
+    const int nbefore = (int)blockIdx.x * TILE;
+    const int valid = min(TILE, nsc - nbefore);
     const bool mine = t < valid;
-    const uint32_t key = sort_key<WIDE>(own_pattern);
-
-    // lanes of the wave that hold the same key
-    uint64_t same = 0;
-    if (wave < kSortTile / 64) {
-        same = __builtin_amdgcn_ballot_w64(mine);
-#pragma unroll
-        for (int bit = 0; bit < (WIDE ? 16 : 15); bit++) {
-            const bool set = (key >> bit) & 1u;
-            const uint64_t with = __builtin_amdgcn_ballot_w64(set);
-            same &= set ? with : ~with;
-        }
-    }
+    const uint32_t key = mine ? signed_key(pairs[nbefore + t] >> 16) : 0u;
+    const auto counter = [&]() { return (hist[hist_slot(key >> 1)] >> (16 * (key & 1))) & 0xffffu; };
+    const uint64_t same = lanes_with<16>(key, key) & __builtin_amdgcn_ballot_w64(mine);
     const uint64_t lower = same & (((uint64_t)1 << lane) - 1u);
-    count_keys<WIDE>(pairs, 0, nbefore, hist, cached);
+    count_signed(pairs, 0, nbefore, hist);
     __syncthreads();
-    int same_before = 0;
+    uint32_t same_before = 0;
 #pragma unroll
-    for (int w = 0; w < kSortTile / 64; w++) {
+    for (int w = 0; w < TILE / 64; w++) {
         if (wave == w && mine) {
-            same_before = counter_of<WIDE>(hist, key) + (int)__popcll(lower);
+            same_before = counter() + (uint32_t)__popcll(lower);
             __builtin_amdgcn_wave_barrier(); // every lane has read before any adds
-            if (lower == 0) {
-                const uint32_t many = (uint32_t)__popcll(same);
-                if (WIDE)
-                    atomicAdd(&hist[hist_slot(key >> 1)], many << (16 * (key & 1)));
-                else
-                    atomicAdd(&hist[hist_slot(key)], many);
-            }
+            if (lower == 0) atomicAdd(&hist[hist_slot(key >> 1)], (uint32_t)__popcll(same) << (16 * (key & 1)));
         }
         __syncthreads();
     }
-    count_keys<WIDE>(pairs, nbefore + valid, nsc, hist, cached);
+    count_signed(pairs, nbefore + valid, nsc, hist);
     __syncthreads();
-    scan_counters<WIDE>(hist, wave_sum);
+    // exclusive scan of the counters in place; thread t owns the words [32 t, 32 t + 32)
+    uint32_t *own = hist + 36 * t; // hist_slot(32 t)
+    uint32_t sum = 0;
+    for (int q = 0; q < 32; q++) sum += (own[q] & 0xffffu) + (own[q] >> 16);
+    const uint32_t incl = wave_scan_inclusive(sum);
+    if (lane == 63) wave_sum[wave] = incl;
     __syncthreads();
-
-    if (mine) {
-        const int pos = counter_of<WIDE>(hist, key) + same_before;
-        const int mid_end = nsc - bottom;
-        int region, at;
-        if (pos < top) region = 0, at = pos;
-        else if (pos < mid_end) region = 1, at = pos - top;
-        else region = 2, at = pos - mid_end;
-        order[(int64_t)region * nsc + at] = own;
-        if (qbits_out) qbits_out[own] = region == 0 ? 8 : (region == 1 ? 4 : 2);
+    uint32_t run = row_sum((lane & 15) < wave ? wave_sum[lane & 15] : 0u) + incl - sum;
+    for (int q = 0; q < 32; q++) {
+        const uint32_t lo = own[q] & 0xffffu, hi = own[q] >> 16;
+        own[q] = (run & 0xffffu) | ((run + lo) << 16); // the prefix of a key present is at most nsc - 1 < 65536
+        run += lo + hi;
     }
+    __syncthreads();
+    if (mine) place_sorted((int)(counter() + same_before), nbefore + t, nsc, top, bottom, qbits_out, order);
 }
 
+template <int TILE, int BATCH>
 __global__ __launch_bounds__(kSortThreads) void sorted_plan_kernel(const uint32_t *__restrict__ pairs, int nsc, int top,
                                                                   int bottom, int64_t *__restrict__ qbits_out,
                                                                   int32_t *__restrict__ order, int32_t *__restrict__ work)
 {
     __shared__ __align__(16) uint32_t hist[kSortLdsWords];
     __shared__ uint32_t wave_sum[kSortThreads / 64];
+    __shared__ uint2 seen[kSortThreads / 64];
+    __shared__ uint32_t rank[TILE];
     __shared__ int any_negative;
-    const int t = threadIdx.x;
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int nbefore = (int)blockIdx.x * TILE;
+    // through a buffer descriptor, which returns 0 beyond the end: no branch and no clamp between the loads
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t *>(pairs), 0, nsc * 4, 0x00020000);
+    uint32_t cached[BATCH], row_pair = 0, col_pair = 0;
+#pragma unroll
+    for (int j = 0; j < BATCH; j++) cached[j] = __builtin_amdgcn_raw_buffer_load_b32(rsrc, (j * kSortThreads + t) * 4, 0, 0);
+    if (wave < kTilePairs<TILE / 64>) {
+        int row, col;
+        tile_pair<TILE / 64>(wave, row, col);
+        row_pair = pairs[min(nbefore + row * 64 + lane, nsc - 1)];
+        col_pair = pairs[min(nbefore + col * 64 + lane, nsc - 1)];
+    }
+    uint4 *h4 = reinterpret_cast<uint4 *>(hist);
+    h4[t] = h4[kSortThreads + t] = make_uint4(0u, 0u, 0u, 0u); // the short layout's counters
+    if (t < TILE) rank[t] = 0;
     if (t == 0) any_negative = 0;
-    // the first kSortBatch * kSortThreads pairs stay in registers for all three passes over them
-    uint32_t cached[kSortBatch];
+    // the greatest pattern, and the complement of the least one other than +0 less one (0 if there is none)
+    uint32_t high = 0, low = 0;
 #pragma unroll
-    for (int j = 0; j < kSortBatch; j++) {
-        const int i = j * kSortThreads + t;
-        cached[j] = i < nsc ? pairs[i] : 0u;
+    for (int j = 0; j < BATCH; j++) {
+        high = max(high, cached[j]);
+        low = max(low, ~(cached[j] - 0x10000u));
     }
-    const int own = (int)blockIdx.x * kSortTile + t;
-    const uint32_t own_pattern = t < kSortTile && own < nsc ? pairs[own] >> 16 : 0u;
-    {
-        uint4 *h4 = reinterpret_cast<uint4 *>(hist);
-        for (int w = t; w < kSortLdsWords / 4; w += kSortThreads) h4[w] = make_uint4(0u, 0u, 0u, 0u);
-    }
+    high = wave_max_upward(high);
+    low = wave_max_upward(low);
+    if (lane == 63) seen[wave] = make_uint2(high, low);
     __syncthreads();
-    // any pattern with the sign bit set that is not a NaN (a NaN is key 0 in both layouts)
-    bool negative = false;
+    high = wave_max_upward(seen[lane & 15].x);
+    low = wave_max_upward(seen[lane & 15].y);
+    const uint32_t first = (uint32_t)__builtin_amdgcn_readlane((int)high, 63) >> 16;
+    const uint32_t under = ~(uint32_t)__builtin_amdgcn_readlane((int)low, 63) >> 16;
+    const uint32_t last = first == 0 ? 0u : first - under; // the key of +0
+    if (first <= (uint32_t)kMaxPattern && last + 64u <= (uint32_t)kShortKeys) {
+        sorted_plan_once<false, TILE>(nsc, top, bottom, qbits_out, order, cached, row_pair, col_pair, max(first, 64u), last, hist, wave_sum,
+                                      rank);
+    } else {
+        for (int w = 2 * kSortThreads + t; w < kSortLdsWords / 4; w += kSortThreads) h4[w] = make_uint4(0u, 0u, 0u, 0u);
+        if (first >= 0x8000u) {
+            bool negative = false; // a sign bit that is not a NaN's
 #pragma unroll
-    for (int j = 0; j < kSortBatch; j++) negative |= (cached[j] >> 31) != 0 && (cached[j] & 0x7fff0000u) <= ((uint32_t)kMaxPattern << 16);
-    for (int i = kSortBatch * kSortThreads + t; i < nsc; i += kSortThreads) {
-        const uint32_t p = pairs[i];
-        negative |= (p >> 31) != 0 && (p & 0x7fff0000u) <= ((uint32_t)kMaxPattern << 16);
+            for (int j = 0; j < BATCH; j++) negative |= (cached[j] >> 31) != 0 && (cached[j] & 0x7fff0000u) <= ((uint32_t)kMaxPattern << 16);
+            if (__builtin_amdgcn_ballot_w64(negative) != 0 && lane == 0) any_negative = 1;
+        }
+        __syncthreads();
+        if (any_negative)
+            sorted_plan_signed<TILE>(pairs, nsc, top, bottom, qbits_out, order, hist, wave_sum);
+        else
+            sorted_plan_once<true, TILE>(nsc, top, bottom, qbits_out, order, cached, row_pair, col_pair,
+                                         (uint32_t)kMaxPattern + 1u, (uint32_t)kMaxPattern + 1u, hist, wave_sum, rank);
     }
-    if (__builtin_amdgcn_ballot_w64(negative) != 0 && (t & 63) == 0) any_negative = 1;
-    __syncthreads();
-    if (any_negative)
-        sorted_plan_body<true>(pairs, nsc, top, bottom, qbits_out, order, cached, own_pattern, hist, wave_sum);
-    else
-        sorted_plan_body<false>(pairs, nsc, top, bottom, qbits_out, order, cached, own_pattern, hist, wave_sum);
     if (blockIdx.x == 0 && t == 0) {
         work[0] = top;
         work[1] = nsc - top - bottom;
@@ -893,12 +996,21 @@ __global__ __launch_bounds__(kSortThreads) void sorted_plan_kernel(const uint32_
 
 } // namespace
 
+// At most 256 workgroups, one per compute unit (the long histogram fills its LDS).  32,768 superchunks fit the registers
+// with 32 a thread and 128 of them a workgroup; the larger instance spills a few of its 64 (32,768 superchunks 6.9 us,
+// 32,769 9.8).
 hipError_t launch_group_plan_sorted(const void *stats, int64_t nsc, int64_t top, int64_t bottom, int64_t *qbits_out,
                                     int32_t *order, int32_t *work, hipStream_t stream)
 {
-    const int ntiles = (int)((nsc + kSortTile - 1) / kSortTile);
-    hipLaunchKernelGGL(sorted_plan_kernel, dim3(ntiles), dim3(kSortThreads), 0, stream,
-                       static_cast<const uint32_t *>(stats), (int)nsc, (int)top, (int)bottom, qbits_out, order, work);
+    const uint32_t *pairs = static_cast<const uint32_t *>(stats);
+    const auto run = [&](auto kernel, int tile) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)((nsc + tile - 1) / tile)), dim3(kSortThreads), 0, stream, pairs, (int)nsc,
+                           (int)top, (int)bottom, qbits_out, order, work);
+    };
+    if (nsc <= 32 * kSortThreads)
+        run(sorted_plan_kernel<128, 32>, 128);
+    else
+        run(sorted_plan_kernel<256, 64>, 256);
     return hipGetLastError();
 }
 

@@ -91,6 +91,36 @@ def test_sorted_plan_matches_argsort(capi, oracle, name, method):
     assert (qb.cpu().numpy() == want_q).all()
 
 
+@pytest.mark.parametrize("nsc", [1, 127, 128, 129, 1025, 32768, 32769, 65535])
+@pytest.mark.parametrize("span", [0, 1, 8127, 8128, 8129, 0x7f80])
+def test_sorted_plan_layouts(capi, oracle, nsc, span):
+    """the norm patterns from `span` below the greatest on (a counter for each up to 8,127, the long histogram beyond it),
+    with none, some and only zeros, NaN, and one negative: at the edges of the tiles and of the two instances"""
+    rng = np.random.default_rng(nsc + span)
+    for kind in ("plain", "zeros", "all zero", "nan", "negative"):
+        top = 0x7f80 if span == 0x7f80 else 0x5000
+        bits = (top - rng.integers(0, span + 1, nsc)).astype(np.uint16)
+        bits[0], bits[-1] = top - span, top
+        if kind == "zeros":
+            bits[rng.integers(0, nsc, nsc // 3)] = 0
+        elif kind == "all zero":
+            bits[:] = 0
+        elif kind == "nan":
+            bits[nsc // 2], bits[nsc // 3] = 0x7fc0, 0xffff
+        elif kind == "negative":
+            bits[nsc // 2] = 0x8000
+        st = _stats(torch.from_numpy(bits.view(np.int16)).view(torch.bfloat16))
+        top_count, bottom_count = nsc // 3, nsc // 5
+        order = torch.full((3 * nsc,), -7, dtype=torch.int32, device=DEV)
+        work = torch.zeros(4, dtype=torch.int32, device=DEV)
+        capi.group_plan_sorted(st, top_count, bottom_count, order, work)
+        want = oracle.argsort_descending_stable(bits)
+        got = order.cpu().numpy()
+        for base, lo, hi in ((0, 0, top_count), (nsc, top_count, nsc - bottom_count), (2 * nsc, nsc - bottom_count, nsc)):
+            assert np.array_equal(got[base:base + hi - lo], want[lo:hi]), (kind, base)
+            assert (got[base + hi - lo:base + nsc] == -7).all(), (kind, base)
+
+
 def test_sorted_plan_wrapper_and_module(capi, eden_utils):
     from dynamiq_sigcomm_artifact_amd import bitrate as B
     g = torch.Generator().manual_seed(5)
