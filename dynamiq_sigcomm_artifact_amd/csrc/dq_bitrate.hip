@@ -7,9 +7,9 @@
 // pattern it is a step function with two steps.  So:
 //   norm_histogram_kernel   counts the norm patterns of a bucket's statistics into a histogram (one pass per
 //                           bucket, accumulated over the buckets of a training step);
-//   bitrate_search_kernel   one workgroup: turns the histogram into suffix counts, then runs the reference's
+//   bitrate_search_kernel   one workgroup: keeps the histogram in LDS with a sum per 256 bins, then runs the reference's
 //                           whole bisection (or its incremental correction) in double, each probe being two
-//                           threshold searches over the patterns and two look-ups.
+//                           threshold searches over the patterns and two sums over a wave.
 // The result (u, average width, target - average) equals what the torch ops of the reference give for the same
 // norms: the counts are exact integers and the arithmetic of the search is the same IEEE double arithmetic.
 #include "dq_bitwidth.cuh"
@@ -30,13 +30,13 @@ __global__ __launch_bounds__(kHistThreads) void norm_histogram_kernel(const uint
 }
 
 // What bounds the search: one workgroup, so everything is a latency.  The histogram (128 KB) comes in as eight coalesced
-// 16-byte loads per thread -- 32 consecutive bins per thread, as first written, fetched every line eight times over -- is
-// turned into suffix counts in registers and lands in LDS, and a round of probes asks for up to eight values of u at once,
+// 16-byte loads per thread -- 32 consecutive bins per thread fetched every line eight times over -- and lands in LDS as it
+// is, with a sum per 256 bins beside it; a count of the norms from a pattern on is then one more sum over a wave.  (Suffix
+// counts of all bins, by shuffles, for the two that a converged correction looks at: 9.1 us instead of 5.0.)  A round of
+// probes asks for up to eight values of u at once,
 // one pair of waves each: the seven midpoints of the next three steps of the bisection, or the next eight corrections, which
-// all follow from the first probe's deficit.  The walk through them is the reference's, probe by probe.
-// Kernel time of a converged correction (one probe): 39.7 -> 10.4 us, 9.0 with the first round's thresholds found while the
-// histogram is on its way.  With the events around it and 200,000 norms: one probe
-// 48 -> 17 us, a bisection of ten probes 60 -> 24 us.
+// all follow from the first probe's deficit.  The walk through them is the reference's, probe by probe.  The first round's
+// thresholds are found while the histogram is on its way.
 constexpr int kBins = 32768;                     // >= kNanBin + 1
 constexpr int kSlabs = kBins / (4 * kSearchThreads);
 constexpr int kSearchWaves = kSearchThreads / 64;
@@ -47,15 +47,16 @@ struct Probe {
     double avg, delta;
 };
 
-// sum over the lanes l' >= l of the wave
-__device__ __forceinline__ uint32_t wave_suffix_sum(uint32_t x, int lane)
+// the sum over the wave
+__device__ __forceinline__ uint32_t wave_sum(uint32_t x)
 {
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        const uint32_t y = (uint32_t)__shfl_down((int)x, off, 64);
-        x += lane + off < 64 ? y : 0u;
-    }
-    return x;
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xf, 0xf, false); // row_shr:1, 2, 4, 8
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xf, 0xf, false);
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xf, 0xf, false);
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xf, 0xf, false);
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xa, 0xf, false); // row_bcast:15 into rows 1 and 3
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xc, 0xf, false); // row_bcast:31 into rows 2 and 3
+    return (uint32_t)__builtin_amdgcn_readlane((int)x, 63);
 }
 
 // out[0..2] = u, average width, target - average; out[3] = number of probes.  hist: pattern counts in, zeros out.
@@ -64,8 +65,8 @@ __global__ __launch_bounds__(kSearchThreads) void bitrate_search_kernel(uint32_t
                                                                        const double *prev_u_dev, double target,
                                                                        double *out)
 {
-    extern __shared__ __attribute__((aligned(16))) uint32_t suffix[]; // suffix[p] = norms of pattern >= p (numbers only)
-    __shared__ uint32_t part[kSlabs][kSearchWaves];
+    extern __shared__ __attribute__((aligned(16))) uint32_t bins[]; // the histogram, numbers only
+    __shared__ __attribute__((aligned(8))) uint32_t part[kSlabs][kSearchWaves];
     __shared__ uint32_t nans;
     __shared__ uint32_t at_least[2][kProbes]; // norms of width >= 4, >= 8
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
@@ -114,8 +115,8 @@ __global__ __launch_bounds__(kSearchThreads) void bitrate_search_kernel(uint32_t
         return mid;
     };
     const double start = __builtin_fmax(u_min, __builtin_fmin(u_max, prev_u));
-    const int p_first = find(mode == 0 ? (pair == 0 ? u_max : node_mid(u_min, u_max)) : start);
-    uint32_t incl[kSlabs];
+    int p_first = 0;
+    if (mode == 0 || pair == 0) p_first = find(mode == 0 ? (pair == 0 ? u_max : node_mid(u_min, u_max)) : start);
 #pragma unroll
     for (int k = 0; k < kSlabs; k++) {
         const int p = 4 * (t + kSearchThreads * k);
@@ -124,38 +125,33 @@ __global__ __launch_bounds__(kSearchThreads) void bitrate_search_kernel(uint32_t
             if (p == kMaxPattern) nans = v[k].y;
             v[k] = make_uint4(p == kMaxPattern ? v[k].x : 0u, 0u, 0u, 0u);
         }
-        incl[k] = wave_suffix_sum(v[k].x + v[k].y + v[k].z + v[k].w, lane);
-        if (lane == 0) part[k][wave] = incl[k];
+        reinterpret_cast<uint4 *>(bins)[t + kSearchThreads * k] = v[k];
+        const uint32_t sum = wave_sum(v[k].x + v[k].y + v[k].z + v[k].w);
+        if (lane == 0) part[k][wave] = sum;
     }
     __syncthreads();
-    // entry (k, w) of part is the sum of its 256 bins; what follows it in bin order: the waves behind it in its slab, and
-    // every slab behind that.  Lane l of each wave looks at entries 2 l and 2 l + 1 of the 128.
+    // entry (k, w) of part is the sum of the 256 bins from 256 (16 k + w) on; lane l of each wave holds entries 2 l and 2 l + 1
     static_assert(kSlabs * kSearchWaves == 128, "two entries per lane");
-    const uint32_t *flat = &part[0][0];
-    const uint32_t e0 = flat[2 * lane], e1 = flat[2 * lane + 1];
-    const uint32_t from = wave_suffix_sum(e0 + e1, lane); // entries >= 2 lane
-#pragma unroll
-    for (int k = 0; k < kSlabs; k++) {
-        const int entry = k * kSearchWaves + wave; // entries > entry: (entries >= 2 (entry / 2)) minus one or two of them
-        const uint32_t base = (uint32_t)__shfl((int)from, entry >> 1, 64), a = (uint32_t)__shfl((int)e0, entry >> 1, 64),
-                       b = (uint32_t)__shfl((int)e1, entry >> 1, 64);
-        const uint32_t behind = base - a - ((entry & 1) ? b : 0u) + incl[k] - (v[k].x + v[k].y + v[k].z + v[k].w);
-        uint4 s;
-        s.w = behind + v[k].w;
-        s.z = s.w + v[k].z;
-        s.y = s.z + v[k].y;
-        s.x = s.y + v[k].x;
-        reinterpret_cast<uint4 *>(suffix)[t + kSearchThreads * k] = s;
-    }
-    __syncthreads();
-    const uint64_t total = (uint64_t)suffix[0] + nans;
+    const uint2 entries = reinterpret_cast<const uint2 *>(&part[0][0])[lane];
+    const uint64_t total = (uint64_t)wave_sum(entries.x + entries.y) + nans;
+    // norms of pattern >= p: the entries behind p's, and what lies in p's own
+    const auto count_from = [&](int p) {
+        if (p > kMaxPattern) return 0u;
+        const int e = p >> 8, first = 4 * lane, from = p & 255;
+        const uint4 q = reinterpret_cast<const uint4 *>(bins)[64 * e + lane];
+        uint32_t sum = (2 * lane > e ? entries.x : 0u) + (2 * lane + 1 > e ? entries.y : 0u);
+        sum += (first >= from ? q.x : 0u) + (first + 1 >= from ? q.y : 0u);
+        sum += (first + 2 >= from ? q.z : 0u) + (first + 3 >= from ? q.w : 0u);
+        return wave_sum(sum);
+    };
 
     // every thread evaluates the same doubles, so the control flow below is uniform without a broadcast
     int probes = 0;
     // one round: waves 2 k and 2 k + 1 hold the thresholds of candidate k
     const auto publish = [&](int p) {
         __syncthreads(); // the previous round has been read
-        if (lane == 0) at_least[wave & 1][wave >> 1] = p <= kMaxPattern ? suffix[p] : 0u;
+        const uint32_t n = count_from(p);
+        if (lane == 0) at_least[wave & 1][wave >> 1] = n;
         __syncthreads();
     };
     const auto result = [&](int k) {

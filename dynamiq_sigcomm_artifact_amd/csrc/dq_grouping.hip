@@ -713,17 +713,6 @@ __device__ __forceinline__ uint32_t signed_key(uint32_t pattern)
     return 0x7fffu - mag;                                   // +inf -> 0x7f, +0 -> 0x7fff
 }
 
-// the largest of the wave's values, in lane 63
-__device__ __forceinline__ uint32_t wave_max_upward(uint32_t x)
-{
-    x = max(x, dpp_from<0x111, 0xf>(x)); // row_shr:1, 2, 4, 8
-    x = max(x, dpp_from<0x112, 0xf>(x));
-    x = max(x, dpp_from<0x114, 0xf>(x));
-    x = max(x, dpp_from<0x118, 0xf>(x));
-    x = max(x, dpp_from<0x142, 0xa>(x)); // row_bcast:15 into rows 1 and 3
-    return max(x, dpp_from<0x143, 0xc>(x)); // row_bcast:31 into rows 2 and 3
-}
-
 // the sum over a row of 16 lanes, in every lane
 __device__ __forceinline__ uint32_t row_sum(uint32_t x)
 {

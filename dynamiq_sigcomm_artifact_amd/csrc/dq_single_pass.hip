@@ -217,16 +217,79 @@ struct TallyArgs {
 };
 
 // A workgroup takes kTallyBatch superchunks of one bucket.  A wave's norms are alike and meet in a few counters of the LDS, so the
-// counting is better spread over more workgroups: 209,716 norms with 8192 each 7.9 us, 4096 6.6, 2048 and 1024 6.4 (5.9 since
-// the thresholds are searched beside the counting).
+// counting is better spread over more workgroups: 209,716 norms with 8192 each 7.9 us, 4096 6.6, 2048 and 1024 6.4.  What is
+// left is a chain of latencies; clearing 64 KB of counters, going over them afterwards and searching the two thresholds for two
+// norms per thread were the longest links (6.0 us; 4.6 with the counters in range alone and the rule applied to each norm).
+// (Clearing each norm's own counter and leaving it to whoever found it at 0 spares a barrier, but scatters the atomics on memory:
+// 4.8 us here, and 42.9 instead of 12.1 for batches of 8192 of 3,000,000 norms.)
 constexpr int kTallyThreads = 1024, kTallyBatch = 2048;
+
+// The norm patterns of a tally's batch, counted in LDS (16-bit counters, two per word) and added to the histogram in memory: begin
+// (two barriers), add, a barrier of the caller's, flush.  Thread t holds the patterns k * kTallyThreads + t, of which those
+// below `have` count.  Only the counters between the batch's least and greatest pattern are cleared and gone over, where zeros
+// (of which a bucket may hold many) and NaN are counted apart.
+template <int PER> struct PatternBatch {
+    uint32_t low, high; // words of counters in use
+    uint32_t zeros, nans;
+
+    __device__ __forceinline__ void begin(const uint32_t (&pattern)[PER], int have, uint32_t *local, uint4 *wave_seen)
+    {
+        const int t = threadIdx.x, lane = t & 63;
+        uint32_t top = 0, under = 0; // the greatest bin, the complement of the least
+        zeros = nans = 0;
+#pragma unroll
+        for (int k = 0; k < PER; k++) {
+            const uint32_t bin = (uint32_t)bin_of(pattern[k]);
+            const bool in = k * kTallyThreads + t < have, zero = bin == 0u, nan = bin == (uint32_t)kNanBin;
+            top = max(top, in && !nan ? bin : 0u);
+            under = max(under, in && !zero && !nan ? ~bin : 0u);
+            zeros += (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(in && zero));
+            nans += (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(in && nan));
+        }
+        top = wave_max_upward(top);
+        under = wave_max_upward(under);
+        if (lane == 63) wave_seen[t >> 6] = make_uint4(top, under, zeros, nans);
+        __syncthreads();
+        static_assert(kTallyThreads / 64 == 16, "a row of 16 lanes holds a value of every wave");
+        const uint4 seen = wave_seen[lane & 15];
+        high = (uint32_t)__builtin_amdgcn_readlane((int)wave_max_upward(seen.x), 63) >> 1;
+        low = ~(uint32_t)__builtin_amdgcn_readlane((int)wave_max_upward(seen.y), 63) >> 1; // (no bin at all: beyond every word)
+        zeros = seen.z;
+        nans = seen.w;
+        for (uint32_t w = low + t; w <= high; w += kTallyThreads) local[w] = 0u;
+        __syncthreads();
+    }
+
+    __device__ __forceinline__ void add(const uint32_t (&pattern)[PER], int have, uint32_t *local) const
+    {
+#pragma unroll
+        for (int k = 0; k < PER; k++) {
+            const int bin = bin_of(pattern[k]);
+            if (k * kTallyThreads + (int)threadIdx.x < have && bin != 0 && bin != kNanBin) atomicAdd(&local[bin >> 1], 1u << (16 * (bin & 1)));
+        }
+    }
+
+    __device__ __forceinline__ void flush(uint32_t *__restrict__ hist, const uint32_t *local) const
+    {
+        // (a word per thread: the counters in use lie side by side)
+        for (uint32_t w = low + threadIdx.x; w <= high; w += kTallyThreads) {
+            const uint32_t pair = local[w];
+            if (pair & 0xffffu) atomicAdd(&hist[2 * w], pair & 0xffffu);
+            if (pair >> 16) atomicAdd(&hist[2 * w + 1], pair >> 16);
+        }
+        if (threadIdx.x < 16) { // an entry of wave_seen each
+            if (zeros) atomicAdd(&hist[0], zeros);
+            if (nans) atomicAdd(&hist[kNanBin], nans);
+        }
+    }
+};
 
 template <bool HIST> __global__ __launch_bounds__(kTallyThreads) void tally_kernel(TallyArgs a)
 {
-    __shared__ __attribute__((aligned(16))) uint32_t local[HIST ? kHistWords : 4];
-    __shared__ int thr[2];
+    __shared__ uint32_t local[HIST ? kHistWords : 1];
+    __shared__ uint4 wave_seen[HIST ? kTallyThreads / 64 : 1];
     __shared__ uint32_t total[2];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63;
     const int at = last_at_most(a.first_block, a.buckets, blockIdx.x);
     const TallyBucket b = a.bucket[at];
     const int64_t begin = (int64_t)(blockIdx.x - a.first_block[at]) * kTallyBatch;
@@ -240,33 +303,18 @@ template <bool HIST> __global__ __launch_bounds__(kTallyThreads) void tally_kern
     for (int k = 0; k < kPer; k++) norm[k] = mine[2 * min(k * kTallyThreads + (int)threadIdx.x, have - 1)];
     const float u = a.rule.u_dev ? (float)*a.rule.u_dev : a.rule.u;
     if (threadIdx.x < 2) total[threadIdx.x] = 0u;
+    PatternBatch<kPer> batch;
     if (HIST) {
-        uint4 *l4 = reinterpret_cast<uint4 *>(local);
-        for (int w = threadIdx.x; w < kHistWords / 4; w += kTallyThreads) l4[w] = make_uint4(0u, 0u, 0u, 0u);
+        batch.begin(norm, have, local, wave_seen);
+        batch.add(norm, have, local);
+    } else {
         __syncthreads();
     }
-    // two waves search the thresholds while the others count
-    if (a.rule.thr[0] >= 0) {
-        if (threadIdx.x < 2) thr[threadIdx.x] = a.rule.thr[threadIdx.x];
-    } else {
-        width_thresholds(u, thr, wave, lane);
-    }
-    if (HIST) {
-#pragma unroll
-        for (int k = 0; k < kPer; k++) {
-            if (k * kTallyThreads + (int)threadIdx.x < have) {
-                const int bin = bin_of(norm[k]);
-                atomicAdd(&local[bin >> 1], 1u << (16 * (bin & 1)));
-            }
-        }
-    }
-    __syncthreads();
-    const int t2[2] = {thr[0], thr[1]};
     uint32_t n8 = 0, n4 = 0;
 #pragma unroll
     for (int k = 0; k < kPer; k++) {
         const bool in = k * kTallyThreads + (int)threadIdx.x < have;
-        const int c = class_of_norm(norm[k], u, t2);
+        const int c = a.rule.thr[0] >= 0 ? class_of_norm(norm[k], u, a.rule.thr) : width_class_of_norm(norm[k], u);
         n8 += (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(in && c == 0));
         n4 += (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(in && c == 1));
     }
@@ -280,14 +328,7 @@ template <bool HIST> __global__ __launch_bounds__(kTallyThreads) void tally_kern
         if (c2) atomicAdd(&b.counts[2], c2);
         if (blockIdx.x == 0 && a.step_dev && a.step_more) *a.step_dev += a.step_more;
     }
-    if (HIST) {
-        // (a word per thread: the counters in use lie side by side)
-        for (int w = threadIdx.x; w < kHistWords; w += kTallyThreads) {
-            const uint32_t pair = local[w];
-            if (pair & 0xffffu) atomicAdd(&a.hist[2 * w], pair & 0xffffu);
-            if (pair >> 16) atomicAdd(&a.hist[2 * w + 1], pair >> 16);
-        }
-    }
+    if (HIST) batch.flush(a.hist, local);
 }
 
 // ---- W ranks --------------------------------------------------------------------------------------------

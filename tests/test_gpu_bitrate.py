@@ -53,6 +53,58 @@ def test_norm_histogram_counts(capi):
     assert want[MAXP] == 2 and want[MAXP + 1] > 0           # +inf (in both calls), NaN
 
 
+@pytest.mark.parametrize("nsc", [1, 1023, 1025, 2047, 2048, 2049, 8191, 8192, 8193, 20000])
+def test_pattern_counts_at_the_edges_of_the_batches(capi, oracle, nsc):
+    """patterns that share a word of counters, one counter for half of the norms, and both ends of every 256 bins; then the
+    search over them, whose sums end inside and at the edges of such a block"""
+    from dynamiq_sigcomm_artifact_amd.bitrate import NormHistogram
+    rng = np.random.default_rng(nsc)
+    bits = (256 * rng.integers(0x34, 0x46, nsc) + rng.choice([0, 1, 127, 128, 254, 255], nsc)).astype(np.uint16)
+    bits[rng.integers(0, nsc, nsc // 2)] = 0x3f80
+    bits[rng.integers(0, nsc, nsc // 50)] = 0x7fc0
+    stats = _stats(torch.from_numpy(bits.view(np.int16)).view(torch.bfloat16))
+    h = NormHistogram(DEV)
+    h.add(stats)
+    bins = np.where(bits > MAXP, MAXP + 1, bits)
+    assert (h.hist.cpu().numpy() == np.bincount(bins, minlength=h.hist.numel())).all()
+    for target in (2.5, 4.375, 6.5):
+        if h.count == 0:
+            h.add(stats)
+        assert h.binary_search_u(target) == tuple(oracle.dynamic_bitrate_binary_search_u([bits], target)), target
+
+
+@pytest.mark.parametrize("nsc", [1, 64, 1023, 1024, 1025, 2047, 2048, 2049, 4097])
+@pytest.mark.parametrize("u_on_device", [True, False])
+def test_pipeline_tally_at_the_edges_of_its_batches(capi, nsc, u_on_device):
+    """the widths' counts and the norm histogram of one bucket against the statistics themselves: norms on both sides of the
+    rule's steps, zeros, infinities and NaN"""
+    from dynamiq_sigcomm_artifact_amd import bitrate as B
+    from dynamiq_sigcomm_artifact_amd.dynamiq_pipeline import SinglePassBuckets
+    g = torch.Generator().manual_seed(nsc)
+    scale = torch.exp2(torch.randint(-24, 24, (nsc, 1), generator=g).float() + torch.rand(nsc, 1, generator=g))
+    x = torch.randn(nsc, 256, generator=g) * scale
+    x[torch.randint(0, nsc, (nsc // 9,), generator=g)] = 0.0
+    x[torch.randint(0, nsc, (nsc // 40,), generator=g), 3] = float("inf")
+    x[torch.randint(0, nsc, (nsc // 40,), generator=g), 7] = float("nan")
+    x = x.reshape(-1).to(torch.bfloat16).to(DEV)
+    u = 6.0
+    hist = B.NormHistogram(DEV)
+    pipe = SinglePassBuckets(DEV, strategy=2, seed=5, norm_histogram=hist,
+                             u=torch.full((1,), u, dtype=torch.float64, device=DEV) if u_on_device else u)
+    pipe.begin_step()
+    pipe.run_all([(x, torch.empty_like(x))])
+    torch.cuda.synchronize()
+    stats = torch.empty((nsc, 2), dtype=torch.bfloat16, device=DEV)
+    capi.superchunk_stats(x, stats, None, x.numel(), 1)
+    order = torch.empty(3 * nsc, dtype=torch.int32, device=DEV)
+    work = torch.zeros(capi.group_plan_work_ints(nsc), dtype=torch.int32, device=DEV)
+    capi.group_plan_stats(stats, u, None, order, work)
+    assert pipe.counts(0).tolist()[:3] == work[:3].tolist()
+    want = torch.zeros_like(hist.hist)
+    capi.norm_histogram(stats, want)
+    assert torch.equal(hist.hist, want)
+
+
 @pytest.mark.parametrize("name", list(_norm_sets().keys()))
 def test_search_equals_the_oracle_on_the_norms(capi, oracle, name):
     from dynamiq_sigcomm_artifact_amd.bitrate import NormHistogram
