@@ -11,12 +11,16 @@
 //           bit plane p of 32 consecutive bins -> packed[p * n/32 + w]; the products centroid[bin] * v are
 //           summed in double, thread t adding elements 16 t + k of the tile (k ascending), then halved -> work[tiles + b]
 //   scale   dot = fold(work[tiles ..]); scale = (norm * norm) / (float)dot
-// Beyond 2^22 elements the fold of sumsq is a launch of its own (eden_norm_kernel): in every workgroup it would read more
-// than the workgroup's own elements; the products then go to work[b].
+// Beyond 1024 partial sums (2^22 elements) the fold of sumsq is a launch of its own (eden_norm_kernel): in every workgroup it
+// would read more than the workgroup's own elements; the products then go to work[b].
+// In compress a rotation of more than one pass leaves the partial sums itself, one per workgroup of its strided pass: no sumsq
+// launch, and at most 1024 of them up to 2^25 elements.  Both directions at 4 bits: 2^20 elements 34.0 -> 30.1 us, 500,000
+// 31.9 -> 29.2, 12,000,000 136.6 -> 128.4.
 // (scale inside bins, by the workgroup that finishes last: its release of the other XCDs' sums costs more than the launch --
 // bins 5.7 -> 10.8 us at 2^20 elements, against 1.8 us for scale.)
-// The sums are in double with a fixed association, so the result does not depend on the launch geometry
-// and the CPU restatement reproduces it bit for bit.
+// The sums are in double with a fixed association, so the result does not depend on the launch geometry, and the CPU
+// restatement reproduces it bit for bit (those of the strided pass are as exact, but associated by its tiles: their
+// float32 differs only where a sum lies within some 2^-50 of it of a rounding boundary).
 #include <mutex>
 #include <vector>
 
@@ -127,7 +131,7 @@ __global__ __launch_bounds__(kEdenThreads) void eden_bins_kernel(QuantizeSet set
     __syncthreads();
     float norm;
     if constexpr (FOLD) {
-        const float sum = (float)fold_array(s.work, tiles, lds);
+        const float sum = (float)fold_array(s.sums, s.sum_count, lds);
         norm = __builtin_sqrtf(sum);
         if (tile == 0 && threadIdx.x == 0) {
             s.result[0] = sum;
@@ -140,7 +144,7 @@ __global__ __launch_bounds__(kEdenThreads) void eden_bins_kernel(QuantizeSet set
     uint16_t *half = in ? reinterpret_cast<uint16_t *>(s.packed) + (first >> 4) : nullptr;
     const double acc = eden_bins16<NBITS>(v, norm, s.sqrt_n, tree, cen, half, s.n >> 5);
     const double total = fold256(in ? acc : 0.0, lds, threadIdx.x);
-    if (threadIdx.x == 0) s.work[(FOLD ? tiles : 0) + tile] = total;
+    if (threadIdx.x == 0) s.work[(FOLD && s.sums == s.work ? tiles : 0) + tile] = total;
 }
 
 // one workgroup per slice: result[1] = (float)dot, result[2] = scale
@@ -149,7 +153,7 @@ __global__ __launch_bounds__(kEdenThreads) void eden_scale_kernel(QuantizeSet se
     __shared__ double lds[kEdenThreads];
     const QuantizeSlice &s = set.s[blockIdx.x];
     const int64_t tiles = eden_tiles(s.n);
-    const double dot = fold_array(s.work + (fold ? tiles : 0), tiles, lds);
+    const double dot = fold_array(s.work + (fold && s.sums == s.work ? tiles : 0), tiles, lds);
     if (threadIdx.x == 0) {
         const float d = (float)dot;
         const float norm = s.result[3];
@@ -261,16 +265,22 @@ hipError_t launch_eden_quantize_slices(const QuantizeSlice *slices, int count, c
     QuantizeSet set;
     set.count = count;
     int64_t blocks = 0;
+    bool have_sums = true;
+    for (int k = 0; k < count; k++) have_sums = have_sums && slices[k].sums;
     for (int k = 0; k < count; k++) {
         set.s[k] = slices[k];
         set.s[k].sqrt_n = (float)sqrt((double)slices[k].n);
+        if (!have_sums) {
+            set.s[k].sums = slices[k].work;
+            set.s[k].sum_count = eden_tiles(slices[k].n);
+        }
         set.first[k] = (unsigned)blocks;
         blocks += eden_tiles(slices[k].n);
     }
-    const bool fold = count > 1 || blocks <= kEdenFoldTiles;
+    const bool fold = count > 1 || set.s[0].sum_count <= kEdenFoldTiles;
     dim3 grid((unsigned)blocks), block(kEdenThreads);
-    hipLaunchKernelGGL(eden_sumsq_kernel, grid, block, 0, stream, set);
-    if (!fold) hipLaunchKernelGGL(eden_norm_kernel, dim3(1), block, 0, stream, slices[0].work, blocks, slices[0].result);
+    if (!have_sums) hipLaunchKernelGGL(eden_sumsq_kernel, grid, block, 0, stream, set);
+    if (!fold) hipLaunchKernelGGL(eden_norm_kernel, dim3(1), block, 0, stream, set.s[0].sums, set.s[0].sum_count, slices[0].result);
 #define DQ_EDEN_BINS(B)                                                                                       \
     do {                                                                                                      \
         if (fold)                                                                                             \
@@ -296,7 +306,7 @@ hipError_t launch_eden_quantize_slices(const QuantizeSlice *slices, int count, c
 hipError_t launch_eden_quantize(const float *vec, int64_t n, const float *boundaries, const float *centroids, int nbits,
                                 uint32_t *packed, float *result, double *work, hipStream_t stream)
 {
-    const QuantizeSlice s{vec, n, packed, result, work, 0.0f};
+    const QuantizeSlice s{vec, n, packed, result, work};
     return launch_eden_quantize_slices(&s, 1, boundaries, centroids, nbits, stream);
 }
 
@@ -416,11 +426,11 @@ hipError_t launch_thc_dequantize(const void *levels, float *out, int64_t n, cons
 // less: the time of a vector of less than a few million elements was its launches.  So the slices travel together:
 //   up to 2^13 elements   one workgroup per slice does all of it, all slices in one launch (dq_eden_short.hip); 2^14 as well
 //                         where no longer slice travels with the next kind's launches anyway
-//   up to 2^22            one launch per pass for all slices: tiles, strided pass, sumsq, bins, scale; tiles, strided pass
+//   up to 2^22            one launch per pass for all slices: tiles, strided pass, bins, scale; tiles, strided pass
 //   beyond                one after the other: their launches fill the GPU, and their diagonal is read from memory
 // Slices that are not plain powers of one rotation (only a caller's own dictionary asks for that) go one by one as well.
-// Both directions at 4 bits, fp32: 2^20 elements (one slice) 94 -> 38 -> 36 us, 20,000 (two) 165 -> 22, 115,387 (four) 364 -> 135 -> 54, 419,364
-// (three) 266 -> 115 -> 37, 6,000,000 (two) 186 -> 80: at first, (with one native call per slice,) together.
+// Both directions at 4 bits, fp32: 2^20 elements (one slice) 94 -> 38 -> 30 us, 20,000 (two) 165 -> 22, 115,387 (four) 364 -> 135 -> 44, 419,364
+// (three) 266 -> 115 -> 30, 6,000,000 (two) 186 -> 80: at first, (with one native call per slice,) together.
 
 namespace {
 
@@ -460,6 +470,9 @@ struct SliceScratch {
     float *vec;
     double *work;
     uint32_t *signs;
+    // the last pass's sums of squares take the place of the signs, which the first pass has read: n / 64 doubles' room, at
+    // most one for every 512 elements
+    double *sums() const { return reinterpret_cast<double *>(signs); }
 };
 
 int64_t round_up(int64_t v) { return (v + 255) & ~(int64_t)255; }
@@ -525,9 +538,16 @@ hipError_t compress_one(const dq_eden_slice_t &x, int dtype, const SliceScratch 
         hipLaunchKernelGGL(eden_pad_kernel, dim3((unsigned)((x.n + 255) / 256)), dim3(256), 0, stream, x.vec, dtype, x.count, x.n, s.vec);
         e = hipGetLastError();
     }
-    for (int i = 0; e == hipSuccess && i < x.rotations; i++)
-        e = rotate(s, x.n, x.seed + i, 0, i == 0 ? compress_ends(x, dtype) : TransformEnds(), stream);
-    return e == hipSuccess ? launch_eden_quantize(s.vec, x.n, x.boundaries, x.centroids, x.nbits, x.packed, x.result, s.work, stream) : e;
+    QuantizeSlice q{s.vec, x.n, x.packed, x.result, s.work};
+    for (int i = 0; e == hipSuccess && i < x.rotations; i++) {
+        TransformEnds ends = i == 0 ? compress_ends(x, dtype) : TransformEnds();
+        if (i == x.rotations - 1) {
+            q.sum_count = rht_sum_count(x.n);
+            if (q.sum_count) q.sums = ends.sums = s.sums();
+        }
+        e = rotate(s, x.n, x.seed + i, 0, ends, stream);
+    }
+    return e == hipSuccess ? launch_eden_quantize_slices(&q, 1, x.boundaries, x.centroids, x.nbits, stream) : e;
 }
 
 hipError_t decompress_one(const dq_eden_slice_t &x, int dtype, const SliceScratch &s, hipStream_t stream)
@@ -593,10 +613,12 @@ hipError_t launch_eden_slices(const dq_eden_slice_t *slices, int count, int dtyp
             t[k].scale = inv_sqrt_of(group[k].n);
             t[k].ends = decompress ? decompress_ends(group[k], dtype, true, true) : compress_ends(group[k], dtype);
             t[k].ends.gen = sign_seed(group[k].n, group[k].seed);
-            q[k] = QuantizeSlice{room[k].vec, group[k].n, group[k].packed, group[k].result, room[k].work, 0.0f};
+            if (!decompress) t[k].ends.sums = room[k].sums();
         }
         const hipError_t r = launch_rht_slices(t, have, decompress ? 1 : 0, stream);
         if (r != hipSuccess || decompress) return r;
+        for (int k = 0; k < have; k++)
+            q[k] = QuantizeSlice{room[k].vec, group[k].n, group[k].packed, group[k].result, room[k].work, room[k].sums(), t[k].sum_count};
         return launch_eden_quantize_slices(q, have, group[0].boundaries, group[0].centroids, group[0].nbits, stream);
     });
     if (e == hipSuccess)

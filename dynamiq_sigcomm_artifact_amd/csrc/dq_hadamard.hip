@@ -243,6 +243,23 @@ static int contiguous_bits(int kb)
     return kb <= 25 ? kb - 10 : kPrefTileBits;
 }
 
+// rows of the next strided pass: the remaining bits split evenly over as few passes as the LDS allows
+static int rows_of_pass(int rem)
+{
+    constexpr int max_rows = kMaxTileBits - kStridedCols;
+    const int passes = (rem + max_rows - 1) / max_rows;
+    return (rem + passes - 1) / passes;
+}
+
+int64_t rht_sum_count(int64_t n)
+{
+    const int kb = ilog2(n);
+    if (kb <= kMaxTileBits) return 0;
+    int rem = kb - contiguous_bits(kb), r = 0;
+    for (; rem > 0; rem -= r) r = rows_of_pass(rem);
+    return r >= 4 ? n >> (r + kStridedCols) : 0;
+}
+
 // transform index bits [0, kb) of every aligned block of 2^kb elements of x[0..n); `thc`: quantisers at the ends
 typedef TransformEnds ThcEnds;
 
@@ -271,7 +288,7 @@ static hipError_t fwht_blocks(float *x, const void *sign, bool sign_packed, int6
     const bool plain = thc.plain();
     const bool ends_ok = plain || (vec16 && (n & 31) == 0 && (reinterpret_cast<uintptr_t>(thc.in_levels) & 15) == 0);
     TransformEnds first = thc, last = thc, none;
-    first.out_levels = nullptr; first.post_scale = nullptr; first.out_dst = nullptr;
+    first.out_levels = nullptr; first.post_scale = nullptr; first.out_dst = nullptr; first.sums = nullptr;
     last.in_levels = nullptr; last.in_planes = nullptr; last.in_src = nullptr;
     // the diagonal belongs to the first pass of a forward transform and to the last of an inverse one
     if (inverse) first.gen = SignSeed();
@@ -310,12 +327,8 @@ static hipError_t fwht_blocks(float *x, const void *sign, bool sign_packed, int6
     a.in_levels = nullptr;
     a.in_planes = nullptr;
     int s = kt;
-    const int max_rows = kMaxTileBits - kStridedCols;
     while (s < kb) {
-        // split the remaining bits evenly over as few passes as the LDS allows
-        const int rem = kb - s;
-        const int passes = (rem + max_rows - 1) / max_rows;
-        const int r = (rem + passes - 1) / passes;
+        const int r = rows_of_pass(kb - s);
         a.kt = r + kStridedCols; a.b0 = kStridedCols; a.b1 = kStridedCols + r;
         a.cbits = kStridedCols; a.sbits = s;
         const bool last_pass = (s + r == kb);
@@ -327,7 +340,7 @@ static hipError_t fwht_blocks(float *x, const void *sign, bool sign_packed, int6
         if (r >= 4 && ends_ok && (n & (((int64_t)1 << (s + r)) - 1)) == 0)
             e = launch_rht_strided(x, sign, sign_packed ? 1 : 0, n, r, s, scale, a.apply_scale, a.sign_mode, a.vec,
                                    last_pass ? last : none, stream);
-        else if (last_pass && (thc.out_dst || thc.gen.bits != 0 || thc.grid.kind != ThcGrid::POINTERS))
+        else if (last_pass && (thc.out_dst || thc.sums || thc.gen.bits != 0 || thc.grid.kind != ThcGrid::POINTERS))
             e = hipErrorInvalidValue; // (not reached: see above and launch_rht_ends)
         else
             e = launch_tile(a, n >> a.kt, stream);
@@ -346,19 +359,20 @@ hipError_t launch_rht_ends(float *x, const void *sign, bool sign_packed, int64_t
                             (sign_packed ? 0 : reinterpret_cast<uintptr_t>(sign));
     if (block < 1024 || n % block != 0 || (every & 15) != 0) return hipErrorInvalidValue;
     // (the strided pass of 256 or 1024 rows behind the first pass is the one that draws)
+    if (ends.sums && (block != n || rht_sum_count(n) == 0)) return hipErrorInvalidValue;
     if (ends.draw.bits >= 0 && (block < kDrawsFrom || block > kDrawsTo || block != n)) return hipErrorInvalidValue;
     return fwht_blocks(x, sign, sign_packed, n, ilog2(block), scale, 1, inverse, stream, ends);
 }
 
 // The longest vector's contiguous pass sets the tile; a shorter one leaves at least four bits to its strided pass.
-hipError_t launch_rht_slices(const TransformSlice *slices, int count, int inverse, hipStream_t stream)
+hipError_t launch_rht_slices(TransformSlice *slices, int count, int inverse, hipStream_t stream)
 {
     TilePass tiles[kMaxEdenSlices], strided[kMaxEdenSlices];
     if (count < 1 || count > kMaxEdenSlices) return hipErrorInvalidValue;
     int most = 10;
     for (int k = 0; k < count; k++) most = std::max(most, contiguous_bits(ilog2(slices[k].n)));
     for (int k = 0; k < count; k++) {
-        const TransformSlice &s = slices[k];
+        TransformSlice &s = slices[k];
         const int kb = ilog2(s.n), kt = std::min(most, kb - 4);
         if (kb < 14 || kb > 22) return hipErrorInvalidValue;
         TilePass &t = tiles[k], &r = strided[k];
@@ -371,7 +385,8 @@ hipError_t launch_rht_slices(const TransformSlice *slices, int count, int invers
         r.sign_mode = inverse ? 2 : 0; r.apply_scale = 1;
         // the ends of the vector go with the pass that works on them, and so does the diagonal
         t.ends = r.ends = s.ends;
-        t.ends.out_dst = nullptr; t.ends.out_levels = nullptr; t.ends.post_scale = nullptr;
+        t.ends.out_dst = nullptr; t.ends.out_levels = nullptr; t.ends.post_scale = nullptr; t.ends.sums = nullptr;
+        s.sum_count = s.ends.sums ? s.n >> (r.rbits + kStridedCols) : 0;
         r.ends.in_src = nullptr; r.ends.in_levels = nullptr; r.ends.in_planes = nullptr;
         (inverse ? t : r).ends.gen = SignSeed();
     }

@@ -201,7 +201,7 @@ struct TransformEnds {
     // the diagonal drawn in the kernels instead of a sign vector
     SignSeed gen;
     bool plain_in() const { return !in_src && !in_levels && !in_planes; }
-    bool plain_out() const { return !out_dst && !out_levels && !post_scale; }
+    bool plain_out() const { return !out_dst && !out_levels && !post_scale && !sums; }
     bool plain() const { return plain_in() && plain_out() && gen.bits == 0; }
 
     // THC: the pass loads float(level) * *in_step + *in_lo instead of x
@@ -217,7 +217,12 @@ struct TransformEnds {
     const float *in_centroids = nullptr;
     int in_nbits = 0;
     const float *post_scale = nullptr;
+    // EDEN: a strided last pass also leaves, in double, the sum of the squares of the values that its workgroup w stores in
+    // sums[w] (rht_sum_count of them)
+    double *sums = nullptr;
 };
+// workgroups of the last pass of a whole-vector transform by launch_rht_ends; 0: that pass knows no sums
+int64_t rht_sum_count(int64_t n);
 
 hipError_t launch_rht_tile(float *x, const void *sign, int sign_bits, int64_t n, int kt, int kb, float scale, int apply_scale,
                            int sign_mode, int vec, const TransformEnds &ends, hipStream_t stream);
@@ -232,8 +237,9 @@ struct TransformSlice {
     int64_t n;
     float scale;
     TransformEnds ends;
+    int64_t sum_count = 0; // set by the call: how many of ends.sums it leaves
 };
-hipError_t launch_rht_slices(const TransformSlice *slices, int count, int inverse, hipStream_t stream);
+hipError_t launch_rht_slices(TransformSlice *slices, int count, int inverse, hipStream_t stream);
 // the two launches behind it: pass k owns the workgroups from `first` on
 struct TilePass {
     float *x;
@@ -255,7 +261,9 @@ struct QuantizeSlice {
     uint32_t *packed;
     float *result;
     double *work;
-    float sqrt_n;
+    const double *sums = nullptr; // partial sums of the squares, if some pass has left them already
+    int64_t sum_count = 0;
+    float sqrt_n = 0.0f;
 };
 int64_t eden_work_doubles(int64_t n);
 hipError_t launch_eden_quantize(const float *vec, int64_t n, const float *boundaries, const float *centroids,

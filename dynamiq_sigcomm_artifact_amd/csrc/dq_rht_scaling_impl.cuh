@@ -770,6 +770,29 @@ template <int B> __device__ __forceinline__ void draw_rows(float (&u)[1 << B], c
     }
 }
 
+// the sum over the wave's active lanes (64, or the first 32 of a workgroup of 32)
+__device__ __forceinline__ double wave_sum_f64(double x)
+{
+    const auto add_from = [&](auto ctrl) {
+        const uint64_t b = (uint64_t)__double_as_longlong(x);
+        const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, decltype(ctrl)::value, 0xf, 0xf, true);
+        const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), decltype(ctrl)::value, 0xf, 0xf, true);
+        x += __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+    };
+    add_from(std::integral_constant<int, 0xB1>());  // quad_perm [1,0,3,2]
+    add_from(std::integral_constant<int, 0x4E>());  // quad_perm [2,3,0,1]
+    add_from(std::integral_constant<int, 0x141>()); // row_half_mirror
+    add_from(std::integral_constant<int, 0x140>()); // row_mirror
+    const uint64_t b = (uint64_t)__double_as_longlong(x);
+    const auto of_row = [&](int lane) {
+        const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)b, lane), hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), lane);
+        return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+    };
+    double sum = of_row(0) + of_row(16);
+    if (blockDim.x > 32) sum += of_row(32) + of_row(48);
+    return sum;
+}
+
 // A later pass of a transform longer than one tile: index bits [sbits, sbits + A + B) of the vector.  A tile is 2^(A + B)
 // rows of 32 consecutive floats (128 bytes), row stride 2^sbits elements.  A thread owns column tid % 32 of 2^A consecutive
 // rows: it loads them (every load instruction of a wave covers two whole 128-byte row segments), does the A lowest row
@@ -781,6 +804,8 @@ template <int B> __device__ __forceinline__ void draw_rows(float (&u)[1 << B], c
 // levels 19.0 -> 17.8 (67 MB read); both directions of THC on 25 MB 82.6 -> 70.2, on 16,000,000 elements 146.7 -> 118.7, EDEN on
 // 500,000 36.5 -> 31.7, on 12,000,000 157 -> 136 (with the first pass below).
 // sign_mode: 0, or 2 = flip on store (the last pass of an inverse).
+// e.sums: the sum of the squares of what the workgroup stores, in double (each square is exact there): EDEN's norm without a pass
+// over the vector for it, 3.1 us of 34 at 2^20 elements, 12 of 137 at 2^24.
 template <bool ENDS, int A, int B>
 __device__ __forceinline__ void strided_rows(float *__restrict__ x, const PassArgs<ENDS> &a, int sbits, int sign_mode, int apply_scale,
                                              const TransformEnds &e, unsigned block, float *lds)
@@ -827,8 +852,8 @@ __device__ __forceinline__ void strided_rows(float *__restrict__ x, const PassAr
             for (int j = 0; j < R1; j++) lds[((group << A) + j) * 32 + col] = v[j];
         }
         __syncthreads();
-        if (!mine) return;
     }
+    double squares = 0.0;
     const bool flips = sign_mode == 2;
     bool drawn = false;
     if constexpr (ENDS) drawn = flips && a.gen.bits != 0;
@@ -921,11 +946,15 @@ __device__ __forceinline__ void strided_rows(float *__restrict__ x, const PassAr
         } else {
 #pragma unroll
             for (int i = 0; i < R2; i++) x[first + ((int64_t)i << (A + sbits))] = w[i];
+            if (ENDS && e.sums) {
+#pragma unroll
+                for (int i = 0; i < R2; i++) squares = __builtin_fma((double)w[i], (double)w[i], squares); // (the square is exact)
+            }
         }
     };
     if constexpr (B > 0) {
 #pragma unroll 1
-        for (int row = group; row < R1; row += R2) {
+        for (int row = mine ? group : R1; row < R1; row += R2) {
             float w[R2];
 #pragma unroll
             for (int i = 0; i < R2; i++) w[i] = lds[((i << A) + row) * 32 + col];
@@ -937,6 +966,20 @@ __device__ __forceinline__ void strided_rows(float *__restrict__ x, const PassAr
         for (int j = 0; j < R1; j++) {
             float w[1] = {v[j]};
             finish(w, j);
+        }
+    }
+    if constexpr (ENDS) {
+        if (e.sums) {
+            const double sum = wave_sum_f64(squares);
+            double *part = reinterpret_cast<double *>(lds);
+            if (B > 0) __syncthreads(); // the rows have been read
+            if ((tid & 63) == 0) part[tid >> 6] = sum;
+            __syncthreads();
+            if (tid == 0) {
+                double all = part[0];
+                for (int w = 1; w < (int)(blockDim.x + 63) / 64; w++) all += part[w];
+                e.sums[block] = all;
+            }
         }
     }
 }
@@ -1015,7 +1058,8 @@ __global__ __launch_bounds__(1024) void rht_tile_passes_kernel(PassSet set)
 __global__ __launch_bounds__(512) void rht_strided_passes_kernel(PassSet set)
 {
     extern __shared__ __attribute__((aligned(16))) float lds[];
-    const TilePass &p = pass_of_block(set);
+    // (a copy: by reference the five bodies use the argument in so many places that the compiler copies all of it to scratch)
+    const TilePass p = pass_of_block(set);
     strided_pass<true>(p.x, pass_args(p), p.rbits, p.sbits, p.sign_mode, p.apply_scale, p.ends, blockIdx.x - p.first, lds);
 }
 #endif

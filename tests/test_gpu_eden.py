@@ -489,6 +489,35 @@ def test_slices_in_one_call_equal_the_single_calls(capi, n, dt):
     assert got.dtype == dt and torch.equal(got, torch.cat(want))
 
 
+@pytest.mark.parametrize("sizes", [(1 << 14, 1 << 15), (1 << 14, 1 << 18, 1 << 22), (1 << 17,), (1 << 19, 1 << 14), (1 << 21, 1 << 20),
+                                   (1 << 23,), (1 << 24,), (1 << 25,), (1 << 26,)])
+def test_scale_from_the_sums_of_the_last_pass(sizes):
+    """EDEN's scale is (norm * norm) / dot of float32s, and the sum of squares behind the norm comes out of the last pass of the
+    rotation: for every number of rows of that pass (16 ones beside longer slices, up to 1024, and 64 behind another strided
+    pass) against the exact sums of the rotated values.  Three roundings to float32 of sums in double: 2^-22."""
+    import math
+    from dynamiq_sigcomm_artifact_amd import capi
+    from dynamiq_sigcomm_artifact_amd.eden import Eden
+    dev, nbits, seed = "cuda:0", 4, 5
+    eden = Eden(device=dev)
+    vec = torch.randn(sum(sizes), generator=torch.Generator(device=dev).manual_seed(1), device=dev) * 1e-2
+    centroids, boundaries = eden._tables(nbits)
+    slices, at = [], 0
+    for n in sizes:
+        slices.append((at, n, n, 1))
+        at += n
+    parts = capi.host().eden_compress(vec, boundaries, centroids, nbits, seed, slices)
+    for (packed, scale), (at, n, _, _) in zip(parts, slices):
+        x = vec[at:at + n].clone()
+        diag = torch.empty(n, device=dev)
+        capi.rand_diag(diag, seed)
+        capi.rht_blocked(x, diag, n, float(np.float32(1.0) / np.float32(math.sqrt(n))), False)
+        bins = eden.EdenBitsToBins(packed, nbits).to(torch.int64)
+        exact = x.double()
+        want = (exact * exact).sum() / (centroids[bins].double() * exact).sum()
+        assert abs(float(scale) / float(want) - 1.0) < 2.0 ** -22, (n, float(scale), float(want))
+
+
 @pytest.mark.parametrize("seed", [2 ** 63 + 5, -(2 ** 63), 2 ** 70 + 9, 2 ** 64 - 1])
 def test_seeds_of_any_size(capi, seed):
     """a seed is taken modulo 2^64, as the single calls take it; one that is no whole number is refused"""
