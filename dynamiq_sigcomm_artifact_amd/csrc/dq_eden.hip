@@ -71,11 +71,16 @@ __global__ __launch_bounds__(kEdenThreads) void eden_sumsq_kernel(QuantizeSet se
 }
 
 // folds work[0 .. count): thread t adds entries t + 256 k (k ascending), then the halving tree
+__device__ __forceinline__ double fold_array(const double *work, int64_t count, double *lds, double acc)
+{
+    for (int64_t i = threadIdx.x + kEdenThreads; i < count; i += kEdenThreads) acc += work[i];
+    return fold256(acc, lds, threadIdx.x);
+}
+// (the thread's first entry may be asked for earlier)
+__device__ __forceinline__ double first_of_array(const double *work, int64_t count) { return threadIdx.x < count ? work[threadIdx.x] : 0.0; }
 __device__ __forceinline__ double fold_array(const double *work, int64_t count, double *lds)
 {
-    double acc = 0.0;
-    for (int64_t i = threadIdx.x; i < count; i += kEdenThreads) acc += work[i];
-    return fold256(acc, lds, threadIdx.x);
+    return fold_array(work, count, lds, first_of_array(work, count));
 }
 
 // result[0] = (float)sumsq, result[3] = norm
@@ -127,11 +132,12 @@ __global__ __launch_bounds__(kEdenThreads) void eden_bins_kernel(QuantizeSet set
 #pragma unroll
         for (int k = 0; k < kEdenPerThread; k++) v[k] = 0.0f;
     }
+    const double part = FOLD ? first_of_array(s.sums, s.sum_count) : 0.0;
     eden_tables<NBITS>(boundaries, centroids, tree, cen, threadIdx.x, kEdenThreads);
     __syncthreads();
     float norm;
     if constexpr (FOLD) {
-        const float sum = (float)fold_array(s.sums, s.sum_count, lds);
+        const float sum = (float)fold_array(s.sums, s.sum_count, lds, part);
         norm = __builtin_sqrtf(sum);
         if (tile == 0 && threadIdx.x == 0) {
             s.result[0] = sum;

@@ -68,20 +68,27 @@ struct RhtPassArgs : RhtTileArgs {
 template <bool ENDS> using PassArgs = typename std::conditional<ENDS, RhtPassArgs, RhtTileArgs>::type;
 
 // Element g of the diagonal of rand_diag (srrcomp.py:61-106; rand_diag_word of dq_hadamard.hip in 32-bit arithmetic: only
-// the low word of every product is used, and the one carry that is, of the addition, is added back by hand).  Four
-// multiplications at a quarter of the rate, about 25 instruction slots per element: cheaper than a launch that writes
-// the bits while the vector is short (the rule is in launch_eden_compress).
-__device__ __forceinline__ uint32_t rand_diag_column(const SignSeed &s, uint32_t j)
+// the low word of every product is used, and the one carry that is, of the addition, is added back by hand).  The two
+// congruential steps at its head are one affine function of the column, so the next column's state is an addition away: two
+// multiplications at a quarter of the rate are left, about 15 instruction slots per element (25 with four).  Cheaper than a
+// launch that writes the bits while the vector is short (the rule is in launch_eden_compress).
+constexpr uint32_t kDiagFirst = 1103515245u, kDiagSecond = 1140671485u, kDiagStep = kDiagFirst * kDiagSecond;
+
+__device__ __forceinline__ uint32_t rand_diag_state(const SignSeed &s, uint32_t j)
 {
-    uint32_t r = j + s.ss;
-    r = 1103515245u * r + 12345u + s.ss;
-    r = 1140671485u * r + 12820163u + s.ss;
+    return kDiagStep * j + (kDiagSecond * (kDiagFirst * s.ss + 12345u + s.ss) + 12820163u + s.ss);
+}
+
+__device__ __forceinline__ uint32_t rand_diag_mix(uint32_t r)
+{
     const uint32_t q = r + 0x9e3779b9u;
     const uint32_t carry = q < r ? 0x10000u : 0u;
     r = (q ^ ((q >> 16) | carry)) * 0x85ebca6bu;
     r = (r ^ (r >> 13)) * 0xc2b2ae35u;
     return r ^ (r >> 16);
 }
+
+__device__ __forceinline__ uint32_t rand_diag_column(const SignSeed &s, uint32_t j) { return rand_diag_mix(rand_diag_state(s, j)); }
 
 // the sign bit of element j of segment k: +1 where the nibble is >= 8
 __device__ __forceinline__ uint32_t nibble_negative(uint32_t r, uint32_t k) { return ~(r << (28 - 4 * k)) & 0x80000000u; }
@@ -112,10 +119,11 @@ __device__ __forceinline__ void flip4(float4 &v, const RhtPassArgs &a, int64_t g
 {
     if (a.gen.bits != 0) {
         const uint32_t k = (uint32_t)(g >> a.gen.bits), j = (uint32_t)g & ((1u << a.gen.bits) - 1u); // the four share a segment
-        v.x = __uint_as_float(__float_as_uint(v.x) ^ rand_diag_negative(a.gen, k, j));
-        v.y = __uint_as_float(__float_as_uint(v.y) ^ rand_diag_negative(a.gen, k, j + 1));
-        v.z = __uint_as_float(__float_as_uint(v.z) ^ rand_diag_negative(a.gen, k, j + 2));
-        v.w = __uint_as_float(__float_as_uint(v.w) ^ rand_diag_negative(a.gen, k, j + 3));
+        const uint32_t r = rand_diag_state(a.gen, j);
+        v.x = __uint_as_float(__float_as_uint(v.x) ^ nibble_negative(rand_diag_mix(r), k));
+        v.y = __uint_as_float(__float_as_uint(v.y) ^ nibble_negative(rand_diag_mix(r + kDiagStep), k));
+        v.z = __uint_as_float(__float_as_uint(v.z) ^ nibble_negative(rand_diag_mix(r + 2 * kDiagStep), k));
+        v.w = __uint_as_float(__float_as_uint(v.w) ^ nibble_negative(rand_diag_mix(r + 3 * kDiagStep), k));
         return;
     }
     flip4(v, static_cast<const RhtTileArgs &>(a), g);
@@ -451,11 +459,16 @@ __device__ __forceinline__ void store_destination(const TransformEnds &e, float4
 __device__ __forceinline__ void load_planes(float (&v)[16], const TransformEnds &e, const float *cen, int64_t g, int64_t words)
 {
     const uint16_t *half = reinterpret_cast<const uint16_t *>(e.in_planes) + (g >> 4);
+    // (eight loads whatever the width, the last plane's again: in a loop over the planes they wait for one another)
+    uint32_t h[8];
+#pragma unroll
+    for (int p = 0; p < 8; p++) h[p] = half[(int64_t)min(p, e.in_nbits - 1) * words * 2];
     uint64_t lo8 = 0, hi8 = 0;
-    for (int p = 0; p < e.in_nbits; p++) {
-        const uint32_t h = half[(int64_t)p * words * 2];
-        lo8 |= (uint64_t)(h & 0xffu) << (8 * p);
-        hi8 |= (uint64_t)(h >> 8) << (8 * p);
+#pragma unroll
+    for (int p = 0; p < 8; p++) {
+        const uint32_t w = p < e.in_nbits ? h[p] : 0u;
+        lo8 |= (uint64_t)(w & 0xffu) << (8 * p);
+        hi8 |= (uint64_t)(w >> 8) << (8 * p);
     }
     lo8 = transpose8x8(lo8);
     hi8 = transpose8x8(hi8);
