@@ -941,6 +941,11 @@ __device__ __forceinline__ void strided_rows(float *__restrict__ x, const PassAr
             const int64_t whole = ((e.out_count - 32 - origin - ((int64_t)last_row << sbits)) >> (A + sbits)) + 1;
             const int rows = (int)min(whole, (int64_t)R2);
             const auto store = [&](auto *out, auto convert) {
+                if (rows == R2) {
+#pragma unroll
+                    for (int i = 0; i < R2; i++) out[first + ((int64_t)i << (A + sbits))] = convert(w[i]);
+                    return;
+                }
 #pragma unroll
                 for (int i = 0; i < R2; i++) {
                     const int64_t g = first + ((int64_t)i << (A + sbits));
@@ -984,19 +989,19 @@ __device__ __forceinline__ void strided_rows(float *__restrict__ x, const PassAr
     if constexpr (ENDS) {
         if (e.sums) {
             const double sum = wave_sum_f64(squares);
-            double *part = reinterpret_cast<double *>(lds);
-            if (B > 0) __syncthreads(); // the rows have been read
+            double *part = reinterpret_cast<double *>(lds + (32 << (A + B))); // (behind the tile: strided_lds_bytes)
             if ((tid & 63) == 0) part[tid >> 6] = sum;
             __syncthreads();
-            if (tid == 0) {
-                double all = part[0];
-                for (int w = 1; w < (int)(blockDim.x + 63) / 64; w++) all += part[w];
-                e.sums[block] = all;
+            if (tid < 64) {
+                const double all = wave_sum_f64(tid < (int)(blockDim.x + 63) / 64 ? part[tid] : 0.0);
+                if (tid == 0) e.sums[block] = all;
             }
         }
     }
 }
 
+// a tile, and a double for each of up to sixteen waves
+__host__ constexpr size_t strided_lds_bytes(int rbits) { return (sizeof(float) << (rbits + 5)) + 16 * sizeof(double); }
 // threads of the tile of a strided pass
 __host__ __device__ constexpr int strided_threads(int rbits) { return rbits >= 9 ? 1 << rbits : 1 << (rbits + 1); }
 
@@ -1045,8 +1050,11 @@ struct PassSet {
     int count;
 };
 
-__device__ __forceinline__ const TilePass &pass_of_block(const PassSet &set)
+// The set, the kernel's only argument, where it lies: by name, in more than a few hundred places, the compiler copies all 2 KB
+// of it to scratch in front of the kernel, and a copy of one pass costs 0.5 us of loads that wait for one another.
+__device__ __forceinline__ const TilePass &pass_of_block()
 {
+    const PassSet &set = *(const PassSet *)(const __attribute__((address_space(4))) PassSet *)__builtin_amdgcn_kernarg_segment_ptr();
     int k = 0;
     for (int i = 1; i < set.count; i++)
         if (blockIdx.x >= set.p[i].first) k = i;
@@ -1064,15 +1072,14 @@ __device__ __forceinline__ RhtPassArgs pass_args(const TilePass &p)
 __global__ __launch_bounds__(1024) void rht_tile_passes_kernel(PassSet set)
 {
     extern __shared__ __attribute__((aligned(16))) float lds[];
-    const TilePass &p = pass_of_block(set);
+    const TilePass &p = pass_of_block();
     first_pass<true>(p.x, pass_args(p), p.sign_mode, p.ends, blockIdx.x - p.first, lds);
 }
 
 __global__ __launch_bounds__(512) void rht_strided_passes_kernel(PassSet set)
 {
     extern __shared__ __attribute__((aligned(16))) float lds[];
-    // (a copy: by reference the five bodies use the argument in so many places that the compiler copies all of it to scratch)
-    const TilePass p = pass_of_block(set);
+    const TilePass &p = pass_of_block();
     strided_pass<true>(p.x, pass_args(p), p.rbits, p.sbits, p.sign_mode, p.apply_scale, p.ends, blockIdx.x - p.first, lds);
 }
 #endif
@@ -1558,7 +1565,7 @@ hipError_t launch_rht_strided(float *x, const void *sign, int sign_bits, int64_t
     a.sign = sign; a.sign_bits = sign_bits; a.n = n; a.kt = rbits + 5; a.kb = 0; a.scale = scale; a.vec = vec; a.gen = ends.gen;
     const RhtTileArgs &plain_args = a;
     const dim3 grid((unsigned)(n >> (rbits + 5))), block((unsigned)strided_threads(rbits));
-    const size_t lds = sizeof(float) << (rbits + 5);
+    const size_t lds = strided_lds_bytes(rbits);
     const auto launch = [&](auto kernel, const auto &args, auto... bits) -> hipError_t {
         const hipError_t e = allow_lds(kernel, lds);
         if (e != hipSuccess) return e;
@@ -1613,7 +1620,7 @@ hipError_t launch_rht_strided_passes(const TilePass *passes, int count, hipStrea
         blocks += (unsigned)(passes[k].n >> (passes[k].rbits + 5));
         most = std::max(most, passes[k].rbits);
     }
-    const size_t lds = sizeof(float) << (most + 5);
+    const size_t lds = strided_lds_bytes(most);
     const hipError_t e = allow_lds(rht_strided_passes_kernel, lds);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(rht_strided_passes_kernel, dim3(blocks), dim3((unsigned)strided_threads(most)), lds, stream, set);
