@@ -338,45 +338,78 @@ struct RankPointers {
 };
 
 constexpr int kStatsWaves = 8; // ranks in flight per workgroup of ranks_stats_kernel
-// From so many tiles (of all ranks) on a wave takes two of a rank and has both on their way before it adds up the first: 454 ->
-// 409 us for 8 x 121,524 tiles.  Below, the second tile is better in a wave of its own: 8.2 -> 8.8 us for 2 x 6,400 (the whole
-// all-reduce of 4 x 15,625: 72.2 -> 73.6 us; of 8 x 15,625 135.5 -> 134.3, about where the two meet).
-constexpr int64_t kStatsTwoTiles = (int64_t)1 << 17;
-
-// A workgroup takes TILES tiles of four superchunks, a wave of it the tiles of one rank (of every kStatsWaves-th one in a larger
+// A workgroup takes GROUPS tiles of four superchunks, a wave of it those of one rank (of every kStatsWaves-th one in a larger
 // world): means and norms per rank, and the statistics all-reduce as the reference's chain of bf16 additions in rank order.
-template <int DT, int TILES>
-__global__ __launch_bounds__(64 * kStatsWaves) void ranks_stats_kernel(RankPointers ranks, int world, int64_t n, int vec,
-                                                                      uint32_t *__restrict__ total, float *__restrict__ mean_out,
-                                                                      WorldDiv wd)
+// Bound by how much is on the way: a wave that adds up what it has just waited for, and then waits at the barrier for the
+// other ranks, asks for nothing meanwhile.  So it has the next tile of its rank on the way while it adds up the current one,
+// and meets the others once in GROUPS tiles.  The tiles come as whole lines (a tile goes through LDS anyway).  NT: loads that
+// leave the caches to others.
+template <int DT, int GROUPS, bool NT>
+__global__ __launch_bounds__(64 * kStatsWaves, 8) void ranks_stats_kernel(RankPointers ranks, int world, int64_t n, int vec,
+                                                                         uint32_t *__restrict__ total, float *__restrict__ mean_out,
+                                                                         WorldDiv wd)
 {
     extern __shared__ __attribute__((aligned(16))) uint8_t tiles[];
-    __shared__ uint32_t pairs[kMaxRanks][TILES * kRowsPerWave];
+    constexpr int kRows = GROUPS * kRowsPerWave;
+    __shared__ uint32_t pairs[kMaxRanks][kRows];
+    typedef StatsTile<DT> ST;
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    constexpr int kSlots = Raw16<DT>::kSlots, kRowBytes = 256 * ST::ESZ;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
     const int row = lane >> 4, j = lane & 15;
     const int64_t nsc = (n + 255) >> 8;
-    const int64_t sc0 = (int64_t)blockIdx.x * (TILES * kRowsPerWave);
-    const int rows_here = (int)min((int64_t)(TILES * kRowsPerWave), nsc - sc0);
-    const bool ragged = (sc0 + TILES * kRowsPerWave) * 256 > n;
-    uint8_t *lds = tiles + wave * StatsTile<DT>::BYTES;
-    const int64_t first = (sc0 + row) * 256;
-    for (int rank = wave; rank < world; rank += waves) {
-        Raw16<DT> v[TILES];
+    const int64_t sc0 = (int64_t)blockIdx.x * kRows;
+    const int rows_here = (int)min((int64_t)kRows, nsc - sc0);
+    uint8_t *lds = tiles + wave * ST::BYTES;
+    if (vec != 0 && (sc0 + kRows) * 256 <= n) {
+        for (int rank = wave; rank < world; rank += waves) {
+            const u32x4 *from = reinterpret_cast<const u32x4 *>(static_cast<const uint8_t *>(ranks.src[rank]) + sc0 * kRowBytes) + lane;
+            u32x4 q[2][kSlots];
 #pragma unroll
-        for (int t = 0; t < TILES; t++) {
-            v[t].zero();
-            if (t * kRowsPerWave + row < rows_here) load_chunk<DT>(v[t], ranks.src[rank], first + t * 1024 + j * 16, n, vec != 0, ragged);
+            for (int k = 0; k < kSlots; k++) q[0][k] = NT ? __builtin_nontemporal_load(from + k * 64) : from[k * 64];
+#pragma unroll
+            for (int g = 0; g < GROUPS; g++) {
+                if (g + 1 < GROUPS) {
+#pragma unroll
+                    for (int k = 0; k < kSlots; k++) {
+                        const u32x4 *next = from + ((g + 1) * kSlots + k) * 64;
+                        q[(g + 1) & 1][k] = NT ? __builtin_nontemporal_load(next) : *next;
+                    }
+                }
+                const int r = g * kRowsPerWave + row;
+#pragma unroll
+                for (int k = 0; k < kSlots; k++) {
+                    const int at = k * 1024 + lane * 16;
+                    *reinterpret_cast<u32x4 *>(lds + (at / kRowBytes) * ST::RS + at % kRowBytes) = q[g & 1][k];
+                }
+                wave_lds_sync();
+                float sum, sq;
+                staged_tile_sums<DT>(wd, lds, lane, sum, sq);
+                wave_lds_sync();
+                if (j == 0) {
+                    const float mean = sum * 0.00390625f;
+                    pairs[rank][r] = f32_to_bf16_bits(mean) | (f32_to_bf16_bits(sq) << 16);
+                    mean_out[rank * nsc + sc0 + r] = mean;
+                }
+            }
         }
-#pragma unroll
-        for (int t = 0; t < TILES; t++) {
-            const int r = t * kRowsPerWave + row;
-            float sum, sq;
-            tile_sums<DT>(v[t], wd, lds, lane, sum, sq);
-            wave_lds_sync();
-            if (j == 0) {
-                const float mean = superchunk_mean(sum, first + t * 1024, n, ragged);
-                pairs[rank][r] = f32_to_bf16_bits(mean) | (f32_to_bf16_bits(sq) << 16);
-                if (r < rows_here) mean_out[rank * nsc + sc0 + r] = mean;
+    } else {
+        for (int rank = wave; rank < world; rank += waves) {
+            for (int g = 0; g * kRowsPerWave < rows_here; g++) {
+                const int r = g * kRowsPerWave + row;
+                const int64_t first = (sc0 + r) * 256;
+                const bool ragged = (sc0 + (g + 1) * kRowsPerWave) * 256 > n;
+                Raw16<DT> v;
+                v.zero();
+                if (r < rows_here) load_chunk<DT>(v, ranks.src[rank], first + j * 16, n, vec != 0, ragged);
+                float sum, sq;
+                tile_sums<DT>(v, wd, lds, lane, sum, sq);
+                wave_lds_sync();
+                if (j == 0 && r < rows_here) {
+                    const float mean = superchunk_mean(sum, first, n, ragged);
+                    pairs[rank][r] = f32_to_bf16_bits(mean) | (f32_to_bf16_bits(sq) << 16);
+                    mean_out[rank * nsc + sc0 + r] = mean;
+                }
             }
         }
     }
@@ -682,6 +715,13 @@ hipError_t launch_roundtrip(const RoundtripDesc *desc, int count, int world, flo
     return hipGetLastError();
 }
 
+// ranks_stats_kernel, us, a tile per wave -> four -> eight (-> eight that pass the caches by): 2 ranks x 6,400 tiles 7.0 -> 6.8 -> 8.3
+// (9.3), 8 x 1,954 7.8 -> 8.2 -> 8.6, 8 x 3,907 14.4 -> 12.9 -> 12.9 (12.8), 8 x 15,625 42.5 -> 39.4 -> 39.6 (39.4), 8 x 32,227 110 ->
+// 102 -> 106 (82), 8 x 121,524 425 -> 375 (324).  The ring that follows reads the vectors again: out of the cache behind the L2
+// (256 MB) if they are there, which loads that pass it by cost 10 us at 8 x 15,625 and nothing at 8 x 32,227.  Both launches,
+// keeping -> passing by: 280 MB 147 -> 151, 320 MB 168 -> 170, 384 MB 215 -> 205.
+constexpr int64_t kStatsOneTile = (int64_t)1 << 14, kStatsCache = (int64_t)300 << 20;
+
 hipError_t launch_ranks_stats(const void *const *src, int world, int64_t n, void *total, float *mean, int dtype, hipStream_t stream)
 {
     RankPointers p;
@@ -691,22 +731,22 @@ hipError_t launch_ranks_stats(const void *const *src, int world, int64_t n, void
         if (r < world && !aligned16(src[r])) vec = 0;
     }
     const int64_t nsc = (n + 255) / 256;
-    const int64_t one = (nsc + kRowsPerWave - 1) / kRowsPerWave;
-    const bool two = one * world >= kStatsTwoTiles;
-    const dim3 grid((unsigned)(two ? (one + 1) / 2 : one));
+    const int64_t tiles = (nsc + kRowsPerWave - 1) / kRowsPerWave;
     const int waves = world < kStatsWaves ? world : kStatsWaves;
     const WorldDiv wd = make_world_div(world, dtype == DQ_F32 ? 4 : 2);
     uint32_t *tot = static_cast<uint32_t *>(total);
-    const dim3 block(64 * waves);
-    if (dtype == DQ_BF16) {
-        const size_t lds = waves * StatsTile<DQ_BF16>::BYTES;
-        if (two) hipLaunchKernelGGL((ranks_stats_kernel<DQ_BF16, 2>), grid, block, lds, stream, p, world, n, vec, tot, mean, wd);
-        else hipLaunchKernelGGL((ranks_stats_kernel<DQ_BF16, 1>), grid, block, lds, stream, p, world, n, vec, tot, mean, wd);
-    } else {
-        const size_t lds = waves * StatsTile<DQ_F32>::BYTES;
-        if (two) hipLaunchKernelGGL((ranks_stats_kernel<DQ_F32, 2>), grid, block, lds, stream, p, world, n, vec, tot, mean, wd);
-        else hipLaunchKernelGGL((ranks_stats_kernel<DQ_F32, 1>), grid, block, lds, stream, p, world, n, vec, tot, mean, wd);
-    }
+    const auto run = [&](auto type, auto groups, auto nt) {
+        constexpr int DT = decltype(type)::value, G = decltype(groups)::value;
+        hipLaunchKernelGGL((ranks_stats_kernel<DT, G, decltype(nt)::value>), dim3((unsigned)((tiles + G - 1) / G)), dim3(64 * waves),
+                           waves * StatsTile<DT>::BYTES, stream, p, world, n, vec, tot, mean, wd);
+    };
+    const auto launch = [&](auto type) {
+        if (tiles * world * StatsTile<decltype(type)::value>::ESZ * 1024 > kStatsCache) run(type, std::integral_constant<int, 8>(), std::true_type());
+        else if (tiles * world > kStatsOneTile) run(type, std::integral_constant<int, 4>(), std::false_type());
+        else run(type, std::integral_constant<int, 1>(), std::false_type());
+    };
+    if (dtype == DQ_BF16) launch(std::integral_constant<int, DQ_BF16>());
+    else launch(std::integral_constant<int, DQ_F32>());
     return hipGetLastError();
 }
 

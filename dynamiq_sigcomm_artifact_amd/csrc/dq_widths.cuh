@@ -432,6 +432,8 @@ template <int DT> struct StatsTile {
 // lane (row r, column j) holds elements j + 16 k of superchunk r -- strides 128 .. 16 are then additions in the lane,
 // strides 8 .. 1 row shifts.  lds: StatsTile<DT>::BYTES, 16-byte aligned, owned by this wave.  sum and sq are complete in
 // the lanes j == 0.
+template <int DT> __device__ __forceinline__ void staged_tile_sums(const WorldDiv &wd, const uint8_t *lds, int lane, float &sum, float &sq);
+
 template <int DT>
 __device__ __forceinline__ void tile_sums(const Raw16<DT> &v, const WorldDiv &wd, uint8_t *lds, int lane, float &sum, float &sq)
 {
@@ -441,6 +443,14 @@ __device__ __forceinline__ void tile_sums(const Raw16<DT> &v, const WorldDiv &wd
     for (int k = 0; k < Raw16<DT>::kSlots; k++)
         *reinterpret_cast<uint4 *>(lds + row * ST::RS + j * 16 * ST::ESZ + 16 * k) = v.slot(k);
     wave_lds_sync();
+    staged_tile_sums<DT>(wd, lds, lane, sum, sq);
+}
+
+// of the tile in LDS
+template <int DT> __device__ __forceinline__ void staged_tile_sums(const WorldDiv &wd, const uint8_t *lds, int lane, float &sum, float &sq)
+{
+    typedef StatsTile<DT> ST;
+    const int row = lane >> 4, j = lane & 15;
     const uint8_t *mine = lds + row * ST::RS + j * ST::ESZ;
     float t[16];
 #pragma unroll

@@ -716,6 +716,38 @@ def test_ranks_on_either_side_of_a_superchunk_per_wave(capi, W, n):
     test_ranks_in_registers_equal_the_ring_in_steps(capi, W, n, torch.bfloat16)
 
 
+@pytest.mark.parametrize("W,n,dt,offset", [
+    (8, 1024 * 2048, torch.bfloat16, 0),           # the last length with a tile per wave of the statistics
+    (8, 1024 * 2048 + 1, torch.bfloat16, 0),       # four tiles per wave; one element in the last of them
+    (3, 1024 * 5464 - 255, torch.float32, 0),
+    (3, 1024 * 5465, torch.bfloat16, 1),           # vectors off the 16 bytes
+    (9, 1024 * 4 * 500 + 256 * 7, torch.bfloat16, 0),
+    (8, 300 << 16, torch.bfloat16, 0),             # the last one that the cache is to keep
+    (8, (300 << 16) + 1024 * 9 + 300, torch.bfloat16, 0),
+    (4, (300 << 16) + 1024 * 3, torch.float32, 1),
+])
+def test_statistics_of_long_vectors(capi, W, n, dt, offset):
+    """the reduced statistics against the sums of the ranks' own in the element type, and the all-reduce behind them against the
+    ring in steps, which has its statistics from other kernels"""
+    from dynamiq_sigcomm_artifact_amd.dynamiq_pipeline import _single_pass_in_steps, dynamic_bitrate_allreduce_single_pass
+    g = torch.Generator(device=DEV).manual_seed(n + W)
+    vecs = []
+    for r in range(W):
+        x = torch.randn(n + offset, generator=g, device=DEV)
+        x.view(-1)[:n // 4096 * 4096].view(-1, 4096).mul_(torch.exp2(torch.randint(-9, 3, (n // 4096, 1), generator=g, device=DEV).float()))
+        vecs.append(x.to(dt)[offset:])
+        del x
+    outs, total, _ = dynamic_bitrate_allreduce_single_pass(vecs, 6.0, strategy=2, seed=3)
+    want = None
+    for v in vecs:
+        stats = torch.empty_like(total)
+        capi.superchunk_stats(v, stats, None, n, W)
+        want = stats if want is None else want + stats
+    assert torch.equal(bits_t(total), bits_t(want))
+    ref, _, _ = _single_pass_in_steps(vecs, 6.0, 2, 3, None, {}, None, None)
+    assert all(torch.equal(bits_t(x), bits_t(y)) for x, y in zip(outs, ref))
+
+
 @pytest.mark.parametrize("W", [1, 3])
 @pytest.mark.parametrize("elsewhere", [False, pytest.param(True, marks=pytest.mark.skipif(
     not torch.cuda.is_available() or torch.cuda.device_count() < 2, reason="needs a second GPU"))])
