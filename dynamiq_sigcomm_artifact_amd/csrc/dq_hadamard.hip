@@ -234,8 +234,9 @@ constexpr int kStridedCols = 5;   // 32 consecutive floats (128 B) per row of a 
 //   to 2^22     256 rows (32 KB), and the contiguous tiles grow with the vector
 //   to 2^25     1024 rows, the most that fit the LDS: anything less makes three passes of it from 2^24 on
 //   beyond      three passes in any case, 32 KB contiguous tiles
-// In place, against 2^13 everywhere: 2^18 9.1 -> 8.2 us, 2^19 10.0 -> 9.4, 2^22 27.3 -> 20.5, 2^24 65.3 -> 54.9,
-// 2^25 127 -> 112; 2^20, 2^21 and 2^23 keep theirs to within 2%.
+// In place, against 2^13 everywhere: 2^18 8.0 -> 6.6 us, 2^19 9.0 -> 7.6, 2^20 10.2 -> 9.4, 2^22 21.5 -> 18.7, 2^24 68.1 -> 54.1,
+// 2^25 127 -> 105; 2^21 and 2^23 keep theirs to within 1%.  (128 rows up to 2^20 or 2^21: EDEN there and back 28.5 -> 30.7 us,
+// 38.6 -> 40.5.)
 static int contiguous_bits(int kb)
 {
     if (kb <= 18) return kb - 7 < 10 ? 10 : kb - 7;
