@@ -73,11 +73,17 @@ __global__ __launch_bounds__(kEdenThreads) void eden_sumsq_kernel(QuantizeSet se
 // folds work[0 .. count): thread t adds entries t + 256 k (k ascending), then the halving tree
 __device__ __forceinline__ double fold_array(const double *work, int64_t count, double *lds, double acc)
 {
-    for (int64_t i = threadIdx.x + kEdenThreads; i < count; i += kEdenThreads) acc += work[i];
-    return fold256(acc, lds, threadIdx.x);
+    if (threadIdx.x < kEdenThreads) { // (of a workgroup with more)
+        for (int64_t i = threadIdx.x + kEdenThreads; i < count; i += kEdenThreads) acc += work[i];
+        lds[threadIdx.x] = acc;
+    }
+    return fold256_of(lds, threadIdx.x);
 }
 // (the thread's first entry may be asked for earlier)
-__device__ __forceinline__ double first_of_array(const double *work, int64_t count) { return threadIdx.x < count ? work[threadIdx.x] : 0.0; }
+__device__ __forceinline__ double first_of_array(const double *work, int64_t count)
+{
+    return threadIdx.x < kEdenThreads && threadIdx.x < count ? work[threadIdx.x] : 0.0;
+}
 __device__ __forceinline__ double fold_array(const double *work, int64_t count, double *lds)
 {
     return fold_array(work, count, lds, first_of_array(work, count));
@@ -96,14 +102,14 @@ __global__ __launch_bounds__(kEdenThreads) void eden_norm_kernel(const double *_
     }
 }
 
-// Every thread owns sixteen consecutive elements (four 16-byte loads), so that it builds its half word of every
-// bit plane in registers.
+// A thread owns PER = 8 or 16 consecutive elements, two or four 16-byte loads, so that it builds its byte or half word of every
+// bit plane in registers; the additions are the same in the same order.
 // FOLD: the norm is not in result[3] yet; the workgroup folds the partial sums in work[0 .. tiles) the way eden_norm_kernel
 // does (the same association: the same bits), workgroup 0 leaves result[0] and result[3] as that kernel would, and the
 // products go to a region of their own (other workgroups are still reading the sums).
-template <int NBITS, bool FOLD>
-__global__ __launch_bounds__(kEdenThreads) void eden_bins_kernel(QuantizeSet set, const float *__restrict__ boundaries,
-                                                                const float *__restrict__ centroids)
+template <int NBITS, bool FOLD, int PER>
+__global__ __launch_bounds__(kEdenTile / PER) void eden_bins_kernel(QuantizeSet set, const float *__restrict__ boundaries,
+                                                                   const float *__restrict__ centroids)
 {
     constexpr int L = 1 << NBITS;
     __shared__ double lds[kEdenThreads];
@@ -112,28 +118,28 @@ __global__ __launch_bounds__(kEdenThreads) void eden_bins_kernel(QuantizeSet set
     const QuantizeSlice &s = set.s[which];
     const int64_t tile = blockIdx.x - (FOLD ? set.first[which] : 0u);
     const int64_t tiles = eden_tiles(s.n);
-    // n is a multiple of 32: the sixteen elements are all inside the vector or all outside
-    const int64_t first = tile * kEdenTile + (int64_t)threadIdx.x * kEdenPerThread;
+    // n is a multiple of 32: the thread's elements are all inside the vector or all outside
+    const int64_t first = tile * kEdenTile + (int64_t)threadIdx.x * PER;
     const bool in = first < s.n;
-    float v[kEdenPerThread];
+    float v[PER];
     if (in) {
         const float *vec = s.vec;
         if ((reinterpret_cast<uintptr_t>(vec) & 15) == 0) { // uniform over the grid
 #pragma unroll
-            for (int q = 0; q < kEdenPerThread / 4; q++) {
+            for (int q = 0; q < PER / 4; q++) {
                 const float4 f = *reinterpret_cast<const float4 *>(vec + first + 4 * q);
                 v[4 * q] = f.x; v[4 * q + 1] = f.y; v[4 * q + 2] = f.z; v[4 * q + 3] = f.w;
             }
         } else {
 #pragma unroll
-            for (int k = 0; k < kEdenPerThread; k++) v[k] = vec[first + k];
+            for (int k = 0; k < PER; k++) v[k] = vec[first + k];
         }
     } else {
 #pragma unroll
-        for (int k = 0; k < kEdenPerThread; k++) v[k] = 0.0f;
+        for (int k = 0; k < PER; k++) v[k] = 0.0f;
     }
     const double part = FOLD ? first_of_array(s.sums, s.sum_count) : 0.0;
-    eden_tables<NBITS>(boundaries, centroids, tree, cen, threadIdx.x, kEdenThreads);
+    eden_tables<NBITS>(boundaries, centroids, tree, cen, threadIdx.x, kEdenTile / PER);
     __syncthreads();
     float norm;
     if constexpr (FOLD) {
@@ -147,9 +153,10 @@ __global__ __launch_bounds__(kEdenThreads) void eden_bins_kernel(QuantizeSet set
         norm = s.result[3];
     }
     // plane p, word (first >> 5), half (first >> 4) & 1; threads past the end hold zeros and drop their sum
-    uint16_t *half = in ? reinterpret_cast<uint16_t *>(s.packed) + (first >> 4) : nullptr;
-    const double acc = eden_bins16<NBITS>(v, norm, s.sqrt_n, tree, cen, half, s.n >> 5);
-    const double total = fold256(in ? acc : 0.0, lds, threadIdx.x);
+    uint8_t *piece = in ? reinterpret_cast<uint8_t *>(s.packed) + (first >> 3) : nullptr;
+    const double acc = eden_bins_of<NBITS, PER>(v, norm, s.sqrt_n, tree, cen, piece, s.n >> 5);
+    if (PER == 16 || (threadIdx.x & 1)) lds[threadIdx.x / (16 / PER)] = in ? acc : 0.0;
+    const double total = fold256_of(lds, threadIdx.x);
     if (threadIdx.x == 0) s.work[(FOLD && s.sums == s.work ? tiles : 0) + tile] = total;
 }
 
@@ -264,6 +271,11 @@ int64_t eden_work_doubles(int64_t n)
     return tiles <= kEdenFoldTiles ? 2 * tiles : tiles;
 }
 
+// Up to so many tiles the bins kernel has eight elements per thread, for twice the waves; beyond, the second table and fold per
+// element is what counts.  Sixteen -> eight, us, 4 bits: 2^18 elements 5.2 -> 4.8, 2^20 5.6 -> 5.0 (8 bits 6.8 -> 5.7), 2^22
+// 9.3 -> 9.2, 2^23 13.7 -> 13.4, 2^24 22.8 -> 23.4, 2^25 37.8 -> 42.5, 2^26 63.0 -> 72.9.
+constexpr int64_t kFewTiles = 2048;
+
 // slices of at most kEdenFoldTiles tiles, or one of any length; bits of an NBITS-wide code for all of them
 hipError_t launch_eden_quantize_slices(const QuantizeSlice *slices, int count, const float *boundaries, const float *centroids,
                                        int nbits, hipStream_t stream)
@@ -284,15 +296,18 @@ hipError_t launch_eden_quantize_slices(const QuantizeSlice *slices, int count, c
         blocks += eden_tiles(slices[k].n);
     }
     const bool fold = count > 1 || set.s[0].sum_count <= kEdenFoldTiles;
+    const bool few = fold && blocks <= kFewTiles;
     dim3 grid((unsigned)blocks), block(kEdenThreads);
     if (!have_sums) hipLaunchKernelGGL(eden_sumsq_kernel, grid, block, 0, stream, set);
     if (!fold) hipLaunchKernelGGL(eden_norm_kernel, dim3(1), block, 0, stream, set.s[0].sums, set.s[0].sum_count, slices[0].result);
 #define DQ_EDEN_BINS(B)                                                                                       \
     do {                                                                                                      \
-        if (fold)                                                                                             \
-            hipLaunchKernelGGL((eden_bins_kernel<B, true>), grid, block, 0, stream, set, boundaries, centroids); \
+        if (few)                                                                                              \
+            hipLaunchKernelGGL((eden_bins_kernel<B, true, 8>), grid, dim3(kEdenTile / 8), 0, stream, set, boundaries, centroids); \
+        else if (fold)                                                                                        \
+            hipLaunchKernelGGL((eden_bins_kernel<B, true, 16>), grid, block, 0, stream, set, boundaries, centroids); \
         else                                                                                                  \
-            hipLaunchKernelGGL((eden_bins_kernel<B, false>), grid, block, 0, stream, set, boundaries, centroids); \
+            hipLaunchKernelGGL((eden_bins_kernel<B, false, 16>), grid, block, 0, stream, set, boundaries, centroids); \
     } while (0)
     switch (nbits) {
     case 1: DQ_EDEN_BINS(1); break;
@@ -435,7 +450,7 @@ hipError_t launch_thc_dequantize(const void *levels, float *out, int64_t n, cons
 //   up to 2^22            one launch per pass for all slices: tiles, strided pass, bins, scale; tiles, strided pass
 //   beyond                one after the other: their launches fill the GPU, and their diagonal is read from memory
 // Slices that are not plain powers of one rotation (only a caller's own dictionary asks for that) go one by one as well.
-// Both directions at 4 bits, fp32: 2^20 elements (one slice) 94 -> 38 -> 30 us, 20,000 (two) 165 -> 22, 115,387 (four) 364 -> 135 -> 44, 419,364
+// Both directions at 4 bits, fp32: 2^20 elements (one slice) 94 -> 38 -> 28 us, 20,000 (two) 165 -> 22, 115,387 (four) 364 -> 135 -> 44, 419,364
 // (three) 266 -> 115 -> 30, 6,000,000 (two) 186 -> 80: at first, (with one native call per slice,) together.
 
 namespace {

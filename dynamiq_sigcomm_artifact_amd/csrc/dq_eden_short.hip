@@ -101,8 +101,8 @@ template <int NBITS> __global__ __launch_bounds__(kShortThreads) void eden_short
     const float sum = (float)fold_tiles(sums, n);
     const float norm = __builtin_sqrtf(sum);
     __syncthreads();
-    uint16_t *half = mine ? reinterpret_cast<uint16_t *>(s.packed) + tid : nullptr;
-    const double dots = eden_bins16<NBITS>(v, norm, set.sqrt_n[blockIdx.x], tree, cen, half, n >> 5);
+    uint8_t *half = mine ? reinterpret_cast<uint8_t *>(s.packed) + 2 * tid : nullptr;
+    const double dots = eden_bins_of<NBITS, kEdenPerThread>(v, norm, set.sqrt_n[blockIdx.x], tree, cen, half, n >> 5);
     fold256(mine ? dots : 0.0, sums + g * kEdenThreads, t);
     if (tid == 0) {
         const float d = (float)fold_tiles(sums, n);
