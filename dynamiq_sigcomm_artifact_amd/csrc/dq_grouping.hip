@@ -687,7 +687,8 @@ __global__ __launch_bounds__(kThreads) void plan_place_stats_kernel(WidthsFromSt
 //   signed  two 16-bit counters per word, so two steps: the superchunks before the tile, whose counts the tile's waves
 //           read in turns, each adding its own, then the rest
 // A superchunk of zeros (+0, of which a bucket may hold many, and atomics on one word take turns) counts in one of 64
-// counters at the end of the keys, its lane's; the reader adds them.  Lanes beyond the bucket's end count as zeros
+// counters at the end of the keys, its lane's (in fewer of them where the least other pattern is below 64); the reader adds
+// them.  Lanes beyond the bucket's end count as zeros
 // behind all others, which moves nobody, so the loads and the counting have neither a branch nor a mask: taken branches
 // in code that runs once cost more (1.3 us for 25,600 superchunks) than what they skip.
 // Norms of 7 layers with scales e^-9 .. e^-3, us, with every pattern counted in one 144 KB histogram in two steps and in
@@ -762,7 +763,7 @@ template <int WAVES> __device__ __forceinline__ void tile_pair(int wave, int &ro
 }
 
 // The short and the long layout.  key = first - pattern for the patterns from `first` down, 0 above (NaN); +0 has the
-// key `last`, the one behind those of all other patterns present.
+// key `last` <= first, the one behind those of all other patterns present.
 template <bool LONG, int TILE, int BATCH>
 __device__ __forceinline__ void sorted_plan_once(int nsc, int top, int bottom, int64_t *__restrict__ qbits_out,
                                                  int32_t *__restrict__ order, const uint32_t (&cached)[BATCH],
@@ -775,7 +776,7 @@ __device__ __forceinline__ void sorted_plan_once(int nsc, int top, int bottom, i
     const uint32_t base = (first << 16) | 0xffffu; // (base - pair) >> 16 = first - pattern
     const auto key_of = [&](uint32_t pair, uint32_t end) -> uint32_t {
         if constexpr (LONG) return pair >> 16 ? __builtin_elementwise_sub_sat(base, pair) >> 16 : end;
-        return min((base - pair) >> 16, end); // (every pattern is at most `first`, +0 comes out at least `end`)
+        return min((base - pair) >> 16, end); // (every pattern is at most `first`, and +0 comes out between `last` and `end`)
     };
     const auto slot = [](uint32_t key) { return LONG ? hist_slot(key) : (int)key; };
     // (behind the last superchunk a prefix may be 65,536)
@@ -958,8 +959,9 @@ __global__ __launch_bounds__(kSortThreads) void sorted_plan_kernel(const uint32_
     const uint32_t under = ~(uint32_t)__builtin_amdgcn_readlane((int)low, 63) >> 16;
     const uint32_t last = first == 0 ? 0u : first - under; // the key of +0
     if (first <= (uint32_t)kMaxPattern && last + 64u <= (uint32_t)kShortKeys) {
-        sorted_plan_once<false, TILE>(nsc, top, bottom, qbits_out, order, cached, row_pair, col_pair, max(first, 64u), last, hist, wave_sum,
-                                      rank);
+        // (zeros alone, key 0: any `first` from 63 on gives every lane its counter)
+        sorted_plan_once<false, TILE>(nsc, top, bottom, qbits_out, order, cached, row_pair, col_pair, first == 0 ? 64u : first, last,
+                                      hist, wave_sum, rank);
     } else {
         for (int w = 2 * kSortThreads + t; w < kSortLdsWords / 4; w += kSortThreads) h4[w] = make_uint4(0u, 0u, 0u, 0u);
         if (first >= 0x8000u) {

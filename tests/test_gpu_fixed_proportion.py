@@ -121,6 +121,58 @@ def test_sorted_plan_layouts(capi, oracle, nsc, span):
             assert (got[base + hi - lo:base + nsc] == -7).all(), (kind, base)
 
 
+@pytest.mark.parametrize("nsc", [1, 2, 129, 1025, 32769, 65535])
+@pytest.mark.parametrize("greatest", [1, 2, 10, 62, 63, 64, 65, 128])
+def test_sorted_plan_of_subnormal_norms(capi, oracle, nsc, greatest):
+    """buckets whose greatest norm is one of the first bf16 patterns, fewer than the counters that zeros are spread over: in
+    descending order for all that, without zeros, with some, and two patterns alone"""
+    rng = np.random.default_rng(nsc + greatest)
+    for kind in ("all patterns", "zeros", "the greatest and zeros", "the greatest and the least"):
+        bits = rng.integers(1, greatest + 1, nsc).astype(np.uint16)
+        if kind == "zeros":
+            bits[rng.integers(0, nsc, (nsc + 2) // 3)] = 0
+        elif kind == "the greatest and zeros":
+            bits = np.where(rng.random(nsc) < 0.5, greatest, 0).astype(np.uint16)
+        elif kind == "the greatest and the least":
+            bits = np.where(rng.random(nsc) < 0.5, greatest, 1).astype(np.uint16)
+        bits[-1] = greatest
+        st = _stats(torch.from_numpy(bits.view(np.int16)).view(torch.bfloat16))
+        top_count, bottom_count = nsc // 3, nsc // 5
+        order = torch.full((3 * nsc,), -7, dtype=torch.int32, device=DEV)
+        work = torch.zeros(4, dtype=torch.int32, device=DEV)
+        capi.group_plan_sorted(st, top_count, bottom_count, order, work)
+        want = oracle.argsort_descending_stable(bits)
+        got = order.cpu().numpy()
+        for base, lo, hi in ((0, 0, top_count), (nsc, top_count, nsc - bottom_count), (2 * nsc, nsc - bottom_count, nsc)):
+            assert np.array_equal(got[base:base + hi - lo], want[lo:hi]), (kind, base)
+
+
+@pytest.mark.parametrize("size", [1e-21, 1.5e-21, 2e-20])
+def test_allreduce_of_gradients_with_subnormal_norms(capi, size):
+    """a bucket of gradients around 1e-21: its superchunks' norms are the first few bf16 patterns and many of them zero"""
+    from dynamiq_sigcomm_artifact_amd.compressors import Aee_Dynamic_Range_GPU_kern as K
+    from dynamiq_sigcomm_artifact_amd.dynamiq_pipeline import fixed_proportion_allreduce, fixed_proportion_allreduce_grouped
+    W, n, thr = 2, 256 * 1500 - 9, {8: 0.35, 4: 0.45, 2: 0.2}
+    g = torch.Generator().manual_seed(3)
+    scale = (size * torch.exp(torch.randn((n + 255) // 256, generator=g) * 0.4)).repeat_interleave(256)[:n]
+    vecs = [(torch.randn(n, generator=g) * scale).to(torch.bfloat16).to(DEV) for _ in range(W)]
+
+    def comps():
+        gen = torch.Generator(device=DEV).manual_seed(5)
+        return {q: [K(q, 16, {"d": {0: n + 256}, "world_size": W, "rank": r}, generator=gen) for r in range(W)] for q in (8, 4, 2)}
+
+    ref, total, idx = fixed_proportion_allreduce([v.clone() for v in vecs], thr, comps())
+    out, total2, order, counts = fixed_proportion_allreduce_grouped([v.clone() for v in vecs], thr, comps())
+    norms = total.view(torch.int16).reshape(-1, 2)[:, 1]
+    assert 0 < int(norms.max()) < (64 if size < 1e-20 else 1024) and norms.unique().numel() > 2
+    assert torch.equal(total.view(torch.int16), total2.view(torch.int16))
+    nsc = (n + 255) // 256
+    for gi, (cnt, ix) in enumerate(zip(counts, idx)):
+        assert torch.equal(order[gi * nsc:gi * nsc + cnt].long(), ix)
+    for a, b in zip(ref, out):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+
+
 def test_sorted_plan_wrapper_and_module(capi, eden_utils):
     from dynamiq_sigcomm_artifact_amd import bitrate as B
     g = torch.Generator().manual_seed(5)
