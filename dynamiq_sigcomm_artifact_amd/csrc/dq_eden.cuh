@@ -2,6 +2,7 @@
 // kernels of long slices (dq_eden.hip) and the one of short slices (dq_eden_short.hip).
 #pragma once
 
+#include "dq_sums.cuh"
 #include "dq_tile16.cuh"
 
 namespace dq {
@@ -13,28 +14,6 @@ constexpr int64_t kEdenFoldTiles = 1024;                 // the most tiles whose
 
 __host__ __device__ inline int64_t eden_tiles(int64_t n) { return (n + kEdenTile - 1) / kEdenTile; }
 
-// x of lane l + SHIFT of the row (0 beyond it)
-template <int SHIFT> __device__ __forceinline__ double row_shift_f64(double x)
-{
-    const uint64_t b = (uint64_t)__double_as_longlong(x);
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, 0x100 + SHIFT, 0xf, 0xf, true);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), 0x100 + SHIFT, 0xf, 0xf, true);
-    return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
-}
-
-// sum[l] += sum[l + 32], then sum[l + 16] (LANES), of the lanes below that
-template <int LANES> __device__ __forceinline__ double add_across_f64(double x)
-{
-    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-    const uint64_t b = (uint64_t)__double_as_longlong(x);
-    const auto both = [](uint32_t w) { // what the lower lanes hold, and what the upper ones hold, in both
-        return LANES == 16 ? __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane16_swap(w, w, false, false))
-                           : __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(w, w, false, false));
-    };
-    const u32x2 lo = both((uint32_t)b), hi = both((uint32_t)(b >> 32));
-    return __longlong_as_double((long long)(((uint64_t)hi[0] << 32) | lo[0])) + __longlong_as_double((long long)(((uint64_t)hi[1] << 32) | lo[1]));
-}
-
 // sum[l] += sum[l + stride], stride 128 .. 1, over 256 values, one per thread; returns the total in every thread.  t: 0 .. 255,
 // lds: 256 doubles of the group's own.  The strides of 128 and 64 meet in LDS, the others inside the first wave, in the same
 // order of additions: three barriers instead of ten, and no trips through the LDS crossbar in between.
@@ -45,10 +24,7 @@ __device__ __forceinline__ double fold256_of(double *lds, int t) // of the 256 v
         double s = (lds[t] + lds[t + 128]) + (lds[t + 64] + lds[t + 192]);
         s = add_across_f64<32>(s);
         s = add_across_f64<16>(s);
-        s += row_shift_f64<8>(s); // (lanes beyond the stride add what nobody reads)
-        s += row_shift_f64<4>(s);
-        s += row_shift_f64<2>(s);
-        s += row_shift_f64<1>(s);
+        s = halve_row_f64(s);
         if (t == 0) lds[0] = s;
     }
     __syncthreads();

@@ -4,7 +4,8 @@
 // torch element-wise ops and reductions around eden_utils.Hadamard.
 //
 // EDEN quantise, three launches, no host synchronisation:
-//   sumsq   tile b = elements [4096 b, 4096 b + 4096): thread t adds v^2 of elements t + 256 k (k ascending)
+//   sumsq   n = 2^k >= 2^14: in the order of dq_sums.cuh; workgroup b adds the pieces b + i n/4096, i < 8 -> work[b].
+//           Any other n: tile b = elements [4096 b, 4096 b + 4096): thread t adds v^2 of elements t + 256 k (k ascending)
 //           in double, the 256 sums are halved (stride 128 .. 1) -> work[b]
 //   bins    every workgroup folds work[] the same way -> sumsq (double); norm = sqrtf((float)sumsq);
 //           x = (v * (float)sqrt(n)) / norm; bin = number of boundaries b with !(b >= x) (torch.bucketize, right=False: NaN -> last bin);
@@ -18,9 +19,8 @@
 // 31.9 -> 29.2, 12,000,000 136.6 -> 128.4.
 // (scale inside bins, by the workgroup that finishes last: its release of the other XCDs' sums costs more than the launch --
 // bins 5.7 -> 10.8 us at 2^20 elements, against 1.8 us for scale.)
-// The sums are in double with a fixed association, so the result does not depend on the launch geometry, and the CPU
-// restatement reproduces it bit for bit (those of the strided pass are as exact, but associated by its tiles: their
-// float32 differs only where a sum lies within some 2^-50 of it of a rounding boundary).
+// The sums are in double with a fixed association, so the result does not depend on the launch geometry -- nor on which launch
+// adds the squares, nor on the slices that travel with this one -- and the CPU restatement reproduces it bit for bit.
 #include <mutex>
 #include <vector>
 
@@ -53,9 +53,23 @@ __global__ __launch_bounds__(kEdenThreads) void eden_sumsq_kernel(QuantizeSet se
     const int which = slice_of_block(set.first, set.count);
     const QuantizeSlice &s = set.s[which];
     const int64_t tile = blockIdx.x - set.first[which], base = tile * kEdenTile;
+    float v[kEdenPerThread];
+    if (sums_by_rows(s.n)) {
+        const int piece = threadIdx.x >> 5;
+        const float *vec = s.vec + (tile + piece * (s.n / kEdenTile)) * 32 + (threadIdx.x & 31);
+#pragma unroll
+        for (int k = 0; k < kEdenPerThread; k++) v[k] = vec[k * (s.n / kEdenPerThread)];
+        const double sum = sum_columns_f64(halve_squares(v));
+        if ((threadIdx.x & 31) == 0) lds[piece] = sum;
+        __syncthreads();
+        if (threadIdx.x < 64) {
+            const double total = halve_row_f64(threadIdx.x < kEdenThreads / 32 ? lds[threadIdx.x] : 0.0);
+            if (threadIdx.x == 0) s.work[tile] = total;
+        }
+        return;
+    }
     const float *vec = s.vec + base + threadIdx.x;
     const int left = (int)min((int64_t)kEdenTile, s.n - base);
-    float v[kEdenPerThread];
     if (left == kEdenTile) {
 #pragma unroll
         for (int k = 0; k < kEdenPerThread; k++) v[k] = vec[kEdenThreads * k];
@@ -88,13 +102,44 @@ __device__ __forceinline__ double fold_array(const double *work, int64_t count, 
 {
     return fold_array(work, count, lds, first_of_array(work, count));
 }
+// the sums of squares of n elements, at most kEdenFoldTiles of them: by rows it is the halving tree all the way (as the fold above
+// is for up to two entries a thread)
+__device__ __forceinline__ double fold_sums(const double *sums, int64_t count, int64_t n, double *lds, double acc)
+{
+    static_assert(kEdenFoldTiles == 4 * kEdenThreads, "four entries a thread at most");
+    if (count == kEdenFoldTiles && sums_by_rows(n)) {
+        if (threadIdx.x < kEdenThreads) {
+            const double *mine = sums + threadIdx.x;
+            lds[threadIdx.x] = (acc + mine[2 * kEdenThreads]) + (mine[kEdenThreads] + mine[3 * kEdenThreads]);
+        }
+        return fold256_of(lds, threadIdx.x);
+    }
+    return fold_array(sums, count, lds, acc);
+}
 
 // result[0] = (float)sumsq, result[3] = norm
-__global__ __launch_bounds__(kEdenThreads) void eden_norm_kernel(const double *__restrict__ work, int64_t count,
-                                                                float *__restrict__ result)
+// By rows a thread halves its entries t + 256 k in place, sixteen at a time (nobody else reads them): compress of 2^26 elements,
+// 32,768 sums, 396 us with one chain of additions per thread, 371 so.
+__global__ __launch_bounds__(kEdenThreads) void eden_norm_kernel(double *sums, int64_t count, int64_t n, float *__restrict__ result)
 {
     __shared__ double lds[kEdenThreads];
-    const double sumsq = fold_array(work, count, lds);
+    if (sums_by_rows(n)) {
+        double *mine = sums + threadIdx.x;
+        int64_t left = count / kEdenThreads;
+        double x[16];
+        while (left > 16) {
+            left /= 16;
+            for (int64_t k = 0; k < left; k++) {
+#pragma unroll
+                for (int i = 0; i < 16; i++) x[i] = mine[(k + i * left) * kEdenThreads];
+                mine[k * kEdenThreads] = halve(x);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 16; i++) x[i] = i < left ? mine[i * kEdenThreads] : 0.0;
+        lds[threadIdx.x] = halve(x);
+    }
+    const double sumsq = sums_by_rows(n) ? fold256_of(lds, threadIdx.x) : fold_array(sums, count, lds);
     if (threadIdx.x == 0) {
         const float s = (float)sumsq;
         result[0] = s;
@@ -104,8 +149,8 @@ __global__ __launch_bounds__(kEdenThreads) void eden_norm_kernel(const double *_
 
 // A thread owns PER = 8 or 16 consecutive elements, two or four 16-byte loads, so that it builds its byte or half word of every
 // bit plane in registers; the additions are the same in the same order.
-// FOLD: the norm is not in result[3] yet; the workgroup folds the partial sums in work[0 .. tiles) the way eden_norm_kernel
-// does (the same association: the same bits), workgroup 0 leaves result[0] and result[3] as that kernel would, and the
+// FOLD: the norm is not in result[3] yet; the workgroup folds the partial sums the way eden_norm_kernel does (the same
+// association: the same bits), workgroup 0 leaves result[0] and result[3] as that kernel would, and the
 // products go to a region of their own (other workgroups are still reading the sums).
 template <int NBITS, bool FOLD, int PER>
 __global__ __launch_bounds__(kEdenTile / PER) void eden_bins_kernel(QuantizeSet set, const float *__restrict__ boundaries,
@@ -143,7 +188,7 @@ __global__ __launch_bounds__(kEdenTile / PER) void eden_bins_kernel(QuantizeSet 
     __syncthreads();
     float norm;
     if constexpr (FOLD) {
-        const float sum = (float)fold_array(s.sums, s.sum_count, lds, part);
+        const float sum = (float)fold_sums(s.sums, s.sum_count, s.n, lds, part);
         norm = __builtin_sqrtf(sum);
         if (tile == 0 && threadIdx.x == 0) {
             s.result[0] = sum;
@@ -299,7 +344,7 @@ hipError_t launch_eden_quantize_slices(const QuantizeSlice *slices, int count, c
     const bool few = fold && blocks <= kFewTiles;
     dim3 grid((unsigned)blocks), block(kEdenThreads);
     if (!have_sums) hipLaunchKernelGGL(eden_sumsq_kernel, grid, block, 0, stream, set);
-    if (!fold) hipLaunchKernelGGL(eden_norm_kernel, dim3(1), block, 0, stream, set.s[0].sums, set.s[0].sum_count, slices[0].result);
+    if (!fold) hipLaunchKernelGGL(eden_norm_kernel, dim3(1), block, 0, stream, set.s[0].sums, set.s[0].sum_count, set.s[0].n, slices[0].result);
 #define DQ_EDEN_BINS(B)                                                                                       \
     do {                                                                                                      \
         if (few)                                                                                              \

@@ -88,17 +88,30 @@ template <int NBITS> __global__ __launch_bounds__(kShortThreads) void eden_short
     __syncthreads();
     // tile g = threads 256 g .. 256 g + 255 (nthreads is a multiple of 256)
     const int t = tid & (kEdenThreads - 1), g = tid / kEdenThreads;
-    double acc = 0.0;
+    float sum;
+    if (sums_by_rows(n)) { // (n is then 16 nthreads: a piece of 32 columns per half of a wave, 32 of them)
+        static_assert(kRowSumsFrom == kEdenShort, "the longest slice here");
+        float w[16];
 #pragma unroll
-    for (int k = 0; k < kEdenPerThread; k++) {
-        const int i = g * kEdenTile + t + kEdenThreads * k;
-        if (i < n) {
-            const double x = (double)lds[pad_idx(i)];
-            acc += x * x;
+        for (int k = 0; k < 16; k++) w[k] = lds[pad_idx(k * kShortThreads + tid)];
+        const double piece = sum_columns_f64(halve_squares(w));
+        if ((tid & 31) == 0) sums[tid >> 5] = piece;
+        __syncthreads();
+        // (every wave the same)
+        sum = (float)first_lane_f64(halve_row_f64(add_across_f64<16>(sums[tid & 31])));
+    } else {
+        double acc = 0.0;
+#pragma unroll
+        for (int k = 0; k < kEdenPerThread; k++) {
+            const int i = g * kEdenTile + t + kEdenThreads * k;
+            if (i < n) {
+                const double x = (double)lds[pad_idx(i)];
+                acc += x * x;
+            }
         }
+        fold256(acc, sums + g * kEdenThreads, t);
+        sum = (float)fold_tiles(sums, n);
     }
-    fold256(acc, sums + g * kEdenThreads, t);
-    const float sum = (float)fold_tiles(sums, n);
     const float norm = __builtin_sqrtf(sum);
     __syncthreads();
     uint8_t *half = mine ? reinterpret_cast<uint8_t *>(s.packed) + 2 * tid : nullptr;

@@ -217,8 +217,8 @@ struct TransformEnds {
     const float *in_centroids = nullptr;
     int in_nbits = 0;
     const float *post_scale = nullptr;
-    // EDEN: a strided last pass also leaves, in double, the sum of the squares of the values that its workgroup w stores in
-    // sums[w] (rht_sum_count of them)
+    // EDEN: a strided last pass over the whole vector also leaves, in double, the sum of the squares of the values that its
+    // workgroup w stores in sums[w] (rht_sum_count of them, in the order of dq_sums.cuh)
     double *sums = nullptr;
 };
 // workgroups of the last pass of a whole-vector transform by launch_rht_ends; 0: that pass knows no sums
@@ -261,7 +261,7 @@ struct QuantizeSlice {
     uint32_t *packed;
     float *result;
     double *work;
-    const double *sums = nullptr; // partial sums of the squares, if some pass has left them already
+    double *sums = nullptr; // partial sums of the squares, if some pass has left them already
     int64_t sum_count = 0;
     float sqrt_n = 0.0f;
 };

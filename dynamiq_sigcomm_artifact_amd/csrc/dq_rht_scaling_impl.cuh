@@ -35,6 +35,7 @@
 #include "dq_fwht.cuh"
 #include "dq_hier16_tiles.cuh"
 #include "dq_launch.h"
+#include "dq_sums.cuh"
 
 #define DQ_RHT_TRANSFORM 1
 #define DQ_RHT_COMPRESS_PHILOX 2
@@ -783,29 +784,6 @@ template <int B> __device__ __forceinline__ void draw_rows(float (&u)[1 << B], c
     }
 }
 
-// the sum over the wave's active lanes (64, or the first 32 of a workgroup of 32)
-__device__ __forceinline__ double wave_sum_f64(double x)
-{
-    const auto add_from = [&](auto ctrl) {
-        const uint64_t b = (uint64_t)__double_as_longlong(x);
-        const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, decltype(ctrl)::value, 0xf, 0xf, true);
-        const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), decltype(ctrl)::value, 0xf, 0xf, true);
-        x += __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
-    };
-    add_from(std::integral_constant<int, 0xB1>());  // quad_perm [1,0,3,2]
-    add_from(std::integral_constant<int, 0x4E>());  // quad_perm [2,3,0,1]
-    add_from(std::integral_constant<int, 0x141>()); // row_half_mirror
-    add_from(std::integral_constant<int, 0x140>()); // row_mirror
-    const uint64_t b = (uint64_t)__double_as_longlong(x);
-    const auto of_row = [&](int lane) {
-        const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)b, lane), hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), lane);
-        return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
-    };
-    double sum = of_row(0) + of_row(16);
-    if (blockDim.x > 32) sum += of_row(32) + of_row(48);
-    return sum;
-}
-
 // A later pass of a transform longer than one tile: index bits [sbits, sbits + A + B) of the vector.  A tile is 2^(A + B)
 // rows of 32 consecutive floats (128 bytes), row stride 2^sbits elements.  A thread owns column tid % 32 of 2^A consecutive
 // rows: it loads them (every load instruction of a wave covers two whole 128-byte row segments), does the A lowest row
@@ -817,8 +795,10 @@ __device__ __forceinline__ double wave_sum_f64(double x)
 // levels 19.0 -> 17.8 (67 MB read); both directions of THC on 25 MB 82.6 -> 70.2, on 16,000,000 elements 146.7 -> 118.7, EDEN on
 // 500,000 36.5 -> 31.7, on 12,000,000 157 -> 136 (with the first pass below).
 // sign_mode: 0, or 2 = flip on store (the last pass of an inverse).
-// e.sums: the sum of the squares of what the workgroup stores, in double (each square is exact there): EDEN's norm without a pass
-// over the vector for it, 3.1 us of 34 at 2^20 elements, 12 of 137 at 2^24.
+// e.sums (the whole vector, its last pass): the sum of the squares of what the workgroup stores, in the order of dq_sums.cuh: EDEN's
+// norm without a pass over the vector for it, 3.1 us of 34 at 2^20 elements, 12 of 137 at 2^24.  The workgroup has 2^(A + B - 4)
+// pieces of 32 columns.  With A = 4 they are its groups of 32 threads, whose rows are the loop's last 4 - B digits below the
+// B of the registers; with A = 5 a group has two, and the piece's number has one more digit in front of the group's.
 template <bool ENDS, int A, int B>
 __device__ __forceinline__ void strided_rows(float *__restrict__ x, const PassArgs<ENDS> &a, int sbits, int sign_mode, int apply_scale,
                                              const TransformEnds &e, unsigned block, float *lds)
@@ -866,7 +846,12 @@ __device__ __forceinline__ void strided_rows(float *__restrict__ x, const PassAr
         }
         __syncthreads();
     }
-    double squares = 0.0;
+    constexpr int kSums = A == 5 ? 2 : 1 << (4 - B);
+    double sums[kSums];
+    if constexpr (ENDS) {
+#pragma unroll
+        for (int q = 0; q < kSums; q++) sums[q] = 0.0;
+    }
     const bool flips = sign_mode == 2;
     bool drawn = false;
     if constexpr (ENDS) drawn = flips && a.gen.bits != 0;
@@ -965,8 +950,14 @@ __device__ __forceinline__ void strided_rows(float *__restrict__ x, const PassAr
 #pragma unroll
             for (int i = 0; i < R2; i++) x[first + ((int64_t)i << (A + sbits))] = w[i];
             if (ENDS && e.sums) {
+                if constexpr (B == 5) {
+                    sums[0] = halve_squares<2>(w);
+                    sums[1] = halve_squares<2>(w, 1);
+                } else {
+                    const double sum = halve_squares(w);
 #pragma unroll
-                for (int i = 0; i < R2; i++) squares = __builtin_fma((double)w[i], (double)w[i], squares); // (the square is exact)
+                    for (int q = 0; q < kSums; q++) sums[q] = q == row >> B ? sum : sums[q];
+                }
             }
         }
     };
@@ -988,20 +979,26 @@ __device__ __forceinline__ void strided_rows(float *__restrict__ x, const PassAr
     }
     if constexpr (ENDS) {
         if (e.sums) {
-            const double sum = wave_sum_f64(squares);
+            double sum;
+            if constexpr (A == 5)
+                sum = sum_columns_f64(sums[0]) + sum_columns_f64(sums[1]);
+            else
+                sum = sum_columns_f64(halve(sums));
             double *part = reinterpret_cast<double *>(lds + (32 << (A + B))); // (behind the tile: strided_lds_bytes)
-            if ((tid & 63) == 0) part[tid >> 6] = sum;
+            if (mine && col == 0) part[group] = sum;
             __syncthreads();
             if (tid < 64) {
-                const double all = wave_sum_f64(tid < (int)(blockDim.x + 63) / 64 ? part[tid] : 0.0);
+                double all = tid < R2 ? part[tid] : 0.0;
+                if (B == 5) all = add_across_f64<16>(all);
+                all = halve_row_f64(all);
                 if (tid == 0) e.sums[block] = all;
             }
         }
     }
 }
 
-// a tile, and a double for each of up to sixteen waves
-__host__ constexpr size_t strided_lds_bytes(int rbits) { return (sizeof(float) << (rbits + 5)) + 16 * sizeof(double); }
+// a tile, and a double for each of up to 32 groups
+__host__ constexpr size_t strided_lds_bytes(int rbits) { return (sizeof(float) << (rbits + 5)) + 32 * sizeof(double); }
 // threads of the tile of a strided pass
 __host__ __device__ constexpr int strided_threads(int rbits) { return rbits >= 9 ? 1 << rbits : 1 << (rbits + 1); }
 

@@ -906,6 +906,35 @@ static double tiled_sum(int64_t n, dqo_term_fn term, void *ctx, int consecutive)
     return halve256(lane);
 }
 
+/* the sum of squares of n = 2^k >= 2^14 elements: element e is in row e / (n / 16) and in column e % 32 of piece
+ * e / 32 % (n / 512); the rows of a column are halved (16 to one), the columns added neighbours first, the pieces halved */
+static double sum_squares_by_rows(const float *vec, int64_t n)
+{
+    const int64_t pieces = n / 512;
+    double *sum = (double *)malloc((size_t)pieces * sizeof(double));
+    for (int64_t p = 0; p < pieces; p++) {
+        double column[32];
+        for (int l = 0; l < 32; l++) {
+            double row[16];
+            for (int t = 0; t < 16; t++) {
+                const double v = (double)vec[t * (n / 16) + p * 32 + l];
+                row[t] = v * v;
+            }
+            for (int stride = 8; stride > 0; stride >>= 1)
+                for (int t = 0; t < stride; t++) row[t] += row[t + stride];
+            column[l] = row[0];
+        }
+        for (int stride = 1; stride < 32; stride <<= 1)
+            for (int l = 0; l < 32; l += 2 * stride) column[l] += column[l + stride];
+        sum[p] = column[0];
+    }
+    for (int64_t stride = pieces / 2; stride > 0; stride >>= 1)
+        for (int64_t p = 0; p < stride; p++) sum[p] += sum[p + stride];
+    const double total = sum[0];
+    free(sum);
+    return total;
+}
+
 struct eden_ctx { const float *vec; const float *cen; const int32_t *bins; };
 static double term_sq(int64_t i, void *c) { double v = (double)((struct eden_ctx *)c)->vec[i]; return v * v; }
 static double term_dot(int64_t i, void *c)
@@ -923,7 +952,8 @@ void dqo_eden_quantize(const float *vec, int64_t n, const float *boundaries, con
 {
     const int nb = (1 << nbits) - 1;
     struct eden_ctx ctx = {vec, centroids, bins};
-    const float sumsq = (float)tiled_sum(n, term_sq, &ctx, 0);
+    const int by_rows = n >= (1 << 14) && (n & (n - 1)) == 0;
+    const float sumsq = (float)(by_rows ? sum_squares_by_rows(vec, n) : tiled_sum(n, term_sq, &ctx, 0));
     const float norm = sqrtf(sumsq);
     const float sqrt_n = (float)sqrt((double)n);
     for (int64_t i = 0; i < n; i++) {

@@ -518,6 +518,62 @@ def test_scale_from_the_sums_of_the_last_pass(sizes):
         assert abs(float(scale) / float(want) - 1.0) < 2.0 ** -22, (n, float(scale), float(want))
 
 
+def _sum_on_a_boundary(bits, shift, which, k):
+    """A vector of 2^bits elements, an even number of bits, whose rotation by H / sqrt(n) is 1,024 values, each in as many places,
+    with a sum of squares within 2^-53 of the middle between two float32s: to which of them it rounds depends on the order in which
+    a double adds the squares.  The 1,024 values are u + b and u - b: u, 512 of them, are whole numbers and exact, b has more
+    fractional digits than a sum of the two keeps (found by trying 2^33 pairs of u and b).  They stay the same with the digits of
+    their index in another order and with the signs of any character of it, and lie `shift` digits up in the vector's index."""
+    seed, b = ((687, 14603885), (1143, 13973873), (1523, 13967869), (2132, 14500689))[which]
+    x = np.zeros(1024, np.float32)
+    x[:512] = np.random.default_rng(seed).integers(-2048, 2049, 512)
+    x[512] = b * 2.0 ** -9
+    rng = np.random.default_rng([bits, shift, which, k])
+    order, character = rng.permutation(9), int(rng.integers(1024))
+    i = np.arange(1024)
+    source, sign = i & 512, np.ones(1024, np.float32)
+    for new, old in enumerate(order):
+        source |= ((i >> new) & 1) << old
+    for d in range(10):
+        if character >> d & 1:
+            sign[(i >> d) & 1 == 1] *= -1.0
+    out = np.zeros(1 << bits, np.float32)
+    out[i << shift] = x[source] * sign
+    return out
+
+
+@pytest.mark.parametrize("bits", [14, 16, 18, 20, 22, 24, 26])
+def test_scale_is_the_slices_own(capi, oracle, bits):
+    """the sums behind a slice's scale, and so its bins, are the same alone, beside longer and shorter slices, in eden_quantize
+    and in the oracle, also where the order of the additions decides the last bit"""
+    from dynamiq_sigcomm_artifact_amd.eden import Eden
+    n, nbits, seed = 1 << bits, 4, 5
+    eden = Eden(device=DEV)
+    centroids, boundaries = eden._tables(nbits)
+    diag = torch.empty(n, device=DEV)
+    capi.rand_diag(diag, seed)
+    others = torch.randn(1 << 22, generator=torch.Generator(device=DEV).manual_seed(1), device=DEV)
+    for shift in sorted({0, (bits - 10) // 2, bits - 10}):
+        for k in range(16 if bits <= 18 else 4 if bits <= 22 else 2):
+            x = torch.from_numpy(_sum_on_a_boundary(bits, shift, k % 4, k)).to(DEV) * diag
+            y = x.clone()
+            capi.rht_blocked(y, diag, n, 2.0 ** (-bits // 2), False)
+            packed = torch.empty(n // 32 * nbits, dtype=torch.int32, device=DEV)
+            result = torch.empty(4, device=DEV)
+            work = torch.empty(capi.eden_work_doubles(n), dtype=torch.float64, device=DEV)
+            capi.eden_quantize(y, boundaries, centroids, nbits, packed, result, work)
+            if bits <= 24 or k == 0:
+                bins_o, res_o = oracle.eden_quantize(y.cpu().numpy(), boundaries.cpu().numpy(), centroids.cpu().numpy(), nbits)
+                assert (result.cpu().numpy().view(np.uint32) == res_o.view(np.uint32)).all(), (shift, k)
+                assert (packed.cpu().numpy().view(np.uint32) == oracle.bins_to_bits(bins_o, nbits)).all(), (shift, k)
+            for size in (0, 1 << 13, 1 << 15, 1 << 18, 1 << 20, 1 << 22):
+                vec = torch.cat([others[:size], x])
+                slices = [(0, size, size, 1)] * (size > 0) + [(size, n, n, 1)]
+                got, scale = capi.host().eden_compress(vec, boundaries, centroids, nbits, seed, slices)[-1]
+                assert torch.equal(scale.view(torch.int32), result[2].view(torch.int32)), (shift, k, size)
+                assert torch.equal(got, packed), (shift, k, size)
+
+
 @pytest.mark.parametrize("seed", [2 ** 63 + 5, -(2 ** 63), 2 ** 70 + 9, 2 ** 64 - 1])
 def test_seeds_of_any_size(capi, seed):
     """a seed is taken modulo 2^64, as the single calls take it; one that is no whole number is refused"""
