@@ -720,6 +720,10 @@ hipError_t launch_roundtrip(const RoundtripDesc *desc, int count, int world, flo
 // 102 -> 106 (82), 8 x 121,524 425 -> 375 (324).  The ring that follows reads the vectors again: out of the cache behind the L2
 // (256 MB) if they are there, which loads that pass it by cost 10 us at 8 x 15,625 and nothing at 8 x 32,227.  Both launches,
 // keeping -> passing by: 280 MB 147 -> 151, 320 MB 168 -> 170, 384 MB 215 -> 205.
+// Vectors off the 16 bytes load element by element, each wave one tile and then the next with nothing on the way: a tile per wave
+// whatever their length (in fours and eights -> one by one: bf16 8 x 2,051 tiles 42 -> 37.5, 8 x 15,626 283 -> 255, 8 x 121,524
+// 1,895 -> 1,794; fp32 8 x 3,907 105 -> 73, 8 x 15,626 409 -> 298, 3 x 29,297 285 -> 220; bf16 8 x 3,907 goes the other way, 60 ->
+// 64.5).
 constexpr int64_t kStatsOneTile = (int64_t)1 << 14, kStatsCache = (int64_t)300 << 20;
 
 hipError_t launch_ranks_stats(const void *const *src, int world, int64_t n, void *total, float *mean, int dtype, hipStream_t stream)
@@ -741,7 +745,8 @@ hipError_t launch_ranks_stats(const void *const *src, int world, int64_t n, void
                            waves * StatsTile<DT>::BYTES, stream, p, world, n, vec, tot, mean, wd);
     };
     const auto launch = [&](auto type) {
-        if (tiles * world * StatsTile<decltype(type)::value>::ESZ * 1024 > kStatsCache) run(type, std::integral_constant<int, 8>(), std::true_type());
+        if (!vec) run(type, std::integral_constant<int, 1>(), std::false_type());
+        else if (tiles * world * StatsTile<decltype(type)::value>::ESZ * 1024 > kStatsCache) run(type, std::integral_constant<int, 8>(), std::true_type());
         else if (tiles * world > kStatsOneTile) run(type, std::integral_constant<int, 4>(), std::false_type());
         else run(type, std::integral_constant<int, 1>(), std::false_type());
     };
