@@ -651,11 +651,19 @@ __global__ __launch_bounds__(64 * kQuadWaves) void ring_quad_kernel(RingArgs<RDT
     for (int rank = 0; rank < world; rank++) store_quarter<DT>(a.out[rank], v, e0, a.n, (a.vec & 2) != 0, ragged);
 }
 
-// Up to here a superchunk per wave, beyond it four: the quads issue more per element (160 instructions per superchunk and step
-// against 90), and from two waves of ring_kernel per SIMD on (8,192 superchunks) that is what counts.  Kernel alone, ring_kernel
-// -> ring_quad_kernel, bf16: 8 ranks x 65,536 15.7 -> 8.7 us, x 1,000,003 20.0 -> 16.2, x 2,000,000 26.3 -> 25.6, x 3,000,000
-// 33.5 -> 35.2; with pools 2 x 100,000 8.1 -> 4.2, 4 x 2,000,000 15.8 -> 12.1, 3 x 4,000,000 15.6 -> 16.8.
-constexpr int kQuadSuperchunks = 8192;
+// Up to so many superchunks one per wave, beyond it four: the quads issue more per element (160 instructions per superchunk and
+// step against 90), and from two waves of ring_kernel per SIMD on (8,192 superchunks) that is what counts.  Kernel alone,
+// ring_kernel -> ring_quad_kernel, us: 8 ranks x 256 superchunks 12.2 -> 7.8 (AEE), 15.9 -> 8.9 (MEE), 19.5 -> 8.3 (AEE from pools);
+// x 8,192 20.4 -> 20.9, 27.0 -> 24.9, 26.2 -> 20.6, fp32 24.6 -> 23.2, 29.0 -> 23.9.  Two to five ranks with the least to do per
+// step -- AEE, values drawn, bf16 (fp32: two) -- have their line at five waves per SIMD, where a sixth would begin: 2 ranks x 4,900
+// 6.9 -> 7.0, x 5,300 6.8 -> 7.4, x 8,192 7.9 -> 9.0; 3 x 4,900 8.9 -> 8.3, x 6,900 9.3 -> 10.1; 5 x 4,900 12.4 -> 11.4, x 5,700 12.5
+// -> 13.2; fp32 2 x 4,900 6.8 -> 6.5, x 5,700 6.8 -> 7.2; but 6 x 6,500 17.3 -> 16.0, fp32 3 x 6,100 9.5 -> 9.1.
+constexpr int kQuadSuperchunks = 8192, kQuadSuperchunksShort = 5120;
+bool a_wave_each(int nsc, int world, int elem_bytes, bool mee, bool pooled)
+{
+    const bool least = !mee && !pooled && world * elem_bytes < 12;
+    return nsc <= (least ? kQuadSuperchunksShort : kQuadSuperchunks);
+}
 
 WidthRule make_rule(float u, const double *u_dev)
 {
@@ -724,7 +732,11 @@ hipError_t launch_roundtrip(const RoundtripDesc *desc, int count, int world, flo
 // whatever their length (in fours and eights -> one by one: bf16 8 x 2,051 tiles 42 -> 37.5, 8 x 15,626 283 -> 255, 8 x 121,524
 // 1,895 -> 1,794; fp32 8 x 3,907 105 -> 73, 8 x 15,626 409 -> 298, 3 x 29,297 285 -> 220; bf16 8 x 3,907 goes the other way, 60 ->
 // 64.5).
-constexpr int64_t kStatsOneTile = (int64_t)1 << 14, kStatsCache = (int64_t)300 << 20;
+// Near the lines, a tile per wave -> four, statistics and ring together: bf16 8 x 2,075 28.8 -> 29.1, 8 x 2,500 30.0 -> 30.6, 8 x 2,550
+// 34.5 -> 30.6, 8 x 2,750 34.6 -> 31.8, 2 x 10,000 27.4 -> 27.4; fp32 8 x 2,075 37.0 -> 37.5, 8 x 2,500 41.2 -> 41.3, 8 x 2,750 46.3 -> 44.4,
+// 3 x 6,500 40.7 -> 41.2, 4 x 4,500 38.7 -> 38.9; in fp32, a tile per wave -> eight that pass the caches by: 2 x 37,500 (307 MB) 147 -> 146,
+// 4 x 19,500 (319 MB) 156.5 -> 159.5, 8 x 10,000 (327 MB) 169 -> 166, 2 x 47,500 202 -> 193.
+constexpr int64_t kStatsOneTile = 19 << 10, kStatsCache = (int64_t)300 << 20;
 
 hipError_t launch_ranks_stats(const void *const *src, int world, int64_t n, void *total, float *mean, int dtype, hipStream_t stream)
 {
@@ -786,7 +798,7 @@ static hipError_t run_ring(const RingDesc &d, bool mee, const MeeParams *mp, hip
     a.key = RandKey{d.seed, 0};
     a.wd = make_world_div(d.world, DT == DQ_F32 ? 4 : 2);
     a.widths = make_width_set(mp, mee);
-    if (a.nsc <= kQuadSuperchunks) {
+    if (a_wave_each(a.nsc, d.world, DT == DQ_F32 ? 4 : 2, mee, POOL)) {
         const dim3 grid((unsigned)((a.nsc + kQuadWaves - 1) / kQuadWaves)), block(64 * kQuadWaves);
         if (mee) hipLaunchKernelGGL((ring_quad_kernel<DT, RDT, true>), grid, block, 0, stream, a);
         else hipLaunchKernelGGL((ring_quad_kernel<DT, RDT, false>), grid, block, 0, stream, a);

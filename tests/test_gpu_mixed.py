@@ -716,9 +716,21 @@ def test_ranks_on_either_side_of_a_superchunk_per_wave(capi, W, n):
     test_ranks_in_registers_equal_the_ring_in_steps(capi, W, n, torch.bfloat16)
 
 
+@pytest.mark.parametrize("W,n,dt", [
+    (2, 256 * 5120, torch.bfloat16), (2, 256 * 5120 + 1, torch.bfloat16), (5, 256 * 5120 + 1, torch.bfloat16),
+    (6, 256 * 5120 + 1, torch.bfloat16), (6, 256 * 8192 + 1, torch.bfloat16),
+    (2, 256 * 5120, torch.float32), (2, 256 * 5120 + 1, torch.float32), (3, 256 * 8192, torch.float32)])
+def test_ranks_on_either_side_of_the_lines_of_a_superchunk_per_wave(capi, W, n, dt):
+    """AEE with the values drawn: few ranks take four superchunks per wave from 5,121 on, more of them and fp32 from 8,193"""
+    test_ranks_in_registers_equal_the_ring_in_steps(capi, W, n, dt)
+
+
 @pytest.mark.parametrize("W,n,dt,offset", [
-    (8, 1024 * 2048, torch.bfloat16, 0),           # the last length with a tile per wave of the statistics
-    (8, 1024 * 2048 + 1, torch.bfloat16, 0),       # four tiles per wave; one element in the last of them
+    (8, 1024 * 2048, torch.bfloat16, 0),           # a tile per wave of the statistics
+    (8, 1024 * 2048 + 1, torch.bfloat16, 0),
+    (8, 1024 * 2432, torch.bfloat16, 0),           # the last length with a tile per wave
+    (8, 1024 * 2432 + 1, torch.bfloat16, 0),       # four tiles per wave; one element in the last of them
+    (3, 1024 * 6486 - 255, torch.float32, 0),
     (3, 1024 * 5464 - 255, torch.float32, 0),
     (3, 1024 * 5465, torch.bfloat16, 1),           # vectors off the 16 bytes
     (9, 1024 * 4 * 500 + 256 * 7, torch.bfloat16, 0),
