@@ -380,11 +380,13 @@ __device__ __forceinline__ float thc_level(float v, float u, float lo, float del
 // through that comparison, so an estimate within e of it decides unless frac(x) - u comes within e of 0 -- or of +-1, where the
 // estimate and the quotient may lie on either side of an integer.  Such elements (one in 10^4 at 64 levels), and everything that is
 // not a number, take thc_level itself.  v_rcp_f32 is good to 1 ulp and the product to half of one, the quotient itself to half: e <
-// top 2^-22, and the clamp can come last.  35 instead of 75 issue cycles per element.
+// top 2^-22, and the clamp can come last.  35 instead of 75 issue cycles per element.  That holds for a reciprocal that is an
+// ordinary number (its subnormal result would be 0): with spacings beyond 2^126 no element counts as decided.  (Below 2^-126 it
+// is infinite or good, and what an infinite one makes of an element is never decided.)
 template <int N> __device__ __forceinline__ void thc_levels(float (&v)[N], const float (&u)[N], float lo, float delta, float top)
 {
     const float rd = __builtin_amdgcn_rcpf(delta);
-    const float sure = 0.5f - (top + 1.0f) * 0x1p-21f;
+    const float sure = __builtin_fabsf(delta) <= 0x1p126f ? 0.5f - (top + 1.0f) * 0x1p-21f : -1.0f;
 #pragma unroll
     for (int i = 0; i < N; i++) {
         const float x = (v[i] - lo) * rd;

@@ -248,6 +248,30 @@ def test_thc_levels_where_the_comparison_is_a_tie(capi, n, levels):
         assert torch.equal(got.view(torch.int16), want.view(torch.int16)), bad
 
 
+@pytest.mark.parametrize("n", [1 << 16, 1 << 20])
+@pytest.mark.parametrize("delta", [2.0 ** -149, 2.0 ** -126, 2.0 ** 126, 2.0 ** 126 * 1.25, 2.0 ** 127 * 1.9])
+def test_thc_levels_of_the_widest_and_the_finest_grid(capi, n, delta):
+    """a spacing whose reciprocal is no ordinary float32: the levels of the folded quantiser are those of the quantiser that
+    divides"""
+    levels = 64 if delta < 1.0 else 4
+    g = torch.Generator().manual_seed(n)
+    x = (torch.randn(n, generator=g) * (delta * 0.15 / math.sqrt(n))).to(DEV)
+    if delta < 1.0:
+        x = (torch.randint(-1, 2, (n,), generator=g).float() * 2.0 ** -149).to(DEV)
+    rot = x.clone()
+    capi.rht_blocked(rot, None, n, 1.0, False)
+    lo = torch.tensor([-delta if delta > 1.0 else -32 * delta], dtype=torch.float32, device=DEV)
+    step = torch.tensor([delta], dtype=torch.float32, device=DEV)
+    q = ((rot.double() - lo.double()) / delta).clamp(0, levels - 1)
+    frac = (q - q.floor()).float()
+    uni = torch.where(torch.arange(n, device=DEV) % 2 == 0, frac, torch.rand(n, generator=g).to(DEV))
+    want, got = torch.empty(n, dtype=torch.bfloat16, device=DEV), torch.empty(n, dtype=torch.bfloat16, device=DEV)
+    capi.thc_quantize(rot, uni, want, lo, step, levels)
+    capi.thc_rht_quantize(x, None, uni, got, n, 1.0, lo, step, levels)
+    assert torch.isfinite(rot).float().mean() > 0.9 and want.unique().numel() > 2
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
 @pytest.mark.parametrize("dim", [1 << k for k in range(18, 27)])
 def test_thc_draws_what_torch_would_draw(dim):
     """compress without uniform values: the levels are those of values that uniform_ drew from a generator in the same state, call
