@@ -812,7 +812,7 @@ py::object thc_compress(py::handle src, int64_t count, py::handle work, py::hand
 // thc_compress with the uniform values that generator.uniform_() would fill a vector with, drawn in the kernel: the generator is
 // moved on as that call moves it.  None where it cannot be: a generator of another device, a stream that records (torch
 // keeps the generator's state on the device then), a GPU whose resident threads are no power of two, a length that the kernel does
-// not draw for.
+// not draw for.  (thc.py asks only beside the torch releases whose launch of uniform_ this restates.)
 py::object thc_compress_drawn(py::handle src, int64_t count, py::handle work, py::handle bits, py::handle generator, double scale,
                               py::handle norm, py::tuple numbers, int levels)
 {

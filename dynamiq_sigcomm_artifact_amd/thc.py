@@ -24,9 +24,19 @@ import torch
 from . import capi
 
 _READ = {torch.float32, torch.bfloat16, torch.float16}         # what the transform's first pass reads itself
-_DRAWN = (1 << 19, 1 << 25)                                     # dimensions whose uniform values the last pass draws itself
+
 _TABLE_FILE = "{table_size}_tablesize_{max_val}_maxval_16_qlevels_{overflow_frequency}_ofreq_data.txt"
 _TABLE_DEFAULTS = {"table_size": 10001, "max_val": 42, "overflow_frequency": 1024}
+
+
+def _drawn_dimensions(torch_version):
+    """(least, greatest) dimension whose uniform values the last pass draws itself; none with a torch whose uniform_ has not been
+    compared with it.  Which thread of how many draws which element is torch's own affair and may change with a release; the
+    values that uniform_ draws are what the levels are defined by."""
+    return (1 << 19, 1 << 25) if torch_version.split(".")[:2] == ["2", "10"] else (1, 0)
+
+
+_DRAWN = _drawn_dimensions(torch.__version__)
 
 
 def _clip_threshold(params):

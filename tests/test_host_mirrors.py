@@ -363,3 +363,15 @@ def test_division_by_the_world_size_as_a_multiplication():
                             rng.integers(0, top + 1, 24, dtype=np.uint64)])
         x = x[x <= top]
         assert ((x * np.uint64(m)) >> np.uint64(40) == x // np.uint64(d)).all(), d
+
+
+def test_uniform_values_are_drawn_only_beside_a_known_torch():
+    """the kernel restates which element of uniform_ comes from where in the generator's stream, as the releases below do it; with
+    any other torch compress leaves the drawing to uniform_"""
+    from dynamiq_sigcomm_artifact_amd import thc
+    for version in ("2.10.0", "2.10.0+rocm7.0", "2.10.1a0"):
+        assert thc._drawn_dimensions(version) == (1 << 19, 1 << 25)
+    for version in ("2.9.1", "2.11.0+rocm7.1", "2.1.0", "3.10.0"):
+        least, greatest = thc._drawn_dimensions(version)
+        assert least > greatest
+    assert thc._DRAWN == thc._drawn_dimensions(torch.__version__)
