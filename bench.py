@@ -24,16 +24,21 @@ host's per-call cost is not part of the figure; `eager_ms_per_step` has it).
 readings of this script, scaled by the copy-kernel calibration), null when the
 file has no entry for the kernel and workload.
 
-`configs` holds one entry per cell of the other baseline configurations, each
-timed the same way (ring of buffer sets where a set is smaller than the cache)
-with a sample of its output compared with the oracle: the 25 MB bucket for
-fp32 / bf16 sources x 4 / 8 bits x AEE / MEE; the ring step of the 8 x 124 M
+The other baseline configurations are measured in the same run, cell by cell,
+each timed the same way (ring of buffer sets where a set is smaller than the
+cache) with a sample of its output compared with the oracle: the 25 MB bucket
+for fp32 / bf16 sources x 4 / 8 bits x AEE / MEE; the ring step of the 8 x 124 M
 ring on a 15,555,072-element chunk at 5 bits and as the dynamic {2, 4, 8} mix;
 the single-pass dynamic-bitrate path per 25 MB bucket of a Llama-3-8B shaped
 set; 2^30 fp32 elements: compress / decompress / fused ring step at 2, 4, 5, 8
 bits and the transform fused with the codec for blocks 2^10 .. 2^15 x four
 widths; and the six rows of the reference's own microbenchmark
-(cuda_kernels/tests/benchmark_scaling_quantization.py:60-112).
+(cuda_kernels/tests/benchmark_scaling_quantization.py:60-112).  The line's
+`configs` has, for each of them, the number of cells, whether all samples were
+equal to the oracle's, and the least and greatest of each fraction of the HBM
+peak and rate: the cells themselves (30 KB) are written to the file that
+--cells names, and the line stays short enough for whatever keeps only the end
+of a program's output.
 
 `cpu_baseline` times the reference's CPU-runnable path for the headline
 workload -- the hierarchical chunk quantiser as a torch op sequence
@@ -60,6 +65,22 @@ HBM_PEAK_GBS = 8000.0
 OVERHEAD_BITS = 0.5625  # hierarchical scale bytes per element, in bits
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "hbm_traffic.json")
 COLD_FOOTPRINT = 640e6   # bytes a ring of buffer sets must exceed
+
+
+def summary(cells):
+    """the cells of every configuration (the part of "workload" in front of the colon) as one short entry"""
+    groups = {}
+    for cell in cells:
+        groups.setdefault(cell["workload"].split(":")[0], []).append(cell)
+    out = {}
+    for name, members in groups.items():
+        exact = [c.get("bit_exact_vs_oracle") for c in members]        # (None: not compared)
+        out[name] = {"cells": len(members), "bit_exact_vs_oracle": None if None in exact else all(exact)}
+        for key in sorted({k for c in members for k in c if k.endswith("frac") or "GBps" in k}):
+            values = [c[key] for c in members if c.get(key) is not None]
+            if values:
+                out[name][key] = [min(values), max(values)]
+    return out
 
 
 def packed_bytes_per_element(nbits):
@@ -576,8 +597,9 @@ def main():
                     help="distinct bucket sets (source, random pool, packed, output) the headline walks; default: as many "
                          "as make up 640 MB, at least 10")
     ap.add_argument("--configs", default="2,3,4,5,ref",
-                    help="which of the other configurations go into `configs` (comma separated: 2, 3, 4, 5, ref; 'none' = "
+                    help="which of the other configurations are measured (comma separated: 2, 3, 4, 5, ref; 'none' = "
                          "headline only, e.g. under a profiler)")
+    ap.add_argument("--cells", metavar="FILE", help="write the line and every cell of the other configurations to FILE")
     ap.add_argument("--no-check", action="store_true", help="skip the oracle parity check of a sample")
     ap.add_argument("--pmc-calibration", action="store_true",
                     help="also run a plain elementwise fp32 copy kernel (out = -in) of the same element count, "
@@ -825,7 +847,6 @@ def main():
         "source_dtype": args.src,
         "packed_bytes": int(nb),
         "bucket_sets": nsets,
-        "configs": configs,
     }
     result = {
         "metric": "compress+decompress GB/s (fp32 grad in) on 1 MI355X, % of HBM peak; NMSE",
@@ -882,13 +903,16 @@ def main():
         "bit_exact_vs_oracle": bit_exact,
         "eager_ms_per_step": round(eager_ms_per_step, 5),
         "host_wall_ms_per_step": round(wall_ms, 5),
-        "configs": configs,
+        "configs": summary(configs),
         "configs_skipped": skipped,
         "configs_seconds": round(configs_seconds, 1),
         "cpu_baseline": cpu,
         "cpu_scalar_port": cpu_scalar,
         "cpu_rht_path": cpu_rht,
     }
+    if args.cells:
+        with open(args.cells, "w") as f:
+            json.dump({"headline": result, "cells": configs}, f, indent=1)
     print(json.dumps(result))
 
 

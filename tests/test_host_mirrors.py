@@ -348,6 +348,33 @@ def test_bench_refuses_more_than_one_gpu():
     assert r.returncode == 2 and "--gpus must be 1" in r.stderr and r.stdout.strip() == ""
 
 
+def test_bench_line_stays_short():
+    """the cells of the other configurations go into the line as one entry per configuration: 49 cells were 30 KB, of which
+    a reader who keeps the last 8 KB of the output had no line left"""
+    import importlib.util
+    import json
+    import os
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    spec = importlib.util.spec_from_file_location("bench_program", os.path.join(root, "bench.py"))
+    bench = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(bench)
+    cells = [{"workload": "config %s: cell %d of many, with a long description of what it is" % (name, k), "compress_us": 10.0 + k,
+              "compress_frac": 0.5 + 0.001 * k, "decompress_frac": 0.6, "fused_frac": 0.7 if k else None, "GBps_fp32_in": 1500.0 + k,
+              "nmse": 0.01, "bit_exact_vs_oracle": True}
+             for name, count in (("2", 8), ("3", 4), ("4", 3), ("5", 28), ("ref", 6)) for k in range(count)]
+    out = bench.summary(cells)
+    assert {k: v["cells"] for k, v in out.items()} == {"config 2": 8, "config 3": 4, "config 4": 3, "config 5": 28, "config ref": 6}
+    assert out["config 5"]["compress_frac"] == [0.5, 0.527] and out["config 3"]["GBps_fp32_in"] == [1500.0, 1503.0]
+    assert out["config 2"]["fused_frac"] == [0.7, 0.7] and "nmse" not in out["config 2"]
+    assert all(v["bit_exact_vs_oracle"] is True for v in out.values())
+    cells[3]["bit_exact_vs_oracle"] = False
+    cells[9]["bit_exact_vs_oracle"] = None
+    out = bench.summary(cells)
+    assert out["config 2"]["bit_exact_vs_oracle"] is False and out["config 3"]["bit_exact_vs_oracle"] is None
+    assert len(json.dumps(out)) < 2000
+    assert bench.summary([]) == {}
+
+
 def test_division_by_the_world_size_as_a_multiplication():
     """The mixed kernels split a group of n superchunks over the ring as ceil(n / world) per rank and compute the
     quotient as (x * ceil(2^40 / world)) >> 40 for x < 2^24 and world <= 2^16 (dq_scaling_mixed.hip: divide_by_world).
