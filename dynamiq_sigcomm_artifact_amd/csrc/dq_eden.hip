@@ -495,8 +495,8 @@ hipError_t launch_thc_dequantize(const void *levels, float *out, int64_t n, cons
 //   up to 2^22            one launch per pass for all slices: tiles, strided pass, bins, scale; tiles, strided pass
 //   beyond                one after the other: their launches fill the GPU, and their diagonal is read from memory
 // Slices that are not plain powers of one rotation (only a caller's own dictionary asks for that) go one by one as well.
-// Both directions at 4 bits, fp32: 2^20 elements (one slice) 94 -> 38 -> 28 us, 20,000 (two) 165 -> 22, 115,387 (four) 364 -> 135 -> 44, 419,364
-// (three) 266 -> 115 -> 30, 6,000,000 (two) 186 -> 80: at first, (with one native call per slice,) together.
+// Both directions at 4 bits, fp32: 2^20 elements (one slice) 94 -> 38 -> 28-32 us, 20,000 (two) 165 -> 20, 115,387 (four) 364 -> 135 -> 43,
+// 419,364 (three) 266 -> 115 -> 29, 6,000,000 (two) 186 -> 62: at first, (with one native call per slice,) now together.
 
 namespace {
 

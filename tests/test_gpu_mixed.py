@@ -712,7 +712,7 @@ def test_ranks_in_registers_equal_the_ring_in_steps(capi, W, n, dt):
 
 @pytest.mark.parametrize("W,n", [(2, 256 * 8192), (3, 256 * 8192 + 1), (5, 256 * 8195)])
 def test_ranks_on_either_side_of_a_superchunk_per_wave(capi, W, n):
-    """the last length that takes a wave per superchunk and the first ones that take four superchunks per wave"""
+    """the last length that takes a wave per superchunk (MEE; AEE below) and the first ones that take four superchunks per wave"""
     test_ranks_in_registers_equal_the_ring_in_steps(capi, W, n, torch.bfloat16)
 
 
