@@ -145,3 +145,48 @@ def test_nan_goes_to_the_last_bin_like_torch_bucketize(oracle):
     x = np.array([-2.0, -1.0, -0.5, 0.0, 0.5, 1.0, 2.0, np.nan] * 4, np.float32)
     got = np.array([sum(1 for b in bnd if not (b >= v)) for v in x])
     assert (got == torch.bucketize(torch.from_numpy(x), torch.from_numpy(bnd)).numpy()).all()
+
+
+def _halve(x):
+    while x.shape[0] > 1:
+        x = x[:x.shape[0] // 2] + x[x.shape[0] // 2:]
+    return x[0]
+
+
+def _sum_by_rows(v):
+    columns = _halve((v.astype(np.float64) ** 2).reshape(16, -1, 32))
+    while columns.shape[1] > 1:
+        columns = columns[:, 0::2] + columns[:, 1::2]
+    return np.float32(_halve(columns[:, 0]))
+
+
+def _sum_by_tiles(v):
+    squares = np.zeros(-(-v.size // 4096) * 4096)
+    squares[:v.size] = v.astype(np.float64) ** 2
+    lanes = np.zeros((squares.size // 4096, 256))
+    for k in range(16):
+        lanes += squares.reshape(-1, 16, 256)[:, k]
+    tiles, total = _halve(lanes.T), np.zeros(256)
+    for k in range(0, tiles.size, 256):
+        total[:tiles[k:k + 256].size] += tiles[k:k + 256]
+    return np.float32(_halve(total))
+
+
+@pytest.mark.parametrize("seed,b,digits", [(1143, 13973873, 4), (2132, 14500689, 4), (687, 14603885, 0)])
+def test_order_of_the_sum_of_squares(oracle, seed, b, digits):
+    """1,024 values u + b, u - b whose sum of squares lies between two float32s: the order in which a double adds them decides the
+    rounding, and the oracle's is by rows for 2^k >= 2^14 elements, by tiles for every other length"""
+    u = np.random.default_rng(seed).integers(-2048, 2049, 512).astype(np.float64)
+    for s in range(9):                                            # H u: whole numbers
+        u = u.reshape(-1, 2, 1 << s)
+        u = np.stack([u[:, 0] + u[:, 1], u[:, 0] - u[:, 1]], 1).reshape(-1)
+    u, b = u.astype(np.float32), np.float32(b * 2.0 ** -9)
+    pattern = np.concatenate([u + b, u - b])
+    cen, bnd = np.float32([-1.0, 1.0]), np.float32([0.0])
+    for n, order in ((1 << 14, _sum_by_rows), (1 << 16, _sum_by_rows), (1 << 12, _sum_by_tiles), (3 << 12, _sum_by_tiles)):
+        low = digits if n > 4096 else min(digits, 2)
+        repeated = np.repeat(np.tile(pattern, max(1, n >> (10 + low))), 1 << low)[:n]
+        _, result = oracle.eden_quantize(np.ascontiguousarray(repeated), bnd, cen, 1)
+        assert result[0] == order(repeated), n
+        if n == 1 << 14:
+            assert _sum_by_rows(repeated) != _sum_by_tiles(repeated)
