@@ -376,28 +376,41 @@ __device__ __forceinline__ float thc_level(float v, float u, float lo, float del
     return fl + ((u < prob) ? 1.0f : 0.0f);
 }
 
-// thc_level of N elements (in and out) with the division as an estimate: the quotient enters level = floor(x) + (u < frac(x)) only
-// through that comparison, so an estimate within e of it decides unless frac(x) - u comes within e of 0 -- or of +-1, where the
-// estimate and the quotient may lie on either side of an integer.  Such elements (one in 10^4 at 64 levels), and everything that is
-// not a number, take thc_level itself.  v_rcp_f32 is good to 1 ulp and the product to half of one, the quotient itself to half: e <
-// top 2^-22, and the clamp can come last.  35 instead of 75 issue cycles per element.  That holds for a reciprocal that is an
-// ordinary number (its subnormal result would be 0): with spacings beyond 2^126 no element counts as decided.  (Below 2^-126 it
-// is infinite or good, and what an infinite one makes of an element is never decided.)
-template <int N> __device__ __forceinline__ void thc_levels(float (&v)[N], const float (&u)[N], float lo, float delta, float top)
+// thc_level of N elements with the division as an estimate.  For x in [0, top] the level is floor(x + 1 - u), unless that number is an
+// integer; below 0 and above top the same with the clamp.  So y = (v - lo) rcp(delta) + (1 + g - u), of which the last two operations are
+// one fused multiply-add, decides where its distance to x + 1 - u is less than g and frac(y) >= 2 g; other elements (one in 10^4 at 64
+// levels), and everything that is not a number, take thc_level itself.  v_rcp_f32 is good to 1 ulp, the quotient of thc_level to half
+// of one, the fused operation and 1 + g - u likewise: together less than (top + 2) 2^-22 < g = (top + 2) 2^-21.  That holds for a
+// reciprocal that is an ordinary number (its subnormal result would be 0): with spacings beyond 2^126 no element counts as decided.
+// (Below 2^-126 it is infinite or good, and what an infinite one makes of an element is never decided.)  25 issue cycles per
+// element, 39 with the level as floor(x) and a comparison of its own, 75 for thc_level.
+// Eight elements at a time, whose chains overlap, and one branch of the wave for all of them.  out[i]: the level as the high half of a
+// word, its bfloat16 (a level has eight significant bits at most: the low half of its binary32 pattern is zero).
+template <int N>
+__device__ __forceinline__ void thc_levels(const float (&v)[N], const float (&u)[N], float lo, float delta, float top, uint32_t (&out)[N])
 {
-    const float rd = __builtin_amdgcn_rcpf(delta);
-    const float sure = __builtin_fabsf(delta) <= 0x1p126f ? 0.5f - (top + 1.0f) * 0x1p-21f : -1.0f;
+    constexpr int kGroup = N < 8 ? N : 8;
+    const float rd = __builtin_amdgcn_rcpf(delta), guard = (top + 2.0f) * 0x1p-21f, bias = 1.0f + guard;
+    const float sure = __builtin_fabsf(delta) <= 0x1p126f ? 2.0f * guard : 2.0f;
 #pragma unroll
-    for (int i = 0; i < N; i++) {
-        const float x = (v[i] - lo) * rd;
-        const float fl = __builtin_floorf(x), w = (x - fl) - u[i];
-        const bool decided = __builtin_fabsf(__builtin_fabsf(w) - 0.5f) <= sure;
-        float level = __builtin_amdgcn_fmed3f(fl + (w > 0.0f ? 1.0f : 0.0f), 0.0f, top);
-        if (__builtin_amdgcn_ballot_w64(!decided) != 0) {
-            asm volatile(""); // (a branch of the wave: the compiler would select otherwise)
-            if (!decided) level = thc_level(v[i], u[i], lo, delta, top);
+    for (int g = 0; g < N; g += kGroup) {
+        uint64_t open[kGroup], any = 0; // lanes whose element is not decided
+#pragma unroll
+        for (int k = 0; k < kGroup; k++) {
+            const float y = __builtin_fmaf(v[g + k] - lo, rd, bias - u[g + k]), fl = __builtin_floorf(y);
+            open[k] = __builtin_amdgcn_ballot_w64(!(y - fl >= sure));
+            any |= open[k];
+            out[g + k] = __float_as_uint(__builtin_amdgcn_fmed3f(fl, 0.0f, top));
         }
-        v[i] = level;
+        if (any != 0) {
+#pragma unroll
+            for (int k = 0; k < kGroup; k++) {
+                if (open[k] != 0) {
+                    asm volatile(""); // (a branch of the wave: the compiler would select otherwise)
+                    if ((open[k] >> (threadIdx.x & 63)) & 1) out[g + k] = f32_to_bf16_bits(thc_level(v[g + k], u[g + k], lo, delta, top)) << 16;
+                }
+            }
+        }
     }
 }
 

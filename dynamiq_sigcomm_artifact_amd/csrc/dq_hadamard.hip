@@ -322,7 +322,14 @@ static hipError_t fwht_blocks(float *x, const void *sign, bool sign_packed, int6
     a.apply_scale = 0; a.sign_mode = sign_fwd; a.vec = vec16;
     a.in_levels = thc.in_levels;
     a.in_planes = thc.in_planes;
-    hipError_t e = ends_ok ? launch_rht_tile(x, sign, sign_packed ? 1 : 0, n, kt, kt, scale, 0, sign_fwd, a.vec, first, stream)
+    // The tiles that lie behind a shorter source are zeros before and after this pass.  The pass that draws THC's uniform values is all
+    // that follows then: nobody writes them and it does not read them.  THC on 25 MB, 6,553,600 of 2^23 elements, 52.9 -> 50.7 us.
+    int64_t tiles_n = n;
+    if (thc.in_src && thc.draw.bits >= 0 && thc.in_count < n) {
+        tiles_n = (thc.in_count + ((int64_t)1 << kt) - 1) >> kt << kt;
+        if (tiles_n < n) last.zeros_from = tiles_n;
+    }
+    hipError_t e = ends_ok ? launch_rht_tile(x, sign, sign_packed ? 1 : 0, tiles_n, kt, kt, scale, 0, sign_fwd, a.vec, first, stream)
                            : launch_tile(a, n >> kt, stream);
     if (e != hipSuccess) return e;
     a.in_levels = nullptr;

@@ -192,6 +192,9 @@ struct TransformEnds {
     const void *in_src = nullptr;
     int in_dtype = 0;
     int64_t in_count = 0;
+    // a strided pass over the whole vector that draws THC's uniform values finds zeros from here on and does not read them (a
+    // multiple of its row stride; negative: it reads everything)
+    int64_t zeros_from = -1;
     // the last pass stores its first out_count elements as out_dtype to out_dst, and nothing to x
     void *out_dst = nullptr;
     int out_dtype = 0;

@@ -576,8 +576,14 @@ template <int RB> __device__ __forceinline__ void stage_of(float (&v)[16])
     }
 }
 
+// Vectors of up to so many elements leave the first pass with the non-temporal hint: what waits in the L2 until the kernel ends, up
+// to 32 MB, is then on its way while others still load.  First pass, us, without -> with: 2^23 elements from bf16 levels 13.8 -> 9.5, from
+// a 25 MB gradient 12.8 -> 11.7, 2^20 5.9 -> 5.6 (the pass that reads them 0.5 to 1 longer); but 2^24, where the L2 is full long before the
+// end, both ways of THC 103 -> 111.5.
+constexpr int64_t kEarlyStores = (int64_t)1 << 23;
+
 // lds_pass whose results go to memory: consecutive lanes hold consecutive elements (P >= 6)
-template <int P, int M> __device__ __forceinline__ void lds_pass_out(const float *lds, int kt, int tid, int nthreads, float *__restrict__ out)
+template <int P, int M> __device__ __forceinline__ void lds_pass_out(const float *lds, int kt, int tid, int nthreads, float *__restrict__ out, bool early)
 {
     for (int u = tid; u < 1 << (kt - M); u += nthreads) {
         const int base = tuple_base<P, M>(u, kt - P - M);
@@ -586,8 +592,15 @@ template <int P, int M> __device__ __forceinline__ void lds_pass_out(const float
 #pragma unroll
         for (int j = 0; j < (1 << M); j++) v[j] = q[tuple_step<P>(j)];
         butterflies<M>(v);
+        if (early) {
+            asm volatile(""); // (the compiler would make one store of the two, without the hint)
 #pragma unroll
-        for (int j = 0; j < (1 << M); j++) out[base + (j << P)] = v[j];
+            for (int j = 0; j < (1 << M); j++) __builtin_nontemporal_store(v[j], out + base + (j << P));
+            asm volatile("");
+        } else {
+#pragma unroll
+            for (int j = 0; j < (1 << M); j++) out[base + (j << P)] = v[j];
+        }
     }
 }
 
@@ -721,12 +734,13 @@ __device__ __forceinline__ void first_pass(float *__restrict__ x, const PassArgs
     }
     __syncthreads();
     float *out = x + origin;
+    const bool early = a.n <= kEarlyStores;
     switch (a.kt) {
-    case 10: lds_pass_out<6, 4>(lds, 10, tid, step, out); break;
-    case 11: lds_pass_out<7, 4>(lds, 11, tid, step, out); break;
-    case 12: lds_pass_out<8, 4>(lds, 12, tid, step, out); break;
-    case 13: lds_pass_out<9, 4>(lds, 13, tid, step, out); break;
-    default: lds_pass_out<10, 4>(lds, 14, tid, step, out); break;
+    case 10: lds_pass_out<6, 4>(lds, 10, tid, step, out, early); break;
+    case 11: lds_pass_out<7, 4>(lds, 11, tid, step, out, early); break;
+    case 12: lds_pass_out<8, 4>(lds, 12, tid, step, out, early); break;
+    case 13: lds_pass_out<9, 4>(lds, 13, tid, step, out, early); break;
+    default: lds_pass_out<10, 4>(lds, 14, tid, step, out, early); break;
     }
 }
 
@@ -799,7 +813,11 @@ template <int B> __device__ __forceinline__ void draw_rows(float (&u)[1 << B], c
 // norm without a pass over the vector for it, 3.1 us of 34 at 2^20 elements, 12 of 137 at 2^24.  The workgroup has 2^(A + B - 4)
 // pieces of 32 columns.  With A = 4 they are its groups of 32 threads, whose rows are the loop's last 4 - B digits below the
 // B of the registers; with A = 5 a group has two, and the piece's number has one more digit in front of the group's.
-template <bool ENDS, int A, int B>
+// DRAW: the pass stores THC's levels and draws their uniform values, while the elements are on their way; it knows e.zeros_from.  A variant of its own: beside
+// loads of uniform values, which may be pending in the registers that the draws go to as far as the compiler can tell, every draw
+// waited for elements it does not need.  2^23 elements to THC's levels, with thc_levels in groups: both ways 54.1 -> 52.8 us, 2^24 103.5 ->
+// 100.5, padded 25 MB (with e.zeros_from) 50.7 -> 48.
+template <bool ENDS, int A, int B, bool DRAW = false>
 __device__ __forceinline__ void strided_rows(float *__restrict__ x, const PassArgs<ENDS> &a, int sbits, int sign_mode, int apply_scale,
                                              const TransformEnds &e, unsigned block, float *lds)
 {
@@ -812,33 +830,51 @@ __device__ __forceinline__ void strided_rows(float *__restrict__ x, const PassAr
     const int col = tid & 31, group = tid >> 5;
     const bool mine = group < R2; // (a launch of several passes has the threads of the largest)
     float v[R1];
+    // of the thread's rows: those behind them are zeros that nobody has written (the last written row's address is asked for instead:
+    // behind a comparison each, the loads would wait for one another)
+    int have = R1;
+    bool whole = true;
+    if (DRAW && e.zeros_from >= 0) {
+        have = min(max((int)(e.zeros_from >> sbits) - (group << A), 0), R1);
+        whole = __builtin_amdgcn_ballot_w64(have < R1) == 0;
+    }
     if (mine) {
         const float *from = x + origin + ((int64_t)(group << A) << sbits) + col;
+        if (whole) {
 #pragma unroll
-        for (int j = 0; j < R1; j++) v[j] = from[(int64_t)j << sbits];
+            for (int j = 0; j < R1; j++) v[j] = from[(int64_t)j << sbits];
+        } else if (__builtin_amdgcn_ballot_w64(have > 0) != 0) {
+#pragma unroll
+            for (int j = 0; j < R1; j++) v[j] = from[(int64_t)min(j, max(have - 1, 0)) << sbits];
+        }
     }
     // THC's uniform values are drawn while the elements are on their way; or they are on their way while the stages run, where one
     // workgroup has a CU to itself (1024 rows; with 256 that gains nothing)
-    constexpr bool kDraws = ENDS && A == B, kAhead = kDraws && A == 5;
+    static_assert(!DRAW || (ENDS && A == B), "a thread has one row of the registers' 2^B to draw for");
+    constexpr bool kAhead = ENDS && !DRAW && A == 5 && B == 5;
+    const bool levels_out = DRAW || (ENDS && e.out_levels);
     float u[R2];
-    bool have_u = false;
-    if constexpr (kDraws) {
-        if (e.out_levels && mine) {
+    bool have_u = DRAW;
+    if constexpr (DRAW || kAhead) {
+        if (levels_out && mine) {
             const int64_t at = origin + ((int64_t)group << sbits) + col;
-            if (e.draw.bits >= 0) {
+            if constexpr (DRAW) {
                 draw_rows<B>(u, e.draw, at, A + sbits);
-                have_u = true;
-            } else if (kAhead) {
+            } else {
 #pragma unroll
                 for (int i = 0; i < R2; i++) u[i] = e.uniform[at + ((int64_t)i << (A + sbits))];
                 have_u = true;
             }
         }
     }
+    if (!whole) {
+#pragma unroll
+        for (int j = 0; j < R1; j++) v[j] = j < have ? v[j] : 0.0f;
+    }
     if (mine) butterflies<A>(v);
     float post = 1.0f, lo = 0.0f, delta = 1.0f;
-    if (ENDS && e.post_scale) post = *e.post_scale;
-    if (ENDS && e.out_levels) grid_of(e.grid, e.out_lo, e.out_delta, lo, delta);
+    if (ENDS && !DRAW && e.post_scale) post = *e.post_scale;
+    if (levels_out) grid_of(e.grid, e.out_lo, e.out_delta, lo, delta);
     if constexpr (B > 0) {
         if (mine) {
 #pragma unroll
@@ -848,11 +884,11 @@ __device__ __forceinline__ void strided_rows(float *__restrict__ x, const PassAr
     }
     constexpr int kSums = A == 5 ? 2 : 1 << (4 - B);
     double sums[kSums];
-    if constexpr (ENDS) {
+    if constexpr (ENDS && !DRAW) {
 #pragma unroll
         for (int q = 0; q < kSums; q++) sums[q] = 0.0;
     }
-    const bool flips = sign_mode == 2;
+    const bool flips = !DRAW && sign_mode == 2;
     bool drawn = false;
     if constexpr (ENDS) drawn = flips && a.gen.bits != 0;
     // rows i 2^A + row, i < 2^B, of one column
@@ -908,18 +944,19 @@ __device__ __forceinline__ void strided_rows(float *__restrict__ x, const PassAr
         }
         // on their way out: EDEN's scale, then the float store, THC's quantiser (thc_hooks.py:161-166) or a destination of
         // another type
-        if (ENDS && e.post_scale) {
+        if (ENDS && !DRAW && e.post_scale) {
 #pragma unroll
             for (int i = 0; i < R2; i++) w[i] *= post;
         }
-        if (ENDS && e.out_levels) {
+        if (levels_out) {
             if (!have_u) {
 #pragma unroll
                 for (int i = 0; i < R2; i++) u[i] = e.uniform[first + ((int64_t)i << (A + sbits))];
             }
-            thc_levels(w, u, lo, delta, e.out_top);
+            uint32_t levels[R2];
+            thc_levels(w, u, lo, delta, e.out_top, levels);
 #pragma unroll
-            for (int i = 0; i < R2; i++) e.out_levels[first + ((int64_t)i << (A + sbits))] = (uint16_t)f32_to_bf16_bits(w[i]);
+            for (int i = 0; i < R2; i++) e.out_levels[first + ((int64_t)i << (A + sbits))] = (uint16_t)(levels[i] >> 16);
         } else if (ENDS && e.out_dst) {
             // rows that lie inside the destination for the whole wave need no test
             const int last_row = __builtin_amdgcn_readfirstlane(B > 0 ? row | 1 : row);
@@ -977,7 +1014,7 @@ __device__ __forceinline__ void strided_rows(float *__restrict__ x, const PassAr
             finish(w, j);
         }
     }
-    if constexpr (ENDS) {
+    if constexpr (ENDS && !DRAW) {
         if (e.sums) {
             double sum;
             if constexpr (A == 5)
@@ -1030,6 +1067,15 @@ __global__ __launch_bounds__(32 << B) void rht_strided_long_kernel(float *__rest
 {
     extern __shared__ __attribute__((aligned(16))) float lds[];
     strided_rows<ENDS, 5, B>(x, a, sbits, sign_mode, apply_scale, e, blockIdx.x, lds);
+}
+
+// 256 (A = 4) or 1024 rows (A = 5) to THC's levels with drawn values
+template <int A>
+__global__ __launch_bounds__(32 << A) void rht_strided_draw_kernel(float *__restrict__ x, RhtPassArgs a, int sbits, int sign_mode,
+                                                                   int apply_scale, TransformEnds e)
+{
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    strided_rows<true, A, A, true>(x, a, sbits, sign_mode, apply_scale, e, blockIdx.x, lds);
 }
 
 template <bool ENDS>
@@ -1557,7 +1603,8 @@ hipError_t launch_rht_strided(float *x, const void *sign, int sign_bits, int64_t
     if (rbits < 4 || rbits > 10 || sbits < 5 || (n & (((int64_t)1 << (sbits + rbits)) - 1)) != 0) return hipErrorInvalidValue;
     const bool plain = ends.plain_out() && ends.gen.bits == 0;
     if (!plain && !vec) return hipErrorInvalidValue;
-    if (ends.out_levels && ends.draw.bits >= 0 && rbits != 8 && rbits != 10) return hipErrorInvalidValue;
+    const bool draws = ends.out_levels && ends.draw.bits >= 0;
+    if (draws && ((rbits != 8 && rbits != 10) || sign_mode == 2 || ends.post_scale || ends.sums)) return hipErrorInvalidValue;
     RhtPassArgs a;
     a.sign = sign; a.sign_bits = sign_bits; a.n = n; a.kt = rbits + 5; a.kb = 0; a.scale = scale; a.vec = vec; a.gen = ends.gen;
     const RhtTileArgs &plain_args = a;
@@ -1574,6 +1621,7 @@ hipError_t launch_rht_strided(float *x, const void *sign, int sign_bits, int64_t
         if (rbits == 9) return launch(rht_strided_long_kernel<false, 4>, plain_args, sbits);
         return launch(rht_strided_kernel<false>, plain_args, rbits, sbits);
     }
+    if (draws) return rbits == 10 ? launch(rht_strided_draw_kernel<5>, a, sbits) : launch(rht_strided_draw_kernel<4>, a, sbits);
     if (rbits == 10) return launch(rht_strided_long_kernel<true, 5>, a, sbits);
     if (rbits == 9) return launch(rht_strided_long_kernel<true, 4>, a, sbits);
     return launch(rht_strided_kernel<true>, a, rbits, sbits);

@@ -294,6 +294,23 @@ def test_thc_draws_what_torch_would_draw(dim):
         assert torch.equal(a.sender_prng.get_state(), b.sender_prng.get_state())
 
 
+@pytest.mark.parametrize("dim,row", [(1 << 19, 1 << 11), (1 << 22, 1 << 14), (1 << 23, 1 << 13), (1 << 25, 1 << 15)])
+def test_thc_draws_behind_a_short_source(dim, row):
+    """sources that end at, before and behind a row of the strided pass, a wave's rows and a thread's: the rows behind them are neither
+    written nor read where the values are drawn, whatever lies there, and the levels are those of the pass that reads them all"""
+    from dynamiq_sigcomm_artifact_amd.thc import OldINCACudaHadamardCompressor
+    key = (0, 0)
+    x = torch.randn(dim, generator=torch.Generator(device=DEV).manual_seed(dim), device=DEV)
+    for used in (1, row, row + 1, 16 * row, 32 * row - 3, 33 * row + 5, 64 * row, dim // 2 + 1, dim - row - 1, dim - row, dim - 1):
+        params = {"d": {key: dim}, "size": {key: used}, "seed": 42, "T": 3.0, "device": DEV, "quantization_levels": 64, "nclients": 4, "rank": 1}
+        a, b = OldINCACudaHadamardCompressor(params), OldINCACudaHadamardCompressor(params)
+        a._buffer(key, "work").fill_(float("nan"))
+        norm = x[:used].norm()
+        got = a.compress(x[:used], key, norm)
+        want = b.compress(x[:used], key, norm, uniform=torch.empty(dim, device=DEV).uniform_(0.0, 1.0, generator=b.sender_prng))
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16)), used
+
+
 def test_thc_recorded_draws_are_torchs():
     """a graph that holds a compress call draws through the generator's registered state: every replay other values, those of an
     eager call from the same state"""
