@@ -264,8 +264,9 @@ __global__ __attribute__((amdgpu_waves_per_eu(8, 8))) void rht_compress_kernel(c
         encode_store_run<NBITS, MEE, kRowsPerWave, false>(v, r, mp, dst + sc0 * RC::REC, rows_here, reinterpret_cast<uint8_t *>(lds) + wave * RC::WIN, threadIdx.x & 63);
 }
 
+// blocks below 2^10 elements, several to a tile
 template <int NBITS, bool MEE>
-__global__ void irht_decompress_kernel(const uint8_t *__restrict__ src, float *__restrict__ x, RhtTileArgs a,
+__global__ void irht_decompress_tile_kernel(const uint8_t *__restrict__ src, float *__restrict__ x, RhtTileArgs a,
                                        MeeArg<NBITS, MEE> mp)
 {
     typedef Rec<NBITS> RC;
@@ -576,6 +577,53 @@ template <int RB> __device__ __forceinline__ void stage_of(float (&v)[16])
     }
 }
 
+// A tile of 2^KT elements with a chunk per thread, in two trips through the LDS: which chunk a thread takes; the stages of strides 1 ..
+// 8, for 2^13 and 2^14 elements one or two more by lane bit 5 (and 4) changing places with a register bit, and the chunk into the LDS;
+// (a barrier;) the next stages; (a barrier.)  What is left then are the four highest stages, on elements tid + j 2^(KT - 4).
+template <int KT> __device__ __forceinline__ int chunk_of(int tid)
+{
+    const int lane = tid & 63;
+    if (KT == 13) return (tid & ~63) | ((lane & 31) << 1) | (lane >> 5);
+    if (KT == 14) return (tid & ~63) | ((lane & 15) << 2) | (((lane >> 4) & 1) << 1) | (lane >> 5);
+    return tid;
+}
+
+template <int KT> __device__ __forceinline__ void chunk_into_tile(float (&v)[16], float *lds, int tid)
+{
+    const int lane = tid & 63, c = chunk_of<KT>(tid);
+    butterflies<4>(v);
+    if constexpr (KT == 13) {
+        swap_lane_bit<32, 0>(v);
+        stage_of<0>(v); // e4
+        float *slot = lds + pad_idx(((c >> 1) << 5) | (lane >> 5));
+#pragma unroll
+        for (int i = 0; i < 16; i++) slot[((i & 1) << 4) | (i & 14)] = v[i];
+    } else if constexpr (KT == 14) {
+        swap_lane_bit<32, 1>(v);
+        stage_of<1>(v); // e4
+        swap_lane_bit<16, 0>(v);
+        stage_of<0>(v); // e5
+        float *slot = lds + pad_idx(((c >> 2) << 6) | ((lane >> 5) << 1) | ((lane >> 4) & 1));
+#pragma unroll
+        for (int i = 0; i < 16; i++) slot[pad_idx(((i & 1) << 5) | (((i >> 1) & 1) << 4) | (i & 12))] = v[i];
+    } else {
+        float *slot = lds + chunk_word(c);
+#pragma unroll
+        for (int i = 0; i < 16; i++) slot[i] = v[i];
+    }
+}
+
+template <int KT> __device__ __forceinline__ void middle_stages(float *lds, int tid, int nthreads)
+{
+    static_assert(KT >= 10 && KT <= 14, "two trips");
+    if (KT == 13)
+        lds_pass<5, 4>(lds, KT, tid, nthreads);
+    else if (KT == 14)
+        lds_pass<6, 4>(lds, KT, tid, nthreads);
+    else
+        lds_pass<4, KT < 13 ? KT - 8 : 4>(lds, KT, tid, nthreads);
+}
+
 // Vectors of up to so many elements leave the first pass with the non-temporal hint: what waits in the L2 until the kernel ends, up
 // to 32 MB, is then on its way while others still load.  First pass, us, without -> with: 2^23 elements from bf16 levels 13.8 -> 9.5, from
 // a 25 MB gradient 12.8 -> 11.7, 2^20 5.9 -> 5.6 (the pass that reads them 0.5 to 1 longer); but 2^24, where the L2 is full long before the
@@ -672,9 +720,7 @@ __device__ __forceinline__ void tile_pass(float *__restrict__ x, const PassArgs<
 
 // The first pass of a long transform: the tile is one block of 2^10 .. 2^14 elements, a chunk per thread, with nothing to do on
 // the way out.  The last stages store from registers, as whole 256-byte runs: one trip through the LDS and one barrier less
-// than tile_pass.  Blocks of 2^13 and 2^14 do one or two more stages in front of the LDS, by lane bit 5 (and 4) changing places with
-// a register bit: what is left then are two passes of four stages that all threads take part in.  Bound like the strided
-// passes; 2^23 elements from bf16 levels 13.4 -> 11.8 us, from a 25 MB gradient 17.3 -> 15.0.
+// than tile_pass.  Bound like the strided passes; 2^23 elements from bf16 levels 13.4 -> 11.8 us, from a 25 MB gradient 17.3 -> 15.0.
 template <bool ENDS>
 __device__ __forceinline__ void first_pass(float *__restrict__ x, const PassArgs<ENDS> &a, int sign_mode, const TransformEnds &e, unsigned block,
                                            float *lds)
@@ -692,45 +738,26 @@ __device__ __forceinline__ void first_pass(float *__restrict__ x, const PassArgs
         __syncthreads();
     }
     const int nthreads = 1 << (a.kt - 4);
-    if (tid < nthreads) { // (a launch of several passes has the threads of the largest; they come in whole waves)
-        const int lane = tid & 63;
+    const auto fetch_into = [&](auto kt) { // (a launch of several passes has the threads of the largest; they come in whole waves)
+        if (tid >= nthreads) return;
         float v[16];
-        if (a.kt == 13) {
-            const int c = (tid & ~63) | ((lane & 31) << 1) | (lane >> 5);
-            fetch_chunk<ENDS>(v, x, in, e, cen, origin + c * 16);
-            butterflies<4>(v);
-            swap_lane_bit<32, 0>(v);
-            stage_of<0>(v); // e4
-            float *slot = lds + pad_idx(((c >> 1) << 5) | (lane >> 5));
-#pragma unroll
-            for (int i = 0; i < 16; i++) slot[((i & 1) << 4) | (i & 14)] = v[i];
-        } else if (a.kt == 14) {
-            const int c = (tid & ~63) | ((lane & 15) << 2) | (((lane >> 4) & 1) << 1) | (lane >> 5);
-            fetch_chunk<ENDS>(v, x, in, e, cen, origin + c * 16);
-            butterflies<4>(v);
-            swap_lane_bit<32, 1>(v);
-            stage_of<1>(v); // e4
-            swap_lane_bit<16, 0>(v);
-            stage_of<0>(v); // e5
-            float *slot = lds + pad_idx(((c >> 2) << 6) | ((lane >> 5) << 1) | ((lane >> 4) & 1));
-#pragma unroll
-            for (int i = 0; i < 16; i++) slot[pad_idx(((i & 1) << 5) | (((i >> 1) & 1) << 4) | (i & 12))] = v[i];
-        } else {
-            fetch_chunk<ENDS>(v, x, in, e, cen, origin + tid * 16);
-            butterflies<4>(v);
-            float *slot = lds + chunk_word(tid);
-#pragma unroll
-            for (int i = 0; i < 16; i++) slot[i] = v[i];
-        }
-    }
+        fetch_chunk<ENDS>(v, x, in, e, cen, origin + chunk_of<decltype(kt)::value>(tid) * 16);
+        chunk_into_tile<decltype(kt)::value>(v, lds, tid);
+    };
+    if (a.kt == 13)
+        fetch_into(std::integral_constant<int, 13>());
+    else if (a.kt == 14)
+        fetch_into(std::integral_constant<int, 14>());
+    else
+        fetch_into(std::integral_constant<int, 12>()); // (and below)
     __syncthreads();
     const int step = blockDim.x;
     switch (a.kt) {
-    case 10: lds_pass<4, 2>(lds, 10, tid, step); break;
-    case 11: lds_pass<4, 3>(lds, 11, tid, step); break;
-    case 12: lds_pass<4, 4>(lds, 12, tid, step); break;
-    case 13: lds_pass<5, 4>(lds, 13, tid, step); break;
-    default: lds_pass<6, 4>(lds, 14, tid, step); break;
+    case 10: middle_stages<10>(lds, tid, step); break;
+    case 11: middle_stages<11>(lds, tid, step); break;
+    case 12: middle_stages<12>(lds, tid, step); break;
+    case 13: middle_stages<13>(lds, tid, step); break;
+    default: middle_stages<14>(lds, tid, step); break;
     }
     __syncthreads();
     float *out = x + origin;
@@ -1224,77 +1251,91 @@ __global__ __launch_bounds__(1 << (HB - 4), 8) void rht_compress_split_kernel(
     }
 }
 
-// the inverse: blocks of 2^(HB + 1) in two halves (PAIR), or two blocks of 2^HB per workgroup (PAIR = false)
-template <int NBITS, bool MEE, int HB, bool PAIR = true>
-__global__ __launch_bounds__(1 << (HB - 4), 8) void irht_decompress_split_kernel(const uint8_t *__restrict__ src,
-                                                                             float *__restrict__ x, RhtTileArgs a,
-                                                                             MeeArg<NBITS, MEE> mp)
+// The inverse: a block of 2^HB elements per workgroup, or (PAIR) one of 2^(HB + 1) in two halves.  A thread decodes a chunk of each half,
+// which goes through the LDS twice (chunk_into_tile, middle_stages); the highest four stages, that between the halves, scale and signs
+// are done on the registers that the last trip fills, and stored from there: consecutive lanes hold consecutive elements, a store of a
+// wave is two whole lines, and their 64 signs are two words of the wave.  Bound by memory: the vector ALU is half busy, the LDS 40 %.
+// Four accesses to the LDS per element where tiles read back by chunks took eight, and 6 barriers instead of 13: 2^30 elements in
+// blocks of 2^13, 5 bits, 1,143 -> 990 us (5.1 TB/s; plain instead of non-temporal stores 1,130).
+template <int NBITS, bool MEE, int HB, bool PAIR>
+__global__ __launch_bounds__(1 << (HB - 4), 8) void irht_decompress_kernel(const uint8_t *__restrict__ src, float *__restrict__ x, RhtTileArgs a,
+                                                                       MeeArg<NBITS, MEE> mp)
 {
     typedef Rec<NBITS> RC;
-    constexpr int kThreads = 1 << (HB - 4), kWaves = kThreads / 64;
+    constexpr int kThreads = 1 << (HB - 4), kWaves = kThreads / 64, kParts = PAIR ? 2 : 1;
     extern __shared__ __attribute__((aligned(16))) float lds[];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int row = lane >> 4, j = lane & 15;
-    const int64_t origin = (int64_t)blockIdx.x << (HB + 1);
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int chunk = chunk_of<HB>(lane), row = chunk >> 4, j = chunk & 15;
+    const int64_t origin = (int64_t)blockIdx.x << (HB + (PAIR ? 1 : 0));
+    // the record windows and the MEE table use the LDS before the tile does
     uint8_t *win_in = reinterpret_cast<uint8_t *>(lds) + wave * RC::WIN;
     float *table = reinterpret_cast<float *>(reinterpret_cast<uint8_t *>(lds) + kWaves * RC::WIN);
+    constexpr int kTotal = kRowsPerWave * RC::REC;
+    const auto records = [&](int h) { return src + ((origin >> 8) + h * (kWaves * kRowsPerWave) + wave * kRowsPerWave) * RC::REC; };
+    WinRegs wr[kParts];
+#pragma unroll
+    for (int h = 0; h < kParts; h++) wr[h] = window_fetch(records(h), kTotal, lane);
     if (MEE) {
         for (int k = tid; k < (1 << NBITS); k += kThreads) table[k] = f16_bits_to_f32(mp.table[k]);
         __syncthreads();
     }
-    float va[16], vb[16];
+    float v[kParts][16];
 #pragma unroll
-    for (int h = 0; h < 2; h++) {
-        const int64_t sc0 = (origin >> 8) + h * (kWaves * kRowsPerWave) + wave * kRowsPerWave;
-        const int total = kRowsPerWave * RC::REC;
-        const uint8_t *g = src + sc0 * RC::REC;
-        const WinRegs wr = window_fetch(g, total, lane);
-        const int mis = window_commit(win_in, wr, g, total, lane);
+    for (int h = 0; h < kParts; h++) {
+        const int mis = window_commit(win_in, wr[h], records(h), kTotal, lane);
         wave_lds_sync();
         const uint8_t *rec = win_in + mis + row * RC::REC;
         uint32_t cw[RC::WORDS], cq;
         chunk_read<NBITS>(rec + j * RC::CB, cw, cq);
         const uint32_t ub = (uint32_t)rec[16 * RC::CB] | ((uint32_t)rec[16 * RC::CB + 1] << 8);
-        float t[16];
-        chunk_decode<NBITS, MEE, false>(cw, cq, ub, table, t);
-#pragma unroll
-        for (int i = 0; i < 16; i++) (h ? vb[i] : va[i]) = t[i];
+        chunk_decode<NBITS, MEE, false>(cw, cq, ub, table, v[h]);
         wave_lds_sync(); // the window is reused for the other half
     }
     __syncthreads(); // windows and table are done with: the tile takes the LDS
-    butterflies<4>(va);
-    butterflies<4>(vb);
-    half_block_stages<HB>(va, lds, tid);
-    half_block_stages<HB>(vb, lds, tid);
+#pragma unroll
+    for (int h = 0; h < kParts; h++) {
+        chunk_into_tile<HB>(v[h], lds, tid);
+        __syncthreads();
+        middle_stages<HB>(lds, tid, kThreads);
+        __syncthreads();
+        const float *q = lds + pad_idx(tid);
+#pragma unroll
+        for (int k = 0; k < 16; k++) v[h][k] = q[tuple_step<HB - 4>(k)];
+        butterflies<4>(v[h]);
+        if (h + 1 < kParts) __syncthreads(); // the half has left the LDS
+    }
     if constexpr (PAIR) {
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
-            const float p = va[i], q = vb[i];
-            va[i] = p + q;
-            vb[i] = p - q;
+        for (int k = 0; k < 16; k++) {
+            const float p = v[0][k], q = v[1][k];
+            v[0][k] = p + q;
+            v[1][k] = p - q;
+            asm volatile("" : "+v"(v[1][k])); // (formed behind the stores of the first half, the differences keep both operands alive)
         }
     }
-    // store one half after the other through the LDS, so that every store instruction covers 1 KiB contiguously
-    float *mine = lds + chunk_word(tid);
+    const int64_t first = origin + 64 * wave; // of the wave's 64 consecutive elements
+    float *out = x + first + lane;
 #pragma unroll
-    for (int h = 0; h < 2; h++) {
+    for (int h = 0; h < kParts; h++) {
 #pragma unroll
-        for (int i = 0; i < 16; i++) mine[i] = h ? vb[i] : va[i];
-        __syncthreads();
-        const int64_t half_origin = origin + ((int64_t)h << HB);
-        if (a.vec) {
-            for (int i = tid * 4; i < (1 << HB); i += kThreads * 4) {
-                const int q = pad_idx(i);
-                float4 v = make_float4(lds[q], lds[q + 1], lds[q + 2], lds[q + 3]);
-                v.x *= a.scale; v.y *= a.scale; v.z *= a.scale; v.w *= a.scale;
-                flip4(v, a, half_origin + i);
-                stream_store(reinterpret_cast<float4 *>(x + half_origin + i), v);
+        for (int k = 0; k < 16; k++) v[h][k] *= a.scale;
+        if (a.sign && a.sign_bits) {
+            // (scalar loads, which the compiler makes of nothing it thinks the stores could change)
+            typedef const __attribute__((address_space(4))) uint32_t *constant_words;
+            const constant_words words = (constant_words)(static_cast<const uint32_t *>(a.sign) + (first >> 5));
+#pragma unroll
+            for (int k = 0; k < 16; k++) {
+                const int at = ((h << HB) + (k << (HB - 4))) >> 5;
+                const uint64_t mask = (uint64_t)words[at] | ((uint64_t)words[at + 1] << 32);
+                asm("v_cndmask_b32_e64 %0, %0, -%0, %1" : "+v"(v[h][k]) : "s"(mask));
             }
-        } else {
-            for (int i = tid; i < (1 << HB); i += kThreads)
-                x[half_origin + i] = flip1(lds[pad_idx(i)] * a.scale, a, half_origin + i);
+        } else if (a.sign) {
+            const float *sign = static_cast<const float *>(a.sign) + first + lane;
+#pragma unroll
+            for (int k = 0; k < 16; k++) v[h][k] *= sign[(h << HB) + (k << (HB - 4))];
         }
-        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < 16; k++) __builtin_nontemporal_store(v[h][k], out + (h << HB) + (k << (HB - 4)));
     }
 }
 
@@ -1434,37 +1475,48 @@ hipError_t run_compress(const float *src, const void *sign, int sign_bits, uint8
     return hipGetLastError();
 }
 
+// The inverse, whole blocks or halves: with halves a thread has twice the loads and stores on the way and a block half the waves that
+// meet at its barriers, while the vector leaves twice the threads idle.  us, whole against halves, 5 bits (4 up to 2^23):
+//   blocks of  2^11          2^12          2^13          2^14
+//   2^21        5.3    6.0    4.5    5.6    5.0    6.0    6.3    6.8
+//   2^23        8.6    9.8    8.6   10.8    8.8   10.2   10.4   10.4  (2^22 8.1 against 7.2)
+//   2^25       25.9   29.5   27.0   30.0   28.0   28.0   35.4   28.6
+//   2^26       53.4   54.8   53.2   58.3   57.0   57.0   65.0   60.0
+//   2^28        251    216    252    251    280    248    314    270
+//   2^30       1000    881   1014    992   1124    983   1315   1074
+// Blocks of 2^10 are one wave each (2^30 882 us; two blocks per wave 909), blocks of 2^15 do not fit as a whole.  Quarters and eighths
+// are slower at every size: 100 and 150 registers.
+constexpr int64_t kWholeInverse = (int64_t)1 << 26, kWholeInverse14 = (int64_t)1 << 21;
+
 template <int PRE, int NBITS, bool MEE>
 hipError_t run_decompress(const uint8_t *src, const void *sign, int sign_bits, float *dst, int64_t n, int64_t block, float scale,
                           const MeeParams &mp, hipStream_t stream)
 {
     const Geometry g = geometry(dst, sign, sign_bits, n, block, scale);
-    const bool halves = n > kWholeTiles || g.a.kb == kSplitBits;
-    if (halves && g.a.kb >= 10 && g.a.kb <= kSplitBits && (n & ((g.a.kb == 10 ? 2048 : (1 << g.a.kb)) - 1)) == 0) {
-        // blocks of 2^11 .. 2^15 in two halves per workgroup, blocks of 2^10 two per wave
-        auto launch = [&](auto kernel, int half_bits) -> hipError_t {
-            const size_t tile = (size_t)padded_tile_floats(half_bits) * sizeof(float);
-            const size_t windows = (size_t)((1 << (half_bits - 4)) / 64) * Rec<NBITS>::WIN + (MEE ? (sizeof(float) << NBITS) : 0);
+    if (g.a.kb >= 10 && g.a.kb <= kSplitBits && (n & (((int64_t)1 << g.a.kb) - 1)) == 0) {
+        const auto launch = [&](auto kernel, int part_bits) -> hipError_t {
+            const size_t tile = (size_t)padded_tile_floats(part_bits) * sizeof(float);
+            const size_t windows = (size_t)((1 << (part_bits - 4)) / 64) * Rec<NBITS>::WIN + (MEE ? (sizeof(float) << NBITS) : 0);
             const size_t lds = std::max(tile, windows);
             hipError_t es = allow_lds(kernel, lds);
             if (es != hipSuccess) return es;
-            hipLaunchKernelGGL(kernel, dim3((unsigned)(n >> (half_bits + 1))), dim3(1 << (half_bits - 4)), lds, stream, src, dst, g.a,
-                               make_arg<NBITS, MEE>(mp));
+            hipLaunchKernelGGL(kernel, dim3((unsigned)(n >> g.a.kb)), dim3(1 << (part_bits - 4)), lds, stream, src, dst, g.a, make_arg<NBITS, MEE>(mp));
             return hipGetLastError();
         };
+        const bool whole = n <= (g.a.kb == 14 ? kWholeInverse14 : kWholeInverse);
         switch (g.a.kb) {
-        case 15: return launch(irht_decompress_split_kernel<NBITS, MEE, 14>, 14);
-        case 14: return launch(irht_decompress_split_kernel<NBITS, MEE, 13>, 13);
-        case 13: return launch(irht_decompress_split_kernel<NBITS, MEE, 12>, 12);
-        case 12: return launch(irht_decompress_split_kernel<NBITS, MEE, 11>, 11);
-        case 11: return launch(irht_decompress_split_kernel<NBITS, MEE, 10>, 10);
-        default: return launch(irht_decompress_split_kernel<NBITS, MEE, 10, false>, 10);
+        case 15: return launch(irht_decompress_kernel<NBITS, MEE, 14, true>, 14);
+        case 14: return whole ? launch(irht_decompress_kernel<NBITS, MEE, 14, false>, 14) : launch(irht_decompress_kernel<NBITS, MEE, 13, true>, 13);
+        case 13: return whole ? launch(irht_decompress_kernel<NBITS, MEE, 13, false>, 13) : launch(irht_decompress_kernel<NBITS, MEE, 12, true>, 12);
+        case 12: return whole ? launch(irht_decompress_kernel<NBITS, MEE, 12, false>, 12) : launch(irht_decompress_kernel<NBITS, MEE, 11, true>, 11);
+        case 11: return whole ? launch(irht_decompress_kernel<NBITS, MEE, 11, false>, 11) : launch(irht_decompress_kernel<NBITS, MEE, 10, true>, 10);
+        default: return launch(irht_decompress_kernel<NBITS, MEE, 10, false>, 10);
         }
     }
     if (g.a.kt >= kSplitBits) return hipErrorInvalidValue;
     const size_t windows = (size_t)(g.threads / 64) * Rec<NBITS>::WIN + (MEE ? (sizeof(float) << NBITS) : 0);
     const size_t lds = std::max(g.lds_floats * sizeof(float), windows);
-    auto kernel = irht_decompress_kernel<NBITS, MEE>;
+    auto kernel = irht_decompress_tile_kernel<NBITS, MEE>;
     hipError_t e = allow_lds(kernel, lds);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(kernel, dim3(g.grid), dim3(g.threads), lds, stream, src, dst, g.a, make_arg<NBITS, MEE>(mp));

@@ -134,6 +134,28 @@ def test_whole_tiles_to_halves(capi, block, blocks_more):
         assert torch.equal(back, ref), (nbits, strategy)
 
 
+@pytest.mark.parametrize("block,whole", [(1 << 10, 1 << 16), (1 << 11, 1 << 26), (1 << 12, 1 << 26), (1 << 13, 1 << 26), (1 << 14, 1 << 21)])
+@pytest.mark.parametrize("blocks_more", [0, 1])
+def test_inverse_whole_blocks_to_halves(capi, block, whole, blocks_more):
+    """where the inverse goes from a block per workgroup to two halves, against the two calls: signs as bits, as floats, none, and
+    outputs and records that are not aligned"""
+    n = whole + blocks_more * block
+    x = torch.randn(n, generator=torch.Generator(device=DEV).manual_seed(block + blocks_more), device=DEV) * 1e-3
+    sign = torch.empty(n // 32, dtype=torch.int32, device=DEV)
+    capi.rand_diag_bits(sign, n, 7)
+    floats = 1.0 - 2.0 * ((sign.view(-1, 1) >> torch.arange(32, dtype=torch.int32, device=DEV)) & 1).view(-1).float()
+    scale = 1.0 / block ** 0.5
+    for nbits, strategy, diagonal in ((2, 2, sign), (4, 3, None), (5, 2, sign), (8, 3, floats)):
+        enc = torch.zeros(capi.required_bytes(n, nbits, 16, strategy) + 3, dtype=torch.uint8, device=DEV)[3:]
+        capi.scaling_compress_philox(x, enc, n, nbits, 16, strategy, 3, 4)
+        ref = torch.empty_like(x)
+        capi.scaling_decompress(enc, ref, n, nbits, 16, strategy)
+        capi.rht_blocked(ref, diagonal, block, scale, True)
+        back = torch.empty(n + 1, device=DEV)[1:]
+        capi.scaling_decompress_irht(enc, diagonal, back, block, scale, nbits, strategy)
+        assert torch.equal(back.view(torch.int32), ref.view(torch.int32)), (nbits, strategy)
+
+
 @pytest.mark.parametrize("n,block", [(256, 256), (256, 16), (512, 512), (768, 256), (1280, 256), (2048, 1024)])
 def test_small_vectors_no_sign_unaligned(capi, n, block):
     g, x, _ = _case(n, n + block)
