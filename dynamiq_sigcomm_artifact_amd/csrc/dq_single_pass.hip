@@ -92,13 +92,10 @@ __device__ __forceinline__ void store_tile(void *dst, const Raw16<DT> &out, cons
 }
 
 // T(T(level * step) + mean)
-template <class RV> __device__ __forceinline__ void decode_with_mean(RV &out, float (&lev)[RV::kCount], float step, float mean)
+template <int DT, class RV> __device__ __forceinline__ void decode_with_mean(RV &out, float (&lev)[RV::kCount], float step, float mean)
 {
 #pragma unroll
-    for (int i = 0; i < RV::kCount; i++) lev[i] = lev[i] * step;
-    out.set(lev);
-#pragma unroll
-    for (int i = 0; i < RV::kCount; i++) lev[i] = out.get(i) + mean;
+    for (int i = 0; i < RV::kCount; i++) lev[i] = round_element<DT>(lev[i] * step) + mean;
     out.set(lev);
 }
 
@@ -191,10 +188,10 @@ template <int DT, bool MEE> __global__ __launch_bounds__(64) void roundtrip_kern
     if (sc0 == 0 && lane < 4) b.counts[lane] = 0; // (tally_kernel adds to them)
 
     const WidthRegs<MEE> w = width_regs<MEE>(a.widths, class_of_norm(norm, u, a.rule.thr), levels);
-    center_loaded<DT>(v, a.wd, active ? mean : 0.0f, e0, n, ragged);
-    float lev[16];
-    const float scale = quantize_chunk<MEE>(v, r, w, lev);
-    decode_with_mean(v, lev, scale, bf16_bits_to_f32(mean_bits));
+    float x[16], lev[16];
+    center_loaded<DT>(x, v, a.wd, active ? mean : 0.0f, e0, n, ragged);
+    const float scale = quantize_chunk<MEE>(x, r, w, lev);
+    decode_with_mean<DT>(v, lev, scale, bf16_bits_to_f32(mean_bits));
     wave_lds_sync(); // the statistics' tile has been read
     stage_tile<DT>(v, reinterpret_cast<uint4 *>(lds), lane);
     store_tile<DT>(b.out, v, reinterpret_cast<const uint4 *>(lds), sc, rows_here, n, b.vec != 0, lane);
@@ -508,11 +505,10 @@ template <int DT, int RDT, bool MEE> __global__ __launch_bounds__(64) void ring_
         }
     };
     fetch(0);
-    Raw16<DT> v;
     float lev[16], scale = 0.0f;
 #pragma unroll 1
     for (int step = 0; step < world; step++) {
-        v = next;
+        const Raw16<DT> v = next;
         Raw16<RDT> r = next_r;
         const float mean = next_mean;
         if (step + 1 < world) fetch(step + 1);
@@ -521,17 +517,18 @@ template <int DT, int RDT, bool MEE> __global__ __launch_bounds__(64) void ring_
             if (rank >= world) rank -= world;
             r.generate(RandKey{a.key.seed + (uint64_t)rank, (uint64_t)step}, sc * 16 + j);
         }
-        center_loaded<DT>(v, a.wd, mean, e0, a.n, ragged);
-        if (step > 0) {
+        float x[16];
+        center_loaded<DT>(x, v, a.wd, mean, e0, a.n, ragged);
+        if (step > 0) { // the sum, in the element type
 #pragma unroll
-            for (int i = 0; i < 16; i++) lev[i] = __builtin_fmaf(lev[i], scale, v.get(i));
-            v.set(lev); // the sum in the element type
+            for (int i = 0; i < 16; i++) x[i] = round_element<DT>(__builtin_fmaf(lev[i], scale, x[i]));
         }
-        scale = quantize_chunk<MEE>(v, r, w, lev);
+        scale = quantize_chunk<MEE>(x, r, w, lev);
     }
-    decode_with_mean(v, lev, scale, bf16_bits_to_f32(total_mean));
-    stage_tile<DT>(v, stage, lane);
-    for (int rank = 0; rank < world; rank++) store_tile<DT>(a.out[rank], v, stage, sc, rows_here, a.n, (a.vec & 2) != 0, lane);
+    Raw16<DT> out;
+    decode_with_mean<DT>(out, lev, scale, bf16_bits_to_f32(total_mean));
+    stage_tile<DT>(out, stage, lane);
+    for (int rank = 0; rank < world; rank++) store_tile<DT>(a.out[rank], out, stage, sc, rows_here, a.n, (a.vec & 2) != 0, lane);
 }
 
 // four elements of a lane, side by side with those of its neighbours
@@ -620,12 +617,11 @@ __global__ __launch_bounds__(64 * kQuadWaves) void ring_quad_kernel(RingArgs<RDT
         if constexpr (RDT != DQ_PHILOX) next_r.load(of_step(my_pool, step), lane * 4, (a.vec & 4) != 0);
     };
     fetch(0);
-    Raw4<DT> v;
     uint32_t draws[4];
     float lev[4], scale = 0.0f;
 #pragma unroll 1
     for (int step = 0; step < world; step++) {
-        v = next;
+        const Raw4<DT> v = next;
         Raw4<RDT> r = next_r;
         const float mean = __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(my_mean), step));
         if (step + 1 < world) fetch(step + 1);
@@ -639,16 +635,17 @@ __global__ __launch_bounds__(64 * kQuadWaves) void ring_quad_kernel(RingArgs<RDT
             r.w = draws[0];
             draws[0] = draws[1]; draws[1] = draws[2]; draws[2] = draws[3];
         }
-        center_loaded<DT>(v, a.wd, mean, e0, a.n, ragged);
-        if (step > 0) {
+        float x[4];
+        center_loaded<DT>(x, v, a.wd, mean, e0, a.n, ragged);
+        if (step > 0) { // the sum, in the element type
 #pragma unroll
-            for (int i = 0; i < 4; i++) lev[i] = __builtin_fmaf(lev[i], scale, v.get(i));
-            v.set(lev); // the sum in the element type
+            for (int i = 0; i < 4; i++) x[i] = round_element<DT>(__builtin_fmaf(lev[i], scale, x[i]));
         }
-        scale = quantize_chunk<MEE>(v, r, w, lev);
+        scale = quantize_chunk<MEE>(x, r, w, lev);
     }
-    decode_with_mean(v, lev, scale, bf16_bits_to_f32(total_mean));
-    for (int rank = 0; rank < world; rank++) store_quarter<DT>(a.out[rank], v, e0, a.n, (a.vec & 2) != 0, ragged);
+    Raw4<DT> out;
+    decode_with_mean<DT>(out, lev, scale, bf16_bits_to_f32(total_mean));
+    for (int rank = 0; rank < world; rank++) store_quarter<DT>(a.out[rank], out, e0, a.n, (a.vec & 2) != 0, ragged);
 }
 
 // Up to so many superchunks one per wave, beyond it four: the quads issue more per element (160 instructions per superchunk and

@@ -5,6 +5,13 @@
 //
 // The levels are those of chunk_encode_* followed by chunk_decode (dq_hier16_tiles.cuh), operation by operation; a code
 // travels as the float level it decodes to instead of a bit field.
+//
+// The kernels on it are bound by the vector ALU.  Additions, products, fused multiply-adds, bitwise operations and right shifts on vector
+// registers and constants issue a wave in 1.2 ns, everything else -- conversions, comparisons, minima, left shifts, double precision,
+// and all of them with a scalar operand -- in 2.2.  So elements stay binary32 numbers in the precision of their type (round_element), the
+// largest and the least of a lane's values come two to an instruction, and the scale byte from an estimate (chunk_ratio).  Kernels, us:
+// one rank, nine 25 MB buckets 46.8 -> 44.1 (MEE 62.7 -> 61.0), ring of 8 x 1,000,003 14.2 -> 13.5 (MEE 16.2 -> 15.4), of 8 x 33,000,001 in
+// MEE 277 -> 256; 8 x 124,439,808 in AEE, which memory bounds, 723 -> 725.
 #pragma once
 
 #include "dq_hier16_tiles.cuh"
@@ -107,12 +114,6 @@ template <> struct Raw4<DQ_BF16> {
         w[0] = f32x2_to_bf16x2(t[0], t[1]);
         w[1] = f32x2_to_bf16x2(t[2], t[3]);
     }
-    // of the lane's four elements, as those of Raw16
-    __device__ __forceinline__ uint32_t absmax_bits() const
-    {
-        const uint32_t m = pk_max_u16(w[0] & 0x7fff7fffu, w[1] & 0x7fff7fffu);
-        return max(m << 16, m & 0xffff0000u);
-    }
     __device__ __forceinline__ bool unit_interval() const
     {
         const uint32_t m = pk_max_u16(w[0], w[1]);
@@ -140,10 +141,6 @@ template <> struct Raw4<DQ_F32> {
     {
 #pragma unroll
         for (int k = 0; k < 4; k++) w[k] = __float_as_uint(t[k]);
-    }
-    __device__ __forceinline__ uint32_t absmax_bits() const
-    {
-        return max(max(w[0] & 0x7fffffffu, w[1] & 0x7fffffffu), max(w[2] & 0x7fffffffu, w[3] & 0x7fffffffu));
     }
     __device__ __forceinline__ bool unit_interval() const { return max(max(w[0], w[1]), max(w[2], w[3])) <= 0x3f800000u; }
 };
@@ -231,15 +228,71 @@ template <int N> __device__ __forceinline__ float superchunk_max(float v)
     }));
 }
 
+// largest magnitude of N values; NaN if one of them is not a number (v_maximum3_f32: two values per instruction)
+template <int N> __device__ __forceinline__ float abs_maximum(const float (&x)[N])
+{
+    float m = __builtin_fabsf(x[0]);
+#pragma unroll
+    for (int i = 1; i + 1 < N; i += 2)
+        m = __builtin_elementwise_maximum(__builtin_elementwise_maximum(m, __builtin_fabsf(x[i])), __builtin_fabsf(x[i + 1]));
+    return N % 2 ? m : __builtin_elementwise_maximum(m, __builtin_fabsf(x[N - 1]));
+}
+
+// the least of N numbers
+template <int N> __device__ __forceinline__ float minimum(const float (&x)[N])
+{
+    float m = x[0];
+#pragma unroll
+    for (int i = 1; i + 1 < N; i += 2) m = __builtin_elementwise_minimum(__builtin_elementwise_minimum(m, x[i]), x[i + 1]);
+    return N % 2 ? m : __builtin_elementwise_minimum(m, x[N - 1]);
+}
+
+// A copy of a lane's random words about which the compiler knows nothing: for a rare path that takes its values from them again, instead
+// of keeping all of them in registers for it.
+template <class RR> __device__ __forceinline__ RR forgotten(const RR &r)
+{
+    static_assert(sizeof(RR) % 4 == 0, "words");
+    union {
+        RR r;
+        uint32_t w[sizeof(RR) / 4];
+    } u = {r};
+#pragma unroll
+    for (size_t k = 0; k < sizeof(RR) / 4; k++) asm volatile("" : "+v"(u.w[k]));
+    return u.r;
+}
+
+// ceil(fl(fl(s / g) * 255)) between 1 and 255, for 1e-7 <= s <= g <= 2^101.  The estimate with the hardware's reciprocal (1 ulp) errs by
+// less than 255 (2^-22 + 2^-23) = 9.2e-5 and decides where no integer is within 2^-13 of it; above 254 the result is 255 whatever it
+// is, which settles the row's largest chunk (s = g).
+__device__ __forceinline__ float chunk_ratio(float s, float g)
+{
+    float ratio = (s * __builtin_amdgcn_rcpf(g)) * 255.0f;
+    const bool doubt = __builtin_fabsf(ratio - __builtin_rintf(ratio)) < 0x1p-13f && ratio < 254.5f;
+    if (__builtin_amdgcn_ballot_w64(doubt) != 0) {
+        asm volatile(""); // (a branch of the wave that the compiler keeps)
+        if (doubt) ratio = div_by(s, recip_f64(g)) * 255.0f;
+    }
+    return __builtin_amdgcn_fmed3f(__builtin_ceilf(ratio), 1.0f, 255.0f);
+}
+
+// t in the precision of the element type.  A bfloat16 behind a zero is its own binary32 pattern: one conversion, where a pair of
+// bfloat16 takes two more instructions to be floats again.
+template <int DT> __device__ __forceinline__ float round_element(float t)
+{
+    if constexpr (DT == DQ_F32)
+        return t;
+    else
+        return __uint_as_float(f32x2_to_bf16x2(0.0f, t));
+}
+
 // the quantiser with every guard of the reference (chunk_encode_guarded): lev[i] = level of element i, returns the
 // chunk's step (chunk_decode's sc)
-template <bool MEE, class RV, class RR>
-__device__ __forceinline__ float quantize_guarded(const RV &v, const RR &rnd, const WidthRegs<MEE> &w, float (&lev)[RV::kCount])
+template <bool MEE, int N, class RR>
+__device__ __forceinline__ float quantize_guarded(const float (&v)[N], const RR &rnd, const WidthRegs<MEE> &w, float (&lev)[N])
 {
-    constexpr int N = RV::kCount;
-    float a = __builtin_fabsf(v.get(0));
+    float a = __builtin_fabsf(v[0]);
 #pragma unroll
-    for (int i = 1; i < N; i++) a = __builtin_fmaxf(a, __builtin_fabsf(v.get(i)));
+    for (int i = 1; i < N; i++) a = __builtin_fmaxf(a, __builtin_fabsf(v[i]));
     a = chunk_max<N>(a);
     const float s = pos_scale(MEE ? a / pos_scale(w.cmm) + 1e-7f : a / w.r + 1e-7f);
     const float g = pos_scale(superchunk_max<N>(s));
@@ -252,7 +305,7 @@ __device__ __forceinline__ float quantize_guarded(const RV &v, const RR &rnd, co
     const int top = (int)w.r;
 #pragma unroll
     for (int i = 0; i < N; i++) {
-        float x = v.get(i) / d;
+        float x = v[i] / d;
         if (MEE) x = mee_inverse_guarded(x, w.c, w.l2b);
         const int level = clamp_code(sr_guarded(x, rnd.get(i)), top) - top;
         lev[i] = MEE ? w.table[level] : (float)level;
@@ -263,43 +316,41 @@ __device__ __forceinline__ float quantize_guarded(const RV &v, const RR &rnd, co
 // chunk_encode_fast + estimate_codes: elements finite and <= 2^100, random values in [0, 1].  The estimate is that of
 // L - r + 1 instead of L - r + R + 1 -- its floor is the signed level -- against the same guard: the constant 1 + kDelta
 // minus r is as exact (1 and 20 bits of fraction), and the fused multiply-add rounds a number of less magnitude.
-template <bool MEE, class RV, class RR>
-__device__ __forceinline__ float quantize_fast(const RV &v, const RR &rnd, uint32_t amax_bits, const WidthRegs<MEE> &w, float (&lev)[RV::kCount])
+// The guard: the estimate's distance from its floor, the least of the lane's first (v_minimum3_f32, two per instruction), and where any lane of
+// the wave is in doubt the elements that are.
+template <bool MEE, int N, class RR>
+__device__ __forceinline__ float quantize_fast(const float (&v)[N], const RR &rnd, float amax, const WidthRegs<MEE> &w, float (&lev)[N])
 {
-    constexpr int N = RV::kCount;
-    const float s = div_by(__uint_as_float(amax_bits), w.inv_top) + 1e-7f; // (2 bits: R = 1, the product with 1)
+    const float s = div_by(amax, w.inv_top) + 1e-7f; // (2 bits: R = 1, the product with 1)
     const float g = superchunk_max_pos<N>(s);
     const float unit = bf16_bits_to_f32(f32_to_bf16_bits(div_by(g, 1.0 / 255.0)));
-    const float ratio = div_by(s, recip_f64(g)) * 255.0f;
-    const int qi = min(max((int)__builtin_ceilf(ratio), 1), 255);
-    const float d = (float)qi * unit;
+    const float q = chunk_ratio(s, g);
+    const float d = q * unit;
     const float rd = __builtin_amdgcn_rcpf(d);
     const float rc = MEE ? (float)w.inv_c : 0.0f, rl2b = MEE ? (float)w.inv_l2b : 0.0f;
-    bool doubt[N];
-    uint64_t lanes_in_doubt[N], any = 0;
+    float above[N];
 #pragma unroll
     for (int i = 0; i < N; i++) {
-        const float vi = v.get(i);
         const float off = below(rnd, i, w.bias);
         float t;
         if (MEE)
-            t = __builtin_fmaf(__builtin_amdgcn_logf(__builtin_fmaf(__builtin_fabsf(vi * rd), rc, 1.0f)), __builtin_copysignf(rl2b, vi), off);
+            t = __builtin_fmaf(__builtin_amdgcn_logf(__builtin_fmaf(__builtin_fabsf(v[i] * rd), rc, 1.0f)), __builtin_copysignf(rl2b, v[i]), off);
         else
-            t = __builtin_fmaf(vi, rd, off);
+            t = __builtin_fmaf(v[i], rd, off);
         // (floor and not t minus its fraction: in -2^-25 < t < 0 the fraction rounds to 1 - 2^-24 and the difference is not -1)
         const float fl = __builtin_floorf(t);
-        doubt[i] = t - fl < w.two_delta;
-        lanes_in_doubt[i] = __builtin_amdgcn_ballot_w64(doubt[i]);
-        any |= lanes_in_doubt[i];
+        above[i] = t - fl;
         lev[i] = __builtin_amdgcn_fmed3f(fl, -w.r, w.r);
     }
-    if (any != 0) {
+    if (__builtin_amdgcn_ballot_w64(minimum(above) < w.two_delta) != 0) {
+        const RR again = forgotten(rnd);
         const double yd = recip_f64(d);
 #pragma unroll
         for (int i = 0; i < N; i++) {
-            if (lanes_in_doubt[i] != 0) {
-                const float sv = (float)exact_code_fast<MEE>(v.get(i), rnd.get(i), d, yd, w);
-                if (doubt[i]) lev[i] = __builtin_amdgcn_fmed3f(sv, -w.r, w.r);
+            const bool doubt = above[i] < w.two_delta;
+            if (__builtin_amdgcn_ballot_w64(doubt) != 0) {
+                const float sv = (float)exact_code_fast<MEE>(v[i], again.get(i), d, yd, w);
+                if (doubt) lev[i] = __builtin_amdgcn_fmed3f(sv, -w.r, w.r);
             }
         }
     }
@@ -307,16 +358,17 @@ __device__ __forceinline__ float quantize_fast(const RV &v, const RR &rnd, uint3
 #pragma unroll
         for (int i = 0; i < N; i++) lev[i] = w.table[(int)lev[i]];
     }
-    return nonneg_scale((float)qi * nonneg_scale(unit));
+    return nonneg_scale(q * nonneg_scale(unit));
 }
 
 // levels of the lane's elements and step of their chunk; every lane of the wave must call
-template <bool MEE, class RV, class RR>
-__device__ __forceinline__ float quantize_chunk(const RV &v, const RR &rnd, const WidthRegs<MEE> &w, float (&lev)[RV::kCount])
+template <bool MEE, int N, class RR>
+__device__ __forceinline__ float quantize_chunk(const float (&v)[N], const RR &rnd, const WidthRegs<MEE> &w, float (&lev)[N])
 {
-    const uint32_t amax = chunk_max<RV::kCount>(v.absmax_bits());
+    // (the pattern of a NaN is above that of infinity)
+    const uint32_t amax = chunk_max<N>(__float_as_uint(abs_maximum(v)));
     const bool lane_fast = amax <= kFastMaxBits && rnd.unit_interval();
-    if (__builtin_amdgcn_ballot_w64(!lane_fast) == 0) return quantize_fast<MEE>(v, rnd, amax, w, lev);
+    if (__builtin_amdgcn_ballot_w64(!lane_fast) == 0) return quantize_fast<MEE>(v, rnd, __uint_as_float(amax), w, lev);
     return quantize_guarded<MEE>(v, rnd, w, lev);
 }
 
@@ -386,18 +438,19 @@ __device__ __forceinline__ void load_chunk(RV &v, const void *src, int64_t e0, i
         load_chunk_guarded<DT>(v, src, e0, n);
 }
 
-// v becomes T(v / world - mean), zero at and beyond element n of the vector (center_chunk without its own loads)
+// t = T(v / world - mean), zero at and beyond element n of the vector (center_chunk without its own loads)
 template <int DT, class RV>
-__device__ __forceinline__ void center_loaded(RV &v, const WorldDiv &wd, float mean, int64_t e0, int64_t n, bool ragged)
+__device__ __forceinline__ void center_loaded(float (&t)[RV::kCount], const RV &v, const WorldDiv &wd, float mean, int64_t e0, int64_t n, bool ragged)
 {
     constexpr int N = RV::kCount;
-    float t[N];
+    float inv = wd.inv;
+    asm("" : "+v"(inv)); // (an instruction with a scalar operand takes nearly twice the time of one without)
     if (DT != DQ_F32 && wd.fuse16) {
 #pragma unroll
-        for (int i = 0; i < N; i++) t[i] = __builtin_fmaf(v.get(i), wd.inv, -mean);
+        for (int i = 0; i < N; i++) t[i] = __builtin_fmaf(v.get(i), inv, -mean);
     } else if (wd.pow2) {
 #pragma unroll
-        for (int i = 0; i < N; i++) t[i] = v.get(i) * wd.inv - mean;
+        for (int i = 0; i < N; i++) t[i] = v.get(i) * inv - mean;
     } else {
 #pragma unroll
         for (int i = 0; i < N; i++) t[i] = v.get(i);
@@ -408,9 +461,14 @@ __device__ __forceinline__ void center_loaded(RV &v, const WorldDiv &wd, float m
     if (ragged) {
         const int left = left_here(n, e0, N);
 #pragma unroll
-        for (int i = 0; i < N; i++) t[i] = i < left ? t[i] : 0.0f;
+        for (int i = 0; i < N; i++) {
+            // (in place: as a selection the tiles that are not ragged copy every element)
+            const uint64_t inside = __builtin_amdgcn_ballot_w64(i < left);
+            asm volatile("v_cndmask_b32_e64 %0, 0, %0, %1" : "+v"(t[i]) : "s"(inside));
+        }
     }
-    v.set(t);
+#pragma unroll
+    for (int i = 0; i < N; i++) t[i] = round_element<DT>(t[i]);
 }
 
 // ---- statistics of a tile of four superchunks -----------------------------------------------------------

@@ -710,6 +710,35 @@ def test_ranks_in_registers_equal_the_ring_in_steps(capi, W, n, dt):
         assert all(torch.equal(bits_t(x), bits_t(y)) for x, y in zip(again, ref))
 
 
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("strategy", [2, 3])
+@pytest.mark.parametrize("W,nsc", [(1, 510), (2, 510), (2, 8704)])
+def test_chunk_scales_on_whole_ratios(capi, W, nsc, strategy, dt):
+    """chunks whose scale is k / 255 of their superchunk's, and a few float32 steps beside it: the scale byte is the ceiling of a number
+    on, just below or just above an integer, which the levels in registers estimate and the packed streams divide out"""
+    from dynamiq_sigcomm_artifact_amd.dynamiq_pipeline import _single_pass_in_steps, dynamic_bitrate_allreduce_single_pass
+    rng = np.random.default_rng(nsc + strategy)
+    top = np.exp(rng.uniform(np.log(1e-3), np.log(1e3), (nsc, 1)))
+    r = np.array([127.0, 7.0, 1.0])[np.arange(nsc) % 3][:, None]
+    k = rng.integers(1, 256, (nsc, 16)).astype(np.float64)
+    k[:, 0] = 255.0
+    a = np.maximum((k / 255.0 * (top * W / r + 1e-7) - 1e-7) * r, 0.0).astype(np.float32)
+    steps = rng.integers(-3, 4, (nsc, 16))
+    steps[:, 0] = 0
+    for _ in range(3):
+        a = np.where(steps > 0, np.nextafter(a, np.float32(np.inf)), np.where(steps < 0, np.nextafter(a, np.float32(0.0)), a))
+        steps = steps - np.sign(steps)
+    # (every value with its negative: the means are zero and the centring changes nothing)
+    body = a[:, :, None] * rng.uniform(0.0, 1.0, (nsc, 16, 8)).astype(np.float32)
+    body[:, :, 3] = a
+    x = torch.from_numpy(np.concatenate([body, -body], axis=2).reshape(-1)).to(DEV).to(dt)
+    vecs = [x] + [torch.zeros_like(x) for _ in range(W - 1)]
+    outs, _, counts = dynamic_bitrate_allreduce_single_pass(vecs, 6.0, strategy=strategy, seed=11)
+    ref, _, counts2 = _single_pass_in_steps(vecs, 6.0, strategy, 11, None, {}, None, None)
+    assert counts.tolist() == counts2.tolist()
+    assert all(torch.equal(bits_t(p), bits_t(q)) for p, q in zip(outs, ref))
+
+
 @pytest.mark.parametrize("W,n", [(2, 256 * 8192), (3, 256 * 8192 + 1), (5, 256 * 8195)])
 def test_ranks_on_either_side_of_a_superchunk_per_wave(capi, W, n):
     """the last length that takes a wave per superchunk (MEE; AEE below) and the first ones that take four superchunks per wave"""
