@@ -13,10 +13,10 @@
 //   ring_kernel        W ranks, after a plan of the reduced statistics: the ring
 //   ring_quad_kernel   the same on short vectors, one superchunk per wave
 //
-// Measured, start -> now (bit-identical results): 8 ranks x 124,439,808 bf16 elements 2,896 -> 1,080 us per all-reduce (one
+// Measured, start -> now (bit-identical results): 8 ranks x 124,439,808 bf16 elements 2,896 -> 1,066 us per all-reduce (one
 // launch per rank and ring step, packed streams and their exchange copies, against three launches whose traffic is the
-// vectors alone), 8 x 1,000,003 elements 1,488 -> 25.6 us (257 launches against 3), a step of nine 25 MB buckets on one rank
-// 252 -> 53 us (four launches per bucket on two streams against two launches per step, and the search for u).
+// vectors alone), 8 x 1,000,003 elements 1,488 -> 24.6 us (257 launches against 3), a step of nine 25 MB buckets on one rank
+// 252 -> 51 us (four launches per bucket on two streams against two launches per step, and the search for u).
 //
 // Numerics: csrc/cuda_hadamard.cu:1257-1369 (centring, mean add), csrc/cuda_hierarchical_mee.cu:203-696 (codec),
 // testbed_evaluation/new_comm_hooks/ring_rdma.py:590-631 (order of the ring), comm_hooks.py:64-70 (widths).
@@ -448,7 +448,9 @@ template <bool POOL> struct RingArgs {
 // Workgroup (x, y): tile x of ring chunk y -- rank y compresses it first, rank y + 1 decodes, adds and recompresses, and
 // so on around the ring; the last one's records are what every rank decodes.  The runs of the chunk follow one another as in
 // dq_scaling_mixed.hip (8-bit, 4-bit, 2-bit), so a wave has one width and one first rank.
-template <int DT, int RDT, bool MEE> __global__ __launch_bounds__(64) void ring_kernel(RingArgs<RDT != DQ_PHILOX> a)
+// (Held to five waves per SIMD, 96 registers, where the compiler takes 97 by itself: the longest vectors wait for memory.)
+template <int DT, int RDT, bool MEE>
+__global__ __launch_bounds__(64, DT == DQ_BF16 && RDT == DQ_PHILOX && !MEE ? 5 : 1) void ring_kernel(RingArgs<RDT != DQ_PHILOX> a)
 {
     __shared__ __attribute__((aligned(16))) uint4 stage[64 * Raw16<DT>::kSlots];
     __shared__ float levels[MEE ? kLevelCount : 1];

@@ -10,8 +10,8 @@
 // registers and constants issue a wave in 1.2 ns, everything else -- conversions, comparisons, minima, left shifts, double precision,
 // and all of them with a scalar operand -- in 2.2.  So elements stay binary32 numbers in the precision of their type (round_element), the
 // largest and the least of a lane's values come two to an instruction, and the scale byte from an estimate (chunk_ratio).  Kernels, us:
-// one rank, nine 25 MB buckets 46.8 -> 44.1 (MEE 62.7 -> 61.0), ring of 8 x 1,000,003 14.2 -> 13.5 (MEE 16.2 -> 15.4), of 8 x 33,000,001 in
-// MEE 277 -> 256; 8 x 124,439,808 in AEE, which memory bounds, 723 -> 725.
+// one rank, nine 25 MB buckets 46.9 -> 43.1 (MEE 64 -> 60.3), ring of 8 x 1,000,003 14.4 -> 12.6 (MEE 16.0 -> 14.6), of 8 x 33,000,001 in
+// MEE 265 -> 255; 8 x 124,439,808 in AEE, which memory bounds, 723 -> 725.
 #pragma once
 
 #include "dq_hier16_tiles.cuh"
@@ -20,8 +20,8 @@ namespace dq {
 
 // 8, 4 and 2 bits, in this order everywhere
 struct WidthConst {
-    double inv_top;            // 1 / R (AEE) or 1 / chunk_max_mee (MEE)
     double inv_c, inv_l2b;     // MEE
+    float inv_top;             // of R (AEE) or chunk_max_mee (MEE)
     float r;                   // R = 2^(bits - 1) - 1
     float bias, two_delta;     // of the level estimate: 1 + kDelta, 2 kDelta
     float c, cmm, l2b;         // MEE
@@ -37,8 +37,8 @@ struct WidthSet {
 
 // one width's constants in registers; table: its level zero among the floats in LDS (MEE)
 template <bool MEE> struct WidthRegs {
-    double inv_top, inv_c, inv_l2b;
-    float r, bias, two_delta, c, cmm, l2b;
+    double inv_c, inv_l2b;
+    float inv_top, r, bias, two_delta, c, cmm, l2b;
     const float *table;
 };
 
@@ -261,18 +261,31 @@ template <class RR> __device__ __forceinline__ RR forgotten(const RR &r)
     return u.r;
 }
 
+// The binary32 quotient a / b by a constant, y its rounded reciprocal: a product and one correction, the correctly rounded quotient for b =
+// 255, the greatest levels and the chunk maxima of the MEE lattices (every significand of a tried: tests/test_exact_division.py).
+// Where a is so small that the remainder is not exact, a / b disappears in the sum with 1e-7.  (Two operations where the product with a
+// reciprocal in double takes three, two of them conversions.)
+__device__ __forceinline__ float divide_by_constant(float a, float b, float y)
+{
+    const float q = a * y;
+    return __builtin_fmaf(__builtin_fmaf(-q, b, a), y, q);
+}
+
 // ceil(fl(fl(s / g) * 255)) between 1 and 255, for 1e-7 <= s <= g <= 2^101.  The estimate with the hardware's reciprocal (1 ulp) errs by
-// less than 255 (2^-22 + 2^-23) = 9.2e-5 and decides where no integer is within 2^-13 of it; above 254 the result is 255 whatever it
-// is, which settles the row's largest chunk (s = g).
+// less than 255 (2^-22 + 2^-23) + 2^-17 < 2^-13 = e, so floor(estimate + e) + 1 is the ceiling where no integer lies within e of the
+// estimate; above 254 it is 255 whatever the ratio, which settles the row's largest chunk (s = g).
 __device__ __forceinline__ float chunk_ratio(float s, float g)
 {
-    float ratio = (s * __builtin_amdgcn_rcpf(g)) * 255.0f;
-    const bool doubt = __builtin_fabsf(ratio - __builtin_rintf(ratio)) < 0x1p-13f && ratio < 254.5f;
+    constexpr float e = 0x1p-13f;
+    const float above = __builtin_fminf(__builtin_fmaf(s * __builtin_amdgcn_rcpf(g), 255.0f, e), 254.75f);
+    const float down = __builtin_floorf(above);
+    float q = down + 1.0f;
+    const bool doubt = above - down < 2.0f * e;
     if (__builtin_amdgcn_ballot_w64(doubt) != 0) {
         asm volatile(""); // (a branch of the wave that the compiler keeps)
-        if (doubt) ratio = div_by(s, recip_f64(g)) * 255.0f;
+        if (doubt) q = __builtin_amdgcn_fmed3f(__builtin_ceilf(div_by(s, recip_f64(g)) * 255.0f), 1.0f, 255.0f);
     }
-    return __builtin_amdgcn_fmed3f(__builtin_ceilf(ratio), 1.0f, 255.0f);
+    return q;
 }
 
 // t in the precision of the element type.  A bfloat16 behind a zero is its own binary32 pattern: one conversion, where a pair of
@@ -321,20 +334,21 @@ __device__ __forceinline__ float quantize_guarded(const float (&v)[N], const RR 
 template <bool MEE, int N, class RR>
 __device__ __forceinline__ float quantize_fast(const float (&v)[N], const RR &rnd, float amax, const WidthRegs<MEE> &w, float (&lev)[N])
 {
-    const float s = div_by(amax, w.inv_top) + 1e-7f; // (2 bits: R = 1, the product with 1)
+    const float s = divide_by_constant(amax, MEE ? w.cmm : w.r, w.inv_top) + 1e-7f;
     const float g = superchunk_max_pos<N>(s);
-    const float unit = bf16_bits_to_f32(f32_to_bf16_bits(div_by(g, 1.0 / 255.0)));
-    const float q = chunk_ratio(s, g);
-    const float d = q * unit;
+    const float d = chunk_ratio(s, g) * round_element<DQ_BF16>(divide_by_constant(g, 255.0f, 1.0f / 255.0f));
     const float rd = __builtin_amdgcn_rcpf(d);
     const float rc = MEE ? (float)w.inv_c : 0.0f, rl2b = MEE ? (float)w.inv_l2b : 0.0f;
+    uint32_t top_bit = 0x80000000u;
+    if (MEE) asm("" : "+v"(top_bit));
     float above[N];
 #pragma unroll
     for (int i = 0; i < N; i++) {
         const float off = below(rnd, i, w.bias);
         float t;
         if (MEE)
-            t = __builtin_fmaf(__builtin_amdgcn_logf(__builtin_fmaf(__builtin_fabsf(v[i] * rd), rc, 1.0f)), __builtin_copysignf(rl2b, v[i]), off);
+            t = __builtin_fmaf(__builtin_amdgcn_logf(__builtin_fmaf(__builtin_fabsf(v[i] * rd), rc, 1.0f)),
+                               __uint_as_float(__builtin_amdgcn_bitop3_b32(__float_as_uint(v[i]), top_bit, __float_as_uint(rl2b), 0x6A)), off); // (v & top_bit) ^ rl2b
         else
             t = __builtin_fmaf(v[i], rd, off);
         // (floor and not t minus its fraction: in -2^-25 < t < 0 the fraction rounds to 1 - 2^-24 and the difference is not -1)
@@ -358,7 +372,7 @@ __device__ __forceinline__ float quantize_fast(const float (&v)[N], const RR &rn
 #pragma unroll
         for (int i = 0; i < N; i++) lev[i] = w.table[(int)lev[i]];
     }
-    return nonneg_scale(q * nonneg_scale(unit));
+    return d; // (positive and finite, as its unit is: chunk_decode's guards are for records from elsewhere)
 }
 
 // levels of the lane's elements and step of their chunk; every lane of the wave must call
@@ -387,7 +401,7 @@ inline WidthSet make_width_set(const MeeParams *mp, bool mee)
         w.bias = 1.0f + delta;
         w.two_delta = 2.0f * delta;
         w.c = mp[k].c; w.cmm = mp[k].cmm; w.l2b = mp[k].l2b;
-        w.inv_top = mee ? 1.0 / (double)mp[k].cmm : 1.0 / (double)top;
+        w.inv_top = 1.0f / (mee ? mp[k].cmm : (float)top);
         w.inv_c = 1.0 / (double)mp[k].c;
         w.inv_l2b = 1.0 / (double)mp[k].l2b;
         for (int j = 0; mee && j < (1 << bits[k]); j++) s.levels[kLevels[k] + j] = mp[k].table[j];

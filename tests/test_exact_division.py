@@ -156,3 +156,25 @@ def test_binary16_rounding_of_a_quotient_of_binary16_operands_sees_no_double_rou
     once = q.astype(np.float16)
     twice = q.astype(np.float32).astype(np.float16)
     assert np.array_equal(once.view(np.uint16), twice.view(np.uint16))
+
+
+# ---- divisors that are constants of the widths: a product and one correction ------------------------------------------
+
+def test_division_by_the_constants_of_the_widths_for_every_significand():
+    """divide_by_constant (csrc/dq_widths.cuh): q = RN32(a y), RN32(fma(fma(-q, b, a), y, q)) with y = RN32(1 / b) is the binary32
+    quotient for the divisors it is used with: 255, the greatest levels and the chunk maxima of 8, 4 and 2 bits.  Every significand
+    of a in one binade covers every a whose remainder is exact.  In double the remainder and its product with y are exact; the sum
+    could round twice only by landing on a binary32 tie, which none does."""
+    import ref_model
+    a = np.arange(1 << 23, 1 << 24, dtype=np.float32)
+    top_of = {nbits: 2.0 ** (nbits - 1) - 1 for nbits in (8, 4, 2)}
+    for b in [255.0, *top_of.values(), *(float(ref_model.mee_table(nbits)[2]) for nbits in (8, 4, 2))]:
+        b = np.float32(b)
+        y = np.float32(1.0) / b
+        q = a * y
+        rem = a.astype(np.float64) - q.astype(np.float64) * np.float64(b)
+        assert np.array_equal(rem.astype(np.float32), rem), b
+        total = q.astype(np.float64) + rem * np.float64(y)
+        ties = (total.view(np.uint64) & np.uint64(0x1fffffff)) == np.uint64(0x10000000)
+        assert not ties.any(), b
+        assert np.array_equal(total.astype(np.float32), a / b), b
