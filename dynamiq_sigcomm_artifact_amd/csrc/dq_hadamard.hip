@@ -398,6 +398,14 @@ hipError_t launch_rht_slices(TransformSlice *slices, int count, int inverse, hip
         r.ends.in_src = nullptr; r.ends.in_levels = nullptr; r.ends.in_planes = nullptr;
         (inverse ? t : r).ends.gen = SignSeed();
     }
+    if (count == 1) {
+        // The arguments of one pass are an eighth of a set's: a launch of more than a kilobyte of them takes the host 0.6 us longer, and
+        // the kernel's search for its pass goes (5.9 -> 5.7 us of the first pass at 2^20).  EDEN there and back, one set -> launches of
+        // their own, us: 2^16 elements 28.2 -> 26.8, 500,000 28.0 -> 26.0, 2^20 30.2 -> 29.0, 2^22 54.9 -> 55.2.
+        const TilePass &t = tiles[0], &r = strided[0];
+        const hipError_t e = launch_rht_tile(t.x, nullptr, 0, t.n, t.kt, t.kb, t.scale, 0, t.sign_mode, 1, t.ends, stream);
+        return e == hipSuccess ? launch_rht_strided(r.x, nullptr, 0, r.n, r.rbits, r.sbits, r.scale, 1, r.sign_mode, 1, r.ends, stream) : e;
+    }
     const hipError_t e = launch_rht_tile_passes(tiles, count, stream);
     return e == hipSuccess ? launch_rht_strided_passes(strided, count, stream) : e;
 }
