@@ -599,7 +599,7 @@ int dq_ranks_max(int pooled) { return pooled ? dq::kMaxPoolRanks : dq::kMaxRanks
 int dq_ranks_allreduce(const dq_ranks_t *r, int stages, int device, dq_stream_t stream)
 {
     if (!r) return fail(DQ_ERR_NULL);
-    if (stages <= 0 || stages > 7) return fail(DQ_ERR_SIZE, "stages must be a combination of DQ_RANKS_*");
+    if (stages <= 0 || (stages > 7 && stages != (7 | DQ_RANKS_NO_LISTS))) return fail(DQ_ERR_SIZE, "stages must be a combination of DQ_RANKS_*");
     if (!(r->n > 0)) return fail(DQ_ERR_N);
     const int64_t nsc = (r->n + 255) / 256;
     int rc = check_mixed(nsc, 0, r->world, r->dtype, r->strategy, false);
@@ -626,8 +626,12 @@ int dq_ranks_allreduce(const dq_ranks_t *r, int stages, int device, dq_stream_t 
     if ((rc = select_device(device))) return rc;
     hipStream_t s = static_cast<hipStream_t>(stream);
     hipError_t e = hipSuccess;
-    if (s_stats) e = dq::launch_ranks_stats(r->src, r->world, r->n, r->total, r->mean, r->dtype, s);
-    if (e == hipSuccess && s_plan) {
+    // a short ring without lists: the words go where the lists would
+    const bool no_plan = (stages & DQ_RANKS_NO_LISTS) && !r->sorted_plan && !r->hist && !r->pool &&
+                         dq::ring_plans_itself(r->n);
+    uint32_t *words = no_plan ? reinterpret_cast<uint32_t *>(r->order) : nullptr;
+    if (s_stats) e = dq::launch_ranks_stats(r->src, r->world, r->n, r->total, r->mean, r->dtype, words, (float)r->u, r->u_dev, s);
+    if (e == hipSuccess && s_plan && !no_plan) {
         // (with u in device memory the histogram is filled by a few more workgroups of the plan launch)
         if (!r->sorted_plan && r->hist && !r->u_dev) e = dq::launch_norm_histogram(r->total, nsc, r->hist, s);
         if (e != hipSuccess) return finish(e);
@@ -644,6 +648,7 @@ int dq_ranks_allreduce(const dq_ranks_t *r, int stages, int device, dq_stream_t 
         memset(&d, 0, sizeof(d));
         d.src = r->src; d.out = r->out; d.world = r->world; d.n = r->n; d.total = r->total; d.mean = r->mean;
         d.order = r->order; d.counts = r->work; d.seed = r->seed; d.pooled = r->pool != nullptr;
+        d.tile_widths = words; d.work = r->work; d.u = (float)r->u; d.u_dev = r->u_dev;
         for (int g = 0; d.pooled && g < 3; g++) {
             for (int k = 0; k < r->world; k++) {
                 d.pool[g][k] = r->pool[g * r->world + k];

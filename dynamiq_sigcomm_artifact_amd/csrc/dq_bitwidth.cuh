@@ -94,6 +94,17 @@ __device__ __forceinline__ uint32_t wave_max_upward(uint32_t x)
     return max(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xc, 0xf, false)); // row_bcast:31 into rows 2 and 3
 }
 
+// the sum of the wave's values, in lane 63
+__device__ __forceinline__ uint32_t wave_sum_upward(uint32_t x)
+{
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xf, 0xf, false);
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xf, 0xf, false);
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xf, 0xf, false);
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xf, 0xf, false);
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xa, 0xf, false);
+    return x + (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xc, 0xf, false);
+}
+
 // A workgroup of kHistThreads threads counts batches of up to 8192 norms in LDS -- 16-bit counters, two per word,
 // so the whole range of patterns fits into 64 KB -- and adds the non-zero counters to the histogram in memory
 // after each batch: a few hundred atomics per batch instead of one per norm, most of which would hit the same

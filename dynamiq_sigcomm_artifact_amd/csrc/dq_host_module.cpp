@@ -474,7 +474,7 @@ bool ranks_dynamic(py::sequence vecs, py::sequence outs, int64_t n, py::handle t
     k.r.u_dev = o.dev;
     k.r.hist = hist_of(a, hist, &k.r.hist_ints);
     k.r.seed = seed;
-    k.enqueue(DQ_RANKS_STATS | DQ_RANKS_PLAN | DQ_RANKS_RING, a.device, stream_of(stream, a.device));
+    k.enqueue(DQ_RANKS_STATS | DQ_RANKS_PLAN | DQ_RANKS_RING | DQ_RANKS_NO_LISTS, a.device, stream_of(stream, a.device));
     return true;
 }
 

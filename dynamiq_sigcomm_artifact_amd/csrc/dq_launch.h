@@ -98,9 +98,12 @@ typedef dq_roundtrip_t RoundtripDesc;
 hipError_t launch_roundtrip(const RoundtripDesc *desc, int count, int world, float u, const double *u_dev, uint64_t seed,
                             uint64_t *step_dev, uint64_t step_more, uint32_t *hist, int dtype, bool mee, const MeeParams *mp,
                             hipStream_t stream);
-// total: bf16 pairs [nsc], mean: float [world][nsc]
+// total: bf16 pairs [nsc], mean: float [world][nsc]; tile_widths (may be null): a word per four superchunks, how many of them u
+// (or *u_dev) gives 8 bits, and 4 bits in the upper half
 hipError_t launch_ranks_stats(const void *const *src, int world, int64_t n, void *total, float *mean, int dtype,
-                              hipStream_t stream);
+                              uint32_t *tile_widths, float u, const double *u_dev, hipStream_t stream);
+// a ring that finds its groups from the words of launch_ranks_stats (in the place of a plan and its lists)
+bool ring_plans_itself(int64_t n);
 struct RingDesc {
     const void *const *src;
     void *const *out;
@@ -110,6 +113,10 @@ struct RingDesc {
     const float *mean;
     const int32_t *order, *counts;
     uint64_t seed;                               // rank r draws from seed + r, step s of the ring from step s
+    const uint32_t *tile_widths;                     // null, or what launch_ranks_stats left there: the ring does without order
+    int32_t *work;                               // (with tile_widths) and writes the group sizes to work[0..3]
+    float u;
+    const double *u_dev;
     bool pooled;                                 // or the random values come from pools:
     const void *pool[3][kMaxPoolRanks];          // by width (8, 4, 2 bits) and rank
     int32_t first[3][kMaxPoolRanks][kMaxPoolRanks]; // first row of 16 values, by width, rank and step

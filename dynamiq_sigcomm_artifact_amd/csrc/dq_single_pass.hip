@@ -11,11 +11,11 @@
 //   tally_kernel       behind it: the widths' counts per bucket and the norm histogram of the search for u
 //   ranks_stats_kernel W ranks: every rank's means, and the reduced statistics
 //   ring_kernel        W ranks, after a plan of the reduced statistics: the ring
-//   ring_quad_kernel   the same on short vectors, one superchunk per wave
+//   ring_quad_kernel   the same on short vectors, one superchunk per wave; with drawn values it does without the plan
 //
 // Measured, start -> now (bit-identical results): 8 ranks x 124,439,808 bf16 elements 2,896 -> 1,066 us per all-reduce (one
 // launch per rank and ring step, packed streams and their exchange copies, against three launches whose traffic is the
-// vectors alone), 8 x 1,000,003 elements 1,488 -> 24.6 us (257 launches against 3), a step of nine 25 MB buckets on one rank
+// vectors alone), 8 x 1,000,003 elements 1,488 -> 20 us (257 launches against 2), a step of nine 25 MB buckets on one rank
 // 252 -> 51 us (four launches per bucket on two streams against two launches per step, and the search for u).
 //
 // Numerics: csrc/cuda_hadamard.cu:1257-1369 (centring, mean add), csrc/cuda_hierarchical_mee.cu:203-696 (codec),
@@ -334,6 +334,11 @@ struct RankPointers {
     const void *src[kMaxRanks];
 };
 
+struct TileWidths {
+    uint32_t *words; // null, or one per four superchunks: how many the rule gives 8 bits, and 4 bits in the upper half
+    WidthRule rule;
+};
+
 constexpr int kStatsWaves = 8; // ranks in flight per workgroup of ranks_stats_kernel
 // A workgroup takes GROUPS tiles of four superchunks, a wave of it those of one rank (of every kStatsWaves-th one in a larger
 // world): means and norms per rank, and the statistics all-reduce as the reference's chain of bf16 additions in rank order.
@@ -344,9 +349,10 @@ constexpr int kStatsWaves = 8; // ranks in flight per workgroup of ranks_stats_k
 template <int DT, int GROUPS, bool NT>
 __global__ __launch_bounds__(64 * kStatsWaves, 8) void ranks_stats_kernel(RankPointers ranks, int world, int64_t n, int vec,
                                                                          uint32_t *__restrict__ total, float *__restrict__ mean_out,
-                                                                         WorldDiv wd)
+                                                                         WorldDiv wd, TileWidths widths)
 {
     extern __shared__ __attribute__((aligned(16))) uint8_t tiles[];
+    const float u = widths.rule.u_dev ? (float)*widths.rule.u_dev : widths.rule.u;
     constexpr int kRows = GROUPS * kRowsPerWave;
     __shared__ uint32_t pairs[kMaxRanks][kRows];
     typedef StatsTile<DT> ST;
@@ -420,11 +426,22 @@ __global__ __launch_bounds__(64 * kStatsWaves, 8) void ranks_stats_kernel(RankPo
             acc = f32_to_bf16_bits(lo) | (f32_to_bf16_bits(hi) << 16);
         }
         total[sc0 + threadIdx.x] = acc;
+        if (widths.words) {
+            const int cls = class_of_norm(acc >> 16, u, widths.rule.thr);
+            const uint64_t eights = __builtin_amdgcn_ballot_w64(cls == 0), fours = __builtin_amdgcn_ballot_w64(cls == 1);
+            if ((threadIdx.x & 3) == 0)
+                widths.words[(sc0 + threadIdx.x) >> 2] = (uint32_t)__popcll((eights >> threadIdx.x) & 15u) |
+                                                         ((uint32_t)__popcll((fours >> threadIdx.x) & 15u) << 16);
+        }
     }
 }
 
 // rounding randomness out of the compressors' pools: which rank uses which rows of which pool in which step
-struct NoPools {};
+struct FromTileWidths {
+    const uint32_t *words; // of ranks_stats_kernel
+    int32_t *counts;       // written: group sizes
+    WidthRule rule;
+};
 struct Pools {
     const void *pool[3][kMaxPoolRanks];                          // one per width (8, 4, 2 bits) and rank
     int32_t first[3][kMaxPoolRanks][kMaxPoolRanks];              // first row of 16 values: [width][rank][step]
@@ -442,7 +459,7 @@ template <bool POOL> struct RingArgs {
     RandKey key;
     WorldDiv wd;
     WidthSet widths;
-    typename std::conditional<POOL, Pools, NoPools>::type pools;
+    typename std::conditional<POOL, Pools, FromTileWidths>::type more;
 };
 
 // Workgroup (x, y): tile x of ring chunk y -- rank y compresses it first, rank y + 1 decodes, adds and recompresses, and
@@ -503,7 +520,7 @@ __global__ __launch_bounds__(64, DT == DQ_BF16 && RDT == DQ_PHILOX && !MEE ? 5 :
             load_chunk<DT>(next, a.src[rank], e0, a.n, a.vec & 1, ragged);
             next_mean = a.mean[(int64_t)rank * a.nsc + sc];
             if constexpr (RDT != DQ_PHILOX)
-                next_r.load(a.pools.pool[cls][rank], ((int64_t)a.pools.first[cls][rank][step] + k0 * 16 + lane) * 16, (a.vec & 4) != 0);
+                next_r.load(a.more.pool[cls][rank], ((int64_t)a.more.first[cls][rank][step] + k0 * 16 + lane) * 16, (a.vec & 4) != 0);
         }
     };
     fetch(0);
@@ -562,19 +579,67 @@ constexpr int kQuadWaves = 4;
 
 // ring_kernel with a superchunk per wave, four elements per lane: short vectors, where a wave's chain of `world` steps is all
 // there is to wait for (2 us a step with one wave of ring_kernel per SIMD, 0.7 us here).
-template <int DT, int RDT, bool MEE>
+//
+// PLANS: without a plan launch in front.  A superchunk's way through the ring depends on the others only by where it starts: on its
+// place among those of its width.  The statistics leave a word per four superchunks with their widths' counts; a workgroup takes
+// four neighbouring superchunks and adds up the words, all of them and those before its own, while the norms of its own are on their way.
+template <int DT, int RDT, bool MEE, bool PLANS = false>
 __global__ __launch_bounds__(64 * kQuadWaves) void ring_quad_kernel(RingArgs<RDT != DQ_PHILOX> a)
 {
     __shared__ float levels[MEE ? kLevelCount : 1];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), world = a.world;
     if (MEE) {
         if (wave == 0) levels_to_lds(a.widths, levels, lane);
-        __syncthreads();
+        if (!PLANS) __syncthreads();
     }
-    // entry `at` of the three lists end to end; sizes clamped as in ring_kernel
     const int at = (int)blockIdx.x * kQuadWaves + wave;
     int cls = 3, k = 0, chunk = 0, in_run = 0;
-    {
+    int64_t sc = 0;
+    if constexpr (PLANS) {
+        static_assert(kQuadWaves == kRowsPerWave, "a workgroup's superchunks are those of one word");
+        __shared__ uint2 part[kQuadWaves];
+        const FromTileWidths &f = a.more;
+        const float u = f.rule.u_dev ? (float)*f.rule.u_dev : f.rule.u;
+        const int tile = blockIdx.x, tiles = (a.nsc + 3) >> 2;
+        const uint32_t norm = a.total[2 * min(4 * tile + (lane & 3), a.nsc - 1) + 1];
+        uint32_t all = 0, before = 0;
+        constexpr int kTogether = 4, kThreads = 64 * kQuadWaves;
+        for (int first = 0; first < tiles; first += kTogether * kThreads) {
+            uint32_t got[kTogether];
+#pragma unroll
+            for (int i = 0; i < kTogether; i++) got[i] = f.words[min(first + i * kThreads + (int)threadIdx.x, tiles - 1)];
+#pragma unroll
+            for (int i = 0; i < kTogether; i++) {
+                const int word = first + i * kThreads + (int)threadIdx.x;
+                all += word < tiles ? got[i] : 0u;
+                before += word < tile ? got[i] : 0u;
+            }
+        }
+        all = wave_sum_upward(all);
+        before = wave_sum_upward(before);
+        if (lane == 63) part[wave] = make_uint2(all, before);
+        const int mine = class_of_norm(norm, u, f.rule.thr); // (of lane & 3)
+        __syncthreads();
+        const uint2 p0 = part[0], p1 = part[1], p2 = part[2], p3 = part[3];
+        all = (uint32_t)__builtin_amdgcn_readfirstlane((int)(p0.x + p1.x + p2.x + p3.x));
+        before = (uint32_t)__builtin_amdgcn_readfirstlane((int)(p0.y + p1.y + p2.y + p3.y));
+        const int m8 = (int)(all & 0xffffu), m4 = (int)(all >> 16), m2 = a.nsc - m8 - m4;
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+            f.counts[0] = m8;
+            f.counts[1] = m4;
+            f.counts[2] = m2;
+            f.counts[3] = 0;
+        }
+        if (at >= a.nsc) return;
+        sc = at;
+        cls = __builtin_amdgcn_readlane(mine, wave);
+        const int m = cls == 0 ? m8 : (cls == 1 ? m4 : m2);
+        const int b8 = (int)(before & 0xffffu), b4 = (int)(before >> 16);
+        k = (cls == 0 ? b8 : (cls == 1 ? b4 : 4 * tile - b8 - b4)) +
+            __popcll(__builtin_amdgcn_ballot_w64(mine == cls) & ((1u << wave) - 1u));
+        chunk = min(k / max((m + world - 1) / world, 1), world - 1); // (within the ranks also with words that are not these norms')
+    } else {
+        // entry `at` of the three lists end to end; sizes clamped as in ring_kernel
         int used = 0;
         const int counts[3] = {a.counts[0], a.counts[1], a.counts[2]};
 #pragma unroll
@@ -589,9 +654,9 @@ __global__ __launch_bounds__(64 * kQuadWaves) void ring_quad_kernel(RingArgs<RDT
             }
             used += m;
         }
+        if (cls == 3) return;
+        sc = a.order[(int64_t)cls * a.nsc + k];
     }
-    if (cls == 3) return;
-    const int64_t sc = a.order[(int64_t)cls * a.nsc + k];
     const int64_t e0 = sc * 256 + lane * 4;
     const bool ragged = sc * 256 + 256 > a.n;
     const WidthRegs<MEE> w = width_regs<MEE>(a.widths, cls, levels);
@@ -604,8 +669,8 @@ __global__ __launch_bounds__(64 * kQuadWaves) void ring_quad_kernel(RingArgs<RDT
     const float my_mean = a.mean[(int64_t)my_rank * a.nsc + sc];
     uint64_t my_pool = 0;
     if constexpr (RDT != DQ_PHILOX)
-        my_pool = reinterpret_cast<uint64_t>(a.pools.pool[cls][my_rank]) +
-                  (int64_t)(a.pools.first[cls][my_rank][my_step] + in_run * 16) * (16 * (RDT == DQ_F32 ? 4 : 2));
+        my_pool = reinterpret_cast<uint64_t>(a.more.pool[cls][my_rank]) +
+                  (int64_t)(a.more.first[cls][my_rank][my_step] + in_run * 16) * (16 * (RDT == DQ_F32 ? 4 : 2));
     const auto of_step = [](uint64_t mine, int step) {
         const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)mine, step);
         const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(mine >> 32), step);
@@ -663,6 +728,13 @@ bool a_wave_each(int nsc, int world, int elem_bytes, bool mee, bool pooled)
     const bool least = !mee && !pooled && world * elem_bytes < 12;
     return nsc <= (least ? kQuadSuperchunksShort : kQuadSuperchunks);
 }
+
+// Up to so many superchunks a ring with drawn values finds its groups itself (ring_quad_kernel, PLANS) in the place of a plan launch of 4 to
+// 6 us, which is also worth a wave per superchunk a little longer.  Statistics, (plan,) ring, us, with a plan -> without, AEE: 8 ranks x
+// 256 superchunks 12.9 -> 11.6, x 3,907 23.9 -> 19.6, x 8,192 31.5 -> 25.9, x 12,288 39.2 -> 36.0, x 16,384 46.0 -> 45.8; 4 x 3,907 16.3
+// -> 12.8, x 12,288 24.2 -> 21.7; 2 x 3,907 13.0 -> 10.4, x 12,288 16.7 -> 16.2, x 16,384 19.5 -> 20.7; MEE 8 x 3,907 25.4 -> 21.2, 2 x
+// 12,288 18.9 -> 17.9; fp32 8 x 3,907 27.7 -> 22.0, 2 x 12,288 20.8 -> 17.1.
+constexpr int64_t kPlansItself = 12288;
 
 WidthRule make_rule(float u, const double *u_dev)
 {
@@ -737,7 +809,8 @@ hipError_t launch_roundtrip(const RoundtripDesc *desc, int count, int world, flo
 // 4 x 19,500 (319 MB) 156.5 -> 159.5, 8 x 10,000 (327 MB) 169 -> 166, 2 x 47,500 202 -> 193.
 constexpr int64_t kStatsOneTile = 19 << 10, kStatsCache = (int64_t)300 << 20;
 
-hipError_t launch_ranks_stats(const void *const *src, int world, int64_t n, void *total, float *mean, int dtype, hipStream_t stream)
+hipError_t launch_ranks_stats(const void *const *src, int world, int64_t n, void *total, float *mean, int dtype, uint32_t *tile_widths,
+                              float u, const double *u_dev, hipStream_t stream)
 {
     RankPointers p;
     int vec = 1;
@@ -750,10 +823,11 @@ hipError_t launch_ranks_stats(const void *const *src, int world, int64_t n, void
     const int waves = world < kStatsWaves ? world : kStatsWaves;
     const WorldDiv wd = make_world_div(world, dtype == DQ_F32 ? 4 : 2);
     uint32_t *tot = static_cast<uint32_t *>(total);
+    const TileWidths widths{tile_widths, tile_widths ? make_rule(u, u_dev) : WidthRule{0.0f, nullptr, {-1, -1}}};
     const auto run = [&](auto type, auto groups, auto nt) {
         constexpr int DT = decltype(type)::value, G = decltype(groups)::value;
         hipLaunchKernelGGL((ranks_stats_kernel<DT, G, decltype(nt)::value>), dim3((unsigned)((tiles + G - 1) / G)), dim3(64 * waves),
-                           waves * StatsTile<DT>::BYTES, stream, p, world, n, vec, tot, mean, wd);
+                           waves * StatsTile<DT>::BYTES, stream, p, world, n, vec, tot, mean, wd, widths);
     };
     const auto launch = [&](auto type) {
         if (!vec) run(type, std::integral_constant<int, 1>(), std::false_type());
@@ -780,9 +854,9 @@ static hipError_t run_ring(const RingDesc &d, bool mee, const MeeParams *mp, hip
         out = out && aligned16(d.out[r]);
         if constexpr (POOL) {
             for (int g = 0; g < 3; g++) {
-                a.pools.pool[g][r] = d.pool[g][r];
+                a.more.pool[g][r] = d.pool[g][r];
                 pool = pool && aligned16(d.pool[g][r]);
-                for (int s = 0; s < d.world; s++) a.pools.first[g][r][s] = d.first[g][r][s];
+                for (int s = 0; s < d.world; s++) a.more.first[g][r][s] = d.first[g][r][s];
             }
         }
     }
@@ -797,8 +871,18 @@ static hipError_t run_ring(const RingDesc &d, bool mee, const MeeParams *mp, hip
     a.key = RandKey{d.seed, 0};
     a.wd = make_world_div(d.world, DT == DQ_F32 ? 4 : 2);
     a.widths = make_width_set(mp, mee);
+    const dim3 block(64 * kQuadWaves);
+    if constexpr (!POOL) {
+        if (d.tile_widths) {
+            a.more = FromTileWidths{d.tile_widths, d.work, make_rule(d.u, d.u_dev)};
+            const dim3 grid((unsigned)((a.nsc + kQuadWaves - 1) / kQuadWaves));
+            if (mee) hipLaunchKernelGGL((ring_quad_kernel<DT, RDT, true, true>), grid, block, 0, stream, a);
+            else hipLaunchKernelGGL((ring_quad_kernel<DT, RDT, false, true>), grid, block, 0, stream, a);
+            return hipGetLastError();
+        }
+    }
     if (a_wave_each(a.nsc, d.world, DT == DQ_F32 ? 4 : 2, mee, POOL)) {
-        const dim3 grid((unsigned)((a.nsc + kQuadWaves - 1) / kQuadWaves)), block(64 * kQuadWaves);
+        const dim3 grid((unsigned)((a.nsc + kQuadWaves - 1) / kQuadWaves));
         if (mee) hipLaunchKernelGGL((ring_quad_kernel<DT, RDT, true>), grid, block, 0, stream, a);
         else hipLaunchKernelGGL((ring_quad_kernel<DT, RDT, false>), grid, block, 0, stream, a);
         return hipGetLastError();
@@ -808,6 +892,11 @@ static hipError_t run_ring(const RingDesc &d, bool mee, const MeeParams *mp, hip
     if (mee) hipLaunchKernelGGL((ring_kernel<DT, RDT, true>), grid, dim3(64), 0, stream, a);
     else hipLaunchKernelGGL((ring_kernel<DT, RDT, false>), grid, dim3(64), 0, stream, a);
     return hipGetLastError();
+}
+
+bool ring_plans_itself(int64_t n)
+{
+    return (n + 255) / 256 <= kPlansItself;
 }
 
 hipError_t launch_ring(const RingDesc &d, int dtype, bool mee, const MeeParams *mp, hipStream_t stream)

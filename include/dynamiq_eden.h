@@ -419,8 +419,10 @@ int dq_bucket_roundtrip(const dq_roundtrip_t *buckets, int count, int dtype, int
  * (seed + r, s, chunk index); or with pool != NULL rank r's random values of
  * step s for the group of width index g (0: 8 bits, 1: 4, 2: 2) are the rows
  * first[(g * world + r) * world + s] onwards of pool[g * world + r], 16 values
- * of dtype per row, one row per chunk of the rank's list of superchunks. */
-enum { DQ_RANKS_STATS = 1, DQ_RANKS_PLAN = 2, DQ_RANKS_RING = 4 };
+ * of dtype per row, one row per chunk of the rank's list of superchunks.
+ * DQ_RANKS_NO_LISTS, with the three stages in one call: the caller has no use
+ * for order, which is scratch; work[0..3] are written as by PLAN. */
+enum { DQ_RANKS_STATS = 1, DQ_RANKS_PLAN = 2, DQ_RANKS_RING = 4, DQ_RANKS_NO_LISTS = 8 };
 
 typedef struct dq_ranks {
     const void *const *src;     /* world pointers to n elements of dtype (DQ_BF16 or DQ_F32) */

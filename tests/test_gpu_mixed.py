@@ -739,6 +739,31 @@ def test_chunk_scales_on_whole_ratios(capi, W, nsc, strategy, dt):
     assert all(torch.equal(bits_t(p), bits_t(q)) for p, q in zip(outs, ref))
 
 
+@pytest.mark.parametrize("W,n,dt", [
+    (8, 1, torch.bfloat16), (2, 256 * 3, torch.float32), (3, 256 * 4 + 1, torch.bfloat16), (16, 256 * 5, torch.bfloat16),
+    (2, 256 * 4096, torch.bfloat16), (5, 256 * 4097, torch.bfloat16),          # as many words as a trip takes, one more
+    (2, 256 * 12288, torch.bfloat16), (3, 256 * 12288 - 255, torch.float32),   # the last length without lists
+    (2, 256 * 12288 + 1, torch.bfloat16)])
+def test_rings_without_lists(capi, W, n, dt):
+    """short rings find their groups from the counts per four superchunks: widths that change from one superchunk to the next, and all
+    of one width, against one launch per rank and ring step, which has its lists from the plan"""
+    from dynamiq_sigcomm_artifact_amd.dynamiq_pipeline import _single_pass_in_steps, dynamic_bitrate_allreduce_single_pass
+    g = torch.Generator(device=DEV).manual_seed(n + W)
+    nsc = (n + 255) // 256
+    scales = torch.exp(torch.randn(nsc, 1, generator=g, device=DEV) * 6.0) * 1e-3
+    vecs = [(torch.randn(nsc, 256, generator=g, device=DEV) * scales).reshape(-1)[:n].to(dt).contiguous() for _ in range(W)]
+    seen = set()
+    for strategy, u in ((2, 6.0), (3, 6.5), (2, -40.0), (2, 60.0), (3, float("nan"))):
+        u_dev = torch.full((1,), u, dtype=torch.float64, device=DEV)
+        ref, total2, counts2 = _single_pass_in_steps(vecs, u_dev, strategy, 11, None, {}, None, None)
+        for offset in (u_dev, u) if u == u else (u_dev,):
+            outs, total, counts = dynamic_bitrate_allreduce_single_pass(vecs, offset, strategy=strategy, seed=11)
+            assert counts.tolist() == counts2.tolist() and torch.equal(bits_t(total), bits_t(total2))
+            assert all(torch.equal(bits_t(x), bits_t(y)) for x, y in zip(outs, ref)), (strategy, u)
+        seen.add(tuple(c > 0 for c in counts.tolist()))
+    assert len(seen) > 1
+
+
 @pytest.mark.parametrize("W,n", [(2, 256 * 8192), (3, 256 * 8192 + 1), (5, 256 * 8195)])
 def test_ranks_on_either_side_of_a_superchunk_per_wave(capi, W, n):
     """the last length that takes a wave per superchunk (MEE; AEE below) and the first ones that take four superchunks per wave"""
