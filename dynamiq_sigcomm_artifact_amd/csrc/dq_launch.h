@@ -6,9 +6,23 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "dq_device.cuh"
 
 namespace dq {
+
+// A kernel whose only argument is `args`.  Short calls wait for the host, and the runtime copies a kernel's arguments one by one to
+// where the GPU reads them: a decoder call of eight arguments and 104 bytes takes 3.8 us, with one argument of 56 bytes 2.9 (and 576
+// bytes 1.1 us more than 64).  Eight ranks' ring of 65,792 elements, 17 calls, 68 -> 55 us of host time.
+template <class K, class A> inline hipError_t launch_with(K *kernel, dim3 grid, dim3 block, hipStream_t stream, const A &args)
+{
+    static_assert(std::is_same<K, void(A)>::value, "the kernel takes these arguments");
+    void *list[] = {const_cast<A *>(&args)};
+    const hipError_t e = hipLaunchKernel(reinterpret_cast<const void *>(kernel), grid, block, list, 0, stream);
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e;
+}
 
 // scaling quantisation, catch-all kernels (dq_scaling_generic.hip)
 hipError_t launch_generic_compress(const void *src, uint8_t *dst, const void *rnd, int64_t n,

@@ -46,11 +46,30 @@ namespace dq {
 // ---- kernels ------------------------------------------------------------------------------------
 
 // workgroup = one wave = one tile; the bodies live in dq_hier16_tiles.cuh
+template <class MP> struct CompressArgs {
+    const void *src;
+    const uint8_t *recv;
+    uint8_t *dst;
+    const void *rnd;
+    const int32_t *rows;
+    int64_t nsc;
+    int vec;
+    RandKey key;
+    MP mp;
+};
+
+template <class MP> struct DecompressArgs {
+    const uint8_t *src;
+    void *dst;
+    const int32_t *rows;
+    const uint16_t *stats;
+    int64_t limit, nsc;
+    int vec;
+    MP mp;
+};
+
 template <int DT, int RDT, int NBITS, bool MEE, bool FUSED>
-__global__ __launch_bounds__(64) void hier16_compress_kernel(const void *__restrict__ src, const uint8_t *__restrict__ recv,
-                                                            uint8_t *__restrict__ dst, const void *__restrict__ rnd,
-                                                            const int32_t *__restrict__ rows, int64_t nsc, int vec,
-                                                            RandKey key, MeeArg<NBITS, MEE> mp)
+__global__ __launch_bounds__(64) void hier16_compress_kernel(CompressArgs<MeeArg<NBITS, MEE>> a)
 {
     typedef Rec<NBITS> RC;
     __shared__ __attribute__((aligned(16))) uint8_t win_out[RC::WIN];
@@ -58,8 +77,8 @@ __global__ __launch_bounds__(64) void hier16_compress_kernel(const void *__restr
     __shared__ float table[(MEE && FUSED) ? (1 << NBITS) : 1];
     const Center none{nullptr, 0, {0.0f, 0.0, 0, 0, 0, 0.0f}};
     const int64_t tile = blockIdx.x;
-    compress_tile<DT, RDT, NBITS, MEE, FUSED>(src, recv, dst, rnd, row_ids_plain(rows), nsc, tile, vec, key, none, mp, win_out,
-                                              win_in, table, threadIdx.x);
+    compress_tile<DT, RDT, NBITS, MEE, FUSED>(a.src, a.recv, a.dst, a.rnd, row_ids_plain(a.rows), a.nsc, tile, a.vec, a.key, none, a.mp,
+                                              win_out, win_in, table, threadIdx.x);
 }
 
 // LONG: the wave takes kTilesPerWaveLong consecutive tiles of a row list and fetches their entries with one load (RowIds).
@@ -69,26 +88,23 @@ __global__ __launch_bounds__(64) void hier16_compress_kernel(const void *__restr
 constexpr int kTilesPerWaveLong = 4;
 
 template <int DT, int NBITS, bool MEE, bool ADD, bool LONG>
-__global__ __launch_bounds__(64) void hier16_decompress_kernel(const uint8_t *__restrict__ src, void *__restrict__ dst,
-                                                              const int32_t *__restrict__ rows,
-                                                              const uint16_t *__restrict__ stats, int64_t limit,
-                                                              int64_t nsc, int vec, MeeArg<NBITS, MEE> mp)
+__global__ __launch_bounds__(64) void hier16_decompress_kernel(DecompressArgs<MeeArg<NBITS, MEE>> a)
 {
     __shared__ __attribute__((aligned(16))) uint8_t win_in[Rec<NBITS>::WIN];
     __shared__ __attribute__((aligned(16))) uint4 tile_out[64 * Raw16<DT>::kSlots];
     __shared__ float table[MEE ? (1 << NBITS) : 1];
     if constexpr (LONG) {
         const int64_t tile0 = (int64_t)blockIdx.x * kTilesPerWaveLong;
-        const RowIds ids = row_ids_prefetch(rows, tile0 * kRowsPerWave, kTilesPerWaveLong * kRowsPerWave, nsc, threadIdx.x);
+        const RowIds ids = row_ids_prefetch(a.rows, tile0 * kRowsPerWave, kTilesPerWaveLong * kRowsPerWave, a.nsc, threadIdx.x);
 #pragma unroll 1
         for (int t = 0; t < kTilesPerWaveLong; t++) {
-            decompress_tile<DT, NBITS, MEE, ADD>(src, dst, ids, stats, limit, nsc, tile0 + t, vec, mp, win_in, tile_out, table);
+            decompress_tile<DT, NBITS, MEE, ADD>(a.src, a.dst, ids, a.stats, a.limit, a.nsc, tile0 + t, a.vec, a.mp, win_in, tile_out, table);
             wave_lds_sync(); // window, table and output tile are reused by the next tile
         }
     } else {
         const int64_t tile = blockIdx.x;
-        decompress_tile<DT, NBITS, MEE, ADD>(src, dst, row_ids_plain(rows), stats, limit, nsc, tile, vec, mp, win_in, tile_out,
-                                             table);
+        decompress_tile<DT, NBITS, MEE, ADD>(a.src, a.dst, row_ids_plain(a.rows), a.stats, a.limit, a.nsc, tile, a.vec, a.mp, win_in,
+                                             tile_out, table);
     }
 }
 
@@ -108,35 +124,26 @@ template <int DT, int RDT, int NBITS, bool MEE>
 static hipError_t run_compress(const void *src, const uint8_t *recv, uint8_t *dst, const void *rnd, const int32_t *rows,
                                int64_t nsc, bool fused, const MeeParams &mp, RandKey key, hipStream_t stream)
 {
-    auto arg = make_arg<NBITS, MEE>(mp);
-    dim3 grid(grid_for(nsc)), block(64);
-    const int vec = (aligned16(src) ? 1 : 0) | (aligned16(rnd) ? 2 : 0);
-    if (fused)
-        hipLaunchKernelGGL((hier16_compress_kernel<DT, RDT, NBITS, MEE, true>), grid, block, 0, stream, src, recv, dst, rnd, rows, nsc, vec, key, arg);
-    else
-        hipLaunchKernelGGL((hier16_compress_kernel<DT, RDT, NBITS, MEE, false>), grid, block, 0, stream, src, recv, dst, rnd, rows, nsc, vec, key, arg);
-    return hipGetLastError();
+    const CompressArgs<MeeArg<NBITS, MEE>> args{src, recv, dst, rnd, rows, nsc, (aligned16(src) ? 1 : 0) | (aligned16(rnd) ? 2 : 0), key,
+                                                make_arg<NBITS, MEE>(mp)};
+    const dim3 grid(grid_for(nsc)), block(64);
+    if (fused) return launch_with(hier16_compress_kernel<DT, RDT, NBITS, MEE, true>, grid, block, stream, args);
+    return launch_with(hier16_compress_kernel<DT, RDT, NBITS, MEE, false>, grid, block, stream, args);
 }
 
 template <int DT, int NBITS, bool MEE>
 static hipError_t run_decompress(const uint8_t *src, void *dst, const int32_t *rows, const uint16_t *stats, int64_t limit,
                                  int64_t nsc, int add, const MeeParams &mp, hipStream_t stream)
 {
-    auto arg = make_arg<NBITS, MEE>(mp);
-    dim3 block(64);
-    const int vec = aligned16(dst) ? 1 : 0;
+    const DecompressArgs<MeeArg<NBITS, MEE>> args{src, dst, rows, stats, limit, nsc, aligned16(dst) ? 1 : 0, make_arg<NBITS, MEE>(mp)};
+    const dim3 block(64);
     if (rows && nsc >= kLongRun && !add) {
         // a long row list (the decoder of the grouped pipelines on the reference's whole-model buckets)
-        hipLaunchKernelGGL((hier16_decompress_kernel<DT, NBITS, MEE, false, true>), dim3(grid_for(nsc, kTilesPerWaveLong)), block, 0,
-                           stream, src, dst, rows, stats, limit, nsc, vec, arg);
-        return hipGetLastError();
+        return launch_with(hier16_decompress_kernel<DT, NBITS, MEE, false, true>, dim3(grid_for(nsc, kTilesPerWaveLong)), block, stream, args);
     }
-    dim3 grid(grid_for(nsc));
-    if (add)
-        hipLaunchKernelGGL((hier16_decompress_kernel<DT, NBITS, MEE, true, false>), grid, block, 0, stream, src, dst, rows, stats, limit, nsc, vec, arg);
-    else
-        hipLaunchKernelGGL((hier16_decompress_kernel<DT, NBITS, MEE, false, false>), grid, block, 0, stream, src, dst, rows, stats, limit, nsc, vec, arg);
-    return hipGetLastError();
+    const dim3 grid(grid_for(nsc));
+    if (add) return launch_with(hier16_decompress_kernel<DT, NBITS, MEE, true, false>, grid, block, stream, args);
+    return launch_with(hier16_decompress_kernel<DT, NBITS, MEE, false, false>, grid, block, stream, args);
 }
 
 #define DQ_COMMA ,

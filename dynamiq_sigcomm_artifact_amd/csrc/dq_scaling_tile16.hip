@@ -97,9 +97,8 @@ __device__ __forceinline__ void half_codes_native(const Raw16<DQ_F16> &v, const 
 }
 
 template <int DT, int RDT, int NBITS, bool HIER, bool MEE>
-__global__ __launch_bounds__(64) void tile16_compress_kernel(const void *__restrict__ src, uint8_t *__restrict__ dst,
-                                                            const void *__restrict__ rnd, int64_t nchunks, int vec,
-                                                            RandKey key, MeeArg<NBITS, MEE> mp)
+__device__ __forceinline__ void tile16_compress(const void *__restrict__ src, uint8_t *__restrict__ dst, const void *__restrict__ rnd,
+                                                int64_t nchunks, int vec, const RandKey &key, const MeeArg<NBITS, MEE> &mp)
 {
     typedef Geo<NBITS, HIER> G;
     constexpr int R = Rec<NBITS>::R;
@@ -250,9 +249,25 @@ __global__ __launch_bounds__(64) void tile16_compress_kernel(const void *__restr
     window_flush(win_out, gout, mis, total, lane);
 }
 
+template <class MP> struct Tile16CompressArgs {
+    const void *src;
+    uint8_t *dst;
+    const void *rnd;
+    int64_t nchunks;
+    int vec;
+    RandKey key;
+    MP mp;
+};
+
+template <int DT, int RDT, int NBITS, bool HIER, bool MEE>
+__global__ __launch_bounds__(64) void tile16_compress_kernel(Tile16CompressArgs<MeeArg<NBITS, MEE>> a)
+{
+    tile16_compress<DT, RDT, NBITS, HIER, MEE>(a.src, a.dst, a.rnd, a.nchunks, a.vec, a.key, a.mp);
+}
+
 template <int DT, int NBITS, bool HIER, bool MEE, bool ADD>
-__global__ __launch_bounds__(64) void tile16_decompress_kernel(const uint8_t *__restrict__ src, void *__restrict__ dst,
-                                                              int64_t nchunks, int vec, MeeArg<NBITS, MEE> mp)
+__device__ __forceinline__ void tile16_decompress(const uint8_t *__restrict__ src, void *__restrict__ dst, int64_t nchunks, int vec,
+                                                  const MeeArg<NBITS, MEE> &mp)
 {
     typedef Geo<NBITS, HIER> G;
     constexpr int R = Rec<NBITS>::R;
@@ -332,41 +347,45 @@ __global__ __launch_bounds__(64) void tile16_decompress_kernel(const uint8_t *__
     }
 }
 
+template <class MP> struct Tile16DecompressArgs {
+    const uint8_t *src;
+    void *dst;
+    int64_t nchunks;
+    int vec;
+    MP mp;
+};
+
+template <int DT, int NBITS, bool HIER, bool MEE, bool ADD>
+__global__ __launch_bounds__(64) void tile16_decompress_kernel(Tile16DecompressArgs<MeeArg<NBITS, MEE>> a)
+{
+    tile16_decompress<DT, NBITS, HIER, MEE, ADD>(a.src, a.dst, a.nchunks, a.vec, a.mp);
+}
+
 inline unsigned grid_for(int64_t nchunks) { return (unsigned)((nchunks + kChunksPerWave - 1) / kChunksPerWave); }
 
 template <int DT, int RDT, int NBITS, bool MEE>
 hipError_t run_compress(const void *src, uint8_t *dst, const void *rnd, int64_t nchunks, bool hier, const MeeParams &mp,
                         RandKey key, hipStream_t stream)
 {
-    auto arg = make_arg<NBITS, MEE>(mp);
-    const int vec = (aligned16(src) ? 1 : 0) | (aligned16(rnd) ? 2 : 0);
-    dim3 grid(grid_for(nchunks)), block(64);
-    if (DT == DQ_F16 && hier)
-        hipLaunchKernelGGL((tile16_compress_kernel<DQ_F16, RDT, NBITS, true, MEE>), grid, block, 0, stream, src, dst, rnd, nchunks, vec, key, arg);
-    else
-        hipLaunchKernelGGL((tile16_compress_kernel<DT, RDT, NBITS, false, MEE>), grid, block, 0, stream, src, dst, rnd, nchunks, vec, key, arg);
-    return hipGetLastError();
+    const Tile16CompressArgs<MeeArg<NBITS, MEE>> args{src, dst, rnd, nchunks, (aligned16(src) ? 1 : 0) | (aligned16(rnd) ? 2 : 0), key,
+                                                      make_arg<NBITS, MEE>(mp)};
+    const dim3 grid(grid_for(nchunks)), block(64);
+    if (DT == DQ_F16 && hier) return launch_with(tile16_compress_kernel<DQ_F16, RDT, NBITS, true, MEE>, grid, block, stream, args);
+    return launch_with(tile16_compress_kernel<DT, RDT, NBITS, false, MEE>, grid, block, stream, args);
 }
 
 template <int DT, int NBITS, bool MEE>
 hipError_t run_decompress(const uint8_t *src, void *dst, int64_t nchunks, bool hier, int add, const MeeParams &mp,
                           hipStream_t stream)
 {
-    auto arg = make_arg<NBITS, MEE>(mp);
-    const int vec = aligned16(dst) ? 1 : 0;
-    dim3 grid(grid_for(nchunks)), block(64);
+    const Tile16DecompressArgs<MeeArg<NBITS, MEE>> args{src, dst, nchunks, aligned16(dst) ? 1 : 0, make_arg<NBITS, MEE>(mp)};
+    const dim3 grid(grid_for(nchunks)), block(64);
     if (DT == DQ_F16 && hier) {
-        if (add)
-            hipLaunchKernelGGL((tile16_decompress_kernel<DQ_F16, NBITS, true, MEE, true>), grid, block, 0, stream, src, dst, nchunks, vec, arg);
-        else
-            hipLaunchKernelGGL((tile16_decompress_kernel<DQ_F16, NBITS, true, MEE, false>), grid, block, 0, stream, src, dst, nchunks, vec, arg);
-    } else {
-        if (add)
-            hipLaunchKernelGGL((tile16_decompress_kernel<DT, NBITS, false, MEE, true>), grid, block, 0, stream, src, dst, nchunks, vec, arg);
-        else
-            hipLaunchKernelGGL((tile16_decompress_kernel<DT, NBITS, false, MEE, false>), grid, block, 0, stream, src, dst, nchunks, vec, arg);
+        if (add) return launch_with(tile16_decompress_kernel<DQ_F16, NBITS, true, MEE, true>, grid, block, stream, args);
+        return launch_with(tile16_decompress_kernel<DQ_F16, NBITS, true, MEE, false>, grid, block, stream, args);
     }
-    return hipGetLastError();
+    if (add) return launch_with(tile16_decompress_kernel<DT, NBITS, false, MEE, true>, grid, block, stream, args);
+    return launch_with(tile16_decompress_kernel<DT, NBITS, false, MEE, false>, grid, block, stream, args);
 }
 
 // the uniform values of the in-kernel stream written out as a tensor: element e = chunk e / 16, byte e % 16

@@ -25,7 +25,14 @@ template <int NBITS, bool MEE> struct MeeArg {
     float c, cmm, l2b;
     uint32_t pad;
     double inv_c, inv_cmm, inv_l2b; // correctly rounded double reciprocals
-    uint16_t table[MEE ? (1 << NBITS) : 4];
+    uint16_t table[1 << NBITS];
+};
+
+// (AEE takes none of it: nothing for the host to write with every launch)
+template <int NBITS> struct MeeArg<NBITS, false> {
+    static constexpr float c = 1.0f, cmm = 1.0f, l2b = 1.0f;
+    static constexpr double inv_c = 1.0, inv_cmm = 1.0, inv_l2b = 1.0;
+    static constexpr uint16_t table[2] = {0, 0};
 };
 
 typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
@@ -544,9 +551,11 @@ __device__ __forceinline__ void estimate_codes(const RV &v, const RR &r, float d
 template <int NBITS, bool MEE> static MeeArg<NBITS, MEE> make_arg(const MeeParams &mp)
 {
     MeeArg<NBITS, MEE> a;
-    a.c = mp.c; a.cmm = mp.cmm; a.l2b = mp.l2b; a.pad = 0;
-    a.inv_c = 1.0 / (double)mp.c; a.inv_cmm = 1.0 / (double)mp.cmm; a.inv_l2b = 1.0 / (double)mp.l2b;
-    for (int k = 0; k < (MEE ? (1 << NBITS) : 4); k++) a.table[k] = mp.table[k];
+    if constexpr (MEE) {
+        a.c = mp.c; a.cmm = mp.cmm; a.l2b = mp.l2b; a.pad = 0;
+        a.inv_c = 1.0 / (double)mp.c; a.inv_cmm = 1.0 / (double)mp.cmm; a.inv_l2b = 1.0 / (double)mp.l2b;
+        for (int k = 0; k < (1 << NBITS); k++) a.table[k] = mp.table[k];
+    }
     return a;
 }
 
