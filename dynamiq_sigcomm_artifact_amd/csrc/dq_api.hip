@@ -10,6 +10,7 @@
 
 #include "dq_device.cuh"
 #include "dq_launch.h"
+#include "dq_mee_levels.cuh"
 
 namespace {
 
@@ -126,10 +127,9 @@ std::once_flag g_lut_once;
 void build_lut()
 {
     // csrc/cuda_hadamard.cu:873-899: fp32 host arithmetic, results kept as binary16
-    static const float epses[9] = {0.0f, 0.23f, 0.23f, 0.18f, 0.18f, 0.18f, 0.1f, 0.1f, 0.1f};
     memset(&g_lut, 0, sizeof(g_lut));
     for (int b = 1; b < 9; b++) {
-        const float eps = epses[b];
+        const float eps = dq::mee_eps(b);
         volatile float two_eps2 = 2.0f * eps * eps;
         volatile float base = 1.0f + two_eps2;
         volatile float one_plus_eps2 = 1.0f + eps * eps;
@@ -137,15 +137,7 @@ void build_lut()
         g_lut.params[b][1] = host_f32_to_f16(one_plus_eps2 / two_eps2);
         g_lut.params[b][3] = host_f32_to_f16(log2f(base));
         const int anchor = (1 << (b - 1)) - 1;
-        volatile float pw = 1.0f;
-        for (int j = 1; j <= anchor; j++) {
-            pw = pw * base;
-            volatile float num = pw - 1.0f;
-            volatile float quo = num / two_eps2;
-            volatile float rep = quo * one_plus_eps2;
-            g_lut.table[b][anchor + j] = host_f32_to_f16(rep);
-            g_lut.table[b][anchor - j] = host_f32_to_f16(-rep);
-        }
+        dq::mee_fill(g_lut.table[b], b);
         g_lut.params[b][2] = g_lut.table[b][anchor * 2];
         dq::MeeParams &m = g_lut.mp[b];
         m.c = host_f16_to_f32(g_lut.params[b][1]);

@@ -173,7 +173,7 @@ template <int DT, bool MEE> __global__ __launch_bounds__(64) void roundtrip_kern
     Raw16<DT> v;
     v.zero();
     if (active) load_chunk<DT>(v, b.src, e0, n, b.vec != 0, ragged);
-    if (MEE) levels_to_lds(a.widths, levels, lane);
+    if (MEE) levels_to_lds(levels, lane);
     // the rounding stream's arithmetic while the elements are on their way
     Raw16<DQ_PHILOX> r;
     r.generate(RandKey{a.seed, b.step + step}, sc * 16 + j);
@@ -503,7 +503,7 @@ __global__ __launch_bounds__(64, DT == DQ_BF16 && RDT == DQ_PHILOX && !MEE ? 5 :
     const int64_t sc = a.order[row0 + k0 + min(row, rows_here - 1)];
     const int64_t e0 = sc * 256 + j * 16;
     const bool ragged = __builtin_amdgcn_ballot_w64(e0 + 16 > a.n) != 0;
-    if (MEE) levels_to_lds(a.widths, levels, lane);
+    if (MEE) levels_to_lds(levels, lane);
     const WidthRegs<MEE> w = width_regs<MEE>(a.widths, cls, levels);
     const uint32_t total_mean = a.total[2 * sc];
 
@@ -589,7 +589,7 @@ __global__ __launch_bounds__(64 * kQuadWaves) void ring_quad_kernel(RingArgs<RDT
     __shared__ float levels[MEE ? kLevelCount : 1];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), world = a.world;
     if (MEE) {
-        if (wave == 0) levels_to_lds(a.widths, levels, lane);
+        if (wave == 0) levels_to_lds(levels, lane);
         if (!PLANS) __syncthreads();
     }
     const int at = (int)blockIdx.x * kQuadWaves + wave;

@@ -5,6 +5,7 @@
 
 #include <type_traits>
 #include "dq_device.cuh"
+#include "dq_mee_levels.cuh"
 
 namespace dq {
 
@@ -25,14 +26,12 @@ template <int NBITS, bool MEE> struct MeeArg {
     float c, cmm, l2b;
     uint32_t pad;
     double inv_c, inv_cmm, inv_l2b; // correctly rounded double reciprocals
-    uint16_t table[1 << NBITS];
 };
 
 // (AEE takes none of it: nothing for the host to write with every launch)
 template <int NBITS> struct MeeArg<NBITS, false> {
     static constexpr float c = 1.0f, cmm = 1.0f, l2b = 1.0f;
     static constexpr double inv_c = 1.0, inv_cmm = 1.0, inv_l2b = 1.0;
-    static constexpr uint16_t table[2] = {0, 0};
 };
 
 typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
@@ -228,7 +227,7 @@ template <class RR> struct DrawnBytes { static constexpr bool value = std::is_sa
 
 // ---- the MEE level table on its way into LDS -------------------------------------------------------
 //
-// The table comes with the kernel arguments as 2^NBITS binary16 patterns.  A lane fetches its pairs of entries with the
+// 2^NBITS binary16 patterns (kMeeLevels).  A lane fetches its pairs of entries with the
 // other loads of its tile (one or two 4-byte loads, no wait in between) and converts and stores them as floats once the
 // tile's own data has arrived.
 template <int NBITS> struct TableRegs {
@@ -237,10 +236,10 @@ template <int NBITS> struct TableRegs {
     uint32_t pair[kPerLane];
 };
 
-template <int NBITS, class ARG> __device__ __forceinline__ TableRegs<NBITS> table_fetch(const ARG &mp, int lane)
+template <int NBITS> __device__ __forceinline__ TableRegs<NBITS> table_fetch(int lane)
 {
     TableRegs<NBITS> t;
-    const uint32_t *pairs = reinterpret_cast<const uint32_t *>(mp.table); // 4-byte aligned inside the argument block
+    const uint32_t *pairs = reinterpret_cast<const uint32_t *>(kMeeLevels<NBITS>.at);
 #pragma unroll
     for (int j = 0; j < TableRegs<NBITS>::kPerLane; j++) {
         const int k = lane + 64 * j;
@@ -554,7 +553,6 @@ template <int NBITS, bool MEE> static MeeArg<NBITS, MEE> make_arg(const MeeParam
     if constexpr (MEE) {
         a.c = mp.c; a.cmm = mp.cmm; a.l2b = mp.l2b; a.pad = 0;
         a.inv_c = 1.0 / (double)mp.c; a.inv_cmm = 1.0 / (double)mp.cmm; a.inv_l2b = 1.0 / (double)mp.l2b;
-        for (int k = 0; k < (1 << NBITS); k++) a.table[k] = mp.table[k];
     }
     return a;
 }

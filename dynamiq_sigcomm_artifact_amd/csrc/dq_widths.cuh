@@ -27,12 +27,8 @@ struct WidthConst {
     float c, cmm, l2b;         // MEE
 };
 
-constexpr int kLevels[3] = {0, 256, 272}; // where each width's level table starts
-constexpr int kLevelCount = 276;
-
 struct WidthSet {
     WidthConst w[3];
-    uint16_t levels[280]; // MEE: binary16 level tables of the three widths end to end
 };
 
 // one width's constants in registers; table: its level zero among the floats in LDS (MEE)
@@ -65,10 +61,10 @@ template <bool MEE> __device__ __forceinline__ WidthRegs<MEE> width_regs(const W
     return x;
 }
 
-// the three level tables into LDS (kLevelCount floats): the kernel-argument loads of every lane leave together
-__device__ __forceinline__ void levels_to_lds(const WidthSet &s, float *levels, int lane)
+// the three level tables into LDS (kLevelCount floats): the loads of every lane leave together
+__device__ __forceinline__ void levels_to_lds(float *levels, int lane)
 {
-    const uint32_t *pairs = reinterpret_cast<const uint32_t *>(s.levels);
+    const uint32_t *pairs = reinterpret_cast<const uint32_t *>(kMeeLevelsOfWidths.at);
     uint32_t p[3];
 #pragma unroll
     for (int k = 0; k < 3; k++) p[k] = lane + 64 * k < kLevelCount / 2 ? pairs[lane + 64 * k] : 0u;
@@ -404,7 +400,6 @@ inline WidthSet make_width_set(const MeeParams *mp, bool mee)
         w.inv_top = 1.0f / (mee ? mp[k].cmm : (float)top);
         w.inv_c = 1.0 / (double)mp[k].c;
         w.inv_l2b = 1.0 / (double)mp[k].l2b;
-        for (int j = 0; mee && j < (1 << bits[k]); j++) s.levels[kLevels[k] + j] = mp[k].table[j];
     }
     return s;
 }
