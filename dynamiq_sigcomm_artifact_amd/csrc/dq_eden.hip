@@ -31,26 +31,30 @@ namespace dq {
 
 namespace {
 
-// several slices in one launch: slice k owns the workgroups from first[k] on, one per tile
-struct QuantizeSet {
-    QuantizeSlice s[kMaxEdenSlices];
-    unsigned first[kMaxEdenSlices];
+// Several slices in one launch: slice k owns the workgroups from first[k] on, one per tile.  A single slice travels alone: 104 bytes of
+// arguments instead of 600, which take the host and the GPU 1 us longer a launch (launch_with).
+template <int MOST> struct QuantizeSet {
+    QuantizeSlice s[MOST];
+    unsigned first[MOST];
     int count;
+    bool fold;
+    const float *boundaries, *centroids;
+    __device__ __forceinline__ int slice_of_block() const
+    {
+        int k = 0;
+        if constexpr (MOST > 1) {
+            for (int i = 1; i < count; i++)
+                if (blockIdx.x >= first[i]) k = i;
+        }
+        return k;
+    }
 };
 
-__device__ __forceinline__ int slice_of_block(const unsigned *first, int count)
-{
-    int k = 0;
-    for (int i = 1; i < count; i++)
-        if (blockIdx.x >= first[i]) k = i;
-    return k;
-}
-
 // A whole tile's loads leave together; behind a comparison each they wait for one another (6.9 -> 3.2 us at 2^20 elements).
-__global__ __launch_bounds__(kEdenThreads) void eden_sumsq_kernel(QuantizeSet set)
+template <int MOST> __global__ __launch_bounds__(kEdenThreads) void eden_sumsq_kernel(QuantizeSet<MOST> set)
 {
     __shared__ double lds[kEdenThreads];
-    const int which = slice_of_block(set.first, set.count);
+    const int which = set.slice_of_block();
     const QuantizeSlice &s = set.s[which];
     const int64_t tile = blockIdx.x - set.first[which], base = tile * kEdenTile;
     float v[kEdenPerThread];
@@ -152,14 +156,13 @@ __global__ __launch_bounds__(kEdenThreads) void eden_norm_kernel(double *sums, i
 // FOLD: the norm is not in result[3] yet; the workgroup folds the partial sums the way eden_norm_kernel does (the same
 // association: the same bits), workgroup 0 leaves result[0] and result[3] as that kernel would, and the
 // products go to a region of their own (other workgroups are still reading the sums).
-template <int NBITS, bool FOLD, int PER>
-__global__ __launch_bounds__(kEdenTile / PER) void eden_bins_kernel(QuantizeSet set, const float *__restrict__ boundaries,
-                                                                   const float *__restrict__ centroids)
+template <int NBITS, bool FOLD, int PER, int MOST>
+__global__ __launch_bounds__(kEdenTile / PER) void eden_bins_kernel(QuantizeSet<MOST> set)
 {
     constexpr int L = 1 << NBITS;
     __shared__ double lds[kEdenThreads];
     __shared__ float tree[L], cen[L];
-    const int which = FOLD ? slice_of_block(set.first, set.count) : 0;
+    const int which = FOLD ? set.slice_of_block() : 0;
     const QuantizeSlice &s = set.s[which];
     const int64_t tile = blockIdx.x - (FOLD ? set.first[which] : 0u);
     const int64_t tiles = eden_tiles(s.n);
@@ -184,7 +187,7 @@ __global__ __launch_bounds__(kEdenTile / PER) void eden_bins_kernel(QuantizeSet 
         for (int k = 0; k < PER; k++) v[k] = 0.0f;
     }
     const double part = FOLD ? first_of_array(s.sums, s.sum_count) : 0.0;
-    eden_tables<NBITS>(boundaries, centroids, tree, cen, threadIdx.x, kEdenTile / PER);
+    eden_tables<NBITS>(set.boundaries, set.centroids, tree, cen, threadIdx.x, kEdenTile / PER);
     __syncthreads();
     float norm;
     if constexpr (FOLD) {
@@ -206,12 +209,12 @@ __global__ __launch_bounds__(kEdenTile / PER) void eden_bins_kernel(QuantizeSet 
 }
 
 // one workgroup per slice: result[1] = (float)dot, result[2] = scale
-__global__ __launch_bounds__(kEdenThreads) void eden_scale_kernel(QuantizeSet set, bool fold)
+template <int MOST> __global__ __launch_bounds__(kEdenThreads) void eden_scale_kernel(QuantizeSet<MOST> set)
 {
     __shared__ double lds[kEdenThreads];
     const QuantizeSlice &s = set.s[blockIdx.x];
     const int64_t tiles = eden_tiles(s.n);
-    const double dot = fold_array(s.work + (fold && s.sums == s.work ? tiles : 0), tiles, lds);
+    const double dot = fold_array(s.work + (set.fold && s.sums == s.work ? tiles : 0), tiles, lds);
     if (threadIdx.x == 0) {
         const float d = (float)dot;
         const float norm = s.result[3];
@@ -321,12 +324,14 @@ int64_t eden_work_doubles(int64_t n)
 // 9.3 -> 9.2, 2^23 13.7 -> 13.4, 2^24 22.8 -> 23.4, 2^25 37.8 -> 42.5, 2^26 63.0 -> 72.9.
 constexpr int64_t kFewTiles = 2048;
 
-// slices of at most kEdenFoldTiles tiles, or one of any length; bits of an NBITS-wide code for all of them
-hipError_t launch_eden_quantize_slices(const QuantizeSlice *slices, int count, const float *boundaries, const float *centroids,
-                                       int nbits, hipStream_t stream)
+template <int MOST>
+static hipError_t quantize_slices(const QuantizeSlice *slices, int count, const float *boundaries, const float *centroids, int nbits,
+                                  hipStream_t stream)
 {
-    QuantizeSet set;
+    QuantizeSet<MOST> set;
     set.count = count;
+    set.boundaries = boundaries;
+    set.centroids = centroids;
     int64_t blocks = 0;
     bool have_sums = true;
     for (int k = 0; k < count; k++) have_sums = have_sums && slices[k].sums;
@@ -340,19 +345,24 @@ hipError_t launch_eden_quantize_slices(const QuantizeSlice *slices, int count, c
         set.first[k] = (unsigned)blocks;
         blocks += eden_tiles(slices[k].n);
     }
-    const bool fold = count > 1 || set.s[0].sum_count <= kEdenFoldTiles;
+    const bool fold = set.fold = count > 1 || set.s[0].sum_count <= kEdenFoldTiles;
     const bool few = fold && blocks <= kFewTiles;
-    dim3 grid((unsigned)blocks), block(kEdenThreads);
-    if (!have_sums) hipLaunchKernelGGL(eden_sumsq_kernel, grid, block, 0, stream, set);
-    if (!fold) hipLaunchKernelGGL(eden_norm_kernel, dim3(1), block, 0, stream, set.s[0].sums, set.s[0].sum_count, set.s[0].n, slices[0].result);
+    const dim3 grid((unsigned)blocks), block(kEdenThreads);
+    hipError_t e = hipSuccess;
+    if (!have_sums) e = launch_with(eden_sumsq_kernel<MOST>, grid, block, stream, set);
+    if (e == hipSuccess && !fold) {
+        hipLaunchKernelGGL(eden_norm_kernel, dim3(1), block, 0, stream, set.s[0].sums, set.s[0].sum_count, set.s[0].n, slices[0].result);
+        e = hipGetLastError();
+    }
+    if (e != hipSuccess) return e;
 #define DQ_EDEN_BINS(B)                                                                                       \
     do {                                                                                                      \
         if (few)                                                                                              \
-            hipLaunchKernelGGL((eden_bins_kernel<B, true, 8>), grid, dim3(kEdenTile / 8), 0, stream, set, boundaries, centroids); \
+            e = launch_with(eden_bins_kernel<B, true, 8, MOST>, grid, dim3(kEdenTile / 8), stream, set);      \
         else if (fold)                                                                                        \
-            hipLaunchKernelGGL((eden_bins_kernel<B, true, 16>), grid, block, 0, stream, set, boundaries, centroids); \
-        else                                                                                                  \
-            hipLaunchKernelGGL((eden_bins_kernel<B, false, 16>), grid, block, 0, stream, set, boundaries, centroids); \
+            e = launch_with(eden_bins_kernel<B, true, 16, MOST>, grid, block, stream, set);                   \
+        else if constexpr (MOST == 1)                                                                         \
+            e = launch_with(eden_bins_kernel<B, false, 16, MOST>, grid, block, stream, set);                  \
     } while (0)
     switch (nbits) {
     case 1: DQ_EDEN_BINS(1); break;
@@ -365,8 +375,15 @@ hipError_t launch_eden_quantize_slices(const QuantizeSlice *slices, int count, c
     default: DQ_EDEN_BINS(8); break;
     }
 #undef DQ_EDEN_BINS
-    hipLaunchKernelGGL(eden_scale_kernel, dim3((unsigned)count), block, 0, stream, set, fold);
-    return hipGetLastError();
+    return e == hipSuccess ? launch_with(eden_scale_kernel<MOST>, dim3((unsigned)count), block, stream, set) : e;
+}
+
+// slices of at most kEdenFoldTiles tiles, or one of any length; bits of an NBITS-wide code for all of them
+hipError_t launch_eden_quantize_slices(const QuantizeSlice *slices, int count, const float *boundaries, const float *centroids,
+                                       int nbits, hipStream_t stream)
+{
+    return count == 1 ? quantize_slices<1>(slices, count, boundaries, centroids, nbits, stream)
+                      : quantize_slices<kMaxEdenSlices>(slices, count, boundaries, centroids, nbits, stream);
 }
 
 hipError_t launch_eden_quantize(const float *vec, int64_t n, const float *boundaries, const float *centroids, int nbits,

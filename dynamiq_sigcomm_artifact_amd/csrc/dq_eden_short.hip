@@ -16,9 +16,10 @@ namespace {
 
 constexpr int kShortThreads = kEdenShort / 16;
 
-struct ShortSet {
-    dq_eden_slice_t s[kMaxEdenSlices];
-    float inv[kMaxEdenSlices], sqrt_n[kMaxEdenSlices]; // 1 / sqrt(n) and sqrt(n) as torch takes them
+// (one slice travels alone: an eighth of the arguments)
+template <int MOST> struct ShortSet {
+    dq_eden_slice_t s[MOST];
+    float inv[MOST], sqrt_n[MOST]; // 1 / sqrt(n) and sqrt(n) as torch takes them
     int dtype;
 };
 
@@ -58,7 +59,7 @@ __device__ __forceinline__ double fold_tiles(const double *sums, int n)
     return (sums[0] + sums[2 * kEdenThreads]) + (sums[kEdenThreads] + sums[3 * kEdenThreads]);
 }
 
-template <int NBITS> __global__ __launch_bounds__(kShortThreads) void eden_short_compress_kernel(ShortSet set)
+template <int NBITS, int MOST> __global__ __launch_bounds__(kShortThreads) void eden_short_compress_kernel(ShortSet<MOST> set)
 {
     constexpr int L = 1 << NBITS;
     extern __shared__ __attribute__((aligned(16))) float lds[];
@@ -126,7 +127,7 @@ template <int NBITS> __global__ __launch_bounds__(kShortThreads) void eden_short
     }
 }
 
-__global__ __launch_bounds__(kShortThreads) void eden_short_decompress_kernel(ShortSet set)
+template <int MOST> __global__ __launch_bounds__(kShortThreads) void eden_short_decompress_kernel(ShortSet<MOST> set)
 {
     extern __shared__ __attribute__((aligned(16))) float lds[];
     __shared__ float cen[256];
@@ -158,7 +159,8 @@ __global__ __launch_bounds__(kShortThreads) void eden_short_decompress_kernel(Sh
 }
 
 // threads: a multiple of 256 that gives every chunk of the longest slice one
-hipError_t short_set(const dq_eden_slice_t *slices, int count, int dtype, ShortSet &set, unsigned *threads, size_t *lds)
+template <int MOST>
+hipError_t short_set(const dq_eden_slice_t *slices, int count, int dtype, ShortSet<MOST> &set, unsigned *threads, size_t *lds)
 {
     int64_t most = 32;
     if (count < 1 || count > kMaxEdenSlices) return hipErrorInvalidValue;
@@ -175,44 +177,49 @@ hipError_t short_set(const dq_eden_slice_t *slices, int count, int dtype, ShortS
     return hipSuccess;
 }
 
+template <int MOST> hipError_t short_compress(const dq_eden_slice_t *slices, int count, int dtype, hipStream_t stream)
+{
+    ShortSet<MOST> set;
+    unsigned threads;
+    size_t lds;
+    const hipError_t e = short_set(slices, count, dtype, set, &threads, &lds);
+    if (e != hipSuccess) return e;
+    const auto go = [&](auto kernel) {
+        const hipError_t allowed = allow_lds(kernel, lds);
+        return allowed == hipSuccess ? launch_with(kernel, dim3((unsigned)count), dim3(threads), stream, set, lds) : allowed;
+    };
+    switch (slices[0].nbits) {
+    case 1: return go(eden_short_compress_kernel<1, MOST>);
+    case 2: return go(eden_short_compress_kernel<2, MOST>);
+    case 3: return go(eden_short_compress_kernel<3, MOST>);
+    case 4: return go(eden_short_compress_kernel<4, MOST>);
+    case 5: return go(eden_short_compress_kernel<5, MOST>);
+    case 6: return go(eden_short_compress_kernel<6, MOST>);
+    case 7: return go(eden_short_compress_kernel<7, MOST>);
+    default: return go(eden_short_compress_kernel<8, MOST>);
+    }
+}
+
+template <int MOST> hipError_t short_decompress(const dq_eden_slice_t *slices, int count, int dtype, hipStream_t stream)
+{
+    ShortSet<MOST> set;
+    unsigned threads;
+    size_t lds;
+    hipError_t e = short_set(slices, count, dtype, set, &threads, &lds);
+    if (e == hipSuccess) e = allow_lds(eden_short_decompress_kernel<MOST>, lds);
+    return e == hipSuccess ? launch_with(eden_short_decompress_kernel<MOST>, dim3((unsigned)count), dim3(threads), stream, set, lds) : e;
+}
+
 } // namespace
 
 hipError_t launch_eden_short_compress(const dq_eden_slice_t *slices, int count, int dtype, hipStream_t stream)
 {
-    ShortSet set;
-    unsigned threads;
-    size_t lds;
-    hipError_t e = short_set(slices, count, dtype, set, &threads, &lds);
-    if (e != hipSuccess) return e;
-    const auto go = [&](auto kernel) {
-        e = allow_lds(kernel, lds);
-        if (e == hipSuccess) hipLaunchKernelGGL(kernel, dim3((unsigned)count), dim3(threads), lds, stream, set);
-    };
-    switch (slices[0].nbits) {
-    case 1: go(eden_short_compress_kernel<1>); break;
-    case 2: go(eden_short_compress_kernel<2>); break;
-    case 3: go(eden_short_compress_kernel<3>); break;
-    case 4: go(eden_short_compress_kernel<4>); break;
-    case 5: go(eden_short_compress_kernel<5>); break;
-    case 6: go(eden_short_compress_kernel<6>); break;
-    case 7: go(eden_short_compress_kernel<7>); break;
-    default: go(eden_short_compress_kernel<8>); break;
-    }
-    if (e != hipSuccess) return e;
-    return hipGetLastError();
+    return count == 1 ? short_compress<1>(slices, count, dtype, stream) : short_compress<kMaxEdenSlices>(slices, count, dtype, stream);
 }
 
 hipError_t launch_eden_short_decompress(const dq_eden_slice_t *slices, int count, int dtype, hipStream_t stream)
 {
-    ShortSet set;
-    unsigned threads;
-    size_t lds;
-    hipError_t e = short_set(slices, count, dtype, set, &threads, &lds);
-    if (e != hipSuccess) return e;
-    e = allow_lds(eden_short_decompress_kernel, lds);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(eden_short_decompress_kernel, dim3((unsigned)count), dim3(threads), lds, stream, set);
-    return hipGetLastError();
+    return count == 1 ? short_decompress<1>(slices, count, dtype, stream) : short_decompress<kMaxEdenSlices>(slices, count, dtype, stream);
 }
 
 } // namespace dq

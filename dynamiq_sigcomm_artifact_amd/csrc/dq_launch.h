@@ -15,11 +15,11 @@ namespace dq {
 // A kernel whose only argument is `args`.  Short calls wait for the host, and the runtime copies a kernel's arguments one by one to
 // where the GPU reads them: a decoder call of eight arguments and 104 bytes takes 3.8 us, with one argument of 56 bytes 2.9 (and 576
 // bytes 1.1 us more than 64).  Eight ranks' ring of 65,792 elements, 17 calls, 68 -> 55 us of host time.
-template <class K, class A> inline hipError_t launch_with(K *kernel, dim3 grid, dim3 block, hipStream_t stream, const A &args)
+template <class K, class A> inline hipError_t launch_with(K *kernel, dim3 grid, dim3 block, hipStream_t stream, const A &args, size_t lds = 0)
 {
     static_assert(std::is_same<K, void(A)>::value, "the kernel takes these arguments");
     void *list[] = {const_cast<A *>(&args)};
-    const hipError_t e = hipLaunchKernel(reinterpret_cast<const void *>(kernel), grid, block, list, 0, stream);
+    const hipError_t e = hipLaunchKernel(reinterpret_cast<const void *>(kernel), grid, block, list, lds, stream);
     if (e != hipSuccess) (void)hipGetLastError();
     return e;
 }
@@ -208,11 +208,23 @@ struct UniformDraw {
 
 // Quantisers folded into the two ends of a transform (all null: the plain transform).  `in_*` replace the load of the
 // first pass, `out_*` / `post_scale` act on the store of the last one.
-struct TransformEnds {
+// What a first pass looks at, and what a strided one does, are kernel arguments by themselves: 264 bytes of both in seven arguments take
+// the host and the GPU 1 us longer a launch (launch_with).
+struct InEnds {
     // the first pass loads in_count elements of in_dtype from in_src, zeros behind them, instead of x
     const void *in_src = nullptr;
     int in_dtype = 0;
     int64_t in_count = 0;
+    // THC: the pass loads float(level) * *in_step + *in_lo instead of x
+    const uint16_t *in_levels = nullptr;
+    const float *in_step = nullptr, *in_lo = nullptr;
+    // EDEN: the pass loads centroids[bin] from the bit planes of the bins
+    const uint32_t *in_planes = nullptr;
+    const float *in_centroids = nullptr;
+    int in_nbits = 0;
+    bool plain_in() const { return !in_src && !in_levels && !in_planes; }
+};
+struct OutEnds {
     // a strided pass over the whole vector that draws THC's uniform values finds zeros from here on and does not read them (a
     // multiple of its row stride; negative: it reads everything)
     int64_t zeros_from = -1;
@@ -220,30 +232,24 @@ struct TransformEnds {
     void *out_dst = nullptr;
     int out_dtype = 0;
     int64_t out_count = 0;
-    // THC with the grid worked out in the kernels instead of in_step / in_lo / out_lo / out_delta
-    ThcGrid grid;
-    // the diagonal drawn in the kernels instead of a sign vector
-    SignSeed gen;
-    bool plain_in() const { return !in_src && !in_levels && !in_planes; }
-    bool plain_out() const { return !out_dst && !out_levels && !post_scale && !sums; }
-    bool plain() const { return plain_in() && plain_out() && gen.bits == 0; }
-
-    // THC: the pass loads float(level) * *in_step + *in_lo instead of x
-    const uint16_t *in_levels = nullptr;
-    const float *in_step = nullptr, *in_lo = nullptr;
     // THC: the pass stores thc_level(value, uniform) as bf16 instead of the value
     uint16_t *out_levels = nullptr;
     const float *uniform = nullptr, *out_lo = nullptr, *out_delta = nullptr;
     float out_top = 0.0f;
     UniformDraw draw; // instead of uniform: transforms of 2^19 .. 2^25 elements
-    // EDEN: the pass loads centroids[bin] from the bit planes of the bins; the last pass multiplies by *post_scale
-    const uint32_t *in_planes = nullptr;
-    const float *in_centroids = nullptr;
-    int in_nbits = 0;
+    // EDEN: the last pass multiplies by *post_scale
     const float *post_scale = nullptr;
     // EDEN: a strided last pass over the whole vector also leaves, in double, the sum of the squares of the values that its
     // workgroup w stores in sums[w] (rht_sum_count of them, in the order of dq_sums.cuh)
     double *sums = nullptr;
+    bool plain_out() const { return !out_dst && !out_levels && !post_scale && !sums; }
+};
+struct TransformEnds : InEnds, OutEnds {
+    // THC with the grid worked out in the kernels instead of in_step / in_lo / out_lo / out_delta
+    ThcGrid grid;
+    // the diagonal drawn in the kernels instead of a sign vector
+    SignSeed gen;
+    bool plain() const { return plain_in() && plain_out() && gen.bits == 0; }
 };
 // workgroups of the last pass of a whole-vector transform by launch_rht_ends; 0: that pass knows no sums
 int64_t rht_sum_count(int64_t n);

@@ -392,7 +392,7 @@ __device__ __forceinline__ void grid_of(const ThcGrid &d, const float *lo_p, con
 }
 
 // sixteen elements of a source of another type or length than the transform
-__device__ __forceinline__ void load_source(float (&v)[16], const TransformEnds &e, int64_t g)
+__device__ __forceinline__ void load_source(float (&v)[16], const InEnds &e, int64_t g)
 {
     const bool whole = g + 16 <= e.in_count && (reinterpret_cast<uintptr_t>(e.in_src) & 15) == 0;
     if (e.in_dtype == DQ_F32) {
@@ -429,7 +429,7 @@ __device__ __forceinline__ void load_source(float (&v)[16], const TransformEnds 
 }
 
 // four elements of a destination of another type or length (out_dst aligned to four elements, or element by element)
-__device__ __forceinline__ void store_destination(const TransformEnds &e, float4 v, int64_t g)
+__device__ __forceinline__ void store_destination(const OutEnds &e, float4 v, int64_t g)
 {
     if (g >= e.out_count) return;
     const float f[4] = {v.x, v.y, v.z, v.w};
@@ -458,7 +458,7 @@ __device__ __forceinline__ void store_destination(const TransformEnds &e, float4
 }
 
 // the centroids of sixteen consecutive bins, from the thread's half word of every plane (two 8 x 8 bit transposes)
-__device__ __forceinline__ void load_planes(float (&v)[16], const TransformEnds &e, const float *cen, int64_t g, int64_t words)
+__device__ __forceinline__ void load_planes(float (&v)[16], const InEnds &e, const float *cen, int64_t g, int64_t words)
 {
     const uint16_t *half = reinterpret_cast<const uint16_t *>(e.in_planes) + (g >> 4);
     // (eight loads whatever the width, the last plane's again: in a loop over the planes they wait for one another)
@@ -485,9 +485,9 @@ __device__ __forceinline__ void load_planes(float (&v)[16], const TransformEnds 
 // pass sees it: the floats of x, or THC's levels times step plus lo (thc_hooks.py:176-178: two roundings), or the
 // centroids of EDEN's bins, read from the bit planes (srrcomp.py:343-354); then the sign flip of a forward transform.
 // cen: the centroid table in LDS.
-template <bool ENDS>
+template <bool ENDS, class E>
 __device__ __forceinline__ void fetch_chunk(float (&v)[16], const float *__restrict__ x, const PassArgs<ENDS> &in,
-                                            const TransformEnds &e, const float *cen, int64_t g)
+                                            const E &e, const float *cen, int64_t g)
 {
     if (!ENDS || (!e.in_levels && !e.in_planes && !e.in_src)) {
         load_chunk(v, x, in, g);
@@ -721,8 +721,8 @@ __device__ __forceinline__ void tile_pass(float *__restrict__ x, const PassArgs<
 // The first pass of a long transform: the tile is one block of 2^10 .. 2^14 elements, a chunk per thread, with nothing to do on
 // the way out.  The last stages store from registers, as whole 256-byte runs: one trip through the LDS and one barrier less
 // than tile_pass.  Bound like the strided passes; 2^23 elements from bf16 levels 13.4 -> 11.8 us, from a 25 MB gradient 17.3 -> 15.0.
-template <bool ENDS>
-__device__ __forceinline__ void first_pass(float *__restrict__ x, const PassArgs<ENDS> &a, int sign_mode, const TransformEnds &e, unsigned block,
+template <bool ENDS, class E>
+__device__ __forceinline__ void first_pass(float *__restrict__ x, const PassArgs<ENDS> &a, int sign_mode, const E &e, unsigned block,
                                            float *lds)
 {
     const int tid = threadIdx.x;
@@ -844,9 +844,9 @@ template <int B> __device__ __forceinline__ void draw_rows(float (&u)[1 << B], c
 // loads of uniform values, which may be pending in the registers that the draws go to as far as the compiler can tell, every draw
 // waited for elements it does not need.  2^23 elements to THC's levels, with thc_levels in groups: both ways 54.1 -> 52.8 us, 2^24 103.5 ->
 // 100.5, padded 25 MB (with e.zeros_from) 50.7 -> 48.
-template <bool ENDS, int A, int B, bool DRAW = false>
+template <bool ENDS, int A, int B, bool DRAW = false, class E>
 __device__ __forceinline__ void strided_rows(float *__restrict__ x, const PassArgs<ENDS> &a, int sbits, int sign_mode, int apply_scale,
-                                             const TransformEnds &e, unsigned block, float *lds)
+                                             const E &e, unsigned block, float *lds)
 {
     constexpr int R1 = 1 << A, R2 = 1 << B;
     const int tid = threadIdx.x;
@@ -1066,9 +1066,9 @@ __host__ constexpr size_t strided_lds_bytes(int rbits) { return (sizeof(float) <
 // threads of the tile of a strided pass
 __host__ __device__ constexpr int strided_threads(int rbits) { return rbits >= 9 ? 1 << rbits : 1 << (rbits + 1); }
 
-template <bool ENDS>
+template <bool ENDS, class E>
 __device__ __forceinline__ void strided_pass(float *__restrict__ x, const PassArgs<ENDS> &a, int rbits, int sbits, int sign_mode,
-                                             int apply_scale, const TransformEnds &e, unsigned block, float *lds)
+                                             int apply_scale, const E &e, unsigned block, float *lds)
 {
     switch (rbits) {
     case 4: strided_rows<ENDS, 4, 0>(x, a, sbits, sign_mode, apply_scale, e, block, lds); break;
@@ -1079,37 +1079,52 @@ __device__ __forceinline__ void strided_pass(float *__restrict__ x, const PassAr
     }
 }
 
-template <bool ENDS>
-__global__ __launch_bounds__(512) void rht_strided_kernel(float *__restrict__ x, PassArgs<ENDS> a, int rbits, int sbits, int sign_mode,
-                                                          int apply_scale, TransformEnds e)
+// the arguments of a pass, and the ends that it looks at
+struct FirstEnds : InEnds {
+    ThcGrid grid;
+};
+struct LastEnds : OutEnds {
+    ThcGrid grid;
+};
+
+template <bool ENDS> struct FirstPass {
+    float *x;
+    PassArgs<ENDS> a;
+    int sign_mode;
+    FirstEnds e;
+};
+
+template <bool ENDS> struct StridedPass {
+    float *x;
+    PassArgs<ENDS> a;
+    int rbits, sbits, sign_mode, apply_scale;
+    LastEnds e;
+};
+
+template <bool ENDS> __global__ __launch_bounds__(512) void rht_strided_kernel(StridedPass<ENDS> p)
 {
     extern __shared__ __attribute__((aligned(16))) float lds[];
-    strided_pass<ENDS>(x, a, rbits, sbits, sign_mode, apply_scale, e, blockIdx.x, lds);
+    strided_pass<ENDS>(p.x, p.a, p.rbits, p.sbits, p.sign_mode, p.apply_scale, p.e, blockIdx.x, lds);
 }
 
 // 512 (B = 4) or 1024 rows (B = 5)
-template <bool ENDS, int B>
-__global__ __launch_bounds__(32 << B) void rht_strided_long_kernel(float *__restrict__ x, PassArgs<ENDS> a, int sbits, int sign_mode,
-                                                                   int apply_scale, TransformEnds e)
+template <bool ENDS, int B> __global__ __launch_bounds__(32 << B) void rht_strided_long_kernel(StridedPass<ENDS> p)
 {
     extern __shared__ __attribute__((aligned(16))) float lds[];
-    strided_rows<ENDS, 5, B>(x, a, sbits, sign_mode, apply_scale, e, blockIdx.x, lds);
+    strided_rows<ENDS, 5, B>(p.x, p.a, p.sbits, p.sign_mode, p.apply_scale, p.e, blockIdx.x, lds);
 }
 
 // 256 (A = 4) or 1024 rows (A = 5) to THC's levels with drawn values
-template <int A>
-__global__ __launch_bounds__(32 << A) void rht_strided_draw_kernel(float *__restrict__ x, RhtPassArgs a, int sbits, int sign_mode,
-                                                                   int apply_scale, TransformEnds e)
+template <int A> __global__ __launch_bounds__(32 << A) void rht_strided_draw_kernel(StridedPass<true> p)
 {
     extern __shared__ __attribute__((aligned(16))) float lds[];
-    strided_rows<true, A, A, true>(x, a, sbits, sign_mode, apply_scale, e, blockIdx.x, lds);
+    strided_rows<true, A, A, true>(p.x, p.a, p.sbits, p.sign_mode, p.apply_scale, p.e, blockIdx.x, lds);
 }
 
-template <bool ENDS>
-__global__ __launch_bounds__(1024) void rht_first_kernel(float *__restrict__ x, PassArgs<ENDS> a, int sign_mode, TransformEnds e)
+template <bool ENDS> __global__ __launch_bounds__(1024) void rht_first_kernel(FirstPass<ENDS> p)
 {
     extern __shared__ __attribute__((aligned(16))) float lds[];
-    first_pass<ENDS>(x, a, sign_mode, e, blockIdx.x, lds);
+    first_pass<ENDS>(p.x, p.a, p.sign_mode, p.e, blockIdx.x, lds);
 }
 
 #if DQ_RHT_PART & DQ_RHT_TRANSFORM
@@ -1628,13 +1643,13 @@ hipError_t launch_rht_tile(float *x, const void *sign, int sign_bits, int64_t n,
     const dim3 grid((unsigned)((n + tile - 1) >> kt));
     if (sign_mode != 2 && !apply_scale && kb == kt && kt <= 14 && vec && (n & (tile - 1)) == 0 && ends.plain_out()) {
         const int mode = diagonal ? sign_mode : 0;
-        const auto launch = [&](auto kernel, const auto &args) -> hipError_t {
+        const auto launch = [&](auto kernel, const auto &pass) -> hipError_t {
             const hipError_t e = allow_lds(kernel, lds);
-            if (e != hipSuccess) return e;
-            hipLaunchKernelGGL(kernel, grid, dim3(threads), lds, stream, x, args, mode, ends);
-            return hipGetLastError();
+            return e == hipSuccess ? launch_with(kernel, grid, dim3(threads), stream, pass, lds) : e;
         };
-        return plain ? launch(rht_first_kernel<false>, plain_args) : launch(rht_first_kernel<true>, a);
+        const FirstEnds e{ends, ends.grid};
+        return plain ? launch(rht_first_kernel<false>, FirstPass<false>{x, plain_args, mode, e})
+                     : launch(rht_first_kernel<true>, FirstPass<true>{x, a, mode, e});
     }
     if (plain) {
         hipError_t e = allow_lds(rht_tile_kernel<false>, lds);
@@ -1662,21 +1677,23 @@ hipError_t launch_rht_strided(float *x, const void *sign, int sign_bits, int64_t
     const RhtTileArgs &plain_args = a;
     const dim3 grid((unsigned)(n >> (rbits + 5))), block((unsigned)strided_threads(rbits));
     const size_t lds = strided_lds_bytes(rbits);
-    const auto launch = [&](auto kernel, const auto &args, auto... bits) -> hipError_t {
+    const int mode = sign || ends.gen.bits != 0 ? sign_mode : 0;
+    const LastEnds last{ends, ends.grid};
+    const auto launch = [&](auto kernel, const auto &pass) -> hipError_t {
         const hipError_t e = allow_lds(kernel, lds);
-        if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(kernel, grid, block, lds, stream, x, args, bits..., sign || ends.gen.bits != 0 ? sign_mode : 0, apply_scale, ends);
-        return hipGetLastError();
+        return e == hipSuccess ? launch_with(kernel, grid, block, stream, pass, lds) : e;
     };
     if (plain) {
-        if (rbits == 10) return launch(rht_strided_long_kernel<false, 5>, plain_args, sbits);
-        if (rbits == 9) return launch(rht_strided_long_kernel<false, 4>, plain_args, sbits);
-        return launch(rht_strided_kernel<false>, plain_args, rbits, sbits);
+        const StridedPass<false> p{x, plain_args, rbits, sbits, mode, apply_scale, last};
+        if (rbits == 10) return launch(rht_strided_long_kernel<false, 5>, p);
+        if (rbits == 9) return launch(rht_strided_long_kernel<false, 4>, p);
+        return launch(rht_strided_kernel<false>, p);
     }
-    if (draws) return rbits == 10 ? launch(rht_strided_draw_kernel<5>, a, sbits) : launch(rht_strided_draw_kernel<4>, a, sbits);
-    if (rbits == 10) return launch(rht_strided_long_kernel<true, 5>, a, sbits);
-    if (rbits == 9) return launch(rht_strided_long_kernel<true, 4>, a, sbits);
-    return launch(rht_strided_kernel<true>, a, rbits, sbits);
+    const StridedPass<true> p{x, a, rbits, sbits, mode, apply_scale, last};
+    if (draws) return rbits == 10 ? launch(rht_strided_draw_kernel<5>, p) : launch(rht_strided_draw_kernel<4>, p);
+    if (rbits == 10) return launch(rht_strided_long_kernel<true, 5>, p);
+    if (rbits == 9) return launch(rht_strided_long_kernel<true, 4>, p);
+    return launch(rht_strided_kernel<true>, p);
 }
 
 // every x 16-byte aligned, n a multiple of 2^kt and 10 <= kt <= 14
