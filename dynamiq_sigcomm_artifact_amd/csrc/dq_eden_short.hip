@@ -21,6 +21,7 @@ template <int MOST> struct ShortSet {
     dq_eden_slice_t s[MOST];
     float inv[MOST], sqrt_n[MOST]; // 1 / sqrt(n) and sqrt(n) as torch takes them
     int dtype;
+    int threads; // of a workgroup
 };
 
 // the diagonal of one rotation (sign_seed of dq_hadamard.hip in 32-bit arithmetic: only low words are used)
@@ -65,7 +66,7 @@ template <int NBITS, int MOST> __global__ __launch_bounds__(kShortThreads) void 
     extern __shared__ __attribute__((aligned(16))) float lds[];
     __shared__ double sums[kShortThreads];
     __shared__ float tree[L], cen[L];
-    const int tid = threadIdx.x, nthreads = blockDim.x;
+    const int tid = threadIdx.x, nthreads = set.threads;
     const dq_eden_slice_t &s = set.s[blockIdx.x];
     const int n = (int)s.n, kb = 31 - __builtin_clz((unsigned)n);
     const bool mine = tid < n / 16;
@@ -131,7 +132,7 @@ template <int MOST> __global__ __launch_bounds__(kShortThreads) void eden_short_
 {
     extern __shared__ __attribute__((aligned(16))) float lds[];
     __shared__ float cen[256];
-    const int tid = threadIdx.x, nthreads = blockDim.x;
+    const int tid = threadIdx.x, nthreads = set.threads;
     const dq_eden_slice_t &s = set.s[blockIdx.x];
     const int n = (int)s.n, kb = 31 - __builtin_clz((unsigned)n);
     const bool mine = tid < n / 16;
@@ -172,7 +173,7 @@ hipError_t short_set(const dq_eden_slice_t *slices, int count, int dtype, ShortS
         set.inv[k] = 1.0f / set.sqrt_n[k];
     }
     set.dtype = dtype;
-    *threads = (unsigned)((most / 16 + kEdenThreads - 1) / kEdenThreads * kEdenThreads);
+    *threads = set.threads = (unsigned)((most / 16 + kEdenThreads - 1) / kEdenThreads * kEdenThreads);
     *lds = (size_t)padded_tile_floats(ilog2(most)) * sizeof(float);
     return hipSuccess;
 }

@@ -66,6 +66,9 @@ struct RhtTileArgs {
 struct RhtPassArgs : RhtTileArgs {
     SignSeed gen;
 };
+// threads of a tile of 2^kt elements: a chunk each.  (Asked of the launch, their number costs 256 bytes of hidden arguments.)
+__host__ __device__ constexpr int tile_threads(int kt) { return kt < 10 ? 64 : (kt > 14 ? 1024 : 1 << (kt - 4)); }
+
 template <bool ENDS> using PassArgs = typename std::conditional<ENDS, RhtPassArgs, RhtTileArgs>::type;
 
 // Element g of the diagonal of rand_diag (srrcomp.py:61-106; rand_diag_word of dq_hadamard.hip in 32-bit arithmetic: only
@@ -213,7 +216,7 @@ __global__ __attribute__((amdgpu_waves_per_eu(8, 8))) void rht_compress_kernel(c
 {
     typedef Rec<NBITS> RC;
     extern __shared__ __attribute__((aligned(16))) float lds[];
-    const int tid = threadIdx.x, nthreads = blockDim.x;
+    const int tid = threadIdx.x, nthreads = tile_threads(a.kt);
     const int tile = 1 << a.kt;
     const int64_t origin = (int64_t)blockIdx.x << a.kt;
 
@@ -271,7 +274,7 @@ __global__ void irht_decompress_tile_kernel(const uint8_t *__restrict__ src, flo
 {
     typedef Rec<NBITS> RC;
     extern __shared__ __attribute__((aligned(16))) float lds[];
-    const int tid = threadIdx.x, nthreads = blockDim.x;
+    const int tid = threadIdx.x, nthreads = tile_threads(a.kt);
     const int tile = 1 << a.kt;
     const int64_t origin = (int64_t)blockIdx.x << a.kt;
     const int lane = tid & 63, wave = tid >> 6, nwaves = nthreads >> 6;
@@ -663,7 +666,7 @@ template <bool ENDS>
 __device__ __forceinline__ void tile_pass(float *__restrict__ x, const PassArgs<ENDS> &a, int sign_mode, int apply_scale,
                                           const TransformEnds &e, unsigned block, float *lds)
 {
-    const int tid = threadIdx.x, nthreads = blockDim.x;
+    const int tid = threadIdx.x, nthreads = tile_threads(a.kt);
     const int tile = 1 << a.kt;
     const int64_t origin = (int64_t)block << a.kt;
     PassArgs<ENDS> in = a;
@@ -723,7 +726,7 @@ __device__ __forceinline__ void tile_pass(float *__restrict__ x, const PassArgs<
 // than tile_pass.  Bound like the strided passes; 2^23 elements from bf16 levels 13.4 -> 11.8 us, from a 25 MB gradient 17.3 -> 15.0.
 template <bool ENDS, class E>
 __device__ __forceinline__ void first_pass(float *__restrict__ x, const PassArgs<ENDS> &a, int sign_mode, const E &e, unsigned block,
-                                           float *lds)
+                                           float *lds, int threads)
 {
     const int tid = threadIdx.x;
     const int64_t origin = (int64_t)block << a.kt;
@@ -734,7 +737,7 @@ __device__ __forceinline__ void first_pass(float *__restrict__ x, const PassArgs
     }
     const float *cen = lds + padded_tile_floats(a.kt); // EDEN's centroids sit behind the tile
     if (ENDS && e.in_planes) {
-        for (int k = tid; k < (1 << e.in_nbits); k += blockDim.x) lds[padded_tile_floats(a.kt) + k] = e.in_centroids[k];
+        for (int k = tid; k < (1 << e.in_nbits); k += threads) lds[padded_tile_floats(a.kt) + k] = e.in_centroids[k];
         __syncthreads();
     }
     const int nthreads = 1 << (a.kt - 4);
@@ -751,7 +754,7 @@ __device__ __forceinline__ void first_pass(float *__restrict__ x, const PassArgs
     else
         fetch_into(std::integral_constant<int, 12>()); // (and below)
     __syncthreads();
-    const int step = blockDim.x;
+    const int step = threads;
     switch (a.kt) {
     case 10: middle_stages<10>(lds, tid, step); break;
     case 11: middle_stages<11>(lds, tid, step); break;
@@ -1124,7 +1127,7 @@ template <int A> __global__ __launch_bounds__(32 << A) void rht_strided_draw_ker
 template <bool ENDS> __global__ __launch_bounds__(1024) void rht_first_kernel(FirstPass<ENDS> p)
 {
     extern __shared__ __attribute__((aligned(16))) float lds[];
-    first_pass<ENDS>(p.x, p.a, p.sign_mode, p.e, blockIdx.x, lds);
+    first_pass<ENDS>(p.x, p.a, p.sign_mode, p.e, blockIdx.x, lds, tile_threads(p.a.kt));
 }
 
 #if DQ_RHT_PART & DQ_RHT_TRANSFORM
@@ -1158,7 +1161,7 @@ __global__ __launch_bounds__(1024) void rht_tile_passes_kernel(PassSet set)
 {
     extern __shared__ __attribute__((aligned(16))) float lds[];
     const TilePass &p = pass_of_block();
-    first_pass<true>(p.x, pass_args(p), p.sign_mode, p.ends, blockIdx.x - p.first, lds);
+    first_pass<true>(p.x, pass_args(p), p.sign_mode, p.ends, blockIdx.x - p.first, lds, blockDim.x);
 }
 
 __global__ __launch_bounds__(512) void rht_strided_passes_kernel(PassSet set)
@@ -1422,8 +1425,7 @@ Geometry geometry(const float *vec, const void *sign, int sign_bits, int64_t n, 
     g.a.sign = sign; g.a.sign_bits = sign_bits; g.a.n = n; g.a.kt = kt; g.a.kb = kb; g.a.scale = scale;
     g.a.vec = aligned16(vec) && (sign == nullptr || sign_bits || aligned16(sign)) ? 1 : 0;
     const int tile = 1 << kt;
-    int threads = tile / 16;
-    g.threads = (unsigned)(threads < 64 ? 64 : (threads > 1024 ? 1024 : threads));
+    g.threads = (unsigned)tile_threads(kt);
     g.grid = (unsigned)((n + tile - 1) >> kt);
     g.lds_floats = (size_t)padded_tile_floats(kt);
     return g;
@@ -1638,7 +1640,7 @@ hipError_t launch_rht_tile(float *x, const void *sign, int sign_bits, int64_t n,
                            sign ? sign_mode : 0, apply_scale);
         return hipGetLastError();
     }
-    const unsigned threads = (unsigned)std::min(1024, tile / 16);
+    const unsigned threads = (unsigned)tile_threads(kt);
     const size_t lds = ((size_t)padded_tile_floats(kt) + (ends.in_planes ? 256 : 0)) * sizeof(float);
     const dim3 grid((unsigned)((n + tile - 1) >> kt));
     if (sign_mode != 2 && !apply_scale && kb == kt && kt <= 14 && vec && (n & (tile - 1)) == 0 && ends.plain_out()) {

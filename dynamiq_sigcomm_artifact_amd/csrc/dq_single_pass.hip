@@ -117,9 +117,10 @@ struct WidthRule {
     int thr[2];          // with u a number: the patterns of width 4 and 8 found on the host, else -1
 };
 
-struct RoundtripArgs {
-    uint32_t first_tile[kMaxBuckets]; // ascending
-    RoundtripBucket bucket[kMaxBuckets];
+// (A launch carries arguments for one bucket, twelve or kMaxBuckets: 2 KB of them take the host and the GPU 2 us longer than 300 bytes.)
+template <int MOST> struct RoundtripArgs {
+    uint32_t first_tile[MOST]; // ascending
+    RoundtripBucket bucket[MOST];
     int buckets;
     WidthRule rule;
     WorldDiv wd;
@@ -151,7 +152,7 @@ __device__ __forceinline__ int last_at_most(const uint32_t *list, int count, uin
     return lo;
 }
 
-template <int DT, bool MEE> __global__ __launch_bounds__(64) void roundtrip_kernel(RoundtripArgs a)
+template <int DT, bool MEE, int MOST> __global__ __launch_bounds__(64) void roundtrip_kernel(RoundtripArgs<MOST> a)
 {
     constexpr int kStage = 64 * Raw16<DT>::kSlots * 16;
     __shared__ __attribute__((aligned(16))) uint8_t lds[StatsTile<DT>::BYTES > kStage ? StatsTile<DT>::BYTES : kStage];
@@ -160,7 +161,7 @@ template <int DT, bool MEE> __global__ __launch_bounds__(64) void roundtrip_kern
 
     uint64_t step = a.step_dev ? *a.step_dev + a.step_more : 0;
     const float u = a.rule.u_dev ? (float)*a.rule.u_dev : a.rule.u;
-    const int at = last_at_most(a.first_tile, a.buckets, blockIdx.x);
+    const int at = MOST == 1 ? 0 : last_at_most(a.first_tile, a.buckets, blockIdx.x);
     const RoundtripBucket &b = a.bucket[at];
     const int64_t n = b.n, nsc = (n + 255) >> 8;
     const int64_t sc0 = (int64_t)(blockIdx.x - a.first_tile[at]) * kRowsPerWave;
@@ -203,9 +204,9 @@ struct TallyBucket {
     int64_t nsc;
 };
 
-struct TallyArgs {
-    uint32_t first_block[kMaxBuckets];
-    TallyBucket bucket[kMaxBuckets];
+template <int MOST> struct TallyArgs {
+    uint32_t first_block[MOST];
+    TallyBucket bucket[MOST];
     int buckets;
     WidthRule rule;
     uint32_t *hist;
@@ -281,13 +282,13 @@ template <int PER> struct PatternBatch {
     }
 };
 
-template <bool HIST> __global__ __launch_bounds__(kTallyThreads) void tally_kernel(TallyArgs a)
+template <bool HIST, int MOST> __global__ __launch_bounds__(kTallyThreads) void tally_kernel(TallyArgs<MOST> a)
 {
     __shared__ uint32_t local[HIST ? kHistWords : 1];
     __shared__ uint4 wave_seen[HIST ? kTallyThreads / 64 : 1];
     __shared__ uint32_t total[2];
     const int lane = threadIdx.x & 63;
-    const int at = last_at_most(a.first_block, a.buckets, blockIdx.x);
+    const int at = MOST == 1 ? 0 : last_at_most(a.first_block, a.buckets, blockIdx.x);
     const TallyBucket b = a.bucket[at];
     const int64_t begin = (int64_t)(blockIdx.x - a.first_block[at]) * kTallyBatch;
     const int64_t end = min(begin + (int64_t)kTallyBatch, b.nsc);
@@ -346,19 +347,33 @@ constexpr int kStatsWaves = 8; // ranks in flight per workgroup of ranks_stats_k
 // other ranks, asks for nothing meanwhile.  So it has the next tile of its rank on the way while it adds up the current one,
 // and meets the others once in GROUPS tiles.  The tiles come as whole lines (a tile goes through LDS anyway).  NT: loads that
 // leave the caches to others.
-template <int DT, int GROUPS, bool NT>
-__global__ __launch_bounds__(64 * kStatsWaves, 8) void ranks_stats_kernel(RankPointers ranks, int world, int64_t n, int vec,
-                                                                         uint32_t *__restrict__ total, float *__restrict__ mean_out,
-                                                                         WorldDiv wd, TileWidths widths)
+struct StatsArgs {
+    RankPointers ranks;
+    int world, vec;
+    int64_t n;
+    uint32_t *total;
+    float *mean;
+    WorldDiv wd;
+    TileWidths widths;
+};
+
+template <int DT, int GROUPS, bool NT> __global__ __launch_bounds__(64 * kStatsWaves, 8) void ranks_stats_kernel(StatsArgs a)
 {
     extern __shared__ __attribute__((aligned(16))) uint8_t tiles[];
+    const RankPointers &ranks = a.ranks;
+    const TileWidths &widths = a.widths;
+    const WorldDiv &wd = a.wd;
+    uint32_t *__restrict__ total = a.total;
+    float *__restrict__ mean_out = a.mean;
+    const int world = a.world, vec = a.vec;
+    const int64_t n = a.n;
     const float u = widths.rule.u_dev ? (float)*widths.rule.u_dev : widths.rule.u;
     constexpr int kRows = GROUPS * kRowsPerWave;
     __shared__ uint32_t pairs[kMaxRanks][kRows];
     typedef StatsTile<DT> ST;
     typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
     constexpr int kSlots = Raw16<DT>::kSlots, kRowBytes = 256 * ST::ESZ;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = min(world, kStatsWaves);
     const int row = lane >> 4, j = lane & 15;
     const int64_t nsc = (n + 255) >> 8;
     const int64_t sc0 = (int64_t)blockIdx.x * kRows;
@@ -748,17 +763,17 @@ WidthRule make_rule(float u, const double *u_dev)
 
 } // namespace
 
-// count <= kMaxBuckets
-hipError_t launch_roundtrip(const RoundtripDesc *desc, int count, int world, float u, const double *u_dev, uint64_t seed,
+template <int MOST>
+static hipError_t run_roundtrip(const RoundtripDesc *desc, int count, int world, float u, const double *u_dev, uint64_t seed,
                             uint64_t *step_dev, uint64_t step_more, uint32_t *hist, int dtype, bool mee, const MeeParams *mp,
                             hipStream_t stream)
 {
-    RoundtripArgs a;
-    TallyArgs t;
+    RoundtripArgs<MOST> a;
+    TallyArgs<MOST> t;
     memset(&t, 0, sizeof(t));
-    memset(&a, 0, offsetof(RoundtripArgs, rule));
+    memset(&a, 0, offsetof(RoundtripArgs<MOST>, rule));
     uint32_t tiles = 0, blocks = 0;
-    for (int k = 0; k < kMaxBuckets; k++) {
+    for (int k = 0; k < MOST; k++) {
         if (k >= count) break;
         const RoundtripDesc &d = desc[k];
         const int64_t nsc = (d.n + 255) / 256;
@@ -780,18 +795,25 @@ hipError_t launch_roundtrip(const RoundtripDesc *desc, int count, int world, flo
     t.hist = hist;
     t.step_dev = step_dev;
     t.step_more = step_more;
-    if (dtype == DQ_BF16) {
-        if (mee) hipLaunchKernelGGL((roundtrip_kernel<DQ_BF16, true>), dim3(tiles), dim3(64), 0, stream, a);
-        else hipLaunchKernelGGL((roundtrip_kernel<DQ_BF16, false>), dim3(tiles), dim3(64), 0, stream, a);
-    } else {
-        if (mee) hipLaunchKernelGGL((roundtrip_kernel<DQ_F32, true>), dim3(tiles), dim3(64), 0, stream, a);
-        else hipLaunchKernelGGL((roundtrip_kernel<DQ_F32, false>), dim3(tiles), dim3(64), 0, stream, a);
-    }
-    const hipError_t e = hipGetLastError();
+    hipError_t e;
+    if (dtype == DQ_BF16)
+        e = mee ? launch_with(roundtrip_kernel<DQ_BF16, true, MOST>, dim3(tiles), dim3(64), stream, a)
+                : launch_with(roundtrip_kernel<DQ_BF16, false, MOST>, dim3(tiles), dim3(64), stream, a);
+    else
+        e = mee ? launch_with(roundtrip_kernel<DQ_F32, true, MOST>, dim3(tiles), dim3(64), stream, a)
+                : launch_with(roundtrip_kernel<DQ_F32, false, MOST>, dim3(tiles), dim3(64), stream, a);
     if (e != hipSuccess) return e;
-    if (hist) hipLaunchKernelGGL(tally_kernel<true>, dim3(blocks), dim3(kTallyThreads), 0, stream, t);
-    else hipLaunchKernelGGL(tally_kernel<false>, dim3(blocks), dim3(kTallyThreads), 0, stream, t);
-    return hipGetLastError();
+    return hist ? launch_with(tally_kernel<true, MOST>, dim3(blocks), dim3(kTallyThreads), stream, t)
+                : launch_with(tally_kernel<false, MOST>, dim3(blocks), dim3(kTallyThreads), stream, t);
+}
+
+// count <= kMaxBuckets
+hipError_t launch_roundtrip(const RoundtripDesc *desc, int count, int world, float u, const double *u_dev, uint64_t seed,
+                            uint64_t *step_dev, uint64_t step_more, uint32_t *hist, int dtype, bool mee, const MeeParams *mp,
+                            hipStream_t stream)
+{
+    const auto run = count == 1 ? run_roundtrip<1> : (count <= 12 ? run_roundtrip<12> : run_roundtrip<kMaxBuckets>);
+    return run(desc, count, world, u, u_dev, seed, step_dev, step_more, hist, dtype, mee, mp, stream);
 }
 
 // ranks_stats_kernel, us, a tile per wave -> four -> eight (-> eight that pass the caches by): 2 ranks x 6,400 tiles 7.0 -> 6.8 -> 8.3
@@ -821,23 +843,20 @@ hipError_t launch_ranks_stats(const void *const *src, int world, int64_t n, void
     const int64_t nsc = (n + 255) / 256;
     const int64_t tiles = (nsc + kRowsPerWave - 1) / kRowsPerWave;
     const int waves = world < kStatsWaves ? world : kStatsWaves;
-    const WorldDiv wd = make_world_div(world, dtype == DQ_F32 ? 4 : 2);
-    uint32_t *tot = static_cast<uint32_t *>(total);
-    const TileWidths widths{tile_widths, tile_widths ? make_rule(u, u_dev) : WidthRule{0.0f, nullptr, {-1, -1}}};
+    const StatsArgs args{p, world, vec, n, static_cast<uint32_t *>(total), mean, make_world_div(world, dtype == DQ_F32 ? 4 : 2),
+                         TileWidths{tile_widths, tile_widths ? make_rule(u, u_dev) : WidthRule{0.0f, nullptr, {-1, -1}}}};
     const auto run = [&](auto type, auto groups, auto nt) {
         constexpr int DT = decltype(type)::value, G = decltype(groups)::value;
-        hipLaunchKernelGGL((ranks_stats_kernel<DT, G, decltype(nt)::value>), dim3((unsigned)((tiles + G - 1) / G)), dim3(64 * waves),
-                           waves * StatsTile<DT>::BYTES, stream, p, world, n, vec, tot, mean, wd, widths);
+        return launch_with(ranks_stats_kernel<DT, G, decltype(nt)::value>, dim3((unsigned)((tiles + G - 1) / G)), dim3(64 * waves), stream,
+                           args, waves * StatsTile<DT>::BYTES);
     };
     const auto launch = [&](auto type) {
-        if (!vec) run(type, std::integral_constant<int, 1>(), std::false_type());
-        else if (tiles * world * StatsTile<decltype(type)::value>::ESZ * 1024 > kStatsCache) run(type, std::integral_constant<int, 8>(), std::true_type());
-        else if (tiles * world > kStatsOneTile) run(type, std::integral_constant<int, 4>(), std::false_type());
-        else run(type, std::integral_constant<int, 1>(), std::false_type());
+        if (!vec) return run(type, std::integral_constant<int, 1>(), std::false_type());
+        if (tiles * world * StatsTile<decltype(type)::value>::ESZ * 1024 > kStatsCache) return run(type, std::integral_constant<int, 8>(), std::true_type());
+        if (tiles * world > kStatsOneTile) return run(type, std::integral_constant<int, 4>(), std::false_type());
+        return run(type, std::integral_constant<int, 1>(), std::false_type());
     };
-    if (dtype == DQ_BF16) launch(std::integral_constant<int, DQ_BF16>());
-    else launch(std::integral_constant<int, DQ_F32>());
-    return hipGetLastError();
+    return dtype == DQ_BF16 ? launch(std::integral_constant<int, DQ_BF16>()) : launch(std::integral_constant<int, DQ_F32>());
 }
 
 template <int DT, int RDT>
@@ -876,22 +895,19 @@ static hipError_t run_ring(const RingDesc &d, bool mee, const MeeParams *mp, hip
         if (d.tile_widths) {
             a.more = FromTileWidths{d.tile_widths, d.work, make_rule(d.u, d.u_dev)};
             const dim3 grid((unsigned)((a.nsc + kQuadWaves - 1) / kQuadWaves));
-            if (mee) hipLaunchKernelGGL((ring_quad_kernel<DT, RDT, true, true>), grid, block, 0, stream, a);
-            else hipLaunchKernelGGL((ring_quad_kernel<DT, RDT, false, true>), grid, block, 0, stream, a);
-            return hipGetLastError();
+            return mee ? launch_with(ring_quad_kernel<DT, RDT, true, true>, grid, block, stream, a)
+                       : launch_with(ring_quad_kernel<DT, RDT, false, true>, grid, block, stream, a);
         }
     }
     if (a_wave_each(a.nsc, d.world, DT == DQ_F32 ? 4 : 2, mee, POOL)) {
         const dim3 grid((unsigned)((a.nsc + kQuadWaves - 1) / kQuadWaves));
-        if (mee) hipLaunchKernelGGL((ring_quad_kernel<DT, RDT, true>), grid, block, 0, stream, a);
-        else hipLaunchKernelGGL((ring_quad_kernel<DT, RDT, false>), grid, block, 0, stream, a);
-        return hipGetLastError();
+        return mee ? launch_with(ring_quad_kernel<DT, RDT, true>, grid, block, stream, a)
+                   : launch_with(ring_quad_kernel<DT, RDT, false>, grid, block, stream, a);
     }
     // every run rounds its superchunks per ring chunk up to whole tiles
     const dim3 grid((unsigned)(a.nsc / (kRowsPerWave * d.world) + 4), (unsigned)d.world);
-    if (mee) hipLaunchKernelGGL((ring_kernel<DT, RDT, true>), grid, dim3(64), 0, stream, a);
-    else hipLaunchKernelGGL((ring_kernel<DT, RDT, false>), grid, dim3(64), 0, stream, a);
-    return hipGetLastError();
+    return mee ? launch_with(ring_kernel<DT, RDT, true>, grid, dim3(64), stream, a)
+               : launch_with(ring_kernel<DT, RDT, false>, grid, dim3(64), stream, a);
 }
 
 bool ring_plans_itself(int64_t n)
