@@ -414,8 +414,7 @@ struct Ranks {
     bool across = false; // an output lies across a vector at another address
     dq_ranks_t r;
 
-    Ranks(Args &a, py::sequence vecs, py::sequence outs, int64_t n, py::handle total, py::handle mean, py::handle order,
-          py::handle work, int strategy)
+    Ranks(Args &a, py::sequence vecs, py::sequence outs, int64_t n, int strategy)
     {
         memset(&r, 0, sizeof(r));
         const size_t world = py::len(vecs);
@@ -438,14 +437,19 @@ struct Ranks {
         }
         for (const Span &w : writes)
             for (const Span &x : reads) across = across || w.across(x);
-        const int64_t nsc = (n + 255) / 256;
         r.src = src.data();
         r.out = out.data();
         r.n = n;
         r.world = (int)world;
         r.strategy = strategy;
+    }
+    Ranks(Args &a, py::sequence vecs, py::sequence outs, int64_t n, py::handle total, py::handle mean, py::handle order,
+          py::handle work, int strategy)
+        : Ranks(a, vecs, outs, n, strategy)
+    {
+        const int64_t nsc = (n + 255) / 256;
         r.total = a.typed(total, at::kBFloat16, 2 * nsc, "total").data_ptr();
-        r.mean = a.typed(mean, at::kFloat, (int64_t)world * nsc, "mean").data_ptr<float>();
+        r.mean = a.typed(mean, at::kFloat, (int64_t)r.world * nsc, "mean").data_ptr<float>();
         r.order = a.typed(order, at::kInt, 3 * nsc, "order").data_ptr<int32_t>();
         const at::Tensor &w = a.typed(work, at::kInt, 4, "work");
         r.work = w.data_ptr<int32_t>();
@@ -647,30 +651,21 @@ struct Codec {
 
 // ---- ranks with random pools --------------------------------------------------------------------------------
 
-// One bucket of the fixed-proportion (sorted_plan) or dynamic all-reduce with compressor objects: codecs holds one list per
-// width (8, 4, 2 bits), group sizes counts.  Walks every codec's LCG as the ring's calls on its non-empty chunks would, in
-// the order of the widths, the steps and the ranks: rank r works on chunk (r - step) mod world in that step.  False: an output
-// lies across a vector, nothing done.
-bool ranks_pooled(py::sequence vecs, py::sequence outs, int64_t n, py::handle total, py::handle mean, py::handle order,
-                  py::handle work, py::sequence codecs, py::sequence counts, int stages, int strategy)
+void enqueue_pooled(Args &a, Ranks &k, at::ScalarType dtype, const py::sequence &codecs, const int64_t (&size)[3], int stages)
 {
-    Args a;
-    Ranks k(a, vecs, outs, n, total, mean, order, work, strategy);
-    if (k.across) return false;
     const int world = k.r.world;
-    const at::ScalarType dtype = THPVariable_Unpack(py::object(vecs[0]).ptr()).scalar_type();
     std::vector<const void *> pool(3 * world, nullptr);
     std::vector<int32_t> first(3 * world * world, 0);
-    int64_t size[3];
-    for (int g = 0; g < 3; g++) size[g] = py::cast<int64_t>(counts[g]);
     for (int g = 0; g < 3; g++) {
         if (size[g] == 0) continue;
         const py::sequence of_width = codecs[g];
+        std::vector<Codec *> codec;
+        for (int r = 0; r < world; r++) codec.push_back(&py::cast<Codec &>(of_width[r]));
         const int64_t per = (size[g] + world - 1) / world;
         // step by step, as the ring's calls go: ranks may share a compressor
         for (int step = 0; step < world; step++) {
             for (int r = 0; r < world; r++) {
-                Codec &c = py::cast<Codec &>(of_width[r]);
+                Codec &c = *codec[r];
                 const at::Tensor &p = c.pool(dtype);
                 need(p.is_cuda() && p.is_contiguous() && p.device().index() == a.device, "rand_pool must be a contiguous tensor on the vectors' device");
                 pool[g * world + r] = p.data_ptr();
@@ -690,7 +685,43 @@ bool ranks_pooled(py::sequence vecs, py::sequence outs, int64_t n, py::handle to
     k.r.top_count = size[0];
     k.r.bottom_count = size[2];
     k.enqueue(stages, a.device, c10::hip::getCurrentHIPStream().stream());
+}
+
+// One bucket of the fixed-proportion (sorted_plan) or dynamic all-reduce with compressor objects: codecs holds one list per
+// width (8, 4, 2 bits), group sizes counts.  Walks every codec's LCG as the ring's calls on its non-empty chunks would, in
+// the order of the widths, the steps and the ranks: rank r works on chunk (r - step) mod world in that step.  False: an output
+// lies across a vector, nothing done.
+bool ranks_pooled(py::sequence vecs, py::sequence outs, int64_t n, py::handle total, py::handle mean, py::handle order,
+                  py::handle work, py::sequence codecs, py::sequence counts, int stages, int strategy)
+{
+    Args a;
+    Ranks k(a, vecs, outs, n, total, mean, order, work, strategy);
+    if (k.across) return false;
+    const int64_t size[3] = {py::cast<int64_t>(counts[0]), py::cast<int64_t>(counts[1]), py::cast<int64_t>(counts[2])};
+    enqueue_pooled(a, k, THPVariable_Unpack(py::object(vecs[0]).ptr()).scalar_type(), codecs, size, stages);
     return true;
+}
+
+// fixed_proportion_allreduce_grouped with compressors of the package: (reduced statistics, row lists), or None where an output lies across
+// a vector and nothing was done.  One block of scratch: row lists, means, plan.
+py::object ranks_fixed(py::sequence vecs, py::sequence outs, int64_t n, py::sequence codecs, int64_t top, int64_t middle, int64_t bottom,
+                       int strategy)
+{
+    Args a;
+    Ranks k(a, vecs, outs, n, strategy);
+    if (k.across) return py::none();
+    const int64_t nsc = (n + 255) / 256, world = k.r.world, plan = dq_group_plan_sorted_work_ints(nsc);
+    const at::Tensor total = at::empty({nsc, 2}, at::TensorOptions().dtype(at::kBFloat16).device(at::kCUDA, (c10::DeviceIndex)a.device));
+    const at::Tensor ints = at::empty({3 * nsc + world * nsc + plan}, at::TensorOptions().dtype(at::kInt).device(at::kCUDA, (c10::DeviceIndex)a.device));
+    k.r.total = total.data_ptr();
+    k.r.order = ints.data_ptr<int32_t>();
+    k.r.mean = reinterpret_cast<float *>(k.r.order + 3 * nsc);
+    k.r.work = k.r.order + 3 * nsc + world * nsc;
+    k.r.work_ints = plan;
+    const int64_t size[3] = {top, middle, bottom};
+    enqueue_pooled(a, k, THPVariable_Unpack(py::object(vecs[0]).ptr()).scalar_type(), codecs, size, DQ_RANKS_STATS | DQ_RANKS_PLAN | DQ_RANKS_RING);
+    return py::make_tuple(py::reinterpret_steal<py::object>(THPVariable_Wrap(total)),
+                          py::reinterpret_steal<py::object>(THPVariable_Wrap(ints.narrow(0, 0, 3 * nsc))));
 }
 
 // ---- EDEN and THC (eden.py, thc.py) --------------------------------------------------------------------------
@@ -1057,6 +1088,7 @@ PYBIND11_MODULE(_host, m)
         .def("decompress", &Codec::decompress)
         .def("dec_comp", &Codec::dec_comp);
     m.def("ranks_pooled", &ranks_pooled);
+    m.def("ranks_fixed", &ranks_fixed);
     m.def("eden_compress", &eden_compress);
     m.def("eden_decompress", &eden_decompress);
     m.def("thc_compress", &thc_compress);

@@ -67,7 +67,7 @@ def dynamic_bitrate_allreduce(rank_vecs, u, compressors, out=None):
     return outs, total, qbits
 
 
-_RANKS_STATS, _RANKS_PLAN, _RANKS_RING = 1, 2, 4
+_RANKS_STATS, _RANKS_RING = 1, 4
 
 
 def _across(out, x):
@@ -84,13 +84,22 @@ def _pooled_codecs(rank_vecs, compressors):
     W = len(rank_vecs)
     if W > capi.ranks_max(True) or rank_vecs[0].dtype != torch.bfloat16:
         return None
-    every = [c for q in (8, 4, 2) for c in compressors.get(q, ())]
-    if not all(type(c) in (Aee_Dynamic_Range_GPU_kern, Mee_Dynamic_Range_GPU_kern) and c.philox_seed is None and c.chunk_size == 16 and
-               c.strategy == every[0].strategy and not c._picks_rows for c in every):
-        return None
-    if any(len(compressors.get(q, ())) < W or any(c.nbits != q for c in compressors[q]) for q in (8, 4, 2)):
-        return None
-    return [[c._codec for c in compressors[q]] for q in (8, 4, 2)]
+    native, strategy = [], None
+    for q in (8, 4, 2):
+        of_width = compressors.get(q, ())
+        if len(of_width) < W:
+            return None
+        native.append([])
+        for c in of_width:
+            if type(c) is not Aee_Dynamic_Range_GPU_kern and type(c) is not Mee_Dynamic_Range_GPU_kern:
+                return None
+            codec = c._codec
+            if strategy is None:
+                strategy = c.strategy
+            if codec.philox or c._picks_rows or c.chunk_size != 16 or c.nbits != q or c.strategy != strategy:
+                return None
+            native[-1].append(codec)
+    return native
 
 
 def dynamic_bitrate_allreduce_grouped(rank_vecs, u, compressors, out=None, work=None, device_qbits=False):
@@ -213,7 +222,6 @@ def fixed_proportion_allreduce_grouped(rank_vecs, thresholds, compressors, out=N
     the whole ring (else the row-list codec calls); the group sizes follow from the fractions on the host, so nothing is
     read back."""
     from . import capi
-    eu = load_eden_utils()
     W = len(rank_vecs)
     n = rank_vecs[0].numel()
     nsc = (n + SUPERCHUNK - 1) // SUPERCHUNK
@@ -223,15 +231,10 @@ def fixed_proportion_allreduce_grouped(rank_vecs, thresholds, compressors, out=N
     if codecs and not (fixed_4bit_only and counts[1] != nsc):
         # three launches for all ranks, steps and widths: statistics, sorted plan, ring
         outs = out if out is not None else [torch.empty(n, dtype=dt, device=dev) for _ in range(W)]
-        total = torch.empty((nsc, 2), dtype=torch.bfloat16, device=dev)
-        # one block of scratch: row lists (they are returned), plan, means
-        plan_ints = capi.group_plan_sorted_work_ints(nsc)
-        ints = torch.empty(3 * nsc + W * nsc + plan_ints, dtype=torch.int32, device=dev)
-        order = ints[:3 * nsc]
-        if capi.host().ranks_pooled(rank_vecs, outs, n, total, ints[3 * nsc:3 * nsc + W * nsc].view(torch.float32), order,
-                                    ints[3 * nsc + W * nsc:], codecs, counts, _RANKS_STATS | _RANKS_PLAN | _RANKS_RING,
-                                    compressors[8][0].strategy):
-            return outs, total, order, counts
+        done = capi.host().ranks_fixed(rank_vecs, outs, n, codecs, *counts, compressors[8][0].strategy)
+        if done is not None:
+            return outs, done[0], done[1], counts
+    eu = load_eden_utils()
     residuals = [torch.empty(nsc * SUPERCHUNK, dtype=dt, device=dev) for _ in range(W)]
     stats = [torch.empty((nsc, 2), dtype=torch.bfloat16, device=dev) for _ in range(W)]
     for r in range(W):
