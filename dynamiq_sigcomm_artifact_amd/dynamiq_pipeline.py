@@ -268,9 +268,9 @@ def dynamic_bitrate_allreduce_single_pass(rank_vecs, u, strategy=2, seed=0, out=
                                           norm_histogram=None):
     """The same all-reduce with every stage kept on the device and without packed streams: the records of a ring step
     between ranks that share this GPU's memory are read by the next step only, so a superchunk goes through the whole
-    ring in registers (csrc/dq_single_pass.hip).  Three launches per bucket (statistics of all ranks, plan, ring) -- two
-    with one rank, where nothing depends on another superchunk -- whatever the number of ranks; nothing is read back, and
-    the launches can be captured once and replayed as a graph.
+    ring in registers (csrc/dq_single_pass.hip).  Three launches per bucket (statistics of all ranks, plan, ring) -- two on
+    short vectors, whose ring plans itself, and with one rank, where nothing depends on another superchunk -- whatever
+    the number of ranks; nothing is read back, and the launches can be captured once and replayed as a graph.
 
     The bit widths follow the device rule of group_plan_stats; the rounding randomness is the in-kernel stream keyed by
     (seed + rank, ring step, index of the chunk in the vector), so results are reproducible but not those of
