@@ -232,7 +232,7 @@ __device__ __forceinline__ void compress_tile(const void *__restrict__ src, cons
     WinRegs wr;
     if (FUSED) wr = window_fetch(recv + sc0 * RC::REC, total, lane);
     TableRegs<NBITS> tr;
-    if (MEE && FUSED) tr = table_fetch<NBITS>(lane);
+    if (MEE && FUSED) tr = table_fetch<NBITS>(mp, lane);
     Raw16<DT> v;
     Raw16<RDT> r;
     v.zero();
@@ -313,7 +313,7 @@ __device__ __forceinline__ void decompress_tile(const uint8_t *__restrict__ src,
     uint32_t mean_bits = 0; // widened where it is used, so that nothing waits for this load here
     if (stats && active) mean_bits = stats[2 * d_own];
     TableRegs<NBITS> tr;
-    if (MEE) tr = table_fetch<NBITS>(lane);
+    if (MEE) tr = table_fetch<NBITS>(mp, lane);
 
     const int mis_in = window_commit(win_in, wr, src + sc0 * RC::REC, total, lane);
     if (MEE) table_commit<NBITS>(table, tr, lane);

@@ -283,7 +283,7 @@ __global__ void irht_decompress_tile_kernel(const uint8_t *__restrict__ src, flo
     uint8_t *win_in = windows + wave * RC::WIN;
     float *table = reinterpret_cast<float *>(windows + nwaves * RC::WIN);
     if (MEE) {
-        for (int k = tid; k < (1 << NBITS); k += nthreads) table[k] = f16_bits_to_f32(kMeeLevels<NBITS>.at[k]);
+        for (int k = tid; k < (1 << NBITS); k += nthreads) table[k] = f16_bits_to_f32(mp.levels()[k]);
         __syncthreads();
     }
 
@@ -1294,7 +1294,7 @@ __global__ __launch_bounds__(1 << (HB - 4), 8) void irht_decompress_kernel(const
 #pragma unroll
     for (int h = 0; h < kParts; h++) wr[h] = window_fetch(records(h), kTotal, lane);
     if (MEE) {
-        for (int k = tid; k < (1 << NBITS); k += kThreads) table[k] = f16_bits_to_f32(kMeeLevels<NBITS>.at[k]);
+        for (int k = tid; k < (1 << NBITS); k += kThreads) table[k] = f16_bits_to_f32(mp.levels()[k]);
         __syncthreads();
     }
     float v[kParts][16];

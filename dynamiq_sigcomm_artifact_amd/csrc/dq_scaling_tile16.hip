@@ -289,7 +289,7 @@ __device__ __forceinline__ void tile16_decompress(const uint8_t *__restrict__ sr
     Raw16<DT> acc;
     if (ADD && active) acc.load(dst, e0 + lane * 16, vec);
     TableRegs<NBITS> tr;
-    if (MEE) tr = table_fetch<NBITS>(lane);
+    if (MEE) tr = table_fetch<NBITS>(mp, lane);
     const int mis_in = window_commit(win_in, wr, gin, total, lane);
     if (MEE) table_commit<NBITS>(table, tr, lane);
     wave_lds_sync();

@@ -22,7 +22,21 @@ template <int NBITS> struct Rec {
     static constexpr int WIN_VECS = WIN / 16;  // <= 70: at most two 128-bit registers per lane
 };
 
-template <int NBITS, bool MEE> struct MeeArg {
+// The level table of up to 3 bits comes along; the longer ones are read where they lie (dq_mee_levels.cuh), which costs every wave's
+// loads a page of their own (a seven-rank ring of 44,954,112 elements at 2 bits 90.1 us, 88.4 with the table among the arguments) but
+// keeps the arguments within 128 bytes: beyond, a launch takes 0.8 us longer (65,536 elements at 8 bits, three launches, 9.7 -> 11.7 us
+// with 4 bytes too many, at 4 bits 11.3 with the table).
+template <int NBITS, bool ALONG = (NBITS <= 3)> struct MeeTable {
+    static constexpr bool kAlong = true;
+    alignas(4) uint16_t table[1 << NBITS];
+    __device__ __forceinline__ const uint16_t *levels() const { return table; }
+};
+template <int NBITS> struct MeeTable<NBITS, false> {
+    static constexpr bool kAlong = false;
+    __device__ __forceinline__ const uint16_t *levels() const { return kMeeLevels<NBITS>.at; }
+};
+
+template <int NBITS, bool MEE> struct MeeArg : MeeTable<NBITS> {
     float c, cmm, l2b;
     uint32_t pad;
     double inv_c, inv_cmm, inv_l2b; // correctly rounded double reciprocals
@@ -32,6 +46,7 @@ template <int NBITS, bool MEE> struct MeeArg {
 template <int NBITS> struct MeeArg<NBITS, false> {
     static constexpr float c = 1.0f, cmm = 1.0f, l2b = 1.0f;
     static constexpr double inv_c = 1.0, inv_cmm = 1.0, inv_l2b = 1.0;
+    __device__ __forceinline__ const uint16_t *levels() const { return nullptr; }
 };
 
 typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
@@ -227,7 +242,7 @@ template <class RR> struct DrawnBytes { static constexpr bool value = std::is_sa
 
 // ---- the MEE level table on its way into LDS -------------------------------------------------------
 //
-// 2^NBITS binary16 patterns (kMeeLevels).  A lane fetches its pairs of entries with the
+// 2^NBITS binary16 patterns.  A lane fetches its pairs of entries with the
 // other loads of its tile (one or two 4-byte loads, no wait in between) and converts and stores them as floats once the
 // tile's own data has arrived.
 template <int NBITS> struct TableRegs {
@@ -236,10 +251,10 @@ template <int NBITS> struct TableRegs {
     uint32_t pair[kPerLane];
 };
 
-template <int NBITS> __device__ __forceinline__ TableRegs<NBITS> table_fetch(int lane)
+template <int NBITS, class ARG> __device__ __forceinline__ TableRegs<NBITS> table_fetch(const ARG &mp, int lane)
 {
     TableRegs<NBITS> t;
-    const uint32_t *pairs = reinterpret_cast<const uint32_t *>(kMeeLevels<NBITS>.at);
+    const uint32_t *pairs = reinterpret_cast<const uint32_t *>(mp.levels());
 #pragma unroll
     for (int j = 0; j < TableRegs<NBITS>::kPerLane; j++) {
         const int k = lane + 64 * j;
@@ -552,6 +567,9 @@ template <int NBITS, bool MEE> static MeeArg<NBITS, MEE> make_arg(const MeeParam
     MeeArg<NBITS, MEE> a;
     if constexpr (MEE) {
         a.c = mp.c; a.cmm = mp.cmm; a.l2b = mp.l2b; a.pad = 0;
+        if constexpr (MeeTable<NBITS>::kAlong) {
+            for (int k = 0; k < (1 << NBITS); k++) a.table[k] = mp.table[k];
+        }
         a.inv_c = 1.0 / (double)mp.c; a.inv_cmm = 1.0 / (double)mp.cmm; a.inv_l2b = 1.0 / (double)mp.l2b;
     }
     return a;
