@@ -1090,44 +1090,165 @@ struct LastEnds : OutEnds {
     ThcGrid grid;
 };
 
-template <bool ENDS> struct FirstPass {
+// The same as kernel arguments.  Beyond 128 bytes of them a launch takes 0.7 us longer (MeeTable of dq_tile16.cuh), and as they stand the
+// arguments, ends and grid are 176 and 224: what excludes one another shares a place, and small numbers take a byte.
+enum { kNoEnd, kOther, kLevelsEnd, kPlanesEnd };
+
+struct FirstPass {
     float *x;
+    const void *sign, *in, *p; // the source, levels or planes; with levels the step or the norm, with planes the centroids
+    const float *in_lo;
+    int64_t n, in_count;
+    float scale, grid[7]; // lo, spacing, step, t, inv_sqrt, inv_levels, inv_clients
+    uint32_t gen_ss;
+    uint8_t kt, kb, vec, sign_bits, sign_mode, gen_bits, end, in_dtype, in_nbits, grid_kind;
+};
+static_assert(sizeof(FirstPass) <= 128, "see above");
+
+struct StridedPass {
+    float *x;
+    const void *sign;
+    void *out;                  // the destination or levels
+    const void *p;              // with levels the uniform values, else the scale of the last pass
+    const void *q, *r;          // with levels its grid: lowest level or norm, spacing; else the sums
+    int64_t n, count;           // with levels zeros_from, else out_count
+    uint64_t draw_seed, draw_counter;
+    float scale, out_top, grid[3]; // lo, spacing; or t, inv_sqrt, inv_levels
+    uint32_t gen_ss;
+    uint8_t rbits, sbits, sign_mode, apply_scale, end, out_dtype, gen_bits, vec, sign_bits, kt, grid_kind;
+    int8_t draw_bits;
+};
+static_assert(sizeof(StridedPass) <= 128, "see above");
+
+template <bool ENDS> __device__ __forceinline__ PassArgs<ENDS> pass_args(const FirstPass &p)
+{
     PassArgs<ENDS> a;
-    int sign_mode;
+    a.sign = p.sign; a.sign_bits = p.sign_bits; a.n = p.n; a.kt = p.kt; a.kb = p.kb; a.scale = p.scale; a.vec = p.vec;
+    if constexpr (ENDS) {
+        a.gen.bits = p.gen_bits;
+        a.gen.ss = p.gen_ss;
+    }
+    return a;
+}
+
+template <bool ENDS> __device__ __forceinline__ PassArgs<ENDS> pass_args(const StridedPass &p)
+{
+    PassArgs<ENDS> a;
+    a.sign = p.sign; a.sign_bits = p.sign_bits; a.n = p.n; a.kt = p.kt; a.kb = 0; a.scale = p.scale; a.vec = p.vec;
+    if constexpr (ENDS) {
+        a.gen.bits = p.gen_bits;
+        a.gen.ss = p.gen_ss;
+    }
+    return a;
+}
+
+__device__ __forceinline__ FirstEnds ends_of(const FirstPass &p)
+{
     FirstEnds e;
-};
+    const bool levels = p.end == kLevelsEnd, planes = p.end == kPlanesEnd;
+    e.in_src = p.end == kOther ? p.in : nullptr;
+    e.in_dtype = p.in_dtype;
+    e.in_count = p.in_count;
+    e.in_levels = levels ? static_cast<const uint16_t *>(p.in) : nullptr;
+    e.in_step = e.grid.norm = static_cast<const float *>(p.p);
+    e.in_lo = p.in_lo;
+    e.in_planes = planes ? static_cast<const uint32_t *>(p.in) : nullptr;
+    e.in_centroids = static_cast<const float *>(p.p);
+    e.in_nbits = p.in_nbits;
+    e.grid.kind = p.grid_kind;
+    e.grid.lo = p.grid[0]; e.grid.spacing = p.grid[1]; e.grid.step = p.grid[2];
+    e.grid.t = p.grid[3]; e.grid.inv_sqrt = p.grid[4]; e.grid.inv_levels = p.grid[5]; e.grid.inv_clients = p.grid[6];
+    return e;
+}
 
-template <bool ENDS> struct StridedPass {
-    float *x;
-    PassArgs<ENDS> a;
-    int rbits, sbits, sign_mode, apply_scale;
+__device__ __forceinline__ LastEnds ends_of(const StridedPass &p)
+{
     LastEnds e;
-};
+    const bool levels = p.end == kLevelsEnd;
+    e.zeros_from = levels ? p.count : -1;
+    e.out_dst = p.end == kOther ? p.out : nullptr;
+    e.out_dtype = p.out_dtype;
+    e.out_count = p.count;
+    e.out_levels = levels ? static_cast<uint16_t *>(p.out) : nullptr;
+    e.uniform = static_cast<const float *>(p.p);
+    e.out_lo = e.grid.norm = static_cast<const float *>(p.q);
+    e.out_delta = static_cast<const float *>(p.r);
+    e.out_top = p.out_top;
+    e.draw.bits = p.draw_bits; e.draw.seed = p.draw_seed; e.draw.counter = p.draw_counter;
+    e.post_scale = levels ? nullptr : static_cast<const float *>(p.p);
+    e.sums = levels ? nullptr : const_cast<double *>(static_cast<const double *>(p.q));
+    e.grid.kind = p.grid_kind;
+    e.grid.lo = e.grid.t = p.grid[0];
+    e.grid.spacing = e.grid.inv_sqrt = p.grid[1];
+    e.grid.inv_levels = p.grid[2];
+    return e;
+}
 
-template <bool ENDS> __global__ __launch_bounds__(512) void rht_strided_kernel(StridedPass<ENDS> p)
+inline FirstPass first_of(float *x, const RhtPassArgs &a, int sign_mode, const TransformEnds &e)
+{
+    FirstPass p;
+    const bool norm = e.grid.kind == ThcGrid::NORM;
+    p.x = x; p.sign = a.sign; p.n = a.n; p.scale = a.scale;
+    p.kt = (uint8_t)a.kt; p.kb = (uint8_t)a.kb; p.vec = (uint8_t)a.vec; p.sign_bits = (uint8_t)a.sign_bits; p.sign_mode = (uint8_t)sign_mode;
+    p.gen_bits = (uint8_t)a.gen.bits; p.gen_ss = a.gen.ss;
+    p.end = e.in_levels ? kLevelsEnd : (e.in_planes ? kPlanesEnd : (e.in_src ? kOther : kNoEnd));
+    p.in = e.in_levels ? (const void *)e.in_levels : (e.in_planes ? (const void *)e.in_planes : e.in_src);
+    p.p = e.in_planes ? e.in_centroids : (norm ? e.grid.norm : e.in_step);
+    p.in_lo = e.in_lo; p.in_count = e.in_count;
+    p.in_dtype = (uint8_t)e.in_dtype; p.in_nbits = (uint8_t)e.in_nbits;
+    p.grid_kind = (uint8_t)e.grid.kind;
+    const float grid[7] = {e.grid.lo, e.grid.spacing, e.grid.step, e.grid.t, e.grid.inv_sqrt, e.grid.inv_levels, e.grid.inv_clients};
+    for (int k = 0; k < 7; k++) p.grid[k] = grid[k];
+    return p;
+}
+
+inline StridedPass strided_of(float *x, const RhtPassArgs &a, int rbits, int sbits, int sign_mode, int apply_scale, const TransformEnds &e)
+{
+    StridedPass p;
+    const bool norm = e.grid.kind == ThcGrid::NORM, levels = e.out_levels != nullptr;
+    p.x = x; p.sign = a.sign; p.n = a.n; p.scale = a.scale;
+    p.kt = (uint8_t)a.kt; p.vec = (uint8_t)a.vec; p.sign_bits = (uint8_t)a.sign_bits; p.sign_mode = (uint8_t)sign_mode;
+    p.rbits = (uint8_t)rbits; p.sbits = (uint8_t)sbits; p.apply_scale = (uint8_t)apply_scale;
+    p.gen_bits = (uint8_t)a.gen.bits; p.gen_ss = a.gen.ss;
+    p.end = levels ? kLevelsEnd : (e.out_dst ? kOther : kNoEnd);
+    p.out = levels ? (void *)e.out_levels : e.out_dst;
+    p.p = levels ? e.uniform : e.post_scale;
+    p.q = levels ? (const void *)(norm ? e.grid.norm : e.out_lo) : (const void *)e.sums;
+    p.r = e.out_delta;
+    p.count = levels ? e.zeros_from : e.out_count;
+    p.out_dtype = (uint8_t)e.out_dtype; p.out_top = e.out_top;
+    p.draw_bits = (int8_t)e.draw.bits; p.draw_seed = e.draw.seed; p.draw_counter = e.draw.counter;
+    p.grid_kind = (uint8_t)e.grid.kind;
+    p.grid[0] = norm ? e.grid.t : e.grid.lo;
+    p.grid[1] = norm ? e.grid.inv_sqrt : e.grid.spacing;
+    p.grid[2] = e.grid.inv_levels;
+    return p;
+}
+
+template <bool ENDS> __global__ __launch_bounds__(512) void rht_strided_kernel(StridedPass p)
 {
     extern __shared__ __attribute__((aligned(16))) float lds[];
-    strided_pass<ENDS>(p.x, p.a, p.rbits, p.sbits, p.sign_mode, p.apply_scale, p.e, blockIdx.x, lds);
+    strided_pass<ENDS>(p.x, pass_args<ENDS>(p), p.rbits, p.sbits, p.sign_mode, p.apply_scale, ends_of(p), blockIdx.x, lds);
 }
 
 // 512 (B = 4) or 1024 rows (B = 5)
-template <bool ENDS, int B> __global__ __launch_bounds__(32 << B) void rht_strided_long_kernel(StridedPass<ENDS> p)
+template <bool ENDS, int B> __global__ __launch_bounds__(32 << B) void rht_strided_long_kernel(StridedPass p)
 {
     extern __shared__ __attribute__((aligned(16))) float lds[];
-    strided_rows<ENDS, 5, B>(p.x, p.a, p.sbits, p.sign_mode, p.apply_scale, p.e, blockIdx.x, lds);
+    strided_rows<ENDS, 5, B>(p.x, pass_args<ENDS>(p), p.sbits, p.sign_mode, p.apply_scale, ends_of(p), blockIdx.x, lds);
 }
 
 // 256 (A = 4) or 1024 rows (A = 5) to THC's levels with drawn values
-template <int A> __global__ __launch_bounds__(32 << A) void rht_strided_draw_kernel(StridedPass<true> p)
+template <int A> __global__ __launch_bounds__(32 << A) void rht_strided_draw_kernel(StridedPass p)
 {
     extern __shared__ __attribute__((aligned(16))) float lds[];
-    strided_rows<true, A, A, true>(p.x, p.a, p.sbits, p.sign_mode, p.apply_scale, p.e, blockIdx.x, lds);
+    strided_rows<true, A, A, true>(p.x, pass_args<true>(p), p.sbits, p.sign_mode, p.apply_scale, ends_of(p), blockIdx.x, lds);
 }
 
-template <bool ENDS> __global__ __launch_bounds__(1024) void rht_first_kernel(FirstPass<ENDS> p)
+template <bool ENDS> __global__ __launch_bounds__(1024) void rht_first_kernel(FirstPass p)
 {
     extern __shared__ __attribute__((aligned(16))) float lds[];
-    first_pass<ENDS>(p.x, p.a, p.sign_mode, p.e, blockIdx.x, lds, tile_threads(p.a.kt));
+    first_pass<ENDS>(p.x, pass_args<ENDS>(p), p.sign_mode, ends_of(p), blockIdx.x, lds, tile_threads(p.kt));
 }
 
 #if DQ_RHT_PART & DQ_RHT_TRANSFORM
@@ -1645,13 +1766,12 @@ hipError_t launch_rht_tile(float *x, const void *sign, int sign_bits, int64_t n,
     const dim3 grid((unsigned)((n + tile - 1) >> kt));
     if (sign_mode != 2 && !apply_scale && kb == kt && kt <= 14 && vec && (n & (tile - 1)) == 0 && ends.plain_out()) {
         const int mode = diagonal ? sign_mode : 0;
-        const auto launch = [&](auto kernel, const auto &pass) -> hipError_t {
+        const FirstPass pass = first_of(x, a, mode, ends);
+        const auto launch = [&](auto kernel) -> hipError_t {
             const hipError_t e = allow_lds(kernel, lds);
             return e == hipSuccess ? launch_with(kernel, grid, dim3(threads), stream, pass, lds) : e;
         };
-        const FirstEnds e{ends, ends.grid};
-        return plain ? launch(rht_first_kernel<false>, FirstPass<false>{x, plain_args, mode, e})
-                     : launch(rht_first_kernel<true>, FirstPass<true>{x, a, mode, e});
+        return plain ? launch(rht_first_kernel<false>) : launch(rht_first_kernel<true>);
     }
     if (plain) {
         hipError_t e = allow_lds(rht_tile_kernel<false>, lds);
@@ -1676,26 +1796,23 @@ hipError_t launch_rht_strided(float *x, const void *sign, int sign_bits, int64_t
     if (draws && ((rbits != 8 && rbits != 10) || sign_mode == 2 || ends.post_scale || ends.sums)) return hipErrorInvalidValue;
     RhtPassArgs a;
     a.sign = sign; a.sign_bits = sign_bits; a.n = n; a.kt = rbits + 5; a.kb = 0; a.scale = scale; a.vec = vec; a.gen = ends.gen;
-    const RhtTileArgs &plain_args = a;
     const dim3 grid((unsigned)(n >> (rbits + 5))), block((unsigned)strided_threads(rbits));
     const size_t lds = strided_lds_bytes(rbits);
-    const int mode = sign || ends.gen.bits != 0 ? sign_mode : 0;
-    const LastEnds last{ends, ends.grid};
-    const auto launch = [&](auto kernel, const auto &pass) -> hipError_t {
+    if (ends.out_levels && (ends.out_dst || ends.post_scale || ends.sums)) return hipErrorInvalidValue; // (they share a place)
+    const StridedPass pass = strided_of(x, a, rbits, sbits, sign || ends.gen.bits != 0 ? sign_mode : 0, apply_scale, ends);
+    const auto launch = [&](auto kernel) -> hipError_t {
         const hipError_t e = allow_lds(kernel, lds);
         return e == hipSuccess ? launch_with(kernel, grid, block, stream, pass, lds) : e;
     };
     if (plain) {
-        const StridedPass<false> p{x, plain_args, rbits, sbits, mode, apply_scale, last};
-        if (rbits == 10) return launch(rht_strided_long_kernel<false, 5>, p);
-        if (rbits == 9) return launch(rht_strided_long_kernel<false, 4>, p);
-        return launch(rht_strided_kernel<false>, p);
+        if (rbits == 10) return launch(rht_strided_long_kernel<false, 5>);
+        if (rbits == 9) return launch(rht_strided_long_kernel<false, 4>);
+        return launch(rht_strided_kernel<false>);
     }
-    const StridedPass<true> p{x, a, rbits, sbits, mode, apply_scale, last};
-    if (draws) return rbits == 10 ? launch(rht_strided_draw_kernel<5>, p) : launch(rht_strided_draw_kernel<4>, p);
-    if (rbits == 10) return launch(rht_strided_long_kernel<true, 5>, p);
-    if (rbits == 9) return launch(rht_strided_long_kernel<true, 4>, p);
-    return launch(rht_strided_kernel<true>, p);
+    if (draws) return rbits == 10 ? launch(rht_strided_draw_kernel<5>) : launch(rht_strided_draw_kernel<4>);
+    if (rbits == 10) return launch(rht_strided_long_kernel<true, 5>);
+    if (rbits == 9) return launch(rht_strided_long_kernel<true, 4>);
+    return launch(rht_strided_kernel<true>);
 }
 
 // every x 16-byte aligned, n a multiple of 2^kt and 10 <= kt <= 14
