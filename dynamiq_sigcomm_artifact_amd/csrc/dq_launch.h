@@ -14,7 +14,8 @@ namespace dq {
 
 // A kernel whose only argument is `args`.  Short calls wait for the host, and the runtime copies a kernel's arguments one by one to
 // where the GPU reads them: a decoder call of eight arguments and 104 bytes takes 3.8 us, with one argument of 56 bytes 2.9 (and 576
-// bytes 1.1 us more than 64).  Eight ranks' ring of 65,792 elements, 17 calls, 68 -> 55 us of host time.
+// bytes 1.1 us more than 64).  In a stream, not in a graph, the GPU takes 0.7 us longer where they are more than 128 bytes.  The host's
+// part of an eight-rank ring of 65,792 elements, 17 calls, 68 -> 55 us.
 template <class K, class A> inline hipError_t launch_with(K *kernel, dim3 grid, dim3 block, hipStream_t stream, const A &args, size_t lds = 0)
 {
     static_assert(std::is_same<K, void(A)>::value, "the kernel takes these arguments");
@@ -208,8 +209,8 @@ struct UniformDraw {
 
 // Quantisers folded into the two ends of a transform (all null: the plain transform).  `in_*` replace the load of the
 // first pass, `out_*` / `post_scale` act on the store of the last one.
-// What a first pass looks at, and what a strided one does, are kernel arguments by themselves: 264 bytes of both in seven arguments take
-// the host and the GPU 1 us longer a launch (launch_with).
+// What a first pass looks at, and what a strided one does: a kernel gets the one or the other (FirstPass and StridedPass of
+// dq_rht_scaling_impl.cuh).
 struct InEnds {
     // the first pass loads in_count elements of in_dtype from in_src, zeros behind them, instead of x
     const void *in_src = nullptr;
