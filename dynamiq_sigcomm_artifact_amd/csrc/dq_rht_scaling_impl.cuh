@@ -627,11 +627,12 @@ template <int KT> __device__ __forceinline__ void middle_stages(float *lds, int 
         lds_pass<4, KT < 13 ? KT - 8 : 4>(lds, KT, tid, nthreads);
 }
 
-// Vectors of up to so many elements leave the first pass with the non-temporal hint: what waits in the L2 until the kernel ends, up
-// to 32 MB, is then on its way while others still load.  First pass, us, without -> with: 2^23 elements from bf16 levels 13.8 -> 9.5, from
-// a 25 MB gradient 12.8 -> 11.7, 2^20 5.9 -> 5.6 (the pass that reads them 0.5 to 1 longer); but 2^24, where the L2 is full long before the
-// end, both ways of THC 103 -> 111.5.
-constexpr int64_t kEarlyStores = (int64_t)1 << 23;
+// Vectors of so many elements leave the first pass with the non-temporal hint: what waits in the L2 until the kernel ends, up to 32 MB, is
+// then on its way while others still load.  First pass, us, without -> with: 2^23 elements from bf16 levels 13.8 -> 9.5, from a 25 MB
+// gradient 12.8 -> 11.7.  The pass that reads them takes 0.5 to 1 longer, which costs shorter ones more than they gain, and 2^24 fill the
+// L2 long before the end.  There and back, without -> with: EDEN 262,144 21.4 -> 22.2, 2^20 26.7 -> 27.0, 2^21 37.3 -> 37.2, 2^22 52.9 ->
+// 54.1, 2^23 74.5 -> 72.6; THC 4,000,000 38.0 -> 38.4, 6,553,600 50.3 -> 45.7, 2^24 103 -> 111.5.
+constexpr int64_t kEarlyFrom = ((int64_t)1 << 22) + 1, kEarlyTo = (int64_t)1 << 23;
 
 // lds_pass whose results go to memory: consecutive lanes hold consecutive elements (P >= 6)
 template <int P, int M> __device__ __forceinline__ void lds_pass_out(const float *lds, int kt, int tid, int nthreads, float *__restrict__ out, bool early)
@@ -764,7 +765,7 @@ __device__ __forceinline__ void first_pass(float *__restrict__ x, const PassArgs
     }
     __syncthreads();
     float *out = x + origin;
-    const bool early = a.n <= kEarlyStores;
+    const bool early = a.n >= kEarlyFrom && a.n <= kEarlyTo;
     switch (a.kt) {
     case 10: lds_pass_out<6, 4>(lds, 10, tid, step, out, early); break;
     case 11: lds_pass_out<7, 4>(lds, 11, tid, step, out, early); break;
