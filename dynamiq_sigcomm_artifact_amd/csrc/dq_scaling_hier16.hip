@@ -126,6 +126,7 @@ static hipError_t run_compress(const void *src, const uint8_t *recv, uint8_t *ds
 {
     const CompressArgs<MeeArg<NBITS, MEE>> args{src, recv, dst, rnd, rows, nsc, (aligned16(src) ? 1 : 0) | (aligned16(rnd) ? 2 : 0), key,
                                                 make_arg<NBITS, MEE>(mp)};
+    static_assert(sizeof(args) <= 128, "beyond, a launch takes 0.8 us longer (MeeTable)");
     const dim3 grid(grid_for(nsc)), block(64);
     if (fused) return launch_with(hier16_compress_kernel<DT, RDT, NBITS, MEE, true>, grid, block, stream, args);
     return launch_with(hier16_compress_kernel<DT, RDT, NBITS, MEE, false>, grid, block, stream, args);

@@ -1118,6 +1118,12 @@ def test_list_of_buckets_of_two_types(capi, kinds):
     assert not pipe._last[0].matches(pairs[::-1])
 
 
+@pytest.mark.parametrize("kinds", ["b" * 12, "b" * 13, "f" * 12 + "b" * 13 + "f"])
+def test_lists_on_either_side_of_a_launchs_room(capi, kinds):
+    """a launch has room for one, twelve or 32 buckets"""
+    test_list_of_buckets_of_two_types(capi, kinds)
+
+
 @pytest.mark.parametrize("shape", ["chain", "rewrite", "reuse", "overlap", "in place", "shared source", "views"])
 def test_list_of_buckets_that_share_memory(capi, shape):
     """buckets of one list that read or write what another of the list writes give the results of one bucket after the other, and
