@@ -471,9 +471,10 @@ __device__ __forceinline__ void center_loaded(float (&t)[RV::kCount], const RV &
         const int left = left_here(n, e0, N);
 #pragma unroll
         for (int i = 0; i < N; i++) {
-            // (in place: as a selection the tiles that are not ragged copy every element)
+            // (In place: as a selection the tiles that are not ragged copy every element.  The comparison that writes the mask may come
+            // directly before, and the two wait states between the two are the compiler's only for its own instructions.)
             const uint64_t inside = __builtin_amdgcn_ballot_w64(i < left);
-            asm volatile("v_cndmask_b32_e64 %0, 0, %0, %1" : "+v"(t[i]) : "s"(inside));
+            asm volatile("s_nop 1\n\tv_cndmask_b32_e64 %0, 0, %0, %1" : "+v"(t[i]) : "s"(inside));
         }
     }
 #pragma unroll

@@ -710,6 +710,26 @@ def test_ranks_in_registers_equal_the_ring_in_steps(capi, W, n, dt):
         assert all(torch.equal(bits_t(x), bits_t(y)) for x, y in zip(again, ref))
 
 
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("W,nsc", [(1, 9), (3, 9), (2, 12289)])
+def test_ragged_ends_under_a_large_mean(capi, W, nsc, dt):
+    """elements behind the vector's end are zeros to the quantiser and not zeros less the mean: one left over would set the scale of a
+    chunk and its superchunk a hundred times too large.  The one-rank pass, the rings with and without lists, against one launch per
+    rank and ring step"""
+    from dynamiq_sigcomm_artifact_amd.dynamiq_pipeline import _single_pass_in_steps, dynamic_bitrate_allreduce_single_pass
+    g = torch.Generator(device=DEV).manual_seed(nsc + W)
+    whole = [(1024.0 + 8.0 * torch.randn(nsc * 256, generator=g, device=DEV)).to(dt) for _ in range(W)]
+    for left in (1, 2, 3, 7, 15, 16, 17, 30, 130, 255) if nsc < 100 else (3, 130):
+        vecs = [v[:nsc * 256 - 256 + left].clone() for v in whole]
+        for strategy, u in ((2, 60.0), (3, 6.0), (2, -60.0)):
+            outs, _, _ = dynamic_bitrate_allreduce_single_pass(vecs, u, strategy=strategy, seed=11)
+            ref, _, _ = _single_pass_in_steps(vecs, u, strategy, 11, None, {}, None, None)
+            assert all(torch.equal(bits_t(x), bits_t(y)) for x, y in zip(outs, ref)), (left, strategy, u)
+            # 8 bits: steps of the residuals' largest, at most 50, / 127 (AEE), and the binary16-wide mean's rounding
+            if u > 50.0:
+                assert float((outs[0].float() - 1024.0).abs().max()) < 64.0, left
+
+
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("strategy", [2, 3])
 @pytest.mark.parametrize("W,nsc", [(1, 510), (2, 510), (2, 8704)])

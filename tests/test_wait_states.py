@@ -1,0 +1,106 @@
+"""The machine code of the built library keeps the wait states that gfx950 asks for between a vector instruction that writes a scalar
+register -- a comparison's mask, a readlane, a carry -- and a vector instruction that reads it: two.  The compiler sees to it for its own
+instructions, but not for those of inline assembly, whose operands may come straight from such an instruction."""
+import os
+import re
+import struct
+import subprocess
+from concurrent.futures import ThreadPoolExecutor
+
+import pytest
+
+OBJDUMP = "/opt/rocm/llvm/bin/llvm-objdump"
+BUNDLE = b"__CLANG_OFFLOAD_BUNDLE__"
+WAIT_STATES = 2
+
+SCALAR = re.compile(r"\bs(\d+)\b|\bs\[(\d+):(\d+)\]|\b(vcc)(?:_lo|_hi)?\b")
+# (operands in front of the first source; which of them may be a scalar register is for SCALAR to say)
+WRITER = re.compile(r"v_(?:(?P<one>cmp_|readlane_|readfirstlane_)|(?:(?:add|sub|subrev|addc|subb|subbrev)_co_|div_scale_|mad_[iu]64_))")
+IMPLICIT_VCC = re.compile(r"v_(?:cndmask_b32_e32|(?:addc|subb|subbrev)_co_u32_e32|div_fmas_)")
+
+
+def _scalars(operands):
+    regs = set()
+    for first, low, high, vcc in SCALAR.findall(operands):
+        regs |= {vcc} if vcc else ({int(first)} if first else set(range(int(low), int(high) + 1)))
+    return regs
+
+
+def hazards(listing):
+    """(writer, reader) of every pair of vector instructions, in the order they lie in, with less than WAIT_STATES between them and a
+    scalar register of the one read by the other"""
+    found, recent = [], []                  # of the last instructions that wrote scalars: wait states since, registers, text
+    for line in listing:
+        if line[:1] != "\t":                # a label: another kernel, or a block of it (which may still follow the last one)
+            continue
+        op, _, rest = line.strip().partition(" ")
+        states = 1
+        if op == "s_nop":
+            states += int(rest.split()[0], 0)
+        elif op in ("s_endpgm", "s_branch", "s_setpc_b64"):
+            recent = []
+        elif op.startswith("v_"):
+            writes = WRITER.match(op)
+            if recent or writes:
+                operands = rest.split("//")[0].split(", ")
+                results = 2 if writes and not writes["one"] else 1
+                if recent:
+                    reads = _scalars(" ".join(operands[results:])) | ({"vcc"} if IMPLICIT_VCC.match(op) else set())
+                    found += [(text, line.strip()) for _, regs, text in recent if regs & reads]
+                if writes:
+                    regs = _scalars(" ".join(operands[:results]))
+                    recent = [(since + 1, r, text) for since, r, text in recent if since + 1 < WAIT_STATES]
+                    if regs:
+                        recent.append((0, regs, line.strip()))
+                    continue
+        if recent:
+            recent = [(since + states, r, text) for since, r, text in recent if since + states < WAIT_STATES]
+    return found
+
+
+def _code_objects(lib):
+    data = open(lib, "rb").read()
+    at = data.find(BUNDLE)
+    while at >= 0:
+        count, = struct.unpack_from("<Q", data, at + len(BUNDLE))
+        entry = at + len(BUNDLE) + 8
+        for _ in range(count):
+            offset, size, length = struct.unpack_from("<QQQ", data, entry)
+            if size and b"gfx950" in data[entry + 24:entry + 24 + length]:
+                yield data[at + offset:at + offset + size]
+            entry += 24 + length
+        at = data.find(BUNDLE, at + 1)
+
+
+def test_the_rule_on_short_listings():
+    def of(*lines):
+        return len(hazards("\t" + line for line in lines))
+    cmp, use = "v_cmp_lt_i64_e64 s[2:3], 0, v[2:3]", "v_cndmask_b32_e64 v5, 0, v5, s[2:3]"
+    assert of(cmp, use) == of(cmp, "s_nop 0", use) == of(cmp, "v_mov_b32_e32 v1, v2", use) == 1
+    assert of(cmp, "s_nop 1", use) == of(cmp, "v_mov_b32_e32 v1, v2", "s_add_u32 s9, s9, 1", use) == 0
+    assert of(cmp, "v_cndmask_b32_e64 v5, 0, v5, s[4:5]") == of(cmp, "s_endpgm", use) == 0
+    assert of("v_readlane_b32 s46, v41, 0", "v_readlane_b32 s47, v41, 16", "v_cndmask_b32_e64 v2, v2, -v2, s[46:47]") == 2
+    assert of("v_cmp_gt_f32_e32 vcc, v1, v2", "v_cndmask_b32_e32 v1, v2, v3, vcc") == 1
+    assert of("v_add_co_u32_e32 v1, vcc, v1, v2", "v_addc_co_u32_e32 v3, vcc, 0, v3, vcc") == 1
+
+
+# code objects by a kernel of theirs
+@pytest.mark.parametrize("kernel", [b"roundtrip_kernel"])
+def test_vector_instructions_wait_for_scalar_registers(kernel, tmp_path):
+    if not os.path.exists(OBJDUMP):
+        pytest.skip("no llvm-objdump")
+    from dynamiq_sigcomm_artifact_amd import capi
+
+    def of_object(index, code):
+        path = tmp_path / ("%d.co" % index)
+        path.write_bytes(code)
+        with subprocess.Popen([OBJDUMP, "-d", "--no-show-raw-insn", str(path)], stdout=subprocess.PIPE, text=True) as p:
+            found = hazards(p.stdout)
+        assert p.returncode == 0
+        return found
+
+    objects = [code for code in _code_objects(capi.LIB_PATH) if kernel in code]
+    assert objects
+    with ThreadPoolExecutor(8) as pool:
+        found = [pair for pairs in pool.map(of_object, range(len(objects)), objects) for pair in pairs]
+    assert not found, (len(found), found[:4])
