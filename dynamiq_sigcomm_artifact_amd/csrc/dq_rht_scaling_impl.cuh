@@ -967,7 +967,8 @@ __device__ __forceinline__ void strided_rows(float *__restrict__ x, const PassAr
             for (int i = 0; i < R2; i++) {
                 const uint32_t low = (uint32_t)__builtin_amdgcn_readlane((int)word, i), high = (uint32_t)__builtin_amdgcn_readlane((int)word, R2 + i);
                 const uint64_t mask = (uint64_t)low | ((uint64_t)high << 32);
-                asm("v_cndmask_b32_e64 %0, %0, -%0, %1" : "+v"(w[i]) : "s"(mask));
+                // (the two wait states behind a readlane are the compiler's only for its own instructions)
+                asm("s_nop 1\n\tv_cndmask_b32_e64 %0, %0, -%0, %1" : "+v"(w[i]) : "s"(mask));
             }
         } else if (flips && a.sign) {
 #pragma unroll

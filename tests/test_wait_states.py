@@ -84,23 +84,21 @@ def test_the_rule_on_short_listings():
     assert of("v_add_co_u32_e32 v1, vcc, v1, v2", "v_addc_co_u32_e32 v3, vcc, 0, v3, vcc") == 1
 
 
-# code objects by a kernel of theirs
-@pytest.mark.parametrize("kernel", [b"roundtrip_kernel"])
-def test_vector_instructions_wait_for_scalar_registers(kernel, tmp_path):
+def test_vector_instructions_wait_for_scalar_registers(tmp_path):
     if not os.path.exists(OBJDUMP):
         pytest.skip("no llvm-objdump")
     from dynamiq_sigcomm_artifact_amd import capi
 
-    def of_object(index, code):
-        path = tmp_path / ("%d.co" % index)
-        path.write_bytes(code)
+    def of_object(index_code):
+        path = tmp_path / ("%d.co" % index_code[0])
+        path.write_bytes(index_code[1])
         with subprocess.Popen([OBJDUMP, "-d", "--no-show-raw-insn", str(path)], stdout=subprocess.PIPE, text=True) as p:
             found = hazards(p.stdout)
         assert p.returncode == 0
         return found
 
-    objects = [code for code in _code_objects(capi.LIB_PATH) if kernel in code]
-    assert objects
     with ThreadPoolExecutor(8) as pool:
-        found = [pair for pairs in pool.map(of_object, range(len(objects)), objects) for pair in pairs]
+        of_objects = list(pool.map(of_object, enumerate(_code_objects(capi.LIB_PATH))))
+    assert of_objects
+    found = [pair for pairs in of_objects for pair in pairs]
     assert not found, (len(found), found[:4])
