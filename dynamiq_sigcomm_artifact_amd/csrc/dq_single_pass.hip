@@ -357,7 +357,7 @@ struct StatsArgs {
     TileWidths widths;
 };
 
-template <int DT, int GROUPS, bool NT> __global__ __launch_bounds__(64 * kStatsWaves, 8) void ranks_stats_kernel(StatsArgs a)
+template <int DT, int GROUPS, bool NT, bool WORDS> __global__ __launch_bounds__(64 * kStatsWaves, 8) void ranks_stats_kernel(StatsArgs a)
 {
     extern __shared__ __attribute__((aligned(16))) uint8_t tiles[];
     const RankPointers &ranks = a.ranks;
@@ -367,7 +367,9 @@ template <int DT, int GROUPS, bool NT> __global__ __launch_bounds__(64 * kStatsW
     float *__restrict__ mean_out = a.mean;
     const int world = a.world, vec = a.vec;
     const int64_t n = a.n;
-    const float u = widths.rule.u_dev ? (float)*widths.rule.u_dev : widths.rule.u;
+    // asked for ahead of the loads of a single tile; behind the last of several, whose 64 registers have no room for it
+    float u = 0.0f;
+    if (WORDS && GROUPS == 1) u = widths.rule.u_dev ? (float)*widths.rule.u_dev : widths.rule.u;
     constexpr int kRows = GROUPS * kRowsPerWave;
     __shared__ uint32_t pairs[kMaxRanks][kRows];
     typedef StatsTile<DT> ST;
@@ -431,6 +433,7 @@ template <int DT, int GROUPS, bool NT> __global__ __launch_bounds__(64 * kStatsW
             }
         }
     }
+    if (WORDS && GROUPS > 1) u = widths.rule.u_dev ? (float)*widths.rule.u_dev : widths.rule.u;
     __syncthreads();
     if (threadIdx.x < rows_here) {
         uint32_t acc = pairs[0][threadIdx.x];
@@ -441,7 +444,7 @@ template <int DT, int GROUPS, bool NT> __global__ __launch_bounds__(64 * kStatsW
             acc = f32_to_bf16_bits(lo) | (f32_to_bf16_bits(hi) << 16);
         }
         total[sc0 + threadIdx.x] = acc;
-        if (widths.words) {
+        if (WORDS) {
             const int cls = class_of_norm(acc >> 16, u, widths.rule.thr);
             const uint64_t eights = __builtin_amdgcn_ballot_w64(cls == 0), fours = __builtin_amdgcn_ballot_w64(cls == 1);
             if ((threadIdx.x & 3) == 0)
@@ -845,16 +848,15 @@ hipError_t launch_ranks_stats(const void *const *src, int world, int64_t n, void
     const int waves = world < kStatsWaves ? world : kStatsWaves;
     const StatsArgs args{p, world, vec, n, static_cast<uint32_t *>(total), mean, make_world_div(world, dtype == DQ_F32 ? 4 : 2),
                          TileWidths{tile_widths, tile_widths ? make_rule(u, u_dev) : WidthRule{0.0f, nullptr, {-1, -1}}}};
-    const auto run = [&](auto type, auto groups, auto nt) {
-        constexpr int DT = decltype(type)::value, G = decltype(groups)::value;
-        return launch_with(ranks_stats_kernel<DT, G, decltype(nt)::value>, dim3((unsigned)((tiles + G - 1) / G)), dim3(64 * waves), stream,
-                           args, waves * StatsTile<DT>::BYTES);
+    const auto run = [&](auto kernel, int groups, int tile_bytes) {
+        return launch_with(kernel, dim3((unsigned)((tiles + groups - 1) / groups)), dim3(64 * waves), stream, args, waves * tile_bytes);
     };
     const auto launch = [&](auto type) {
-        if (!vec) return run(type, std::integral_constant<int, 1>(), std::false_type());
-        if (tiles * world * StatsTile<decltype(type)::value>::ESZ * 1024 > kStatsCache) return run(type, std::integral_constant<int, 8>(), std::true_type());
-        if (tiles * world > kStatsOneTile) return run(type, std::integral_constant<int, 4>(), std::false_type());
-        return run(type, std::integral_constant<int, 1>(), std::false_type());
+        constexpr int DT = decltype(type)::value, kTile = StatsTile<DT>::BYTES;
+        if (vec && tiles * world * StatsTile<DT>::ESZ * 1024 > kStatsCache && !tile_widths) return run(ranks_stats_kernel<DT, 8, true, false>, 8, kTile);
+        if (vec && tiles * world > kStatsOneTile)
+            return tile_widths ? run(ranks_stats_kernel<DT, 4, false, true>, 4, kTile) : run(ranks_stats_kernel<DT, 4, false, false>, 4, kTile);
+        return tile_widths ? run(ranks_stats_kernel<DT, 1, false, true>, 1, kTile) : run(ranks_stats_kernel<DT, 1, false, false>, 1, kTile);
     };
     return dtype == DQ_BF16 ? launch(std::integral_constant<int, DQ_BF16>()) : launch(std::integral_constant<int, DQ_F32>());
 }

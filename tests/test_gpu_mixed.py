@@ -784,6 +784,12 @@ def test_rings_without_lists(capi, W, n, dt):
     assert len(seen) > 1
 
 
+@pytest.mark.parametrize("W,n,dt", [(8, 256 * 12288, torch.bfloat16), (16, 256 * 8705 - 3, torch.float32)])
+def test_rings_without_lists_behind_several_tiles_per_wave(capi, W, n, dt):
+    """so many ranks that the statistics take four tiles per wave while the ring still goes by their counts"""
+    test_rings_without_lists(capi, W, n, dt)
+
+
 @pytest.mark.parametrize("W,n", [(2, 256 * 8192), (3, 256 * 8192 + 1), (5, 256 * 8195)])
 def test_ranks_on_either_side_of_a_superchunk_per_wave(capi, W, n):
     """the last length that takes a wave per superchunk (MEE; AEE below) and the first ones that take four superchunks per wave"""

@@ -1,6 +1,10 @@
-"""The machine code of the built library keeps the wait states that gfx950 asks for between a vector instruction that writes a scalar
-register -- a comparison's mask, a readlane, a carry -- and a vector instruction that reads it: two.  The compiler sees to it for its own
-instructions, but not for those of inline assembly, whose operands may come straight from such an instruction."""
+"""What the machine code of the built library keeps to.
+
+Wait states: gfx950 asks for two between a vector instruction that writes a scalar register -- a comparison's mask, a readlane, a carry
+-- and a vector instruction that reads it.  The compiler sees to it for its own instructions, but not for those of inline assembly, whose
+operands may come straight from such an instruction.
+
+Scratch: kernels that are held to a number of registers fit into it."""
 import os
 import re
 import struct
@@ -10,6 +14,7 @@ from concurrent.futures import ThreadPoolExecutor
 import pytest
 
 OBJDUMP = "/opt/rocm/llvm/bin/llvm-objdump"
+READELF = "/opt/rocm/llvm/bin/llvm-readelf"
 BUNDLE = b"__CLANG_OFFLOAD_BUNDLE__"
 WAIT_STATES = 2
 
@@ -102,3 +107,20 @@ def test_vector_instructions_wait_for_scalar_registers(tmp_path):
     assert of_objects
     found = [pair for pairs in of_objects for pair in pairs]
     assert not found, (len(found), found[:4])
+
+
+def test_statistics_of_all_ranks_fit_their_registers(tmp_path):
+    """ranks_stats_kernel is held to 64 registers: every variant, with and without the words of short rings, without scratch"""
+    if not os.path.exists(READELF):
+        pytest.skip("no llvm-readelf")
+    from dynamiq_sigcomm_artifact_amd import capi
+    code = next(c for c in _code_objects(capi.LIB_PATH) if b"ranks_stats_kernel" in c)
+    path = tmp_path / "single_pass.co"
+    path.write_bytes(code)
+    notes = subprocess.run([READELF, "--notes", str(path)], stdout=subprocess.PIPE, text=True, check=True).stdout
+    scratch = {}
+    for kernel in notes.split("- .agpr_count")[1:]:
+        field = dict(re.findall(r"^\s+\.(name|private_segment_fixed_size):\s+(\S+)", kernel, re.M))
+        scratch[field["name"]] = int(field["private_segment_fixed_size"])
+    stats = {name: size for name, size in scratch.items() if "ranks_stats_kernel" in name}
+    assert len(stats) >= 6 and not any(stats.values()), stats
