@@ -627,11 +627,16 @@ template <int KT> __device__ __forceinline__ void middle_stages(float *lds, int 
         lds_pass<4, KT < 13 ? KT - 8 : 4>(lds, KT, tid, nthreads);
 }
 
-// Vectors of so many elements leave the first pass with the non-temporal hint: what waits in the L2 until the kernel ends, up to 32 MB, is
-// then on its way while others still load.  First pass, us, without -> with: 2^23 elements from bf16 levels 13.8 -> 9.5, from a 25 MB
-// gradient 12.8 -> 11.7.  The pass that reads them takes 0.5 to 1 longer, which costs shorter ones more than they gain, and 2^24 fill the
-// L2 long before the end.  There and back, without -> with: EDEN 262,144 21.4 -> 22.2, 2^20 26.7 -> 27.0, 2^21 37.3 -> 37.2, 2^22 52.9 ->
-// 54.1, 2^23 74.5 -> 72.6; THC 4,000,000 38.0 -> 38.4, 6,553,600 50.3 -> 45.7, 2^24 103 -> 111.5.
+// First passes with a source of another type or length store so many elements with the non-temporal hint: what waits in the L2 until the
+// kernel ends, more than half of its 32 MB, is then on its way while others still load.  2^23 elements from bf16 levels 13.8 -> 9.5 us, from
+// a 25 MB gradient 12.8 -> 11.7.  The pass that reads them takes 0.5 to 1 longer, which costs fewer elements more than they gain, and more
+// than 32 MB fill the L2 long before the end.  Where the pass reads what it overwrites it gains nothing.  The whole call, us, without ->
+// with:
+//   THC compress    4,194,304 18.0 18.2; of 2^23: 4,300,000 25.7 23.8, 6,553,600 25.9 24.2, all 26.3 25.3; of 2^24: 4,300,000 30.2 30.0,
+//                   6,553,600 31.7 30.1, 8,300,000 33.4 32.8, 10,000,000 40.0 41.4, all 49.7 53.5
+//   THC decompress  2^22 19.5 19.6, 2^23 25.3 24.4, 2^24 46.5 49.4
+//   EDEN            compress 2^22 32.8 33.2, 2^23 46.7 47.0, 2^24 81.8 86.0; decompress 20.4 20.9, 36.3 34.8, 54.1 57.4
+//   in place        forward, blocks of 2^18: 4.5 x 2^20 22.5 22.2, 6 x 2^20 21.6 21.9, 7 x 2^20 21.0 21.7, 2^23 22.7 23.8, 2^24 42.3 42.9
 constexpr int64_t kEarlyFrom = ((int64_t)1 << 22) + 1, kEarlyTo = (int64_t)1 << 23;
 
 // lds_pass whose results go to memory: consecutive lanes hold consecutive elements (P >= 6)
@@ -727,7 +732,7 @@ __device__ __forceinline__ void tile_pass(float *__restrict__ x, const PassArgs<
 // than tile_pass.  Bound like the strided passes; 2^23 elements from bf16 levels 13.4 -> 11.8 us, from a 25 MB gradient 17.3 -> 15.0.
 template <bool ENDS, class E>
 __device__ __forceinline__ void first_pass(float *__restrict__ x, const PassArgs<ENDS> &a, int sign_mode, const E &e, unsigned block,
-                                           float *lds, int threads)
+                                           float *lds, int threads, bool early)
 {
     const int tid = threadIdx.x;
     const int64_t origin = (int64_t)block << a.kt;
@@ -765,7 +770,6 @@ __device__ __forceinline__ void first_pass(float *__restrict__ x, const PassArgs
     }
     __syncthreads();
     float *out = x + origin;
-    const bool early = a.n >= kEarlyFrom && a.n <= kEarlyTo;
     switch (a.kt) {
     case 10: lds_pass_out<6, 4>(lds, 10, tid, step, out, early); break;
     case 11: lds_pass_out<7, 4>(lds, 11, tid, step, out, early); break;
@@ -1103,7 +1107,7 @@ struct FirstPass {
     int64_t n, in_count;
     float scale, grid[7]; // lo, spacing, step, t, inv_sqrt, inv_levels, inv_clients
     uint32_t gen_ss;
-    uint8_t kt, kb, vec, sign_bits, sign_mode, gen_bits, end, in_dtype, in_nbits, grid_kind;
+    uint8_t kt, kb, vec, sign_bits, sign_mode, gen_bits, end, in_dtype, in_nbits, grid_kind, early;
 };
 static_assert(sizeof(FirstPass) <= 128, "see above");
 
@@ -1199,6 +1203,7 @@ inline FirstPass first_of(float *x, const RhtPassArgs &a, int sign_mode, const T
     p.in_lo = e.in_lo; p.in_count = e.in_count;
     p.in_dtype = (uint8_t)e.in_dtype; p.in_nbits = (uint8_t)e.in_nbits;
     p.grid_kind = (uint8_t)e.grid.kind;
+    p.early = !e.plain_in() && a.n >= kEarlyFrom && a.n <= kEarlyTo;
     const float grid[7] = {e.grid.lo, e.grid.spacing, e.grid.step, e.grid.t, e.grid.inv_sqrt, e.grid.inv_levels, e.grid.inv_clients};
     for (int k = 0; k < 7; k++) p.grid[k] = grid[k];
     return p;
@@ -1250,7 +1255,7 @@ template <int A> __global__ __launch_bounds__(32 << A) void rht_strided_draw_ker
 template <bool ENDS> __global__ __launch_bounds__(1024) void rht_first_kernel(FirstPass p)
 {
     extern __shared__ __attribute__((aligned(16))) float lds[];
-    first_pass<ENDS>(p.x, pass_args<ENDS>(p), p.sign_mode, ends_of(p), blockIdx.x, lds, tile_threads(p.kt));
+    first_pass<ENDS>(p.x, pass_args<ENDS>(p), p.sign_mode, ends_of(p), blockIdx.x, lds, tile_threads(p.kt), ENDS && p.early);
 }
 
 #if DQ_RHT_PART & DQ_RHT_TRANSFORM
@@ -1284,7 +1289,7 @@ __global__ __launch_bounds__(1024) void rht_tile_passes_kernel(PassSet set)
 {
     extern __shared__ __attribute__((aligned(16))) float lds[];
     const TilePass &p = pass_of_block();
-    first_pass<true>(p.x, pass_args(p), p.sign_mode, p.ends, blockIdx.x - p.first, lds, blockDim.x);
+    first_pass<true>(p.x, pass_args(p), p.sign_mode, p.ends, blockIdx.x - p.first, lds, blockDim.x, false); // (slices end at 2^22 elements)
 }
 
 __global__ __launch_bounds__(512) void rht_strided_passes_kernel(PassSet set)

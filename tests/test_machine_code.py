@@ -4,7 +4,9 @@ Wait states: gfx950 asks for two between a vector instruction that writes a scal
 -- and a vector instruction that reads it.  The compiler sees to it for its own instructions, but not for those of inline assembly, whose
 operands may come straight from such an instruction.
 
-Scratch: kernels that are held to a number of registers fit into it."""
+Scratch: kernels that are held to a number of registers fit into it.
+
+Hints: the first pass of a transform in place stores without the non-temporal hint, which costs it up to 4 %."""
 import os
 import re
 import struct
@@ -107,6 +109,25 @@ def test_vector_instructions_wait_for_scalar_registers(tmp_path):
     assert of_objects
     found = [pair for pairs in of_objects for pair in pairs]
     assert not found, (len(found), found[:4])
+
+
+def test_the_first_pass_in_place_stores_without_a_hint(tmp_path):
+    if not os.path.exists(OBJDUMP):
+        pytest.skip("no llvm-objdump")
+    from dynamiq_sigcomm_artifact_amd import capi
+    stores = {}
+    for k, code in enumerate(c for c in _code_objects(capi.LIB_PATH) if b"rht_first_kernel" in c):
+        path = tmp_path / ("%d.co" % k)
+        path.write_bytes(code)
+        listing = subprocess.run([OBJDUMP, "-d", "--no-show-raw-insn", str(path)], stdout=subprocess.PIPE, text=True, check=True).stdout
+        for kernel in re.split(r"^[0-9a-f]+ <", listing, flags=re.M):
+            name = re.match(r"\S*rht_first_kernelILb([01])E", kernel)
+            if name:
+                found = re.findall(r"^\t(global_store_dword\w* .*?)\s*(?://|$)", kernel, re.M)
+                stores.setdefault(name[1] == "1", []).append((len(found), sum(" nt" in store for store in found)))
+    assert set(stores) == {False, True}
+    assert all(count > 0 and hinted == 0 for count, hinted in stores[False]), stores
+    assert all(hinted > 0 for _, hinted in stores[True]), stores
 
 
 def test_statistics_of_all_ranks_fit_their_registers(tmp_path):
