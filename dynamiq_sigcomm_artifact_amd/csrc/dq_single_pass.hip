@@ -117,7 +117,10 @@ struct WidthRule {
     int thr[2];          // with u a number: the patterns of width 4 and 8 found on the host, else -1
 };
 
-// (A launch carries arguments for one bucket, twelve or kMaxBuckets: 2 KB of them take the host and the GPU 2 us longer than 300 bytes.)
+// A launch carries arguments for one bucket or for kMaxBuckets, 296 bytes or 2,152.  A call on one bucket, us, in a stream, with room for
+// one, two, 8, 32: 4,096 elements 7.3, 7.5, 7.8, 7.9; 10^6 elements 7.4, 8.2, 8.4, 8.5.  Lists gain little by less room (two of
+// 65,536, with room for two, 8, 32: 7.8, 8.5, 8.2; nine, with room for twelve and 32: 8.8 and 8.8, recorded 8.8 and 8.7, the first pass
+// 48 and 46), so they have one.
 template <int MOST> struct RoundtripArgs {
     uint32_t first_tile[MOST]; // ascending
     RoundtripBucket bucket[MOST];
@@ -815,7 +818,7 @@ hipError_t launch_roundtrip(const RoundtripDesc *desc, int count, int world, flo
                             uint64_t *step_dev, uint64_t step_more, uint32_t *hist, int dtype, bool mee, const MeeParams *mp,
                             hipStream_t stream)
 {
-    const auto run = count == 1 ? run_roundtrip<1> : (count <= 12 ? run_roundtrip<12> : run_roundtrip<kMaxBuckets>);
+    const auto run = count == 1 ? run_roundtrip<1> : run_roundtrip<kMaxBuckets>;
     return run(desc, count, world, u, u_dev, seed, step_dev, step_more, hist, dtype, mee, mp, stream);
 }
 
