@@ -114,7 +114,7 @@ hipError_t launch_roundtrip(const RoundtripDesc *desc, int count, int world, flo
                             uint64_t *step_dev, uint64_t step_more, uint32_t *hist, int dtype, bool mee, const MeeParams *mp,
                             hipStream_t stream);
 // total: bf16 pairs [nsc], mean: float [world][nsc]; tile_widths (may be null): a word per four superchunks, how many of them u
-// (or *u_dev) gives 8 bits, and 4 bits in the upper half
+// (or *u_dev) gives 8 bits, and 4 bits in the upper half (added up as words: at most 65,535 superchunks, see ring_plans_itself)
 hipError_t launch_ranks_stats(const void *const *src, int world, int64_t n, void *total, float *mean, int dtype,
                               uint32_t *tile_widths, float u, const double *u_dev, hipStream_t stream);
 // a ring that finds its groups from the words of launch_ranks_stats (in the place of a plan and its lists)

@@ -756,6 +756,7 @@ bool a_wave_each(int nsc, int world, int elem_bytes, bool mee, bool pooled)
 // -> 12.8, x 12,288 24.2 -> 21.7; 2 x 3,907 13.0 -> 10.4, x 12,288 16.7 -> 16.2, x 16,384 19.5 -> 20.7; MEE 8 x 3,907 25.4 -> 21.2, 2 x
 // 12,288 18.9 -> 17.9; fp32 8 x 3,907 27.7 -> 22.0, 2 x 12,288 20.8 -> 17.1.
 constexpr int64_t kPlansItself = 12288;
+static_assert(kPlansItself <= 0xffff, "a width's count over all superchunks is half a word (ring_quad_kernel, PLANS)");
 
 WidthRule make_rule(float u, const double *u_dev)
 {
