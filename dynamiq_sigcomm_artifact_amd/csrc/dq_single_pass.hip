@@ -13,10 +13,10 @@
 //   ring_kernel        W ranks, after a plan of the reduced statistics: the ring
 //   ring_quad_kernel   the same on short vectors, one superchunk per wave; with drawn values it does without the plan
 //
-// Measured, start -> now (bit-identical results): 8 ranks x 124,439,808 bf16 elements 2,896 -> 1,066 us per all-reduce (one
+// Measured, start -> now (bit-identical results): 8 ranks x 124,439,808 bf16 elements 2,896 -> 1,070 us per all-reduce (one
 // launch per rank and ring step, packed streams and their exchange copies, against three launches whose traffic is the
-// vectors alone), 8 x 1,000,003 elements 1,488 -> 20 us (257 launches against 2), a step of nine 25 MB buckets on one rank
-// 252 -> 51 us (four launches per bucket on two streams against two launches per step, and the search for u).
+// vectors alone), 8 x 1,000,003 elements 1,488 -> 21 us (257 launches against 2), a step of nine 25 MB buckets on one rank
+// 252 -> 52 us (four launches per bucket on two streams against two launches per step, and the search for u).
 //
 // Numerics: csrc/cuda_hadamard.cu:1257-1369 (centring, mean add), csrc/cuda_hierarchical_mee.cu:203-696 (codec),
 // testbed_evaluation/new_comm_hooks/ring_rdma.py:590-631 (order of the ring), comm_hooks.py:64-70 (widths).
