@@ -1107,7 +1107,7 @@ struct FirstPass {
     int64_t n, in_count;
     float scale, grid[7]; // lo, spacing, step, t, inv_sqrt, inv_levels, inv_clients
     uint32_t gen_ss;
-    uint8_t kt, kb, vec, sign_bits, sign_mode, gen_bits, end, in_dtype, in_nbits, grid_kind, early;
+    uint8_t kt, kb, vec, sign_bits, sign_mode, gen_bits, end, in_dtype, in_nbits, grid_kind;
 };
 static_assert(sizeof(FirstPass) <= 128, "see above");
 
@@ -1203,7 +1203,6 @@ inline FirstPass first_of(float *x, const RhtPassArgs &a, int sign_mode, const T
     p.in_lo = e.in_lo; p.in_count = e.in_count;
     p.in_dtype = (uint8_t)e.in_dtype; p.in_nbits = (uint8_t)e.in_nbits;
     p.grid_kind = (uint8_t)e.grid.kind;
-    p.early = !e.plain_in() && a.n >= kEarlyFrom && a.n <= kEarlyTo;
     const float grid[7] = {e.grid.lo, e.grid.spacing, e.grid.step, e.grid.t, e.grid.inv_sqrt, e.grid.inv_levels, e.grid.inv_clients};
     for (int k = 0; k < 7; k++) p.grid[k] = grid[k];
     return p;
@@ -1232,6 +1231,10 @@ inline StridedPass strided_of(float *x, const RhtPassArgs &a, int rbits, int sbi
     return p;
 }
 
+// Code of 20 to 40 KB a kernel: where it begins shows in passes of 10 us.  THC on 25 MB, the same instructions 2.8 KB further on, 45.7 -> 46.7
+// us; at the beginning of a page 45.8 wherever that lies.
+#define DQ_OWN_PAGES __attribute__((aligned(4096)))
+
 template <bool ENDS> __global__ __launch_bounds__(512) void rht_strided_kernel(StridedPass p)
 {
     extern __shared__ __attribute__((aligned(16))) float lds[];
@@ -1239,23 +1242,24 @@ template <bool ENDS> __global__ __launch_bounds__(512) void rht_strided_kernel(S
 }
 
 // 512 (B = 4) or 1024 rows (B = 5)
-template <bool ENDS, int B> __global__ __launch_bounds__(32 << B) void rht_strided_long_kernel(StridedPass p)
+template <bool ENDS, int B> DQ_OWN_PAGES __global__ __launch_bounds__(32 << B) void rht_strided_long_kernel(StridedPass p)
 {
     extern __shared__ __attribute__((aligned(16))) float lds[];
     strided_rows<ENDS, 5, B>(p.x, pass_args<ENDS>(p), p.sbits, p.sign_mode, p.apply_scale, ends_of(p), blockIdx.x, lds);
 }
 
 // 256 (A = 4) or 1024 rows (A = 5) to THC's levels with drawn values
-template <int A> __global__ __launch_bounds__(32 << A) void rht_strided_draw_kernel(StridedPass p)
+template <int A> DQ_OWN_PAGES __global__ __launch_bounds__(32 << A) void rht_strided_draw_kernel(StridedPass p)
 {
     extern __shared__ __attribute__((aligned(16))) float lds[];
     strided_rows<true, A, A, true>(p.x, pass_args<true>(p), p.sbits, p.sign_mode, p.apply_scale, ends_of(p), blockIdx.x, lds);
 }
 
-template <bool ENDS> __global__ __launch_bounds__(1024) void rht_first_kernel(FirstPass p)
+template <bool ENDS> DQ_OWN_PAGES __global__ __launch_bounds__(1024) void rht_first_kernel(FirstPass p)
 {
     extern __shared__ __attribute__((aligned(16))) float lds[];
-    first_pass<ENDS>(p.x, pass_args<ENDS>(p), p.sign_mode, ends_of(p), blockIdx.x, lds, tile_threads(p.kt), ENDS && p.early);
+    first_pass<ENDS>(p.x, pass_args<ENDS>(p), p.sign_mode, ends_of(p), blockIdx.x, lds, tile_threads(p.kt),
+                     ENDS && p.end != kNoEnd && p.n >= kEarlyFrom && p.n <= kEarlyTo);
 }
 
 #if DQ_RHT_PART & DQ_RHT_TRANSFORM
