@@ -117,10 +117,12 @@ struct WidthRule {
     int thr[2];          // with u a number: the patterns of width 4 and 8 found on the host, else -1
 };
 
-// A launch carries arguments for one bucket or for kMaxBuckets, 296 bytes or 2,152.  A call on one bucket, us, in a stream, with room for
-// one, two, 8, 32: 4,096 elements 7.3, 7.5, 7.8, 7.9; 10^6 elements 7.4, 8.2, 8.4, 8.5.  Lists gain little by less room (two of
-// 65,536, with room for two, 8, 32: 7.8, 8.5, 8.2; nine, with room for twelve and 32: 8.8 and 8.8, recorded 8.8 and 8.7, the first pass
-// 48 and 46), so they have one.
+// A launch carries arguments for one bucket, kFewBuckets or kMaxBuckets: 296, 952 or 2,152 bytes.  A call on one bucket, us, in a stream,
+// with room for one, two, 8, 32: 4,096 elements 7.3, 7.5, 7.8, 7.9; 10^6 elements 7.4, 8.2, 8.4, 8.5.  Streams and replays of lists gain
+// less than 0.3 by less room, but recording them takes longer beyond a kilobyte: the first pass of a step of nine buckets of 10^6 elements,
+// by room, 9: 101, 12: 100, 13 (1,012 bytes): 100, 14 (1,072): 153, 16: 145, 24: 143, 32: 144; of twelve 104, and 149 with room for 32.
+constexpr int kFewBuckets = 12;
+
 template <int MOST> struct RoundtripArgs {
     uint32_t first_tile[MOST]; // ascending
     RoundtripBucket bucket[MOST];
@@ -777,6 +779,7 @@ static hipError_t run_roundtrip(const RoundtripDesc *desc, int count, int world,
 {
     RoundtripArgs<MOST> a;
     TallyArgs<MOST> t;
+    static_assert(MOST > kFewBuckets || sizeof(a) <= 1024, "see RoundtripArgs");
     memset(&t, 0, sizeof(t));
     memset(&a, 0, offsetof(RoundtripArgs<MOST>, rule));
     uint32_t tiles = 0, blocks = 0;
@@ -819,7 +822,7 @@ hipError_t launch_roundtrip(const RoundtripDesc *desc, int count, int world, flo
                             uint64_t *step_dev, uint64_t step_more, uint32_t *hist, int dtype, bool mee, const MeeParams *mp,
                             hipStream_t stream)
 {
-    const auto run = count == 1 ? run_roundtrip<1> : run_roundtrip<kMaxBuckets>;
+    const auto run = count == 1 ? run_roundtrip<1> : (count <= kFewBuckets ? run_roundtrip<kFewBuckets> : run_roundtrip<kMaxBuckets>);
     return run(desc, count, world, u, u_dev, seed, step_dev, step_more, hist, dtype, mee, mp, stream);
 }
 

@@ -1146,7 +1146,7 @@ def test_list_of_buckets_of_two_types(capi, kinds):
 
 @pytest.mark.parametrize("kinds", ["b" * 12, "b" * 13, "f" * 12 + "b" * 13 + "f"])
 def test_lists_on_either_side_of_a_launchs_room(capi, kinds):
-    """a launch has room for one bucket or 32, whatever the list's length"""
+    """a launch has room for one, twelve or 32 buckets"""
     test_list_of_buckets_of_two_types(capi, kinds)
 
 
