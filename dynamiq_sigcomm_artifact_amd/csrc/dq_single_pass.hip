@@ -118,9 +118,9 @@ struct WidthRule {
 };
 
 // A launch carries arguments for one bucket, kFewBuckets or kMaxBuckets: 296, 952 or 2,152 bytes.  A call on one bucket, us, in a stream,
-// with room for one, two, 8, 32: 4,096 elements 7.3, 7.5, 7.8, 7.9; 10^6 elements 7.4, 8.2, 8.4, 8.5.  Streams and replays of lists gain
-// less than 0.3 by less room, but recording them takes longer beyond a kilobyte: the first pass of a step of nine buckets of 10^6 elements,
-// by room, 9: 101, 12: 100, 13 (1,012 bytes): 100, 14 (1,072): 153, 16: 145, 24: 143, 32: 144; of twelve 104, and 149 with room for 32.
+// with room for one, two, 8, 32: 4,096 elements 7.3, 7.5, 7.8, 7.9; 10^6 elements 7.4, 8.2, 8.4, 8.5.  Steady steps of lists gain less
+// than 0.3 by less room, but beyond a kilobyte the host takes longer for the first step of a new object on new tensors: nine buckets of 10^6
+// elements, by room, 9: 101, 12: 100, 13 (1,012 bytes): 100, 14 (1,072): 153, 16: 145, 24: 143, 32: 144; twelve 104, and 149 with 32.
 constexpr int kFewBuckets = 12;
 
 template <int MOST> struct RoundtripArgs {
