@@ -1231,8 +1231,8 @@ inline StridedPass strided_of(float *x, const RhtPassArgs &a, int rbits, int sbi
     return p;
 }
 
-// Code of 20 to 40 KB a kernel: where it begins shows in passes of 10 us.  THC on 25 MB, the same instructions 2.8 KB further on, 45.7 -> 46.7
-// us; at the beginning of a page 45.8 wherever that lies.
+// 30 to 50 KB of code a kernel: where it begins shows in passes of 10 us.  THC on 25 MB, nearly the same instructions 2.8 KB further on,
+// 45.7 -> 46.7 us; begun at a multiple of 1 KB 46.5, of 4 KB 45.8, of 64 KB 45.5.
 #define DQ_OWN_PAGES __attribute__((aligned(4096)))
 
 template <bool ENDS> __global__ __launch_bounds__(512) void rht_strided_kernel(StridedPass p)
