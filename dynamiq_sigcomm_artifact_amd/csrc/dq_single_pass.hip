@@ -11,11 +11,11 @@
 //   tally_kernel       behind it: the widths' counts per bucket and the norm histogram of the search for u
 //   ranks_stats_kernel W ranks: every rank's means, and the reduced statistics
 //   ring_kernel        W ranks, after a plan of the reduced statistics: the ring
-//   ring_quad_kernel   the same on short vectors, one superchunk per wave; with drawn values it does without the plan
+//   ring_parts_kernel  the same on short vectors, one or two superchunks per wave; with drawn values it does without the plan
 //
 // Measured, start -> now (bit-identical results): 8 ranks x 124,439,808 bf16 elements 2,896 -> 1,070 us per all-reduce (one
 // launch per rank and ring step, packed streams and their exchange copies, against three launches whose traffic is the
-// vectors alone), 8 x 1,000,003 elements 1,488 -> 21 us (257 launches against 2), a step of nine 25 MB buckets on one rank
+// vectors alone), 8 x 1,000,003 elements 1,488 -> 20 us (257 launches against 2), a step of nine 25 MB buckets on one rank
 // 252 -> 52 us (four launches per bucket on two streams against two launches per step, and the search for u).
 //
 // Numerics: csrc/cuda_hadamard.cu:1257-1369 (centring, mean add), csrc/cuda_hierarchical_mee.cu:203-696 (codec),
@@ -573,22 +573,25 @@ __global__ __launch_bounds__(64, DT == DQ_BF16 && RDT == DQ_PHILOX && !MEE ? 5 :
     for (int rank = 0; rank < world; rank++) store_tile<DT>(a.out[rank], out, stage, sc, rows_here, a.n, (a.vec & 2) != 0, lane);
 }
 
-// four elements of a lane, side by side with those of its neighbours
-template <int DT> __device__ __forceinline__ void store_quarter(void *dst, const Raw4<DT> &out, int64_t e, int64_t n, bool vec, bool ragged)
+// a lane's part of a chunk, side by side with those of its neighbours
+template <int DT, int N> __device__ __forceinline__ void store_part(void *dst, const RawPart<DT, N> &out, int64_t e, int64_t n, bool vec, bool ragged)
 {
+    constexpr int W = RawPart<DT, N>::kWords;
     if (vec && !ragged) {
-        if constexpr (DT == DQ_F32) {
-            stream_store(reinterpret_cast<uint4 *>(static_cast<uint32_t *>(dst) + e), make_uint4(out.w[0], out.w[1], out.w[2], out.w[3]));
-        } else {
+        uint32_t *p = static_cast<uint32_t *>(dst) + e * W / N;
+        if constexpr (W == 2) {
             typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
             const u32x2 t = {out.w[0], out.w[1]};
-            __builtin_nontemporal_store(t, reinterpret_cast<u32x2 *>(static_cast<uint16_t *>(dst) + e));
+            __builtin_nontemporal_store(t, reinterpret_cast<u32x2 *>(p));
+        } else {
+#pragma unroll
+            for (int k = 0; k < W; k += 4) stream_store(reinterpret_cast<uint4 *>(p + k), make_uint4(out.w[k], out.w[k + 1], out.w[k + 2], out.w[k + 3]));
         }
         return;
     }
-    const int left = left_here(n, e, 4);
+    const int left = left_here(n, e, N);
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
+    for (int i = 0; i < N; i++) {
         if (i < left) {
             if constexpr (DT == DQ_F32)
                 static_cast<uint32_t *>(dst)[e + i] = out.w[i];
@@ -598,50 +601,76 @@ template <int DT> __device__ __forceinline__ void store_quarter(void *dst, const
     }
 }
 
-constexpr int kQuadWaves = 4;
+// x / y for 0 <= x < 2^23, 0 < y, inv = 1 / y to within an ulp or two
+__device__ __forceinline__ int small_quotient(int x, int y, float inv)
+{
+    int q = (int)((float)x * inv);
+    const int r = x - q * y;
+    return q + (r >= y ? 1 : 0) - (r < 0 ? 1 : 0);
+}
 
-// ring_kernel with a superchunk per wave, four elements per lane: short vectors, where a wave's chain of `world` steps is all
-// there is to wait for (2 us a step with one wave of ring_kernel per SIMD, 0.7 us here).
+constexpr int kPartWaves = 4;
+
+// ring_kernel with N = 4 or 8 elements per lane, a superchunk or two per wave: short vectors, where a wave's chain of `world` steps is all
+// there is to wait for (2 us a step with one wave of ring_kernel per SIMD, 0.7 us with four elements).
 //
 // PLANS: without a plan launch in front.  A superchunk's way through the ring depends on the others only by where it starts: on its
 // place among those of its width.  The statistics leave a word per four superchunks with their widths' counts; a workgroup takes
-// four neighbouring superchunks and adds up the words, all of them and those before its own, while the norms of its own are on their way.
-template <int DT, int RDT, bool MEE, bool PLANS = false>
-__global__ __launch_bounds__(64 * kQuadWaves) void ring_quad_kernel(RingArgs<RDT != DQ_PHILOX> a)
+// neighbouring superchunks and adds up the words, all of them and those before its own, while the norms of its own are on their way.
+template <int DT, int RDT, bool MEE, int N, bool PLANS>
+__global__ __launch_bounds__(64 * kPartWaves) void ring_parts_kernel(RingArgs<RDT != DQ_PHILOX> a)
 {
+    constexpr int P = N / 4, kLanes = 64 / P, kHere = P * kPartWaves; // superchunks of a wave, lanes of one, superchunks of the workgroup
+    constexpr bool POOL = RDT != DQ_PHILOX;
     __shared__ float levels[MEE ? kLevelCount : 1];
+    // What a step needs besides its elements, by rank and once more, so that the ranks from any on lie side by side: the address of the
+    // vector and the mean.  (Loaded step by step through the scalar cache they are half of a step's time.)
+    __shared__ uint4 of_rank[kPartWaves][P][2 * kMaxRanks];
+    __shared__ uint64_t pool_of_step[POOL ? kPartWaves : 1][P][kMaxPoolRanks];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), world = a.world;
+    const int half = lane / kLanes; // (0 where a wave has one superchunk)
+    const int rank_here = lane & (2 * kMaxRanks - 1), my_rank = min(rank_here < world ? rank_here : rank_here - world, world - 1);
+    const int which = P == 1 ? 0 : lane >> 5; // superchunk whose ranks the lane fetches
+    const uint64_t my_src = reinterpret_cast<uint64_t>(a.src[my_rank]);
     if (MEE) {
         if (wave == 0) levels_to_lds(levels, lane);
         if (!PLANS) __syncthreads();
     }
-    const int at = (int)blockIdx.x * kQuadWaves + wave;
-    int cls = 3, k = 0, chunk = 0, in_run = 0;
-    int64_t sc = 0;
+    const int at0 = ((int)blockIdx.x * kPartWaves + wave) * P;
+    int cls[P], chunk[P], in_run[P];
+    int64_t sc[P];
+    float my_mean = 0.0f;
+    uint32_t total_mean = 0;
+    int have = 0; // of the wave's superchunks; the others repeat the first
     if constexpr (PLANS) {
-        static_assert(kQuadWaves == kRowsPerWave, "a workgroup's superchunks are those of one word");
-        __shared__ uint2 part[kQuadWaves];
+        static_assert(kHere % kRowsPerWave == 0, "a workgroup's superchunks are those of whole words");
+        __shared__ uint2 part[kPartWaves];
         const FromTileWidths &f = a.more;
-        const float u = f.rule.u_dev ? (float)*f.rule.u_dev : f.rule.u;
-        const int tile = blockIdx.x, tiles = (a.nsc + 3) >> 2;
-        const uint32_t norm = a.total[2 * min(4 * tile + (lane & 3), a.nsc - 1) + 1];
+        const int first_word = (int)blockIdx.x * P, words = (a.nsc + 3) >> 2;
+        const uint32_t norm = a.total[2 * min(kHere * (int)blockIdx.x + (lane & (kHere - 1)), a.nsc - 1) + 1];
+        // (neither waits for the place in the list)
+        my_mean = a.mean[(int64_t)my_rank * a.nsc + min(at0 + which, a.nsc - 1)];
+        total_mean = a.total[2 * min(at0 + half, a.nsc - 1)];
+        // (without a branch, behind which the other loads would only leave when it has arrived; where there is none, of what lies at hand)
+        const double u_dev = *(f.rule.u_dev ? f.rule.u_dev : reinterpret_cast<const double *>(f.counts));
         uint32_t all = 0, before = 0;
-        constexpr int kTogether = 4, kThreads = 64 * kQuadWaves;
-        for (int first = 0; first < tiles; first += kTogether * kThreads) {
+        constexpr int kTogether = 4, kThreads = 64 * kPartWaves;
+        for (int first = 0; first < words; first += kTogether * kThreads) {
             uint32_t got[kTogether];
 #pragma unroll
-            for (int i = 0; i < kTogether; i++) got[i] = f.words[min(first + i * kThreads + (int)threadIdx.x, tiles - 1)];
+            for (int i = 0; i < kTogether; i++) got[i] = f.words[min(first + i * kThreads + (int)threadIdx.x, words - 1)];
 #pragma unroll
             for (int i = 0; i < kTogether; i++) {
                 const int word = first + i * kThreads + (int)threadIdx.x;
-                all += word < tiles ? got[i] : 0u;
-                before += word < tile ? got[i] : 0u;
+                all += word < words ? got[i] : 0u;
+                before += word < first_word ? got[i] : 0u;
             }
         }
         all = wave_sum_upward(all);
         before = wave_sum_upward(before);
         if (lane == 63) part[wave] = make_uint2(all, before);
-        const int mine = class_of_norm(norm, u, f.rule.thr); // (of lane & 3)
+        const float u = f.rule.u_dev ? (float)u_dev : f.rule.u;
+        const int mine = class_of_norm(norm, u, f.rule.thr); // (of lane & (kHere - 1))
         __syncthreads();
         const uint2 p0 = part[0], p1 = part[1], p2 = part[2], p3 = part[3];
         all = (uint32_t)__builtin_amdgcn_readfirstlane((int)(p0.x + p1.x + p2.x + p3.x));
@@ -653,112 +682,165 @@ __global__ __launch_bounds__(64 * kQuadWaves) void ring_quad_kernel(RingArgs<RDT
             f.counts[2] = m2;
             f.counts[3] = 0;
         }
-        if (at >= a.nsc) return;
-        sc = at;
-        cls = __builtin_amdgcn_readlane(mine, wave);
-        const int m = cls == 0 ? m8 : (cls == 1 ? m4 : m2);
+        have = min(a.nsc - at0, P);
+        if (have <= 0) return;
         const int b8 = (int)(before & 0xffffu), b4 = (int)(before >> 16);
-        k = (cls == 0 ? b8 : (cls == 1 ? b4 : 4 * tile - b8 - b4)) +
-            __popcll(__builtin_amdgcn_ballot_w64(mine == cls) & ((1u << wave) - 1u));
-        chunk = min(k / max((m + world - 1) / world, 1), world - 1); // (within the ranks also with words that are not these norms')
+#pragma unroll
+        for (int h = 0; h < P; h++) {
+            const int of = h < have ? h : 0, bit = wave * P + of;
+            sc[h] = at0 + of;
+            cls[h] = __builtin_amdgcn_readlane(mine, bit);
+            const int m = cls[h] == 0 ? m8 : (cls[h] == 1 ? m4 : m2);
+            const int k = (cls[h] == 0 ? b8 : (cls[h] == 1 ? b4 : kRowsPerWave * first_word - b8 - b4)) +
+                          __popcll(__builtin_amdgcn_ballot_w64(mine == cls[h]) & ((1u << bit) - 1u));
+            // (within the ranks also with words that are not these norms')
+            const int per = max(small_quotient(max(m + world - 1, 0), world, a.wd.inv), 1);
+            chunk[h] = max(min(small_quotient(max(k, 0), per, __builtin_amdgcn_rcpf((float)per)), world - 1), 0);
+            in_run[h] = 0;
+        }
     } else {
-        // entry `at` of the three lists end to end; sizes clamped as in ring_kernel
-        int used = 0;
+        // entry at0 + h of the three lists end to end; sizes clamped as in ring_kernel
         const int counts[3] = {a.counts[0], a.counts[1], a.counts[2]};
 #pragma unroll
-        for (int g = 0; g < 3; g++) {
-            const int m = min(max(counts[g], 0), a.nsc - used);
-            if (cls == 3 && at - used < m) {
-                const int per = (m + world - 1) / world;
-                cls = g;
-                k = at - used;
-                chunk = k / per;
-                in_run = k - chunk * per;
+        for (int h = 0; h < P; h++) {
+            int used = 0, k = 0;
+            cls[h] = 3;
+#pragma unroll
+            for (int g = 0; g < 3; g++) {
+                const int m = min(max(counts[g], 0), a.nsc - used);
+                if (cls[h] == 3 && at0 + h - used < m) {
+                    const int per = small_quotient(m + world - 1, world, a.wd.inv);
+                    cls[h] = g;
+                    k = at0 + h - used;
+                    chunk[h] = small_quotient(k, per, __builtin_amdgcn_rcpf((float)per));
+                    in_run[h] = k - chunk[h] * per;
+                }
+                used += m;
             }
-            used += m;
+            if (cls[h] == 3) {
+                if (h == 0) return;
+                cls[h] = cls[0]; chunk[h] = chunk[0]; in_run[h] = in_run[0]; sc[h] = sc[0];
+            } else {
+                sc[h] = a.order[(int64_t)cls[h] * a.nsc + k];
+                have = h + 1;
+            }
         }
-        if (cls == 3) return;
-        sc = a.order[(int64_t)cls * a.nsc + k];
+        my_mean = a.mean[(int64_t)my_rank * a.nsc + sc[P - 1 < which ? P - 1 : which]];
+        total_mean = a.total[2 * sc[half]];
     }
-    const int64_t e0 = sc * 256 + lane * 4;
-    const bool ragged = sc * 256 + 256 > a.n;
-    const WidthRegs<MEE> w = width_regs<MEE>(a.widths, cls, levels);
-    const uint32_t total_mean = a.total[2 * sc];
+    const int64_t my_sc = P == 1 || half == 0 ? sc[0] : sc[P - 1];
+    const int my_chunk = P == 1 || half == 0 ? chunk[0] : chunk[P - 1], my_cls = P == 1 || half == 0 ? cls[0] : cls[P - 1];
+    const int64_t e0 = my_sc * 256 + (lane & (kLanes - 1)) * N;
+    const bool ragged = max(sc[0], sc[P - 1]) * 256 + 256 > a.n;
+    // The vector's end may lie inside a lane's elements: it loads the last N there are and drops those before its own when it comes to
+    // them.  (Loaded one by one and put together on the spot, the one ragged wave of a launch waited for memory in every step and
+    // outlasted all others: 15.8 us where they had ended at 11 to 13, 8 x 1,000,003 elements.)
+    const bool whole_loads = (a.vec & 1) != 0 && a.n >= N;
+    const int64_t from = min(e0, a.n - N);
+    const WidthRegs<MEE> w = width_regs<MEE>(a.widths, my_cls, levels);
+    if (rank_here < 2 * world && (P > 1 || lane < 2 * kMaxRanks))
+        of_rank[wave][which][rank_here] = make_uint4((uint32_t)my_src, (uint32_t)(my_src >> 32), __float_as_uint(my_mean), 0u);
+    if constexpr (POOL) {
+        const int step = lane & (kMaxPoolRanks - 1), h = (lane / kMaxPoolRanks) & (P - 1);
+        const int c = h == 0 ? chunk[0] : chunk[P - 1], g = h == 0 ? cls[0] : cls[P - 1], in = h == 0 ? in_run[0] : in_run[P - 1];
+        if (step < world) {
+            const int rank = c + step < world ? c + step : c + step - world;
+            pool_of_step[wave][h][step] = reinterpret_cast<uint64_t>(a.more.pool[g][rank]) +
+                                          (int64_t)(a.more.first[g][rank][step] + in * 16) * (16 * (RDT == DQ_F32 ? 4 : 2));
+        }
+    }
+    wave_lds_sync();
+    const uint4 *ranks = of_rank[wave][half] + my_chunk;
 
-    // What a step needs besides its elements, in the lanes of a few registers: lane s has the addresses and the mean of the
-    // rank of step s.  (Loaded step by step through the scalar cache they are half of a step's time.)
-    const int my_step = min(lane, world - 1), my_rank = chunk + my_step < world ? chunk + my_step : chunk + my_step - world;
-    const uint64_t my_src = reinterpret_cast<uint64_t>(a.src[my_rank]);
-    const float my_mean = a.mean[(int64_t)my_rank * a.nsc + sc];
-    uint64_t my_pool = 0;
-    if constexpr (RDT != DQ_PHILOX)
-        my_pool = reinterpret_cast<uint64_t>(a.more.pool[cls][my_rank]) +
-                  (int64_t)(a.more.first[cls][my_rank][my_step] + in_run * 16) * (16 * (RDT == DQ_F32 ? 4 : 2));
-    const auto of_step = [](uint64_t mine, int step) {
-        const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)mine, step);
-        const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(mine >> 32), step);
-        return reinterpret_cast<const void *>((uint64_t)lo | ((uint64_t)hi << 32));
-    };
-    Raw4<DT> next;
-    Raw4<RDT> next_r;
+    // (memory, and the compiler is told so: what it only knows as an address it loads through instructions that may also mean the LDS,
+    // and every read of the LDS then waits for the elements of the step to come)
+    typedef const __attribute__((address_space(1))) void *global;
+    const auto pointer = [](uint64_t at) { return (const void *)(global)at; };
+    RawPart<DT, N> next;
+    RawPart<RDT, N> next_r;
     next_r.zero();
+    float next_mean = 0.0f;
     const auto fetch = [&](int step) {
-        load_chunk<DT>(next, of_step(my_src, step), e0, a.n, a.vec & 1, ragged);
-        if constexpr (RDT != DQ_PHILOX) next_r.load(of_step(my_pool, step), lane * 4, (a.vec & 4) != 0);
+        const uint4 of = ranks[step];
+        const void *src = pointer((uint64_t)of.x | ((uint64_t)of.y << 32));
+        next_mean = __uint_as_float(of.z);
+        if (whole_loads)
+            next.load_anywhere(src, from);
+        else
+            load_chunk<DT>(next, src, e0, a.n, a.vec & 1, ragged);
+        if constexpr (POOL) next_r.load(pointer(pool_of_step[wave][half][step]), (lane & (kLanes - 1)) * N, (a.vec & 4) != 0);
     };
     fetch(0);
     uint32_t draws[4];
-    float lev[4], scale = 0.0f;
+    float lev[N], scale = 0.0f;
 #pragma unroll 1
     for (int step = 0; step < world; step++) {
-        const Raw4<DT> v = next;
-        Raw4<RDT> r = next_r;
-        const float mean = __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(my_mean), step));
+        RawPart<DT, N> v = next;
+        RawPart<RDT, N> r = next_r;
+        const float mean = next_mean;
         if (step + 1 < world) fetch(step + 1);
-        if constexpr (RDT == DQ_PHILOX) {
-            if ((step & 3) == 0) {
-                const int mine = step + (lane & 3);
-                int rank = chunk + mine; // (draws of steps beyond the last go unused)
-                if (rank >= world) rank -= world;
-                quad_words(RandKey{a.key.seed + (uint64_t)rank, (uint64_t)mine}, sc * 16 + (lane >> 2), lane, draws);
+        if (whole_loads && ragged) v.drop((int)min((int64_t)N, e0 - from));
+        if constexpr (!POOL) {
+            constexpr int kTogether = 16 / N; // lanes of a chunk
+            if ((step & (kTogether - 1)) == 0) {
+                const int mine = step + (lane & (kTogether - 1));
+                int of = my_chunk + mine; // (draws of steps beyond the last go unused)
+                if (of >= world) of -= world;
+                part_words<N>(RandKey{a.key.seed + (uint64_t)of, (uint64_t)mine}, my_sc * 16 + ((lane & (kLanes - 1)) / kTogether), lane, draws);
             }
-            r.w = draws[0];
-            draws[0] = draws[1]; draws[1] = draws[2]; draws[2] = draws[3];
+#pragma unroll
+            for (int k = 0; k < N / 4; k++) r.w[k] = draws[k];
+#pragma unroll
+            for (int k = 0; k < 4 - N / 4; k++) draws[k] = draws[k + N / 4];
         }
-        float x[4];
+        float x[N];
         center_loaded<DT>(x, v, a.wd, mean, e0, a.n, ragged);
         if (step > 0) { // the sum, in the element type
 #pragma unroll
-            for (int i = 0; i < 4; i++) x[i] = round_element<DT>(__builtin_fmaf(lev[i], scale, x[i]));
+            for (int i = 0; i < N; i++) x[i] = round_element<DT>(__builtin_fmaf(lev[i], scale, x[i]));
         }
         scale = quantize_chunk<MEE>(x, r, w, lev);
     }
-    Raw4<DT> out;
+    RawPart<DT, N> out;
     decode_with_mean<DT>(out, lev, scale, bf16_bits_to_f32(total_mean));
-    for (int rank = 0; rank < world; rank++) store_quarter<DT>(a.out[rank], out, e0, a.n, (a.vec & 2) != 0, ragged);
+    if (half >= have) return;
+    for (int rank = 0; rank < world; rank++) store_part<DT, N>(a.out[rank], out, e0, a.n, (a.vec & 2) != 0, ragged);
 }
 
-// Up to so many superchunks one per wave, beyond it four: the quads issue more per element (160 instructions per superchunk and
-// step against 90), and from two waves of ring_kernel per SIMD on (8,192 superchunks) that is what counts.  Kernel alone,
-// ring_kernel -> ring_quad_kernel, us: 8 ranks x 256 superchunks 12.2 -> 7.8 (AEE), 15.9 -> 8.9 (MEE), 19.5 -> 8.3 (AEE from pools);
-// x 8,192 20.4 -> 20.9, 27.0 -> 24.9, 26.2 -> 20.6, fp32 24.6 -> 23.2, 29.0 -> 23.9.  Two to five ranks with the least to do per
-// step -- AEE, values drawn, bf16 (fp32: two) -- have their line at five waves per SIMD, where a sixth would begin: 2 ranks x 4,900
-// 6.9 -> 7.0, x 5,300 6.8 -> 7.4, x 8,192 7.9 -> 9.0; 3 x 4,900 8.9 -> 8.3, x 6,900 9.3 -> 10.1; 5 x 4,900 12.4 -> 11.4, x 5,700 12.5
-// -> 13.2; fp32 2 x 4,900 6.8 -> 6.5, x 5,700 6.8 -> 7.2; but 6 x 6,500 17.3 -> 16.0, fp32 3 x 6,100 9.5 -> 9.1.
-constexpr int kQuadSuperchunks = 8192, kQuadSuperchunksShort = 5120;
-bool a_wave_each(int nsc, int world, int elem_bytes, bool mee, bool pooled)
+// How many elements a lane of the ring takes, 16 being ring_kernel.  Fewer issue more per element (160 instructions per superchunk and step
+// with four, 110 with eight, 95 with sixteen), and from five waves per SIMD on that is what counts.  Statistics and ring without a plan,
+// bf16, us, before there were eights (and with four elements loaded as in ring_parts_kernel's comment) -> four -> eight elements:
+//   2 ranks  x 4,000 superchunks 10.9 9.8 10.8 (AEE), 11.5 11.3 11.3 (MEE), x 5,300 12.5 12.1 11.8, 13.3 13.0 12.8, x 8,000 13.4 12.7 12.9,
+//            14.3 14.9 13.8, x 12,000 17.1 16.9 14.9, 18.5 18.7 17.4
+//   5 ranks  x 4,000 15.7 15.2 15.5, 16.7 16.5 16.6, x 5,000 18.1 17.4 18.2, 19.8 19.1 19.9, x 8,000 23.3 22.6 21.0, 25.5 25.3 23.1,
+//            x 12,000 30.8 29.5 26.4, 33.6 32.9 30.4
+//   8 ranks  x 2,000 (500,000 elements) 16.2 15.1 17.1, x 4,000 20.6 19.3 20.0, 22.3 21.0 21.7, x 5,000 24.0 22.6 24.0, 26.2 24.8 26.4,
+//            x 8,000 31.8 29.3 28.6, 34.9 32.8 31.3, x 12,000 40.8 37.5 34.9, 44.7 42.6 40.9
+// With fp32 elements eight are 32 bytes of a lane and its loads half lines: 5 ranks x 8,000 27.8 26.8 31.3, so fp32 stays with four; pools
+// do as well (bf16, 4 x 4,600 in AEE 18.0 17.8 30.3).
+constexpr int kFoursTo = 5120;
+
+// With lists from a plan, up to so many superchunks in parts.  bf16 with drawn values, plan and all, us, sixteen -> eight: 2 ranks x 12,000 17.7 ->
+// 17.1 (AEE), 20.0 -> 20.2 (MEE), x 16,000 19.5 -> 20.0; 5 x 16,000 35.9 -> 34.5, 40.2 -> 40.0, x 20,000 41.9 -> 40.0, 47.1 -> 45.6; 8 x 20,000
+// 54.8 -> 52.7, 63.1 -> 60.1.  The others, kernel alone, sixteen -> four: 8 ranks x 256 superchunks 12.2 -> 7.8 (AEE), 15.9 -> 8.9 (MEE),
+// 19.5 -> 8.3 (AEE from pools); x 8,192 from pools 26.2 -> 20.6, fp32 24.6 -> 23.2, 29.0 -> 23.9.  Two ranks in fp32 AEE with drawn values
+// have their line at five waves per SIMD: x 4,900 6.8 -> 6.5, x 5,700 6.8 -> 7.2.
+constexpr int kParts = 8192;
+int parts_to(int world, bool bf16, bool mee, bool pooled)
 {
-    const bool least = !mee && !pooled && world * elem_bytes < 12;
-    return nsc <= (least ? kQuadSuperchunksShort : kQuadSuperchunks);
+    if (pooled) return kParts;
+    if (bf16) return world >= 4 ? 20480 : 12288;
+    return !mee && world < 3 ? kFoursTo : kParts;
 }
 
-// Up to so many superchunks a ring with drawn values finds its groups itself (ring_quad_kernel, PLANS) in the place of a plan launch of 4 to
-// 6 us, which is also worth a wave per superchunk a little longer.  Statistics, (plan,) ring, us, with a plan -> without, AEE: 8 ranks x
-// 256 superchunks 12.9 -> 11.6, x 3,907 23.9 -> 19.6, x 8,192 31.5 -> 25.9, x 12,288 39.2 -> 36.0, x 16,384 46.0 -> 45.8; 4 x 3,907 16.3
-// -> 12.8, x 12,288 24.2 -> 21.7; 2 x 3,907 13.0 -> 10.4, x 12,288 16.7 -> 16.2, x 16,384 19.5 -> 20.7; MEE 8 x 3,907 25.4 -> 21.2, 2 x
-// 12,288 18.9 -> 17.9; fp32 8 x 3,907 27.7 -> 22.0, 2 x 12,288 20.8 -> 17.1.
-constexpr int64_t kPlansItself = 12288;
-static_assert(kPlansItself <= 0xffff, "a width's count over all superchunks is half a word (ring_quad_kernel, PLANS)");
+// Up to so many superchunks a ring with drawn values finds its groups itself (ring_parts_kernel, PLANS) in the place of a plan launch of 4 to
+// 6 us, which is also worth fewer elements per lane a little longer.  Statistics, (plan,) ring, us, with plan and ring_kernel -> without,
+// bf16: 2 ranks x 16,000 19.6 -> 18.2 (AEE), 21.5 -> 20.4 (MEE), x 24,000 24.4 -> 24.4, 27.6 -> 28.5; 3 x 16,000 25.3 -> 23.7, 27.5 -> 26.7,
+// x 24,000 31.5 -> 32.2, 35.5 -> 37.1; 8 x 16,000 48.6 -> 42.8, 53.9 -> 47.9, x 24,000 65.0 -> 61.8, 73.5 -> 70.0.  fp32, with four elements per
+// lane: 2 x 12,000 20.3 -> 19.3, 22.0 -> 20.4, x 16,000 24.5 -> 24.1, 24.5 -> 25.7; 5 x 16,000 49.7 -> 46.9, 51.1 -> 48.4; 8 x 16,000 78.5 ->
+// 74.9, 77.9 -> 75.8, x 20,000 96.9 -> 96.9, 98.9 -> 98.5.
+constexpr int kPlansItself = 20480, kPlansItself32 = 16384, kPlansItselfFew32 = 12288;
+static_assert(kPlansItself <= 0xffff, "a width's count over all superchunks is half a word (ring_parts_kernel, PLANS)");
 
 WidthRule make_rule(float u, const double *u_dev)
 {
@@ -899,29 +981,33 @@ static hipError_t run_ring(const RingDesc &d, bool mee, const MeeParams *mp, hip
     a.key = RandKey{d.seed, 0};
     a.wd = make_world_div(d.world, DT == DQ_F32 ? 4 : 2);
     a.widths = make_width_set(mp, mee);
-    const dim3 block(64 * kQuadWaves);
+    const auto parts = [&](auto plans) {
+        const auto go = [&](auto kernel, int here) {
+            return launch_with(kernel, dim3((unsigned)((a.nsc + here - 1) / here)), dim3(64 * kPartWaves), stream, a);
+        };
+        constexpr bool PLANS = decltype(plans)::value;
+        if constexpr (DT == DQ_BF16 && !POOL) {
+            if (a.nsc > kFoursTo)
+                return mee ? go(ring_parts_kernel<DT, RDT, true, 8, PLANS>, 2 * kPartWaves) : go(ring_parts_kernel<DT, RDT, false, 8, PLANS>, 2 * kPartWaves);
+        }
+        return mee ? go(ring_parts_kernel<DT, RDT, true, 4, PLANS>, kPartWaves) : go(ring_parts_kernel<DT, RDT, false, 4, PLANS>, kPartWaves);
+    };
     if constexpr (!POOL) {
         if (d.tile_widths) {
             a.more = FromTileWidths{d.tile_widths, d.work, make_rule(d.u, d.u_dev)};
-            const dim3 grid((unsigned)((a.nsc + kQuadWaves - 1) / kQuadWaves));
-            return mee ? launch_with(ring_quad_kernel<DT, RDT, true, true>, grid, block, stream, a)
-                       : launch_with(ring_quad_kernel<DT, RDT, false, true>, grid, block, stream, a);
+            return parts(std::integral_constant<bool, true>());
         }
     }
-    if (a_wave_each(a.nsc, d.world, DT == DQ_F32 ? 4 : 2, mee, POOL)) {
-        const dim3 grid((unsigned)((a.nsc + kQuadWaves - 1) / kQuadWaves));
-        return mee ? launch_with(ring_quad_kernel<DT, RDT, true>, grid, block, stream, a)
-                   : launch_with(ring_quad_kernel<DT, RDT, false>, grid, block, stream, a);
-    }
+    if (a.nsc <= parts_to(d.world, DT == DQ_BF16, mee, POOL)) return parts(std::integral_constant<bool, false>());
     // every run rounds its superchunks per ring chunk up to whole tiles
     const dim3 grid((unsigned)(a.nsc / (kRowsPerWave * d.world) + 4), (unsigned)d.world);
     return mee ? launch_with(ring_kernel<DT, RDT, true>, grid, dim3(64), stream, a)
                : launch_with(ring_kernel<DT, RDT, false>, grid, dim3(64), stream, a);
 }
 
-bool ring_plans_itself(int64_t n)
+bool ring_plans_itself(int64_t n, int world, int dtype)
 {
-    return (n + 255) / 256 <= kPlansItself;
+    return (n + 255) / 256 <= (dtype == DQ_BF16 ? kPlansItself : (world < 4 ? kPlansItselfFew32 : kPlansItself32));
 }
 
 hipError_t launch_ring(const RingDesc &d, int dtype, bool mee, const MeeParams *mp, hipStream_t stream)

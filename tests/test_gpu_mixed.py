@@ -805,6 +805,36 @@ def test_ranks_on_either_side_of_the_lines_of_a_superchunk_per_wave(capi, W, n, 
     test_ranks_in_registers_equal_the_ring_in_steps(capi, W, n, dt)
 
 
+@pytest.mark.parametrize("W,n,dt", [
+    (2, 256 * 5121 - 255, torch.bfloat16), (3, 256 * 5122 - 250, torch.bfloat16), (4, 256 * 5123 - 247, torch.bfloat16),
+    (7, 256 * 5127 - 5, torch.bfloat16), (2, 256 * 12288 - 1, torch.bfloat16), (3, 256 * 12289, torch.bfloat16),
+    (4, 256 * 20480 - 13, torch.bfloat16), (5, 256 * 20481 - 13, torch.bfloat16)])
+def test_rings_of_eight_elements_per_lane(capi, W, n, dt):
+    """bf16 with the values drawn, from 5,121 superchunks on: two superchunks of different widths and first ranks per wave, the last wave
+    with one or both of them, the vector's end at every place in a lane's eight; lists to 12,288 or 20,480 superchunks"""
+    test_ranks_in_registers_equal_the_ring_in_steps(capi, W, n, dt)
+
+
+@pytest.mark.parametrize("W,n,dt", [
+    (2, 256 * 5120 - 254, torch.bfloat16), (2, 256 * 5121 - 6, torch.bfloat16), (2, 256 * 20480 - 3, torch.bfloat16),
+    (2, 256 * 20480 + 1, torch.bfloat16), (3, 256 * 12288 + 3, torch.float32), (4, 256 * 16384 - 2, torch.float32), (4, 256 * 16384 + 1, torch.float32)])
+def test_lines_of_the_rings_without_lists(capi, W, n, dt):
+    test_rings_without_lists(capi, W, n, dt)
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+def test_ends_inside_a_lane_of_a_short_ring(capi, dt):
+    """vectors of one to nine elements, and every end in the last superchunk's first and last lanes"""
+    from dynamiq_sigcomm_artifact_amd.dynamiq_pipeline import _single_pass_in_steps, dynamic_bitrate_allreduce_single_pass
+    g = torch.Generator(device=DEV).manual_seed(17)
+    whole = [torch.randn(256 * 3, generator=g, device=DEV).to(dt) for _ in range(3)]
+    for n in list(range(1, 10)) + [256 + k for k in range(1, 10)] + [768 - k for k in range(10)]:
+        vecs = [v[:n].clone() for v in whole]
+        outs, _, _ = dynamic_bitrate_allreduce_single_pass(vecs, 6.0, strategy=2, seed=11)
+        ref, _, _ = _single_pass_in_steps(vecs, 6.0, 2, 11, None, {}, None, None)
+        assert all(torch.equal(bits_t(x), bits_t(y)) for x, y in zip(outs, ref)), n
+
+
 @pytest.mark.parametrize("W,n,dt,offset", [
     (8, 1024 * 2048, torch.bfloat16, 0),           # a tile per wave of the statistics
     (8, 1024 * 2048 + 1, torch.bfloat16, 0),
