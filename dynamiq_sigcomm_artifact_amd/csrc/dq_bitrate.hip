@@ -36,7 +36,8 @@ __global__ __launch_bounds__(kHistThreads) void norm_histogram_kernel(const uint
 // probes asks for up to eight values of u at once,
 // one pair of waves each: the seven midpoints of the next three steps of the bisection, or the next eight corrections, which
 // all follow from the first probe's deficit.  The walk through them is the reference's, probe by probe.  The first round's
-// thresholds are found while the histogram is on its way.
+// thresholds are found while the histogram is on its way, those of a correction by all waves in one round of 0.5 us (three rounds in two
+// waves: 1.2).  What is left of 4.0 us (4.8 with zeros written over zeros, and summed): 2.9 until one CU has the 128 KB.
 constexpr int kBins = 32768;                     // >= kNanBin + 1
 constexpr int kSlabs = kBins / (4 * kSearchThreads);
 constexpr int kSearchWaves = kSearchThreads / 64;
@@ -69,40 +70,31 @@ __global__ __launch_bounds__(kSearchThreads) void bitrate_search_kernel(uint32_t
     __shared__ __attribute__((aligned(8))) uint32_t part[kSlabs][kSearchWaves];
     __shared__ uint32_t nans;
     __shared__ uint32_t at_least[2][kProbes]; // norms of width >= 4, >= 8
+    __shared__ __attribute__((aligned(16))) uint32_t below[2][kProbes]; // patterns of the window below the width
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
 
-    if (prev_u_dev) prev_u = *prev_u_dev; // (the first load: waited for alone; read by every thread long before thread 0 writes out[])
+    // (the first load, without a branch in front of the others; read by every thread long before thread 0 writes out[])
+    const double read_u = *(prev_u_dev ? prev_u_dev : reinterpret_cast<const double *>(hist));
     uint4 v[kSlabs]; // bins 4 (t + 1024 k) ..
-    // (read, then left zeroed for the next accumulation)
-    if ((reinterpret_cast<uintptr_t>(hist) & 15) == 0) {
-        uint4 *h4 = reinterpret_cast<uint4 *>(hist);
+    const bool whole = (reinterpret_cast<uintptr_t>(hist) & 15) == 0;
+    if (whole) {
+        const uint4 *h4 = reinterpret_cast<const uint4 *>(hist);
 #pragma unroll
         for (int k = 0; k < kSlabs; k++) v[k] = h4[t + kSearchThreads * k];
-#pragma unroll
-        for (int k = 0; k < kSlabs; k++) h4[t + kSearchThreads * k] = make_uint4(0u, 0u, 0u, 0u);
     } else {
 #pragma unroll
         for (int k = 0; k < kSlabs; k++) {
-            uint32_t *h = hist + 4 * (t + kSearchThreads * k);
+            const uint32_t *h = hist + 4 * (t + kSearchThreads * k);
             v[k] = make_uint4(h[0], h[1], h[2], h[3]);
-            h[0] = h[1] = h[2] = h[3] = 0u;
         }
     }
+    if (prev_u_dev) prev_u = read_u;
     // the thresholds of a value of u, for the wave's share of them; they need nothing of the histogram, so those of the first
     // round are found while it is on its way
     const double u_min = -10.0, u_max = 60.0, tol = 0.1;
     const int pair = wave >> 1;
     const auto find = [&](double mine) {
-        const float u = (float)mine;
-        const int64_t width = (wave & 1) ? 8 : 4;
-        int p = kMaxPattern + 1;
-        const int a = first_width_probe(u, -1, 512, lane, width);
-        if (a < 64) {
-            const int lo = -1 + 512 * a;
-            const int lo2 = lo + 8 * first_width_probe(u, lo, 8, lane, width);
-            p = lo2 + 1 + first_width_probe(u, lo2, 1, lane, width);
-        }
-        return p;
+        return width_threshold((float)mine, lane, (wave & 1) ? 8 : 4);
     };
     // the midpoint of this pair's node below [l, h]
     const auto node_mid = [&](double l, double h) {
@@ -115,21 +107,47 @@ __global__ __launch_bounds__(kSearchThreads) void bitrate_search_kernel(uint32_t
         return mid;
     };
     const double start = __builtin_fmax(u_min, __builtin_fmin(u_max, prev_u));
-    int p_first = 0;
-    if (mode == 0 || pair == 0) p_first = find(mode == 0 ? (pair == 0 ? u_max : node_mid(u_min, u_max)) : start);
+    // A correction's first probe is one value of u for all waves: eight of them look at 64 patterns each around either estimate, in one round.
+    int p_first = 0, window = 0;
+    if (mode == 0) {
+        p_first = find(pair == 0 ? u_max : node_mid(u_min, u_max));
+    } else {
+        const int64_t width = (wave & 1) ? 8 : 4;
+        window = min(max(width_near((float)start, width) - 256, 0), kMaxPattern - 511);
+        const uint64_t under = __builtin_amdgcn_ballot_w64(qbits_of_norm((uint32_t)(window + 64 * pair + lane), (float)start) < width);
+        if (lane == 0) below[wave & 1][pair] = (uint32_t)__popcll(under);
+    }
 #pragma unroll
     for (int k = 0; k < kSlabs; k++) {
+        // Of the 128 times 256 bins most are empty, and nothing is done for those: no zeros to memory or to LDS, no sum over the wave.
         const int p = 4 * (t + kSearchThreads * k);
-        static_assert(kMaxPattern % 4 == 0 && kNanBin == kMaxPattern + 1, "infinity and the NaN norms share a load");
-        if (p >= kMaxPattern) {
-            if (p == kMaxPattern) nans = v[k].y;
-            v[k] = make_uint4(p == kMaxPattern ? v[k].x : 0u, 0u, 0u, 0u);
+        const bool some = (v[k].x | v[k].y | v[k].z | v[k].w) != 0u;
+        uint32_t sum = 0;
+        if (p == kMaxPattern) nans = v[k].y;
+        if (__builtin_amdgcn_ballot_w64(some) != 0) {
+            if (some) { // (read, then left zeroed for the next accumulation)
+                uint32_t *h = hist + p;
+                if (whole)
+                    *reinterpret_cast<uint4 *>(h) = make_uint4(0u, 0u, 0u, 0u);
+                else
+                    h[0] = h[1] = h[2] = h[3] = 0u;
+            }
+            static_assert(kMaxPattern % 4 == 0 && kNanBin == kMaxPattern + 1, "infinity and the NaN norms share a load");
+            if (p >= kMaxPattern) v[k] = make_uint4(p == kMaxPattern ? v[k].x : 0u, 0u, 0u, 0u);
+            reinterpret_cast<uint4 *>(bins)[t + kSearchThreads * k] = v[k];
+            sum = wave_sum(v[k].x + v[k].y + v[k].z + v[k].w);
         }
-        reinterpret_cast<uint4 *>(bins)[t + kSearchThreads * k] = v[k];
-        const uint32_t sum = wave_sum(v[k].x + v[k].y + v[k].z + v[k].w);
         if (lane == 0) part[k][wave] = sum;
     }
     __syncthreads();
+    if (mode != 0 && pair == 0) {
+        static_assert(kProbes == 8, "the window's 512 patterns");
+        const uint4 b0 = reinterpret_cast<const uint4 *>(below[wave & 1])[0], b1 = reinterpret_cast<const uint4 *>(below[wave & 1])[1];
+        const int count = __builtin_amdgcn_readfirstlane((int)(b0.x + b0.y + b0.z + b0.w + b1.x + b1.y + b1.z + b1.w));
+        p_first = window + count;
+        if (!((count > 0 || window == 0) && (count < 512 || window + 511 == kMaxPattern)))
+            p_first = width_threshold_anywhere((float)start, lane, (wave & 1) ? 8 : 4);
+    }
     // entry (k, w) of part is the sum of the 256 bins from 256 (16 k + w) on; lane l of each wave holds entries 2 l and 2 l + 1
     static_assert(kSlabs * kSearchWaves == 128, "two entries per lane");
     const uint2 entries = reinterpret_cast<const uint2 *>(&part[0][0])[lane];
@@ -137,19 +155,22 @@ __global__ __launch_bounds__(kSearchThreads) void bitrate_search_kernel(uint32_t
     // norms of pattern >= p: the entries behind p's, and what lies in p's own
     const auto count_from = [&](int p) {
         if (p > kMaxPattern) return 0u;
-        const int e = p >> 8, first = 4 * lane, from = p & 255;
-        const uint4 q = reinterpret_cast<const uint4 *>(bins)[64 * e + lane];
+        const int e = __builtin_amdgcn_readfirstlane(p >> 8), first = 4 * lane, from = p & 255;
         uint32_t sum = (2 * lane > e ? entries.x : 0u) + (2 * lane + 1 > e ? entries.y : 0u);
-        sum += (first >= from ? q.x : 0u) + (first + 1 >= from ? q.y : 0u);
-        sum += (first + 2 >= from ? q.z : 0u) + (first + 3 >= from ? q.w : 0u);
+        // (an empty entry's bins are not in the LDS)
+        if (__builtin_amdgcn_readlane((int)((e & 1) ? entries.y : entries.x), e >> 1) != 0) {
+            const uint4 q = reinterpret_cast<const uint4 *>(bins)[64 * e + lane];
+            sum += (first >= from ? q.x : 0u) + (first + 1 >= from ? q.y : 0u);
+            sum += (first + 2 >= from ? q.z : 0u) + (first + 3 >= from ? q.w : 0u);
+        }
         return wave_sum(sum);
     };
 
     // every thread evaluates the same doubles, so the control flow below is uniform without a broadcast
     int probes = 0;
     // one round: waves 2 k and 2 k + 1 hold the thresholds of candidate k
-    const auto publish = [&](int p) {
-        __syncthreads(); // the previous round has been read
+    const auto publish = [&](int p, bool again) {
+        if (again) __syncthreads(); // the previous round has been read
         const uint32_t n = count_from(p);
         if (lane == 0) at_least[wave & 1][wave >> 1] = n;
         __syncthreads();
@@ -169,7 +190,7 @@ __global__ __launch_bounds__(kSearchThreads) void bitrate_search_kernel(uint32_t
         double low = u_min, high = u_max, best_u = high, best_avg = 0.0, best_delta = 0.0;
         bool done = false, first = true;
         for (int it = 0; it < 32 && !done;) {
-            publish(first ? p_first : find(pair == 0 ? high : node_mid(low, high)));
+            publish(first ? p_first : find(pair == 0 ? high : node_mid(low, high)), !first);
             if (first) {
                 const Probe r = result(0);
                 best_avg = r.avg;
@@ -198,7 +219,7 @@ __global__ __launch_bounds__(kSearchThreads) void bitrate_search_kernel(uint32_t
         res_u = best_u; res_avg = best_avg; res_delta = best_delta;
     } else {
         // comm_hooks.py:117-139
-        publish(p_first);
+        publish(p_first, false);
         Probe r = result(0);
         res_u = start; res_avg = r.avg; res_delta = r.delta;
         if (!(__builtin_fabs(r.delta) <= tol)) {
@@ -208,7 +229,7 @@ __global__ __launch_bounds__(kSearchThreads) void bitrate_search_kernel(uint32_t
             for (int it = 0; it < 32 && !done; it += kProbes) {
                 double mine = step;
                 for (int k = 0; k < pair; k++) mine *= 0.5;
-                publish(find(__builtin_fmax(u_min, __builtin_fmin(u_max, start + mine))));
+                publish(find(__builtin_fmax(u_min, __builtin_fmin(u_max, start + mine))), true);
                 for (int k = 0; k < kProbes && !done; k++) {
                     const double cand = __builtin_fmax(u_min, __builtin_fmin(u_max, start + step));
                     r = result(k);

@@ -55,20 +55,42 @@ __device__ __forceinline__ int first_width_probe(float u, int lo, int step, int 
     return hit ? __builtin_ctzll(hit) : 64;
 }
 
+// Where the score scale log2(F) + u of the rule is the target.  The rule changes its width within 0.074 of there (width_class_of_norm), 71
+// patterns.  (A NaN gives some pattern, as does what lies beyond binary32: who starts here looks at the widths around it.)
+__device__ __forceinline__ int width_near(float u, int64_t target)
+{
+    return (int)(__float_as_uint(__builtin_amdgcn_exp2f(((float)target - u) * (float)(512.0 / 17.0 / 4.0))) >> 16) & 0x7fff;
+}
+
+// The smallest pattern of width >= target (kMaxPattern + 1: none), for one wave, from anywhere: three rounds of probes
+__device__ __forceinline__ int width_threshold_anywhere(float u, int lane, int64_t target)
+{
+    const int a = first_width_probe(u, -1, 512, lane, target);
+    if (a >= 64) return kMaxPattern + 1;
+    const int from = -1 + 512 * a, next = from + 8 * first_width_probe(u, from, 8, lane, target);
+    return next + 1 + first_width_probe(u, next, 1, lane, target);
+}
+
+// The same: two rounds, a round being a chain of 0.4 us, on the 256 patterns around the estimate; three where it is not there
+__device__ __forceinline__ int width_threshold(float u, int lane, int64_t target)
+{
+    const int lo = min(max(width_near(u, target) - 128, 0), kMaxPattern - 255);
+    const int a = first_width_probe(u, lo - 1, 4, lane, target); // patterns lo + 3, lo + 7, ..
+    if (a < 64 || lo + 255 == kMaxPattern) {
+        if (a >= 64) return kMaxPattern + 1;
+        const int from = lo + 4 * a; // one of from .. from + 3 is the first, unless it is even before those
+        const int f = first_width_probe(u, max(from - 2, -1), 1, lane, target);
+        if (f > 0 || from == 0) return max(from - 1, 0) + f;
+    }
+    return width_threshold_anywhere(u, lane, target);
+}
+
 // wave 0 finds thr[0] = the smallest pattern of width >= 4, wave 1 thr[1] = that of width 8
 // (kMaxPattern + 1 when no pattern reaches it); other waves do nothing.  No barrier inside.
 __device__ __forceinline__ void width_thresholds(float u, int *thr, int wave, int lane)
 {
     if (wave > 1) return;
-    const int64_t target = wave == 0 ? 4 : 8;
-    int t = kMaxPattern + 1;
-    const int a = first_width_probe(u, -1, 512, lane, target);
-    if (a < 64) {
-        const int lo = -1 + 512 * a;
-        const int b = first_width_probe(u, lo, 8, lane, target);
-        const int lo2 = lo + 8 * b;
-        t = lo2 + 1 + first_width_probe(u, lo2, 1, lane, target);
-    }
+    const int t = width_threshold(u, lane, wave == 0 ? 4 : 8);
     if (lane == 0) thr[wave] = t;
 }
 

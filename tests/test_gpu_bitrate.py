@@ -127,6 +127,19 @@ def test_search_equals_the_oracle_on_the_norms(capi, oracle, name):
             assert got == tuple(want2), (name, target, prev, got, want2)
 
 
+def test_thresholds_of_every_offset(capi, oracle):
+    """every pattern once, so that a threshold one pattern off changes the average: corrections from offsets all over the range, whose
+    thresholds lie at any place of the window that is looked at first, or beyond the patterns"""
+    from dynamiq_sigcomm_artifact_amd.bitrate import NormHistogram
+    bits = np.arange(MAXP + 1, dtype=np.uint16)
+    stats = _stats(torch.from_numpy(bits.view(np.int16)).view(torch.bfloat16))
+    h = NormHistogram(DEV)
+    for prev in list(np.linspace(-10.0, 60.0, 57)) + [3.999, 4.0, 7.97, 8.0, 12.5, 20.7, 24.8, 25.1]:
+        h.add(stats)
+        assert h.adjust_u(float(prev), 4.375) == tuple(oracle.dynamic_bitrate_adjust_u([bits], float(prev), 4.375)), prev
+        assert int(h.hist.abs().sum()) == 0
+
+
 def test_search_equals_the_torch_op_sequence_on_the_device():
     """the reference's own functions as mirrored in bitrate.py, on device tensors (the scalar u enters the add in
     binary32 there, as in the reference's CUDA run)"""
