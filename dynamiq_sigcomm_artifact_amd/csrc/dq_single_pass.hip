@@ -16,7 +16,7 @@
 // Measured, start -> now (bit-identical results): 8 ranks x 124,439,808 bf16 elements 2,896 -> 1,070 us per all-reduce (one
 // launch per rank and ring step, packed streams and their exchange copies, against three launches whose traffic is the
 // vectors alone), 8 x 1,000,003 elements 1,488 -> 20 us (257 launches against 2), a step of nine 25 MB buckets on one rank
-// 252 -> 52 us (four launches per bucket on two streams against two launches per step, and the search for u).
+// 252 -> 50 us (four launches per bucket on two streams against two launches per step, and the search for u).
 //
 // Numerics: csrc/cuda_hadamard.cu:1257-1369 (centring, mean add), csrc/cuda_hierarchical_mee.cu:203-696 (codec),
 // testbed_evaluation/new_comm_hooks/ring_rdma.py:590-631 (order of the ring), comm_hooks.py:64-70 (widths).
@@ -157,13 +157,21 @@ __device__ __forceinline__ int last_at_most(const uint32_t *list, int count, uin
     return lo;
 }
 
+// The one-rank pass is bound by the vector ALU (470 instructions a tile, 504 before) with memory right behind it: a step of nine 25 MB
+// buckets 41 us at 5.2 TB/s.  So a tile's elements become numbers once, for the sums and for the quantiser, a row's results come from its
+// first lane without the LDS, and a whole tile leaves as the one run it is.  Whole calls, us: 1 x 30,761,978 in MEE 34.0 -> 32.1, 1 x
+// 1,761,978 8.2 -> 8.0; with the tally below, 11 buckets of 12.2 M in MEE 134 -> 128, nine of 3 M 31.2 -> 28.6.
+// lane 0 of the lane's row of sixteen
+__device__ __forceinline__ uint32_t of_row(uint32_t x) { return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x150, 0xf, 0xf, true); } // row_newbcast:0
+
 template <int DT, bool MEE, int MOST> __global__ __launch_bounds__(64) void roundtrip_kernel(RoundtripArgs<MOST> a)
 {
-    constexpr int kStage = 64 * Raw16<DT>::kSlots * 16;
-    __shared__ __attribute__((aligned(16))) uint8_t lds[StatsTile<DT>::BYTES > kStage ? StatsTile<DT>::BYTES : kStage];
+    constexpr int kSlots = Raw16<DT>::kSlots, kStage = 64 * kSlots * 16;
+    __shared__ __attribute__((aligned(16))) uint8_t lds[kFloatTileBytes > kStage ? kFloatTileBytes : kStage];
     __shared__ float levels[MEE ? kLevelCount : 1];
     const int lane = threadIdx.x, row = lane >> 4, j = lane & 15;
 
+    // (ahead of the elements' loads, behind which they would be loads of the lanes and wait for those)
     uint64_t step = a.step_dev ? *a.step_dev + a.step_more : 0;
     const float u = a.rule.u_dev ? (float)*a.rule.u_dev : a.rule.u;
     const int at = MOST == 1 ? 0 : last_at_most(a.first_tile, a.buckets, blockIdx.x);
@@ -171,36 +179,61 @@ template <int DT, bool MEE, int MOST> __global__ __launch_bounds__(64) void roun
     const int64_t n = b.n, nsc = (n + 255) >> 8;
     const int64_t sc0 = (int64_t)(blockIdx.x - a.first_tile[at]) * kRowsPerWave;
     if (sc0 >= nsc) return;
-    const int rows_here = (int)min((int64_t)kRowsPerWave, nsc - sc0);
-    const bool active = row < rows_here, ragged = (sc0 + kRowsPerWave) * 256 > n;
-    const int64_t sc = sc0 + min(row, rows_here - 1);
+    const bool ragged = (sc0 + kRowsPerWave) * 256 > n; // (and fewer than four superchunks, at times)
+    const int rows_here = ragged ? (int)min((int64_t)kRowsPerWave, nsc - sc0) : kRowsPerWave;
+    const bool active = row < rows_here;
+    const int64_t sc = sc0 + (ragged ? min(row, rows_here - 1) : row);
     const int64_t e0 = sc * 256 + j * 16;
 
     Raw16<DT> v;
     v.zero();
-    if (active) load_chunk<DT>(v, b.src, e0, n, b.vec != 0, ragged);
+    if (!ragged) {
+        v.load(b.src, e0, b.vec != 0);
+    } else if (active) {
+        load_chunk_guarded<DT>(v, b.src, e0, n);
+    }
     if (MEE) levels_to_lds(levels, lane);
     // the rounding stream's arithmetic while the elements are on their way
     Raw16<DQ_PHILOX> r;
     r.generate(RandKey{a.seed, b.step + step}, sc * 16 + j);
     r.pin();
 
+    float t[16];
+#pragma unroll
+    for (int i = 0; i < 16; i++) t[i] = v.get(i);
+    if (!a.wd.pow2) {
+        a.wd.divide(t);
+    } else if (a.wd.inv != 1.0f) {
+#pragma unroll
+        for (int i = 0; i < 16; i++) t[i] *= a.wd.inv;
+    }
     float sum, sq;
-    tile_sums<DT>(v, a.wd, lds, lane, sum, sq);
-    const float mean = __shfl(superchunk_mean(sum, sc * 256, n, ragged), lane & 48, 64);
-    const uint32_t norm = (uint32_t)__shfl((int)f32_to_bf16_bits(sq), lane & 48, 64);
+    float_tile_sums(t, reinterpret_cast<float *>(lds), lane, sum, sq);
+    const float mean = __uint_as_float(of_row(__float_as_uint(superchunk_mean(sum, sc * 256, n, ragged))));
+    const uint32_t norm = of_row(f32_to_bf16_bits(sq));
     const uint32_t mean_bits = f32_to_bf16_bits(mean);
     if (active && j == 0) b.stats[sc] = mean_bits | (norm << 16);
     if (sc0 == 0 && lane < 4) b.counts[lane] = 0; // (tally_kernel adds to them)
 
     const WidthRegs<MEE> w = width_regs<MEE>(a.widths, class_of_norm(norm, u, a.rule.thr), levels);
-    float x[16], lev[16];
-    center_loaded<DT>(x, v, a.wd, active ? mean : 0.0f, e0, n, ragged);
-    const float scale = quantize_chunk<MEE>(x, r, w, lev);
+    // (v / world - mean: center_loaded forms the same number, in one rounding or two)
+#pragma unroll
+    for (int i = 0; i < 16; i++) t[i] -= mean;
+    finish_centered<DT>(t, e0, n, ragged);
+    float lev[16];
+    const float scale = quantize_chunk<MEE>(t, r, w, lev);
     decode_with_mean<DT>(v, lev, scale, bf16_bits_to_f32(mean_bits));
     wave_lds_sync(); // the statistics' tile has been read
     stage_tile<DT>(v, reinterpret_cast<uint4 *>(lds), lane);
-    store_tile<DT>(b.out, v, reinterpret_cast<const uint4 *>(lds), sc, rows_here, n, b.vec != 0, lane);
+    if (!ragged && b.vec != 0) {
+        // the tile is one run
+        const uint4 *stage = reinterpret_cast<const uint4 *>(lds);
+        uint4 *to = reinterpret_cast<uint4 *>(static_cast<char *>(b.out) + sc0 * (kStage / kRowsPerWave)) + lane;
+#pragma unroll
+        for (int k = 0; k < kSlots; k++) stream_store(to + 64 * k, stage[swz(64 * k + lane)]);
+    } else {
+        store_tile<DT>(b.out, v, reinterpret_cast<const uint4 *>(lds), sc, rows_here, n, b.vec != 0, lane);
+    }
 }
 
 struct TallyBucket {
@@ -222,7 +255,8 @@ template <int MOST> struct TallyArgs {
 // A workgroup takes kTallyBatch superchunks of one bucket.  A wave's norms are alike and meet in a few counters of the LDS, so the
 // counting is better spread over more workgroups: 209,716 norms with 8192 each 7.9 us, 4096 6.6, 2048 and 1024 6.4.  What is
 // left is a chain of latencies; clearing 64 KB of counters, going over them afterwards and searching the two thresholds for two
-// norms per thread were the longest links (6.0 us; 4.6 with the counters in range alone and the rule applied to each norm).
+// norms per thread were the longest links (6.0 us; 4.6 with the counters in range alone and the rule applied to each norm), then a search
+// for the bucket by halving, a load per step, and a barrier of the widths' own.
 // (Clearing each norm's own counter and leaving it to whoever found it at 0 spares a barrier, but scatters the atomics on memory:
 // 4.8 us here, and 42.9 instead of 12.1 for batches of 8192 of 3,000,000 norms.)
 constexpr int kTallyThreads = 1024, kTallyBatch = 2048;
@@ -233,13 +267,14 @@ constexpr int kTallyThreads = 1024, kTallyBatch = 2048;
 // (of which a bucket may hold many) and NaN are counted apart.
 template <int PER> struct PatternBatch {
     uint32_t low, high; // words of counters in use
-    uint32_t zeros, nans;
+    uint32_t zeros_nans; // of wave lane & 15
 
-    __device__ __forceinline__ void begin(const uint32_t (&pattern)[PER], int have, uint32_t *local, uint4 *wave_seen)
+    // mine: what else the waves have to tell one another (n4 | n8 << 16); returned for wave lane & 15
+    __device__ __forceinline__ uint32_t begin(const uint32_t (&pattern)[PER], int have, uint32_t mine, uint32_t *local, uint4 *wave_seen)
     {
         const int t = threadIdx.x, lane = t & 63;
         uint32_t top = 0, under = 0; // the greatest bin, the complement of the least
-        zeros = nans = 0;
+        uint32_t zeros = 0, nans = 0;
 #pragma unroll
         for (int k = 0; k < PER; k++) {
             const uint32_t bin = (uint32_t)bin_of(pattern[k]);
@@ -251,16 +286,16 @@ template <int PER> struct PatternBatch {
         }
         top = wave_max_upward(top);
         under = wave_max_upward(under);
-        if (lane == 63) wave_seen[t >> 6] = make_uint4(top, under, zeros, nans);
+        if (lane == 63) wave_seen[t >> 6] = make_uint4(top, under, zeros | (nans << 16), mine);
         __syncthreads();
         static_assert(kTallyThreads / 64 == 16, "a row of 16 lanes holds a value of every wave");
         const uint4 seen = wave_seen[lane & 15];
         high = (uint32_t)__builtin_amdgcn_readlane((int)wave_max_upward(seen.x), 63) >> 1;
         low = ~(uint32_t)__builtin_amdgcn_readlane((int)wave_max_upward(seen.y), 63) >> 1; // (no bin at all: beyond every word)
-        zeros = seen.z;
-        nans = seen.w;
+        zeros_nans = seen.z;
         for (uint32_t w = low + t; w <= high; w += kTallyThreads) local[w] = 0u;
         __syncthreads();
+        return seen.w;
     }
 
     __device__ __forceinline__ void add(const uint32_t (&pattern)[PER], int have, uint32_t *local) const
@@ -281,8 +316,8 @@ template <int PER> struct PatternBatch {
             if (pair >> 16) atomicAdd(&hist[2 * w + 1], pair >> 16);
         }
         if (threadIdx.x < 16) { // an entry of wave_seen each
-            if (zeros) atomicAdd(&hist[0], zeros);
-            if (nans) atomicAdd(&hist[kNanBin], nans);
+            if (zeros_nans & 0xffffu) atomicAdd(&hist[0], zeros_nans & 0xffffu);
+            if (zeros_nans >> 16) atomicAdd(&hist[kNanBin], zeros_nans >> 16);
         }
     }
 };
@@ -290,48 +325,73 @@ template <int PER> struct PatternBatch {
 template <bool HIST, int MOST> __global__ __launch_bounds__(kTallyThreads) void tally_kernel(TallyArgs<MOST> a)
 {
     __shared__ uint32_t local[HIST ? kHistWords : 1];
-    __shared__ uint4 wave_seen[HIST ? kTallyThreads / 64 : 1];
-    __shared__ uint32_t total[2];
+    __shared__ uint4 wave_seen[kTallyThreads / 64];
     const int lane = threadIdx.x & 63;
-    const int at = MOST == 1 ? 0 : last_at_most(a.first_block, a.buckets, blockIdx.x);
-    const TallyBucket b = a.bucket[at];
-    const int64_t begin = (int64_t)(blockIdx.x - a.first_block[at]) * kTallyBatch;
-    const int64_t end = min(begin + (int64_t)kTallyBatch, b.nsc);
+    TallyBucket b;
+    uint32_t first = 0;
+    if constexpr (MOST == 1) {
+        b = a.bucket[0];
+    } else {
+        // A lane per bucket, and the right lane's: one load's time.  (Behind the last bucket first_block is greater than any block.)
+        static_assert(MOST <= 64, "a bucket per lane");
+        const int k = min(lane, MOST - 1);
+        const uint32_t starts = a.first_block[k];
+        const TallyBucket mine = a.bucket[k];
+        const int at = __popcll(__builtin_amdgcn_ballot_w64(lane < MOST && starts <= blockIdx.x)) - 1;
+        const auto of = [at](uint64_t x) {
+            const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)x, at), hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(x >> 32), at);
+            return (uint64_t)lo | ((uint64_t)hi << 32);
+        };
+        // (addresses of memory, which the compiler knows of an argument but not of a lane's register)
+        b.stats = (const uint16_t *)(const __attribute__((address_space(1))) uint16_t *)of(reinterpret_cast<uint64_t>(mine.stats));
+        b.counts = (int32_t *)(__attribute__((address_space(1))) int32_t *)of(reinterpret_cast<uint64_t>(mine.counts));
+        b.nsc = (int64_t)of((uint64_t)mine.nsc);
+        first = (uint32_t)__builtin_amdgcn_readlane((int)starts, at);
+    }
+    const int64_t begin = (int64_t)(blockIdx.x - first) * kTallyBatch;
     constexpr int kPer = kTallyBatch / kTallyThreads;
     // (the last norm's address beyond the end: behind a comparison each, the loads would wait for one another)
-    const int have = (int)(end - begin);
+    const int have = (int)min((int64_t)kTallyBatch, b.nsc - begin);
     const uint16_t *mine = b.stats + 2 * begin + 1;
     uint32_t norm[kPer];
 #pragma unroll
     for (int k = 0; k < kPer; k++) norm[k] = mine[2 * min(k * kTallyThreads + (int)threadIdx.x, have - 1)];
     const float u = a.rule.u_dev ? (float)*a.rule.u_dev : a.rule.u;
-    if (threadIdx.x < 2) total[threadIdx.x] = 0u;
-    PatternBatch<kPer> batch;
-    if (HIST) {
-        batch.begin(norm, have, local, wave_seen);
-        batch.add(norm, have, local);
-    } else {
-        __syncthreads();
-    }
-    uint32_t n8 = 0, n4 = 0;
+    uint32_t counts = 0; // of the wave: n4 | n8 << 16
 #pragma unroll
     for (int k = 0; k < kPer; k++) {
         const bool in = k * kTallyThreads + (int)threadIdx.x < have;
         const int c = a.rule.thr[0] >= 0 ? class_of_norm(norm[k], u, a.rule.thr) : width_class_of_norm(norm[k], u);
-        n8 += (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(in && c == 0));
-        n4 += (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(in && c == 1));
+        counts += (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(in && c == 1)) + ((uint32_t)__popcll(__builtin_amdgcn_ballot_w64(in && c == 0)) << 16);
     }
-    if (lane == 0 && n8) atomicAdd(&total[0], n8);
-    if (lane == 0 && n4) atomicAdd(&total[1], n4);
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        const int c8 = (int)total[0], c4 = (int)total[1], c2 = have - c8 - c4;
-        if (c8) atomicAdd(&b.counts[0], c8);
-        if (c4) atomicAdd(&b.counts[1], c4);
-        if (c2) atomicAdd(&b.counts[2], c2);
-        if (blockIdx.x == 0 && a.step_dev && a.step_more) *a.step_dev += a.step_more;
+    static_assert(kTallyBatch <= 0xffff, "two counts in a word");
+    PatternBatch<kPer> batch;
+    if (HIST) {
+        counts = batch.begin(norm, have, counts, local, wave_seen);
+    } else {
+        if (lane == 0) wave_seen[threadIdx.x >> 6].w = counts;
+        __syncthreads();
+        counts = wave_seen[lane & 15].w;
     }
-    if (HIST) batch.flush(a.hist, local);
+    if (HIST) {
+        batch.add(norm, have, local);
+        __syncthreads();
+        batch.flush(a.hist, local);
+    }
+    if (threadIdx.x >= kTallyThreads - 64) { // (the wave with the least to flush)
+        // sums over the row of sixteen lanes, a wave's each, in the last of them
+        counts += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)counts, 0x111, 0xf, 0xf, true); // row_shr:1, 2, 4, 8
+        counts += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)counts, 0x112, 0xf, 0xf, true);
+        counts += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)counts, 0x114, 0xf, 0xf, true);
+        counts += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)counts, 0x118, 0xf, 0xf, true);
+        if (lane == 15) {
+            const int c8 = (int)(counts >> 16), c4 = (int)(counts & 0xffffu), c2 = have - c8 - c4;
+            if (c8) atomicAdd(&b.counts[0], c8);
+            if (c4) atomicAdd(&b.counts[1], c4);
+            if (c2) atomicAdd(&b.counts[2], c2);
+            if (blockIdx.x == 0 && a.step_dev && a.step_more) *a.step_dev += a.step_more;
+        }
+    }
 }
 
 // ---- W ranks --------------------------------------------------------------------------------------------
@@ -863,6 +923,7 @@ static hipError_t run_roundtrip(const RoundtripDesc *desc, int count, int world,
     TallyArgs<MOST> t;
     static_assert(MOST > kFewBuckets || sizeof(a) <= 1024, "see RoundtripArgs");
     memset(&t, 0, sizeof(t));
+    memset(t.first_block, 0xff, sizeof(t.first_block));
     memset(&a, 0, offsetof(RoundtripArgs<MOST>, rule));
     uint32_t tiles = 0, blocks = 0;
     for (int k = 0; k < MOST; k++) {

@@ -518,6 +518,23 @@ __device__ __forceinline__ void load_chunk(RV &v, const void *src, int64_t e0, i
         load_chunk_guarded<DT>(v, src, e0, n);
 }
 
+// zeros at and beyond element n of the vector, and the precision of the element type
+template <int DT, int N> __device__ __forceinline__ void finish_centered(float (&t)[N], int64_t e0, int64_t n, bool ragged)
+{
+    if (ragged) {
+        const int left = left_here(n, e0, N);
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            // (In place: as a selection the tiles that are not ragged copy every element.  The comparison that writes the mask may come
+            // directly before, and the two wait states between the two are the compiler's only for its own instructions.)
+            const uint64_t inside = __builtin_amdgcn_ballot_w64(i < left);
+            asm volatile("s_nop 1\n\tv_cndmask_b32_e64 %0, 0, %0, %1" : "+v"(t[i]) : "s"(inside));
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < N; i++) t[i] = round_element<DT>(t[i]);
+}
+
 // t = T(v / world - mean), zero at and beyond element n of the vector (center_chunk without its own loads)
 template <int DT, class RV>
 __device__ __forceinline__ void center_loaded(float (&t)[RV::kCount], const RV &v, const WorldDiv &wd, float mean, int64_t e0, int64_t n, bool ragged)
@@ -538,18 +555,7 @@ __device__ __forceinline__ void center_loaded(float (&t)[RV::kCount], const RV &
 #pragma unroll
         for (int i = 0; i < N; i++) t[i] -= mean;
     }
-    if (ragged) {
-        const int left = left_here(n, e0, N);
-#pragma unroll
-        for (int i = 0; i < N; i++) {
-            // (In place: as a selection the tiles that are not ragged copy every element.  The comparison that writes the mask may come
-            // directly before, and the two wait states between the two are the compiler's only for its own instructions.)
-            const uint64_t inside = __builtin_amdgcn_ballot_w64(i < left);
-            asm volatile("s_nop 1\n\tv_cndmask_b32_e64 %0, 0, %0, %1" : "+v"(t[i]) : "s"(inside));
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < N; i++) t[i] = round_element<DT>(t[i]);
+    finish_centered<DT>(t, e0, n, ragged);
 }
 
 // ---- statistics of a tile of four superchunks -----------------------------------------------------------
@@ -585,6 +591,26 @@ __device__ __forceinline__ void tile_sums(const Raw16<DT> &v, const WorldDiv &wd
     staged_tile_sums<DT>(wd, lds, lane, sum, sq);
 }
 
+// strides 64 .. 1 of the sums and the squares
+__device__ __forceinline__ void fold_tile_sums(float (&a)[8], float (&b)[8], float &sum, float &sq)
+{
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        a[k] += a[k + 4];
+        b[k] += b[k + 4];
+    }
+    sum = (a[0] + a[2]) + (a[1] + a[3]);
+    sq = (b[0] + b[2]) + (b[1] + b[3]);
+    sum += dpp_row_shift<0x108>(sum);
+    sq += dpp_row_shift<0x108>(sq);
+    sum += dpp_row_shift<0x104>(sum);
+    sq += dpp_row_shift<0x104>(sq);
+    sum += dpp_row_shift<0x102>(sum);
+    sq += dpp_row_shift<0x102>(sq);
+    sum += dpp_row_shift<0x101>(sum);
+    sq += dpp_row_shift<0x101>(sq);
+}
+
 // of the tile in LDS
 template <int DT> __device__ __forceinline__ void staged_tile_sums(const WorldDiv &wd, const uint8_t *lds, int lane, float &sum, float &sq)
 {
@@ -613,21 +639,33 @@ template <int DT> __device__ __forceinline__ void staged_tile_sums(const WorldDi
         a[k] = t[k] + t[k + 8];
         b[k] = t[k] * t[k] + t[k + 8] * t[k + 8];
     }
+    fold_tile_sums(a, b, sum, sq);
+}
+
+// The same where the lane has its elements as numbers, already divided by world, and needs them as such again: they go through the LDS in
+// binary32, which spares the kernel of one rank sixteen conversions and a second division.  The 16-byte pieces of a lane change
+// places by its number, so that eight lanes writing theirs touch 32 different banks.
+constexpr int kFloatRow = 256 + 16, kFloatTileBytes = 4 * kFloatRow * (int)sizeof(float);
+
+__device__ __forceinline__ void float_tile_sums(const float (&t)[16], float *lds, int lane, float &sum, float &sq)
+{
+    const int row = lane >> 4, j = lane & 15;
+    float *mine = lds + row * kFloatRow + j * 16;
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
-        a[k] += a[k + 4];
-        b[k] += b[k + 4];
+    for (int p = 0; p < 4; p++)
+        *reinterpret_cast<float4 *>(mine + 4 * (p ^ ((j >> 1) & 3))) = make_float4(t[4 * p], t[4 * p + 1], t[4 * p + 2], t[4 * p + 3]);
+    wave_lds_sync();
+    // element j of lane k's sixteen
+    float x[16];
+#pragma unroll
+    for (int k = 0; k < 16; k++) x[k] = lds[row * kFloatRow + 16 * k + (j ^ (4 * ((k >> 1) & 3)))];
+    float a[8], b[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        a[k] = x[k] + x[k + 8];
+        b[k] = x[k] * x[k] + x[k + 8] * x[k + 8];
     }
-    sum = (a[0] + a[2]) + (a[1] + a[3]);
-    sq = (b[0] + b[2]) + (b[1] + b[3]);
-    sum += dpp_row_shift<0x108>(sum);
-    sq += dpp_row_shift<0x108>(sq);
-    sum += dpp_row_shift<0x104>(sum);
-    sq += dpp_row_shift<0x104>(sq);
-    sum += dpp_row_shift<0x102>(sum);
-    sq += dpp_row_shift<0x102>(sq);
-    sum += dpp_row_shift<0x101>(sum);
-    sq += dpp_row_shift<0x101>(sq);
+    fold_tile_sums(a, b, sum, sq);
 }
 
 // the mean the reference divides out: sum / 256 exactly, or by the count of a ragged last superchunk
