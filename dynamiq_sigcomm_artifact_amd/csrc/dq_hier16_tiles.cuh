@@ -144,10 +144,10 @@ __device__ __forceinline__ void encode_store_run(const RV &v, const RR &r, const
     uint32_t w[RC::WORDS], q, ub;
     const uint32_t amax = v.absmax_bits();
     const bool lane_fast = amax <= kFastMaxBits && r.unit_interval();
-    if (__builtin_amdgcn_ballot_w64(!lane_fast) == 0)
-        chunk_encode_fast<NBITS, MEE>(v, r, amax, mp, w, q, ub);
-    else
+    if (DQ_UNLIKELY(__builtin_amdgcn_ballot_w64(!lane_fast) != 0))
         chunk_encode_guarded<NBITS, MEE>(v, r, mp, w, q, ub);
+    else
+        chunk_encode_fast<NBITS, MEE>(v, r, amax, mp, w, q, ub);
 
 #pragma unroll
     for (int p = 0; p < kRowsPerWave; p += WROWS) {
@@ -236,7 +236,7 @@ __device__ __forceinline__ void compress_tile(const void *__restrict__ src, cons
     Raw16<DT> v;
     Raw16<RDT> r;
     v.zero();
-    r.zero();
+    r.halves();
     const int64_t sc_src = row_id(rows, sc0 + min(row, rows_here - 1)); // every lane asks, for an entry of the list
     int64_t e0 = 0;
     float mean = 0.0f;

@@ -260,7 +260,7 @@ __global__ __attribute__((amdgpu_waves_per_eu(8, 8))) void rht_compress_kernel(c
         for (int i = 0; i < 16; i++) v.w[i] = __float_as_uint(mine[i] * a.scale);
     } else {
         v.zero();
-        r.zero();
+        r.halves();
     }
     __syncthreads();
     if (rows_here > 0)

@@ -121,7 +121,7 @@ __device__ __forceinline__ void tile16_compress(const void *__restrict__ src, ui
             r.load(rnd, (c0 + lane) * 16, vec & 2);
     } else {
         v.zero();
-        r.zero();
+        r.halves();
     }
 
     float a;
