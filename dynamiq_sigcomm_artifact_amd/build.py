@@ -27,7 +27,7 @@ LIB_PATH = os.path.join(PKG_DIR, LIB_NAME)
 HIP_SOURCES = [
     "dq_api.hip",
     "dq_scaling_generic.hip",
-    "dq_scaling_hier16.hip",
+    "dq_scaling_hier16.hip", "dq_scaling_hier16_short.hip",
     "dq_scaling_tile16.hip",
     "dq_grouping.hip", "dq_bitrate.hip", "dq_sort.hip",
     "dq_scaling_mixed.hip",

@@ -6,38 +6,39 @@
 // (fused decompress-accumulate-recompress).
 #pragma once
 
-#include "dq_tile16.cuh"
+#include "dq_parts.cuh"
 
 namespace dq {
 
 // ---- the math of one chunk ---------------------------------------------------------------------
 
-// decode 16 levels of one chunk: t = lev*sc (+ t when ADD)
-template <int NBITS, bool MEE, bool ADD>
-__device__ __forceinline__ void chunk_decode(const uint32_t (&w)[Rec<NBITS>::WORDS], uint32_t q, uint32_t unit_bits,
-                                             const float *table, float (&t)[16])
+// decode the levels that a lane has of a chunk, all 16 or a part: t = lev*sc (+ t when ADD)
+template <int NBITS, bool MEE, bool ADD, int N = 16>
+__device__ __forceinline__ void chunk_decode(const uint32_t (&w)[(N * NBITS + 31) / 32], uint32_t q, uint32_t unit_bits,
+                                             const float *table, float (&t)[N])
 {
     const float us = nonneg_scale(bf16_bits_to_f32(unit_bits));
     const float sc = nonneg_scale((float)q * us);
 #pragma unroll
-    for (int i = 0; i < 16; i++) {
+    for (int i = 0; i < N; i++) {
         const uint32_t code = words_get<NBITS>(w, i);
         const float lev = MEE ? table[code] : (float)((int)code - Rec<NBITS>::R);
         t[i] = ADD ? __builtin_fmaf(lev, sc, t[i]) : lev * sc;
     }
 }
 
-// general (guarded) quantiser of one chunk against its superchunk row
-template <int NBITS, bool MEE, class RV, class RR, class ARG>
+// general (guarded) quantiser of one chunk against its superchunk; a lane has N elements of the chunk
+template <int NBITS, bool MEE, int N = 16, class RV, class RR, class ARG>
 __device__ __forceinline__ void chunk_encode_guarded(const RV &v, const RR &r, const ARG &mp,
-                                                     uint32_t (&w)[Rec<NBITS>::WORDS], uint32_t &q, uint32_t &unit_bits)
+                                                     uint32_t (&w)[(N * NBITS + 31) / 32], uint32_t &q, uint32_t &unit_bits)
 {
     constexpr int R = Rec<NBITS>::R;
     float a = __builtin_fabsf(v.get(0));
 #pragma unroll
-    for (int i = 1; i < 16; i++) a = __builtin_fmaxf(a, __builtin_fabsf(v.get(i)));
+    for (int i = 1; i < N; i++) a = __builtin_fmaxf(a, __builtin_fabsf(v.get(i)));
+    a = chunk_max<N>(a);
     const float s = pos_scale(MEE ? a / pos_scale(mp.cmm) + 1e-7f : a / (float)R + 1e-7f);
-    const float g = pos_scale(row16_max(s));
+    const float g = pos_scale(superchunk_max<N>(s));
     unit_bits = f32_to_bf16_bits(pos_scale(g / 255.0f));
     const float unit = pos_scale(bf16_bits_to_f32(unit_bits));
     float ratio = pos_scale(s) / pos_scale(g) * 255.0f;
@@ -47,9 +48,9 @@ __device__ __forceinline__ void chunk_encode_guarded(const RV &v, const RR &r, c
     q = (uint32_t)qi;
     const float d = pos_scale(pos_scale((float)qi * unit));
 #pragma unroll
-    for (int k = 0; k < Rec<NBITS>::WORDS; k++) w[k] = 0;
+    for (int k = 0; k < (N * NBITS + 31) / 32; k++) w[k] = 0;
 #pragma unroll
-    for (int i = 0; i < 16; i++) {
+    for (int i = 0; i < N; i++) {
         float x = v.get(i) / d;
         if (MEE) x = mee_inverse_guarded(x, mp.c, mp.l2b);
         words_put<NBITS>(w, i, (uint32_t)clamp_code(sr_guarded(x, r.get(i)), R));
@@ -59,9 +60,9 @@ __device__ __forceinline__ void chunk_encode_guarded(const RV &v, const RR &r, c
 // the same quantiser for a wave whose elements are all finite and <= 2^100 in
 // magnitude (amax_bits is the integer-order maximum of |v|) and whose random
 // values all lie in [0, 1]: none of the guards can fire
-template <int NBITS, bool MEE, class RV, class RR, class ARG>
+template <int NBITS, bool MEE, int N = 16, class RV, class RR, class ARG>
 __device__ __forceinline__ void chunk_encode_fast(const RV &v, const RR &r, uint32_t amax_bits, const ARG &mp,
-                                                  uint32_t (&w)[Rec<NBITS>::WORDS], uint32_t &q, uint32_t &unit_bits)
+                                                  uint32_t (&w)[(N * NBITS + 31) / 32], uint32_t &q, uint32_t &unit_bits)
 {
     constexpr int R = Rec<NBITS>::R;
     const float a = __uint_as_float(amax_bits);
@@ -70,7 +71,7 @@ __device__ __forceinline__ void chunk_encode_fast(const RV &v, const RR &r, uint
         s = div_by(a, mp.inv_cmm) + 1e-7f;
     else
         s = (R == 1 ? a : div_by(a, 1.0 / (double)R)) + 1e-7f; // >= 1e-7, finite
-    const float g = row16_max_pos(s); // s >= 1e-7, finite
+    const float g = superchunk_max_pos<N>(s); // s >= 1e-7, finite
     unit_bits = f32_to_bf16_bits(div_by(g, 1.0 / 255.0));
     const float unit = bf16_bits_to_f32(unit_bits);
     const float ratio = div_by(s, recip_f64(g)) * 255.0f;
@@ -79,8 +80,8 @@ __device__ __forceinline__ void chunk_encode_fast(const RV &v, const RR &r, uint
     q = (uint32_t)qi;
     const float d = (float)qi * unit; // exact: 8 x 8 significant bits
 #pragma unroll
-    for (int k = 0; k < Rec<NBITS>::WORDS; k++) w[k] = 0;
-    estimate_codes<NBITS, MEE>(v, r, d, mp, w);
+    for (int k = 0; k < (N * NBITS + 31) / 32; k++) w[k] = 0;
+    estimate_codes<NBITS, MEE, N>(v, r, d, mp, w);
 }
 
 constexpr uint32_t kFastMaxBits = 0x71800000u; // 2^100

@@ -33,6 +33,12 @@ hipError_t launch_generic_decompress(const uint8_t *src, void *dst, int64_t n, i
                                      int dtype, int strategy, const MeeParams &mp, int add,
                                      hipStream_t stream);
 
+// the same without a row list, for vectors of few superchunks (dq_scaling_hier16_short.hip); recv != null: the fused ring step
+hipError_t launch_hier16_short_compress(const void *src, const uint8_t *recv, uint8_t *dst, const void *rnd, int64_t nsc, int nbits,
+                                        int dtype, bool mee, const MeeParams &mp, const RandKey *philox, hipStream_t stream);
+hipError_t launch_hier16_short_decompress(const uint8_t *src, void *dst, int64_t nsc, int nbits, int dtype, bool mee, const MeeParams &mp,
+                                          hipStream_t stream);
+
 // scaling quantisation, vectorised chunk-16 hierarchical kernels
 // (dq_scaling_hier16.hip); dtype BF16 or F32, element pointers 16-byte aligned
 hipError_t launch_hier16_compress(const void *src, uint8_t *dst, const void *rnd, int64_t n,

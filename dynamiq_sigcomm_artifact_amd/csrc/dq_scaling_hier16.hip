@@ -120,6 +120,33 @@ static inline unsigned grid_for(int64_t nsc, int tiles = 1)
 
 constexpr int64_t kLongRun = 262144; // superchunks of a row list: 16384 waves of four tiles, two rounds of a full chip
 
+// Vectors without a row list that take eight elements per lane (dq_scaling_hier16_short.hip).  Kernels in a graph, us, sixteen -> eight:
+//   superchunks                              1,024         2,048         3,072         6,144         10,240        16,384
+//   compress  bf16, 4 bits, AEE, pool        2.56 -> 2.51  2.66 -> 2.60  2.70 -> 2.86  3.14 -> 3.30
+//             bf16, 5 bits, MEE, drawn       2.84 -> 2.79  2.90 -> 2.82  2.99 -> 3.18  3.54 -> 3.64
+//             bf16, 8 bits, MEE, pool        3.07 -> 2.73  3.20 -> 2.83  3.34 -> 3.20  4.09 -> 3.79  6.02 -> 5.31  6.87 -> 6.35
+//             fp32, 5 bits, MEE, pool                                    3.16 -> 3.08  4.60 -> 4.03  5.94 -> 5.34  7.22 -> 6.79
+//             fp32, 8 bits, AEE, pool                                    3.09 -> 2.92  4.31 -> 3.89  5.49 -> 5.19  6.92 -> 6.66
+//   ring step bf16, 4 bits, AEE, pool        2.73 -> 2.66  2.88 -> 2.80  2.93 -> 3.05  3.73 -> 3.86
+//             bf16, 8 bits, MEE, pool        3.46 -> 3.08  3.65 -> 3.25  3.72 -> 3.70  5.19 -> 5.05  6.94 -> 6.56  7.93 -> 8.07
+//             fp32, 8 bits, AEE, pool                                    3.51 -> 3.40  5.16 -> 4.74  6.21 -> 5.76  7.73 -> 7.65
+//             bf16, 7 bits, MEE, pool                                    3.60 -> 3.78  4.76 -> 5.09
+//   decompress bf16, 4 bits, AEE             2.10 -> 2.03  2.24 -> 2.11  2.39 -> 2.26  2.76 -> 2.67  (8,192: 2.84 -> 3.02)
+//             fp32, 8 bits, MEE              2.56 -> 2.18  2.61 -> 2.35  2.76 -> 2.66  3.21 -> 3.51
+// (in the columns of 3,072 of 5 bits and of 8 bits in AEE, and of 7: 3,584).  Up to 2,048 superchunks every wave of eights has a SIMD to
+// itself, and half of the SIMDs would have none of sixteens.  Beyond, a short chain is worth the chunk's work done twice where the chain is
+// long and nothing is drawn: at 16-bit elements MEE from 6 bits on, at 32 bits from 5 bits MEE and from 8 bits AEE on; a ring step, which decodes on top, at
+// 8 bits only.
+constexpr int64_t kShortRun = 2048, kShortDecode = 3072, kLongChainRun = 16384, kLongChainStep = 12288;
+
+static bool short_encode(int64_t nsc, bool fused, int nbits, bool f32, bool mee, bool drawn)
+{
+    if (nsc <= kShortRun) return true;
+    if (drawn) return false;
+    if (fused) return nsc <= kLongChainStep && nbits == 8 && (mee || f32);
+    return nsc <= kLongChainRun && (mee ? nbits >= (f32 ? 5 : 6) : nbits == 8 && f32);
+}
+
 template <int DT, int RDT, int NBITS, bool MEE>
 static hipError_t run_compress(const void *src, const uint8_t *recv, uint8_t *dst, const void *rnd, const int32_t *rows,
                                int64_t nsc, bool fused, const MeeParams &mp, RandKey key, hipStream_t stream)
@@ -154,6 +181,8 @@ static hipError_t dispatch_compress(const void *src, const uint8_t *recv, uint8_
                                     const int32_t *rows, int64_t nsc, bool fused, int nbits, int dtype, bool mee,
                                     const MeeParams &mp, hipStream_t stream, const RandKey *philox = nullptr)
 {
+    if (!rows && short_encode(nsc, fused, nbits, (dtype & 0xf) == DQ_F32, mee, philox != nullptr))
+        return launch_hier16_short_compress(src, fused ? recv : nullptr, dst, rnd, nsc, nbits, dtype, mee, mp, philox, stream);
     const bool rb16 = (dtype & DQ_RAND_BF16) != 0;
     dtype &= 0xf;
     const RandKey key = philox ? *philox : RandKey{0, 0};
@@ -203,6 +232,8 @@ static hipError_t dispatch_decompress(const uint8_t *src, void *dst, const int32
                                       int64_t limit, int64_t nsc, int nbits, int dtype, bool mee, const MeeParams &mp,
                                       int add, hipStream_t stream)
 {
+    if (!rows && !stats && !add && limit >= nsc * 256 && nsc <= kShortDecode)
+        return launch_hier16_short_decompress(src, dst, nsc, nbits, dtype, mee, mp, stream);
     if ((dtype & 0xf) == DQ_BF16) {
         DQ_NBITS_MEE(run_decompress, DQ_BF16, src, dst, rows, stats, limit, nsc, add, mp, stream)
     } else {

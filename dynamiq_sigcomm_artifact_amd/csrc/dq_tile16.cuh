@@ -354,7 +354,7 @@ __device__ __forceinline__ void window_flush(const uint8_t *win, uint8_t *g, int
 
 // ---- per-chunk code words -----------------------------------------------------------------
 
-template <int NBITS> __device__ __forceinline__ void words_put(uint32_t (&w)[Rec<NBITS>::WORDS], int i, uint32_t code)
+template <int NBITS, int W> __device__ __forceinline__ void words_put(uint32_t (&w)[W], int i, uint32_t code)
 {
     const int bit = i * NBITS;
     w[bit >> 5] |= code << (bit & 31);
@@ -362,7 +362,7 @@ template <int NBITS> __device__ __forceinline__ void words_put(uint32_t (&w)[Rec
 }
 
 // replaces the code of element i
-template <int NBITS> __device__ __forceinline__ void words_set(uint32_t (&w)[Rec<NBITS>::WORDS], int i, uint32_t code)
+template <int NBITS, int W> __device__ __forceinline__ void words_set(uint32_t (&w)[W], int i, uint32_t code)
 {
     constexpr uint32_t kMask = (1u << NBITS) - 1u;
     const int bit = i * NBITS;
@@ -373,7 +373,7 @@ template <int NBITS> __device__ __forceinline__ void words_set(uint32_t (&w)[Rec
     }
 }
 
-template <int NBITS> __device__ __forceinline__ uint32_t words_get(const uint32_t (&w)[Rec<NBITS>::WORDS], int i)
+template <int NBITS, int W> __device__ __forceinline__ uint32_t words_get(const uint32_t (&w)[W], int i)
 {
     const int bit = i * NBITS;
     uint32_t v = w[bit >> 5] >> (bit & 31);
@@ -539,8 +539,9 @@ template <int NBITS> __device__ __forceinline__ uint32_t clamp_fields(uint32_t w
 // pass the guard unnoticed) with |v| <= (R + 1) d and random values in [0, 1]: estimate, guard, exact redo.  w must
 // be zeroed.  -1 < T' < 2 R + 2, so the conversion to a signed integer (towards zero) is the lower clamp, and for the
 // widths that divide 32 the upper clamp is done on the packed words (clamp_fields).
-template <int NBITS, bool MEE, class RV, class RR, class ARG>
-__device__ __forceinline__ void estimate_codes(const RV &v, const RR &r, float d, const ARG &mp, uint32_t (&w)[Rec<NBITS>::WORDS])
+// N: the elements, those of a lane.
+template <int NBITS, bool MEE, int N = 16, class RV, class RR, class ARG>
+__device__ __forceinline__ void estimate_codes(const RV &v, const RR &r, float d, const ARG &mp, uint32_t (&w)[(N * NBITS + 31) / 32])
 {
     constexpr int R = Rec<NBITS>::R;
     constexpr bool kFields = NBITS == 2 || NBITS == 4 || NBITS == 8;
@@ -549,10 +550,10 @@ __device__ __forceinline__ void estimate_codes(const RV &v, const RR &r, float d
     constexpr float kDelta = EstimateGuard<NBITS, MEE>::kDelta;
     // (the wave-wide view of each flag is taken where the comparison is made: there it is the comparison's own lane mask, and
     // the tests further down are scalar)
-    bool doubt[16];
-    uint64_t lanes_in_doubt[16], any = 0;
+    bool doubt[N];
+    uint64_t lanes_in_doubt[N], any = 0;
 #pragma unroll
-    for (int i = 0; i < 16; i++) {
+    for (int i = 0; i < N; i++) {
         const float t = estimate_coordinate<NBITS, MEE>(v, r, i, rd, rc, rl2b);
         doubt[i] = __builtin_amdgcn_fractf(t) < 2.0f * kDelta;
         lanes_in_doubt[i] = __builtin_amdgcn_ballot_w64(doubt[i]);
@@ -564,12 +565,12 @@ __device__ __forceinline__ void estimate_codes(const RV &v, const RR &r, float d
     }
     if (kFields) {
 #pragma unroll
-        for (int k = 0; k < Rec<NBITS>::WORDS; k++) w[k] = clamp_fields<kFields ? NBITS : 2>(w[k]);
+        for (int k = 0; k < (N * NBITS + 31) / 32; k++) w[k] = clamp_fields<kFields ? NBITS : 2>(w[k]);
     }
     if (DQ_UNLIKELY(any != 0)) {
         const double yd = recip_f64(d);
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
+        for (int i = 0; i < N; i++) {
             if (DQ_UNLIKELY(lanes_in_doubt[i] != 0)) {
                 // (among them the zero elements -- padding, sparse input -- whose random value is exactly 0 or 1: their
                 // T is an integer, and the chain's ceil(-r) is 0, or -1 at r = 1)

@@ -152,6 +152,58 @@ def test_production_shape_random(capi, oracle, dt, nbits, strategy):
 
 
 @pytest.mark.parametrize("dt", [BF16, F32])
+@pytest.mark.parametrize("nbits,strategy,nscs", [(4, 2, (2047, 2049, 3073)), (5, 3, (2048, 3072, 16385)), (7, 3, (2049, 16384)),
+                                                 (8, 2, (2, 12288, 16385)), (8, 3, (2050, 12289, 16384))])
+def test_either_side_of_eight_elements_per_lane(capi, oracle, dt, nbits, strategy, nscs):
+    """The codec takes eight elements per lane up to 2,048 superchunks (decoding 3,072; long chains 12,288 and 16,384) and sixteen
+    beyond: the same bytes on either side of every line, with waves on the guarded path, elements on the boundaries of the
+    rounding, and buffers off the 16 bytes."""
+    tdt = TORCH_DT[dt]
+    g = torch.Generator().manual_seed(nbits * 7 + strategy)
+    for nsc in nscs:
+        n = nsc * 256
+        src = (torch.randn(nsc, 256, generator=g) * torch.exp(torch.randn(nsc, 1, generator=g) * 3.0 - 7.0)).reshape(-1)
+        src[::997] = 0.0
+        src[300] = float("inf")
+        src[n // 2] = float("nan")
+        src[-256:] = torch.where(torch.rand(256, generator=g) < 0.5, -1.0, 1.0) * 0.7
+        rnd = torch.rand(n, generator=g)
+        rnd[::13] = 0.0
+        rnd[5::17] = 1.0
+        src, rnd = src.to(tdt), rnd.to(tdt)
+        tag = "dt=%d b=%d s=%d nsc=%d" % (dt, nbits, strategy, nsc)
+        nbytes = capi.required_bytes(n, nbits, 16, strategy)
+        want = oracle.scaling_compress(to_bits(src), to_bits(rnd), n, nbits, 16, strategy, dt)
+        inp = (torch.randn(n, generator=g) * 2e-3).to(tdt)
+        want_step = oracle.scaling_dec_comp(want, to_bits(inp), to_bits(rnd.flip(0)), n, nbits, 16, strategy, dt)
+        want_out = np.zeros(n, np.float32 if dt == F32 else np.uint16)
+        oracle.scaling_decompress(want, want_out, n, nbits, 16, strategy, dt)
+        for off in (0, 1):                          # elements and bytes that the buffers start behind an aligned address
+            def placed(t):
+                buf = torch.zeros(t.numel() + 8, dtype=t.dtype, device=DEV)
+                buf[off:off + t.numel()] = t.to(DEV)
+                return buf[off:off + t.numel()]
+            enc, step = (torch.full((nbytes + 24,), 0xAB, dtype=torch.uint8, device=DEV)[off:] for _ in range(2))
+            capi.scaling_compress(placed(src), enc, placed(rnd), n, nbits, 16, strategy)
+            capi.scaling_dec_comp(enc, placed(inp), step, placed(rnd.flip(0)), n, nbits, 16, strategy)
+            out = placed(torch.zeros(n, dtype=tdt))
+            capi.scaling_decompress(enc, out, n, nbits, 16, strategy)
+            for name, got, expected in (("compress", enc, want), ("step", step, want_step)):
+                _cmp_bits("%s %s %d" % (tag, name, off), got[:nbytes].cpu().numpy(), expected)
+                assert bool((got[nbytes:] == 0xAB).all()), tag + " wrote past the packed stream"
+            _cmp_bits("%s decompress %d" % (tag, off), to_bits(out), want_out)
+            if off == 0:                            # drawn values: the pool they stand for
+                uni, drawn = torch.empty(n, dtype=tdt, device=DEV), torch.zeros(nbytes, dtype=torch.uint8, device=DEV)
+                capi.philox_uniform(uni, 3, nsc)
+                capi.scaling_compress(src.to(DEV), step, uni, n, nbits, 16, strategy)
+                capi.scaling_compress_philox(src.to(DEV), drawn, n, nbits, 16, strategy, 3, nsc)
+                assert torch.equal(step[:nbytes], drawn), tag
+                capi.scaling_dec_comp(enc, inp.to(DEV), step, uni, n, nbits, 16, strategy)
+                capi.scaling_dec_comp_philox(enc, inp.to(DEV), drawn, n, nbits, 16, strategy, 3, nsc)
+                assert torch.equal(step[:nbytes], drawn), tag + " step"
+
+
+@pytest.mark.parametrize("dt", [BF16, F32])
 @pytest.mark.parametrize("strategy", [2, 3])
 def test_special_values(capi, oracle, dt, strategy):
     """zeros, denormals, huge values, inf/nan inputs, rand exactly 0 and 1."""
