@@ -493,11 +493,13 @@ __device__ __forceinline__ int exact_code_fast(float vi, float ri, float d, doub
 //        (R + 1) 2^-26 otherwise, and the fma rounds a value below 2 (R + 1): e stays below 0.27 (R + 1) 2^-20.
 //   MEE: estimate = fma(v_log_f32(fma(|v rcp(d)|, 1 / c, 1)), +-1 / log2(base), (R + 1 + kDelta) - r), v_log_f32 being
 //        good to 1 ulp; estimate and exact chain both approximate log2(|v| / (d c) + 1) / log2(base), their distance is
-//        bounded by (1.44 * 5e-7 + 2.7 ulp(log)) / log2(base) + 2 ulp(2 R): < 6.9e-5 for 6..8 bits (log2(base) = 0.0286,
-//        log < 4) and < 1.2e-5 below (log2(base) >= 0.09, log < 1.5); measured over 4e9 random operands per width: 1.5e-5
+//        bounded by (1.44 * 5e-7 + 2.7 ulp(log)) / log2(base) + 2 ulp(2 R): < 8e-5 for 6..8 bits (log2(base) = 0.0286,
+//        log < 4) and < 1.6e-5 below (log2(base) >= 0.09, log < 1.5); measured over 4e9 random operands per width: 1.5e-5
 //        and 4.8e-6 (without the constant in the last fma, which adds at most 3.8e-6 and 1e-6).
+// kDelta is the power of two above these bounds (half a unit of (R + 1) 2^-20, 1.2e-4, 3.1e-5).  With twice as much, twice the waves redo
+// elements: at 8 bits in MEE 40 instead of 22 %, compress of 524,288 elements 2.84 -> 2.74 us, ring step of 6,553,600 10.5 -> 10.3.
 template <int NBITS, bool MEE> struct EstimateGuard {
-    static constexpr float kDelta = MEE ? (NBITS >= 6 ? 0x1p-12f : 0x1p-14f) : (float)(1 << (NBITS - 1)) * 0x1p-20f;
+    static constexpr float kDelta = MEE ? (NBITS >= 6 ? 0x1p-13f : 0x1p-15f) : (float)(1 << (NBITS - 1)) * 0x1p-21f;
 };
 
 // bias - r_i; exact for the in-kernel random bytes ((256 bias - odd byte) / 256 needs 16 bits)
@@ -513,7 +515,7 @@ template <int NBITS, bool MEE, class RV, class RR>
 __device__ __forceinline__ float estimate_coordinate(const RV &v, const RR &r, int i, float rd, float rc, float rl2b)
 {
     const float vi = v.get(i);
-    const float off = below(r, i, (float)(Rec<NBITS>::R + 1) + EstimateGuard<NBITS, MEE>::kDelta); // the constant is exact: <= 21 bits
+    const float off = below(r, i, (float)(Rec<NBITS>::R + 1) + EstimateGuard<NBITS, MEE>::kDelta); // the constant is exact: <= 22 bits
     if (MEE) {
         const float est = __builtin_amdgcn_logf(__builtin_fmaf(__builtin_fabsf(vi * rd), rc, 1.0f));
         return __builtin_fmaf(est, __builtin_copysignf(rl2b, vi), off);
