@@ -227,7 +227,7 @@ constexpr int kMaxTileBits = 15; // 2^15 floats = 128 KiB (+ padding) of the 160
 constexpr int kPrefTileBits = 13; // 32 KiB tiles keep several workgroups per CU in flight
 constexpr int kStridedCols = 5;   // 32 consecutive floats (128 B) per row of a strided tile
 
-// How a transform of 2^kb > 2^15 elements is divided: index bits of the contiguous pass, the rest go to strided passes.
+// How a transform of 2^kb > 2^15 elements (and few blocks of 2^15) is divided: index bits of the contiguous pass, the rest go to strided passes.
 // Both passes are bound by memory (or, short, by how many workgroups there are to hide its latency), so the tiles should be
 // small enough for several workgroups per CU and there should be two passes:
 //   up to 2^18  128 rows per strided tile (16 KB): the vector has only 32 to 128 tiles of that size
@@ -243,6 +243,12 @@ static int contiguous_bits(int kb)
     if (kb <= 22) return kb - 8;
     return kb <= 25 ? kb - 10 : kPrefTileBits;
 }
+
+// Blocks of 2^15 go in two passes of 2^10 and 32 rows as well where there are few of them: as one tile each, a block is a workgroup that has
+// a CU to itself for 10 us, with most of the others idle.  Blocked transform in a graph, us, forward, one pass -> two: one block 9.8 -> 5.7, 8
+// blocks 10.1 -> 6.3, 16 10.2 -> 7.4, 32 10.6 -> 9.7 (64, one pass: 11.2); back 11.1 -> 6.9 and 11.7 -> 10.8.  THC there and back, 17,000 to
+// 32,768 elements, 31.0 -> 23.6.  (Blocks of 2^14: 5.4 -> 5.6, back 6.1 -> 7.4, THC 20.4 -> 26.4.)
+constexpr int64_t kFewTo = (int64_t)32 << kMaxTileBits;
 
 // rows of the next strided pass: the remaining bits split evenly over as few passes as the LDS allows
 static int rows_of_pass(int rem)
@@ -295,7 +301,8 @@ static hipError_t fwht_blocks(float *x, const void *sign, bool sign_packed, int6
     if (inverse) first.gen = SignSeed();
     else last.gen = SignSeed();
 
-    if (kb <= kMaxTileBits) {
+    const bool few = kb == kMaxTileBits && n <= kFewTo && ends_ok && (n & (((int64_t)1 << kb) - 1)) == 0;
+    if (kb <= kMaxTileBits && !few) {
         // single pass; small blocks share a tile
         int kt = kb < kPrefTileBits ? kPrefTileBits : kb;
         while (kt > kb && kt > 10 && (n >> kt) < 512) kt--; // short vectors: two workgroups per CU before larger tiles

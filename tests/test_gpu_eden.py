@@ -333,6 +333,44 @@ def test_thc_recorded_draws_are_torchs():
         assert torch.equal(got.view(torch.int16), want.view(torch.int16))
 
 
+@pytest.mark.parametrize("blocks", [1, 3, 32])
+def test_few_blocks_of_2p15_are_those_of_a_long_vector(capi, blocks):
+    """up to 32 blocks of 2^15 take two passes, more of them one: the same bits, with packed and float signs, either way, and with THC's
+    quantisers at the ends"""
+    block, levels = 1 << 15, 64
+    n, many = blocks * block, 40 * block
+    g = torch.Generator(device=DEV).manual_seed(blocks)
+    x = torch.randn(many, generator=g, device=DEV)
+    sign = torch.randint(0, 2, (many,), generator=g, device=DEV).float() * 2.0 - 1.0
+    scale = 1.0 / block ** 0.5
+    for packed in (False, True):
+        for inverse in (False, True):
+            long, few = x.clone(), x[:n].clone()
+            capi.rht_blocked(long, capi.pack_signs(sign) if packed else sign, block, scale, inverse)
+            capi.rht_blocked(few, capi.pack_signs(sign[:n]) if packed else sign[:n], block, scale, inverse)
+            assert torch.equal(few.view(torch.int32), long[:n].view(torch.int32)), (packed, inverse)
+    odd = torch.zeros(n + 1, device=DEV)[1:].copy_(x[:n])       # off the 16 bytes: as before
+    capi.rht_blocked(odd, sign[:n], block, scale, True)
+    long = x.clone()
+    capi.rht_blocked(long, sign, block, scale, True)
+    assert torch.equal(odd.view(torch.int32), long[:n].view(torch.int32))
+    lo, step = torch.tensor([-3.0], device=DEV), torch.tensor([6.0 / (levels - 1)], device=DEV)
+    uni, bits = torch.rand(n, generator=g, device=DEV), capi.pack_signs(sign[:n])
+    long, few = x.clone(), x[:n].clone()
+    capi.rht_blocked(long, sign, block, scale, False)
+    want, got = (torch.empty(n, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    capi.thc_quantize(long[:n].contiguous(), uni, want, lo, step, levels)
+    capi.thc_rht_quantize(few, bits, uni, got, block, scale, lo, step, levels)
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16)) and want.unique().numel() > 32
+    back = torch.zeros(many, device=DEV)
+    out = torch.empty(n, device=DEV)
+    capi.thc_dequantize(want, out, step, lo)
+    back[:n] = out
+    capi.rht_blocked(back, sign, block, scale, True)
+    capi.thc_dequantize_irht(want, bits, out, block, scale, step, lo)
+    assert torch.equal(out.view(torch.int32), back[:n].view(torch.int32))
+
+
 @pytest.mark.parametrize("bits,shift", [(14, 0), (16, 1), (17, 0), (18, 3), (21, 0), (24, 1), (26, 0), (27, 0), (30, 0)])
 def test_long_transforms_of_a_unit_vector(capi, bits, shift):
     """H e_k = (-1)^popcount(j & k): every element of the contiguous pass and of strided passes of four to ten row bits, on vectors
