@@ -877,7 +877,9 @@ __global__ __launch_bounds__(64 * kPartWaves) void ring_parts_kernel(RingArgs<RD
 //   8 ranks  x 2,000 (500,000 elements) 16.2 15.1 17.1, x 4,000 20.6 19.3 20.0, 22.3 21.0 21.7, x 5,000 24.0 22.6 24.0, 26.2 24.8 26.4,
 //            x 8,000 31.8 29.3 28.6, 34.9 32.8 31.3, x 12,000 40.8 37.5 34.9, 44.7 42.6 40.9
 // With fp32 elements eight are 32 bytes of a lane and its loads half lines: 5 ranks x 8,000 27.8 26.8 31.3, so fp32 stays with four; pools
-// do as well (bf16, 4 x 4,600 in AEE 18.0 17.8 30.3).
+// do as well (bf16, 4 x 4,600 in AEE 18.0 17.8 30.3).  Vectors off the 16 bytes stay with four at every length: they load and store element by
+// element, and with eight of them a lane has half as many on the way.  All of them an element off, four -> eight: 2 x 5,200 17.5 -> 19.5,
+// 8 x 5,200 48.4 -> 63.2, 8 x 8,192 63.6 -> 80.6, 8 x 16,000 117 -> 147, in MEE 4 x 12,000 54.1 -> 68.9.
 constexpr int kFoursTo = 5120;
 
 // With lists from a plan, up to so many superchunks in parts.  bf16 with drawn values, plan and all, us, sixteen -> eight: 2 ranks x 12,000 17.7 ->
@@ -1048,7 +1050,7 @@ static hipError_t run_ring(const RingDesc &d, bool mee, const MeeParams *mp, hip
         };
         constexpr bool PLANS = decltype(plans)::value;
         if constexpr (DT == DQ_BF16 && !POOL) {
-            if (a.nsc > kFoursTo)
+            if (a.nsc > kFoursTo && (a.vec & 3) == 3)
                 return mee ? go(ring_parts_kernel<DT, RDT, true, 8, PLANS>, 2 * kPartWaves) : go(ring_parts_kernel<DT, RDT, false, 8, PLANS>, 2 * kPartWaves);
         }
         return mee ? go(ring_parts_kernel<DT, RDT, true, 4, PLANS>, kPartWaves) : go(ring_parts_kernel<DT, RDT, false, 4, PLANS>, kPartWaves);

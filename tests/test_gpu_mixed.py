@@ -822,6 +822,30 @@ def test_lines_of_the_rings_without_lists(capi, W, n, dt):
     test_rings_without_lists(capi, W, n, dt)
 
 
+@pytest.mark.parametrize("W,nsc", [(2, 5121), (3, 12288), (5, 12289), (4, 20480)])
+@pytest.mark.parametrize("off_in,off_out", [(1, 3), (0, 1), (2, 0)])
+def test_rings_off_the_16_bytes(capi, W, nsc, off_in, off_out):
+    """bf16 vectors or outputs (or both) off the 16 bytes take four elements per lane where aligned ones take eight, with lists and
+    without"""
+    from dynamiq_sigcomm_artifact_amd.bitrate import NormHistogram
+    from dynamiq_sigcomm_artifact_amd.dynamiq_pipeline import _single_pass_in_steps, dynamic_bitrate_allreduce_single_pass
+    n = nsc * 256 - 3
+    g = torch.Generator(device=DEV).manual_seed(nsc + W)
+    scales = torch.exp(torch.randn(nsc, 1, generator=g, device=DEV) * 6.0) * 1e-3
+    vecs = []
+    for _ in range(W):
+        v = torch.zeros(n + 8, dtype=torch.bfloat16, device=DEV)
+        vecs.append(v[off_in:off_in + n].copy_((torch.randn(nsc, 256, generator=g, device=DEV) * scales).reshape(-1)[:n]))
+    for strategy, u in ((2, 6.0), (3, 6.5)):
+        ref, _, _ = _single_pass_in_steps(vecs, u, strategy, 11, None, {}, None, None)
+        for hist in (None, NormHistogram(DEV)):
+            rooms = [torch.full((n + 8,), 7.0, dtype=torch.bfloat16, device=DEV) for _ in range(W)]
+            outs = [r[off_out:off_out + n] for r in rooms]
+            dynamic_bitrate_allreduce_single_pass(vecs, u, strategy=strategy, seed=11, out=outs, norm_histogram=hist)
+            assert all(torch.equal(bits_t(x), bits_t(y)) for x, y in zip(outs, ref)), (strategy, hist is None)
+            assert all(bool((r[:off_out] == 7.0).all()) and bool((r[off_out + n:] == 7.0).all()) for r in rooms)
+
+
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
 def test_ends_inside_a_lane_of_a_short_ring(capi, dt):
     """vectors of one to nine elements, and every end in the last superchunk's first and last lanes"""
