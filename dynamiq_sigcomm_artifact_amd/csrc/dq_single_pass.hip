@@ -686,7 +686,7 @@ __global__ __launch_bounds__(64 * kPartWaves) void ring_parts_kernel(RingArgs<RD
     // What a step needs besides its elements, by rank and once more, so that the ranks from any on lie side by side: the address of the
     // vector and the mean.  (Loaded step by step through the scalar cache they are half of a step's time.)
     __shared__ uint4 of_rank[kPartWaves][P][2 * kMaxRanks];
-    __shared__ uint64_t pool_of_step[POOL ? kPartWaves : 1][P][kMaxPoolRanks];
+    __shared__ uint64_t pool_of_step[POOL ? kPartWaves : 1][kMaxPoolRanks];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), world = a.world;
     const int half = lane / kLanes; // (0 where a wave has one superchunk)
     const int rank_here = lane & (2 * kMaxRanks - 1), my_rank = min(rank_here < world ? rank_here : rank_here - world, world - 1);
@@ -798,19 +798,13 @@ __global__ __launch_bounds__(64 * kPartWaves) void ring_parts_kernel(RingArgs<RD
     const bool whole_loads = (a.vec & 1) != 0 && a.n >= N;
     const int64_t from = min(e0, a.n - N);
     const WidthRegs<MEE> w = width_regs<MEE>(a.widths, my_cls, levels);
-    if (rank_here < 2 * world && (P > 1 || lane < 2 * kMaxRanks))
-        of_rank[wave][which][rank_here] = make_uint4((uint32_t)my_src, (uint32_t)(my_src >> 32), __float_as_uint(my_mean), 0u);
+    uint64_t my_pool = 0; // of step `lane`
     if constexpr (POOL) {
-        const int step = lane & (kMaxPoolRanks - 1), h = (lane / kMaxPoolRanks) & (P - 1);
-        const int c = h == 0 ? chunk[0] : chunk[P - 1], g = h == 0 ? cls[0] : cls[P - 1], in = h == 0 ? in_run[0] : in_run[P - 1];
-        if (step < world) {
-            const int rank = c + step < world ? c + step : c + step - world;
-            pool_of_step[wave][h][step] = reinterpret_cast<uint64_t>(a.more.pool[g][rank]) +
-                                          (int64_t)(a.more.first[g][rank][step] + in * 16) * (16 * (RDT == DQ_F32 ? 4 : 2));
-        }
+        static_assert(P == 1, "pools are for a superchunk per wave");
+        const int step = min(lane & (kMaxPoolRanks - 1), world - 1), rank = chunk[0] + step < world ? chunk[0] + step : chunk[0] + step - world;
+        my_pool = reinterpret_cast<uint64_t>(a.more.pool[cls[0]][rank]) +
+                  (int64_t)(a.more.first[cls[0]][rank][step] + in_run[0] * 16) * (16 * (RDT == DQ_F32 ? 4 : 2));
     }
-    wave_lds_sync();
-    const uint4 *ranks = of_rank[wave][half] + my_chunk;
 
     // (memory, and the compiler is told so: what it only knows as an address it loads through instructions that may also mean the LDS,
     // and every read of the LDS then waits for the elements of the step to come)
@@ -820,17 +814,39 @@ __global__ __launch_bounds__(64 * kPartWaves) void ring_parts_kernel(RingArgs<RD
     RawPart<RDT, N> next_r;
     next_r.zero();
     float next_mean = 0.0f;
+    const auto load = [&](uint64_t src, uint64_t pool) {
+        if (whole_loads)
+            next.load_anywhere(pointer(src), from);
+        else
+            load_chunk<DT>(next, pointer(src), e0, a.n, a.vec & 1, ragged);
+        if constexpr (POOL) next_r.load(pointer(pool), lane * N, (a.vec & 4) != 0);
+    };
+    // With lists the means wait for an entry of the list, and the first step's elements not for them: its addresses come from the lanes
+    // instead of the table (fixed proportions, 4 x 64 superchunks 13.9 -> 13.4 us, 2 x 256 in MEE 12.6 -> 12.4).
+    if constexpr (!PLANS) {
+        const auto of_lane = [](uint64_t x, int at) {
+            return (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)x, at) |
+                   (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(x >> 32), at) << 32;
+        };
+        const uint64_t first = of_lane(my_src, chunk[0]), second = P == 1 ? first : of_lane(my_src, chunk[P - 1]);
+        load(half == 0 ? first : second, POOL ? of_lane(my_pool, 0) : 0);
+    }
+    if (rank_here < 2 * world && (P > 1 || lane < 2 * kMaxRanks))
+        of_rank[wave][which][rank_here] = make_uint4((uint32_t)my_src, (uint32_t)(my_src >> 32), __float_as_uint(my_mean), 0u);
+    if constexpr (POOL) {
+        if (lane < kMaxPoolRanks) pool_of_step[wave][lane] = my_pool;
+    }
+    wave_lds_sync();
+    const uint4 *ranks = of_rank[wave][half] + my_chunk;
     const auto fetch = [&](int step) {
         const uint4 of = ranks[step];
-        const void *src = pointer((uint64_t)of.x | ((uint64_t)of.y << 32));
         next_mean = __uint_as_float(of.z);
-        if (whole_loads)
-            next.load_anywhere(src, from);
-        else
-            load_chunk<DT>(next, src, e0, a.n, a.vec & 1, ragged);
-        if constexpr (POOL) next_r.load(pointer(pool_of_step[wave][half][step]), (lane & (kLanes - 1)) * N, (a.vec & 4) != 0);
+        load((uint64_t)of.x | ((uint64_t)of.y << 32), POOL ? pool_of_step[wave][step] : 0);
     };
-    fetch(0);
+    if (PLANS)
+        fetch(0);
+    else
+        next_mean = __uint_as_float(ranks[0].z);
     uint32_t draws[4];
     float lev[N], scale = 0.0f;
 #pragma unroll 1
