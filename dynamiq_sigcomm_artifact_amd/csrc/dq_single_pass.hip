@@ -677,6 +677,10 @@ constexpr int kPartWaves = 4;
 // PLANS: without a plan launch in front.  A superchunk's way through the ring depends on the others only by where it starts: on its
 // place among those of its width.  The statistics leave a word per four superchunks with their widths' counts; a workgroup takes
 // neighbouring superchunks and adds up the words, all of them and those before its own, while the norms of its own are on their way.
+//
+// Fours in MEE stay within 64 vector and 80 scalar registers (79 with bf16), or a SIMD has room for seven waves instead of eight, whatever the
+// compiler counts: with 81, 96 and the trap handler's 16 are taken.  MEE from 7,169 superchunks on, all vectors an element off the 16 bytes, with
+// 81 -> 79, us: 2 x 8,192 23.6 -> 22.5, 8 x 8,192 71.0 -> 65.2.
 template <int DT, int RDT, bool MEE, int N, bool PLANS>
 __global__ __launch_bounds__(64 * kPartWaves) void ring_parts_kernel(RingArgs<RDT != DQ_PHILOX> a)
 {

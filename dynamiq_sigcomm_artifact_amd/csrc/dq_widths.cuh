@@ -318,7 +318,8 @@ template <int DT, int N> __device__ __forceinline__ void finish_centered(float (
     for (int i = 0; i < N; i++) t[i] = round_element<DT>(t[i]);
 }
 
-// t = T(v / world - mean), zero at and beyond element n of the vector (center_chunk without its own loads)
+// t = T(v / world - mean), zero at and beyond element n of the vector (center_chunk without its own loads).  For 16-bit elements every
+// power of two that a ring has ranks is fuse16's (and the general quotient is right for the others).
 template <int DT, class RV>
 __device__ __forceinline__ void center_loaded(float (&t)[RV::kCount], const RV &v, const WorldDiv &wd, float mean, int64_t e0, int64_t n, bool ragged)
 {
@@ -328,7 +329,7 @@ __device__ __forceinline__ void center_loaded(float (&t)[RV::kCount], const RV &
     if (DT != DQ_F32 && wd.fuse16) {
 #pragma unroll
         for (int i = 0; i < N; i++) t[i] = __builtin_fmaf(v.get(i), inv, -mean);
-    } else if (wd.pow2) {
+    } else if (DT == DQ_F32 && wd.pow2) {
 #pragma unroll
         for (int i = 0; i < N; i++) t[i] = v.get(i) * inv - mean;
     } else {
