@@ -900,7 +900,12 @@ __global__ __launch_bounds__(64 * kPartWaves) void ring_parts_kernel(RingArgs<RD
 // do as well (bf16, 4 x 4,600 in AEE 18.0 17.8 30.3).  Vectors off the 16 bytes stay with four at every length: they load and store element by
 // element, and with eight of them a lane has half as many on the way.  All of them an element off, four -> eight: 2 x 5,200 17.5 -> 19.5,
 // 8 x 5,200 48.4 -> 63.2, 8 x 8,192 63.6 -> 80.6, 8 x 16,000 117 -> 147, in MEE 4 x 12,000 54.1 -> 68.9.
-constexpr int kFoursTo = 5120;
+// From five ranks without a plan on, three with one, the steps are most of the time, and fours keep the lead up to seven waves per SIMD.  Of
+// the time before there were eights, eight / four: 8 ranks x 5,200 0.994 / 0.932 (AEE), 1.000 / 0.936 (MEE), x
+// 7,000 1.012 / 0.926, 1.044 / 0.951, x 7,300 0.943 / 0.933, 0.931 / 0.935; 5 x 7,000 0.992 / 0.964, 1.007 / 0.965; 4 x 7,000 0.958 / 0.959,
+// 0.969 / 0.963; with lists 8 x 7,000 0.986 / 0.946, 0.994 / 0.947, 3 x 7,000 0.986 / 0.965, 1.001 / 0.982, 2 x 7,000 0.975 / 0.998, 0.976 / 0.986.
+constexpr int kFoursTo = 5120, kFoursToMany = 7168;
+constexpr int fours_to(int world, bool plans) { return world >= (plans ? 5 : 3) ? kFoursToMany : kFoursTo; }
 
 // With lists from a plan, up to so many superchunks in parts.  bf16 with drawn values, plan and all, us, sixteen -> eight: 2 ranks x 12,000 17.7 ->
 // 17.1 (AEE), 20.0 -> 20.2 (MEE), x 16,000 19.5 -> 20.0; 5 x 16,000 35.9 -> 34.5, 40.2 -> 40.0, x 20,000 41.9 -> 40.0, 47.1 -> 45.6; 8 x 20,000
@@ -1070,7 +1075,7 @@ static hipError_t run_ring(const RingDesc &d, bool mee, const MeeParams *mp, hip
         };
         constexpr bool PLANS = decltype(plans)::value;
         if constexpr (DT == DQ_BF16 && !POOL) {
-            if (a.nsc > kFoursTo && (a.vec & 3) == 3)
+            if (a.nsc > fours_to(d.world, PLANS) && (a.vec & 3) == 3)
                 return mee ? go(ring_parts_kernel<DT, RDT, true, 8, PLANS>, 2 * kPartWaves) : go(ring_parts_kernel<DT, RDT, false, 8, PLANS>, 2 * kPartWaves);
         }
         return mee ? go(ring_parts_kernel<DT, RDT, true, 4, PLANS>, kPartWaves) : go(ring_parts_kernel<DT, RDT, false, 4, PLANS>, kPartWaves);

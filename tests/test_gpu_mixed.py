@@ -822,6 +822,14 @@ def test_lines_of_the_rings_without_lists(capi, W, n, dt):
     test_rings_without_lists(capi, W, n, dt)
 
 
+@pytest.mark.parametrize("W,n", [(3, 256 * 7168), (3, 256 * 7169 - 250), (4, 256 * 7168 - 3), (4, 256 * 7169), (5, 256 * 7168 - 1), (5, 256 * 7169 - 7),
+                                 (8, 256 * 7169)])
+def test_rings_on_either_side_of_eight_elements_per_lane(capi, W, n):
+    """bf16: three and more ranks with lists, five and more without, take four elements per lane to 7,168 superchunks"""
+    test_ranks_in_registers_equal_the_ring_in_steps(capi, W, n, torch.bfloat16)
+    test_rings_without_lists(capi, W, n, torch.bfloat16)
+
+
 @pytest.mark.parametrize("W,nsc", [(2, 5121), (3, 12288), (5, 12289), (4, 20480)])
 @pytest.mark.parametrize("off_in,off_out", [(1, 3), (0, 1), (2, 0)])
 def test_rings_off_the_16_bytes(capi, W, nsc, off_in, off_out):
