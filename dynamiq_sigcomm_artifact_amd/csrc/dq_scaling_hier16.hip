@@ -125,19 +125,28 @@ constexpr int64_t kLongRun = 262144; // superchunks of a row list: 16384 waves o
 //   compress  bf16, 4 bits, AEE, pool        2.56 -> 2.51  2.66 -> 2.60  2.70 -> 2.86  3.14 -> 3.30
 //             bf16, 5 bits, MEE, drawn       2.84 -> 2.79  2.90 -> 2.82  2.99 -> 3.18  3.54 -> 3.64
 //             bf16, 8 bits, MEE, pool        3.07 -> 2.73  3.20 -> 2.83  3.34 -> 3.20  4.09 -> 3.79  6.02 -> 5.31  6.87 -> 6.35
+//             bf16, 6 bits, MEE, pool        3.15 -> 2.66  3.21 -> 2.80  3.25 -> 3.08  4.22 -> 3.75  5.88 -> 5.10  7.00 -> 6.18
+//             bf16, 7 bits, MEE, pool        3.13 -> 2.73  3.23 -> 2.78  3.40 -> 3.13  4.07 -> 3.74  5.98 -> 5.12  6.87 -> 6.23
 //             fp32, 5 bits, MEE, pool                                    3.16 -> 3.08  4.60 -> 4.03  5.94 -> 5.34  7.22 -> 6.79
+//             fp32, 6 bits, MEE, pool        3.14 -> 2.64  3.26 -> 2.79  3.34 -> 3.07  5.16 -> 4.49  6.13 -> 5.43  7.49 -> 6.87
+//             fp32, 7 bits, MEE, pool        3.17 -> 2.66  3.27 -> 2.78  3.41 -> 3.09  5.19 -> 4.49  6.26 -> 5.43  7.57 -> 6.90
 //             fp32, 8 bits, AEE, pool                                    3.09 -> 2.92  4.31 -> 3.89  5.49 -> 5.19  6.92 -> 6.66
 //   ring step bf16, 4 bits, AEE, pool        2.73 -> 2.66  2.88 -> 2.80  2.93 -> 3.05  3.73 -> 3.86
 //             bf16, 8 bits, MEE, pool        3.46 -> 3.08  3.65 -> 3.25  3.72 -> 3.70  5.19 -> 5.05  6.94 -> 6.56  7.93 -> 8.07
 //             fp32, 8 bits, AEE, pool                                    3.51 -> 3.40  5.16 -> 4.74  6.21 -> 5.76  7.73 -> 7.65
+//             fp32, 8 bits, MEE, pool        3.69 -> 3.01  3.89 -> 3.17  4.15 -> 3.59  6.02 -> 5.53  7.36 -> 6.68  8.76 -> 8.46
 //             bf16, 7 bits, MEE, pool                                    3.60 -> 3.78  4.76 -> 5.09
 //   decompress bf16, 4 bits, AEE             2.10 -> 2.03  2.24 -> 2.11  2.39 -> 2.26  2.76 -> 2.67  (8,192: 2.84 -> 3.02)
+//             bf16, 7 bits, AEE              2.20 -> 2.10  2.40 -> 2.27  2.45 -> 2.50  (2,560: 2.40 -> 2.39; 2,944: 2.44 -> 2.49)
+//             bf16, 7 bits, MEE              2.29 -> 2.14  2.44 -> 2.27  2.49 -> 2.53  (2,560: 2.48 -> 2.44)
+//             bf16, 8 bits, AEE              2.10 -> 2.03  2.28 -> 2.12  2.34 -> 2.24
+//             bf16, 8 bits, MEE              2.23 -> 2.08  2.42 -> 2.19  2.52 -> 2.36
 //             fp32, 8 bits, MEE              2.56 -> 2.18  2.61 -> 2.35  2.76 -> 2.66  3.21 -> 3.51
-// (in the columns of 3,072 of 5 bits and of 8 bits in AEE, and of 7: 3,584).  Up to 2,048 superchunks every wave of eights has a SIMD to
+// (in the columns of 3,072 of 5 bits, of 8 bits in AEE encoding, and of the ring step at 7: 3,584).  Up to 2,048 superchunks every wave of eights has a SIMD to
 // itself, and half of the SIMDs would have none of sixteens.  Beyond, a short chain is worth the chunk's work done twice where the chain is
 // long and nothing is drawn: at 16-bit elements MEE from 6 bits on, at 32 bits from 5 bits MEE and from 8 bits AEE on; a ring step, which decodes on top, at
-// 8 bits only.
-constexpr int64_t kShortRun = 2048, kShortDecode = 3072, kLongChainRun = 16384, kLongChainStep = 12288;
+// 8 bits only.  Half a chunk of 7-bit codes is seven bytes that a lane reads one by one, and 16-bit elements do not hide that as long.
+constexpr int64_t kShortRun = 2048, kShortDecode = 3072, kShortDecode7 = 2560, kLongChainRun = 16384, kLongChainStep = 12288;
 
 static bool short_encode(int64_t nsc, bool fused, int nbits, bool f32, bool mee, bool drawn)
 {
@@ -232,7 +241,7 @@ static hipError_t dispatch_decompress(const uint8_t *src, void *dst, const int32
                                       int64_t limit, int64_t nsc, int nbits, int dtype, bool mee, const MeeParams &mp,
                                       int add, hipStream_t stream)
 {
-    if (!rows && !stats && !add && limit >= nsc * 256 && nsc <= kShortDecode)
+    if (!rows && !stats && !add && limit >= nsc * 256 && nsc <= (nbits == 7 && (dtype & 0xf) == DQ_BF16 ? kShortDecode7 : kShortDecode))
         return launch_hier16_short_decompress(src, dst, nsc, nbits, dtype, mee, mp, stream);
     if ((dtype & 0xf) == DQ_BF16) {
         DQ_NBITS_MEE(run_decompress, DQ_BF16, src, dst, rows, stats, limit, nsc, add, mp, stream)

@@ -203,6 +203,12 @@ def test_either_side_of_eight_elements_per_lane(capi, oracle, dt, nbits, strateg
                 assert torch.equal(step[:nbytes], drawn), tag + " step"
 
 
+@pytest.mark.parametrize("strategy", [2, 3])
+def test_either_side_of_eight_7_bit_codes_per_lane(capi, oracle, strategy):
+    """bf16 vectors of 7-bit codes are decoded with eight elements per lane to 2,560 superchunks"""
+    test_either_side_of_eight_elements_per_lane(capi, oracle, BF16, 7, strategy, (2560, 2561, 3072))
+
+
 @pytest.mark.parametrize("dt", [BF16, F32])
 @pytest.mark.parametrize("strategy", [2, 3])
 def test_special_values(capi, oracle, dt, strategy):
