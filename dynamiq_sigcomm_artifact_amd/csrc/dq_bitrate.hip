@@ -74,7 +74,7 @@ __global__ __launch_bounds__(kSearchThreads) void bitrate_search_kernel(uint32_t
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
 
     // (the first load, without a branch in front of the others; read by every thread long before thread 0 writes out[])
-    const double read_u = *(prev_u_dev ? prev_u_dev : reinterpret_cast<const double *>(hist));
+    const double read_u = *(prev_u_dev ? prev_u_dev : &kNoOffset);
     uint4 v[kSlabs]; // bins 4 (t + 1024 k) ..
     const bool whole = (reinterpret_cast<uintptr_t>(hist) & 15) == 0;
     if (whole) {

@@ -6,6 +6,10 @@
 
 namespace dq {
 
+// What stands in for an offset that is a number of the launch and not in device memory, where it is loaded all the same: behind a branch, the
+// loads that follow would only leave when the offset has arrived.
+static __device__ double kNoOffset = 0.0; // (never written; a constant would lie in another address space and make the load one of either)
+
 __device__ __forceinline__ float round_bf16(float x) { return bf16_bits_to_f32(f32_to_bf16_bits(x)); }
 
 // testbed_evaluation/new_comm_hooks/comm_hooks.py:64-70 on a bf16 norm: every torch op computes in

@@ -140,6 +140,25 @@ def test_thresholds_of_every_offset(capi, oracle):
         assert int(h.hist.abs().sum()) == 0
 
 
+@pytest.mark.parametrize("shift", [1, 2])
+def test_search_of_a_histogram_off_the_16_bytes(capi, oracle, shift):
+    """a histogram aligned to its 32-bit counters alone, with the starting point a number and in device memory"""
+    norms = _norm_sets()[list(_norm_sets().keys())[0]]
+    bits_list = [to_bits(t) for t in norms]
+    room = torch.full((capi.bitrate_hist_ints() + 8,), 5, dtype=torch.int32, device=DEV)
+    hist, result = room[shift:shift + capi.bitrate_hist_ints()], torch.zeros(4, dtype=torch.float64, device=DEV)
+    hist.zero_()
+    assert hist.data_ptr() % 16 == 4 * shift
+    for mode, prev in ((0, 60.0), (1, 9.25), (1, torch.full((1,), 9.25, dtype=torch.float64, device=DEV))):
+        for t in norms:
+            capi.norm_histogram(_stats(t), hist)
+        capi.bitrate_search(hist, mode, prev, 4.375, result)
+        want = oracle.dynamic_bitrate_adjust_u(bits_list, 9.25, 4.375) if mode else oracle.dynamic_bitrate_binary_search_u(bits_list, 4.375)
+        assert tuple(result.tolist()[:3]) == tuple(want), (mode, prev)
+        assert int(hist.abs().sum()) == 0
+    assert bool((room[:shift] == 5).all()) and bool((room[shift + capi.bitrate_hist_ints():] == 5).all())
+
+
 def test_search_equals_the_torch_op_sequence_on_the_device():
     """the reference's own functions as mirrored in bitrate.py, on device tensors (the scalar u enters the add in
     binary32 there, as in the reference's CUDA run)"""
