@@ -715,8 +715,7 @@ __global__ __launch_bounds__(64 * kPartWaves) void ring_parts_kernel(RingArgs<RD
         // (neither waits for the place in the list)
         my_mean = a.mean[(int64_t)my_rank * a.nsc + min(at0 + which, a.nsc - 1)];
         total_mean = a.total[2 * min(at0 + half, a.nsc - 1)];
-        // (without a branch, behind which the other loads would only leave when it has arrived; where there is none, of what lies at hand)
-        const double u_dev = *(f.rule.u_dev ? f.rule.u_dev : reinterpret_cast<const double *>(f.counts));
+        const double u_dev = *(f.rule.u_dev ? f.rule.u_dev : &kNoOffset);
         uint32_t all = 0, before = 0;
         constexpr int kTogether = 4, kThreads = 64 * kPartWaves;
         for (int first = 0; first < words; first += kTogether * kThreads) {

@@ -784,6 +784,28 @@ def test_rings_without_lists(capi, W, n, dt):
     assert len(seen) > 1
 
 
+@pytest.mark.parametrize("shift", [1, 2, 3])
+def test_rings_without_lists_with_counts_off_the_16_bytes(capi, shift):
+    """group sizes and lists aligned to their 32-bit numbers alone, with the offset a number and in device memory"""
+    from dynamiq_sigcomm_artifact_amd.dynamiq_pipeline import dynamic_bitrate_allreduce_single_pass
+    W, n, dt = 3, 256 * 301 - 7, torch.bfloat16
+    nsc = (n + 255) // 256
+    g = torch.Generator(device=DEV).manual_seed(n)
+    scales = torch.exp(torch.randn(nsc, 1, generator=g, device=DEV) * 6.0) * 1e-3
+    vecs = [(torch.randn(nsc, 256, generator=g, device=DEV) * scales).reshape(-1)[:n].to(dt).contiguous() for _ in range(W)]
+    want, total, counts = dynamic_bitrate_allreduce_single_pass(vecs, 6.0, seed=11)
+    ints = lambda m: torch.zeros(m + 4, dtype=torch.int32, device=DEV)[shift:shift + m]
+    work = {"key": ("single_pass", nsc, dt, W), "total": torch.empty((nsc, 2), dtype=torch.bfloat16, device=DEV),
+            "mean": torch.empty(W * nsc, dtype=torch.float32, device=DEV), "plan": ints(capi.group_plan_work_ints(nsc)), "order": ints(3 * nsc)}
+    work["counts"] = work["plan"][:4]
+    assert work["counts"].data_ptr() % 16 == 4 * shift
+    for u in (6.0, torch.full((1,), 6.0, dtype=torch.float64, device=DEV)):
+        outs, total2, counts2 = dynamic_bitrate_allreduce_single_pass(vecs, u, seed=11, work=work)
+        assert counts2.data_ptr() == work["counts"].data_ptr() and counts2.tolist() == counts.tolist()
+        assert torch.equal(bits_t(total), bits_t(total2)) and all(torch.equal(bits_t(x), bits_t(y)) for x, y in zip(outs, want))
+        work["counts"].fill_(-1)
+
+
 @pytest.mark.parametrize("W,n,dt", [(8, 256 * 12288, torch.bfloat16), (16, 256 * 8705 - 3, torch.float32)])
 def test_rings_without_lists_behind_several_tiles_per_wave(capi, W, n, dt):
     """so many ranks that the statistics take four tiles per wave while the ring still goes by their counts"""
