@@ -678,11 +678,11 @@ constexpr int kPartWaves = 4;
 // place among those of its width.  The statistics leave a word per four superchunks with their widths' counts; a workgroup takes
 // neighbouring superchunks and adds up the words, all of them and those before its own, while the norms of its own are on their way.
 //
-// Fours in MEE stay within 64 vector and 80 scalar registers (79 with bf16), or a SIMD has room for seven waves instead of eight, whatever the
-// compiler counts: with 81, 96 and the trap handler's 16 are taken.  MEE from 7,169 superchunks on, all vectors an element off the 16 bytes, with
-// 81 -> 79, us: 2 x 8,192 23.6 -> 22.5, 8 x 8,192 71.0 -> 65.2.
+// Fours with drawn values are held to 64 vector registers and stay within 80 scalar ones, or a SIMD has room for seven waves instead of eight,
+// whatever the compiler counts: with 81, 96 and the trap handler's 16 are taken.  MEE from 7,169 superchunks on, all vectors an element off the
+// 16 bytes, with 81 -> 79, us: 2 x 8,192 23.6 -> 22.5, 8 x 8,192 71.0 -> 65.2.
 template <int DT, int RDT, bool MEE, int N, bool PLANS>
-__global__ __launch_bounds__(64 * kPartWaves) void ring_parts_kernel(RingArgs<RDT != DQ_PHILOX> a)
+__global__ __launch_bounds__(64 * kPartWaves, N == 4 && RDT == DQ_PHILOX ? 8 : 1) void ring_parts_kernel(RingArgs<RDT != DQ_PHILOX> a)
 {
     constexpr int P = N / 4, kLanes = 64 / P, kHere = P * kPartWaves; // superchunks of a wave, lanes of one, superchunks of the workgroup
     constexpr bool POOL = RDT != DQ_PHILOX;
@@ -797,8 +797,10 @@ __global__ __launch_bounds__(64 * kPartWaves) void ring_parts_kernel(RingArgs<RD
     const bool ragged = max(sc[0], sc[P - 1]) * 256 + 256 > a.n;
     // The vector's end may lie inside a lane's elements: it loads the last N there are and drops those before its own when it comes to
     // them.  (Loaded one by one and put together on the spot, the one ragged wave of a launch waited for memory in every step and
-    // outlasted all others: 15.8 us where they had ended at 11 to 13, 8 x 1,000,003 elements.)
-    const bool whole_loads = (a.vec & 1) != 0 && a.n >= N;
+    // outlasted all others: 15.8 us where they had ended at 11 to 13, 8 x 1,000,003 elements.)  Vectors off the 16 bytes are loaded in one piece
+    // too: element by element, a lane waited for each.  Statistics and ring, all vectors an element off, us: 8 x 7,000 superchunks 57.7 -> 50.1,
+    // 16 x 7,000 111 -> 96, 2 x 12,288 29.8 -> 27.8, fp32 8 x 3,907 52.0 -> 47.8.
+    const bool whole_loads = a.n >= N;
     const int64_t from = min(e0, a.n - N);
     const WidthRegs<MEE> w = width_regs<MEE>(a.widths, my_cls, levels);
     uint64_t my_pool = 0; // of step `lane`
@@ -821,7 +823,7 @@ __global__ __launch_bounds__(64 * kPartWaves) void ring_parts_kernel(RingArgs<RD
         if (whole_loads)
             next.load_anywhere(pointer(src), from);
         else
-            load_chunk<DT>(next, pointer(src), e0, a.n, a.vec & 1, ragged);
+            load_chunk_guarded<DT>(next, pointer(src), e0, a.n);
         if constexpr (POOL) next_r.load(pointer(pool), lane * N, (a.vec & 4) != 0);
     };
     // With lists the means wait for an entry of the list, and the first step's elements not for them: its addresses come from the lanes

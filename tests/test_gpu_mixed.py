@@ -882,6 +882,20 @@ def test_rings_off_the_16_bytes(capi, W, nsc, off_in, off_out):
             assert all(bool((r[:off_out] == 7.0).all()) and bool((r[off_out + n:] == 7.0).all()) for r in rooms)
 
 
+@pytest.mark.parametrize("dt,off", [(torch.bfloat16, k) for k in range(1, 8)] + [(torch.float32, k) for k in (1, 2, 3)])
+def test_short_rings_at_every_offset_from_the_16_bytes(capi, dt, off):
+    """a lane's elements in one piece from any element on, with ends at every place in the last lane and vectors shorter than a lane's
+    share; eight elements per lane at the last length"""
+    from dynamiq_sigcomm_artifact_amd.dynamiq_pipeline import _single_pass_in_steps, dynamic_bitrate_allreduce_single_pass
+    g = torch.Generator(device=DEV).manual_seed(off)
+    whole = [torch.full((256 * 5200 + 16,), 3.0, device=DEV).to(dt) for _ in range(2)]
+    for n in (1, 2, 3, 4, 5, 7, 8, 9, 255, 256, 257, 764, 768 + off, 256 * 5122 - off):
+        vecs = [w[off:off + n].copy_(torch.randn(n, generator=g, device=DEV)) for w in whole]
+        outs, _, _ = dynamic_bitrate_allreduce_single_pass(vecs, 6.0, strategy=2, seed=11)
+        ref, _, _ = _single_pass_in_steps(vecs, 6.0, 2, 11, None, {}, None, None)
+        assert all(torch.equal(bits_t(x), bits_t(y)) for x, y in zip(outs, ref)), n
+
+
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
 def test_ends_inside_a_lane_of_a_short_ring(capi, dt):
     """vectors of one to nine elements, and every end in the last superchunk's first and last lanes"""
