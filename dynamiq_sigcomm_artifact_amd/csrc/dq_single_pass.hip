@@ -898,9 +898,10 @@ __global__ __launch_bounds__(64 * kPartWaves, N == 4 && RDT == DQ_PHILOX ? 8 : 1
 //   8 ranks  x 2,000 (500,000 elements) 16.2 15.1 17.1, x 4,000 20.6 19.3 20.0, 22.3 21.0 21.7, x 5,000 24.0 22.6 24.0, 26.2 24.8 26.4,
 //            x 8,000 31.8 29.3 28.6, 34.9 32.8 31.3, x 12,000 40.8 37.5 34.9, 44.7 42.6 40.9
 // With fp32 elements eight are 32 bytes of a lane and its loads half lines: 5 ranks x 8,000 27.8 26.8 31.3, so fp32 stays with four; pools
-// do as well (bf16, 4 x 4,600 in AEE 18.0 17.8 30.3).  Vectors off the 16 bytes stay with four at every length: they load and store element by
-// element, and with eight of them a lane has half as many on the way.  All of them an element off, four -> eight: 2 x 5,200 17.5 -> 19.5,
-// 8 x 5,200 48.4 -> 63.2, 8 x 8,192 63.6 -> 80.6, 8 x 16,000 117 -> 147, in MEE 4 x 12,000 54.1 -> 68.9.
+// do as well (bf16, 4 x 4,600 18.0 -> 18.7, 8 x 5,200 27.2 -> 28.5, in MEE 19.3 -> 20.4, 29.0 -> 30.3).  Outputs off the 16 bytes are stored element by
+// element, of which eight lie twice as far from the neighbour's, and fours stay at every length: 2 x 8,192 14.6 -> 15.6, 4 x 12,288 26.6 -> 32.0,
+// 8 x 16,000 53.1 -> 70.4, in MEE 58.4 -> 74.3.  (Vectors off them alone are loaded in one piece: 2 x 8,192 19.4 -> 17.9, 4 x 12,288 42.7 -> 43.2, 8 x
+// 16,000 94.8 -> 91.6.)
 // From five ranks without a plan on, three with one, the steps are most of the time, and fours keep the lead up to seven waves per SIMD.  Of
 // the time before there were eights, eight / four: 8 ranks x 5,200 0.994 / 0.932 (AEE), 1.000 / 0.936 (MEE), x
 // 7,000 1.012 / 0.926, 1.044 / 0.951, x 7,300 0.943 / 0.933, 0.931 / 0.935; 5 x 7,000 0.992 / 0.964, 1.007 / 0.965; 4 x 7,000 0.958 / 0.959,
@@ -1079,7 +1080,7 @@ static hipError_t run_ring(const RingDesc &d, bool mee, const MeeParams *mp, hip
         };
         constexpr bool PLANS = decltype(plans)::value;
         if constexpr (DT == DQ_BF16 && !POOL) {
-            if (a.nsc > fours_to(d.world, PLANS) && (a.vec & 3) == 3)
+            if (a.nsc > fours_to(d.world, PLANS) && (a.vec & 2) != 0)
                 return mee ? go(ring_parts_kernel<DT, RDT, true, 8, PLANS>, 2 * kPartWaves) : go(ring_parts_kernel<DT, RDT, false, 8, PLANS>, 2 * kPartWaves);
         }
         return mee ? go(ring_parts_kernel<DT, RDT, true, 4, PLANS>, kPartWaves) : go(ring_parts_kernel<DT, RDT, false, 4, PLANS>, kPartWaves);

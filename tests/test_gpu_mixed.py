@@ -861,8 +861,8 @@ def test_few_ranks_on_either_side_of_their_last_ring_without_a_plan(capi, W, n):
 @pytest.mark.parametrize("W,nsc", [(2, 5121), (3, 12288), (5, 12289), (3, 17409), (4, 20480)])
 @pytest.mark.parametrize("off_in,off_out", [(1, 3), (0, 1), (2, 0)])
 def test_rings_off_the_16_bytes(capi, W, nsc, off_in, off_out):
-    """bf16 vectors or outputs (or both) off the 16 bytes take four elements per lane where aligned ones take eight, with lists and
-    without"""
+    """bf16 vectors or outputs (or both) off the 16 bytes; outputs off them take four elements per lane where aligned ones take eight, with
+    lists and without"""
     from dynamiq_sigcomm_artifact_amd.bitrate import NormHistogram
     from dynamiq_sigcomm_artifact_amd.dynamiq_pipeline import _single_pass_in_steps, dynamic_bitrate_allreduce_single_pass
     n = nsc * 256 - 3
