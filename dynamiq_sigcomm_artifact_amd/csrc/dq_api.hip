@@ -620,7 +620,7 @@ int dq_ranks_allreduce(const dq_ranks_t *r, int stages, int device, dq_stream_t 
     hipError_t e = hipSuccess;
     // a short ring without lists: the words go where the lists would
     const bool no_plan = (stages & DQ_RANKS_NO_LISTS) && !r->sorted_plan && !r->hist && !r->pool &&
-                         dq::ring_plans_itself(r->src, r->out, r->n, r->world, r->dtype);
+                         dq::ring_plans_itself(r->n, r->world, r->dtype);
     uint32_t *words = no_plan ? reinterpret_cast<uint32_t *>(r->order) : nullptr;
     if (s_stats) e = dq::launch_ranks_stats(r->src, r->world, r->n, r->total, r->mean, r->dtype, words, (float)r->u, r->u_dev, s);
     if (e == hipSuccess && s_plan && !no_plan) {

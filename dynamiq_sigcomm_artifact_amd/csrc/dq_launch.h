@@ -124,7 +124,7 @@ hipError_t launch_roundtrip(const RoundtripDesc *desc, int count, int world, flo
 hipError_t launch_ranks_stats(const void *const *src, int world, int64_t n, void *total, float *mean, int dtype,
                               uint32_t *tile_widths, float u, const double *u_dev, hipStream_t stream);
 // a ring that finds its groups from the words of launch_ranks_stats (in the place of a plan and its lists)
-bool ring_plans_itself(const void *const *src, void *const *out, int64_t n, int world, int dtype);
+bool ring_plans_itself(int64_t n, int world, int dtype);
 struct RingDesc {
     const void *const *src;
     void *const *out;

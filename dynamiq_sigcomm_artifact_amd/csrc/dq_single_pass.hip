@@ -909,8 +909,8 @@ __global__ __launch_bounds__(64 * kPartWaves, N == 4 && RDT == DQ_PHILOX ? 8 : 1
 constexpr int kFoursTo = 5120, kFoursToMany = 7168;
 constexpr int fours_to(int world, bool plans) { return world >= (plans ? 5 : 3) ? kFoursToMany : kFoursTo; }
 
-// With lists from a plan, up to so many superchunks in parts.  bf16 with drawn values, plan and all, us, sixteen -> eight: 2 ranks x 10,240 19.1 ->
-// 17.3 (AEE), 20.3 -> 18.4 (MEE), x 12,000 18.0 -> 17.9, 20.8 -> 20.2, x 16,000 19.5 -> 20.0; 5 x 16,000 35.9 -> 34.5, 40.2 -> 40.0, x 20,000 41.9 -> 40.0, 47.1 -> 45.6; 8 x 20,000
+// With lists from a plan, up to so many superchunks in parts.  bf16 with drawn values, plan and all, us, sixteen -> eight: 2 ranks x 12,000 17.7 ->
+// 17.1 (AEE), 20.0 -> 20.2 (MEE), x 16,000 19.5 -> 20.0; 5 x 16,000 35.9 -> 34.5, 40.2 -> 40.0, x 20,000 41.9 -> 40.0, 47.1 -> 45.6; 8 x 20,000
 // 54.8 -> 52.7, 63.1 -> 60.1.  The others, kernel alone, sixteen -> four: 8 ranks x 256 superchunks 12.2 -> 7.8 (AEE), 15.9 -> 8.9 (MEE),
 // 19.5 -> 8.3 (AEE from pools); x 8,192 from pools 26.2 -> 20.6, fp32 24.6 -> 23.2, 29.0 -> 23.9.  Two ranks in fp32 AEE with drawn values
 // have their line at five waves per SIMD: x 4,900 6.8 -> 6.5, x 5,700 6.8 -> 7.2.
@@ -927,11 +927,8 @@ int parts_to(int world, bool bf16, bool mee, bool pooled)
 // bf16: 2 ranks x 16,000 19.6 -> 18.2 (AEE), 21.5 -> 20.4 (MEE), x 24,000 24.4 -> 24.4, 27.6 -> 28.5; 3 x 16,000 25.3 -> 23.7, 27.5 -> 26.7,
 // x 24,000 31.5 -> 32.2, 35.5 -> 37.1; 8 x 16,000 48.6 -> 42.8, 53.9 -> 47.9, x 24,000 65.0 -> 61.8, 73.5 -> 70.0.  fp32, with four elements per
 // lane: 2 x 12,000 20.3 -> 19.3, 22.0 -> 20.4, x 16,000 24.5 -> 24.1, 24.5 -> 25.7; 5 x 16,000 49.7 -> 46.9, 51.1 -> 48.4; 8 x 16,000 78.5 ->
-// 74.9, 77.9 -> 75.8, x 20,000 96.9 -> 96.9, 98.9 -> 98.5.  Two and three ranks of bf16 near their line, again with a plan -> without: 2 x 17,000
-// 20.1 -> 19.9, 22.9 -> 22.5, x 17,500 20.8 -> 21.0, 24.0 -> 23.5, x 18,500 21.2 -> 21.9, 24.6 -> 24.3, x 19,500 21.6 -> 22.4, 24.6 -> 25.0; 3 x 17,500 27.1 ->
-// 27.0, 30.9 -> 30.1, x 18,500 27.5 -> 28.1, 31.1 -> 31.1, x 19,500 28.3 -> 29.3, 31.9 -> 32.2.  Off the 16 bytes, where the plan's ring has sixteen
-// elements to load one by one, the longer line holds for them too: 2 x 20,480 82.8 -> 53, 3 x 20,480 116 -> 68.
-constexpr int kPlansItself = 20480, kPlansItselfFew = 17408, kPlansItself32 = 16384, kPlansItselfFew32 = 12288;
+// 74.9, 77.9 -> 75.8, x 20,000 96.9 -> 96.9, 98.9 -> 98.5.
+constexpr int kPlansItself = 20480, kPlansItself32 = 16384, kPlansItselfFew32 = 12288;
 static_assert(kPlansItself <= 0xffff, "a width's count over all superchunks is half a word (ring_parts_kernel, PLANS)");
 
 WidthRule make_rule(float u, const double *u_dev)
@@ -1098,14 +1095,9 @@ static hipError_t run_ring(const RingDesc &d, bool mee, const MeeParams *mp, hip
                : launch_with(ring_kernel<DT, RDT, false>, grid, dim3(64), stream, a);
 }
 
-bool ring_plans_itself(const void *const *src, void *const *out, int64_t n, int world, int dtype)
+bool ring_plans_itself(int64_t n, int world, int dtype)
 {
-    const int64_t nsc = (n + 255) / 256;
-    if (dtype != DQ_BF16) return nsc <= (world < 4 ? kPlansItselfFew32 : kPlansItself32);
-    if (world >= 4 || nsc <= kPlansItselfFew) return nsc <= kPlansItself;
-    bool aligned = true;
-    for (int r = 0; r < world; r++) aligned = aligned && aligned16(src[r]) && aligned16(out[r]);
-    return !aligned && nsc <= kPlansItself;
+    return (n + 255) / 256 <= (dtype == DQ_BF16 ? kPlansItself : (world < 4 ? kPlansItselfFew32 : kPlansItself32));
 }
 
 hipError_t launch_ring(const RingDesc &d, int dtype, bool mee, const MeeParams *mp, hipStream_t stream)

@@ -852,13 +852,7 @@ def test_rings_on_either_side_of_eight_elements_per_lane(capi, W, n):
     test_rings_without_lists(capi, W, n, torch.bfloat16)
 
 
-@pytest.mark.parametrize("W,n", [(2, 256 * 17408), (2, 256 * 17409 - 255), (3, 256 * 17408 - 3), (3, 256 * 17409), (4, 256 * 17409)])
-def test_few_ranks_on_either_side_of_their_last_ring_without_a_plan(capi, W, n):
-    """bf16: two and three ranks plan themselves to 17,408 superchunks, four and more to 20,480"""
-    test_rings_without_lists(capi, W, n, torch.bfloat16)
-
-
-@pytest.mark.parametrize("W,nsc", [(2, 5121), (3, 12288), (5, 12289), (3, 17409), (4, 20480)])
+@pytest.mark.parametrize("W,nsc", [(2, 5121), (3, 12288), (5, 12289), (4, 20480)])
 @pytest.mark.parametrize("off_in,off_out", [(1, 3), (0, 1), (2, 0)])
 def test_rings_off_the_16_bytes(capi, W, nsc, off_in, off_out):
     """bf16 vectors or outputs (or both) off the 16 bytes; outputs off them take four elements per lane where aligned ones take eight, with
