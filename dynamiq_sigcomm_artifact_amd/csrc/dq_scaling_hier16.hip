@@ -145,14 +145,17 @@ constexpr int64_t kLongRun = 262144; // superchunks of a row list: 16384 waves o
 // (in the columns of 3,072 of 5 bits, of 8 bits in AEE encoding, and of the ring step at 7: 3,584).  Up to 2,048 superchunks every wave of eights has a SIMD to
 // itself, and half of the SIMDs would have none of sixteens.  Beyond, a short chain is worth the chunk's work done twice where the chain is
 // long and nothing is drawn: at 16-bit elements MEE from 6 bits on, at 32 bits from 5 bits MEE and from 8 bits AEE on; a ring step, which decodes on top, at
-// 8 bits only.  Half a chunk of 7-bit codes is seven bytes that a lane reads one by one, and 16-bit elements do not hide that as long.
-constexpr int64_t kShortRun = 2048, kShortDecode = 3072, kShortDecode7 = 2560, kLongChainRun = 16384, kLongChainStep = 12288;
+// 8 bits only, and less far: with vectors that no cache holds, us, MEE bf16 x 9,728 7.19 -> 6.90, x 10,240 7.38 -> 7.30, x 11,264 7.78 -> 7.68 but read
+// again 5.52 -> 5.75, x 12,288 5.62 -> 5.97; fp32 x 10,240 8.45 -> 8.34, x 12,288 9.16 -> 9.29; AEE fp32 x 9,216 7.17 -> 7.11, x 10,240 7.51 -> 7.68,
+// x 12,288 8.30 -> 8.62.  (Compress of 7 bits in MEE, bf16, x 12,288 6.08 -> 5.50, x 16,384 7.05 -> 6.73, but the same vector again and
+// again 4.68 -> 4.86, 5.32 -> 5.50.)  Half a chunk of 7-bit codes is seven bytes that a lane reads one by one, and 16-bit elements do not hide that as long.
+constexpr int64_t kShortRun = 2048, kShortDecode = 3072, kShortDecode7 = 2560, kLongChainRun = 16384, kLongChainStepMee = 10240, kLongChainStep = 9216;
 
 static bool short_encode(int64_t nsc, bool fused, int nbits, bool f32, bool mee, bool drawn)
 {
     if (nsc <= kShortRun) return true;
     if (drawn) return false;
-    if (fused) return nsc <= kLongChainStep && nbits == 8 && (mee || f32);
+    if (fused) return nbits == 8 && (mee ? nsc <= kLongChainStepMee : f32 && nsc <= kLongChainStep);
     return nsc <= kLongChainRun && (mee ? nbits >= (f32 ? 5 : 6) : nbits == 8 && f32);
 }
 

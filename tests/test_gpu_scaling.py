@@ -155,7 +155,7 @@ def test_production_shape_random(capi, oracle, dt, nbits, strategy):
 @pytest.mark.parametrize("nbits,strategy,nscs", [(4, 2, (2047, 2049, 3073)), (5, 3, (2048, 3072, 16385)), (7, 3, (2049, 16384)),
                                                  (8, 2, (2, 12288, 16385)), (8, 3, (2050, 12289, 16384))])
 def test_either_side_of_eight_elements_per_lane(capi, oracle, dt, nbits, strategy, nscs):
-    """The codec takes eight elements per lane up to 2,048 superchunks (decoding 3,072; long chains 12,288 and 16,384) and sixteen
+    """The codec takes eight elements per lane up to 2,048 superchunks (decoding 3,072; long chains 9,216, 10,240 and 16,384) and sixteen
     beyond: the same bytes on either side of every line, with waves on the guarded path, elements on the boundaries of the
     rounding, and buffers off the 16 bytes."""
     tdt = TORCH_DT[dt]
@@ -207,6 +207,12 @@ def test_either_side_of_eight_elements_per_lane(capi, oracle, dt, nbits, strateg
 def test_either_side_of_eight_7_bit_codes_per_lane(capi, oracle, strategy):
     """bf16 vectors of 7-bit codes are decoded with eight elements per lane to 2,560 superchunks"""
     test_either_side_of_eight_elements_per_lane(capi, oracle, BF16, 7, strategy, (2560, 2561, 3072))
+
+
+@pytest.mark.parametrize("dt,strategy,nscs", [(F32, 2, (9216, 9217)), (F32, 3, (10240, 10241)), (BF16, 3, (10240, 10241))])
+def test_either_side_of_eight_elements_per_lane_in_ring_steps(capi, oracle, dt, strategy, nscs):
+    """ring steps of 8 bits take eight elements per lane to 9,216 superchunks, in MEE to 10,240"""
+    test_either_side_of_eight_elements_per_lane(capi, oracle, dt, 8, strategy, nscs)
 
 
 @pytest.mark.parametrize("dt", [BF16, F32])
