@@ -496,10 +496,11 @@ __device__ __forceinline__ int exact_code_fast(float vi, float ri, float d, doub
 //        bounded by (1.44 * 5e-7 + 2.7 ulp(log)) / log2(base) + 2 ulp(2 R): < 8e-5 for 6..8 bits (log2(base) = 0.0286,
 //        log < 4) and < 1.6e-5 below (log2(base) >= 0.09, log < 1.5); measured over 4e9 random operands per width: 1.5e-5
 //        and 4.8e-6 (without the constant in the last fma, which adds at most 3.8e-6 and 1e-6).
-// kDelta is the power of two above these bounds (half a unit of (R + 1) 2^-20, 1.2e-4, 3.1e-5).  With twice as much, twice the waves redo
+// kDelta is the power of two above these bounds, 1.5 to 1.9 times as much (half a unit of (R + 1) 2^-20, 1.2e-4, 3.1e-5).  With twice as much, twice the waves redo
 // elements: at 8 bits in MEE 40 instead of 22 %, compress of 524,288 elements 2.84 -> 2.74 us, ring step of 6,553,600 10.5 -> 10.3.
+constexpr float estimate_delta(int nbits, bool mee) { return mee ? (nbits >= 6 ? 0x1p-13f : 0x1p-15f) : (float)(1 << (nbits - 1)) * 0x1p-21f; }
 template <int NBITS, bool MEE> struct EstimateGuard {
-    static constexpr float kDelta = MEE ? (NBITS >= 6 ? 0x1p-13f : 0x1p-15f) : (float)(1 << (NBITS - 1)) * 0x1p-21f;
+    static constexpr float kDelta = estimate_delta(NBITS, MEE);
 };
 
 // bias - r_i; exact for the in-kernel random bytes ((256 bias - odd byte) / 256 needs 16 bits)

@@ -245,8 +245,7 @@ inline WidthSet make_width_set(const MeeParams *mp, bool mee)
     for (int k = 0; k < 3; k++) {
         WidthConst &w = s.w[k];
         const int top = (1 << (bits[k] - 1)) - 1;
-        // EstimateGuard: kDelta of estimate_codes
-        const float delta = mee ? (bits[k] >= 6 ? 0x1p-13f : 0x1p-15f) : (float)(1 << (bits[k] - 1)) * 0x1p-21f;
+        const float delta = estimate_delta(bits[k], mee); // (kDelta of estimate_codes)
         w.r = (float)top;
         w.bias = 1.0f + delta;
         w.two_delta = 2.0f * delta;
