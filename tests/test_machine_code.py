@@ -145,3 +145,19 @@ def test_statistics_of_all_ranks_fit_their_registers(tmp_path):
         scratch[field["name"]] = int(field["private_segment_fixed_size"])
     stats = {name: size for name, size in scratch.items() if "ranks_stats_kernel" in name}
     assert len(stats) >= 6 and not any(stats.values()), stats
+
+
+def test_short_rings_leave_room_for_eight_waves(tmp_path):
+    """ring_parts_kernel with four elements per lane and drawn values: 64 vector and 80 scalar registers, no scratch"""
+    if not os.path.exists(READELF):
+        pytest.skip("no llvm-readelf")
+    from dynamiq_sigcomm_artifact_amd import capi
+    path = tmp_path / "single_pass.co"
+    path.write_bytes(next(c for c in _code_objects(capi.LIB_PATH) if b"ring_parts_kernel" in c))
+    notes = subprocess.run([READELF, "--notes", str(path)], stdout=subprocess.PIPE, text=True, check=True).stdout
+    fields = [dict(re.findall(r"^\s+\.(name|private_segment_fixed_size|vgpr_count|sgpr_count):\s+(\S+)", text, re.M))
+              for text in notes.split("- .agpr_count")[1:]]
+    fours = [f for f in fields if re.search(r"ring_parts_kernelILi\dELi3ELb[01]ELi4E", f["name"])]
+    assert len(fours) == 8, fields
+    for f in fours:
+        assert int(f["private_segment_fixed_size"]) == 0 and int(f["vgpr_count"]) <= 64 and int(f["sgpr_count"]) <= 80, f
