@@ -199,7 +199,6 @@ template <int N> struct RawPart<DQ_PHILOX, N> {
             asm("" : "+v"(w[k]));
         }
     }
-    __device__ __forceinline__ void load(const void *, int64_t, bool) {}
     __device__ __forceinline__ float odd_byte(int i) const { return (float)((w[i >> 2] >> (8 * (i & 3))) & 0xffu); }
     __device__ __forceinline__ float get(int i) const { return odd_byte(i) * 0.00390625f; }
     __device__ __forceinline__ bool unit_interval() const { return true; }

@@ -245,7 +245,6 @@ struct TallyBucket {
 template <int MOST> struct TallyArgs {
     uint32_t first_block[MOST];
     TallyBucket bucket[MOST];
-    int buckets;
     WidthRule rule;
     uint32_t *hist;
     uint64_t *step_dev;
@@ -927,7 +926,9 @@ int parts_to(int world, bool bf16, bool mee, bool pooled)
 // bf16: 2 ranks x 16,000 19.6 -> 18.2 (AEE), 21.5 -> 20.4 (MEE), x 24,000 24.4 -> 24.4, 27.6 -> 28.5; 3 x 16,000 25.3 -> 23.7, 27.5 -> 26.7,
 // x 24,000 31.5 -> 32.2, 35.5 -> 37.1; 8 x 16,000 48.6 -> 42.8, 53.9 -> 47.9, x 24,000 65.0 -> 61.8, 73.5 -> 70.0.  fp32, with four elements per
 // lane: 2 x 12,000 20.3 -> 19.3, 22.0 -> 20.4, x 16,000 24.5 -> 24.1, 24.5 -> 25.7; 5 x 16,000 49.7 -> 46.9, 51.1 -> 48.4; 8 x 16,000 78.5 ->
-// 74.9, 77.9 -> 75.8, x 20,000 96.9 -> 96.9, 98.9 -> 98.5.
+// 74.9, 77.9 -> 75.8, x 20,000 96.9 -> 96.9, 98.9 -> 98.5.  Few ranks of bf16 near their line, with a plan -> without: 2 x 18,432 21.1 -> 19.8, 24.5 ->
+// 22.8, x 19,000 21.4 -> 21.4, 24.6 -> 24.5, x 19,500 21.5 -> 21.3, 24.5 -> 24.9, x 20,480 21.6 -> 21.4, 26.0 -> 24.8; 3 x 18,432 27.9 -> 26.2, 31.7 ->
+// 29.6, x 19,500 27.4 -> 28.1, 31.8 -> 32.1, x 20,000 28.1 -> 27.9, 31.7 -> 31.8, x 20,480 30.4 -> 27.9, 34.1 -> 31.9.
 constexpr int kPlansItself = 20480, kPlansItself32 = 16384, kPlansItselfFew32 = 12288;
 static_assert(kPlansItself <= 0xffff, "a width's count over all superchunks is half a word (ring_parts_kernel, PLANS)");
 
@@ -967,7 +968,7 @@ static hipError_t run_roundtrip(const RoundtripDesc *desc, int count, int world,
         tiles += (uint32_t)((nsc + kRowsPerWave - 1) / kRowsPerWave);
         blocks += (uint32_t)((nsc + kTallyBatch - 1) / kTallyBatch);
     }
-    a.buckets = t.buckets = count;
+    a.buckets = count;
     a.rule = t.rule = make_rule(u, u_dev);
     a.wd = make_world_div(world, dtype == DQ_F32 ? 4 : 2);
     a.seed = seed;
