@@ -349,7 +349,7 @@ def test_few_blocks_of_2p15_are_those_of_a_long_vector(capi, blocks):
             capi.rht_blocked(long, capi.pack_signs(sign) if packed else sign, block, scale, inverse)
             capi.rht_blocked(few, capi.pack_signs(sign[:n]) if packed else sign[:n], block, scale, inverse)
             assert torch.equal(few.view(torch.int32), long[:n].view(torch.int32)), (packed, inverse)
-    odd = torch.zeros(n + 1, device=DEV)[1:].copy_(x[:n])       # off the 16 bytes: as before
+    odd = torch.zeros(n + 1, device=DEV)[1:].copy_(x[:n])       # off the 16 bytes: two passes as well
     capi.rht_blocked(odd, sign[:n], block, scale, True)
     long = x.clone()
     capi.rht_blocked(long, sign, block, scale, True)
@@ -726,7 +726,39 @@ def test_many_slices_share_launches(capi, sizes, nbits, dt):
 
 
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("n,dim", [(1024, 1024), (40000, 65536), (1 << 20, 1 << 20), (1000, 1024), ((1 << 21) + 5, 1 << 22)])
+@pytest.mark.parametrize("n", [16385, 20255, 1 << 15])
+def test_thc_of_one_block_of_2p15_is_that_of_a_long_vector(capi, n, dt):
+    """THC's compress and decompress of one block of 2^15 in two passes, with a source and a destination shorter than the block and the grid
+    from a norm on the device, against the first of 40 blocks, which take one pass, with the quantisers on their own"""
+    from dynamiq_sigcomm_artifact_amd.thc import OldINCACudaHadamardCompressor
+    dim, name = 1 << 15, (0, 1)
+    c = OldINCACudaHadamardCompressor({"d": {name: dim}, "size": {name: n}, "T": 2.7, "device": DEV, "nclients": 6, "rank": 0})
+    g = torch.Generator(device=DEV).manual_seed(n)
+    x = torch.randn(n, generator=g, device=DEV).to(dt)
+    norm, u = x.float().norm(), torch.rand(dim, generator=g, device=DEV)
+    levels = c.compress(x, name, norm, uniform=u)
+    rot = c.hadamards[name]
+    low, spacing = c._grid(norm, dim)
+    signs = torch.cat([rot.diagonal_bits] * 40)
+    long = torch.zeros(40 * dim, device=DEV)
+    long[:n] = x.float()
+    capi.rht_blocked(long, signs, dim, rot.inv_sqrt, False)
+    want = torch.empty(dim, dtype=torch.bfloat16, device=DEV)
+    capi.thc_quantize(long[:dim].contiguous(), u, want, low.reshape(1), spacing.reshape(1), 64)
+    assert torch.equal(levels.view(torch.int16), want.view(torch.int16)) and want.unique().numel() > 32
+    total = (levels.float() * 6).to(torch.bfloat16)
+    got = c.decompress(total, name).clone()
+    back = torch.empty(dim, device=DEV)
+    capi.thc_dequantize(total, back, (spacing / 6).reshape(1), low.reshape(1))
+    long.zero_()
+    long[:dim] = back
+    capi.rht_blocked(long, signs, dim, rot.inv_sqrt, True)
+    assert got.numel() == n and torch.equal(got.view(torch.int32), long[:n].view(torch.int32))
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n,dim", [(1024, 1024), (40000, 65536), (1 << 20, 1 << 20), (1000, 1024), ((1 << 21) + 5, 1 << 22),
+                                   (20255, 1 << 15), (16385, 1 << 15), (1 << 15, 1 << 15)])
 def test_thc_grid_and_source_in_the_passes(capi, n, dim, dt):
     """THC's compress and decompress with the grid from a norm on the device, from a number, and as torch works it out
     (a norm of another type takes the single calls); sources of another type, length and alignment than the transform"""

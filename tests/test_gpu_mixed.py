@@ -762,7 +762,7 @@ def test_chunk_scales_on_whole_ratios(capi, W, nsc, strategy, dt):
 @pytest.mark.parametrize("W,n,dt", [
     (8, 1, torch.bfloat16), (2, 256 * 3, torch.float32), (3, 256 * 4 + 1, torch.bfloat16), (16, 256 * 5, torch.bfloat16),
     (2, 256 * 4096, torch.bfloat16), (5, 256 * 4097, torch.bfloat16),          # as many words as a trip takes, one more
-    (2, 256 * 12288, torch.bfloat16), (3, 256 * 12288 - 255, torch.float32),   # the last length without lists
+    (2, 256 * 12288, torch.bfloat16), (3, 256 * 12288 - 255, torch.float32),   # the last length of two and three fp32 ranks
     (2, 256 * 12288 + 1, torch.bfloat16)])
 def test_rings_without_lists(capi, W, n, dt):
     """short rings find their groups from the counts per four superchunks: widths that change from one superchunk to the next, and all
@@ -814,16 +814,18 @@ def test_rings_without_lists_behind_several_tiles_per_wave(capi, W, n, dt):
 
 @pytest.mark.parametrize("W,n", [(2, 256 * 8192), (3, 256 * 8192 + 1), (5, 256 * 8195)])
 def test_ranks_on_either_side_of_a_superchunk_per_wave(capi, W, n):
-    """the last length that takes a wave per superchunk (MEE; AEE below) and the first ones that take four superchunks per wave"""
+    """bf16 beyond the last length of four elements per lane: two superchunks per wave, the last wave with one of them, with lists and
+    without"""
     test_ranks_in_registers_equal_the_ring_in_steps(capi, W, n, torch.bfloat16)
 
 
 @pytest.mark.parametrize("W,n,dt", [
     (2, 256 * 5120, torch.bfloat16), (2, 256 * 5120 + 1, torch.bfloat16), (5, 256 * 5120 + 1, torch.bfloat16),
     (6, 256 * 5120 + 1, torch.bfloat16), (6, 256 * 8192 + 1, torch.bfloat16),
-    (2, 256 * 5120, torch.float32), (2, 256 * 5120 + 1, torch.float32), (3, 256 * 8192, torch.float32)])
+    (2, 256 * 5120, torch.float32), (2, 256 * 5120 + 1, torch.float32), (3, 256 * 8192, torch.float32), (3, 256 * 8192 + 1, torch.float32)])
 def test_ranks_on_either_side_of_the_lines_of_a_superchunk_per_wave(capi, W, n, dt):
-    """AEE with the values drawn: few ranks take four superchunks per wave from 5,121 on, more of them and fp32 from 8,193"""
+    """with lists and the values drawn: two bf16 ranks take a superchunk per wave to 5,120 superchunks and two per wave beyond, more of them
+    to 7,168; fp32 a superchunk per wave to 8,192, two ranks in AEE to 5,120, and four per wave beyond"""
     test_ranks_in_registers_equal_the_ring_in_steps(capi, W, n, dt)
 
 
@@ -832,8 +834,8 @@ def test_ranks_on_either_side_of_the_lines_of_a_superchunk_per_wave(capi, W, n, 
     (7, 256 * 5127 - 5, torch.bfloat16), (2, 256 * 12288 - 1, torch.bfloat16), (3, 256 * 12289, torch.bfloat16),
     (4, 256 * 20480 - 13, torch.bfloat16), (5, 256 * 20481 - 13, torch.bfloat16)])
 def test_rings_of_eight_elements_per_lane(capi, W, n, dt):
-    """bf16 with the values drawn, from 5,121 superchunks on: two superchunks of different widths and first ranks per wave, the last wave
-    with one or both of them, the vector's end at every place in a lane's eight; lists to 12,288 or 20,480 superchunks"""
+    """bf16 with the values drawn, from 5,121 superchunks on (few ranks): two superchunks of different widths and first ranks per wave, the
+    last wave with one or both of them, the vector's end at places all over a lane's eight; lists to 12,288 or 20,480 superchunks"""
     test_ranks_in_registers_equal_the_ring_in_steps(capi, W, n, dt)
 
 
