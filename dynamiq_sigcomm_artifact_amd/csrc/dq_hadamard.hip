@@ -247,7 +247,8 @@ static int contiguous_bits(int kb)
 // Blocks of 2^15 go in two passes of 2^10 and 32 rows as well where there are few of them: as one tile each, a block is a workgroup that has
 // a CU to itself for 10 us, with most of the others idle.  Blocked transform in a graph, us, forward, one pass -> two: one block 9.8 -> 5.7, 8
 // blocks 10.1 -> 6.3, 16 10.2 -> 7.4, 32 10.6 -> 9.7 (64, one pass: 11.2); back 11.1 -> 6.9 and 11.7 -> 10.8.  THC there and back, 17,000 to
-// 32,768 elements, 31.0 -> 23.6.  (Blocks of 2^14: 5.4 -> 5.6, back 6.1 -> 7.4, THC 20.4 -> 26.4.)
+// 32,768 elements, 31.0 -> 23.2 (21.5 in one process of four).  Off the 16 bytes the passes go element by element either way: one block 23.5 to 37 ->
+// 8 to 9.7, 32 blocks 24.3 to 38 -> 14.7 to 16.7.  (Blocks of 2^14: 5.4 -> 5.6, back 6.1 -> 7.4, THC 20.4 -> 26.4.)
 constexpr int64_t kFewTo = (int64_t)32 << kMaxTileBits;
 
 // rows of the next strided pass: the remaining bits split evenly over as few passes as the LDS allows

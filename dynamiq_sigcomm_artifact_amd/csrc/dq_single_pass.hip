@@ -908,8 +908,8 @@ __global__ __launch_bounds__(64 * kPartWaves, N == 4 && RDT == DQ_PHILOX ? 8 : 1
 constexpr int kFoursTo = 5120, kFoursToMany = 7168;
 constexpr int fours_to(int world, bool plans) { return world >= (plans ? 5 : 3) ? kFoursToMany : kFoursTo; }
 
-// With lists from a plan, up to so many superchunks in parts.  bf16 with drawn values, plan and all, us, sixteen -> eight: 2 ranks x 12,000 17.7 ->
-// 17.1 (AEE), 20.0 -> 20.2 (MEE), x 16,000 19.5 -> 20.0; 5 x 16,000 35.9 -> 34.5, 40.2 -> 40.0, x 20,000 41.9 -> 40.0, 47.1 -> 45.6; 8 x 20,000
+// With lists from a plan, up to so many superchunks in parts.  bf16 with drawn values, plan and all, us, sixteen -> eight: 2 ranks x 10,240 19.1 ->
+// 17.3 (AEE), 20.3 -> 18.4 (MEE), x 12,000 18.0 -> 17.9, 20.8 -> 20.2, x 16,000 19.5 -> 20.0; 5 x 16,000 35.9 -> 34.5, 40.2 -> 40.0, x 20,000 41.9 -> 40.0, 47.1 -> 45.6; 8 x 20,000
 // 54.8 -> 52.7, 63.1 -> 60.1.  The others, kernel alone, sixteen -> four: 8 ranks x 256 superchunks 12.2 -> 7.8 (AEE), 15.9 -> 8.9 (MEE),
 // 19.5 -> 8.3 (AEE from pools); x 8,192 from pools 26.2 -> 20.6, fp32 24.6 -> 23.2, 29.0 -> 23.9.  Two ranks in fp32 AEE with drawn values
 // have their line at five waves per SIMD: x 4,900 6.8 -> 6.5, x 5,700 6.8 -> 7.2.
